@@ -30,6 +30,7 @@ struct FwdLoss {
     float *g_actor_out, *g_values, *kl;                   // [mb, head], [mb], [mb]
     float *kl_part;                                       // [row tiles] sums of the tiles' KL estimates, for the test
     int32_t *kl_flag;                                     // null: no test (nothing is left in kl_part)
+    int dw_in_tiles;                                      // forward + backward: the row tiles leave their dW1 as well
     int mb, A, continuous, clip_value;                    // A = actions (discrete) or action width (continuous)
     float clip_eps, ent_coef, value_coef, target_kl;
 };

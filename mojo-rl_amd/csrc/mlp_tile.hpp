@@ -326,11 +326,36 @@ MRL_DEV void head_rows(const float *w2s, int A, const float *h2, float *out, int
     }
 }
 
+// The head of ROWS rows (a multiple of 16) as one chain of fused multiply-adds per output in ascending n, on
+// v_mfma_f32_16x16x4_f32 (lane = 16 g + n: A[row n][k g], B[k g][column n] -> D[row 4 g + v][column n]): a
+// wavefront per 16 rows, H / 4 dependent instructions.  Nets of hidden width 128 take it: the sums of the
+// layer-by-layer kernels, whose bits their sampled actions depend on.
+// PITCH = floats per weight row in w2s, biases behind the H rows.
+template <int H, int ROWS, int PITCH>
+MRL_DEV void head_chain(const float *w2s, int A, const float *h2, float *out, int out_ld, int t) {
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    const int tile = t >> 6, g = (t >> 4) & 3, n = t & 15;
+    if (tile >= ROWS / 16) return;
+    f4 acc = {0};
+#pragma unroll 8
+    for (int kk = 0; kk < H / 4; ++kk) {
+        const int k = 4 * kk + g;
+        const float b = n < A ? w2s[k * PITCH + n] : 0.0f;
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(h2[(16 * tile + n) * (H + 1) + k], b, acc, 0, 0, 0);
+    }
+    if (n < A) {
+        const float b2 = w2s[H * PITCH + n];
+#pragma unroll
+        for (int v = 0; v < 4; ++v) out[(16 * tile + 4 * g + v) * out_ld + n] = acc[v] + b2;
+    }
+}
+
 // t = index of the calling thread among the `nthreads` (a multiple of H / 16) that share the work;
 // by default the first H threads of the net call it, two (row, part) pairs each
 template <int H>
 MRL_DEV void head(const float *w2s, int A, const float *h2, float *out, int out_ld, int t = threadIdx.x % H,
                   int nthreads = H) {
+    if constexpr (H == 128) return head_chain<H, PR, PA_MAX>(w2s, A, h2, out, out_ld, t);
     if (A == 1) head_rows<H, 1>(w2s, A, h2, out, out_ld, t, nthreads);
     else if (A <= 4) head_rows<H, 4>(w2s, A, h2, out, out_ld, t, nthreads);
     else head_rows<H, 8>(w2s, A, h2, out, out_ld, t, nthreads);

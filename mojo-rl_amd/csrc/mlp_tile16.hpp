@@ -205,9 +205,17 @@ MRL_DEV void head_rows16(const float *w2s, int A, const float *h2, float *out, i
 
 template <int H>
 MRL_DEV void head16(const float *w2s, int A, const float *h2, float *out, int out_ld, int t, int nthreads) {
+    if constexpr (H == 128) return head_chain<H, PR16, PA_MAX>(w2s, A, h2, out, out_ld, t);
     if (A == 1) head_rows16<H, 1, PA_MAX>(w2s, A, h2, out, out_ld, t, nthreads);
     else if (A <= 4) head_rows16<H, 4, PA_MAX>(w2s, A, h2, out, out_ld, t, nthreads);
     else head_rows16<H, 8, PA_MAX>(w2s, A, h2, out, out_ld, t, nthreads);
+}
+
+// the critic's head: weights as a plain column of H, then the bias
+template <int H>
+MRL_DEV void head16_value(const float *w2c, const float *h2, float *out, int t, int nthreads) {
+    if constexpr (H == 128) head_chain<H, PR16, 1>(w2c, 1, h2, out, 1, t);
+    else head_rows16<H, 1, 1>(w2c, 1, h2, out, 1, t, nthreads);
 }
 
 }  // namespace mrl

@@ -1,4 +1,4 @@
-// Fused kernels for the update path of three-layer nets  IN -> H -> H -> out  (H in {64, 256},
+// Fused kernels for the update path of three-layer nets  IN -> H -> H -> out  (H in {64, 128, 256},
 // IN <= 32, out <= 8 or a StochasticActor head of <= 8 actions): the shapes of every actor and
 // critic the PPO agents build (deep_agents/ppo/ppo.mojo:779-817, ppo_continuous.mojo:171-194).
 //
@@ -541,11 +541,11 @@ __global__ __launch_bounds__(2 * H) void mlp3_fb_kernel(int B, int IN, Mlp3Nets 
         if (t < A) db_part[2 * H + t] = cs2;
         else ls_part[(long)blockIdx.x * A + (t - A)] = cs2;
     }
-    if constexpr (H == 64) {
-        // Hidden width 64: the hidden layer's weight gradient of the tile, dW1[k][n] = sum_r h1[r][k] g1[r][n],
-        // is four 32 x 32 tiles of 16 k-steps.  It is taken here, from h1 and g1 while both lie in LDS, as one
-        // more per-tile piece for the sum kernel (wavefront w: columns [32w, 32w + 32)), instead of in a launch
-        // of its own that reads h1 and g1 back from global memory: that launch was 10 us of a 37 us minibatch.
+    if (fl.dw_in_tiles) {
+        // The hidden layer's weight gradient of the tile, dW1[k][n] = sum_r h1[r][k] g1[r][n], is (H / 32)^2
+        // 32 x 32 tiles of 16 k-steps.  It is taken here, from h1 and g1 while both lie in LDS, as one more
+        // per-tile piece for the sum kernel (wavefront w: columns [32w, 32w + 32)), instead of in a launch of its
+        // own that reads h1 and g1 back from global memory, where the launch is the larger part (dw_in_tiles_pays).
         __syncthreads();   // gT complete
         float *o1 = thin_part + (size_t)IN * H + (size_t)H * A;
 #pragma unroll
@@ -829,7 +829,7 @@ bool mlp3_fusable(const mrl_mlp_desc &d, int *H, int *act, bool *gauss) {
     const int k2 = d.layers[2].kind;
     if (k2 != MRL_LINEAR && k2 != MRL_STOCHASTIC_ACTOR) return false;
     const int h = d.layers[0].out_dim;
-    if ((h != 64 && h != 256) || d.layers[1].out_dim != h) return false;
+    if ((h != 64 && h != 128 && h != 256) || d.layers[1].out_dim != h) return false;
     if (d.layers[0].in_dim > PIN_MAX || d.layers[2].out_dim > PA_MAX) return false;
     *H = h;
     *act = k0 == MRL_LINEAR_RELU ? 1 : 2;
@@ -841,6 +841,13 @@ static int net_P(const mrl_mlp_desc &d) {
     const int IN = d.layers[0].in_dim, H = d.layers[0].out_dim, A = d.layers[2].out_dim;
     return (IN + 1) * H + (H + 1) * H + (H + 1) * A + (d.layers[2].kind == MRL_STOCHASTIC_ACTOR ? A : 0);
 }
+
+// Whether the fused forward + backward kernel takes the hidden layer's weight gradient of its row tile itself
+// (H^2 floats per tile and net, added up by the sum kernel) or leaves h1 and g1 to a launch of dw3_kernel.  Per
+// minibatch of 64 / 1024 / 4096 / 8192 rows (Walker2d's nets), in the tile against the launch: H = 128
+// 29.6 / 32.0 / 38.8 / 62.3 against 31.7 / 38.6 / 43.7 / 65.6 us; H = 256 53.8 / 63.0 / 72.1 / 131.8 against
+// 49.1 / 58.1 / 67.8 / 112.3 us.  (Beyond 8192 rows the pieces would be a workspace of more than 32 MB.)
+static bool dw_in_tiles_pays(int H, int tiles) { return H == 64 || (H == 128 && tiles <= 256); }
 
 // true when the two nets can share launches: both fusable, same input width, width and activation
 bool mlp3_pair_fusable(const mrl_mlp_desc &a, const mrl_mlp_desc &b) {
@@ -884,6 +891,8 @@ int mlp3_forward_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, i
     }
     if (H == 256 && act == 1) launch_fwd_t<256, 1>(ctx, batch, IN, io, n_nets, fl);
     else if (H == 256) launch_fwd_t<256, 2>(ctx, batch, IN, io, n_nets, fl);
+    else if (H == 128 && act == 1) launch_fwd_t<128, 1>(ctx, batch, IN, io, n_nets, fl);
+    else if (H == 128) launch_fwd_t<128, 2>(ctx, batch, IN, io, n_nets, fl);
     else if (act == 1) launch_fwd_t<64, 1>(ctx, batch, IN, io, n_nets, fl);
     else launch_fwd_t<64, 2>(ctx, batch, IN, io, n_nets, fl);
     MRL_CHECK_LAUNCH();
@@ -906,7 +915,7 @@ size_t mlp3_backward_ws(const mrl_mlp_desc *const *descs, int n_nets, int batch)
         const int IN = descs[i]->layers[0].in_dim, A = descs[i]->layers[2].out_dim;
         total += (size_t)2 * batch * H +
                  (size_t)((batch + PR - 1) / PR) * (2 * PA_MAX + 2 * H + (size_t)IN * H + (size_t)H * A +
-                                                    (H == 64 ? (size_t)H * H : 0));
+                                                    (dw_in_tiles_pays(H, (batch + PR - 1) / PR) ? (size_t)H * H : 0));
         P += net_P(*descs[i]);
     }
     return total + (size_t)32 * P;
@@ -933,7 +942,7 @@ int mlp3_backward_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, 
     int splits = std::max(1, std::min(32, batch / 256));
     int rows_per = ((batch + splits - 1) / splits + DKC - 1) / DKC * DKC;
     splits = (batch + rows_per - 1) / rows_per;
-    const bool hh_in_tiles = fused != nullptr && H == 64;
+    const bool hh_in_tiles = fused != nullptr && dw_in_tiles_pays(H, tiles);
     // workspace: per net g1 [B, H] | g0 [B, H] | ls_part [tiles, PA_MAX] | db_part [tiles, 2H + PA_MAX] |
     // thin_part [tiles, IN H + H A]; then partial [splits, Ptot]
     float *w = ws;
@@ -942,7 +951,7 @@ int mlp3_backward_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, 
         io.n[i].g0 = w; w += (size_t)batch * H;
         io.n[i].ls_part = w; w += (size_t)tiles * PA_MAX;
         io.n[i].db_part = w; w += (size_t)tiles * (2 * H + PA_MAX);
-        // (the fused forward + backward kernel of the 64-wide nets leaves the tile's dW1 there as well)
+        // (the fused forward + backward kernel may leave the tile's dW1 there as well)
         io.n[i].thin_stride = IN * H + H * descs[i]->layers[2].out_dim + (hh_in_tiles ? H * H : 0);
         io.n[i].thin_part = w; w += (size_t)tiles * (size_t)io.n[i].thin_stride;
     }
@@ -951,10 +960,13 @@ int mlp3_backward_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, 
     if (fused != nullptr) {
         fl = *fused;
         fl.enabled = 1;
+        fl.dw_in_tiles = hh_in_tiles ? 1 : 0;
         fused = &fl;
     }
     if (H == 256 && act == 1) launch_bwd_t<256, 1>(ctx, batch, IN, io, n_nets, fused);
     else if (H == 256) launch_bwd_t<256, 2>(ctx, batch, IN, io, n_nets, fused);
+    else if (H == 128 && act == 1) launch_bwd_t<128, 1>(ctx, batch, IN, io, n_nets, fused);
+    else if (H == 128) launch_bwd_t<128, 2>(ctx, batch, IN, io, n_nets, fused);
     else if (act == 1) launch_bwd_t<64, 1>(ctx, batch, IN, io, n_nets, fused);
     else launch_bwd_t<64, 2>(ctx, batch, IN, io, n_nets, fused);
     MRL_CHECK_LAUNCH();

@@ -26,7 +26,7 @@ namespace mrl {
 static_assert(SAMPLE_A_MAX == PA_MAX, "the sampler's action limit is the policy tile's");
 
 template <int H, int ACT, bool GAUSS, int TPW>
-__global__ __launch_bounds__(TPW == 1 ? 2 * H : 4 * H / TPW) void policy_kernel(
+__global__ __launch_bounds__(H == 256 && TPW == 1 ? 2 * H : 4 * H / TPW) void policy_kernel(
     const float *__restrict__ obs, int n, int IN, int A, const float *__restrict__ actor_p,
     const float *__restrict__ critic_p, uint32_t seed, float *__restrict__ actions,
     float *__restrict__ r_obs, float *__restrict__ r_actions, float *__restrict__ r_logp,
@@ -123,7 +123,7 @@ bool policy_fusable(const mrl_mlp_desc &a, const mrl_mlp_desc &c, bool gauss, in
     if (a.layers[2].kind != (gauss ? MRL_STOCHASTIC_ACTOR : MRL_LINEAR) || c.layers[2].kind != MRL_LINEAR)
         return false;
     const int h = a.layers[0].out_dim;
-    if (h != 64 && h != 256) return false;
+    if (h != 64 && h != 128 && h != 256) return false;
     if (a.layers[2].out_dim > PA_MAX || c.layers[2].out_dim != 1) return false;
     *H = h;
     *act = (k0 == MRL_LINEAR_RELU) ? 1 : 2;
@@ -143,8 +143,8 @@ int launch_policy(mrl_ctx *ctx, const mrl_mlp_desc &a, const mrl_mlp_desc &c, bo
     const bool split = 2 * tiles <= POLICY_SPLIT_BELOW;
     dim3 grid(tiles, split ? 2 : 1);
 #define MRL_LAUNCH(HH, AA, GG)                                                                         \
-    if (split && HH == 256)                                                                             \
-        hipLaunchKernelGGL((policy_kernel<HH, AA, GG, 1>), grid, dim3(2 * HH), 0, ctx->stream, obs,     \
+    if ((split && HH == 256) || HH == 128)                                                              \
+        hipLaunchKernelGGL((policy_kernel<HH, AA, GG, 1>), grid, dim3((split ? 2 : 4) * HH), 0, ctx->stream, obs, \
                            n, IN, A, ap, cp, seed, actions, r_obs, r_actions, r_logp, r_values);        \
     else                                                                                                \
         hipLaunchKernelGGL((policy_kernel<HH, AA, GG, PTPW>), grid, dim3((split ? 2 : 4) * HH / PTPW), 0, ctx->stream, obs, \
@@ -152,11 +152,15 @@ int launch_policy(mrl_ctx *ctx, const mrl_mlp_desc &a, const mrl_mlp_desc &c, bo
     if (gauss) {
         if (H == 256 && act == 1) MRL_LAUNCH(256, 1, true);
         else if (H == 256 && act == 2) MRL_LAUNCH(256, 2, true);
+        else if (H == 128 && act == 1) MRL_LAUNCH(128, 1, true);
+        else if (H == 128) MRL_LAUNCH(128, 2, true);
         else if (H == 64 && act == 1) MRL_LAUNCH(64, 1, true);
         else MRL_LAUNCH(64, 2, true);
     } else {
         if (H == 256 && act == 1) MRL_LAUNCH(256, 1, false);
         else if (H == 256 && act == 2) MRL_LAUNCH(256, 2, false);
+        else if (H == 128 && act == 1) MRL_LAUNCH(128, 1, false);
+        else if (H == 128) MRL_LAUNCH(128, 2, false);
         else if (H == 64 && act == 1) MRL_LAUNCH(64, 1, false);
         else MRL_LAUNCH(64, 2, false);
     }
