@@ -9,7 +9,10 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libmrl_hip.so")
-SOURCES = ["mrl_core.hip", "mrl_env.hip", "mrl_mlp.hip", "mrl_mlp3.hip", "mrl_ppo.hip", "mrl_policy.hip", "mrl_rollout.hip", "mrl_collect.hip", "mrl_collect_walkers.hip", "mrl_update.hip", "mrl_shuffle.hip"]
+SOURCES = ["mrl_core.hip", "mrl_env.hip", "mrl_mlp.hip", "mrl_mlp3.hip", "mrl_ppo.hip", "mrl_policy.hip", "mrl_rollout.hip", "mrl_collect.hip", "mrl_update.hip", "mrl_shuffle.hip"]
+# the 16-row collection kernels, a translation unit per hidden width
+COLLECT16 = ["mrl_collect%s_h%d.hip" % (k, h) for k in ("16", "_walkers") for h in (256, 128, 64)]
+SOURCES = COLLECT16 + SOURCES   # (the longest to compile go first)
 # -ffp-contract=off: fp32/fp64 results follow the written order of operations (the GEMM inner
 # loops spell out fmaf / MFMA themselves).  The -target-feature pair switches packed-fp32
 # code generation off.
@@ -20,8 +23,7 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=o
 # coefficients of exp / log / sincos, two registers each) out of the loop into registers of their own,
 # the register allocator then spills them, and every use becomes a dependent load from private memory in
 # the middle of the solver wavefront's chain.  Without that pass these kernels need no private memory.
-EXTRA_FLAGS = {"mrl_collect.hip": ["-mllvm", "-disable-machine-licm"],
-               "mrl_collect_walkers.hip": ["-mllvm", "-disable-machine-licm"]}
+EXTRA_FLAGS = {f: ["-mllvm", "-disable-machine-licm"] for f in ["mrl_collect.hip"] + COLLECT16}
 
 
 def _run(cmd, verbose):

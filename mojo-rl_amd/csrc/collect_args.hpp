@@ -18,8 +18,10 @@ struct CollectArgs {
     int car_trait_form;                   // CarRacingV2: reward / termination arithmetic of the GPU trait's step
 };
 
-// BipedalWalker / HalfCheetah with the agents' 256-wide Gaussian nets: true when `a` was launched
-bool collect_walker_fusable(const mrl_rollout *r, int *act);
-int launch_collect_walker(mrl_ctx *ctx, const mrl_rollout *r, const CollectArgs &a, int act);
+// entries of the kernels of collect_walkers.hpp and collect16.hpp (each hidden width in a translation unit of its own)
+template <int H, int ACT>
+int launch_collect_walker_t(mrl_ctx *ctx, const mrl_rollout *r, const CollectArgs &a);
+template <int H, int ACT>
+int launch_collect16_t(mrl_ctx *ctx, const mrl_rollout *r, const CollectArgs &a, int32_t *side);
 
 }  // namespace mrl

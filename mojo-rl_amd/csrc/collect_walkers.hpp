@@ -1,9 +1,9 @@
 // Fused collection kernels of the continuous-control envs beyond the classic ones (BipedalWalker,
-// HalfCheetah planar, CarRacingV2, HopperPlanar, Walker2dPlanar) with the agents' 256-wide Gaussian nets: many rollout steps of a
-// block's 16 envs in ONE launch, like the kernels of mrl_collect.hip.  The env rows (CarRacing: the 40
+// HalfCheetah planar, CarRacingV2, HopperPlanar, Walker2dPlanar) with the agents' Gaussian nets (hidden width H = 64, 128 or 256): many rollout
+// steps of a block's 16 envs in ONE launch, like the kernels of mrl_collect.hip.  The env rows (CarRacing: the 40
 // floats in front of the track) stay in LDS from the first step to the last; per step and block
-//   policy   the actor  OBS -> 256 -> 256 -> A  on wavefronts 0 .. 3 and the critic  OBS -> 256 -> 256 -> 1
-//            on four others, on the fp32 matrix cores (the 16-row tiles of mlp_tile16.hpp, 64 columns
+//   policy   the actor  OBS -> H -> H -> A  on wavefronts 0 .. 3 and the critic  OBS -> H -> H -> 1
+//            on four others, on the fp32 matrix cores (the 16-row tiles of mlp_tile16.hpp, H / 4 columns
 //            per wavefront, weights streamed from L2), heads out of LDS.  The walkers: only the actor runs
 //            ahead of the env step; the critic, whose value is only stored, runs beside the one-lane-per-
 //            body solver on wavefronts 2, 3, 6 and 7 (the two SIMDs that the solver's wavefronts 0 and 1
@@ -25,6 +25,7 @@
 // It gives what n_steps calls of mrl_rollout_step give (same per-env streams: seeds are affine in
 // the step number), except that the finished-episode list is appended in the order in which blocks
 // get there rather than step by step.
+#pragma once
 #include "mrl_host.hpp"
 #include "mrl_device.hpp"
 #include "mlp_tile.hpp"
@@ -51,18 +52,18 @@ constexpr int wmax() { return A > B ? A : B; }
 // Gaussian sampling on one lane per (env, action component) -- the log-probability is the sum of the
 // components' terms in component order --, rollout row t of action, log-prob and value.  Leaves the
 // actions in act[env][AW]; ends with the block in step (everything above complete).
-template <int IN, int AW, int ACT, class ObsAt>
+template <int H, int IN, int AW, int ACT, class ObsAt>
 MRL_DEV void policy16_gauss(const CollectArgs &a, ObsAt obs_at, int tid, int ne, int A, int zero, size_t row,
                             uint32_t sseed, int env0, float *xs, float *tiles, const float *w2a, const float *w2c,
                             float *logits, float *vals, float *act, float *part) {
-    constexpr int H = 256, R = PR16, T = 512, KBA = 8;
+    constexpr int R = PR16, T = 512, KBA = 8, NT = H / 64;
     const int wave = tid / WAVE, lane = tid % WAVE;
     const int net = wave >> 2;                           // 0: actor, 1: critic
     {
         const float *p = (net ? a.critic_p : a.actor_p) + zero;
         float *tile = tiles + net * (H * HT16_LD);
-        Hidden16Operands<H, IN, 4, KBA> ops;
-        ops.load(p, 64 * (wave & 3), lane);
+        Hidden16Operands<H, IN, NT, KBA> ops;
+        ops.load(p, 16 * NT * (wave & 3), lane);
         for (int i = tid; i < R * IN; i += T) {
             const int r = i / IN, c = i - r * IN;
             float v = 0.0f;
@@ -74,9 +75,9 @@ MRL_DEV void policy16_gauss(const CollectArgs &a, ObsAt obs_at, int tid, int ne,
         }
         __syncthreads();
         BlockSync bs;
-        hidden_stack16<H, IN, ACT, 4, KBA, true>(p, xs, tile, tile, ops, 64 * (wave & 3), lane, bs);
+        hidden_stack16<H, IN, ACT, NT, KBA, true>(p, xs, tile, tile, ops, 16 * NT * (wave & 3), lane, bs);
         if (net == 0) head16<H>(w2a, A, tile, logits, PA_MAX + 1, tid, T / 2);
-        else head_rows16<H, 1, 1>(w2c, 1, tile, vals, 1, tid - T / 2, T / 2);
+        else head16_value<H>(w2c, tile, vals, tid - T / 2, T / 2);
         __syncthreads();   // means and values complete; the tiles are dead from here on
     }
     for (int e = tid; e < ne * A; e += T) {
@@ -99,16 +100,16 @@ MRL_DEV void policy16_gauss(const CollectArgs &a, ObsAt obs_at, int tid, int ne,
 // The actor's half of policy16_gauss by wavefronts 0 .. 3 alone (the observation tile xs is complete, every
 // thread of the four passes its tid): hidden stack on `tile`, Gaussian sampling, rollout row t of action and
 // log-prob; leaves the actions in act[env][AW].  The four wavefronts meet at `sync`, five rounds per call.
-template <int IN, int AW, int ACT>
+template <int H, int IN, int AW, int ACT>
 MRL_DEV void actor16_gauss(const CollectArgs &a, int tid, int ne, int A, int zero, size_t row, uint32_t sseed, int env0,
                            const float *xs, float *tile, const float *w2a, float *logits, float *act, float *part,
                            WaveGroupSync &sync) {
-    constexpr int H = 256, KBA = 8, TA = 4 * WAVE;
+    constexpr int KBA = 8, TA = 4 * WAVE, NT = H / 64;
     const int wave = tid / WAVE, lane = tid % WAVE;
     const float *p = a.actor_p + zero;
-    Hidden16Operands<H, IN, 4, KBA> ops;
-    ops.load(p, 64 * wave, lane);
-    hidden_stack16<H, IN, ACT, 4, KBA, true>(p, xs, tile, tile, ops, 64 * wave, lane, sync);
+    Hidden16Operands<H, IN, NT, KBA> ops;
+    ops.load(p, 16 * NT * wave, lane);
+    hidden_stack16<H, IN, ACT, NT, KBA, true>(p, xs, tile, tile, ops, 16 * NT * wave, lane, sync);
     head16<H>(w2a, A, tile, logits, PA_MAX + 1, tid, TA);
     sync();   // means complete
     for (int e = tid; e < ne * A; e += TA) {
@@ -130,25 +131,25 @@ constexpr unsigned ACTOR16_ROUNDS = 5, CRITIC16_ROUNDS = 3;
 
 // The critic's half by wavefronts 2, 3, 6 and 7 (the two SIMDs that do not host wavefronts 0 and 1), on a
 // barrier of their own: values of the block's rows into vals.
-template <int IN, int ACT>
+template <int H, int IN, int ACT>
 MRL_DEV void critic16_side(const CollectArgs &a, int zero, int k, int tid, const float *xs, float *tile, const float *w2c,
                            float *vals, unsigned *sync_word, unsigned *failed) {
-    constexpr int H = 256, KBA = 8;
+    constexpr int KBA = 8, NT = H / 64;
     const int wave = tid / WAVE, lane = tid % WAVE;
     if (!(wave & 2)) return;
     const int g = (wave & 1) + ((wave >> 2) << 1);   // 0 .. 3
     const float *p = a.critic_p + zero;
     WaveGroupSync sync{sync_word, (unsigned)k * CRITIC16_ROUNDS * 4u, 4u, failed, a.spin_limit};
-    Hidden16Operands<H, IN, 4, KBA> ops;
-    ops.load(p, 64 * g, lane);
-    hidden_stack16<H, IN, ACT, 4, KBA, true>(p, xs, tile, tile, ops, 64 * g, lane, sync);
-    head_rows16<H, 1, 1>(w2c, 1, tile, vals, 1, g * WAVE + lane, 4 * WAVE);
+    Hidden16Operands<H, IN, NT, KBA> ops;
+    ops.load(p, 16 * NT * g, lane);
+    hidden_stack16<H, IN, ACT, NT, KBA, true>(p, xs, tile, tile, ops, 16 * NT * g, lane, sync);
+    head16_value<H>(w2c, tile, vals, g * WAVE + lane, 4 * WAVE);
 }
 
-template <class E, int ACT, bool LANES>
+template <class E, int H, int ACT, bool LANES>
 __global__ __launch_bounds__(512) void collect_walker_kernel(CollectArgs a) {
     using S = Stage<E>;
-    constexpr int H = 256, IN = E::OBS, AW = E::ACT_W, R = PR16, T = 512, KBA = 8;
+    constexpr int IN = E::OBS, AW = E::ACT_W, R = PR16, T = 512;
     static_assert(E::EPB == R && E::THREADS == T && IN <= PIN_MAX && AW <= PA_MAX, "16 envs per workgroup of eight wavefronts");
     __shared__ float rows[R * S::STRIDE];
     __shared__ float xs[R * XS_LD];
@@ -164,8 +165,10 @@ __global__ __launch_bounds__(512) void collect_walker_kernel(CollectArgs a) {
     // the two activation tiles and the env step's scratch (contact lists) are never live together
     constexpr int LIST_F = detect_list_floats<E>() + 1;
     constexpr int ENV_F = R * S::CSTRIDE + LIST_F + detect_count_ints<E>();
-    __shared__ float overlay[wmax<2 * H * HT16_LD, ENV_F>()];
-    static_assert(R * S::CSTRIDE <= H * HT16_LD, "the solver's contact scratch stays below the critic's tile");
+    // the critic's tile: above the actor's and above the solver's contact scratch, below the merged counts
+    constexpr int CRITIC_OFF = wmax<H * HT16_LD, R * S::CSTRIDE>();
+    __shared__ float overlay[wmax<CRITIC_OFF + H * HT16_LD, ENV_F>()];
+    static_assert(LANES || CRITIC_OFF + H * HT16_LD <= R * S::CSTRIDE + LIST_F, "the critic's tile lies over spent contact lists only");
     float *cts = overlay, *dlist = cts + R * S::CSTRIDE;
     int *dcount = reinterpret_cast<int *>(dlist + LIST_F);
 
@@ -212,9 +215,9 @@ __global__ __launch_bounds__(512) void collect_walker_kernel(CollectArgs a) {
         __syncthreads();
         if (wave < 4) {
             WaveGroupSync actor_sync{&sync_actor, (unsigned)k * ACTOR16_ROUNDS * 4u, 4u, &sync_failed, a.spin_limit};
-            actor16_gauss<IN, AW, ACT>(a, tid, ne, A, zero, row, sseed, env0, xs, overlay, w2a, logits, act, part, actor_sync);
+            actor16_gauss<H, IN, AW, ACT>(a, tid, ne, A, zero, row, sseed, env0, xs, overlay, w2a, logits, act, part, actor_sync);
         }
-        float *critic_tile = overlay + H * HT16_LD;   // (above the env step's contact scratch cts)
+        float *critic_tile = overlay + CRITIC_OFF;   // (above the env step's contact scratch cts)
         // ---- env step with auto-reset, reward / done into rollout row t, episode accounting
         Accounting acc = a.acc;
         acc.r_rewards = a.r_rewards + (size_t)(a.t0 + k) * N;
@@ -223,7 +226,7 @@ __global__ __launch_bounds__(512) void collect_walker_kernel(CollectArgs a) {
         if constexpr (!LANES) {
             // (the critic's tile lies over contact lists that are spent by the time the solver runs)
             auto side = [&](int th) {
-                critic16_side<IN, ACT>(a, zero, k, th, xs, critic_tile, w2c, vals, &sync_critic, &sync_failed);
+                critic16_side<H, IN, ACT>(a, zero, k, th, xs, critic_tile, w2c, vals, &sync_critic, &sync_failed);
             };
             phys_step_block<E, true>(rows, cts, shapes, dlist, dcount, &was_reset, act, nullptr, nullptr, env0, ne,
                                      rseed, acc, tid, side);
@@ -245,7 +248,7 @@ __global__ __launch_bounds__(512) void collect_walker_kernel(CollectArgs a) {
                     if (d > 0.5f) E::reset(rowp, rseed, env);
                 }
             } else {
-                critic16_side<IN, ACT>(a, zero, k, tid, xs, critic_tile, w2c, vals, &sync_critic, &sync_failed);
+                critic16_side<H, IN, ACT>(a, zero, k, tid, xs, critic_tile, w2c, vals, &sync_critic, &sync_failed);
             }
         }
         __syncthreads();   // env step done: the rows hold the next observation
@@ -272,9 +275,9 @@ __global__ __launch_bounds__(512) void collect_walker_kernel(CollectArgs a) {
 // over the whole launch.  Env step: a wavefront per env in two rounds of eight; each wavefront stages its
 // env's tile table through LDS (over the activation tiles, which are dead by then), steps, accounts, and
 // rebuilds the env when it finished (one lane walks the new track: only this block waits for it).
-template <int ACT>
+template <int H, int ACT>
 __global__ __launch_bounds__(512) void collect_car_kernel(CollectArgs a) {
-    constexpr int H = 256, IN = cr::OBS, AW = cr::ACT, R = PR16, T = 512, HEAD = cr::TRACK;
+    constexpr int IN = cr::OBS, AW = cr::ACT, R = PR16, T = 512, HEAD = cr::TRACK;
     static_assert(IN <= PIN_MAX && AW <= PA_MAX && cr::TABLE % 4 == 0, "tile limits");
     __shared__ float heads[R * (HEAD + 1)];
     __shared__ float xs[R * XS_LD];
@@ -305,7 +308,7 @@ __global__ __launch_bounds__(512) void collect_car_kernel(CollectArgs a) {
         const uint32_t sseed = a.sample_seed + (uint32_t)k * a.sample_stride;
         const uint64_t rseed = a.reset_seed + (uint64_t)k * a.reset_stride;
         const int wave = tid / WAVE, sub = tid % WAVE;
-        policy16_gauss<IN, AW, ACT>(a, [&](int r, int c) { return heads[r * (HEAD + 1) + c]; }, tid, ne, A, zero, row, sseed,
+        policy16_gauss<H, IN, AW, ACT>(a, [&](int r, int c) { return heads[r * (HEAD + 1) + c]; }, tid, ne, A, zero, row, sseed,
                                     env0, xs, overlay, w2a, w2c, logits, vals, act, part);
         Accounting acc = a.acc;
         acc.r_rewards = a.r_rewards + (size_t)(a.t0 + k) * N;
@@ -357,9 +360,9 @@ __global__ __launch_bounds__(512) void collect_car_kernel(CollectArgs a) {
 // observation) stay in LDS over the whole launch; the actor runs on wavefronts 0 .. 3, then lanes 0 .. 15 of
 // wavefront 0 step one env each (Float64, state in registers for the four sub-steps), account and rebuild
 // finished rows in place, while the critic runs beside them on wavefronts 2, 3, 6 and 7.
-template <class M, int ACT>
+template <class M, int H, int ACT>
 __global__ __launch_bounds__(512) void collect_planar_kernel(CollectArgs a) {
-    constexpr int H = 256, IN = M::OBS, AW = M::ACT, R = PR16, T = 512;
+    constexpr int IN = M::OBS, AW = M::ACT, R = PR16, T = 512;
     static_assert(IN <= PIN_MAX && AW <= PA_MAX && M::STATE % 2 == 0, "tile limits; rows are whole doubles");
     __shared__ __align__(16) float rows[R * M::STATE];
     __shared__ float xs[R * XS_LD];
@@ -408,7 +411,7 @@ __global__ __launch_bounds__(512) void collect_planar_kernel(CollectArgs a) {
         __syncthreads();
         if (wave < 4) {
             WaveGroupSync actor_sync{&sync_actor, (unsigned)k * ACTOR16_ROUNDS * 4u, 4u, &sync_failed, a.spin_limit};
-            actor16_gauss<IN, AW, ACT>(a, tid, ne, A, zero, row, sseed, env0, xs, tiles, w2a, logits, act, part, actor_sync);
+            actor16_gauss<H, IN, AW, ACT>(a, tid, ne, A, zero, row, sseed, env0, xs, tiles, w2a, logits, act, part, actor_sync);
         }
         if (wave == 0) {
             if (lane < ne) {
@@ -426,7 +429,7 @@ __global__ __launch_bounds__(512) void collect_planar_kernel(CollectArgs a) {
                 s.store(rowp);
             }
         } else {
-            critic16_side<IN, ACT>(a, zero, k, tid, xs, tiles + H * HT16_LD, w2c, vals, &sync_critic, &sync_failed);
+            critic16_side<H, IN, ACT>(a, zero, k, tid, xs, tiles + H * HT16_LD, w2c, vals, &sync_critic, &sync_failed);
         }
         __syncthreads();   // env step done: the rows hold the next observation
         if (tid < ne) a.r_values[row + tid] = vals[tid];
@@ -444,54 +447,22 @@ __global__ __launch_bounds__(512) void collect_planar_kernel(CollectArgs a) {
     for (int i = t; i < nenv * (M::STATE / 2); i += T) g2[i] = l2[i];
 }
 
-bool collect_walker_fusable(const mrl_rollout *r, int *act) {
-    if (r->num_actions != 0) return false;
-    int obs, aw;
-    if (r->env_id == MRL_ENV_BIPEDAL) { obs = BipedalWalker::OBS; aw = BipedalWalker::ACT_W; }
-    else if (r->env_id == MRL_ENV_HALFCHEETAH) { obs = HalfCheetah::OBS; aw = HalfCheetah::ACT_W; }
-    else if (r->env_id == MRL_ENV_CARRACING) { obs = cr::OBS; aw = cr::ACT; }
-    else if (r->env_id == MRL_ENV_HOPPER_PLANAR) { obs = planar::Hopper::OBS; aw = planar::Hopper::ACT; }
-    else if (r->env_id == MRL_ENV_WALKER2D_PLANAR) { obs = planar::Walker2d::OBS; aw = planar::Walker2d::ACT; }
-    else return false;
-    // (the planar rows hold doubles)
-    if (r->env_id >= MRL_ENV_HOPPER_PLANAR && reinterpret_cast<uintptr_t>(r->states) % 8 != 0) return false;
-    const mrl_mlp_desc &a = r->actor, &c = r->critic;
-    if (a.n_layers != 3 || c.n_layers != 3) return false;
-    const int k0 = a.layers[0].kind;
-    if (k0 != MRL_LINEAR_RELU && k0 != MRL_LINEAR_TANH) return false;
-    for (const mrl_mlp_desc *d : {&a, &c}) {
-        if (d->layers[0].kind != k0 || d->layers[1].kind != k0) return false;
-        if (d->layers[0].in_dim != obs || d->layers[0].out_dim != 256 || d->layers[1].out_dim != 256) return false;
-    }
-    if (a.layers[2].kind != MRL_STOCHASTIC_ACTOR || a.layers[2].out_dim != aw) return false;
-    if (c.layers[2].kind != MRL_LINEAR || c.layers[2].out_dim != 1) return false;
-    // 16-byte loads of the weight rows
-    if (reinterpret_cast<uintptr_t>(r->actor_params) % 16 != 0 || reinterpret_cast<uintptr_t>(r->critic_params) % 16 != 0)
-        return false;
-    *act = (k0 == MRL_LINEAR_RELU) ? 1 : 2;
-    return true;
-}
-
-int launch_collect_walker(mrl_ctx *ctx, const mrl_rollout *r, const CollectArgs &args, int act) {
+template <int H, int ACT>
+int launch_collect_walker_t(mrl_ctx *ctx, const mrl_rollout *r, const CollectArgs &args) {
     CollectArgs a = args;
     const dim3 grid(grid_for(r->n_envs, PR16)), block(512);
     if (r->env_id == MRL_ENV_BIPEDAL) {
         a.shapes = ctx->bw_shapes;
-        if (act == 1) hipLaunchKernelGGL((collect_walker_kernel<BipedalWalker, 1, false>), grid, block, 0, ctx->stream, a);
-        else hipLaunchKernelGGL((collect_walker_kernel<BipedalWalker, 2, false>), grid, block, 0, ctx->stream, a);
+        hipLaunchKernelGGL((collect_walker_kernel<BipedalWalker, H, ACT, false>), grid, block, 0, ctx->stream, a);
     } else if (r->env_id == MRL_ENV_CARRACING) {
-        if (act == 1) hipLaunchKernelGGL((collect_car_kernel<1>), grid, block, 0, ctx->stream, a);
-        else hipLaunchKernelGGL((collect_car_kernel<2>), grid, block, 0, ctx->stream, a);
+        hipLaunchKernelGGL((collect_car_kernel<H, ACT>), grid, block, 0, ctx->stream, a);
     } else if (r->env_id == MRL_ENV_HOPPER_PLANAR) {
-        if (act == 1) hipLaunchKernelGGL((collect_planar_kernel<planar::Hopper, 1>), grid, block, 0, ctx->stream, a);
-        else hipLaunchKernelGGL((collect_planar_kernel<planar::Hopper, 2>), grid, block, 0, ctx->stream, a);
+        hipLaunchKernelGGL((collect_planar_kernel<planar::Hopper, H, ACT>), grid, block, 0, ctx->stream, a);
     } else if (r->env_id == MRL_ENV_WALKER2D_PLANAR) {
-        if (act == 1) hipLaunchKernelGGL((collect_planar_kernel<planar::Walker2d, 1>), grid, block, 0, ctx->stream, a);
-        else hipLaunchKernelGGL((collect_planar_kernel<planar::Walker2d, 2>), grid, block, 0, ctx->stream, a);
+        hipLaunchKernelGGL((collect_planar_kernel<planar::Walker2d, H, ACT>), grid, block, 0, ctx->stream, a);
     } else {
         a.shapes = ctx->hc_shapes;
-        if (act == 1) hipLaunchKernelGGL((collect_walker_kernel<HalfCheetah16, 1, true>), grid, block, 0, ctx->stream, a);
-        else hipLaunchKernelGGL((collect_walker_kernel<HalfCheetah16, 2, true>), grid, block, 0, ctx->stream, a);
+        hipLaunchKernelGGL((collect_walker_kernel<HalfCheetah16, H, ACT, true>), grid, block, 0, ctx->stream, a);
     }
     MRL_CHECK_LAUNCH();
     return MRL_OK;

@@ -79,6 +79,86 @@ struct Hidden16Operands {
     }
 };
 
+// Layer 0 of a tile: xs[16][XS_LD] holds the inputs, hT [H][HT16_LD] receives act(layer 0) k-major.
+template <int H, int IN, int ACT, int NT, int KB>
+MRL_DEV void hidden16_layer0(const float *xs, float *hT, const Hidden16Operands<H, IN, NT, KB> &ops, int c0, int lane) {
+    constexpr int K0 = (IN + 3) / 4;
+    const int g = lane >> 4, n = lane & 15;
+    float a0[K0];
+#pragma unroll
+    for (int kk = 0; kk < K0; ++kk) {
+        const int k = 4 * kk + g;
+        a0[kk] = k < IN ? xs[n * XS_LD + k] : 0.0f;
+    }
+    floatx4 c[NT];
+#pragma unroll
+    for (int q = 0; q < NT; ++q) c[q] = floatx4{0};
+#pragma unroll
+    for (int kk = 0; kk < K0; ++kk) {
+#pragma unroll
+        for (int q = 0; q < NT; ++q)
+            c[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0[kk], ops.w0[kk][q], c[q], 0, 0, 0);
+    }
+#pragma unroll
+    for (int q = 0; q < NT; ++q) {
+        const int col = tile16_col<NT>(c0, q, n);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) hT[col * HT16_LD + 4 * g + v] = activate<ACT>(c[q][v] + ops.bias0[q]);
+    }
+}
+
+// Layer 1: weights streamed from L2 one block of KB k-steps ahead of the MFMAs (KB = H / 4: all of them are in
+// `ops`, which is then left as it is); h2 [16][H + 1] receives act(layer 1) row-major.  before_h2() is called between
+// the last read of hT and the first write of h2.
+template <int H, int IN, int ACT, int NT, int KB, class Before>
+MRL_DEV void hidden16_layer1(const float *__restrict__ p, const float *hT, float *h2, Hidden16Operands<H, IN, NT, KB> &ops,
+                             int c0, int lane, Before &&before_h2) {
+    static_assert((H / 4) % KB == 0, "whole blocks of k-steps");
+    const int g = lane >> 4, n = lane & 15;
+    const float *W1 = p + IN * H + H;
+    floatx4 c[NT];
+#pragma unroll
+    for (int q = 0; q < NT; ++q) c[q] = floatx4{0};
+    float a[KB], na[KB], nb[KB][NT];
+#pragma unroll
+    for (int j = 0; j < KB; ++j) a[j] = hT[(4 * j + g) * HT16_LD + n];
+    constexpr int NBLK = H / (4 * KB);
+    for (int blk = 0; blk < NBLK; ++blk) {
+        const bool more = blk + 1 < NBLK;
+        if (more) {
+#pragma unroll
+            for (int j = 0; j < KB; ++j) {
+                const int k = 4 * ((blk + 1) * KB + j) + g;
+                na[j] = hT[k * HT16_LD + n];
+                tile16_load_b<NT>(W1 + k * H + c0, n, nb[j]);
+            }
+        }
+        // keep the next block's loads ahead of this block's MFMAs
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < KB; ++j) {
+#pragma unroll
+            for (int q = 0; q < NT; ++q)
+                c[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], ops.bv[j][q], c[q], 0, 0, 0);
+        }
+        if (more) {
+#pragma unroll
+            for (int j = 0; j < KB; ++j) {
+                a[j] = na[j];
+#pragma unroll
+                for (int q = 0; q < NT; ++q) ops.bv[j][q] = nb[j][q];
+            }
+        }
+    }
+    before_h2();
+#pragma unroll
+    for (int q = 0; q < NT; ++q) {
+        const int col = tile16_col<NT>(c0, q, n);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) h2[(4 * g + v) * (H + 1) + col] = activate<ACT>(c[q][v] + ops.bias1[q]);
+    }
+}
+
 // Hidden stack of one net for the block's 16 rows on the wavefronts that share it (each with its
 // own c0 / NT; `lane` = lane of the calling wavefront).  xs[16][XS_LD] holds the inputs, hT
 // [H][HT16_LD] receives act(layer 0) k-major, h2 [16][H + 1] act(layer 1) row-major; h2 may share
@@ -88,77 +168,9 @@ template <int H, int IN, int ACT, int NT, int KB, bool H2_ON_HT, class Sync>
 MRL_DEV void hidden_stack16(const float *__restrict__ p, const float *xs, float *hT, float *h2,
                             Hidden16Operands<H, IN, NT, KB> &ops, int c0, int lane, Sync &sync) {
     static_assert(PR16 * (H + 1) <= H * HT16_LD, "h2 fits into hT");
-    static_assert((H / 4) % KB == 0, "whole blocks of k-steps");
-    constexpr int K0 = (IN + 3) / 4;
-    const int g = lane >> 4, n = lane & 15;
-    const float *W1 = p + IN * H + H;
-    {   // layer 0
-        float a0[K0];
-#pragma unroll
-        for (int kk = 0; kk < K0; ++kk) {
-            const int k = 4 * kk + g;
-            a0[kk] = k < IN ? xs[n * XS_LD + k] : 0.0f;
-        }
-        floatx4 c[NT];
-#pragma unroll
-        for (int q = 0; q < NT; ++q) c[q] = floatx4{0};
-#pragma unroll
-        for (int kk = 0; kk < K0; ++kk) {
-#pragma unroll
-            for (int q = 0; q < NT; ++q)
-                c[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0[kk], ops.w0[kk][q], c[q], 0, 0, 0);
-        }
-#pragma unroll
-        for (int q = 0; q < NT; ++q) {
-            const int col = tile16_col<NT>(c0, q, n);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) hT[col * HT16_LD + 4 * g + v] = activate<ACT>(c[q][v] + ops.bias0[q]);
-        }
-    }
+    hidden16_layer0<H, IN, ACT, NT, KB>(xs, hT, ops, c0, lane);
     sync();
-    {   // layer 1: weights streamed from L2 one block of KB k-steps ahead of the MFMAs
-        floatx4 c[NT];
-#pragma unroll
-        for (int q = 0; q < NT; ++q) c[q] = floatx4{0};
-        float a[KB], na[KB], nb[KB][NT];
-#pragma unroll
-        for (int j = 0; j < KB; ++j) a[j] = hT[(4 * j + g) * HT16_LD + n];
-        constexpr int NBLK = H / (4 * KB);
-        for (int blk = 0; blk < NBLK; ++blk) {
-            const bool more = blk + 1 < NBLK;
-            if (more) {
-#pragma unroll
-                for (int j = 0; j < KB; ++j) {
-                    const int k = 4 * ((blk + 1) * KB + j) + g;
-                    na[j] = hT[k * HT16_LD + n];
-                    tile16_load_b<NT>(W1 + k * H + c0, n, nb[j]);
-                }
-            }
-            // keep the next block's loads ahead of this block's MFMAs
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int j = 0; j < KB; ++j) {
-#pragma unroll
-                for (int q = 0; q < NT; ++q)
-                    c[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], ops.bv[j][q], c[q], 0, 0, 0);
-            }
-            if (more) {
-#pragma unroll
-                for (int j = 0; j < KB; ++j) {
-                    a[j] = na[j];
-#pragma unroll
-                    for (int q = 0; q < NT; ++q) ops.bv[j][q] = nb[j][q];
-                }
-            }
-        }
-        if (H2_ON_HT) sync();
-#pragma unroll
-        for (int q = 0; q < NT; ++q) {
-            const int col = tile16_col<NT>(c0, q, n);
-#pragma unroll
-            for (int v = 0; v < 4; ++v) h2[(4 * g + v) * (H + 1) + col] = activate<ACT>(c[q][v] + ops.bias1[q]);
-        }
-    }
+    hidden16_layer1<H, IN, ACT, NT, KB>(p, hT, h2, ops, c0, lane, [&]() { if (H2_ON_HT) sync(); });
     sync();
 }
 

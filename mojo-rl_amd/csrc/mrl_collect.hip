@@ -25,17 +25,20 @@
 #include "mrl_host.hpp"
 #include "mrl_device.hpp"
 #include "mlp_tile.hpp"
-#include "mlp_tile16.hpp"
 #include "policy_sample.hpp"
-#include "env_block.hpp"
-#include "env_classic.hpp"
-#include "collect_args.hpp"
+#include "env_car.hpp"
+#include "env_planar.hpp"
+#include "collect16.hpp"
 
 namespace mrl {
 
-
-template <int A, int B>
-constexpr int cmax() { return A > B ? A : B; }
+// compiled in mrl_collect16_h*.hip
+extern template int launch_collect16_t<64, 1>(mrl_ctx *, const mrl_rollout *, const CollectArgs &, int32_t *);
+extern template int launch_collect16_t<64, 2>(mrl_ctx *, const mrl_rollout *, const CollectArgs &, int32_t *);
+extern template int launch_collect16_t<128, 1>(mrl_ctx *, const mrl_rollout *, const CollectArgs &, int32_t *);
+extern template int launch_collect16_t<128, 2>(mrl_ctx *, const mrl_rollout *, const CollectArgs &, int32_t *);
+extern template int launch_collect16_t<256, 1>(mrl_ctx *, const mrl_rollout *, const CollectArgs &, int32_t *);
+extern template int launch_collect16_t<256, 2>(mrl_ctx *, const mrl_rollout *, const CollectArgs &, int32_t *);
 
 template <class E, int H, int ACT, bool GAUSS>
 __global__ __launch_bounds__(E::THREADS) void collect_kernel(CollectArgs a) {
@@ -231,200 +234,6 @@ __global__ __launch_bounds__(E::THREADS) void collect_kernel(CollectArgs a) {
     S::out(rows, gbase, nenv, t, 0, E::STATE);
 }
 
-// ---------------------------------------------------------------- 16 rows per workgroup
-// The same step for a workgroup of four wavefronts and 16 envs, for launches with at most 16 envs
-// per CU.  A step is a chain -- actor on the matrix cores, then sampling and the env step on ONE
-// wavefront's vector unit -- and the env step costs the same whether 16 or 32 lanes carry an env,
-// while the actor of 16 rows takes half the matrix time of 32 (v_mfma_f32_16x16x4_f32, same bits as
-// the 32-row tiles): few envs are stepped faster spread 16 to a CU than packed 32 to half the CUs.
-//   all four wavefronts     actor  OBS -> H -> H -> A, 64 columns each;
-//   the solver wavefront    sampling, env step (one env per lane 0 .. 15), accounting, resets;
-//   the other three         contact detection, then the critic (80 / 96 / 80 columns) at a barrier
-//                           of their own.
-// Two such workgroups fit a CU (LDS, registers), but running them side by side does not pay: on this
-// hardware a SIMD issues either a matrix or a vector instruction, never both at once (a wavefront of
-// dependent v_fma_f32 that shares its SIMD with a wavefront issuing v_mfma back to back takes the sum
-// of both times), so one workgroup's env step does not hide behind the other's forward passes, and
-// two solver wavefronts of 16 envs cost twice the vector time of one with 32.  With more than 16 envs
-// per CU the 32-row kernel above is the faster one (8192 envs: 38.6 against 39.8 us per step).
-// The solver wavefront is 0 in the lower half of the grid and 2 in the upper half: workgroups i and
-// i + grid / 2 share a CU when the grid is twice the CU count, and their solvers then sit on
-// different SIMDs.
-template <class EB, int ACT, bool GAUSS>
-__global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
-    using E = Rows16<EB>;
-    using S = Stage<E>;
-    constexpr int H = 256, IN = E::OBS, AW = E::ACT_W, R = PR16, T = E::THREADS;
-    constexpr int CAP = 3;      // records per (body, vertex) list: two contacts, the third signals overflow
-    constexpr int KBA = 8;      // k-steps of layer-1 weights fetched ahead
-    static_assert(IN <= PIN_MAX && AW <= PA_MAX && E::DETECT_TASKS > 0 && E::DETECT_TASKS <= 24, "tile limits; split-off detection");
-    __shared__ float rows[R * S::STRIDE];
-    __shared__ float xs[R * XS_LD];
-    __shared__ __align__(16) float w2a[HEAD_LDS(H)];
-    __shared__ float w2c[H + 1];                    // the critic's head: column of H weights, then the bias
-    __shared__ float logits[R * (PA_MAX + 1)];
-    __shared__ float vals[R];
-    __shared__ float act[R * PA_MAX];
-    __shared__ float shapes[E::NSHAPE];
-    __shared__ unsigned long long was_reset;
-    __shared__ unsigned sync_critic, sync_detect, sync_failed;
-    __shared__ float hTc[H * HT16_LD];              // the critic's activation tile (live during the env step)
-    // the actor's activation tile and the env step's contact scratch are never live together
-    constexpr int LIST_F = detect_list_floats<E, CAP>() + 1;
-    constexpr int ENV_F = R * S::CSTRIDE + LIST_F + detect_count_ints<E>();
-    __shared__ float overlay[cmax<H * HT16_LD, ENV_F>()];
-    float *cts = overlay, *dlist = cts + R * S::CSTRIDE;
-    int *dcount = reinterpret_cast<int *>(dlist + LIST_F);
-
-    const int t = threadIdx.x;
-    const int env0 = blockIdx.x * R;
-    const int nenv = min(R, a.n_envs - env0);
-    const int N = a.n_envs;
-    const int sw = (2 * blockIdx.x >= gridDim.x && gridDim.x > 1) ? 2 : 0;   // the solver wavefront
-    float *gbase = a.states + (size_t)env0 * E::STATE;
-
-    S::in(rows, gbase, nenv, t);
-    for (int i = t; i < E::NSHAPE; i += T) shapes[i] = a.shapes[i];
-    stage_head(a.actor_p + IN * H + H + H * H + H, H, a.A, GAUSS, w2a, t, T);
-    for (int i = t; i < H + 1; i += T) w2c[i] = a.critic_p[IN * H + H + H * H + H + i];
-    if (t == 0) {
-        was_reset = 0;
-        sync_critic = 0;
-        sync_detect = 0;
-        sync_failed = 0;
-    }
-    __syncthreads();
-    // solver wavefront, lane = env slot: the env's running episode return and length stay in registers
-    const bool owner = (t >> 6) == sw && (t & 63) < nenv;
-    float ep_return = owner ? a.acc.ep_return[env0 + (t & 63)] : 0.0f;
-    float ep_length = owner ? a.acc.ep_length[env0 + (t & 63)] : 0.0f;
-
-    for (int k = 0; k < a.n_steps; ++k) {
-        // Nothing but the rows is carried from one step to the next: the thread index, the block's
-        // env count and the parameter pointers pass through empty asm statements at the top of each
-        // step, so the optimiser cannot keep what it derives from them live through the env step,
-        // whose solver needs the registers.
-        int tid = t, ne = __builtin_amdgcn_readfirstlane(nenv), A = __builtin_amdgcn_readfirstlane(a.A), zero = 0;
-        asm volatile("" : "+v"(tid), "+s"(zero), "+s"(ne), "+s"(A) : : "memory");
-        const float *pa = a.actor_p + zero, *pc = a.critic_p + zero;
-        const size_t row = (size_t)(a.t0 + k) * N + env0;   // this block's slice of rollout row t
-        const uint32_t sseed = a.sample_seed + (uint32_t)k * a.sample_stride;
-        const int wave = tid / WAVE, lane = tid % WAVE;
-        const int vw = (wave - sw) & 3;                     // 0: solver, 1 .. 3: helpers
-        // the helpers' barriers, rebuilt every step from the step number (the critic's hidden stack meets
-        // three times per step, the detection once): nothing of them stays in registers through the env step
-        WaveGroupSync critic_sync{&sync_critic, (unsigned)k * 9u, 3u, &sync_failed, a.spin_limit};
-        WaveGroupSync detect_sync{&sync_detect, (unsigned)k * 3u, 3u, &sync_failed, a.spin_limit};
-        // ---- actor, all wavefronts
-        {
-            Hidden16Operands<H, IN, 4, KBA> ops;
-            ops.load(pa, 64 * wave, lane);
-            for (int i = tid; i < R * IN; i += T) {
-                const int r = i / IN, c = i - r * IN;
-                float v = 0.0f;
-                if (r < ne) {
-                    v = rows[r * S::STRIDE + c];
-                    a.r_obs[row * IN + i] = v;
-                }
-                xs[r * XS_LD + c] = v;
-            }
-            __syncthreads();
-            BlockSync bs;
-            hidden_stack16<H, IN, ACT, 4, KBA, true>(pa, xs, overlay, overlay, ops, 64 * wave, lane, bs);
-            head16<H>(w2a, A, overlay, logits, PA_MAX + 1, tid, T);
-            __syncthreads();   // logits complete; the actor's tile is dead from here on
-        }
-        if (vw == 0) {
-            // ---- sample, then the env step of env_block.hpp with the contacts the helpers detect
-            typename E::Carry carry{};
-            if (lane < ne) {
-                const int i = env0 + lane;
-                float logp;
-                if (GAUSS) {
-                    float av[PA_MAX];
-                    logp = sample_gaussian(logits + lane * (PA_MAX + 1), w2a + HEAD_LOG_STD(H), A, sseed, i, av);
-                    for (int j = 0; j < A; ++j) {
-                        act[lane * AW + j] = av[j];
-                        a.r_actions[(row + lane) * AW + j] = av[j];
-                    }
-                } else {
-                    int sel;
-                    sample_categorical_few(logits + lane * (PA_MAX + 1), A, sseed, i, sel, logp);
-                    act[lane] = (float)sel;
-                    a.r_actions[row + lane] = (float)sel;
-                }
-                a.r_logp[row + lane] = logp;
-                carry = E::step_begin(rows + lane * S::STRIDE, i, act + lane * AW, shapes);
-            }
-            detect_sync.target += detect_sync.nwaves;
-            detect_sync.wait_for(detect_sync.target);
-            bool finished = false;
-            if (lane < ne) {
-                float *mine = cts + lane * S::CSTRIDE;
-                const int n = merge_vertex_lists<E, CAP>(dlist, dcount, lane, mine);
-                float r, d;
-                E::step_finish(rows + lane * S::STRIDE, mine, n, shapes, carry, r, d);
-                a.r_rewards[row + lane] = r;
-                a.r_dones[row + lane] = d;
-                ep_return = ep_return + r;
-                ep_length = ep_length + 1.0f;
-                finished = d > 0.5f;
-                if (finished) {
-                    const int slot = atomicAdd(a.acc.done_count, 1);
-                    if (slot < a.acc.done_cap) {
-                        a.acc.done_returns[slot] = ep_return;
-                        a.acc.done_lengths[slot] = ep_length;
-                    }
-                    ep_return = 0.0f;
-                    ep_length = 0.0f;
-                }
-            }
-            reset_rows<E>(rows, &was_reset, __ballot(finished), a.reset_seed + (uint64_t)k * a.reset_stride, env0, lane);
-        } else {
-            // ---- contact detection: (body, vertex) task m * 4 + lane / 16 of env slot lane % 16, a
-            // second pass on helper 0 for the tasks beyond twelve
-            const int m = vw - 1, e = lane % R;
-            if (e < ne)
-                for (int task = m * 4 + lane / R; task < E::DETECT_TASKS; task += 12)
-                    detect_vertex_task<E, CAP>(rows, shapes, dlist, dcount, task, e);
-            detect_sync.arrive();
-            // ---- critic on the three helpers, at their own barrier: helper 1 takes six column
-            // tiles, helpers 0 (which had the second detection pass) and 2 five each
-            const int tl = m * WAVE + lane;
-            if (m == 1) {
-                Hidden16Operands<H, IN, 6, KBA> ops;
-                ops.load(pc, 80, lane);
-                hidden_stack16<H, IN, ACT, 6, KBA, true>(pc, xs, hTc, hTc, ops, 80, lane, critic_sync);
-            } else {
-                const int c0 = m == 0 ? 0 : 176;
-                Hidden16Operands<H, IN, 5, KBA> ops;
-                ops.load(pc, c0, lane);
-                hidden_stack16<H, IN, ACT, 5, KBA, true>(pc, xs, hTc, hTc, ops, c0, lane, critic_sync);
-            }
-            head_rows16<H, 1, 1>(w2c, 1, hTc, vals, 1, tl, 3 * WAVE);
-        }
-        __syncthreads();   // env step done, values complete
-        if (tid < ne) a.r_values[row + tid] = vals[tid];
-        // a wait that gave up: the block's results are void from here on; leave the loop (every
-        // thread reads the same word after the barrier) and end normally
-        if (sync_failed != 0u) break;
-    }
-    if (sync_failed != 0u) {   // as in collect_kernel: nothing of a block whose wait gave up is stored
-        if (t == 0) *a.sync_error = 1;
-        return;
-    }
-
-    if (owner) {
-        a.acc.ep_return[env0 + (t & 63)] = ep_return;
-        a.acc.ep_length[env0 + (t & 63)] = ep_length;
-    }
-    for (int i = t; i < nenv * E::OBS; i += T) {
-        const int r = i / E::OBS, c = i - r * E::OBS;
-        a.obs[(size_t)env0 * E::OBS + i] = rows[r * S::STRIDE + c];
-    }
-    S::out(rows, gbase, nenv, t, 0, E::STATE);
-}
-
 // ---------------------------------------------------------------- CartPole / Pendulum
 // The same idea for the envs whose state is a handful of floats: a workgroup of four wavefronts
 // (two on the actor, two on the critic, hidden width 64, one 32-column tile each) takes its 32
@@ -434,41 +243,6 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
 // accounting and reset in place.  A step is one dependent chain (observation -> two layers on
 // the matrix cores -> head -> sample -> env step), so the time of a step does not depend on the
 // number of envs until there are more workgroups than the chip holds at once.
-struct CartPoleSlot {
-    static constexpr int OBS = cartpole::OBS, ACT_W = 1;
-    float s[4];
-    int32_t steps;
-    MRL_DEV void load(const float *states, const int32_t *side, int i) {
-        const float4 v = reinterpret_cast<const float4 *>(states)[i];
-        s[0] = v.x; s[1] = v.y; s[2] = v.z; s[3] = v.w;
-        steps = side[i];
-    }
-    MRL_DEV void store(float *states, int32_t *side, int i) const {
-        reinterpret_cast<float4 *>(states)[i] = make_float4(s[0], s[1], s[2], s[3]);
-        side[i] = steps;
-    }
-    MRL_DEV float obs(int k) const { return s[k]; }
-    MRL_DEV void step(const float *act, float &r, float &d) { cartpole::step(s, steps, (int)act[0], r, d); }
-    MRL_DEV void reset(int i, uint64_t seed) { cartpole::reset(s, steps, i, (uint32_t)seed); }
-};
-struct PendulumSlot {
-    static constexpr int OBS = pendulum::OBS, ACT_W = 1;
-    float s[8];
-    MRL_DEV void load(const float *states, const int32_t *, int i) {
-        const float4 *row = reinterpret_cast<const float4 *>(states) + 2 * (size_t)i;
-        const float4 a = row[0], b = row[1];
-        s[0] = a.x; s[1] = a.y; s[2] = a.z; s[3] = a.w; s[4] = b.x; s[5] = b.y; s[6] = b.z; s[7] = b.w;
-    }
-    MRL_DEV void store(float *states, int32_t *, int i) const {
-        float4 *row = reinterpret_cast<float4 *>(states) + 2 * (size_t)i;
-        row[0] = make_float4(s[0], s[1], s[2], s[3]);
-        row[1] = make_float4(s[4], s[5], s[6], s[7]);
-    }
-    MRL_DEV float obs(int k) const { return s[k]; }
-    MRL_DEV void step(const float *act, float &r, float &d) { pendulum::step(s, act[0], r, d); }
-    MRL_DEV void reset(int i, uint64_t seed) { pendulum::reset(s, i, seed); }
-};
-
 constexpr int CLASSIC_TPW = 1;   // accumulator tiles per wavefront: 1 = two wavefronts per net
 constexpr int CLASSIC_THREADS = 2 * hidden_threads(64, CLASSIC_TPW);
 
@@ -572,28 +346,83 @@ __global__ __launch_bounds__(CLASSIC_THREADS) void collect_classic_kernel(Collec
     }
 }
 
-// true when mrl_rollout_steps can run the descriptor through collect_kernel
-// (the wide kernel: LunarLander with hidden width 256; the two-wavefront kernel: CartPole and
-// Pendulum with hidden width 64)
-static bool collect_fusable(const mrl_rollout *r, bool gauss, int *act) {
-    int obs, hidden;
-    if (r->env_id == MRL_ENV_LUNARLANDER && !gauss) { obs = LunarLander::OBS; hidden = 256; }
-    else if (r->env_id == MRL_ENV_LUNARLANDER_CONTINUOUS && gauss) { obs = LunarLander::OBS; hidden = 256; }
-    else if (r->env_id == MRL_ENV_CARTPOLE && !gauss) { obs = cartpole::OBS; hidden = 64; }
-    else if (r->env_id == MRL_ENV_PENDULUM && gauss) { obs = pendulum::OBS; hidden = 64; }
-    else return false;
+// What mrl_rollout_steps runs a descriptor with.
+enum CollectForm {
+    FORM_STEPS,      // no fused kernel: the steps are issued one by one
+    FORM_WALKER,     // collect_walkers.hpp
+    FORM_ROWS16,     // collect16.hpp
+    FORM_LANDER32,   // collect_kernel
+    FORM_CLASSIC32   // collect_classic_kernel
+};
+struct CollectPlan {
+    CollectForm form;
+    int H, act;   // hidden width; 1: ReLU, 2: tanh
+};
+
+// Actor and critic must be the agents' nets: two equal hidden layers of 64, 128 or 256 and the env's heads.
+static bool agent_nets(const mrl_rollout *r, int obs, int head, bool gauss, int *H, int *act) {
     const mrl_mlp_desc &a = r->actor, &c = r->critic;
     if (a.n_layers != 3 || c.n_layers != 3) return false;
-    const int k0 = a.layers[0].kind;
+    const int k0 = a.layers[0].kind, h = a.layers[0].out_dim;
     if (k0 != MRL_LINEAR_RELU && k0 != MRL_LINEAR_TANH) return false;
+    if (h != 64 && h != 128 && h != 256) return false;
     for (const mrl_mlp_desc *d : {&a, &c}) {
         if (d->layers[0].kind != k0 || d->layers[1].kind != k0) return false;
-        if (d->layers[0].in_dim != obs || d->layers[0].out_dim != hidden || d->layers[1].out_dim != hidden) return false;
+        if (d->layers[0].in_dim != obs || d->layers[0].out_dim != h || d->layers[1].out_dim != h) return false;
     }
     if (a.layers[2].kind != (gauss ? MRL_STOCHASTIC_ACTOR : MRL_LINEAR) || c.layers[2].kind != MRL_LINEAR) return false;
-    if (a.layers[2].out_dim > PA_MAX || c.layers[2].out_dim != 1) return false;
+    if (a.layers[2].out_dim > PA_MAX || (head > 0 && a.layers[2].out_dim != head) || c.layers[2].out_dim != 1) return false;
+    *H = h;
     *act = (k0 == MRL_LINEAR_RELU) ? 1 : 2;
     return true;
+}
+
+// n_cus = 0: the form for a device of unknown size is asked for (mrl_rollout_fused has no context)
+static CollectPlan collect_plan(const mrl_rollout *r, int n_cus) {
+    const bool gauss = r->num_actions == 0;
+    CollectPlan p{FORM_STEPS, 0, 0};
+    if (n_cus == 0) n_cus = 256;
+    const int id = r->env_id;
+    int obs = 0, head = 0;
+    // Up to this many envs per CU the walkers' fused kernels are the faster way; with more, their 16-env workgroups
+    // come round after round while the stand-alone kernels fill the chip.  us per step, fused against two launches,
+    // hidden width 64 / 256: HalfCheetah (one workgroup per CU) 4096 envs 69 / 73 : 84 / 88, 8192 envs 136 / 146 :
+    // 82 / 99; Walker2d 8192 envs 23.6 / 43.6 : 26.2 / 44.7, 16384 envs 46.6 / 86.6 : 31.2 / 76.5; CarRacing 8192 envs
+    // 38 / 61 : 46 / 65, 16384 envs 76 / 121 : 72 / 116; Hopper 16384 envs 19 / 69 : 25 / 69, 32768 envs 38 / 136 :
+    // 35 / 130; BipedalWalker 32768 envs 265 / 305 : 318 / 409.
+    int envs_per_cu = 0;   // 0: no limit
+    if (id == MRL_ENV_BIPEDAL) { obs = BipedalWalker::OBS; head = BipedalWalker::ACT_W; }
+    else if (id == MRL_ENV_HALFCHEETAH) { obs = HalfCheetah::OBS; head = HalfCheetah::ACT_W; envs_per_cu = 16; }
+    else if (id == MRL_ENV_CARRACING) { obs = cr::OBS; head = cr::ACT; envs_per_cu = 32; }
+    else if (id == MRL_ENV_HOPPER_PLANAR) { obs = planar::Hopper::OBS; head = planar::Hopper::ACT; envs_per_cu = 64; }
+    else if (id == MRL_ENV_WALKER2D_PLANAR) { obs = planar::Walker2d::OBS; head = planar::Walker2d::ACT; envs_per_cu = 32; }
+    if (head > 0) {
+        if (envs_per_cu > 0 && r->n_envs > envs_per_cu * n_cus) return p;
+        // (the planar rows hold doubles; the weight rows are read with 16-byte loads)
+        if (id >= MRL_ENV_HOPPER_PLANAR && reinterpret_cast<uintptr_t>(r->states) % 8 != 0) return p;
+        if (reinterpret_cast<uintptr_t>(r->actor_params) % 16 != 0 || reinterpret_cast<uintptr_t>(r->critic_params) % 16 != 0)
+            return p;
+        if (gauss && agent_nets(r, obs, head, true, &p.H, &p.act)) p.form = FORM_WALKER;
+        return p;
+    }
+    if ((id == MRL_ENV_LUNARLANDER && !gauss) || (id == MRL_ENV_LUNARLANDER_CONTINUOUS && gauss)) {
+        if (!agent_nets(r, LunarLander::OBS, 0, gauss, &p.H, &p.act)) return p;
+        // With at most 16 envs per CU the 16-row kernel (a shorter chain per step); beyond that, at hidden width
+        // 256, the 32-row kernel, whose single solver wavefront per CU steps twice the envs in the same time; the
+        // narrower nets stay with two 16-row workgroups per CU, and above those with the stand-alone kernels
+        // (from there on their env step runs one lane per env).
+        if (r->n_envs <= n_cus * PR16 || (p.H != 256 && r->n_envs <= 2 * n_cus * PR16)) p.form = FORM_ROWS16;
+        else if (p.H == 256) p.form = FORM_LANDER32;
+        return p;
+    }
+    if (id == MRL_ENV_CARTPOLE && !gauss) obs = cartpole::OBS;
+    else if (id == MRL_ENV_PENDULUM && gauss) obs = pendulum::OBS;
+    else return p;
+    if (!agent_nets(r, obs, 0, gauss, &p.H, &p.act)) return p;
+    // (hidden width 64, us per step of CartPole at 1024 / 4096 / 8192 / 16384 envs: 16 rows 3.75 / 3.71 / 5.20 / 9.86,
+    // 32 rows 4.88 / 4.66 / 4.75 / 6.20: with more than 16 envs per CU a second workgroup shares the matrix units)
+    p.form = (p.H == 64 && r->n_envs > n_cus * PR16) ? FORM_CLASSIC32 : FORM_ROWS16;
+    return p;
 }
 
 }  // namespace mrl
@@ -603,8 +432,7 @@ using namespace mrl;
 extern "C" {
 
 int mrl_rollout_fused(const mrl_rollout *r) {
-    int act = 0;
-    return r != nullptr && (collect_fusable(r, r->num_actions == 0, &act) || collect_walker_fusable(r, &act)) ? 1 : 0;
+    return r != nullptr && collect_plan(r, 0).form != FORM_STEPS ? 1 : 0;
 }
 
 int mrl_rollout_steps(mrl_ctx *ctx, const mrl_rollout *r, int t0, int n_steps, uint32_t sample_seed,
@@ -614,9 +442,8 @@ int mrl_rollout_steps(mrl_ctx *ctx, const mrl_rollout *r, int t0, int n_steps, u
     MRL_CHECK_ARG(t0 >= 0 && n_steps >= 0, "mrl_rollout_steps: bad step range");
     if (n_steps == 0) return MRL_OK;
     const bool gauss = r->num_actions == 0;
-    int act = 0;
-    const bool walker = collect_walker_fusable(r, &act);
-    if (!walker && !collect_fusable(r, gauss, &act)) {
+    const CollectPlan plan = collect_plan(r, ctx->n_cus);
+    if (plan.form == FORM_STEPS) {
         for (int k = 0; k < n_steps; ++k) {
             int rc = mrl_rollout_step(ctx, r, t0 + k, sample_seed + (uint32_t)k * sample_stride,
                                       step_seed + (uint64_t)k * step_stride, reset_seed + (uint64_t)k * reset_stride);
@@ -649,11 +476,7 @@ int mrl_rollout_steps(mrl_ctx *ctx, const mrl_rollout *r, int t0, int n_steps, u
     a.spin_limit = ctx->spin_limit;
     a.sync_error = ctx->sync_error;
     a.car_trait_form = ctx->car_trait_form;
-    // LunarLander: with at most 16 envs per CU the 16-row kernel (a shorter chain per step); beyond that
-    // the 32-row kernel, whose single solver wavefront per CU steps twice the envs in the same time
-    const bool lander = r->env_id == MRL_ENV_LUNARLANDER || r->env_id == MRL_ENV_LUNARLANDER_CONTINUOUS;
-    const bool rows16 = lander && r->n_envs <= ctx->n_cus * PR16;
-    const dim3 grid(grid_for(r->n_envs, rows16 ? PR16 : PR));
+    const dim3 grid(grid_for(r->n_envs, PR));
     int32_t *side = nullptr;
     if (r->env_id == MRL_ENV_CARTPOLE) {
         rc = cartpole_side(ctx, r->states, r->n_envs, &side);
@@ -661,30 +484,29 @@ int mrl_rollout_steps(mrl_ctx *ctx, const mrl_rollout *r, int t0, int n_steps, u
     }
     profile_step_begin(ctx);
     profile_mark(ctx, -1);
-    if (walker) {
-        rc = launch_collect_walker(ctx, r, a, act);
+    if (plan.form == FORM_WALKER || plan.form == FORM_ROWS16) {
+        const bool w = plan.form == FORM_WALKER, relu = plan.act == 1;
+#define MRL_COLLECT(HH)                                                                                          \
+    rc = w ? (relu ? launch_collect_walker_t<HH, 1>(ctx, r, a) : launch_collect_walker_t<HH, 2>(ctx, r, a))       \
+           : (relu ? launch_collect16_t<HH, 1>(ctx, r, a, side) : launch_collect16_t<HH, 2>(ctx, r, a, side))
+        if (plan.H == 64) MRL_COLLECT(64);
+        else if (plan.H == 128) MRL_COLLECT(128);
+        else MRL_COLLECT(256);
+#undef MRL_COLLECT
         if (rc) return rc;
-    } else if (r->env_id == MRL_ENV_LUNARLANDER && rows16) {
-        const dim3 block(Rows16<LunarLander>::THREADS);
-        if (act == 1) hipLaunchKernelGGL((collect16_kernel<LunarLander, 1, false>), grid, block, 0, ctx->stream, a);
-        else hipLaunchKernelGGL((collect16_kernel<LunarLander, 2, false>), grid, block, 0, ctx->stream, a);
-    } else if (r->env_id == MRL_ENV_LUNARLANDER_CONTINUOUS && rows16) {
-        const dim3 block(Rows16<LunarLander>::THREADS);
-        if (act == 1) hipLaunchKernelGGL((collect16_kernel<LunarLanderContinuous, 1, true>), grid, block, 0, ctx->stream, a);
-        else hipLaunchKernelGGL((collect16_kernel<LunarLanderContinuous, 2, true>), grid, block, 0, ctx->stream, a);
     } else if (r->env_id == MRL_ENV_LUNARLANDER) {
         const dim3 block(LunarLander::THREADS);
-        if (act == 1) hipLaunchKernelGGL((collect_kernel<LunarLander, 256, 1, false>), grid, block, 0, ctx->stream, a);
+        if (plan.act == 1) hipLaunchKernelGGL((collect_kernel<LunarLander, 256, 1, false>), grid, block, 0, ctx->stream, a);
         else hipLaunchKernelGGL((collect_kernel<LunarLander, 256, 2, false>), grid, block, 0, ctx->stream, a);
     } else if (r->env_id == MRL_ENV_LUNARLANDER_CONTINUOUS) {
         const dim3 block(LunarLander::THREADS);
-        if (act == 1) hipLaunchKernelGGL((collect_kernel<LunarLanderContinuous, 256, 1, true>), grid, block, 0, ctx->stream, a);
+        if (plan.act == 1) hipLaunchKernelGGL((collect_kernel<LunarLanderContinuous, 256, 1, true>), grid, block, 0, ctx->stream, a);
         else hipLaunchKernelGGL((collect_kernel<LunarLanderContinuous, 256, 2, true>), grid, block, 0, ctx->stream, a);
     } else if (r->env_id == MRL_ENV_CARTPOLE) {
-        if (act == 1) hipLaunchKernelGGL((collect_classic_kernel<CartPoleSlot, 1, false>), grid, dim3(CLASSIC_THREADS), 0, ctx->stream, a, side);
+        if (plan.act == 1) hipLaunchKernelGGL((collect_classic_kernel<CartPoleSlot, 1, false>), grid, dim3(CLASSIC_THREADS), 0, ctx->stream, a, side);
         else hipLaunchKernelGGL((collect_classic_kernel<CartPoleSlot, 2, false>), grid, dim3(CLASSIC_THREADS), 0, ctx->stream, a, side);
     } else {
-        if (act == 1) hipLaunchKernelGGL((collect_classic_kernel<PendulumSlot, 1, true>), grid, dim3(CLASSIC_THREADS), 0, ctx->stream, a, side);
+        if (plan.act == 1) hipLaunchKernelGGL((collect_classic_kernel<PendulumSlot, 1, true>), grid, dim3(CLASSIC_THREADS), 0, ctx->stream, a, side);
         else hipLaunchKernelGGL((collect_classic_kernel<PendulumSlot, 2, true>), grid, dim3(CLASSIC_THREADS), 0, ctx->stream, a, side);
     }
     MRL_CHECK_LAUNCH();

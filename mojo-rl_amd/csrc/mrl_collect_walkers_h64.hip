@@ -1,0 +1,7 @@
+// The walkers' fused collection kernels (collect_walkers.hpp) at hidden width 64.
+#include "collect_walkers.hpp"
+
+namespace mrl {
+template int launch_collect_walker_t<64, 1>(mrl_ctx *, const mrl_rollout *, const CollectArgs &);
+template int launch_collect_walker_t<64, 2>(mrl_ctx *, const mrl_rollout *, const CollectArgs &);
+}  // namespace mrl
