@@ -12,18 +12,25 @@ struct Mlp3Net {
     float *cache;            // forward: written when non-null; backward: read
     const float *grad_out;   // backward
     float *g1, *g0, *ls_part, *db_part, *thin_part;  // backward workspace (set by the host function)
+    float *h1;                                       // fused update: layer-0 outputs [B, H] for the weight-gradient launch
+    const unsigned short *wf, *wb;                   // fused update: the hidden layer's weights split (mlp_split.hpp), forward / W^T
     int A, gauss;            // set by the host function from the description
     int thin_stride;         // floats per row tile in thin_part: IN H + H A, + H H where the tiles carry dW1 too
 };
 struct Mlp3Nets { Mlp3Net n[2]; };
 
-// PPO tail of a paired forward (net 0 = actor, net 1 = critic) over minibatch rows that are still
+// split operand copies of the nets' hidden-layer weights (mlp_split.hpp)
+struct SplitNets {
+    const float *w1[2];
+    unsigned short *wf[2], *wb[2];
+};
+
+// The PPO part of the fused update (net 0 = actor, net 1 = critic) over minibatch rows that are still
 // where the rollout left them: the forward reads its input rows through `idx`, and every row tile
 // goes straight on to its loss gradients (deep_agents/ppo/ppo.mojo:285-378, 538-633;
 // kernels.mojo:230-486) and to its share of the KL early-stop test, so that neither a gather nor a
-// loss launch is needed.  enabled = 0: plain forward.
+// loss launch is needed.
 struct FwdLoss {
-    int enabled;
     const int32_t *idx;                                   // [mb] rollout rows of the minibatch
     const float *r_obs, *r_act, *r_adv, *r_ret, *r_logp, *r_val;
     const float *adv_stats;                               // {mean, std} of the minibatch's advantages; null: as they are
@@ -39,18 +46,30 @@ bool mlp3_fusable(const mrl_mlp_desc &d, int *H, int *act, bool *gauss);
 bool mlp3_pair_fusable(const mrl_mlp_desc &a, const mrl_mlp_desc &b);
 int mlp3_forward(mrl_ctx *ctx, const mrl_mlp_desc &d, int batch, const float *in, const float *params,
                  float *out, float *cache);
-int mlp3_forward_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, int batch, Mlp3Nets io,
-                   const FwdLoss *loss = nullptr);
 size_t mlp3_backward_ws(const mrl_mlp_desc *const *descs, int n_nets, int batch);
 int mlp3_backward(mrl_ctx *ctx, const mrl_mlp_desc &d, int batch, const float *grad_out, const float *params,
                   const float *cache, float *grads, float *ws);
+int mlp3_backward_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, int batch, Mlp3Nets io,
+                    float *const *grads, float *ws);
+
+// The fused update of two nets: one kernel per row tile runs forward (inputs read through loss.idx, io.n[i].out
+// written), loss gradients and the way back (mrl_fb.hip), then the H x H weight gradients and the sums over the tiles.
+// Workspace: UpdateWs, carved from the context's.
+struct UpdateWs {
+    int rows, tiles;          // batch rows per tile
+    bool dw_in_tiles;
+    SplitNets split;          // copies of the hidden layers' weights that io.n[i].wf / wb read
+    Mlp3Net net[2];           // g1, h1, ls_part, db_part, thin_part, thin_stride
+    float *partial;
+    int splits, rows_per;     // batch splits of the weight-gradient launch
+};
+int mlp3_update_ws(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int batch, const float *const *params, UpdateWs *out);
+int launch_split_weights(mrl_ctx *ctx, int H, const SplitNets &s, int n_nets);
 // sq_part (nullable): receives per-block sums of squares of the gradients, [net * 1024 + block];
 // *sq_blocks = number of blocks written (0 when none were)
-// fused (nullable): the nets have not gone forward yet -- one kernel per row tile runs forward
-// (inputs read through fused->idx, io.n[i].out written, h1 into the cache's c1 rows), loss
-// gradients and the way back, in place of a forward launch, a loss launch and the dx launch
-int mlp3_backward_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, int batch, Mlp3Nets io,
-                    float *const *grads, float *ws, float *sq_part, int *sq_blocks, const FwdLoss *fused = nullptr);
+int mlp3_update_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int batch, Mlp3Nets io, const UpdateWs &ws,
+                  float *const *grads, float *sq_part, int *sq_blocks, const FwdLoss &loss);
+int launch_fb(mrl_ctx *ctx, int H, int act, int batch, int IN, int rows, const Mlp3Nets &nets, const FwdLoss &fl);
 // grows the context's MLP workspace to at least `floats`
 int mlp_ensure_ws(mrl_ctx *ctx, size_t floats, float **out);
 

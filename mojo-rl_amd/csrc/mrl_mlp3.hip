@@ -1,27 +1,28 @@
-// Fused kernels for the update path of three-layer nets  IN -> H -> H -> out  (H in {64, 128, 256},
-// IN <= 32, out <= 8 or a StochasticActor head of <= 8 actions): the shapes of every actor and
-// critic the PPO agents build (deep_agents/ppo/ppo.mojo:779-817, ppo_continuous.mojo:171-194).
+// Fused kernels for three-layer nets  IN -> H -> H -> out  (H in {64, 128, 256}, IN <= 32, out <= 8 or a
+// StochasticActor head of <= 8 actions): the shapes of every actor and critic the PPO agents build
+// (deep_agents/ppo/ppo.mojo:779-817, ppo_continuous.mojo:171-194).
 //
 //   mlp3_fwd_kernel     the whole forward of a 32-row tile in one launch (hidden activations
 //                       stay in LDS), writing the reference's per-layer cache on the way;
 //   mlp3_bwd_dx_kernel  the chain  g2 -> g1 = (g2 W2^T) * act' -> g0 = (g1 W1^T) * act'  of a
 //                       32-row tile in one launch; g1 and g0 go to a workspace;
-//   dw3_kernel          [dW | db] of all three layers in one launch, split over the batch;
-//   sum3_kernel         sum of the splits straight into the flat gradient vector (+ log_std).
+//   dw3_kernel          dW of the hidden layer, split over the batch;
+//   sum3_kernel         sum of the splits and of the row tiles' pieces straight into the flat gradient vector.
 // They replace 3 + 2 + 3 + 3 launches of the per-layer kernels (which remain the path for any
-// other shape, and for callers that ask for the gradient with respect to the input).
+// other shape, and for callers that ask for the gradient with respect to the input).  The minibatch update's
+// row tiles (mrl_fb.hip) share the last two.
 #include "mrl_host.hpp"
 #include "mrl_device.hpp"
 #include "mlp_tile.hpp"
+#include "mlp_split.hpp"
 #include "mlp3.hpp"
-#include "ppo_grads.hpp"
 
 namespace mrl {
 
 // grid = (row tiles, nets): blockIdx.y picks the net, so that an actor and a critic that read the
 // same inputs go through the chip side by side
 template <int H, int ACT>
-__global__ __launch_bounds__(2 * H) void mlp3_fwd_kernel(int B, int IN, Mlp3Nets nets, FwdLoss fl) {
+__global__ __launch_bounds__(2 * H) void mlp3_fwd_kernel(int B, int IN, Mlp3Nets nets) {
     constexpr int T = 2 * H;   // one 32-column accumulator tile per wavefront
     __shared__ float xs[PR * XS_LD];
     __shared__ float hT[H * HT_LD];
@@ -54,8 +55,7 @@ __global__ __launch_bounds__(2 * H) void mlp3_fwd_kernel(int B, int IN, Mlp3Nets
         const int i = t + q * T;
         xv[q] = 0.0f;
         if (i < PR * IN && i / IN < nrow) {
-            const int r = i / IN;
-            xv[q] = fl.enabled ? fl.r_obs[(size_t)fl.idx[row0 + r] * IN + (i - r * IN)] : x[row0 * IN + i];
+            xv[q] = x[row0 * IN + i];
         }
     }
     stage_head(params + IN * H + H + H * H + H, H, A, GAUSS, w2s, t, T);
@@ -85,51 +85,6 @@ __global__ __launch_bounds__(2 * H) void mlp3_fwd_kernel(int B, int IN, Mlp3Nets
         }
         out[(row0 + r) * ld + a] = v;
     }
-    if (!fl.enabled) return;
-    // ---- loss gradients of the tile's rows, one lane per row (wavefront 0)
-    if (t >= 64) return;
-    const int b = (int)row0 + t;
-    const bool mine = t < nrow;
-    const long src = mine ? fl.idx[b] : 0;
-    if (blockIdx.y == 1) {   // critic
-        if (mine)
-            fl.g_values[b] = critic_grad_value(ys[t * (PA_MAX + 1)], fl.clip_value ? fl.r_val[src] : 0.0f, fl.r_ret[src],
-                                               fl.mb, fl.continuous, fl.clip_value, fl.value_coef, fl.clip_eps);
-        return;
-    }
-    float kl = 0.0f;
-    if (mine) {
-        float adv = fl.r_adv[src];
-        if (fl.adv_stats != nullptr) adv = (adv - fl.adv_stats[0]) / (fl.adv_stats[1] + 1e-8f);
-        const float old_logp = fl.r_logp[src];
-        float o[2 * PA_MAX], g[2 * PA_MAX];
-#pragma unroll
-        for (int a = 0; a < PA_MAX; ++a) {
-            o[a] = ys[t * (PA_MAX + 1) + a];
-            float ls = w2s[HEAD_LOG_STD(H) + a];
-            o[PA_MAX + a] = ls;
-        }
-        if (fl.continuous) {
-            float oo[2 * PA_MAX], act[PA_MAX];
-            for (int j = 0; j < A; ++j) {
-                oo[j] = o[j];
-                oo[A + j] = o[PA_MAX + j];   // clamped inside the gradient, as in the stored output
-                act[j] = fl.r_act[src * A + j];
-            }
-            kl = actor_grad_gaussian_row(oo, act, adv, old_logp, fl.mb, A, fl.clip_eps, fl.ent_coef, g);
-            for (int j = 0; j < 2 * A; ++j) fl.g_actor_out[(size_t)b * 2 * A + j] = g[j];
-        } else {
-            kl = actor_grad_discrete_row(o, (int)fl.r_act[src], adv, old_logp, fl.mb, A, fl.clip_eps, fl.ent_coef, g);
-            for (int a = 0; a < A; ++a) fl.g_actor_out[(size_t)b * A + a] = g[a];
-        }
-        fl.kl[b] = kl;
-    }
-    if (fl.kl_flag == nullptr) return;
-    // KL test: every actor tile leaves the sum of its rows' estimates; the kernel that applies the
-    // update adds the tiles up and compares the mean with target_kl
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) kl += __shfl_xor(kl, off, 64);
-    if (t == 0) fl.kl_part[blockIdx.x] = kl;
 }
 
 template <int ACT>
@@ -303,312 +258,6 @@ __global__ __launch_bounds__(2 * H) void mlp3_bwd_dx_kernel(int B, int IN, Mlp3N
         g0[(row0 + row) * H + col] = val;
         gv[v] = val;
         cs += val;
-    }
-    // the two halves of the wavefront hold the other 16 rows of the same column
-    cs += __shfl_xor(cs, 32, 64);
-    if (half == 0) db_part[col] = cs;   // bias gradient of layer 0, this tile's rows
-    // dW0[i][col] of the tile = sum_r x[r][i] g0[r][col]
-    for (int i = 0; i < IN; ++i) {
-        float s = 0.0f;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) s = fmaf(xs[(8 * (v >> 2) + 4 * half + (v & 3)) * XS_LD + i], gv[v], s);
-        s += __shfl_xor(s, 32, 64);
-        if (half == 0) thin_part[(size_t)i * H + col] = s;
-    }
-}
-
-// ---------------------------------------------------------------- forward + loss + backward of a tile
-// The PPO minibatch never needs the activations outside the workgroup that made them: a row tile
-// goes forward (as mlp3_fwd_kernel with its loss tail), and while h1 and h2 are still in LDS the
-// same workgroup takes the loss gradient back through the three layers (as mlp3_bwd_dx_kernel).
-// Only what the H x H weight gradient needs leaves the chip -- h1 (into the cache's c1 rows) and
-// g1 -- next to the per-tile bias / thin-layer partials.  act' comes from the activation's output
-// (y > 0 for ReLU, 1 - y^2 for tanh), which is what the cached entries decide as well.
-template <int ACT>
-MRL_DEV float act_deriv_out(float y) {
-    if (ACT == 1) return y > 0.0f ? 1.0f : 0.0f;
-    if (ACT == 2) return 1.0f - y * y;
-    return 1.0f;
-}
-
-template <int H, int ACT>
-__global__ __launch_bounds__(2 * H) void mlp3_fb_kernel(int B, int IN, Mlp3Nets nets, FwdLoss fl) {
-    constexpr int T = 2 * H, KCH = 64;
-    static_assert(KCH * (H + 1) <= H * HT_LD + PR * (H + 1), "the W1 staging buffer fits over the two activation tiles");
-    __shared__ float xs[PR * XS_LD];
-    __shared__ float big[H * HT_LD + PR * (H + 1)];   // hT | h2 going forward, W1 chunks going back
-    __shared__ float ys[PR * (PA_MAX + 1)];
-    __shared__ __align__(16) float w2s[HEAD_LDS(H)];
-    __shared__ float g2s[PR * (2 * PA_MAX + 1)];
-    __shared__ float gT[H * HT_LD];                   // g1 of the tile, k-major
-    float *hT = big, *h2 = big + H * HT_LD, *wT = big;
-    const Mlp3Net &nn = nets.n[blockIdx.y];
-    const float *__restrict__ params = nn.params;
-    float *__restrict__ out = nn.out;
-    float *__restrict__ g1 = nn.g1;
-    float *__restrict__ ls_part = nn.ls_part;
-    float *__restrict__ db_part = nn.db_part + (size_t)blockIdx.x * (2 * H + PA_MAX);
-    const int A = nn.A;
-    float *__restrict__ thin_part = nn.thin_part + (size_t)blockIdx.x * (size_t)nn.thin_stride;
-    const bool GAUSS = nn.gauss != 0;
-    const int ld = GAUSS ? 2 * A : A;
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6, half = lane >> 5, l31 = lane & 31;
-    const long row0 = (long)blockIdx.x * PR;
-    const int nrow = (int)min((long)PR, B - row0);
-    const float *W1 = params + IN * H + H;
-    TileCache tc{nullptr, nn.cache + (size_t)B * (IN + H), nullptr, row0, nrow};   // h1 only
-
-    // ---- forward
-    HiddenOperands<H, 1, 32> ops;
-    ops.load(params, IN);
-    constexpr int NX = (PR * PIN_MAX + T - 1) / T;
-    float xv[NX];
-#pragma unroll
-    for (int q = 0; q < NX; ++q) {
-        const int i = t + q * T;
-        xv[q] = 0.0f;
-        if (i < PR * IN && i / IN < nrow) {
-            const int r = i / IN;
-            xv[q] = fl.r_obs[(size_t)fl.idx[row0 + r] * IN + (i - r * IN)];
-        }
-    }
-    stage_head(params + IN * H + H + H * H + H, H, A, GAUSS, w2s, t, T);
-    for (int i = t; i < PR * (2 * PA_MAX + 1); i += T) g2s[i] = 0.0f;
-    // The loss lanes ask for their rows' rollout entries now.  Critic: the lane of row t (wavefront 0).
-    // Actor: eight lanes per row, lane lj on logit / action component lj (rows lr, lr + T / 8, ...), so
-    // that a row's exponentials and logarithms are taken side by side instead of one after the other.
-    static_assert(PA_MAX == 8 && T % 8 == 0, "eight lanes per row");
-    constexpr int LR = (PR + T / 8 - 1) / (T / 8);   // rows per actor loss lane (lanes past the tile's rows idle)
-    const bool loss_lane = t < nrow;
-    const int lr = t >> 3, lj = t & 7;
-    float l_ret = 0.0f, l_val = 0.0f, l_mean = 0.0f, l_std = 1.0f;
-    float l_adv[LR], l_logp[LR], l_act[LR];   // l_act: the action (discrete) or its component lj
-    if (blockIdx.y == 1) {
-        if (loss_lane) {
-            const long src = fl.idx[row0 + t];
-            l_ret = fl.r_ret[src];
-            if (fl.clip_value) l_val = fl.r_val[src];
-        }
-    } else {
-        if (fl.adv_stats != nullptr) { l_mean = fl.adv_stats[0]; l_std = fl.adv_stats[1]; }
-#pragma unroll
-        for (int q = 0; q < LR; ++q) {
-            const int r = lr + q * (T / 8);
-            l_adv[q] = 0.0f; l_logp[q] = 0.0f; l_act[q] = 0.0f;
-            if (r < nrow) {
-                const long src = fl.idx[row0 + r];
-                l_adv[q] = fl.r_adv[src];
-                l_logp[q] = fl.r_logp[src];
-                if (!fl.continuous) l_act[q] = fl.r_act[src];
-                else if (lj < A) l_act[q] = fl.r_act[src * A + lj];
-            }
-        }
-    }
-#pragma unroll
-    for (int q = 0; q < NX; ++q) {
-        const int i = t + q * T;
-        if (i < PR * IN) xs[(i / IN) * XS_LD + (i % IN)] = xv[q];
-    }
-    __syncthreads();
-    hidden_stack<H, ACT, 1>(params, IN, xs, hT, h2, tc, ops);
-    head<H>(w2s, A, h2, ys, PA_MAX + 1, t, 2 * H);
-    __syncthreads();
-    for (int i = t; i < nrow * ld; i += T) {
-        const int r = i / ld, a = i - r * ld;
-        float v;
-        if (a < A) {
-            v = ys[r * (PA_MAX + 1) + a];
-        } else {   // state-independent log_std, clamped (deep_rl/model/stochastic_actor.mojo:260-275)
-            v = w2s[HEAD_LOG_STD(H) + (a - A)];
-            if (v < -5.0f) v = -5.0f;
-            else if (v > 2.0f) v = 2.0f;
-        }
-        out[(row0 + r) * ld + a] = v;
-    }
-    // what the way back needs from the forward tiles before their memory is reused: act'(h1) at
-    // this lane's accumulator positions; and the first chunk of W1
-    const int col = 32 * w + l31;
-    float d0[16];
-#pragma unroll
-    for (int v = 0; v < 16; ++v) d0[v] = act_deriv_out<ACT>(hT[col * HT_LD + 8 * (v >> 2) + 4 * half + (v & 3)]);
-    const int wrow = t % H, wseg = (t / H) * (KCH / 2);   // thread copies W1[wrow][o0 + wseg .. + KCH / 2)
-    float4 nxt[KCH / 8];
-    auto fetch = [&](int o0) {
-        const float4 *src = reinterpret_cast<const float4 *>(W1 + (size_t)wrow * H + o0 + wseg);
-#pragma unroll
-        for (int q = 0; q < KCH / 8; ++q) nxt[q] = src[q];
-    };
-    fetch(0);
-
-    // ---- loss gradients of the tile's rows into g2s and out
-    if (blockIdx.y == 1) {   // critic: one lane per row
-        if (loss_lane) {
-            const float g = critic_grad_value(ys[t * (PA_MAX + 1)], l_val, l_ret, fl.mb, fl.continuous, fl.clip_value,
-                                              fl.value_coef, fl.clip_eps);
-            g2s[t * (2 * PA_MAX + 1)] = g;
-            fl.g_values[(int)row0 + t] = g;
-        }
-    } else {
-        // (rows past nrow are worked on like the others -- their lanes take part in the exchanges -- and not stored)
-#pragma unroll
-        for (int q = 0; q < LR; ++q) {
-            const int r = lr + q * (T / 8), b = (int)row0 + r;
-            float *g2row = g2s + r * (2 * PA_MAX + 1);
-            float adv = l_adv[q];
-            if (fl.adv_stats != nullptr) adv = (adv - l_mean) / (l_std + 1e-8f);
-            const float mine = ys[(r < PR ? r : 0) * (PA_MAX + 1) + lj];
-            float kl;
-            if (fl.continuous) {
-                float gm, gs;   // (log_std is clamped inside the gradient, as in the stored output)
-                kl = actor_grad_gaussian_lanes(mine, w2s[HEAD_LOG_STD(H) + lj], l_act[q], lj, lane & ~7, adv, l_logp[q], fl.mb,
-                                               A, fl.clip_eps, fl.ent_coef, gm, gs);
-                if (r < nrow && lj < A) {
-                    g2row[lj] = gm;
-                    g2row[A + lj] = gs;
-                    fl.g_actor_out[(size_t)b * ld + lj] = gm;
-                    fl.g_actor_out[(size_t)b * ld + A + lj] = gs;
-                }
-            } else {
-                float g;
-                kl = actor_grad_discrete_lanes(mine, lj, lane & ~7, (int)l_act[q], adv, l_logp[q], fl.mb, A, fl.clip_eps,
-                                               fl.ent_coef, g);
-                if (r < nrow && lj < A) {
-                    g2row[lj] = g;
-                    fl.g_actor_out[(size_t)b * ld + lj] = g;
-                }
-            }
-            if (r < nrow && lj == 0) {
-                fl.kl[b] = kl;
-                g2row[2 * PA_MAX] = kl;   // (the spare float of the row, for the tile's sum below)
-            }
-        }
-    }
-    __syncthreads();   // g2s complete
-    if (fl.kl_flag != nullptr && blockIdx.y == 0 && t < 64) {
-        // KL test: every actor tile leaves the sum of its rows' estimates; the kernel that applies the
-        // update (clip + Adam) adds the tiles up and compares the mean with target_kl, so that nothing
-        // here waits for other workgroups
-        float kl = t < nrow ? g2s[t * (2 * PA_MAX + 1) + 2 * PA_MAX] : 0.0f;
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) kl += __shfl_xor(kl, off, 64);
-        if (t == 0) fl.kl_part[blockIdx.x] = kl;
-    }
-
-    // ---- back through the head and layer 1's activation, on the matrix cores; wavefront w owns
-    // columns [32w, 32w + 32) of the hidden layers throughout
-    {   // g1[r][n] = (sum_a g2[r][a] W2[n][a]) * act'(layer 1): K = PA_MAX (W2 rows are zero beyond A)
-        floatx16 c = {0};
-#pragma unroll
-        for (int kk = 0; kk < PA_MAX / 2; ++kk) {
-            const int k = 2 * kk + half;
-            c = __builtin_amdgcn_mfma_f32_32x32x2f32(g2s[l31 * (2 * PA_MAX + 1) + k], w2s[col * PA_MAX + k], c, 0, 0, 0);
-        }
-        float colsum = 0.0f;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const int row = 8 * (v >> 2) + 4 * half + (v & 3);
-            float g = 0.0f;
-            if (row < nrow) {
-                g = c[v] * act_deriv_out<ACT>(h2[row * (H + 1) + col]);
-                g1[(row0 + row) * H + col] = g;
-            }
-            gT[col * HT_LD + row] = g;
-            colsum += g;
-        }
-        colsum += __shfl_xor(colsum, 32, 64);
-        if (half == 0) db_part[H + col] = colsum;   // bias gradient of layer 1, this tile's rows
-    }
-    {   // dW2[n][a] of the tile = sum_r h2[r][n] g2[r][a]: K = the tile's 32 rows (g2 rows beyond nrow are zero)
-        floatx16 c = {0};
-#pragma unroll
-        for (int kk = 0; kk < PR / 2; ++kk) {
-            const int r = 2 * kk + half;
-            const float gb = l31 < 2 * PA_MAX ? g2s[r * (2 * PA_MAX + 1) + l31] : 0.0f;
-            c = __builtin_amdgcn_mfma_f32_32x32x2f32(h2[r * (H + 1) + col], gb, c, 0, 0, 0);
-        }
-        if (l31 < A) {
-            float *o2 = thin_part + (size_t)IN * H + l31;
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int n = 32 * w + 8 * (v >> 2) + 4 * half + (v & 3);
-                o2[(size_t)n * A] = c[v];
-            }
-        }
-    }
-    if (t < ld) {   // column sums of the tile: bias gradient of the head, log_std gradient
-        float cs2 = 0.0f;
-        for (int r = 0; r < PR; ++r) cs2 += g2s[r * (2 * PA_MAX + 1) + t];
-        if (t < A) db_part[2 * H + t] = cs2;
-        else ls_part[(long)blockIdx.x * A + (t - A)] = cs2;
-    }
-    if (fl.dw_in_tiles) {
-        // The hidden layer's weight gradient of the tile, dW1[k][n] = sum_r h1[r][k] g1[r][n], is (H / 32)^2
-        // 32 x 32 tiles of 16 k-steps.  It is taken here, from h1 and g1 while both lie in LDS, as one more
-        // per-tile piece for the sum kernel (wavefront w: columns [32w, 32w + 32)), instead of in a launch of its
-        // own that reads h1 and g1 back from global memory, where the launch is the larger part (dw_in_tiles_pays).
-        __syncthreads();   // gT complete
-        float *o1 = thin_part + (size_t)IN * H + (size_t)H * A;
-#pragma unroll
-        for (int kt = 0; kt < H / 32; ++kt) {
-            floatx16 c = {0};
-#pragma unroll
-            for (int kk = 0; kk < PR / 2; ++kk) {
-                const int r = 2 * kk + half;
-                c = __builtin_amdgcn_mfma_f32_32x32x2f32(hT[(32 * kt + l31) * HT_LD + r], gT[col * HT_LD + r], c, 0, 0, 0);
-            }
-#pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int k = 32 * kt + 8 * (v >> 2) + 4 * half + (v & 3);
-                o1[(size_t)k * H + col] = c[v];
-            }
-        }
-    }
-    // ---- dh1 = g1 W1^T: wavefront w owns input columns [32w, 32w + 32); the next chunk of W1 is
-    // fetched into registers while the matrix cores work on the current one
-    floatx16 acc = {0};
-    for (int o0 = 0; o0 < H; o0 += KCH) {
-        __syncthreads();   // gT complete and the activation tiles read (first round) / previous chunk consumed
-#pragma unroll
-        for (int q = 0; q < KCH / 8; ++q) {
-            wT[(wseg + 4 * q + 0) * (H + 1) + wrow] = nxt[q].x;
-            wT[(wseg + 4 * q + 1) * (H + 1) + wrow] = nxt[q].y;
-            wT[(wseg + 4 * q + 2) * (H + 1) + wrow] = nxt[q].z;
-            wT[(wseg + 4 * q + 3) * (H + 1) + wrow] = nxt[q].w;
-        }
-        __syncthreads();
-        if (o0 + KCH < H) fetch(o0 + KCH);
-        __builtin_amdgcn_sched_barrier(0);   // keep the loads ahead of the MFMAs that hide them
-        // operands of eight k-steps are read from LDS while the previous eight are multiplied
-        constexpr int G = 8;
-        float a[G], b[G], na[G], nb[G];
-#pragma unroll
-        for (int j = 0; j < G; ++j) {
-            a[j] = gT[(o0 + 2 * j + half) * HT_LD + l31];
-            b[j] = wT[(2 * j + half) * (H + 1) + col];
-        }
-#pragma unroll
-        for (int g = 0; g < KCH / 2 / G; ++g) {
-            if (g + 1 < KCH / 2 / G) {
-#pragma unroll
-                for (int j = 0; j < G; ++j) {
-                    const int k = 2 * ((g + 1) * G + j) + half;
-                    na[j] = gT[(o0 + k) * HT_LD + l31];
-                    nb[j] = wT[k * (H + 1) + col];
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < G; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j], b[j], acc, 0, 0, 0);
-#pragma unroll
-            for (int j = 0; j < G; ++j) { a[j] = na[j]; b[j] = nb[j]; }
-        }
-    }
-    float cs = 0.0f;
-    float gv[16];
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        const int row = 8 * (v >> 2) + 4 * half + (v & 3);
-        gv[v] = row < nrow ? acc[v] * d0[v] : 0.0f;
-        cs += gv[v];
     }
     // the two halves of the wavefront hold the other 16 rows of the same column
     cs += __shfl_xor(cs, 32, 64);
@@ -842,12 +491,18 @@ static int net_P(const mrl_mlp_desc &d) {
     return (IN + 1) * H + (H + 1) * H + (H + 1) * A + (d.layers[2].kind == MRL_STOCHASTIC_ACTOR ? A : 0);
 }
 
-// Whether the fused forward + backward kernel takes the hidden layer's weight gradient of its row tile itself
-// (H^2 floats per tile and net, added up by the sum kernel) or leaves h1 and g1 to a launch of dw3_kernel.  Per
-// minibatch of 64 / 1024 / 4096 / 8192 rows (Walker2d's nets), in the tile against the launch: H = 128
-// 29.6 / 32.0 / 38.8 / 62.3 against 31.7 / 38.6 / 43.7 / 65.6 us; H = 256 53.8 / 63.0 / 72.1 / 131.8 against
-// 49.1 / 58.1 / 67.8 / 112.3 us.  (Beyond 8192 rows the pieces would be a workspace of more than 32 MB.)
-static bool dw_in_tiles_pays(int H, int tiles) { return H == 64 || (H == 128 && tiles <= 256); }
+// Rows per tile of the fused update kernel: 16 while both nets' tiles fit the chip's CUs in one go, else 32 (a weight
+// operand then serves two row tiles, and half as many per-tile pieces are added up).  us per minibatch of 256 / 1024 /
+// 2048 / 4096 rows, 16 against 32: H = 64 14.0 / 15.5 / 17.8 / 23.3 : 18.1 / 17.7 / 18.0 / 20.6; H = 256 33.8 / 37.3 /
+// 40.8 / 60.5 : 40.9 / 42.3 / 45.1 / 50.4; H = 128, whose pieces hold the H x H gradient as well, 17.6 / 21.9 / 26.5 /
+// 33.3 : 22.9 / 23.1 / 25.8 / 29.9, hence half the bound there.
+static int fb_tile_rows(int n_cus, int H, int batch) {
+    return 2 * ((batch + 15) / 16) <= (H == 128 ? n_cus / 2 : n_cus) ? 16 : 32;
+}
+
+// Whether the fused update kernel takes the hidden layer's weight gradient of its row tile itself
+// (H^2 floats per tile and net, added up by the sum kernel) or leaves h1 and g1 to a launch of dw3_kernel.
+static bool dw_in_tiles_pays(int H, int batch) { return H == 64 || (H == 128 && batch <= 8192); }
 
 // true when the two nets can share launches: both fusable, same input width, width and activation
 bool mlp3_pair_fusable(const mrl_mlp_desc &a, const mrl_mlp_desc &b) {
@@ -858,53 +513,33 @@ bool mlp3_pair_fusable(const mrl_mlp_desc &a, const mrl_mlp_desc &b) {
 }
 
 template <int H, int ACT>
-static void launch_fwd_t(mrl_ctx *ctx, int batch, int IN, const Mlp3Nets &nets, int n_nets, const FwdLoss &fl) {
-    dim3 grid((batch + PR - 1) / PR, n_nets);
-    hipLaunchKernelGGL((mlp3_fwd_kernel<H, ACT>), grid, dim3(2 * H), 0, ctx->stream, batch, IN, nets, fl);
+static void launch_fwd_t(mrl_ctx *ctx, int batch, int IN, const Mlp3Nets &nets) {
+    hipLaunchKernelGGL((mlp3_fwd_kernel<H, ACT>), dim3((batch + PR - 1) / PR), dim3(2 * H), 0, ctx->stream, batch, IN, nets);
 }
 template <int H, int ACT>
-static void launch_bwd_t(mrl_ctx *ctx, int batch, int IN, const Mlp3Nets &nets, int n_nets, const FwdLoss *fused) {
+static void launch_bwd_t(mrl_ctx *ctx, int batch, int IN, const Mlp3Nets &nets, int n_nets) {
     dim3 grid((batch + PR - 1) / PR, n_nets);
-    if (fused != nullptr)
-        hipLaunchKernelGGL((mlp3_fb_kernel<H, ACT>), grid, dim3(2 * H), 0, ctx->stream, batch, IN, nets, *fused);
-    else
-        hipLaunchKernelGGL((mlp3_bwd_dx_kernel<H, ACT>), grid, dim3(2 * H), 0, ctx->stream, batch, IN, nets);
-}
-
-// forward of one or two nets (descs[i], io.n[i]) in one launch
-int mlp3_forward_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, int batch, Mlp3Nets io,
-                   const FwdLoss *loss) {
-    int H = 0, act = 0;
-    bool gauss = false;
-    for (int i = 0; i < n_nets; ++i) {
-        if (!mlp3_fusable(*descs[i], &H, &act, &gauss)) return MRL_E_UNSUPPORTED;
-        io.n[i].A = descs[i]->layers[2].out_dim;
-        io.n[i].gauss = gauss ? 1 : 0;
-    }
-    if (n_nets == 2 && !mlp3_pair_fusable(*descs[0], *descs[1])) return MRL_E_UNSUPPORTED;
-    const int IN = descs[0]->layers[0].in_dim;
-    FwdLoss fl{};
-    if (loss != nullptr) {
-        if (n_nets != 2 || (batch + PR - 1) / PR > 1024) return MRL_E_UNSUPPORTED;   // one KL partial per row tile
-        fl = *loss;
-        fl.enabled = 1;
-    }
-    if (H == 256 && act == 1) launch_fwd_t<256, 1>(ctx, batch, IN, io, n_nets, fl);
-    else if (H == 256) launch_fwd_t<256, 2>(ctx, batch, IN, io, n_nets, fl);
-    else if (H == 128 && act == 1) launch_fwd_t<128, 1>(ctx, batch, IN, io, n_nets, fl);
-    else if (H == 128) launch_fwd_t<128, 2>(ctx, batch, IN, io, n_nets, fl);
-    else if (act == 1) launch_fwd_t<64, 1>(ctx, batch, IN, io, n_nets, fl);
-    else launch_fwd_t<64, 2>(ctx, batch, IN, io, n_nets, fl);
-    MRL_CHECK_LAUNCH();
-    return MRL_OK;
+    hipLaunchKernelGGL((mlp3_bwd_dx_kernel<H, ACT>), grid, dim3(2 * H), 0, ctx->stream, batch, IN, nets);
 }
 
 int mlp3_forward(mrl_ctx *ctx, const mrl_mlp_desc &d, int batch, const float *in, const float *params,
                  float *out, float *cache) {
+    int H = 0, act = 0;
+    bool gauss = false;
+    if (!mlp3_fusable(d, &H, &act, &gauss)) return MRL_E_UNSUPPORTED;
     Mlp3Nets io{};
     io.n[0].x = in; io.n[0].params = params; io.n[0].out = out; io.n[0].cache = cache;
-    const mrl_mlp_desc *ds[1] = {&d};
-    return mlp3_forward_n(ctx, ds, 1, batch, io);
+    io.n[0].A = d.layers[2].out_dim;
+    io.n[0].gauss = gauss ? 1 : 0;
+    const int IN = d.layers[0].in_dim;
+    if (H == 256 && act == 1) launch_fwd_t<256, 1>(ctx, batch, IN, io);
+    else if (H == 256) launch_fwd_t<256, 2>(ctx, batch, IN, io);
+    else if (H == 128 && act == 1) launch_fwd_t<128, 1>(ctx, batch, IN, io);
+    else if (H == 128) launch_fwd_t<128, 2>(ctx, batch, IN, io);
+    else if (act == 1) launch_fwd_t<64, 1>(ctx, batch, IN, io);
+    else launch_fwd_t<64, 2>(ctx, batch, IN, io);
+    MRL_CHECK_LAUNCH();
+    return MRL_OK;
 }
 
 // floats of workspace mlp3_backward_n needs for these nets
@@ -914,64 +549,27 @@ size_t mlp3_backward_ws(const mrl_mlp_desc *const *descs, int n_nets, int batch)
         const int H = descs[i]->layers[0].out_dim;
         const int IN = descs[i]->layers[0].in_dim, A = descs[i]->layers[2].out_dim;
         total += (size_t)2 * batch * H +
-                 (size_t)((batch + PR - 1) / PR) * (2 * PA_MAX + 2 * H + (size_t)IN * H + (size_t)H * A +
-                                                    (dw_in_tiles_pays(H, (batch + PR - 1) / PR) ? (size_t)H * H : 0));
+                 (size_t)((batch + PR - 1) / PR) * (2 * PA_MAX + 2 * H + (size_t)IN * H + (size_t)H * A);
         P += net_P(*descs[i]);
     }
     return total + (size_t)32 * P;
 }
 
-// backward (parameter gradients only) of one or two nets: io.n[i].grad_out / params / cache in,
-// grads[i] out; ws as sized by mlp3_backward_ws
-int mlp3_backward_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, int batch, Mlp3Nets io,
-                    float *const *grads, float *ws, float *sq_part, int *sq_blocks, const FwdLoss *fused) {
-    if (fused != nullptr && (n_nets != 2 || (batch + PR - 1) / PR > 1024)) return MRL_E_UNSUPPORTED;
-    int H = 0, act = 0;
-    bool gauss = false;
-    for (int i = 0; i < n_nets; ++i) {
-        if (!mlp3_fusable(*descs[i], &H, &act, &gauss)) return MRL_E_UNSUPPORTED;
-        io.n[i].A = descs[i]->layers[2].out_dim;
-        io.n[i].gauss = gauss ? 1 : 0;
-        // the W1 rows are staged with 16-byte loads
-        const int IN = descs[i]->layers[0].in_dim;
-        if (reinterpret_cast<uintptr_t>(io.n[i].params + IN * H + H) % 16 != 0) return MRL_E_UNSUPPORTED;
-    }
-    if (n_nets == 2 && !mlp3_pair_fusable(*descs[0], *descs[1])) return MRL_E_UNSUPPORTED;
-    const int IN = descs[0]->layers[0].in_dim;
-    const int tiles = (batch + PR - 1) / PR;
-    int splits = std::max(1, std::min(32, batch / 256));
-    int rows_per = ((batch + splits - 1) / splits + DKC - 1) / DKC * DKC;
-    splits = (batch + rows_per - 1) / rows_per;
-    const bool hh_in_tiles = fused != nullptr && dw_in_tiles_pays(H, tiles);
-    // workspace: per net g1 [B, H] | g0 [B, H] | ls_part [tiles, PA_MAX] | db_part [tiles, 2H + PA_MAX] |
-    // thin_part [tiles, IN H + H A]; then partial [splits, Ptot]
-    float *w = ws;
-    for (int i = 0; i < n_nets; ++i) {
-        io.n[i].g1 = w; w += (size_t)batch * H;
-        io.n[i].g0 = w; w += (size_t)batch * H;
-        io.n[i].ls_part = w; w += (size_t)tiles * PA_MAX;
-        io.n[i].db_part = w; w += (size_t)tiles * (2 * H + PA_MAX);
-        // (the fused forward + backward kernel may leave the tile's dW1 there as well)
-        io.n[i].thin_stride = IN * H + H * descs[i]->layers[2].out_dim + (hh_in_tiles ? H * H : 0);
-        io.n[i].thin_part = w; w += (size_t)tiles * (size_t)io.n[i].thin_stride;
-    }
-    float *partial = w;
-    FwdLoss fl{};
-    if (fused != nullptr) {
-        fl = *fused;
-        fl.enabled = 1;
-        fl.dw_in_tiles = hh_in_tiles ? 1 : 0;
-        fused = &fl;
-    }
-    if (H == 256 && act == 1) launch_bwd_t<256, 1>(ctx, batch, IN, io, n_nets, fused);
-    else if (H == 256) launch_bwd_t<256, 2>(ctx, batch, IN, io, n_nets, fused);
-    else if (H == 128 && act == 1) launch_bwd_t<128, 1>(ctx, batch, IN, io, n_nets, fused);
-    else if (H == 128) launch_bwd_t<128, 2>(ctx, batch, IN, io, n_nets, fused);
-    else if (act == 1) launch_bwd_t<64, 1>(ctx, batch, IN, io, n_nets, fused);
-    else launch_bwd_t<64, 2>(ctx, batch, IN, io, n_nets, fused);
-    MRL_CHECK_LAUNCH();
+// batch splits of the weight-gradient launch: slices of whole k-chunks
+static void dw_splits(int batch, int *splits, int *rows_per) {
+    int s = std::max(1, std::min(32, batch / 256));
+    *rows_per = ((batch + s - 1) / s + DKC - 1) / DKC * DKC;
+    *splits = (batch + *rows_per - 1) / *rows_per;
+}
+
+// What follows the row tiles: the H x H weight gradients (X[i] = layer-1 inputs [batch, xs], io.n[i].g1) unless the
+// tiles left them (hh_in_tiles), then the sums over tiles and batch splits into the flat gradients.
+static int dw_and_sum(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, int batch, const Mlp3Nets &io,
+                      const float *const *X, int xs, int tiles, bool hh_in_tiles, float *partial, int splits, int rows_per,
+                      float *const *grads, float *sq_part, int *sq_blocks) {
+    const int IN = descs[0]->layers[0].in_dim, H = descs[0]->layers[0].out_dim;
     DwSet dw;
-    dw.n = n_nets;   // the H x H layer of each net; the thin layers come out of the dx kernel
+    dw.n = n_nets;   // the H x H layer of each net; the thin layers come out of the row tiles
     SumNets sn{};
     sn.n = n_nets;
     sn.IN = IN;
@@ -980,13 +578,11 @@ int mlp3_backward_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, 
     int base = 0, total_tiles = 0;
     for (int i = 0; i < n_nets; ++i) {
         const Mlp3Net &nn = io.n[i];
-        const int A = nn.A;
-        const float *c1 = nn.cache + (size_t)batch * (IN + H);
         DwProblem &p = dw.p[i];
-        p.X = c1; p.xs = 2 * H; p.G = nn.g1; p.gs = H; p.K = H; p.N = H; p.poff = base + (IN + 1) * H;
+        p.X = X[i]; p.xs = xs; p.G = nn.g1; p.gs = H; p.K = H; p.N = H; p.poff = base + (IN + 1) * H;
         p.tiles_n = (H + DBN - 1) / DBN;
         p.tiles = p.tiles_n * ((H + DBM - 1) / DBM);
-        p.vec = (H % 64 == 0 && reinterpret_cast<uintptr_t>(c1) % 16 == 0 &&
+        p.vec = (H % 64 == 0 && reinterpret_cast<uintptr_t>(X[i]) % 16 == 0 &&
                  reinterpret_cast<uintptr_t>(nn.g1) % 16 == 0) ? 1 : 0;
         total_tiles += p.tiles;
         sn.grads[i] = grads[i];
@@ -995,7 +591,7 @@ int mlp3_backward_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, 
         sn.thin_part[i] = nn.thin_part;
         sn.thin_stride[i] = nn.thin_stride;
         sn.P[i] = net_P(*descs[i]);
-        sn.A[i] = A;
+        sn.A[i] = nn.A;
         sn.gauss[i] = nn.gauss;
         base += sn.P[i];
     }
@@ -1013,13 +609,123 @@ int mlp3_backward_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, 
     return MRL_OK;
 }
 
+// backward (parameter gradients only) of one or two nets: io.n[i].grad_out / params / cache in,
+// grads[i] out; ws as sized by mlp3_backward_ws
+int mlp3_backward_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, int batch, Mlp3Nets io,
+                    float *const *grads, float *ws) {
+    int H = 0, act = 0;
+    bool gauss = false;
+    for (int i = 0; i < n_nets; ++i) {
+        if (!mlp3_fusable(*descs[i], &H, &act, &gauss)) return MRL_E_UNSUPPORTED;
+        io.n[i].A = descs[i]->layers[2].out_dim;
+        io.n[i].gauss = gauss ? 1 : 0;
+        // the W1 rows are staged with 16-byte loads
+        const int IN = descs[i]->layers[0].in_dim;
+        if (reinterpret_cast<uintptr_t>(io.n[i].params + IN * H + H) % 16 != 0) return MRL_E_UNSUPPORTED;
+    }
+    if (n_nets == 2 && !mlp3_pair_fusable(*descs[0], *descs[1])) return MRL_E_UNSUPPORTED;
+    const int IN = descs[0]->layers[0].in_dim;
+    const int tiles = (batch + PR - 1) / PR;
+    int splits, rows_per;
+    dw_splits(batch, &splits, &rows_per);
+    // workspace: per net g1 [B, H] | g0 [B, H] | ls_part [tiles, PA_MAX] | db_part [tiles, 2H + PA_MAX] |
+    // thin_part [tiles, IN H + H A]; then partial [splits, Ptot]
+    float *w = ws;
+    const float *X[2];
+    for (int i = 0; i < n_nets; ++i) {
+        io.n[i].g1 = w; w += (size_t)batch * H;
+        io.n[i].g0 = w; w += (size_t)batch * H;
+        io.n[i].ls_part = w; w += (size_t)tiles * PA_MAX;
+        io.n[i].db_part = w; w += (size_t)tiles * (2 * H + PA_MAX);
+        io.n[i].thin_stride = IN * H + H * descs[i]->layers[2].out_dim;
+        io.n[i].thin_part = w; w += (size_t)tiles * (size_t)io.n[i].thin_stride;
+        X[i] = io.n[i].cache + (size_t)batch * (IN + H);
+    }
+    if (H == 256 && act == 1) launch_bwd_t<256, 1>(ctx, batch, IN, io, n_nets);
+    else if (H == 256) launch_bwd_t<256, 2>(ctx, batch, IN, io, n_nets);
+    else if (H == 128 && act == 1) launch_bwd_t<128, 1>(ctx, batch, IN, io, n_nets);
+    else if (H == 128) launch_bwd_t<128, 2>(ctx, batch, IN, io, n_nets);
+    else if (act == 1) launch_bwd_t<64, 1>(ctx, batch, IN, io, n_nets);
+    else launch_bwd_t<64, 2>(ctx, batch, IN, io, n_nets);
+    MRL_CHECK_LAUNCH();
+    return dw_and_sum(ctx, descs, n_nets, batch, io, X, 2 * H, tiles, false, w, splits, rows_per, grads, nullptr, nullptr);
+}
+
+// carves (and if need be grows) the context's workspace for the fused update of two nets
+int mlp3_update_ws(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int batch, const float *const *params, UpdateWs *out) {
+    const int H = descs[0]->layers[0].out_dim, IN = descs[0]->layers[0].in_dim;
+    UpdateWs &u = *out;
+    u = UpdateWs{};
+    u.rows = fb_tile_rows(ctx->n_cus, H, batch);
+    u.tiles = (batch + u.rows - 1) / u.rows;
+    u.dw_in_tiles = dw_in_tiles_pays(H, batch);
+    dw_splits(batch, &u.splits, &u.rows_per);
+    size_t need = 0, P = 0;
+    float *base = nullptr;
+    for (int pass = 0; pass < 2; ++pass) {   // sizes, then pointers (every piece a multiple of four floats)
+        size_t at = 0;
+        auto take = [&](size_t floats) {
+            float *p = pass ? base + at : nullptr;
+            at += (floats + 3) / 4 * 4;
+            return p;
+        };
+        P = 0;
+        for (int i = 0; i < 2; ++i) {
+            const int A = descs[i]->layers[2].out_dim;
+            u.split.w1[i] = params[i] + IN * H + H;
+            u.split.wf[i] = reinterpret_cast<unsigned short *>(take(split_elems(H) / 2));
+            u.split.wb[i] = reinterpret_cast<unsigned short *>(take(split_elems(H) / 2));
+            if (!u.dw_in_tiles) {
+                u.net[i].g1 = take((size_t)batch * H);
+                u.net[i].h1 = take((size_t)batch * H);
+            }
+            u.net[i].ls_part = take((size_t)u.tiles * PA_MAX);
+            u.net[i].db_part = take((size_t)u.tiles * (2 * H + PA_MAX));
+            u.net[i].thin_stride = IN * H + H * A + (u.dw_in_tiles ? H * H : 0);
+            u.net[i].thin_part = take((size_t)u.tiles * (size_t)u.net[i].thin_stride);
+            P += net_P(*descs[i]);
+        }
+        u.partial = take(u.dw_in_tiles ? 4 : (size_t)u.splits * P);
+        need = at;
+        if (pass == 0) {
+            int rc = mlp_ensure_ws(ctx, need, &base);
+            if (rc) return rc;
+        }
+    }
+    return MRL_OK;
+}
+
+int mlp3_update_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int batch, Mlp3Nets io, const UpdateWs &ws,
+                  float *const *grads, float *sq_part, int *sq_blocks, const FwdLoss &loss) {
+    int H = 0, act = 0;
+    bool gauss = false;
+    const float *X[2];
+    for (int i = 0; i < 2; ++i) {
+        if (!mlp3_fusable(*descs[i], &H, &act, &gauss)) return MRL_E_UNSUPPORTED;
+        Mlp3Net &nn = io.n[i];
+        const Mlp3Net &from = ws.net[i];
+        nn.A = descs[i]->layers[2].out_dim;
+        nn.gauss = gauss ? 1 : 0;
+        nn.g1 = from.g1; nn.h1 = from.h1; nn.ls_part = from.ls_part; nn.db_part = from.db_part;
+        nn.thin_part = from.thin_part; nn.thin_stride = from.thin_stride;
+        nn.wf = ws.split.wf[i]; nn.wb = ws.split.wb[i];
+        X[i] = nn.h1;
+    }
+    FwdLoss fl = loss;
+    fl.dw_in_tiles = ws.dw_in_tiles ? 1 : 0;
+    int rc = launch_fb(ctx, H, act, batch, descs[0]->layers[0].in_dim, ws.rows, io, fl);
+    if (rc) return rc;
+    return dw_and_sum(ctx, descs, 2, batch, io, X, H, ws.tiles, ws.dw_in_tiles, ws.partial, ws.splits, ws.rows_per, grads,
+                      sq_part, sq_blocks);
+}
+
 int mlp3_backward(mrl_ctx *ctx, const mrl_mlp_desc &d, int batch, const float *grad_out, const float *params,
                   const float *cache, float *grads, float *ws) {
     Mlp3Nets io{};
     io.n[0].grad_out = grad_out; io.n[0].params = params; io.n[0].cache = const_cast<float *>(cache);
     const mrl_mlp_desc *ds[1] = {&d};
     float *gs[1] = {grads};
-    return mlp3_backward_n(ctx, ds, 1, batch, io, gs, ws, nullptr, nullptr);
+    return mlp3_backward_n(ctx, ds, 1, batch, io, gs, ws);
 }
 
 }  // namespace mrl

@@ -4,9 +4,9 @@
 // forward, loss gradients, KL test, backward, global-norm clip, Adam (and the log_std clamp).
 // The actor and the critic do not depend on each other inside a minibatch, so when both have one
 // of the fused shapes they run side by side in every launch, and a row tile never leaves its
-// workgroup between the forward pass and the way back: 4 launches per minibatch (forward + loss
-// gradients + KL test + backward dx; dW; sum; clip + Adam) instead of about 40.  The minibatch is
-// not gathered: the forward reads its rows from the rollout through the indices and the loss
+// workgroup between the forward pass and the way back (mrl_fb.hip): 3 or 4 launches per minibatch (forward + loss
+// gradients + KL test + backward; dW of the hidden layer, where the tiles do not leave it; sum; clip + Adam) instead
+// of about 40.  The minibatch is not gathered: the forward reads its rows from the rollout through the indices and the loss
 // normalises the advantage with statistics computed ahead (once per epoch for all minibatches).
 // Other net shapes go layer by layer: gather + normalise, forward, loss gradients + KL test,
 // backward, clip + Adam.
@@ -20,6 +20,7 @@
 // that were applied, for the host's optimiser step counters.
 #include "mrl_host.hpp"
 #include "mrl_device.hpp"
+#include "mlp_split.hpp"
 #include "mlp3.hpp"
 #include "ppo_grads.hpp"
 
@@ -239,70 +240,160 @@ __global__ __launch_bounds__(UTPB) void sq_partial2_kernel(AdamNets nets, float 
     if (threadIdx.x == 0) partial[blockIdx.y * gridDim.x + blockIdx.x] = s;
 }
 
-// global-norm clip (ppo.mojo:382-534; actor and critic separately) + Adam (adam.mojo:52-105)
-// + log_std clamp (kernels.mojo:842-873); grid = (blocks, nets).  Does nothing once stop[0] != 0.
-// kl_part != nullptr: the KL early-stop test of this minibatch has not been made yet: kl_part[0 .. kl_n)
-// hold the row tiles' sums of the per-sample estimates.  Every workgroup adds them up in the same order,
-// so all of them come to the same verdict; workgroup (0, 0) records it (stop[0] raised and sticky,
-// stop[1] = the mean's bits).
-__global__ __launch_bounds__(UTPB) void clip_adam2_kernel(AdamNets nets, const float *__restrict__ partial,
-                                                          int nb, int part_stride, float max_norm, float beta1,
-                                                          float beta2,
-                                                          float omb1, float omb2, float eps,
-                                                          int32_t *__restrict__ stop,
-                                                          const float *__restrict__ kl_part, int kl_n, int kl_mb,
-                                                          float target_kl) {
-    __shared__ float smem[4];
-    __shared__ float scale_s;
+struct AdamArgs {
+    AdamNets nets;
+    const float *partial;   // sums of squares of the gradients, [net * part_stride + block], nb blocks
+    int nb, part_stride;
+    float max_norm, beta1, beta2, omb1, omb2, eps;
+    int32_t *stop;          // the KL early stop's flag words (null: no test)
+    // not null: the KL early-stop test of this minibatch has not been made yet: kl_part[0 .. kl_n) hold the row
+    // tiles' sums of the per-sample estimates
+    const float *kl_part;
+    int kl_n, kl_mb;
+    float target_kl;
+};
+
+// Whether the update is applied (it is not once stop[0] != 0), and the factor of the global-norm clip (ppo.mojo:382-534;
+// actor and critic separately).  Every workgroup adds the tiles' KL sums up in the same order, so all of them come to the
+// same verdict; workgroup (0, 0) records it (stop[0] raised and sticky, stop[1] = the mean's bits, stop[2] counts the
+// updates applied).  Both sums are taken side by side.
+MRL_DEV bool clip_verdict(const AdamArgs &a, float *smem, float &scale) {
     __shared__ int stop_s;
-    if (stop != nullptr && stop[0] != 0) return;
-    if (stop != nullptr && kl_part != nullptr) {
-        if (threadIdx.x < 64) {
-            float sum = 0.0f;
-            for (int i = threadIdx.x; i < kl_n; i += 64) sum += kl_part[i];
+    if (a.stop != nullptr && a.stop[0] != 0) return false;
+    scale = 1.0f;
+    const bool test = a.stop != nullptr && a.kl_part != nullptr;
+    float s = 0.0f;
+    if (a.max_norm > 0.0f)
+        for (int i = threadIdx.x; i < a.nb; i += UTPB) s += a.partial[blockIdx.y * a.part_stride + i];
+    if (test && threadIdx.x < 64) {
+        float sum = 0.0f;
+        for (int i = threadIdx.x; i < a.kl_n; i += 64) sum += a.kl_part[i];
 #pragma unroll
-            for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
-            if (threadIdx.x == 0) {
-                const float mean = sum / (float)kl_mb;
-                stop_s = mean > target_kl;
-                if (blockIdx.x == 0 && blockIdx.y == 0) {
-                    stop[1] = __float_as_int(mean);
-                    if (mean > target_kl) stop[0] = 1;
-                }
+        for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+        if (threadIdx.x == 0) {
+            const float mean = sum / (float)a.kl_mb;
+            stop_s = mean > a.target_kl;
+            if (blockIdx.x == 0 && blockIdx.y == 0) {
+                a.stop[1] = __float_as_int(mean);
+                if (mean > a.target_kl) a.stop[0] = 1;
             }
         }
-        __syncthreads();
-        if (stop_s) return;
     }
-    const AdamNet &a = nets.n[blockIdx.y];
-    float scale = 1.0f;
-    if (max_norm > 0.0f) {
-        float s = 0.0f;
-        for (int i = threadIdx.x; i < nb; i += UTPB) s += partial[blockIdx.y * part_stride + i];
-        s = u_block_sum<4>(s, smem);
-        if (threadIdx.x == 0) {
-            const float norm = sqrtf(s);
-            scale_s = norm > max_norm ? max_norm / (norm + 1e-8f) : 1.0f;
-        }
-        __syncthreads();
-        scale = scale_s;
+    s = u_block_sum<4>(s, smem);
+    if (test && stop_s) return false;
+    if (a.max_norm > 0.0f) {
+        const float norm = sqrtf(s);
+        scale = norm > a.max_norm ? a.max_norm / (norm + 1e-8f) : 1.0f;
     }
-    if (stop != nullptr && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) stop[2] = stop[2] + 1;
+    if (a.stop != nullptr && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) a.stop[2] = a.stop[2] + 1;
+    return true;
+}
+
+// Adam (adam.mojo:52-105) on one parameter: gi = its clipped gradient
+MRL_DEV float adam_one(const AdamArgs &a, const AdamNet &net, float p, float gi, float &m, float &v) {
+    m = a.beta1 * m + a.omb1 * gi;
+    v = a.beta2 * v + a.omb2 * gi * gi;
+    const float m_hat = m / net.bc1, v_hat = v / net.bc2;
+    return p - net.lr * m_hat / (sqrtf(v_hat) + a.eps);
+}
+
+// clip + Adam + log_std clamp (kernels.mojo:842-873) of element i
+MRL_DEV void adam_element(const AdamArgs &a, const AdamNet &net, int i, float p0, float g0, float2 mv, float scale) {
+    const float gi = g0 * scale;
+    net.g[i] = gi;
+    float p = adam_one(a, net, p0, gi, mv.x, mv.y);
+    net.state[i] = mv;
+    if (i >= net.clamp_off && i < net.clamp_off + net.clamp_n) p = p < -5.0f ? -5.0f : (p > 2.0f ? 2.0f : p);
+    net.p[i] = p;
+}
+
+// any nets; grid = (blocks, nets)
+__global__ __launch_bounds__(UTPB) void clip_adam2_kernel(AdamArgs a) {
+    __shared__ float smem[4];
+    const AdamNet &net = a.nets.n[blockIdx.y];
     const int i = blockIdx.x * UTPB + threadIdx.x;
-    if (i >= a.n) return;
-    const float gi = a.g[i] * scale;
-    a.g[i] = gi;
-    const float2 mv = a.state[i];
-    const float m_new = beta1 * mv.x + omb1 * gi;
-    const float v_new = beta2 * mv.y + omb2 * gi * gi;
-    a.state[i] = make_float2(m_new, v_new);
-    const float m_hat = m_new / a.bc1, v_hat = v_new / a.bc2;
-    float p = a.p[i] - a.lr * m_hat / (sqrtf(v_hat) + eps);
-    if (i >= a.clamp_off && i < a.clamp_off + a.clamp_n) {
-        if (p < -5.0f) p = -5.0f;
-        else if (p > 2.0f) p = 2.0f;
+    float p = 0.0f, g = 0.0f;
+    float2 mv = make_float2(0.0f, 0.0f);
+    if (i < net.n) { p = net.p[i]; g = net.g[i]; mv = net.state[i]; }
+    float scale;
+    if (!clip_verdict(a, smem, scale)) return;
+    if (i < net.n) adam_element(a, net, i, p, g, mv, scale);
+}
+
+// The fused nets (hidden width H, W1 at offset o1): the first H * H / 2048 workgroups take eight consecutive columns of
+// W1 per thread and keep the split operand copies of mlp_split.hpp in step (null: not kept); the others take the
+// remaining parameters one per thread.  Everything that does not depend on the verdict is requested ahead of it.
+template <int H>
+__global__ __launch_bounds__(UTPB) void clip_adam_split_kernel(AdamArgs a, int o1, SplitNets sp) {
+    constexpr int WB = H * H / (8 * UTPB), ROWS = 8 * UTPB / H, TLD = H + 4;
+    __shared__ float smem[4];
+    __shared__ __align__(16) float tile[ROWS * TLD];
+    const AdamNet &net = a.nets.n[blockIdx.y];
+    const int t = threadIdx.x;
+    float scale;
+    if (blockIdx.x >= WB) {
+        int i = (blockIdx.x - WB) * UTPB + t;
+        if (i >= o1) i += H * H;
+        float p = 0.0f, g = 0.0f;
+        float2 mv = make_float2(0.0f, 0.0f);
+        if (i < net.n) { p = net.p[i]; g = net.g[i]; mv = net.state[i]; }
+        if (!clip_verdict(a, smem, scale)) return;
+        if (i < net.n) adam_element(a, net, i, p, g, mv, scale);
+        return;
     }
-    a.p[i] = p;
+    const int rl = t / (H / 8), c8 = t % (H / 8), row = blockIdx.x * ROWS + rl;
+    const size_t off = (size_t)o1 + (size_t)row * H + 8 * c8;
+    f32x4 p[2], g[2], st[4];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        p[k] = *reinterpret_cast<const f32x4 *>(net.p + off + 4 * k);
+        g[k] = *reinterpret_cast<const f32x4 *>(net.g + off + 4 * k);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) st[k] = *reinterpret_cast<const f32x4 *>(net.state + off + 2 * k);
+    if (!clip_verdict(a, smem, scale)) return;
+    f32x8 pn;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const float gi = g[k >> 2][k & 3] * scale;
+        g[k >> 2][k & 3] = gi;
+        float m = st[k >> 1][2 * (k & 1)], v = st[k >> 1][2 * (k & 1) + 1];
+        pn[k] = adam_one(a, net, p[k >> 2][k & 3], gi, m, v);
+        st[k >> 1][2 * (k & 1)] = m;
+        st[k >> 1][2 * (k & 1) + 1] = v;
+    }
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        *reinterpret_cast<f32x4 *>(net.g + off + 4 * k) = g[k];
+        const f32x4 q = {pn[4 * k], pn[4 * k + 1], pn[4 * k + 2], pn[4 * k + 3]};
+        *reinterpret_cast<f32x4 *>(net.p + off + 4 * k) = q;
+        *reinterpret_cast<f32x4 *>(tile + rl * TLD + 8 * c8 + 4 * k) = q;
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) *reinterpret_cast<f32x4 *>(net.state + off + 2 * k) = st[k];
+    if (sp.wf[0] == nullptr) return;
+    bf16x8 pc[SPLIT];
+    split8(pn, pc);
+    unsigned short *wb = sp.wb[blockIdx.y], *wf = sp.wf[blockIdx.y];
+#pragma unroll
+    for (int i = 0; i < SPLIT; ++i)
+        *reinterpret_cast<bf16x8 *>(wb + split_frag<H>(c8 >> 2, row >> 4, i, (c8 & 3) * 16 + (row & 15))) = pc[i];
+    __syncthreads();
+    const int col = t % H, kg = t / H, k8 = blockIdx.x * (ROWS / 8) + kg;
+    f32x8 x;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = tile[(8 * kg + j) * TLD + col];
+    split8(x, pc);
+#pragma unroll
+    for (int i = 0; i < SPLIT; ++i)
+        *reinterpret_cast<bf16x8 *>(wf + split_frag<H>(k8 >> 2, col >> 4, i, (k8 & 3) * 16 + (col & 15))) = pc[i];
+}
+
+template <int H>
+static void launch_adam_split(hipStream_t st, const AdamArgs &a, int o1, const SplitNets &sp) {
+    const int nmax = std::max(a.nets.n[0].n, a.nets.n[1].n);
+    hipLaunchKernelGGL(clip_adam_split_kernel<H>, dim3(H * H / (8 * UTPB) + grid_for(nmax - H * H, UTPB), 2), dim3(UTPB), 0,
+                       st, a, o1, sp);
 }
 
 }  // namespace mrl
@@ -338,126 +429,158 @@ static int update_check(const mrl_update *u, const char *who) {
 // advantage statistics of up to STATS_MAX minibatches
 constexpr int SCR_KL = 0, SCR_ARRIVED = 1024, SCR_SQ = 2048, SCR_STATS = 4096, STATS_MAX = 2048;
 
+// both nets of the fused shapes, buffers that 16-byte accesses can reach, a KL sum per row tile
 static bool update_paired(const mrl_update *u) {
-    return mlp3_pair_fusable(u->actor, u->critic) && reinterpret_cast<uintptr_t>(u->actor_params) % 16 == 0 &&
-           reinterpret_cast<uintptr_t>(u->critic_params) % 16 == 0 && (u->minibatch + 31) / 32 <= 1024;
+    uintptr_t all = 0;
+    for (const float *p : {u->actor_params, u->critic_params, u->actor_grads, u->critic_grads, u->actor_state, u->critic_state})
+        all |= reinterpret_cast<uintptr_t>(p);
+    return mlp3_pair_fusable(u->actor, u->critic) && all % 16 == 0 && (u->minibatch + 31) / 32 <= 1024;
 }
 
-// stats: {mean, std} of this minibatch's advantages on the device, already enqueued (paired nets
-// only); null: worked out here
-static int update_minibatch(mrl_ctx *ctx, const mrl_update *u, const int32_t *indices, int actor_t, int critic_t,
-                            const float *stats) {
-    int rc;
-    const int mb = u->minibatch, head = mrl_mlp_out_dim(&u->actor);
+static void adam_args(const mrl_update *u, int actor_t, int critic_t, AdamArgs &a) {
     const int Pa = mrl_mlp_param_size(&u->actor), Pc = mrl_mlp_param_size(&u->critic);
+    auto fill = [&](AdamNet &n, float *p, float *g, float *st, int size, double lr, int t) {
+        n.p = p; n.g = g; n.state = reinterpret_cast<float2 *>(st); n.n = size; n.lr = (float)lr;
+        // bias corrections in fp64 then rounded, as the host code of the reference does
+        n.bc1 = (float)(1.0 - pow(u->beta1, (double)t));
+        n.bc2 = (float)(1.0 - pow(u->beta2, (double)t));
+        n.clamp_off = 0; n.clamp_n = 0;
+    };
+    fill(a.nets.n[0], u->actor_params, u->actor_grads, u->actor_state, Pa, u->actor_lr, actor_t);
+    fill(a.nets.n[1], u->critic_params, u->critic_grads, u->critic_state, Pc, u->critic_lr, critic_t);
+    if (u->continuous) { a.nets.n[0].clamp_off = Pa - u->act_width; a.nets.n[0].clamp_n = u->act_width; }
+    a.max_norm = u->max_grad_norm;
+    a.beta1 = (float)u->beta1; a.beta2 = (float)u->beta2;
+    a.omb1 = (float)(1.0 - u->beta1); a.omb2 = (float)(1.0 - u->beta2); a.eps = (float)u->eps;
+    a.stop = u->target_kl > 0.0f ? u->kl_flag : nullptr;
+    a.kl_mb = u->minibatch;
+    a.target_kl = u->target_kl;
+}
+
+// One minibatch of the fused nets; stats: {mean, std} of its advantages on the device (null: not normalised).
+// ws.split holds the hidden layers' current weights; keep_split: it is to hold the updated ones afterwards.
+static int update_minibatch_paired(mrl_ctx *ctx, const mrl_update *u, const int32_t *indices, int actor_t, int critic_t,
+                                   const float *stats, const UpdateWs &ws, bool keep_split) {
     const bool cont = u->continuous != 0;
-    const bool paired = update_paired(u);
-
-    if (paired && u->norm_adv_per_minibatch && stats == nullptr) {
-        float *st = ctx->upd_scratch + SCR_STATS;
-        hipLaunchKernelGGL(adv_stats_kernel, dim3(1), dim3(UTPB), 0, ctx->stream, indices, u->advantages, mb, st);
-        MRL_CHECK_LAUNCH();
-        stats = st;
-    }
-    if (!paired) {
-        GatherArgs g{indices, u->r_obs, u->r_actions, u->advantages, u->returns, u->r_log_probs, u->r_values,
-                     u->mb_obs, u->mb_actions, u->mb_adv, u->mb_ret, u->mb_logp, u->mb_val,
-                     mb, u->obs_dim, u->act_width, u->norm_adv_per_minibatch};
-        MRL_CHECK_ARG(u->act_width <= u->obs_dim, "mrl_ppo_update_minibatch: action wider than observation");
-        hipLaunchKernelGGL(gather_norm_kernel, dim3(grid_for((long)mb * u->obs_dim, UTPB) + 1), dim3(UTPB), 0,
-                           ctx->stream, g);
-        MRL_CHECK_LAUNCH();
-    }
-
+    const int mb = u->minibatch, head = mrl_mlp_out_dim(&u->actor);
     const mrl_mlp_desc *descs[2] = {&u->actor, &u->critic};
     Mlp3Nets io{};
-    io.n[0].x = u->mb_obs; io.n[0].params = u->actor_params; io.n[0].out = u->actor_out; io.n[0].cache = u->actor_cache;
-    io.n[1].x = u->mb_obs; io.n[1].params = u->critic_params; io.n[1].out = u->values; io.n[1].cache = u->critic_cache;
+    io.n[0].params = u->actor_params; io.n[0].out = u->actor_out;
+    io.n[1].params = u->critic_params; io.n[1].out = u->values;
     FwdLoss fl{};
-    if (paired) {
-        // both nets go forward straight from the rollout rows, on to their loss gradients and the KL
-        // test and back again in one launch per row tile (mlp3_backward_n below)
-        fl.idx = indices;
-        fl.r_obs = u->r_obs; fl.r_act = u->r_actions; fl.r_adv = u->advantages; fl.r_ret = u->returns;
-        fl.r_logp = u->r_log_probs; fl.r_val = u->r_values;
-        fl.adv_stats = u->norm_adv_per_minibatch ? stats : nullptr;
-        fl.g_actor_out = u->g_actor_out; fl.g_values = u->g_values; fl.kl = u->kl;
-        fl.kl_part = ctx->upd_scratch + SCR_KL;
-        fl.kl_flag = u->target_kl > 0.0f ? u->kl_flag : nullptr;
-        fl.mb = mb; fl.A = cont ? u->act_width : head; fl.continuous = cont ? 1 : 0;
-        fl.clip_value = u->clip_value ? 1 : 0;
-        fl.clip_eps = u->clip_epsilon; fl.ent_coef = u->entropy_coef; fl.value_coef = u->value_loss_coef;
-        fl.target_kl = u->target_kl;
-    } else {
-        rc = mrl_mlp_forward(ctx, &u->actor, mb, u->mb_obs, u->actor_params, u->actor_out, u->actor_cache);
-        if (rc) return rc;
-        rc = mrl_mlp_forward(ctx, &u->critic, mb, u->mb_obs, u->critic_params, u->values, u->critic_cache);
+    fl.idx = indices;
+    fl.r_obs = u->r_obs; fl.r_act = u->r_actions; fl.r_adv = u->advantages; fl.r_ret = u->returns;
+    fl.r_logp = u->r_log_probs; fl.r_val = u->r_values;
+    fl.adv_stats = u->norm_adv_per_minibatch ? stats : nullptr;
+    fl.g_actor_out = u->g_actor_out; fl.g_values = u->g_values; fl.kl = u->kl;
+    fl.kl_part = ctx->upd_scratch + SCR_KL;
+    fl.kl_flag = u->target_kl > 0.0f ? u->kl_flag : nullptr;
+    fl.mb = mb; fl.A = cont ? u->act_width : head; fl.continuous = cont ? 1 : 0;
+    fl.clip_value = u->clip_value ? 1 : 0;
+    fl.clip_eps = u->clip_epsilon; fl.ent_coef = u->entropy_coef; fl.value_coef = u->value_loss_coef;
+    fl.target_kl = u->target_kl;
+    float *grads[2] = {u->actor_grads, u->critic_grads};
+    int sq_blocks = 0;   // > 0: the sums over the tiles already left the sum-of-squares partials
+    int rc = mlp3_update_n(ctx, descs, mb, io, ws, grads, u->max_grad_norm > 0.0f ? ctx->upd_scratch + SCR_SQ : nullptr,
+                           &sq_blocks, fl);
+    if (rc) return rc;
+    AdamArgs a{};
+    adam_args(u, actor_t, critic_t, a);
+    a.partial = ctx->upd_scratch + SCR_SQ;
+    a.nb = sq_blocks;
+    a.part_stride = 1024;
+    a.kl_part = u->target_kl > 0.0f ? ctx->upd_scratch + SCR_KL : nullptr;
+    a.kl_n = ws.tiles;
+    const int H = u->actor.layers[0].out_dim, o1 = (u->obs_dim + 1) * H;
+    SplitNets sp{};
+    if (keep_split) sp = ws.split;
+    if (H == 256) launch_adam_split<256>(ctx->stream, a, o1, sp);
+    else if (H == 128) launch_adam_split<128>(ctx->stream, a, o1, sp);
+    else launch_adam_split<64>(ctx->stream, a, o1, sp);
+    MRL_CHECK_LAUNCH();
+    return MRL_OK;
+}
+
+// One minibatch of any other nets, layer by layer.
+static int update_minibatch_layers(mrl_ctx *ctx, const mrl_update *u, const int32_t *indices, int actor_t, int critic_t) {
+    int rc;
+    const int mb = u->minibatch, head = mrl_mlp_out_dim(&u->actor);
+    const bool cont = u->continuous != 0;
+    GatherArgs g{indices, u->r_obs, u->r_actions, u->advantages, u->returns, u->r_log_probs, u->r_values,
+                 u->mb_obs, u->mb_actions, u->mb_adv, u->mb_ret, u->mb_logp, u->mb_val,
+                 mb, u->obs_dim, u->act_width, u->norm_adv_per_minibatch};
+    MRL_CHECK_ARG(u->act_width <= u->obs_dim, "mrl_ppo_update_minibatch: action wider than observation");
+    hipLaunchKernelGGL(gather_norm_kernel, dim3(grid_for((long)mb * u->obs_dim, UTPB) + 1), dim3(UTPB), 0,
+                       ctx->stream, g);
+    MRL_CHECK_LAUNCH();
+    rc = mrl_mlp_forward(ctx, &u->actor, mb, u->mb_obs, u->actor_params, u->actor_out, u->actor_cache);
+    if (rc) return rc;
+    rc = mrl_mlp_forward(ctx, &u->critic, mb, u->mb_obs, u->critic_params, u->values, u->critic_cache);
+    if (rc) return rc;
+    const int nblk = grid_for(mb, UTPB);
+    const bool test = u->target_kl > 0.0f && nblk <= 1024;
+    LossArgs l{u->actor_out, u->mb_logp, u->mb_adv, u->mb_actions, u->values, u->mb_val, u->mb_ret,
+               u->g_actor_out, u->g_values, u->kl, ctx->upd_scratch + SCR_KL,
+               reinterpret_cast<int *>(ctx->upd_scratch + SCR_ARRIVED), test ? u->kl_flag : nullptr,
+               mb, cont ? u->act_width : head, cont ? 1 : 0, u->clip_value ? 1 : 0,
+               u->clip_epsilon, u->entropy_coef, u->value_loss_coef, u->target_kl};
+    hipLaunchKernelGGL(loss_grads_kernel, dim3(nblk, 2), dim3(UTPB), 0, ctx->stream, l);
+    MRL_CHECK_LAUNCH();
+    if (u->target_kl > 0.0f && !test) {
+        rc = mrl_kl_check(ctx, u->kl, mb, u->target_kl, u->kl_flag);
         if (rc) return rc;
     }
+    rc = mrl_mlp_backward(ctx, &u->actor, mb, u->g_actor_out, u->actor_params, u->actor_cache, u->actor_grads,
+                          nullptr);
+    if (rc) return rc;
+    rc = mrl_mlp_backward(ctx, &u->critic, mb, u->g_values, u->critic_params, u->critic_cache, u->critic_grads,
+                          nullptr);
+    if (rc) return rc;
+    AdamArgs a{};
+    adam_args(u, actor_t, critic_t, a);
+    const int nmax = std::max(a.nets.n[0].n, a.nets.n[1].n);
+    if (u->max_grad_norm > 0.0f) {
+        float *part = ctx->reduce_scratch + 1024;   // [2][nb], nb <= 256
+        a.nb = std::min(256, grid_for(nmax, UTPB));
+        a.part_stride = a.nb;
+        a.partial = part;
+        hipLaunchKernelGGL(sq_partial2_kernel, dim3(a.nb, 2), dim3(UTPB), 0, ctx->stream, a.nets, part);
+    }
+    hipLaunchKernelGGL(clip_adam2_kernel, dim3(grid_for(nmax, UTPB), 2), dim3(UTPB), 0, ctx->stream, a);
+    MRL_CHECK_LAUNCH();
+    return MRL_OK;
+}
 
-    if (!paired) {
-        const int nblk = grid_for(mb, UTPB);
-        const bool test = u->target_kl > 0.0f && nblk <= 1024;
-        LossArgs a{u->actor_out, u->mb_logp, u->mb_adv, u->mb_actions, u->values, u->mb_val, u->mb_ret,
-                   u->g_actor_out, u->g_values, u->kl, ctx->upd_scratch,
-                   reinterpret_cast<int *>(ctx->upd_scratch + 1024), test ? u->kl_flag : nullptr,
-                   mb, cont ? u->act_width : head, cont ? 1 : 0, u->clip_value ? 1 : 0,
-                   u->clip_epsilon, u->entropy_coef, u->value_loss_coef, u->target_kl};
-        hipLaunchKernelGGL(loss_grads_kernel, dim3(nblk, 2), dim3(UTPB), 0, ctx->stream, a);
-        MRL_CHECK_LAUNCH();
-        if (u->target_kl > 0.0f && !test) {
-            rc = mrl_kl_check(ctx, u->kl, mb, u->target_kl, u->kl_flag);
+// Minibatches 0 .. n - 1 of `indices`, with step counts t0 + 1 ..
+static int update_minibatches(mrl_ctx *ctx, const mrl_update *u, const int32_t *indices, int n, int actor_t0, int critic_t0) {
+    int rc;
+    if (!update_paired(u)) {
+        for (int k = 0; k < n; ++k) {
+            rc = update_minibatch_layers(ctx, u, indices + (size_t)k * u->minibatch, actor_t0 + k + 1, critic_t0 + k + 1);
             if (rc) return rc;
         }
+        return MRL_OK;
     }
-
-    io.n[0].grad_out = u->g_actor_out;
-    io.n[1].grad_out = u->g_values;
-    float *grads[2] = {u->actor_grads, u->critic_grads};
-    int sq_blocks = 0;   // > 0: the backward pass already left the sum-of-squares partials
-    if (paired) {
-        float *ws = nullptr;
-        rc = mlp_ensure_ws(ctx, mlp3_backward_ws(descs, 2, mb), &ws);
-        if (rc) return rc;
-        rc = mlp3_backward_n(ctx, descs, 2, mb, io, grads, ws,
-                             u->max_grad_norm > 0.0f ? ctx->upd_scratch + SCR_SQ : nullptr, &sq_blocks, &fl);
-        if (rc) return rc;
-    } else {
-        rc = mrl_mlp_backward(ctx, &u->actor, mb, u->g_actor_out, u->actor_params, u->actor_cache, u->actor_grads,
-                              nullptr);
-        if (rc) return rc;
-        rc = mrl_mlp_backward(ctx, &u->critic, mb, u->g_values, u->critic_params, u->critic_cache, u->critic_grads,
-                              nullptr);
+    // the split copies of the hidden layers' weights are made here, from the parameters as the caller left them, and
+    // kept in step by the Adam kernel between this call's minibatches
+    const mrl_mlp_desc *descs[2] = {&u->actor, &u->critic};
+    const float *params[2] = {u->actor_params, u->critic_params};
+    UpdateWs ws;
+    rc = mlp3_update_ws(ctx, descs, u->minibatch, params, &ws);
+    if (rc) return rc;
+    rc = launch_split_weights(ctx, u->actor.layers[0].out_dim, ws.split, 2);
+    if (rc) return rc;
+    float *stats = ctx->upd_scratch + SCR_STATS;
+    for (int k = 0; k < n; ++k) {
+        if (u->norm_adv_per_minibatch && k % STATS_MAX == 0) {   // the advantage statistics of many minibatches in one launch
+            hipLaunchKernelGGL(adv_stats_kernel, dim3(std::min(STATS_MAX, n - k)), dim3(UTPB), 0, ctx->stream,
+                               indices + (size_t)k * u->minibatch, u->advantages, u->minibatch, stats);
+            MRL_CHECK_LAUNCH();
+        }
+        rc = update_minibatch_paired(ctx, u, indices + (size_t)k * u->minibatch, actor_t0 + k + 1, critic_t0 + k + 1,
+                                     stats + 2 * (k % STATS_MAX), ws, k + 1 < n);
         if (rc) return rc;
     }
-
-    AdamNets an{};
-    auto fill = [&](AdamNet &a, float *p, float *g, float *st, int n, double lr, int t) {
-        a.p = p; a.g = g; a.state = reinterpret_cast<float2 *>(st); a.n = n; a.lr = (float)lr;
-        // bias corrections in fp64 then rounded, as the host code of the reference does
-        a.bc1 = (float)(1.0 - pow(u->beta1, (double)t));
-        a.bc2 = (float)(1.0 - pow(u->beta2, (double)t));
-        a.clamp_off = 0; a.clamp_n = 0;
-    };
-    fill(an.n[0], u->actor_params, u->actor_grads, u->actor_state, Pa, u->actor_lr, actor_t);
-    fill(an.n[1], u->critic_params, u->critic_grads, u->critic_state, Pc, u->critic_lr, critic_t);
-    if (cont) { an.n[0].clamp_off = Pa - u->act_width; an.n[0].clamp_n = u->act_width; }
-    const int nmax = std::max(Pa, Pc);
-    int nb = sq_blocks, stride = 1024;
-    const float *part = ctx->upd_scratch + 2048;
-    if (u->max_grad_norm > 0.0f && sq_blocks == 0) {
-        nb = std::min(256, grid_for(nmax, UTPB));
-        stride = nb;
-        float *p2 = ctx->reduce_scratch + 1024;   // [2][nb], nb <= 256
-        hipLaunchKernelGGL(sq_partial2_kernel, dim3(nb, 2), dim3(UTPB), 0, ctx->stream, an, p2);
-        part = p2;
-    }
-    hipLaunchKernelGGL(clip_adam2_kernel, dim3(grid_for(nmax, UTPB), 2), dim3(UTPB), 0, ctx->stream, an, part, nb,
-                       stride, u->max_grad_norm, (float)u->beta1, (float)u->beta2, (float)(1.0 - u->beta1),
-                       (float)(1.0 - u->beta2), (float)u->eps, u->target_kl > 0.0f ? u->kl_flag : nullptr,
-                       paired && u->target_kl > 0.0f ? ctx->upd_scratch + SCR_KL : nullptr, grid_for(mb, 32), mb,
-                       u->target_kl);
-    MRL_CHECK_LAUNCH();
     return MRL_OK;
 }
 
@@ -468,7 +591,7 @@ int mrl_ppo_update_minibatch(mrl_ctx *ctx, const mrl_update *u, const int32_t *i
     if (rc) return rc;
     MRL_CHECK_ARG(indices != nullptr && actor_t >= 1 && critic_t >= 1,
                   "mrl_ppo_update_minibatch: need indices and step counts >= 1");
-    return update_minibatch(ctx, u, indices, actor_t, critic_t, nullptr);
+    return update_minibatches(ctx, u, indices, 1, actor_t - 1, critic_t - 1);
 }
 
 int mrl_minibatch_adv_stats(mrl_ctx *ctx, const int32_t *indices, const float *advantages, int minibatch,
@@ -491,22 +614,7 @@ int mrl_ppo_update_epoch(mrl_ctx *ctx, const mrl_update *u, const int32_t *indic
     if (rc) return rc;
     MRL_CHECK_ARG(n_minibatches >= 0 && actor_t0 >= 0 && critic_t0 >= 0, "mrl_ppo_update_epoch: negative count");
     MRL_CHECK_ARG(n_minibatches == 0 || indices != nullptr, "mrl_ppo_update_epoch: indices is NULL");
-    const bool ahead = update_paired(u) && u->norm_adv_per_minibatch;
-    for (int k0 = 0; k0 < n_minibatches; k0 += STATS_MAX) {
-        const int n = std::min(STATS_MAX, n_minibatches - k0);
-        float *stats = ctx->upd_scratch + SCR_STATS;
-        if (ahead) {   // the advantage statistics of all these minibatches in one launch
-            hipLaunchKernelGGL(adv_stats_kernel, dim3(n), dim3(UTPB), 0, ctx->stream,
-                               indices + (size_t)k0 * u->minibatch, u->advantages, u->minibatch, stats);
-            MRL_CHECK_LAUNCH();
-        }
-        for (int k = k0; k < k0 + n; ++k) {
-            rc = update_minibatch(ctx, u, indices + (size_t)k * u->minibatch, actor_t0 + k + 1, critic_t0 + k + 1,
-                                  ahead ? stats + 2 * (k - k0) : nullptr);
-            if (rc) return rc;
-        }
-    }
-    return MRL_OK;
+    return n_minibatches == 0 ? MRL_OK : update_minibatches(ctx, u, indices, n_minibatches, actor_t0, critic_t0);
 }
 
 }  // extern "C"
