@@ -36,6 +36,15 @@ MRL_DEV float act_deriv_out(float y) {
     return 1.0f;
 }
 
+// sum over the sixteen lanes of a row (DPP rotations within the row), on all of them
+MRL_DEV float row16_sum(float x) {
+    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x128, 0xf, 0xf, false));   // row_ror:8
+    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x124, 0xf, 0xf, false));   // row_ror:4
+    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x122, 0xf, 0xf, false));   // row_ror:2
+    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x121, 0xf, 0xf, false));   // row_ror:1
+    return x;
+}
+
 constexpr int fb_threads(int H) { return H == 64 ? 256 : 512; }
 
 template <int H, int ACT, int RT>
@@ -46,7 +55,7 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
     constexpr int K0 = PIN_MAX / 4;
     constexpr int PF = KS < 3 ? KS : 3;          // k-steps of hidden-layer weights requested ahead
     constexpr bool DW_IN_TILE = H <= 128;        // (when the caller asks for it)
-    static_assert(R * 8 <= T, "eight loss lanes per row");
+    static_assert(R * 8 <= T && (H == 64 || R * 8 < T), "eight loss lanes per row; wavefronts left to store h1 where it is stored");
     __shared__ __align__(16) float xs[R * XLD];
     __shared__ __align__(16) __bf16 pieces[SPLIT][R * PLD];   // h1 going forward, g1 going back
     __shared__ __align__(16) float h1f[R * FLD];
@@ -92,16 +101,6 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
             bias1[q] = *reinterpret_cast<const f32x4 *>(b1 + c + 4 * g);
         }
     }
-    bf16x8 wq[PF][NT][SPLIT];
-    auto fetch = [&](const unsigned short *__restrict__ src, int ks, bf16x8 (&dst)[NT][SPLIT]) {
-#pragma unroll
-        for (int q = 0; q < NT; ++q)
-#pragma unroll
-            for (int p = 0; p < SPLIT; ++p)
-                dst[q][p] = *reinterpret_cast<const bf16x8 *>(src + split_frag<H>(ks, NT * w + q, p, lane));
-    };
-#pragma unroll
-    for (int i = 0; i < PF; ++i) fetch(nn.wf, i, wq[i]);
     stage_head(params + IN * H + H + H * H + H, H, A, GAUSS, w2s, t, T);
 #pragma unroll
     for (int q = 0; q < XQ; ++q) {
@@ -125,6 +124,19 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
         }
     }
     if (actor && fl.adv_stats != nullptr) { l_mean = fl.adv_stats[0]; l_std = fl.adv_stats[1]; }
+    // (the weights last: a wavefront's loads come back in order, and the rows are waited for first)
+    __builtin_amdgcn_sched_barrier(0);
+    bf16x8 wq[PF][NT][SPLIT];
+    auto fetch = [&](const unsigned short *__restrict__ src, int ks, bf16x8 (&dst)[NT][SPLIT]) {
+#pragma unroll
+        for (int q = 0; q < NT; ++q)
+#pragma unroll
+            for (int p = 0; p < SPLIT; ++p)
+                dst[q][p] = *reinterpret_cast<const bf16x8 *>(src + split_frag<H>(ks, NT * w + q, p, lane));
+    };
+#pragma unroll
+    for (int i = 0; i < PF; ++i) fetch(nn.wf, i, wq[i]);
+    __builtin_amdgcn_sched_barrier(0);
     for (int i = t; i < R * GLD; i += T) g2s[i] = 0.0f;
 #pragma unroll
     for (int q = 0; q < XQ; ++q) {
@@ -138,29 +150,43 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
     __syncthreads();
 
     // ---- layer 0, transposed: D[column 4 g + v][batch row n]
+    {
+        float x[RT][K0];
 #pragma unroll
-    for (int q = 0; q < NT; ++q) {
-        const int c = 16 * (NT * w + q) + 4 * g;
+        for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-            const int r = 16 * rt + n;
-            f32x4 d = {0.0f, 0.0f, 0.0f, 0.0f};
+            for (int s = 0; s < K0; ++s)
+                x[rt][s] = 4 * s + g < IN ? xs[(16 * rt + n) * XLD + 4 * s + g] : 0.0f;
+        f32x4 d[NT][RT];
 #pragma unroll
-            for (int s = 0; s < K0; ++s) {
-                if (4 * s < IN) {
-                    const float b = 4 * s + g < IN ? xs[r * XLD + 4 * s + g] : 0.0f;
-                    d = __builtin_amdgcn_mfma_f32_16x16x4f32(w0[q][s], b, d, 0, 0, 0);
-                }
+        for (int q = 0; q < NT; ++q)
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) d[q][rt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int s = 0; s < K0; ++s) {
+            if (4 * s < IN) {
+#pragma unroll
+                for (int q = 0; q < NT; ++q)
+#pragma unroll
+                    for (int rt = 0; rt < RT; ++rt)
+                        d[q][rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(w0[q][s], x[rt][s], d[q][rt], 0, 0, 0);
             }
-            f32x4 y;
+        }
 #pragma unroll
-            for (int v = 0; v < 4; ++v) y[v] = activate<ACT>(d[v] + bias0[q][v]);
-            *reinterpret_cast<f32x4 *>(h1f + r * FLD + c) = y;
-            bf16x4 p[SPLIT];
-            split4(y, p);
+        for (int q = 0; q < NT; ++q) {
+            const int c = 16 * (NT * w + q) + 4 * g;
 #pragma unroll
-            for (int i = 0; i < SPLIT; ++i) *reinterpret_cast<bf16x4 *>(&pieces[i][r * PLD + c]) = p[i];
-            if (!fl.dw_in_tiles && r < nrow) *reinterpret_cast<f32x4 *>(nn.h1 + (row0 + r) * H + c) = y;
+            for (int rt = 0; rt < RT; ++rt) {
+                const int r = 16 * rt + n;
+                f32x4 y;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) y[v] = activate<ACT>(d[q][rt][v] + bias0[q][v]);
+                *reinterpret_cast<f32x4 *>(h1f + r * FLD + c) = y;
+                bf16x4 p[SPLIT];
+                split4(y, p);
+#pragma unroll
+                for (int i = 0; i < SPLIT; ++i) *reinterpret_cast<bf16x4 *>(&pieces[i][r * PLD + c]) = p[i];
+            }
         }
     }
     __syncthreads();
@@ -202,20 +228,27 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
             }
         }
         // head: this wavefront's columns' share of out^T[a][row]; k-slot g of step v is column 4 g + v
+        float a[NT][4];
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-            f32x4 d = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int q = 0; q < NT; ++q)
 #pragma unroll
-            for (int q = 0; q < NT; ++q)
+            for (int v = 0; v < 4; ++v)
+                a[q][v] = n < PA_MAX ? w2s[(16 * (NT * w + q) + 4 * g + v) * PA_MAX + n] : 0.0f;
+        f32x4 d[RT];
 #pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const float a = n < PA_MAX ? w2s[(16 * (NT * w + q) + 4 * g + v) * PA_MAX + n] : 0.0f;
-                    d = __builtin_amdgcn_mfma_f32_16x16x4f32(a, h2v[rt][q][v], d, 0, 0, 0);
-                }
-            if (g < PA_MAX / 4) {
+        for (int rt = 0; rt < RT; ++rt) d[rt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                for (int v = 0; v < 4; ++v) red[(w * R + 16 * rt + n) * (PA_MAX + 1) + 4 * g + v] = d[v];
-            }
+        for (int q = 0; q < NT; ++q)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt)
+                    d[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[q][v], h2v[rt][q][v], d[rt], 0, 0, 0);
+        if (g < PA_MAX / 4) {
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) red[(w * R + 16 * rt + n) * (PA_MAX + 1) + 4 * g + v] = d[rt][v];
         }
     }
     __syncthreads();
@@ -267,47 +300,72 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
                 g2row[2 * PA_MAX] = kl;   // (the spare float of the row, for the tile's sum below)
             }
         }
+    } else if (!fl.dw_in_tiles) {
+        // the wavefronts without loss rows: h1 out to the weight-gradient launch, whole rows at a time
+        for (int r = w - R / 8; r < nrow; r += NW - R / 8)
+            if (4 * lane < H)
+                *reinterpret_cast<f32x4 *>(nn.h1 + (row0 + r) * H + 4 * lane) = *reinterpret_cast<const f32x4 *>(h1f + r * FLD + 4 * lane);
     }
     __syncthreads();
 
     // ---- back through the head and layer 1's activation: g1^T, on the lanes that hold h2
+    {
+        float w2[NT][PA_MAX / 4], gb[RT][PA_MAX / 4], gr[4 * RT];
 #pragma unroll
-    for (int q = 0; q < NT; ++q) {
-        const int c = 16 * (NT * w + q);
-        f32x4 cs = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int s = 0; s < PA_MAX / 4; ++s) {
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-            const int r = 16 * rt + n;
-            f32x4 d = {0.0f, 0.0f, 0.0f, 0.0f};
+            for (int q = 0; q < NT; ++q) w2[q][s] = w2s[(16 * (NT * w + q) + n) * PA_MAX + 4 * s + g];
 #pragma unroll
-            for (int s = 0; s < PA_MAX / 4; ++s)   // (W2's rows are zero beyond A)
-                d = __builtin_amdgcn_mfma_f32_16x16x4f32(w2s[(c + n) * PA_MAX + 4 * s + g], g2s[r * GLD + 4 * s + g], d, 0, 0, 0);
-            f32x4 y;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) y[v] = d[v] * act_deriv_out<ACT>(h2v[rt][q][v]);
-            cs = cs + y;
-            bf16x4 p[SPLIT];
-            split4(y, p);
-#pragma unroll
-            for (int i = 0; i < SPLIT; ++i) *reinterpret_cast<bf16x4 *>(&pieces[i][r * PLD + c + 4 * g]) = p[i];
-            if constexpr (DW_IN_TILE) *reinterpret_cast<f32x4 *>(g1f + r * FLD + c + 4 * g) = y;
-            if (!fl.dw_in_tiles && r < nrow) *reinterpret_cast<f32x4 *>(nn.g1 + (row0 + r) * H + c + 4 * g) = y;
+            for (int rt = 0; rt < RT; ++rt) gb[rt][s] = g2s[(16 * rt + n) * GLD + 4 * s + g];
         }
-        // bias gradient of layer 1: over the rows, which are the sixteen lanes n
 #pragma unroll
-        for (int off = 8; off > 0; off >>= 1) {
+        for (int s = 0; s < 4 * RT; ++s) gr[s] = g2s[(4 * s + g) * GLD + n];
+        f32x4 d[NT][RT], d2[NT];
 #pragma unroll
-            for (int v = 0; v < 4; ++v) cs[v] += __shfl_xor(cs[v], off, 64);
+        for (int q = 0; q < NT; ++q) {
+            d2[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) d[q][rt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         }
-        if (n == 0) *reinterpret_cast<f32x4 *>(db_part + H + c + 4 * g) = cs;
+#pragma unroll
+        for (int s = 0; s < PA_MAX / 4; ++s)   // (W2's rows are zero beyond A)
+#pragma unroll
+            for (int q = 0; q < NT; ++q)
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt)
+                    d[q][rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(w2[q][s], gb[rt][s], d[q][rt], 0, 0, 0);
         // dW2[col][a] of the tile = sum over rows of h2[row][col] g2[row][a]
-        f32x4 d = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int s = 0; s < 4 * RT; ++s)
-            d = __builtin_amdgcn_mfma_f32_16x16x4f32(h2f[(4 * s + g) * FLD + c + n], g2s[(4 * s + g) * GLD + n], d, 0, 0, 0);
-        if (n < A) {
 #pragma unroll
-            for (int v = 0; v < 4; ++v) thin_part[(size_t)IN * H + (size_t)(c + 4 * g + v) * A + n] = d[v];
+            for (int q = 0; q < NT; ++q)
+                d2[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(h2f[(4 * s + g) * FLD + 16 * (NT * w + q) + n], gr[s], d2[q], 0, 0, 0);
+#pragma unroll
+        for (int q = 0; q < NT; ++q) {
+            const int c = 16 * (NT * w + q) + 4 * g;
+            f32x4 cs = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                const int r = 16 * rt + n;
+                f32x4 y;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) y[v] = d[q][rt][v] * act_deriv_out<ACT>(h2v[rt][q][v]);
+                cs = cs + y;
+                bf16x4 p[SPLIT];
+                split4(y, p);
+#pragma unroll
+                for (int i = 0; i < SPLIT; ++i) *reinterpret_cast<bf16x4 *>(&pieces[i][r * PLD + c]) = p[i];
+                if constexpr (DW_IN_TILE) *reinterpret_cast<f32x4 *>(g1f + r * FLD + c) = y;
+                if (!fl.dw_in_tiles && r < nrow) *reinterpret_cast<f32x4 *>(nn.g1 + (row0 + r) * H + c) = y;
+            }
+            // bias gradient of layer 1: over the rows, which are the sixteen lanes n
+#pragma unroll
+            for (int v = 0; v < 4; ++v) cs[v] = row16_sum(cs[v]);
+            if (n == 0) *reinterpret_cast<f32x4 *>(db_part + H + c) = cs;
+            if (n < A) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) thin_part[(size_t)IN * H + (size_t)(c + v) * A + n] = d2[q][v];
+            }
         }
     }
     if (w == NW - 1 && lane < ld) {   // column sums of the tile: bias gradient of the head, log_std gradient
@@ -349,31 +407,40 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
             if (ks + PF < KS) fetch(nn.wb, ks + PF, wq[ks % PF]);
             __builtin_amdgcn_sched_barrier(0);
         }
+        float g0[NT][RT][4];
 #pragma unroll
-        for (int q = 0; q < NT; ++q) {
-            const int c = 16 * (NT * w + q) + n;
-            float g0[RT][4];
+        for (int q = 0; q < NT; ++q)
 #pragma unroll
             for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
                 for (int v = 0; v < 4; ++v)
-                    g0[rt][v] = (hi[rt][q][v] + lo[rt][q][v]) * act_deriv_out<ACT>(h1f[(16 * rt + 4 * g + v) * FLD + c]);
-            // dW0[i][c] of the tile = sum over rows of x[row][i] g0[row][c]; row IN of x^T holds ones
-            for (int it = 0; 16 * it <= IN; ++it) {
-                const int i = 16 * it + n;
-                f32x4 d = {0.0f, 0.0f, 0.0f, 0.0f};
+                    g0[q][rt][v] = (hi[rt][q][v] + lo[rt][q][v]) *
+                                   act_deriv_out<ACT>(h1f[(16 * rt + 4 * g + v) * FLD + 16 * (NT * w + q) + n]);
+        // dW0[i][c] of the tile = sum over rows of x[row][i] g0[row][c]; row IN of x^T holds ones
+        for (int it = 0; 16 * it <= IN; ++it) {
+            const int i = 16 * it + n;
+            float x[RT][4];
 #pragma unroll
-                for (int rt = 0; rt < RT; ++rt)
+            for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        const float x = i <= IN ? xs[(16 * rt + 4 * g + v) * XLD + i] : 0.0f;
-                        d = __builtin_amdgcn_mfma_f32_16x16x4f32(x, g0[rt][v], d, 0, 0, 0);
-                    }
+                for (int v = 0; v < 4; ++v) x[rt][v] = i <= IN ? xs[(16 * rt + 4 * g + v) * XLD + i] : 0.0f;
+            f32x4 d[NT];
 #pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    const int row = 16 * it + 4 * g + v;
-                    if (row < IN) thin_part[(size_t)row * H + c] = d[v];
-                    else if (row == IN) db_part[c] = d[v];
+            for (int q = 0; q < NT; ++q) d[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+#pragma unroll
+                    for (int q = 0; q < NT; ++q)
+                        d[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[rt][v], g0[q][rt][v], d[q], 0, 0, 0);
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int row = 16 * it + 4 * g + v;
+                float *o = row < IN ? thin_part + (size_t)row * H : db_part;
+                if (row <= IN) {
+#pragma unroll
+                    for (int q = 0; q < NT; ++q) o[16 * (NT * w + q) + n] = d[q][v];
                 }
             }
         }
