@@ -12,7 +12,9 @@ struct Mlp3Net {
     float *cache;            // forward: written when non-null; backward: read
     const float *grad_out;   // backward
     float *g1, *g0, *ls_part, *db_part, *thin_part;  // backward workspace (set by the host function)
-    float *h1;                                       // fused update: layer-0 outputs [B, H] for the weight-gradient launch
+    // fused update, for the weight-gradient launch: h1 and g1 split, as operands contracted over the batch rows
+    // (mlp_split.hpp: k-step = 32 batch rows, the other index = column)
+    unsigned short *h1q, *g1q;
     const unsigned short *wf, *wb;                   // fused update: the hidden layer's weights split (mlp_split.hpp), forward / W^T
     int A, gauss;            // set by the host function from the description
     int thin_stride;         // floats per row tile in thin_part: IN H + H A, + H H where the tiles carry dW1 too
@@ -59,9 +61,9 @@ struct UpdateWs {
     int rows, tiles;          // batch rows per tile
     bool dw_in_tiles;
     SplitNets split;          // copies of the hidden layers' weights that io.n[i].wf / wb read
-    Mlp3Net net[2];           // g1, h1, ls_part, db_part, thin_part, thin_stride
+    Mlp3Net net[2];           // h1q, g1q, ls_part, db_part, thin_part, thin_stride
     float *partial;
-    int splits, rows_per;     // batch splits of the weight-gradient launch
+    int splits, steps_per;    // batch splits of the weight-gradient launch, k-steps of 32 rows each
 };
 int mlp3_update_ws(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int batch, const float *const *params, UpdateWs *out);
 int launch_split_weights(mrl_ctx *ctx, int H, const SplitNets &s, int n_nets);
@@ -69,6 +71,7 @@ int launch_split_weights(mrl_ctx *ctx, int H, const SplitNets &s, int n_nets);
 // *sq_blocks = number of blocks written (0 when none were)
 int mlp3_update_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int batch, Mlp3Nets io, const UpdateWs &ws,
                   float *const *grads, float *sq_part, int *sq_blocks, const FwdLoss &loss);
+int launch_dw_frag(mrl_ctx *ctx, int H, int batch, const UpdateWs &ws, int P0, int Ptot, int w1_off);
 int launch_fb(mrl_ctx *ctx, int H, int act, int batch, int IN, int rows, const Mlp3Nets &nets, const FwdLoss &fl);
 // grows the context's MLP workspace to at least `floats`
 int mlp_ensure_ws(mrl_ctx *ctx, size_t floats, float **out);

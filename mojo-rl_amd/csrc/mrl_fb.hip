@@ -29,6 +29,11 @@
 
 namespace mrl {
 
+struct DwFrag {
+    const unsigned short *x[2], *g[2];
+    int off[2];   // of the net's W1 gradient in a split's partial vector
+};
+
 template <int ACT>
 MRL_DEV float act_deriv_out(float y) {
     if (ACT == 1) return y > 0.0f ? 1.0f : 0.0f;
@@ -45,6 +50,28 @@ MRL_DEV float row16_sum(float x) {
     return x;
 }
 
+// A tile's rows of column tile ct (RT = 1: of ct and ct + 1) of f [16 RT][LD] (LDS), split, as the operand pieces that a
+// product contracted over the batch rows reads (k-step = 32 rows): lane 16 g + n holds rows 8 g .. 8 g + 7 of column n.
+// A tile of 16 rows fills half a k-step: it takes two column tiles per wavefront; the last tile of an odd count puts
+// zeros where the other half would be.
+template <int H, int RT, int LD>
+MRL_DEV void batch_operand(const float *f, unsigned short *dst, int ct, int lane) {
+    const int g = lane >> 4, n = lane & 15;
+    const int c = ct + (RT == 1 ? g >> 1 : 0), rg = RT == 1 ? g & 1 : g;
+    const int ks = RT == 1 ? blockIdx.x >> 1 : blockIdx.x, gs = RT == 1 ? 2 * (blockIdx.x & 1) + rg : g;
+    f32x8 x;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) x[j] = f[(8 * rg + j) * LD + 16 * c + n];
+    bf16x8 p[SPLIT];
+    split8(x, p);
+    const bool pad = RT == 1 && blockIdx.x == gridDim.x - 1 && (blockIdx.x & 1) == 0;
+#pragma unroll
+    for (int i = 0; i < SPLIT; ++i) {
+        *reinterpret_cast<bf16x8 *>(dst + split_frag<H>(ks, c, i, 16 * gs + n)) = p[i];
+        if (pad) *reinterpret_cast<uint4 *>(dst + split_frag<H>(ks, c, i, 16 * (gs + 2) + n)) = make_uint4(0, 0, 0, 0);
+    }
+}
+
 constexpr int fb_threads(int H) { return H == 64 ? 256 : 512; }
 
 template <int H, int ACT, int RT>
@@ -55,12 +82,14 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
     constexpr int K0 = PIN_MAX / 4;
     constexpr int PF = KS < 3 ? KS : 3;          // k-steps of hidden-layer weights requested ahead
     constexpr bool DW_IN_TILE = H <= 128;        // (when the caller asks for it)
+    constexpr bool BATCH_OPERANDS = H > 64 && NT % (2 / RT) == 0;   // (where the caller may ask for the weight-gradient launch)
     static_assert(R * 8 <= T && (H == 64 || R * 8 < T), "eight loss lanes per row; wavefronts left to store h1 where it is stored");
     __shared__ __align__(16) float xs[R * XLD];
     __shared__ __align__(16) __bf16 pieces[SPLIT][R * PLD];   // h1 going forward, g1 going back
     __shared__ __align__(16) float h1f[R * FLD];
     __shared__ __align__(16) float h2f[R * FLD];
-    __shared__ __align__(16) float g1f[DW_IN_TILE ? R * FLD : 4];
+    // (g1 lies over h2: a wavefront writes only columns whose h2 it alone reads, after it has read them)
+    float *g1f = h2f;
     __shared__ __align__(16) float w2s[HEAD_LDS(H)];
     __shared__ float red[NW * R * (PA_MAX + 1)];
     __shared__ float g2s[R * GLD];
@@ -300,11 +329,9 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
                 g2row[2 * PA_MAX] = kl;   // (the spare float of the row, for the tile's sum below)
             }
         }
-    } else if (!fl.dw_in_tiles) {
-        // the wavefronts without loss rows: h1 out to the weight-gradient launch, whole rows at a time
-        for (int r = w - R / 8; r < nrow; r += NW - R / 8)
-            if (4 * lane < H)
-                *reinterpret_cast<f32x4 *>(nn.h1 + (row0 + r) * H + 4 * lane) = *reinterpret_cast<const f32x4 *>(h1f + r * FLD + 4 * lane);
+    } else if (BATCH_OPERANDS && !fl.dw_in_tiles) {
+        // the wavefronts without loss rows: h1 out to the weight-gradient launch
+        for (int ct = (w - R / 8) * (2 / RT); ct < H / 16; ct += (NW - R / 8) * (2 / RT)) batch_operand<H, RT, FLD>(h1f, nn.h1q, ct, lane);
     }
     __syncthreads();
 
@@ -355,8 +382,7 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
                 split4(y, p);
 #pragma unroll
                 for (int i = 0; i < SPLIT; ++i) *reinterpret_cast<bf16x4 *>(&pieces[i][r * PLD + c]) = p[i];
-                if constexpr (DW_IN_TILE) *reinterpret_cast<f32x4 *>(g1f + r * FLD + c) = y;
-                if (!fl.dw_in_tiles && r < nrow) *reinterpret_cast<f32x4 *>(nn.g1 + (row0 + r) * H + c) = y;
+                *reinterpret_cast<f32x4 *>(g1f + r * FLD + c) = y;
             }
             // bias gradient of layer 1: over the rows, which are the sixteen lanes n
 #pragma unroll
@@ -366,6 +392,12 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
 #pragma unroll
                 for (int v = 0; v < 4; ++v) thin_part[(size_t)IN * H + (size_t)(c + v) * A + n] = d2[q][v];
             }
+        }
+        if (BATCH_OPERANDS && !fl.dw_in_tiles) {
+            // g1 out to the weight-gradient launch (its columns were written by this wavefront)
+            asm volatile("" : : : "memory");
+#pragma unroll
+            for (int q = 0; q < NT; q += 2 / RT) batch_operand<H, RT, FLD>(g1f, nn.g1q, NT * w + q, lane);
         }
     }
     if (w == NW - 1 && lane < ld) {   // column sums of the tile: bias gradient of the head, log_std gradient
@@ -469,6 +501,110 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
             }
         }
     }
+}
+
+// dW = h1^T g1 of the hidden layer of both nets over a split of the batch: partial[split][Ptot].  Operands as the row
+// tiles left them (split, in operand order), straight from global memory into registers: no LDS, no barrier.  A
+// workgroup makes one 64 x 128 output tile (four wavefronts, 32 x 64 each) twice over, two groups of wavefronts taking
+// alternate k-steps of 32 batch rows and adding up at the end.
+// What bounds it: fetching the operands (25 MB at a minibatch of 4096, written by the launch before), then the matrix
+// cores (48 instructions of 16 cycles per wavefront and k-step; a k-step's operands are in flight while the one before
+// is multiplied).  256 rows per split give every CU one workgroup at a minibatch of 4096 and
+// H = 256; more splits would be more partial sums to write and read back.  H = 256, 4096 rows, both nets: 12.6 us, against
+// 16.1 us with fp32 matrix instructions and 16.3 us when every workgroup splits its fp32 rows itself.
+// Workgroups go to the chip's eight XCDs in turn, and each XCD has an L2 of its own: the tiles of one (net, split) read
+// the same rows, so the flat list of workgroups gives them to ONE XCD.
+template <int H>
+__global__ __launch_bounds__(512) void dw_frag_kernel(DwFrag d, int steps, int steps_per, int splits, int Ptot,
+                                                      float *__restrict__ partial) {
+    constexpr int XCDS = 8, TN = 128, tiles_n = H / TN, tiles = tiles_n * (H / 64), NB = 4, RLD = TN + 4;
+    static_assert(H % TN == 0, "whole tiles");
+    __shared__ float sum[64 * RLD];
+    const int groups = 2 * splits;
+    // workgroup n = (round r, XCD x): the r-th workgroup that XCD x receives.  An XCD walks its groups x, x + 8, ... one
+    // after the other, `tiles` workgroups each; the workgroups of a short last round keep the plain order.
+    int grp, tile;
+    {
+        const int nwg = blockIdx.x, full = (groups / XCDS) * XCDS * tiles;
+        const int x = nwg % XCDS, q = nwg / XCDS, m = nwg - full;
+        tile = nwg < full ? q % tiles : m % tiles;
+        grp = nwg < full ? (q / tiles) * XCDS + x : (groups / XCDS) * XCDS + m / tiles;
+    }
+    const int net = grp / splits, z = grp % splits;
+    const int t = threadIdx.x, lane = t & 63, half = t >> 8, wr = (t >> 7) & 1, wc = (t >> 6) & 1, g = lane >> 4, n = lane & 15;
+    const int ct_a = (tile / tiles_n) * 4 + 2 * wr, ct_b = (tile % tiles_n) * (TN / 16) + NB * wc;
+    const int k0 = z * steps_per + half, k1 = min(z * steps_per + steps_per, steps);
+    const unsigned short *__restrict__ X = d.x[net], *__restrict__ G = d.g[net];
+    f32x4 hi[2][NB], lo[2][NB];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) hi[a][b] = lo[a][b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    bf16x8 fa[2][2][SPLIT], fb[2][NB][SPLIT];   // [buffer]
+    auto fetch = [&](int ks, int u) {
+#pragma unroll
+        for (int q = 0; q < SPLIT; ++q) {
+#pragma unroll
+            for (int a = 0; a < 2; ++a) fa[u][a][q] = *reinterpret_cast<const bf16x8 *>(X + split_frag<H>(ks, ct_a + a, q, lane));
+#pragma unroll
+            for (int b = 0; b < NB; ++b) fb[u][b][q] = *reinterpret_cast<const bf16x8 *>(G + split_frag<H>(ks, ct_b + b, q, lane));
+        }
+    };
+    auto multiply = [&](int u) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int a = 0; a < 2; ++a) mfma_split(fa[u][a], fb[u][b], hi[a][b], lo[a][b]);
+    };
+    if (k0 < k1) fetch(k0, 0);
+    for (int k = k0; k < k1; k += 4) {   // two k-steps per round, so that the buffers keep their names
+        if (k + 2 < k1) fetch(k + 2, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(0);
+        if (k + 2 < k1) {
+            if (k + 4 < k1) fetch(k + 4, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(1);
+        }
+    }
+    if (half == 1) {
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    sum[(32 * wr + 16 * a + 4 * g + v) * RLD + 64 * wc + 16 * b + n] = hi[a][b][v] + lo[a][b][v];
+    }
+    __syncthreads();
+    if (half == 1) return;
+    float *out = partial + (size_t)z * Ptot + d.off[net] + (size_t)(tile / tiles_n) * 64 * H + (tile % tiles_n) * TN;
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int r = 32 * wr + 16 * a + 4 * g + v, c = 64 * wc + 16 * b + n;
+                out[(size_t)r * H + c] = sum[r * RLD + c] + (hi[a][b][v] + lo[a][b][v]);
+            }
+}
+
+// P0: parameters of the first net, w1_off: offset of W1 in a net's parameters
+int launch_dw_frag(mrl_ctx *ctx, int H, int batch, const UpdateWs &ws, int P0, int Ptot, int w1_off) {
+    DwFrag d;
+    for (int i = 0; i < 2; ++i) {
+        d.x[i] = ws.net[i].h1q;
+        d.g[i] = ws.net[i].g1q;
+        d.off[i] = (i ? P0 : 0) + w1_off;
+    }
+    const int steps = (batch + 31) / 32;
+    const dim3 grid(2 * ws.splits * (H / 64) * (H / 128)), block(512);
+    if (H == 256) hipLaunchKernelGGL(dw_frag_kernel<256>, grid, block, 0, ctx->stream, d, steps, ws.steps_per, ws.splits, Ptot, ws.partial);
+    else if (H == 128) hipLaunchKernelGGL(dw_frag_kernel<128>, grid, block, 0, ctx->stream, d, steps, ws.steps_per, ws.splits, Ptot, ws.partial);
+    else return MRL_E_UNSUPPORTED;
+    MRL_CHECK_LAUNCH();
+    return MRL_OK;
 }
 
 // Split operand copies of the hidden layer's weights of one or two nets, both orientations; grid = (H * H / 8 / 256

@@ -10,7 +10,7 @@
 //   sum3_kernel         sum of the splits and of the row tiles' pieces straight into the flat gradient vector.
 // They replace 3 + 2 + 3 + 3 launches of the per-layer kernels (which remain the path for any
 // other shape, and for callers that ask for the gradient with respect to the input).  The minibatch update's
-// row tiles (mrl_fb.hip) share the last two.
+// row tiles (mrl_fb.hip) share the last one.
 #include "mrl_host.hpp"
 #include "mrl_device.hpp"
 #include "mlp_tile.hpp"
@@ -501,7 +501,7 @@ static int fb_tile_rows(int n_cus, int H, int batch) {
 }
 
 // Whether the fused update kernel takes the hidden layer's weight gradient of its row tile itself
-// (H^2 floats per tile and net, added up by the sum kernel) or leaves h1 and g1 to a launch of dw3_kernel.
+// (H^2 floats per tile and net, added up by the sum kernel) or leaves h1 and g1 to a launch of dw_frag_kernel.
 static bool dw_in_tiles_pays(int H, int batch) { return H == 64 || (H == 128 && batch <= 8192); }
 
 // true when the two nets can share launches: both fusable, same input width, width and activation
@@ -562,29 +562,19 @@ static void dw_splits(int batch, int *splits, int *rows_per) {
     *splits = (batch + *rows_per - 1) / *rows_per;
 }
 
-// What follows the row tiles: the H x H weight gradients (X[i] = layer-1 inputs [batch, xs], io.n[i].g1) unless the
-// tiles left them (hh_in_tiles), then the sums over tiles and batch splits into the flat gradients.
-static int dw_and_sum(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, int batch, const Mlp3Nets &io,
-                      const float *const *X, int xs, int tiles, bool hh_in_tiles, float *partial, int splits, int rows_per,
-                      float *const *grads, float *sq_part, int *sq_blocks) {
+// The sums over row tiles and batch splits into the flat gradients (hh_in_tiles: the tiles left the H x H weight
+// gradients too).
+static int sum_tiles(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, const Mlp3Nets &io, int tiles, bool hh_in_tiles,
+                     const float *partial, int splits, float *const *grads, float *sq_part, int *sq_blocks) {
     const int IN = descs[0]->layers[0].in_dim, H = descs[0]->layers[0].out_dim;
-    DwSet dw;
-    dw.n = n_nets;   // the H x H layer of each net; the thin layers come out of the row tiles
     SumNets sn{};
     sn.n = n_nets;
     sn.IN = IN;
     sn.H = H;
     sn.hh_in_tiles = hh_in_tiles ? 1 : 0;
-    int base = 0, total_tiles = 0;
+    int Ptot = 0;
     for (int i = 0; i < n_nets; ++i) {
         const Mlp3Net &nn = io.n[i];
-        DwProblem &p = dw.p[i];
-        p.X = X[i]; p.xs = xs; p.G = nn.g1; p.gs = H; p.K = H; p.N = H; p.poff = base + (IN + 1) * H;
-        p.tiles_n = (H + DBN - 1) / DBN;
-        p.tiles = p.tiles_n * ((H + DBM - 1) / DBM);
-        p.vec = (H % 64 == 0 && reinterpret_cast<uintptr_t>(X[i]) % 16 == 0 &&
-                 reinterpret_cast<uintptr_t>(nn.g1) % 16 == 0) ? 1 : 0;
-        total_tiles += p.tiles;
         sn.grads[i] = grads[i];
         sn.ls_part[i] = nn.ls_part;
         sn.db_part[i] = nn.db_part;
@@ -593,13 +583,8 @@ static int dw_and_sum(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets
         sn.P[i] = net_P(*descs[i]);
         sn.A[i] = nn.A;
         sn.gauss[i] = nn.gauss;
-        base += sn.P[i];
+        Ptot += sn.P[i];
     }
-    const int Ptot = base;
-    // (both nets have the same width: every problem has the same number of tiles, see dw3_kernel)
-    if (!hh_in_tiles)
-        hipLaunchKernelGGL(dw3_kernel, dim3(total_tiles * splits), dim3(256), 0, ctx->stream, dw, batch, rows_per,
-                           Ptot, partial, splits);
     const int sum_blocks = grid_for(Ptot, 256);
     if (sum_blocks > 1024) sq_part = nullptr;   // more partials than the caller's buffer holds
     if (sq_blocks) *sq_blocks = sq_part ? sum_blocks : 0;
@@ -631,7 +616,6 @@ int mlp3_backward_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, 
     // workspace: per net g1 [B, H] | g0 [B, H] | ls_part [tiles, PA_MAX] | db_part [tiles, 2H + PA_MAX] |
     // thin_part [tiles, IN H + H A]; then partial [splits, Ptot]
     float *w = ws;
-    const float *X[2];
     for (int i = 0; i < n_nets; ++i) {
         io.n[i].g1 = w; w += (size_t)batch * H;
         io.n[i].g0 = w; w += (size_t)batch * H;
@@ -639,7 +623,6 @@ int mlp3_backward_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, 
         io.n[i].db_part = w; w += (size_t)tiles * (2 * H + PA_MAX);
         io.n[i].thin_stride = IN * H + H * descs[i]->layers[2].out_dim;
         io.n[i].thin_part = w; w += (size_t)tiles * (size_t)io.n[i].thin_stride;
-        X[i] = io.n[i].cache + (size_t)batch * (IN + H);
     }
     if (H == 256 && act == 1) launch_bwd_t<256, 1>(ctx, batch, IN, io, n_nets);
     else if (H == 256) launch_bwd_t<256, 2>(ctx, batch, IN, io, n_nets);
@@ -648,7 +631,25 @@ int mlp3_backward_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, 
     else if (act == 1) launch_bwd_t<64, 1>(ctx, batch, IN, io, n_nets);
     else launch_bwd_t<64, 2>(ctx, batch, IN, io, n_nets);
     MRL_CHECK_LAUNCH();
-    return dw_and_sum(ctx, descs, n_nets, batch, io, X, 2 * H, tiles, false, w, splits, rows_per, grads, nullptr, nullptr);
+    DwSet dw;
+    dw.n = n_nets;   // the H x H layer of each net; the thin layers come out of the row tiles
+    int base = 0, total_tiles = 0;
+    for (int i = 0; i < n_nets; ++i) {
+        const float *c1 = io.n[i].cache + (size_t)batch * (IN + H);
+        DwProblem &p = dw.p[i];
+        p.X = c1; p.xs = 2 * H; p.G = io.n[i].g1; p.gs = H; p.K = H; p.N = H; p.poff = base + (IN + 1) * H;
+        p.tiles_n = (H + DBN - 1) / DBN;
+        p.tiles = p.tiles_n * ((H + DBM - 1) / DBM);
+        p.vec = (H % 64 == 0 && reinterpret_cast<uintptr_t>(c1) % 16 == 0 &&
+                 reinterpret_cast<uintptr_t>(io.n[i].g1) % 16 == 0) ? 1 : 0;
+        total_tiles += p.tiles;
+        base += net_P(*descs[i]);
+    }
+    // (both nets have the same width: every problem has the same number of tiles, see dw3_kernel)
+    hipLaunchKernelGGL(dw3_kernel, dim3(total_tiles * splits), dim3(256), 0, ctx->stream, dw, batch, rows_per, base, w,
+                       splits);
+    MRL_CHECK_LAUNCH();
+    return sum_tiles(ctx, descs, n_nets, io, tiles, false, w, splits, grads, nullptr, nullptr);
 }
 
 // carves (and if need be grows) the context's workspace for the fused update of two nets
@@ -659,7 +660,10 @@ int mlp3_update_ws(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int batch, co
     u.rows = fb_tile_rows(ctx->n_cus, H, batch);
     u.tiles = (batch + u.rows - 1) / u.rows;
     u.dw_in_tiles = dw_in_tiles_pays(H, batch);
-    dw_splits(batch, &u.splits, &u.rows_per);
+    int rows_per;
+    dw_splits(batch, &u.splits, &rows_per);
+    u.steps_per = rows_per / 32;
+    static_assert(DKC == 32, "splits of whole k-steps");
     size_t need = 0, P = 0;
     float *base = nullptr;
     for (int pass = 0; pass < 2; ++pass) {   // sizes, then pointers (every piece a multiple of four floats)
@@ -676,8 +680,9 @@ int mlp3_update_ws(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int batch, co
             u.split.wf[i] = reinterpret_cast<unsigned short *>(take(split_elems(H) / 2));
             u.split.wb[i] = reinterpret_cast<unsigned short *>(take(split_elems(H) / 2));
             if (!u.dw_in_tiles) {
-                u.net[i].g1 = take((size_t)batch * H);
-                u.net[i].h1 = take((size_t)batch * H);
+                const size_t elems = (size_t)SPLIT * ((batch + 31) / 32) * 32 * H;
+                u.net[i].h1q = reinterpret_cast<unsigned short *>(take(elems / 2));
+                u.net[i].g1q = reinterpret_cast<unsigned short *>(take(elems / 2));
             }
             u.net[i].ls_part = take((size_t)u.tiles * PA_MAX);
             u.net[i].db_part = take((size_t)u.tiles * (2 * H + PA_MAX));
@@ -699,24 +704,26 @@ int mlp3_update_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int batch, Mlp
                   float *const *grads, float *sq_part, int *sq_blocks, const FwdLoss &loss) {
     int H = 0, act = 0;
     bool gauss = false;
-    const float *X[2];
     for (int i = 0; i < 2; ++i) {
         if (!mlp3_fusable(*descs[i], &H, &act, &gauss)) return MRL_E_UNSUPPORTED;
         Mlp3Net &nn = io.n[i];
         const Mlp3Net &from = ws.net[i];
         nn.A = descs[i]->layers[2].out_dim;
         nn.gauss = gauss ? 1 : 0;
-        nn.g1 = from.g1; nn.h1 = from.h1; nn.ls_part = from.ls_part; nn.db_part = from.db_part;
+        nn.g1q = from.g1q; nn.h1q = from.h1q; nn.ls_part = from.ls_part; nn.db_part = from.db_part;
         nn.thin_part = from.thin_part; nn.thin_stride = from.thin_stride;
         nn.wf = ws.split.wf[i]; nn.wb = ws.split.wb[i];
-        X[i] = nn.h1;
     }
     FwdLoss fl = loss;
     fl.dw_in_tiles = ws.dw_in_tiles ? 1 : 0;
     int rc = launch_fb(ctx, H, act, batch, descs[0]->layers[0].in_dim, ws.rows, io, fl);
     if (rc) return rc;
-    return dw_and_sum(ctx, descs, 2, batch, io, X, H, ws.tiles, ws.dw_in_tiles, ws.partial, ws.splits, ws.rows_per, grads,
-                      sq_part, sq_blocks);
+    if (!ws.dw_in_tiles) {
+        const int P0 = net_P(*descs[0]);
+        rc = launch_dw_frag(ctx, H, batch, ws, P0, P0 + net_P(*descs[1]), (descs[0]->layers[0].in_dim + 1) * H);
+        if (rc) return rc;
+    }
+    return sum_tiles(ctx, descs, 2, io, ws.tiles, ws.dw_in_tiles, ws.partial, ws.splits, grads, sq_part, sq_blocks);
 }
 
 int mlp3_backward(mrl_ctx *ctx, const mrl_mlp_desc &d, int batch, const float *grad_out, const float *params,
