@@ -136,41 +136,176 @@ __global__ __launch_bounds__(64) void gae_kernel(int T, int N, const float *__re
     }
 }
 
+// Below about one wavefront of envs per CU the plain scan waits for memory most of the time (T = 1000,
+// N = 4096: 63 waits on 64 CUs).  A = delta + decay * A is a serial chain per env, but a short one: three dependent instructions a
+// step.  What a plain scan waits for is memory, so the chain gets a wavefront of its own and eight
+// others feed it: a workgroup has G envs; its loaders fetch K = 512 / G * R steps at a time (index
+// t * N + env: rows of G consecutive floats), form delta, which needs no neighbour but the value one
+// step later, and leave (delta, done) in LDS; one wavefront scans the chunk in place; the loaders
+// store advantages and returns.  Three chunks are in LDS at once, one per stage, and the next one's
+// loads are in flight meanwhile.  What bounds it now is the chain (about 50 cycles a step) up to 16 envs
+// per CU, then the memory (T = 1000, N = 8192: 5.6 TB/s).  Same operations in the same order as the scan.  A chunk's rows, and
+// the value row above it, are read two barriers before the first of them is stored, so outputs may
+// share memory with the inputs.  deep_agents/ppo/ppo.mojo:2317-2353
+constexpr int GAE_LOADERS = 512;   // threads; one more wavefront scans
+
+template <int G, int R>
+__global__ __launch_bounds__(GAE_LOADERS + 64) void gae_fed_kernel(int T, int N, const float *rewards, const float *values,
+                                                               const float *dones, const float *bootstrap, float gamma,
+                                                               float decay, float *adv, float *ret) {
+    constexpr int K = GAE_LOADERS / G * R, U = 16;
+    static_assert(K % U == 0, "");
+    __shared__ float2 buf[3][K * G];
+    // two groups of 16 share a 128-byte line: they go to one XCD (workgroup b runs on XCD b % 8), eight
+    // workgroups apart, so that one L2 sees both halves
+    const int b = blockIdx.x;
+    const int group = G == 16 ? ((b >> 4) * 8 + (b & 7)) * 2 + ((b >> 3) & 1) : b;
+    const int lane = threadIdx.x % G, top = threadIdx.x / G * R;   // this thread's env, its first row of a chunk
+    const int e = group * G + lane, ec = min(e, N - 1);
+    const bool scanner = threadIdx.x >= GAE_LOADERS;
+    const int C = (T + K - 1) / K;
+    if (group * G >= N) return;
+
+    float r[R], v[R], d[R], v1[R], v2[R], next = 0.0f, gae = 0.0f;
+    // A chunk's rows end at its uniform base row T - (c + 1) K (below 0 in a ragged last chunk; only rows t >= 0 are
+    // addressed), a thread's offsets from it are the same in every chunk.
+    unsigned off[R];
+#pragma unroll
+    for (int j = 0; j < R; ++j) off[j] = ((unsigned)(K - 1 - top - j) * N + ec) * 4u;
+    auto in = [](const float *p, long row0, unsigned o) { return *reinterpret_cast<const float *>(reinterpret_cast<const char *>(p + row0) + o); };
+    auto out = [](float *p, long row0, unsigned o, float x) { *reinterpret_cast<float *>(reinterpret_cast<char *>(p + row0) + o) = x; };
+    auto request = [&](int c) {   // rows t < 0 read row 0, envs past N the last env; nothing uses the values
+        const int t0 = T - (c + 1) * K;
+        const long row0 = (long)t0 * N;
+        const unsigned low = t0 < 0 ? (unsigned)(-t0 * N + ec) * 4u : 0u;
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            const unsigned o = max(off[j], low);
+            r[j] = in(rewards, row0, o); v[j] = in(values, row0, o); d[j] = in(dones, row0, o);
+        }
+        if (c == 0 && top == 0) next = bootstrap[ec];
+        else next = in(values, row0, max(off[0] + 4u * N, low));
+    };
+    if (!scanner) request(0);
+    else __builtin_amdgcn_s_setprio(3);   // the chain goes before the loaders of its SIMD
+    for (int it = 0; it < C + 2; ++it) {
+        if (!scanner) {
+            if (it < C) {
+                float2 *B = buf[it % 3] + top * G + lane;
+                float nv = next;
+#pragma unroll
+                for (int j = 0; j < R; ++j) {
+                    B[j * G] = make_float2(r[j] + gamma * (d[j] > 0.5f ? 0.0f : nv) - v[j], d[j]);
+                    nv = v[j];
+                }
+            }
+            float vs[R];
+#pragma unroll
+            for (int j = 0; j < R; ++j) { vs[j] = v2[j]; v2[j] = v1[j]; v1[j] = v[j]; }
+            if (it + 1 < C) request(it + 1);
+            if (it >= 2) {
+                const float2 *B = buf[(it - 2) % 3] + top * G + lane;
+                const int t0 = T - (it - 1) * K;
+                const long row0 = (long)t0 * N;
+                float a[R];
+#pragma unroll
+                for (int j = 0; j < R; ++j) a[j] = B[j * G].x;
+                if (t0 >= 0 && group * G + G <= N) {
+#pragma unroll
+                    for (int j = 0; j < R; ++j) { out(adv, row0, off[j], a[j]); out(ret, row0, off[j], a[j] + vs[j]); }
+                } else {
+#pragma unroll
+                    for (int j = 0; j < R; ++j)
+                        if (t0 + K - 1 - top - j >= 0 && e < N) { out(adv, row0, off[j], a[j]); out(ret, row0, off[j], a[j] + vs[j]); }
+                }
+            }
+        } else if (it >= 1 && it <= C && threadIdx.x < GAE_LOADERS + G) {
+            float2 *B = buf[(it - 1) % 3] + lane;
+            const int rows = min(K, T - (it - 1) * K);   // (up to U - 1 rows below t = 0 are scanned and never stored)
+            float2 x[U], n[U];
+#pragma unroll
+            for (int j = 0; j < U; ++j) x[j] = B[j * G];
+#pragma unroll 2
+            for (int k = 0; k < rows; k += U) {
+                const int kn = min(k + U, K - U);
+#pragma unroll
+                for (int j = 0; j < U; ++j) n[j] = B[(kn + j) * G];
+#pragma unroll
+                for (int j = 0; j < U; ++j) {
+                    if (x[j].y > 0.5f) gae = 0.0f;
+                    gae = x[j].x + decay * gae;
+                    B[(k + j) * G].x = gae;
+                }
+#pragma unroll
+                for (int j = 0; j < U; ++j) x[j] = n[j];
+            }
+        }
+        __syncthreads();
+    }
+}
+
 // ---------------------------------------------------------------- advantage normalisation
-// pass 1: per-block sums -> scratch[0..nb); pass 2: mean; pass 3: per-block sum of squared
-// deviations; pass 4: (x - mean) / (sqrt(var + 1e-8) + 1e-8).  Two-pass variance like the
-// reference (ppo.mojo:2356-2371), with fp32 sums taken blockwise.
+// Three launches: per-block sums; per-block sums of squared deviations; (x - mean) /
+// (sqrt(var + 1e-8) + 1e-8).  Two-pass variance like the reference (ppo.mojo:2356-2371), with fp32
+// sums taken blockwise.  Every block of the second and third launch adds the (at most 1024) block
+// sums up itself, all in the same order: a few L2 reads against two more launches of one block.
+constexpr int NORM_BLOCKS = 1024, NORM_U = 4;
+
+// sum(in[0..nb)) / n in every thread
+MRL_DEV float mean_of_blocks(const float *__restrict__ in, int nb, int n, float *smem) {
+    float s = 0.0f;
+    for (int i = threadIdx.x; i < nb; i += blockDim.x) s += in[i];
+    s = block_sum(s, smem);
+    if (threadIdx.x == 0) smem[0] = s / (float)n;
+    __syncthreads();
+    const float m = smem[0];
+    __syncthreads();
+    return m;
+}
+
+// sums == nullptr: out[b] = sum x; else out[b] = sum (x - mean)^2, sums = the first form's block sums
 __global__ __launch_bounds__(TPB) void partial_sum_kernel(const float *__restrict__ x, int n,
-                                                          const float *__restrict__ mean_ptr,
+                                                          const float *__restrict__ sums,
                                                           float *__restrict__ out) {
     __shared__ float smem[4];
-    const float mean = mean_ptr ? *mean_ptr : 0.0f;
+    const long stride = (long)gridDim.x * blockDim.x;
+    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    float a[NORM_U];
+    const bool full = i + (NORM_U - 1) * stride < n;
+    if (full)   // the first elements are on their way while the mean is formed
+#pragma unroll
+        for (int k = 0; k < NORM_U; ++k) a[k] = x[i + k * stride];
+    const float mean = sums ? mean_of_blocks(sums, gridDim.x, n, smem) : 0.0f;
     float s = 0.0f;
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
-        float d = x[i] - mean;
-        s += mean_ptr ? d * d : x[i];
+    auto add = [&](float v) {
+        const float d = v - mean;
+        s += sums ? d * d : v;
+    };
+    if (full) {
+        for (;;) {
+#pragma unroll
+            for (int k = 0; k < NORM_U; ++k) add(a[k]);
+            i += NORM_U * stride;
+            if (i + (NORM_U - 1) * stride >= n) break;
+#pragma unroll
+            for (int k = 0; k < NORM_U; ++k) a[k] = x[i + k * stride];
+        }
     }
+    for (; i < n; i += stride) add(x[i]);
     s = block_sum(s, smem);
     if (threadIdx.x == 0) out[blockIdx.x] = s;
 }
 
-// out[0] = sum(in[0..nb)) / n
-__global__ __launch_bounds__(TPB) void finish_mean_kernel(const float *__restrict__ in, int nb, int n,
-                                                          float *__restrict__ out) {
+__global__ __launch_bounds__(TPB) void normalize_apply_kernel(float *__restrict__ x, int n, int nb,
+                                                              const float *__restrict__ sums,
+                                                              const float *__restrict__ squares) {
     __shared__ float smem[4];
-    float s = 0.0f;
-    for (int i = threadIdx.x; i < nb; i += blockDim.x) s += in[i];
-    s = block_sum(s, smem);
-    if (threadIdx.x == 0) out[0] = s / (float)n;
-}
-
-__global__ __launch_bounds__(TPB) void normalize_apply_kernel(float *__restrict__ x, int n,
-                                                              const float *__restrict__ stats) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float mean = stats[0], variance = stats[1];
+    const float mean = mean_of_blocks(sums, nb, n, smem);
+    const float variance = mean_of_blocks(squares, nb, n, smem);
     const float std = sqrtf(variance + 1e-8f);
-    x[i] = (x[i] - mean) / (std + 1e-8f);
+    const long stride = (long)gridDim.x * blockDim.x;
+#pragma unroll NORM_U
+    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) x[i] = (x[i] - mean) / (std + 1e-8f);
 }
 
 // ---------------------------------------------------------------- reward RunningMeanStd
@@ -532,8 +667,20 @@ int mrl_gae(mrl_ctx *ctx, int T, int N, const float *rewards, const float *value
     MRL_CHECK_ARG(T >= 0 && N >= 0, "mrl_gae: negative size");
     if (T == 0 || N == 0) return MRL_OK;
     MRL_CHECK_ARG(rewards && values && dones && bootstrap && adv && ret, "mrl_gae: NULL buffer");
-    hipLaunchKernelGGL(gae_kernel, dim3(grid_for(N, 64)), dim3(64), 0, ctx->stream, T, N, rewards,
-                       values, dones, bootstrap, (float)gamma, (float)(gamma * lam), adv, ret);
+    // The narrowest groups that still give every group a CU of its own; with a wavefront of envs per CU the plain scan
+    // is the faster one.  us, plain / groups of 16 / 32 / 64: T = 1000, N = 1000: 57.5 / 22.2 / 26.3 / 30.5; N = 4096:
+    // 57.7 / 23.2 / 26.2 / 32.0; N = 8192: 58.0 / 43.0 / 29.1 / 35.2; T = 64, N = 16384: 6.4 / 10.6 / 7.4 / 5.8;
+    // N = 65536: 13.4 / - / - / 21.2.
+    const float g = (float)gamma, decay = (float)(gamma * lam);
+    auto launch = [&](auto kernel, int groups, int threads = GAE_LOADERS + 64) {
+        hipLaunchKernelGGL(kernel, dim3(groups), dim3(threads), 0, ctx->stream, T, N, rewards, values, dones,
+                           bootstrap, g, decay, adv, ret);
+    };
+    if (T > 1 << 30) launch(gae_kernel, grid_for(N, 64), 64);   // (the chunked form counts rows past T in 32 bits)
+    else if (N <= 16 * ctx->n_cus) launch(gae_fed_kernel<16, 2>, (grid_for(N, 16) + 15) / 16 * 16);
+    else if (N <= 32 * ctx->n_cus) launch(gae_fed_kernel<32, 4>, grid_for(N, 32));
+    else if (N <= 64 * ctx->n_cus) launch(gae_fed_kernel<64, 4>, grid_for(N, 64));
+    else launch(gae_kernel, grid_for(N, 64), 64);
     MRL_CHECK_LAUNCH();
     return MRL_OK;
 }
@@ -543,14 +690,11 @@ int mrl_normalize_advantages(mrl_ctx *ctx, float *x, int n) {
     MRL_CHECK_ARG(n >= 0, "mrl_normalize_advantages: negative size");
     if (n == 0) return MRL_OK;
     MRL_CHECK_ARG(x, "mrl_normalize_advantages: NULL buffer");
-    int nb = std::min(1024, grid_for(n, TPB));
-    float *part = ctx->reduce_scratch;         // [0, nb)
-    float *stats = ctx->reduce_scratch + 2048;  // mean, variance
-    hipLaunchKernelGGL(partial_sum_kernel, dim3(nb), dim3(TPB), 0, ctx->stream, x, n, (const float *)nullptr, part);
-    hipLaunchKernelGGL(finish_mean_kernel, dim3(1), dim3(TPB), 0, ctx->stream, part, nb, n, stats);
-    hipLaunchKernelGGL(partial_sum_kernel, dim3(nb), dim3(TPB), 0, ctx->stream, x, n, (const float *)stats, part);
-    hipLaunchKernelGGL(finish_mean_kernel, dim3(1), dim3(TPB), 0, ctx->stream, part, nb, n, stats + 1);
-    hipLaunchKernelGGL(normalize_apply_kernel, dim3(grid_for(n, TPB)), dim3(TPB), 0, ctx->stream, x, n, stats);
+    const int nb = std::min(NORM_BLOCKS, grid_for(n, TPB));
+    float *sums = ctx->reduce_scratch, *squares = sums + NORM_BLOCKS;
+    hipLaunchKernelGGL(partial_sum_kernel, dim3(nb), dim3(TPB), 0, ctx->stream, x, n, (const float *)nullptr, sums);
+    hipLaunchKernelGGL(partial_sum_kernel, dim3(nb), dim3(TPB), 0, ctx->stream, x, n, (const float *)sums, squares);
+    hipLaunchKernelGGL(normalize_apply_kernel, dim3(nb), dim3(TPB), 0, ctx->stream, x, n, nb, sums, squares);
     MRL_CHECK_LAUNCH();
     return MRL_OK;
 }
