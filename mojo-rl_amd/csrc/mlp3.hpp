@@ -1,4 +1,4 @@
-// Host-side interface of the fused three-layer MLP kernels (mrl_mlp3.hip).
+// Host-side interface of the fused three-layer MLP kernels (mrl_mlp3.hip, mrl_rows.hip, mrl_fb.hip).
 #pragma once
 #include "mrl_host.hpp"
 
@@ -11,8 +11,9 @@ struct Mlp3Net {
     float *out;              // forward: [B, A] or [B, 2A]
     float *cache;            // forward: written when non-null; backward: read
     const float *grad_out;   // backward
-    float *g1, *g0, *ls_part, *db_part, *thin_part;  // backward workspace (set by the host function)
-    // fused update, for the weight-gradient launch: h1 and g1 split, as operands contracted over the batch rows
+    float *grad_in;          // backward: written when non-null
+    float *ls_part, *db_part, *thin_part;            // workspace: the row tiles' pieces (set by the host function)
+    // for the weight-gradient launch: h1 and g1 split, as operands contracted over the batch rows
     // (mlp_split.hpp: k-step = 32 batch rows, the other index = column)
     unsigned short *h1q, *g1q;
     const unsigned short *wf, *wb;                   // fused update: the hidden layer's weights split (mlp_split.hpp), forward / W^T
@@ -48,15 +49,12 @@ bool mlp3_fusable(const mrl_mlp_desc &d, int *H, int *act, bool *gauss);
 bool mlp3_pair_fusable(const mrl_mlp_desc &a, const mrl_mlp_desc &b);
 int mlp3_forward(mrl_ctx *ctx, const mrl_mlp_desc &d, int batch, const float *in, const float *params,
                  float *out, float *cache);
-size_t mlp3_backward_ws(const mrl_mlp_desc *const *descs, int n_nets, int batch);
 int mlp3_backward(mrl_ctx *ctx, const mrl_mlp_desc &d, int batch, const float *grad_out, const float *params,
-                  const float *cache, float *grads, float *ws);
-int mlp3_backward_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, int batch, Mlp3Nets io,
-                    float *const *grads, float *ws);
+                  const float *cache, float *grads, float *grad_in);
 
 // The fused update of two nets: one kernel per row tile runs forward (inputs read through loss.idx, io.n[i].out
 // written), loss gradients and the way back (mrl_fb.hip), then the H x H weight gradients and the sums over the tiles.
-// Workspace: UpdateWs, carved from the context's.
+// Workspace: UpdateWs, carved from the context's; the backward of one net (mrl_rows.hip) uses it as well.
 struct UpdateWs {
     int rows, tiles;          // batch rows per tile
     bool dw_in_tiles;
@@ -65,13 +63,15 @@ struct UpdateWs {
     float *partial;
     int splits, steps_per;    // batch splits of the weight-gradient launch, k-steps of 32 rows each
 };
-int mlp3_update_ws(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int batch, const float *const *params, UpdateWs *out);
+int mlp3_update_ws(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, int batch, const float *const *params, UpdateWs *out);
 int launch_split_weights(mrl_ctx *ctx, int H, const SplitNets &s, int n_nets);
 // sq_part (nullable): receives per-block sums of squares of the gradients, [net * 1024 + block];
 // *sq_blocks = number of blocks written (0 when none were)
 int mlp3_update_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int batch, Mlp3Nets io, const UpdateWs &ws,
                   float *const *grads, float *sq_part, int *sq_blocks, const FwdLoss &loss);
-int launch_dw_frag(mrl_ctx *ctx, int H, int batch, const UpdateWs &ws, int P0, int Ptot, int w1_off);
+int launch_fwd16(mrl_ctx *ctx, int H, int act, int batch, int IN, const Mlp3Net &nn);
+int launch_bwd(mrl_ctx *ctx, int H, int act, int batch, int IN, int rows, const Mlp3Net &nn, bool dw_in_tiles);
+int launch_dw_frag(mrl_ctx *ctx, int H, int n_nets, int batch, const UpdateWs &ws, int P0, int Ptot, int w1_off);
 int launch_fb(mrl_ctx *ctx, int H, int act, int batch, int IN, int rows, const Mlp3Nets &nets, const FwdLoss &fl);
 // grows the context's MLP workspace to at least `floats`
 int mlp_ensure_ws(mrl_ctx *ctx, size_t floats, float **out);

@@ -25,54 +25,16 @@
 #include "mlp_tile.hpp"
 #include "mlp_split.hpp"
 #include "mlp3.hpp"
+#include "mlp_rows16.hpp"
 #include "ppo_grads.hpp"
 
 namespace mrl {
 
 struct DwFrag {
+    int n;        // nets
     const unsigned short *x[2], *g[2];
     int off[2];   // of the net's W1 gradient in a split's partial vector
 };
-
-template <int ACT>
-MRL_DEV float act_deriv_out(float y) {
-    if (ACT == 1) return y > 0.0f ? 1.0f : 0.0f;
-    if (ACT == 2) return 1.0f - y * y;
-    return 1.0f;
-}
-
-// sum over the sixteen lanes of a row (DPP rotations within the row), on all of them
-MRL_DEV float row16_sum(float x) {
-    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x128, 0xf, 0xf, false));   // row_ror:8
-    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x124, 0xf, 0xf, false));   // row_ror:4
-    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x122, 0xf, 0xf, false));   // row_ror:2
-    x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x121, 0xf, 0xf, false));   // row_ror:1
-    return x;
-}
-
-// A tile's rows of column tile ct (RT = 1: of ct and ct + 1) of f [16 RT][LD] (LDS), split, as the operand pieces that a
-// product contracted over the batch rows reads (k-step = 32 rows): lane 16 g + n holds rows 8 g .. 8 g + 7 of column n.
-// A tile of 16 rows fills half a k-step: it takes two column tiles per wavefront; the last tile of an odd count puts
-// zeros where the other half would be.
-template <int H, int RT, int LD>
-MRL_DEV void batch_operand(const float *f, unsigned short *dst, int ct, int lane) {
-    const int g = lane >> 4, n = lane & 15;
-    const int c = ct + (RT == 1 ? g >> 1 : 0), rg = RT == 1 ? g & 1 : g;
-    const int ks = RT == 1 ? blockIdx.x >> 1 : blockIdx.x, gs = RT == 1 ? 2 * (blockIdx.x & 1) + rg : g;
-    f32x8 x;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) x[j] = f[(8 * rg + j) * LD + 16 * c + n];
-    bf16x8 p[SPLIT];
-    split8(x, p);
-    const bool pad = RT == 1 && blockIdx.x == gridDim.x - 1 && (blockIdx.x & 1) == 0;
-#pragma unroll
-    for (int i = 0; i < SPLIT; ++i) {
-        *reinterpret_cast<bf16x8 *>(dst + split_frag<H>(ks, c, i, 16 * gs + n)) = p[i];
-        if (pad) *reinterpret_cast<uint4 *>(dst + split_frag<H>(ks, c, i, 16 * (gs + 2) + n)) = make_uint4(0, 0, 0, 0);
-    }
-}
-
-constexpr int fb_threads(int H) { return H == 64 ? 256 : 512; }
 
 template <int H, int ACT, int RT>
 __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, Mlp3Nets nets, FwdLoss fl) {
@@ -503,7 +465,7 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
     }
 }
 
-// dW = h1^T g1 of the hidden layer of both nets over a split of the batch: partial[split][Ptot].  Operands as the row
+// dW = h1^T g1 of the hidden layer of one or two nets over a split of the batch: partial[split][Ptot].  Operands as the row
 // tiles left them (split, in operand order), straight from global memory into registers: no LDS, no barrier.  A
 // workgroup makes one 64 x 128 output tile (four wavefronts, 32 x 64 each) twice over, two groups of wavefronts taking
 // alternate k-steps of 32 batch rows and adding up at the end.
@@ -520,7 +482,7 @@ __global__ __launch_bounds__(512) void dw_frag_kernel(DwFrag d, int steps, int s
     constexpr int XCDS = 8, TN = 128, tiles_n = H / TN, tiles = tiles_n * (H / 64), NB = 4, RLD = TN + 4;
     static_assert(H % TN == 0, "whole tiles");
     __shared__ float sum[64 * RLD];
-    const int groups = 2 * splits;
+    const int groups = d.n * splits;
     // workgroup n = (round r, XCD x): the r-th workgroup that XCD x receives.  An XCD walks its groups x, x + 8, ... one
     // after the other, `tiles` workgroups each; the workgroups of a short last round keep the plain order.
     int grp, tile;
@@ -591,15 +553,16 @@ __global__ __launch_bounds__(512) void dw_frag_kernel(DwFrag d, int steps, int s
 }
 
 // P0: parameters of the first net, w1_off: offset of W1 in a net's parameters
-int launch_dw_frag(mrl_ctx *ctx, int H, int batch, const UpdateWs &ws, int P0, int Ptot, int w1_off) {
-    DwFrag d;
-    for (int i = 0; i < 2; ++i) {
+int launch_dw_frag(mrl_ctx *ctx, int H, int n_nets, int batch, const UpdateWs &ws, int P0, int Ptot, int w1_off) {
+    DwFrag d{};
+    d.n = n_nets;
+    for (int i = 0; i < n_nets; ++i) {
         d.x[i] = ws.net[i].h1q;
         d.g[i] = ws.net[i].g1q;
         d.off[i] = (i ? P0 : 0) + w1_off;
     }
     const int steps = (batch + 31) / 32;
-    const dim3 grid(2 * ws.splits * (H / 64) * (H / 128)), block(512);
+    const dim3 grid(n_nets * ws.splits * (H / 64) * (H / 128)), block(512);
     if (H == 256) hipLaunchKernelGGL(dw_frag_kernel<256>, grid, block, 0, ctx->stream, d, steps, ws.steps_per, ws.splits, Ptot, ws.partial);
     else if (H == 128) hipLaunchKernelGGL(dw_frag_kernel<128>, grid, block, 0, ctx->stream, d, steps, ws.steps_per, ws.splits, Ptot, ws.partial);
     else return MRL_E_UNSUPPORTED;

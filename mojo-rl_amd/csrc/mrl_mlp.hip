@@ -367,18 +367,8 @@ int mrl_mlp_backward(mrl_ctx *ctx, const mrl_mlp_desc *d, int batch, const float
     if (rc) return rc;
     MRL_CHECK_ARG(batch > 0, "mrl_mlp_backward: batch must be positive");
     MRL_CHECK_ARG(grad_out && params && cache && grads, "mrl_mlp_backward: NULL buffer");
-    {
-        int fh, fa;
-        bool fg;
-        if (grad_in == nullptr && mlp3_fusable(*d, &fh, &fa, &fg)) {
-            float *fws = nullptr;
-            const mrl_mlp_desc *ds[1] = {d};
-            rc = ensure_ws(ctx, mlp3_backward_ws(ds, 1, batch), &fws);
-            if (rc) return rc;
-            rc = mlp3_backward(ctx, *d, batch, grad_out, params, cache, grads, fws);
-            if (rc != MRL_E_UNSUPPORTED) return rc;
-        }
-    }
+    rc = mlp3_backward(ctx, *d, batch, grad_out, params, cache, grads, grad_in);
+    if (rc != MRL_E_UNSUPPORTED) return rc;
 
     size_t poff[MRL_MAX_LAYERS], coff[MRL_MAX_LAYERS];
     size_t p = 0, c = 0;

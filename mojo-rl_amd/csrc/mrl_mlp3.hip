@@ -1,16 +1,13 @@
-// Fused kernels for three-layer nets  IN -> H -> H -> out  (H in {64, 128, 256}, IN <= 32, out <= 8 or a
+// The fused passes over three-layer nets  IN -> H -> H -> out  (H in {64, 128, 256}, IN <= 32, out <= 8 or a
 // StochasticActor head of <= 8 actions): the shapes of every actor and critic the PPO agents build
 // (deep_agents/ppo/ppo.mojo:779-817, ppo_continuous.mojo:171-194).
 //
 //   mlp3_fwd_kernel     the whole forward of a 32-row tile in one launch (hidden activations
-//                       stay in LDS), writing the reference's per-layer cache on the way;
-//   mlp3_bwd_dx_kernel  the chain  g2 -> g1 = (g2 W2^T) * act' -> g0 = (g1 W1^T) * act'  of a
-//                       32-row tile in one launch; g1 and g0 go to a workspace;
-//   dw3_kernel          dW of the hidden layer, split over the batch;
-//   sum3_kernel         sum of the splits and of the row tiles' pieces straight into the flat gradient vector.
-// They replace 3 + 2 + 3 + 3 launches of the per-layer kernels (which remain the path for any
-// other shape, and for callers that ask for the gradient with respect to the input).  The minibatch update's
-// row tiles (mrl_fb.hip) share the last one.
+//                       stay in LDS), writing the reference's per-layer cache on the way, for batches
+//                       beyond those that the 16-row tiles of mrl_rows.hip take;
+//   sum3_kernel         sum of the batch splits and of the row tiles' pieces straight into the flat gradient vector;
+// and the host side of these, of the backward (mrl_rows.hip) and of the minibatch update (mrl_fb.hip).  The per-layer
+// kernels (mrl_mlp.hip) remain the path for any other shape.
 #include "mrl_host.hpp"
 #include "mrl_device.hpp"
 #include "mlp_tile.hpp"
@@ -84,301 +81,6 @@ __global__ __launch_bounds__(2 * H) void mlp3_fwd_kernel(int B, int IN, Mlp3Nets
             else if (v > 2.0f) v = 2.0f;
         }
         out[(row0 + r) * ld + a] = v;
-    }
-}
-
-template <int ACT>
-MRL_DEV float act_deriv(float cached) {
-    if (ACT == 1) return cached > 0.0f ? 1.0f : 0.0f;
-    if (ACT == 2) return 1.0f - cached * cached;
-    return 1.0f;
-}
-
-// grad_out [B, ld] (ld = A, or 2A for the Gaussian head: mean gradients first); g1, g0 [B, H];
-// ls_part [tiles, A]: per-tile sums of the log_std gradient columns.  grid = (row tiles, nets).
-template <int H, int ACT>
-__global__ __launch_bounds__(2 * H) void mlp3_bwd_dx_kernel(int B, int IN, Mlp3Nets nets) {
-    constexpr int T = 2 * H;   // one 32-column accumulator tile per wavefront
-    const Mlp3Net &nn = nets.n[blockIdx.y];
-    const float *__restrict__ grad_out = nn.grad_out;
-    const float *__restrict__ params = nn.params;
-    const float *__restrict__ cache = nn.cache;
-    float *__restrict__ g1 = nn.g1;
-    float *__restrict__ g0 = nn.g0;
-    float *__restrict__ ls_part = nn.ls_part;
-    float *__restrict__ db_part = nn.db_part + (size_t)blockIdx.x * (2 * H + PA_MAX);   // this tile's slice
-    const int A = nn.A;
-    // this tile's share of the two thin weight gradients: [dW0 (IN x H) | dW2 (H x A)]
-    float *__restrict__ thin_part = nn.thin_part + (size_t)blockIdx.x * (size_t)nn.thin_stride;
-    const bool GAUSS = nn.gauss != 0;
-    constexpr int KCH = 64;                       // k-chunk of W1 staged per round
-    __shared__ float g2s[PR * (2 * PA_MAX + 1)];
-    __shared__ float xs[PR * XS_LD];              // the tile's inputs, for dW0
-    __shared__ float gT[H * HT_LD];               // g1 of the tile, k-major
-    __shared__ float wT[KCH * (H + 1)];           // W1[i][o0 + k] stored as [k][i]
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6, half = lane >> 5, l31 = lane & 31;
-    const long row0 = (long)blockIdx.x * PR;
-    const int nrow = (int)min((long)PR, B - row0);
-    const int ld = GAUSS ? 2 * A : A;
-    const float *c0 = cache, *c1 = cache + (size_t)B * (IN + H), *c2 = c1 + (size_t)B * 2 * H;
-    const float *W1 = params + IN * H + H;
-    const float *W2 = W1 + H * H + H;
-    // what the later phases need from global memory is requested now, in few wide loads (a
-    // wavefront can keep 64 vector-memory instructions in flight), so that the block waits for
-    // memory once: the cached activations behind act' of both hidden layers as row tiles, the head
-    // weights, the first chunk of W1
-    static_assert(PR * H == 4 * 4 * T && 2 * PR * H <= KCH * (H + 1), "tile staging layout");
-    float4 t1[4], t2[4];   // 32 x H tiles of the layer-1 cache entries and of h2, 16 bytes per thread and load
-    float w2row[PA_MAX];   // thread t < H: W2[t][:]
-    float d0[16];          // layer-0 cache entries at this lane's accumulator positions
-    const int wrow = t % H, wseg = (t / H) * (KCH / 2);   // thread copies W1[wrow][o0 + wseg .. + KCH / 2)
-    float4 nxt[KCH / 8];
-    auto fetch = [&](int o0) {
-        const float4 *src = reinterpret_cast<const float4 *>(W1 + (size_t)wrow * H + o0 + wseg);
-#pragma unroll
-        for (int q = 0; q < KCH / 8; ++q) nxt[q] = src[q];
-    };
-    {
-        const bool vec = ((reinterpret_cast<uintptr_t>(c1) | reinterpret_cast<uintptr_t>(c2)) & 15) == 0;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int e = 4 * (t + q * T), r = e / H, ci = e % H;
-            const float *s1 = c1 + (row0 + r) * (2 * H) + H + ci;
-            const float *s2 = c2 + (row0 + r) * H + ci;
-            t1[q] = t2[q] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            if (r < nrow) {
-                if (vec) {
-                    t1[q] = *reinterpret_cast<const float4 *>(s1);
-                    t2[q] = *reinterpret_cast<const float4 *>(s2);
-                } else {
-                    t1[q] = make_float4(s1[0], s1[1], s1[2], s1[3]);
-                    t2[q] = make_float4(s2[0], s2[1], s2[2], s2[3]);
-                }
-            }
-        }
-#pragma unroll
-        for (int a = 0; a < PA_MAX; ++a) w2row[a] = a < A ? W2[wrow * A + a] : 0.0f;
-        const int colq = 32 * w + l31;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const int row = 8 * (v >> 2) + 4 * half + (v & 3);
-            d0[v] = row < nrow ? c0[(row0 + row) * (IN + H) + IN + colq] : 0.0f;
-        }
-        fetch(0);
-    }
-    for (int i = t; i < PR * ld; i += T) {
-        const int r = i / ld, a = i - r * ld;
-        g2s[r * (2 * PA_MAX + 1) + a] = r < nrow ? grad_out[row0 * ld + i] : 0.0f;
-    }
-    for (int i = t; i < PR * IN; i += T) {
-        const int r = i / IN, k = i - r * IN;
-        xs[r * XS_LD + k] = r < nrow ? c0[(row0 + r) * (IN + H) + k] : 0.0f;
-    }
-    // the two tiles rest in the W1 staging buffer until the chunk loop claims it
-    float *tile1 = wT, *tile2 = wT + PR * H;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int e = 4 * (t + q * T);
-        *reinterpret_cast<float4 *>(tile1 + e) = t1[q];
-        *reinterpret_cast<float4 *>(tile2 + e) = t2[q];
-    }
-    __syncthreads();
-    if (t < H) {   // g1[r][n] = (sum_a g2[r][a] W2[n][a]) * act'(layer 1); thread t owns column n = t
-        float colsum = 0.0f;
-#pragma unroll
-        for (int r = 0; r < PR; ++r) {
-            float s = 0.0f;
-#pragma unroll
-            for (int a = 0; a < PA_MAX; ++a)
-                if (a < A) s = fmaf(g2s[r * (2 * PA_MAX + 1) + a], w2row[a], s);
-            float g = 0.0f;
-            if (r < nrow) {
-                g = s * act_deriv<ACT>(tile1[r * H + t]);
-                g1[(row0 + r) * H + t] = g;
-            }
-            gT[t * HT_LD + r] = g;
-            colsum += g;
-        }
-        db_part[H + t] = colsum;   // bias gradient of layer 1, this tile's rows
-    } else {       // meanwhile the other half of the block: dW2[n][a] of the tile = sum_r h2[r][n] g2[r][a]
-        const int n = t - H;
-        float s[PA_MAX];
-#pragma unroll
-        for (int a = 0; a < PA_MAX; ++a) s[a] = 0.0f;
-#pragma unroll
-        for (int r = 0; r < PR; ++r) {
-            const float h = tile2[r * H + n];
-#pragma unroll
-            for (int a = 0; a < PA_MAX; ++a)
-                if (a < A) s[a] = fmaf(h, g2s[r * (2 * PA_MAX + 1) + a], s[a]);
-        }
-        float *o2 = thin_part + (size_t)IN * H + (size_t)n * A;
-#pragma unroll
-        for (int a = 0; a < PA_MAX; ++a)
-            if (a < A) o2[a] = s[a];
-        if (n < ld) {   // column sums of the tile: bias gradient of the head, log_std gradient
-            float cs2 = 0.0f;
-            for (int r = 0; r < PR; ++r) cs2 += g2s[r * (2 * PA_MAX + 1) + n];
-            if (n < A) db_part[2 * H + n] = cs2;
-            else ls_part[(long)blockIdx.x * A + (n - A)] = cs2;
-        }
-    }
-    // dh1 = g1 W1^T: wavefront w owns input columns [32w, 32w + 32).  The next chunk of W1 is
-    // fetched into registers while the matrix cores work on the current one.
-    floatx16 acc = {0};
-    const int col = 32 * w + l31;
-    for (int o0 = 0; o0 < H; o0 += KCH) {
-        __syncthreads();   // gT complete (first round) / previous chunk consumed
-#pragma unroll
-        for (int q = 0; q < KCH / 8; ++q) {
-            wT[(wseg + 4 * q + 0) * (H + 1) + wrow] = nxt[q].x;
-            wT[(wseg + 4 * q + 1) * (H + 1) + wrow] = nxt[q].y;
-            wT[(wseg + 4 * q + 2) * (H + 1) + wrow] = nxt[q].z;
-            wT[(wseg + 4 * q + 3) * (H + 1) + wrow] = nxt[q].w;
-        }
-        __syncthreads();
-        if (o0 + KCH < H) fetch(o0 + KCH);
-        __builtin_amdgcn_sched_barrier(0);   // keep the loads ahead of the MFMAs that hide them
-#pragma unroll
-        for (int kk = 0; kk < KCH / 2; ++kk) {
-            const int k = 2 * kk + half;
-            const float a = gT[(o0 + k) * HT_LD + l31];
-            const float b = wT[k * (H + 1) + col];
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, acc, 0, 0, 0);
-        }
-    }
-    float cs = 0.0f;
-    float gv[16];
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        const int row = 8 * (v >> 2) + 4 * half + (v & 3);
-        gv[v] = 0.0f;
-        if (row >= nrow) continue;
-        const float val = acc[v] * act_deriv<ACT>(d0[v]);
-        g0[(row0 + row) * H + col] = val;
-        gv[v] = val;
-        cs += val;
-    }
-    // the two halves of the wavefront hold the other 16 rows of the same column
-    cs += __shfl_xor(cs, 32, 64);
-    if (half == 0) db_part[col] = cs;   // bias gradient of layer 0, this tile's rows
-    // dW0[i][col] of the tile = sum_r x[r][i] g0[r][col]
-    for (int i = 0; i < IN; ++i) {
-        float s = 0.0f;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) s = fmaf(xs[(8 * (v >> 2) + 4 * half + (v & 3)) * XS_LD + i], gv[v], s);
-        s += __shfl_xor(s, 32, 64);
-        if (half == 0) thin_part[(size_t)i * H + col] = s;
-    }
-}
-
-// ---------------------------------------------------------------- [dW | db] of the three layers
-constexpr int DBM = 64, DBN = 64, DKC = 32, DLD = 65;
-
-struct DwProblem {
-    const float *X;   // layer input per batch row (row stride xs)
-    const float *G;   // gradient at the layer's pre-activation (row stride gs)
-    int xs, gs, K, N; // K inputs, N outputs: the block written is dW [K, N]
-    int poff;         // offset of the layer's W in the flat parameter vector
-    int tiles_n, tiles;   // tiles_n = ceil(N / 64); tiles = tiles_n * ceil(K / 64)
-    int vec;              // rows of X and G can be read with 16-byte loads, K and N are multiples of 64
-};
-struct DwSet { DwProblem p[6]; int n; };
-
-// dW = X^T G of every problem, split over the batch: grid.x = sum of the problems' tiles,
-// grid.y = batch splits; partial[z][P].  The next 32-row chunk is fetched into registers while
-// the matrix cores work on the current one.
-// Workgroups go to the chip's eight XCDs in turn (workgroup n to XCD n % 8), and each XCD has an L2 of its
-// own.  The tiles of one (problem, batch split) read the same rows of X and G -- every 64-column block of X
-// is wanted by all tiles of its tile row, every block of G by all tiles of its tile column --, so the
-// launch is a flat list of workgroups ordered so that those tiles sit on ONE XCD: the group is fetched
-// from memory once and its re-reads are L2 hits (measured: 50 MB -> 17 MB fetched per launch at a
-// minibatch of 4096, which is what X and G hold).  groups = problems x splits, `tiles` workgroups each
-// (every problem of a launch has the same number of tiles); group g runs on XCD g % 8.
-constexpr int XCDS = 8;
-
-__global__ __launch_bounds__(256) void dw3_kernel(DwSet d, int M, int rows_per_split, int P,
-                                                  float *__restrict__ partial, int splits) {
-    __shared__ float As[DKC * DLD];
-    __shared__ float Bs[DKC * DLD];
-    const int tiles = d.p[0].tiles, groups = d.n * splits;
-    // workgroup n = (round r, XCD x): the r-th workgroup that XCD x receives.  An XCD walks its groups
-    // g = x, x + 8, ... one after the other, `tiles` workgroups each; with a group count that is not a
-    // multiple of 8 the last round is short and its workgroups keep the plain order.
-    int g, tile;
-    {
-        const int n = blockIdx.x, full = (groups / XCDS) * XCDS * tiles;   // workgroups of whole rounds of 8 groups
-        if (n < full) {
-            const int x = n % XCDS, q = n / XCDS;
-            tile = q % tiles;
-            g = (q / tiles) * XCDS + x;
-        } else {
-            const int m = n - full;
-            tile = m % tiles;
-            g = (groups / XCDS) * XCDS + m / tiles;
-        }
-    }
-    const int li = g / splits, z = g % splits;
-    const DwProblem &pr = d.p[li];
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6, wr = w >> 1, wc = w & 1;
-    const int half = lane >> 5, l31 = lane & 31;
-    const int j0 = (tile % pr.tiles_n) * DBN, i0 = (tile / pr.tiles_n) * DBM;
-    const long b_begin = (long)z * rows_per_split;
-    long b_end = b_begin + rows_per_split;
-    if (b_end > M) b_end = M;
-    floatx16 acc = {0};
-    const int bb = t >> 3, seg = (t & 7) * 8;
-    float xa[8], gb[8];
-    // each thread moves 8 consecutive floats of X and of G per chunk: two 16-byte loads each when
-    // the problem allows (whole tiles inside K and N, 16-byte aligned rows), scalar loads otherwise
-    const bool vec = pr.vec != 0;
-    auto fetch = [&](long b0) {
-        const long b = b0 + bb;
-        const bool inb = b < b_end;
-        if (vec) {
-            float4 x0 = {0, 0, 0, 0}, x1 = x0, g0 = x0, g1 = x0;
-            if (inb) {
-                const float4 *px = reinterpret_cast<const float4 *>(pr.X + b * pr.xs + i0 + seg);
-                const float4 *pg = reinterpret_cast<const float4 *>(pr.G + b * pr.gs + j0 + seg);
-                x0 = px[0]; x1 = px[1]; g0 = pg[0]; g1 = pg[1];
-            }
-            xa[0] = x0.x; xa[1] = x0.y; xa[2] = x0.z; xa[3] = x0.w; xa[4] = x1.x; xa[5] = x1.y; xa[6] = x1.z; xa[7] = x1.w;
-            gb[0] = g0.x; gb[1] = g0.y; gb[2] = g0.z; gb[3] = g0.w; gb[4] = g1.x; gb[5] = g1.y; gb[6] = g1.z; gb[7] = g1.w;
-            return;
-        }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int ii = i0 + seg + i, j = j0 + seg + i;
-            xa[i] = (inb && ii < pr.K) ? pr.X[b * pr.xs + ii] : 0.0f;
-            gb[i] = (inb && j < pr.N) ? pr.G[b * pr.gs + j] : 0.0f;
-        }
-    };
-    fetch(b_begin);
-    for (long b0 = b_begin; b0 < b_end; b0 += DKC) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            As[bb * DLD + seg + i] = xa[i];
-            Bs[bb * DLD + seg + i] = gb[i];
-        }
-        __syncthreads();
-        if (b0 + DKC < b_end) fetch(b0 + DKC);
-        __builtin_amdgcn_sched_barrier(0);   // keep the loads ahead of the MFMAs that hide them
-#pragma unroll
-        for (int kk = 0; kk < DKC; kk += 2) {
-            const float a = As[(kk + half) * DLD + 32 * wr + l31];
-            const float bv = Bs[(kk + half) * DLD + 32 * wc + l31];
-            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a, bv, acc, 0, 0, 0);
-        }
-        __syncthreads();
-    }
-    const int col = j0 + 32 * wc + l31;
-    if (col < pr.N) {
-        float *out = partial + (size_t)z * P + pr.poff;
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const int row = i0 + 32 * wr + 8 * (v >> 2) + 4 * half + (v & 3);
-            if (row < pr.K) out[(size_t)row * pr.N + col] = acc[v];
-        }
     }
 }
 
@@ -496,8 +198,8 @@ static int net_P(const mrl_mlp_desc &d) {
 // 2048 / 4096 rows, 16 against 32: H = 64 14.0 / 15.5 / 17.8 / 23.3 : 18.1 / 17.7 / 18.0 / 20.6; H = 256 33.8 / 37.3 /
 // 40.8 / 60.5 : 40.9 / 42.3 / 45.1 / 50.4; H = 128, whose pieces hold the H x H gradient as well, 17.6 / 21.9 / 26.5 /
 // 33.3 : 22.9 / 23.1 / 25.8 / 29.9, hence half the bound there.
-static int fb_tile_rows(int n_cus, int H, int batch) {
-    return 2 * ((batch + 15) / 16) <= (H == 128 ? n_cus / 2 : n_cus) ? 16 : 32;
+static int fb_tile_rows(int n_cus, int H, int n_nets, int batch) {
+    return n_nets * ((batch + 15) / 16) <= (H == 128 ? n_cus / 2 : n_cus) ? 16 : 32;
 }
 
 // Whether the fused update kernel takes the hidden layer's weight gradient of its row tile itself
@@ -512,16 +214,18 @@ bool mlp3_pair_fusable(const mrl_mlp_desc &a, const mrl_mlp_desc &b) {
            a.layers[0].in_dim == b.layers[0].in_dim;
 }
 
+// Whether the forward takes 16 rows per workgroup (mrl_rows.hip) or 32: 16 while a CU gets one workgroup at H = 256 (its
+// eight wavefronts hold W1 in registers, a second one waits for them), two at H = 128, and as far as measured at H = 64.
+// us, 16 against 32 rows, cache written, tanh, 24 inputs: H = 256 13.9 : 18.5 (33 rows), 17.7 : 20.9 (4096), 31.6 : 22.9
+// (8191); H = 128 7.1 : 10.6 (33), 11.7 : 13.7 (8191), 18.5 : 18.3 (16384); H = 64 5.7 : 10.4 (33), 10.1 : 15.7 (16384).
+static bool fwd_rows_16(int n_cus, int H, int batch) {
+    return (batch + 15) / 16 <= (H == 256 ? 1 : H == 128 ? 2 : 16) * n_cus;
+}
+
 template <int H, int ACT>
 static void launch_fwd_t(mrl_ctx *ctx, int batch, int IN, const Mlp3Nets &nets) {
     hipLaunchKernelGGL((mlp3_fwd_kernel<H, ACT>), dim3((batch + PR - 1) / PR), dim3(2 * H), 0, ctx->stream, batch, IN, nets);
 }
-template <int H, int ACT>
-static void launch_bwd_t(mrl_ctx *ctx, int batch, int IN, const Mlp3Nets &nets, int n_nets) {
-    dim3 grid((batch + PR - 1) / PR, n_nets);
-    hipLaunchKernelGGL((mlp3_bwd_dx_kernel<H, ACT>), grid, dim3(2 * H), 0, ctx->stream, batch, IN, nets);
-}
-
 int mlp3_forward(mrl_ctx *ctx, const mrl_mlp_desc &d, int batch, const float *in, const float *params,
                  float *out, float *cache) {
     int H = 0, act = 0;
@@ -532,6 +236,7 @@ int mlp3_forward(mrl_ctx *ctx, const mrl_mlp_desc &d, int batch, const float *in
     io.n[0].A = d.layers[2].out_dim;
     io.n[0].gauss = gauss ? 1 : 0;
     const int IN = d.layers[0].in_dim;
+    if (fwd_rows_16(ctx->n_cus, H, batch)) return launch_fwd16(ctx, H, act, batch, IN, io.n[0]);
     if (H == 256 && act == 1) launch_fwd_t<256, 1>(ctx, batch, IN, io);
     else if (H == 256) launch_fwd_t<256, 2>(ctx, batch, IN, io);
     else if (H == 128 && act == 1) launch_fwd_t<128, 1>(ctx, batch, IN, io);
@@ -542,23 +247,10 @@ int mlp3_forward(mrl_ctx *ctx, const mrl_mlp_desc &d, int batch, const float *in
     return MRL_OK;
 }
 
-// floats of workspace mlp3_backward_n needs for these nets
-size_t mlp3_backward_ws(const mrl_mlp_desc *const *descs, int n_nets, int batch) {
-    size_t total = 0, P = 0;
-    for (int i = 0; i < n_nets; ++i) {
-        const int H = descs[i]->layers[0].out_dim;
-        const int IN = descs[i]->layers[0].in_dim, A = descs[i]->layers[2].out_dim;
-        total += (size_t)2 * batch * H +
-                 (size_t)((batch + PR - 1) / PR) * (2 * PA_MAX + 2 * H + (size_t)IN * H + (size_t)H * A);
-        P += net_P(*descs[i]);
-    }
-    return total + (size_t)32 * P;
-}
-
 // batch splits of the weight-gradient launch: slices of whole k-chunks
-static void dw_splits(int batch, int *splits, int *rows_per) {
-    int s = std::max(1, std::min(32, batch / 256));
-    *rows_per = ((batch + s - 1) / s + DKC - 1) / DKC * DKC;
+static void dw_splits(int n_nets, int batch, int *splits, int *rows_per) {
+    int s = std::max(1, std::min(32, batch / (128 * n_nets)));
+    *rows_per = ((batch + s - 1) / s + 31) / 32 * 32;
     *splits = (batch + *rows_per - 1) / *rows_per;
 }
 
@@ -594,76 +286,18 @@ static int sum_tiles(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets,
     return MRL_OK;
 }
 
-// backward (parameter gradients only) of one or two nets: io.n[i].grad_out / params / cache in,
-// grads[i] out; ws as sized by mlp3_backward_ws
-int mlp3_backward_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, int batch, Mlp3Nets io,
-                    float *const *grads, float *ws) {
-    int H = 0, act = 0;
-    bool gauss = false;
-    for (int i = 0; i < n_nets; ++i) {
-        if (!mlp3_fusable(*descs[i], &H, &act, &gauss)) return MRL_E_UNSUPPORTED;
-        io.n[i].A = descs[i]->layers[2].out_dim;
-        io.n[i].gauss = gauss ? 1 : 0;
-        // the W1 rows are staged with 16-byte loads
-        const int IN = descs[i]->layers[0].in_dim;
-        if (reinterpret_cast<uintptr_t>(io.n[i].params + IN * H + H) % 16 != 0) return MRL_E_UNSUPPORTED;
-    }
-    if (n_nets == 2 && !mlp3_pair_fusable(*descs[0], *descs[1])) return MRL_E_UNSUPPORTED;
-    const int IN = descs[0]->layers[0].in_dim;
-    const int tiles = (batch + PR - 1) / PR;
-    int splits, rows_per;
-    dw_splits(batch, &splits, &rows_per);
-    // workspace: per net g1 [B, H] | g0 [B, H] | ls_part [tiles, PA_MAX] | db_part [tiles, 2H + PA_MAX] |
-    // thin_part [tiles, IN H + H A]; then partial [splits, Ptot]
-    float *w = ws;
-    for (int i = 0; i < n_nets; ++i) {
-        io.n[i].g1 = w; w += (size_t)batch * H;
-        io.n[i].g0 = w; w += (size_t)batch * H;
-        io.n[i].ls_part = w; w += (size_t)tiles * PA_MAX;
-        io.n[i].db_part = w; w += (size_t)tiles * (2 * H + PA_MAX);
-        io.n[i].thin_stride = IN * H + H * descs[i]->layers[2].out_dim;
-        io.n[i].thin_part = w; w += (size_t)tiles * (size_t)io.n[i].thin_stride;
-    }
-    if (H == 256 && act == 1) launch_bwd_t<256, 1>(ctx, batch, IN, io, n_nets);
-    else if (H == 256) launch_bwd_t<256, 2>(ctx, batch, IN, io, n_nets);
-    else if (H == 128 && act == 1) launch_bwd_t<128, 1>(ctx, batch, IN, io, n_nets);
-    else if (H == 128) launch_bwd_t<128, 2>(ctx, batch, IN, io, n_nets);
-    else if (act == 1) launch_bwd_t<64, 1>(ctx, batch, IN, io, n_nets);
-    else launch_bwd_t<64, 2>(ctx, batch, IN, io, n_nets);
-    MRL_CHECK_LAUNCH();
-    DwSet dw;
-    dw.n = n_nets;   // the H x H layer of each net; the thin layers come out of the row tiles
-    int base = 0, total_tiles = 0;
-    for (int i = 0; i < n_nets; ++i) {
-        const float *c1 = io.n[i].cache + (size_t)batch * (IN + H);
-        DwProblem &p = dw.p[i];
-        p.X = c1; p.xs = 2 * H; p.G = io.n[i].g1; p.gs = H; p.K = H; p.N = H; p.poff = base + (IN + 1) * H;
-        p.tiles_n = (H + DBN - 1) / DBN;
-        p.tiles = p.tiles_n * ((H + DBM - 1) / DBM);
-        p.vec = (H % 64 == 0 && reinterpret_cast<uintptr_t>(c1) % 16 == 0 &&
-                 reinterpret_cast<uintptr_t>(io.n[i].g1) % 16 == 0) ? 1 : 0;
-        total_tiles += p.tiles;
-        base += net_P(*descs[i]);
-    }
-    // (both nets have the same width: every problem has the same number of tiles, see dw3_kernel)
-    hipLaunchKernelGGL(dw3_kernel, dim3(total_tiles * splits), dim3(256), 0, ctx->stream, dw, batch, rows_per, base, w,
-                       splits);
-    MRL_CHECK_LAUNCH();
-    return sum_tiles(ctx, descs, n_nets, io, tiles, false, w, splits, grads, nullptr, nullptr);
-}
-
-// carves (and if need be grows) the context's workspace for the fused update of two nets
-int mlp3_update_ws(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int batch, const float *const *params, UpdateWs *out) {
+// carves (and if need be grows) the context's workspace for the fused update of two nets, or the backward of one (params
+// null: no copies of the weights)
+int mlp3_update_ws(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, int batch, const float *const *params, UpdateWs *out) {
     const int H = descs[0]->layers[0].out_dim, IN = descs[0]->layers[0].in_dim;
     UpdateWs &u = *out;
     u = UpdateWs{};
-    u.rows = fb_tile_rows(ctx->n_cus, H, batch);
+    u.rows = fb_tile_rows(ctx->n_cus, H, n_nets, batch);
     u.tiles = (batch + u.rows - 1) / u.rows;
     u.dw_in_tiles = dw_in_tiles_pays(H, batch);
     int rows_per;
-    dw_splits(batch, &u.splits, &rows_per);
+    dw_splits(n_nets, batch, &u.splits, &rows_per);
     u.steps_per = rows_per / 32;
-    static_assert(DKC == 32, "splits of whole k-steps");
     size_t need = 0, P = 0;
     float *base = nullptr;
     for (int pass = 0; pass < 2; ++pass) {   // sizes, then pointers (every piece a multiple of four floats)
@@ -674,11 +308,13 @@ int mlp3_update_ws(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int batch, co
             return p;
         };
         P = 0;
-        for (int i = 0; i < 2; ++i) {
+        for (int i = 0; i < n_nets; ++i) {
             const int A = descs[i]->layers[2].out_dim;
-            u.split.w1[i] = params[i] + IN * H + H;
-            u.split.wf[i] = reinterpret_cast<unsigned short *>(take(split_elems(H) / 2));
-            u.split.wb[i] = reinterpret_cast<unsigned short *>(take(split_elems(H) / 2));
+            if (params != nullptr) {
+                u.split.w1[i] = params[i] + IN * H + H;
+                u.split.wf[i] = reinterpret_cast<unsigned short *>(take(split_elems(H) / 2));
+                u.split.wb[i] = reinterpret_cast<unsigned short *>(take(split_elems(H) / 2));
+            }
             if (!u.dw_in_tiles) {
                 const size_t elems = (size_t)SPLIT * ((batch + 31) / 32) * 32 * H;
                 u.net[i].h1q = reinterpret_cast<unsigned short *>(take(elems / 2));
@@ -720,19 +356,49 @@ int mlp3_update_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int batch, Mlp
     if (rc) return rc;
     if (!ws.dw_in_tiles) {
         const int P0 = net_P(*descs[0]);
-        rc = launch_dw_frag(ctx, H, batch, ws, P0, P0 + net_P(*descs[1]), (descs[0]->layers[0].in_dim + 1) * H);
+        rc = launch_dw_frag(ctx, H, 2, batch, ws, P0, P0 + net_P(*descs[1]), (descs[0]->layers[0].in_dim + 1) * H);
         if (rc) return rc;
     }
     return sum_tiles(ctx, descs, 2, io, ws.tiles, ws.dw_in_tiles, ws.partial, ws.splits, grads, sq_part, sq_blocks);
 }
 
+// true when [a, a + na) and [b, b + nb) (floats) share memory
+static bool overlap(const float *a, size_t na, const float *b, size_t nb) {
+    const uintptr_t pa = reinterpret_cast<uintptr_t>(a), pb = reinterpret_cast<uintptr_t>(b);
+    return pa < pb + 4 * nb && pb < pa + 4 * na;
+}
+
+// Backward of one net; MRL_E_UNSUPPORTED where the row tiles cannot take it: other shapes, parameters that 16-byte loads
+// do not reach, and an input gradient that lies over something that other tiles still read.
 int mlp3_backward(mrl_ctx *ctx, const mrl_mlp_desc &d, int batch, const float *grad_out, const float *params,
-                  const float *cache, float *grads, float *ws) {
-    Mlp3Nets io{};
-    io.n[0].grad_out = grad_out; io.n[0].params = params; io.n[0].cache = const_cast<float *>(cache);
+                  const float *cache, float *grads, float *grad_in) {
+    int H = 0, act = 0;
+    bool gauss = false;
+    if (!mlp3_fusable(d, &H, &act, &gauss) || reinterpret_cast<uintptr_t>(params) % 16 != 0) return MRL_E_UNSUPPORTED;
+    const int IN = d.layers[0].in_dim, A = d.layers[2].out_dim, P = net_P(d);
+    const size_t n_in = (size_t)batch * IN;
+    if (grad_in != nullptr &&
+        (overlap(grad_in, n_in, grad_out, (size_t)batch * (gauss ? 2 * A : A)) || overlap(grad_in, n_in, params, P) ||
+         overlap(grad_in, n_in, grads, P) || overlap(grad_in, n_in, cache, (size_t)batch * (IN + 4 * H))))
+        return MRL_E_UNSUPPORTED;
     const mrl_mlp_desc *ds[1] = {&d};
     float *gs[1] = {grads};
-    return mlp3_backward_n(ctx, ds, 1, batch, io, gs, ws);
+    UpdateWs ws;
+    int rc = mlp3_update_ws(ctx, ds, 1, batch, nullptr, &ws);
+    if (rc) return rc;
+    Mlp3Nets io{};
+    Mlp3Net &nn = io.n[0];
+    nn = ws.net[0];
+    nn.A = A;
+    nn.gauss = gauss ? 1 : 0;
+    nn.grad_out = grad_out; nn.params = params; nn.cache = const_cast<float *>(cache); nn.grad_in = grad_in;
+    rc = launch_bwd(ctx, H, act, batch, IN, ws.rows, nn, ws.dw_in_tiles);
+    if (rc) return rc;
+    if (!ws.dw_in_tiles) {
+        rc = launch_dw_frag(ctx, H, 1, batch, ws, P, P, (IN + 1) * H);
+        if (rc) return rc;
+    }
+    return sum_tiles(ctx, ds, 1, io, ws.tiles, ws.dw_in_tiles, ws.partial, ws.splits, gs, nullptr, nullptr);
 }
 
 }  // namespace mrl

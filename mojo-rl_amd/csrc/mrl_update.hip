@@ -566,7 +566,7 @@ static int update_minibatches(mrl_ctx *ctx, const mrl_update *u, const int32_t *
     const mrl_mlp_desc *descs[2] = {&u->actor, &u->critic};
     const float *params[2] = {u->actor_params, u->critic_params};
     UpdateWs ws;
-    rc = mlp3_update_ws(ctx, descs, u->minibatch, params, &ws);
+    rc = mlp3_update_ws(ctx, descs, 2, u->minibatch, params, &ws);
     if (rc) return rc;
     rc = launch_split_weights(ctx, u->actor.layers[0].out_dim, ws.split, 2);
     if (rc) return rc;
