@@ -9,7 +9,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(HERE, "build")
 LIB = os.path.join(HERE, "libmrl_hip.so")
-SOURCES = ["mrl_core.hip", "mrl_env.hip", "mrl_mlp.hip", "mrl_mlp3.hip", "mrl_fb.hip", "mrl_rows.hip", "mrl_ppo.hip", "mrl_policy.hip", "mrl_rollout.hip", "mrl_collect.hip", "mrl_update.hip", "mrl_shuffle.hip"]
+SOURCES = ["mrl_core.hip", "mrl_env.hip", "mrl_env_many.hip", "mrl_mlp.hip", "mrl_mlp3.hip", "mrl_fb.hip", "mrl_rows.hip", "mrl_ppo.hip", "mrl_policy.hip", "mrl_rollout.hip", "mrl_collect.hip", "mrl_update.hip", "mrl_shuffle.hip"]
 # the 16-row collection kernels, a translation unit per hidden width
 COLLECT16 = ["mrl_collect%s_h%d.hip" % (k, h) for k in ("16", "_walkers") for h in (256, 128, 64)]
 SOURCES = COLLECT16 + SOURCES   # (the longest to compile go first)

@@ -101,7 +101,7 @@ struct LunarLanderContinuous : LunarLander {
 struct BipedalWalker {
     using L = bw::L;
     static constexpr int STATE = bw::STATE, OBS = bw::OBS, ACT_W = bw::ACT, EPB = 16, THREADS = 512;
-    static constexpr int LANE_FROM = 0;      // (never: the lane form is no faster for this env at any batch)
+    static constexpr int LANE_FROM = 0;      // (never: mrl_env_many.hip takes large batches)
     static constexpr int DYN_END = L::EDGES_OFF, NSHAPE = bw::NSHAPE_FLOATS;
     // the ten lidar rays of the observation are left out of the step and run afterwards, spread
     // over all wavefronts of the block: task k = part k % 3 of the edges for ray k / 3; the parts of
@@ -163,14 +163,14 @@ struct BipedalWalker {
     static MRL_DEV bool lanes_ok(const float *row) { return bw::lanes_row_ok(row); }
     static MRL_DEV void physics_lanes(float *row, float *cts, int n, int lane) { bw::physics_lanes(row, cts, n, lane); }
     static MRL_DEV void step_tail(float *row, const float *cts, int n, const Carry &c, float &r, float &d) {
-        bw::step_tail<false, false>(row, cts, n, c.act, r, d);
+        bw::step_tail<false, false>(row, cts, n, c.act, r, d, row + L::META_OFF);
     }
 };
 
 struct HalfCheetah {
     using L = hc::L;
     static constexpr int STATE = hc::STATE, OBS = hc::OBS, ACT_W = hc::ACT, EPB = 64, THREADS = 256;
-    static constexpr int LANE_FROM = 0;      // (never: the lane form is no faster for this env at any batch)
+    static constexpr int LANE_FROM = 0;      // (never: mrl_env_many.hip takes large batches)
     static constexpr int DYN_END = L::EDGES_OFF, NSHAPE = hc::NSHAPE_FLOATS;
     static MRL_DEV void step(float *row, float *cts, const float *shapes, int env, const float *a,
                              float &r, float &d) {

@@ -401,18 +401,20 @@ MRL_DEV void step_motors(float *row, const float *action, float *act) {
 // contacts of the step, whose body indices are still in `contacts`
 // STATE_OBS = false: observation entries 0 .. 7 and 9 .. 12 are in the row already (physics_lanes leaves them)
 template <bool LIDAR = true, bool STATE_OBS = true>
-MRL_DEV void step_tail(float *row, const float *contacts, int n, const float *act, float &reward, float &done);
+MRL_DEV void step_tail(float *row, const float *contacts, int n, const float *act, float &reward, float &done,
+                       float *M);   // M = the row's metadata
 
 template <bool LIDAR = true>
 MRL_DEV void step_finish(float *row, float *contacts, int n_given, const float *shapes, const float *act,
                          float &reward, float &done) {
     int n = reg_physics_substep<L, Topology, false, false>(row, shapes, contacts, (float)0.0, (float)-10.0, (float)(1.0 / FPS),
                                       (float)2.5, (float)0.0, (float)0.2, (float)0.005, 6, 2, n_given);
-    step_tail<LIDAR>(row, contacts, n, act, reward, done);
+    step_tail<LIDAR>(row, contacts, n, act, reward, done, row + L::META_OFF);
 }
 
 template <bool LIDAR, bool STATE_OBS>
-MRL_DEV void step_tail(float *row, const float *contacts, int n, const float *act, float &reward, float &done) {
+MRL_DEV void step_tail(float *row, const float *contacts, int n, const float *act, float &reward, float &done,
+                       float *M) {
     bool left = false, right = false, hull = false;
     for (int c = 0; c < n; ++c) {
         int b = (int)contacts[c * CONTACT_SIZE + C_BODY_A];
@@ -420,7 +422,6 @@ MRL_DEV void step_tail(float *row, const float *contacts, int n, const float *ac
         else if (b == 4) right = true;
         if (b == 0) hull = true;
     }
-    float *M = row + L::META_OFF;
     M[META_LEFT] = left ? 1.0f : 0.0f;
     M[META_RIGHT] = right ? 1.0f : 0.0f;
     if (hull) M[META_GAME_OVER] = 1.0f;

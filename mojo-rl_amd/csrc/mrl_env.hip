@@ -7,7 +7,7 @@
 // detect its contacts where the env splits that off, and the fields that a step can change are
 // copied back with coalesced stores.  HBM sees each row once in and the changed part once out;
 // nothing is re-read.  (LunarLander above 8192 envs: one lane per env on rows left in global memory,
-// phys_step_lane_kernel.)
+// phys_step_lane_kernel; BipedalWalker above 4096 and HalfCheetah above 8192 envs: mrl_env_many.hip.)
 #include <cmath>
 #include "mrl_host.hpp"
 #include "env_classic.hpp"
@@ -558,6 +558,11 @@ static int env_step_impl(mrl_ctx *ctx, int env_id, int batch, float *states, con
     MRL_CHECK_ARG(batch >= 0, "mrl_env_step: negative batch");
     if (batch == 0) return MRL_OK;
     MRL_CHECK_ARG(states && actions && rewards && dones && obs, "mrl_env_step: NULL argument");
+    if (env_step_many_pays(ctx, env_id, batch)) {
+        env_step_many(ctx, env_id, batch, states, actions, rewards, dones, obs, autoreset, reset_seed, acc);
+        MRL_CHECK_LAUNCH();
+        return MRL_OK;
+    }
     switch (env_id) {
         case MRL_ENV_CARTPOLE: {
             int32_t *steps;

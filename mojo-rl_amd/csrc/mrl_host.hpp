@@ -31,9 +31,11 @@ struct mrl_ctx {
     float *rollout_ws;
     size_t rollout_ws_floats;
     // scratch of the minibatch update: per-block KL partials [0, 1024), their arrival counter
-    // (int, at float index 1024; zero between launches), sum-of-squares partials [2048, 4096),
+    // (int, at float index 1024; zero between launches), the word of env_step_many (int, FOREIGN_WORD),
+    // sum-of-squares partials [2048, 4096),
     // advantage {mean, std} of up to 2048 minibatches [4096, 8192)
     float *upd_scratch;
+    int foreign_call;   // env_step_many calls so far
     // Kernels whose wavefronts meet at barriers of their own (counters in LDS) bound every wait by
     // spin_limit polls; a wait that gives up raises *sync_error (pinned host memory that the device
     // writes directly) and the kernel ends normally.  mrl_ctx_synchronize reports and clears it.
@@ -83,6 +85,13 @@ struct Accounting {
 int env_step_accounting(mrl_ctx *ctx, int env_id, int batch, float *states, const float *actions,
                         float *rewards, float *dones, float *obs, uint64_t step_seed, uint64_t reset_seed,
                         const Accounting &acc);
+
+// The step of BipedalWalker / HalfCheetah batches that give every SIMD several wavefronts (mrl_env_many.hip): which they
+// are, and the launches.  A row that the eight-lane kernel does not step sets the word to the call's number.
+constexpr int FOREIGN_WORD = 1028;
+bool env_step_many_pays(const mrl_ctx *ctx, int env_id, int batch);
+void env_step_many(mrl_ctx *ctx, int env_id, int batch, float *states, const float *actions, float *rewards, float *dones,
+                   float *obs, bool autoreset, uint64_t reset_seed, const Accounting &acc);
 
 // CartPole's per-env step counters for the rows at `states` (created zeroed on first use)
 int cartpole_side(mrl_ctx *ctx, const float *states, int batch, int32_t **out);
