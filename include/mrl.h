@@ -369,8 +369,8 @@ int mrl_rollout_fused(const mrl_rollout *r);
  * KL early stop (target_kl > 0): the mean KL is tested on the device; kl_flag is 4 int32 --
  * [0] raised (and left raised) when a minibatch's mean KL exceeds target_kl, [1] bits of the
  * last mean, [2] number of updates applied since the caller cleared it; once [0] is up the call
- * still computes gradients but leaves parameters and optimiser state untouched, which is where
- * the reference's `break` (ppo.mojo:2566-2573) leaves them. */
+ * still computes gradients (mrl_ppo_update_epoch: those of its last minibatch) but leaves parameters
+ * and optimiser state untouched, which is where the reference's `break` (ppo.mojo:2566-2573) leaves them. */
 typedef struct {
     int32_t minibatch, obs_dim, act_width, continuous;
     mrl_mlp_desc actor, critic;

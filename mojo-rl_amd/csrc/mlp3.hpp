@@ -40,6 +40,7 @@ struct FwdLoss {
     float *g_actor_out, *g_values, *kl;                   // [mb, head], [mb], [mb]
     float *kl_part;                                       // [row tiles] sums of the tiles' KL estimates, for the test
     int32_t *kl_flag;                                     // null: no test (nothing is left in kl_part)
+    const int32_t *skip;                                  // not null and *skip != 0: nothing of this minibatch is needed
     int dw_in_tiles;                                      // forward + backward: the row tiles leave their dW1 as well
     int mb, A, continuous, clip_value;                    // A = actions (discrete) or action width (continuous)
     float clip_eps, ent_coef, value_coef, target_kl;
@@ -71,7 +72,7 @@ int mlp3_update_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int batch, Mlp
                   float *const *grads, float *sq_part, int *sq_blocks, const FwdLoss &loss);
 int launch_fwd16(mrl_ctx *ctx, int H, int act, int batch, int IN, const Mlp3Net &nn);
 int launch_bwd(mrl_ctx *ctx, int H, int act, int batch, int IN, int rows, const Mlp3Net &nn, bool dw_in_tiles);
-int launch_dw_frag(mrl_ctx *ctx, int H, int n_nets, int batch, const UpdateWs &ws, int P0, int Ptot, int w1_off);
+int launch_dw_frag(mrl_ctx *ctx, int H, int n_nets, int batch, const UpdateWs &ws, int P0, int Ptot, int w1_off, const int32_t *skip);
 int launch_fb(mrl_ctx *ctx, int H, int act, int batch, int IN, int rows, const Mlp3Nets &nets, const FwdLoss &fl);
 // grows the context's MLP workspace to at least `floats`
 int mlp_ensure_ws(mrl_ctx *ctx, size_t floats, float **out);

@@ -34,6 +34,7 @@ struct DwFrag {
     int n;        // nets
     const unsigned short *x[2], *g[2];
     int off[2];   // of the net's W1 gradient in a split's partial vector
+    const int32_t *skip;   // as FwdLoss::skip
 };
 
 template <int H, int ACT, int RT>
@@ -68,6 +69,7 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
     const bool actor = blockIdx.y == 0;
 
     // ---- everything that does not depend on an earlier phase is requested first.  Rows: sixteen lanes each.
+    const int skip = fl.skip != nullptr ? *fl.skip : 0;   // (tested once these requests are out)
     constexpr int XQ = (R * 16 + T - 1) / T;
     long xsrc[XQ];
     float xa[XQ], xb[XQ];
@@ -115,6 +117,7 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
         }
     }
     if (actor && fl.adv_stats != nullptr) { l_mean = fl.adv_stats[0]; l_std = fl.adv_stats[1]; }
+    if (skip != 0) return;
     // (the weights last: a wavefront's loads come back in order, and the rows are waited for first)
     __builtin_amdgcn_sched_barrier(0);
     bf16x8 wq[PF][NT][SPLIT];
@@ -479,6 +482,7 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
 template <int H>
 __global__ __launch_bounds__(512) void dw_frag_kernel(DwFrag d, int steps, int steps_per, int splits, int Ptot,
                                                       float *__restrict__ partial) {
+    if (d.skip != nullptr && *d.skip != 0) return;
     constexpr int XCDS = 8, TN = 128, tiles_n = H / TN, tiles = tiles_n * (H / 64), NB = 4, RLD = TN + 4;
     static_assert(H % TN == 0, "whole tiles");
     __shared__ float sum[64 * RLD];
@@ -553,9 +557,11 @@ __global__ __launch_bounds__(512) void dw_frag_kernel(DwFrag d, int steps, int s
 }
 
 // P0: parameters of the first net, w1_off: offset of W1 in a net's parameters
-int launch_dw_frag(mrl_ctx *ctx, int H, int n_nets, int batch, const UpdateWs &ws, int P0, int Ptot, int w1_off) {
+int launch_dw_frag(mrl_ctx *ctx, int H, int n_nets, int batch, const UpdateWs &ws, int P0, int Ptot, int w1_off,
+                   const int32_t *skip) {
     DwFrag d{};
     d.n = n_nets;
+    d.skip = skip;
     for (int i = 0; i < n_nets; ++i) {
         d.x[i] = ws.net[i].h1q;
         d.g[i] = ws.net[i].g1q;

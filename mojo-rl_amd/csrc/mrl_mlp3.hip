@@ -94,6 +94,7 @@ struct SumNets {
     int P[2], A[2], gauss[2];
     int n, IN, H;
     int thin_stride[2];   // floats per row tile in thin_part, per net
+    const int32_t *skip;   // as FwdLoss::skip
     int hh_in_tiles;   // the H x H block is summed from the row tiles' pieces (behind dW0 and dW2) instead of `partial`
 };
 
@@ -130,6 +131,7 @@ MRL_DEV float sum_strided(const float *__restrict__ p, size_t stride, int n) {
 
 __global__ __launch_bounds__(256) void sum3_kernel(const float *__restrict__ partial, int splits, int Ptot,
                                                    int tiles, SumNets sn, float *__restrict__ sq_part) {
+    if (sn.skip != nullptr && *sn.skip != 0) return;
     __shared__ float red[2][4];
     const int gi = blockIdx.x * blockDim.x + threadIdx.x;
     int net = 0;
@@ -271,11 +273,12 @@ static void dw_splits(int n_nets, int batch, int *splits, int *rows_per) {
 // The sums over row tiles and batch splits into the flat gradients (hh_in_tiles: the tiles left the H x H weight
 // gradients too).
 static int sum_tiles(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, const Mlp3Nets &io, int tiles, bool hh_in_tiles,
-                     const float *partial, int splits, float *const *grads, float *sq_part, int *sq_blocks) {
+                     const float *partial, int splits, float *const *grads, float *sq_part, int *sq_blocks, const int32_t *skip) {
     const int IN = descs[0]->layers[0].in_dim, H = descs[0]->layers[0].out_dim;
     SumNets sn{};
     sn.n = n_nets;
     sn.IN = IN;
+    sn.skip = skip;
     sn.H = H;
     sn.hh_in_tiles = hh_in_tiles ? 1 : 0;
     int Ptot = 0;
@@ -370,10 +373,10 @@ int mlp3_update_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int batch, Mlp
     if (rc) return rc;
     if (!ws.dw_in_tiles) {
         const int P0 = net_P(*descs[0]);
-        rc = launch_dw_frag(ctx, H, 2, batch, ws, P0, P0 + net_P(*descs[1]), (descs[0]->layers[0].in_dim + 1) * H);
+        rc = launch_dw_frag(ctx, H, 2, batch, ws, P0, P0 + net_P(*descs[1]), (descs[0]->layers[0].in_dim + 1) * H, fl.skip);
         if (rc) return rc;
     }
-    return sum_tiles(ctx, descs, 2, io, ws.tiles, ws.dw_in_tiles, ws.partial, ws.splits, grads, sq_part, sq_blocks);
+    return sum_tiles(ctx, descs, 2, io, ws.tiles, ws.dw_in_tiles, ws.partial, ws.splits, grads, sq_part, sq_blocks, fl.skip);
 }
 
 // true when [a, a + na) and [b, b + nb) (floats) share memory
@@ -409,10 +412,10 @@ int mlp3_backward(mrl_ctx *ctx, const mrl_mlp_desc &d, int batch, const float *g
     rc = launch_bwd(ctx, H, act, batch, IN, ws.rows, nn, ws.dw_in_tiles);
     if (rc) return rc;
     if (!ws.dw_in_tiles) {
-        rc = launch_dw_frag(ctx, H, 1, batch, ws, P, P, (IN + 1) * H);
+        rc = launch_dw_frag(ctx, H, 1, batch, ws, P, P, (IN + 1) * H, nullptr);
         if (rc) return rc;
     }
-    return sum_tiles(ctx, ds, 1, io, ws.tiles, ws.dw_in_tiles, ws.partial, ws.splits, gs, nullptr, nullptr);
+    return sum_tiles(ctx, ds, 1, io, ws.tiles, ws.dw_in_tiles, ws.partial, ws.splits, gs, nullptr, nullptr, nullptr);
 }
 
 }  // namespace mrl

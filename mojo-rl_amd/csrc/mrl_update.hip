@@ -458,9 +458,11 @@ static void adam_args(const mrl_update *u, int actor_t, int critic_t, AdamArgs &
 }
 
 // One minibatch of the fused nets; stats: {mean, std} of its advantages on the device (null: not normalised).
-// ws.split holds the hidden layers' current weights; keep_split: it is to hold the updated ones afterwards.
+// ws.split holds the hidden layers' current weights; more: another minibatch of the same call follows.  Then the copies
+// are kept in step with the updated weights, and once the KL stop is up nothing is computed: no parameter moves any more,
+// and what else the call leaves (gradients, outputs, KL estimates) is its last minibatch's, which is always computed.
 static int update_minibatch_paired(mrl_ctx *ctx, const mrl_update *u, const int32_t *indices, int actor_t, int critic_t,
-                                   const float *stats, const UpdateWs &ws, bool keep_split) {
+                                   const float *stats, const UpdateWs &ws, bool more) {
     const bool cont = u->continuous != 0;
     const int mb = u->minibatch, head = mrl_mlp_out_dim(&u->actor);
     const mrl_mlp_desc *descs[2] = {&u->actor, &u->critic};
@@ -475,6 +477,7 @@ static int update_minibatch_paired(mrl_ctx *ctx, const mrl_update *u, const int3
     fl.g_actor_out = u->g_actor_out; fl.g_values = u->g_values; fl.kl = u->kl;
     fl.kl_part = ctx->upd_scratch + SCR_KL;
     fl.kl_flag = u->target_kl > 0.0f ? u->kl_flag : nullptr;
+    fl.skip = more ? fl.kl_flag : nullptr;
     fl.mb = mb; fl.A = cont ? u->act_width : head; fl.continuous = cont ? 1 : 0;
     fl.clip_value = u->clip_value ? 1 : 0;
     fl.clip_eps = u->clip_epsilon; fl.ent_coef = u->entropy_coef; fl.value_coef = u->value_loss_coef;
@@ -493,7 +496,7 @@ static int update_minibatch_paired(mrl_ctx *ctx, const mrl_update *u, const int3
     a.kl_n = ws.tiles;
     const int H = u->actor.layers[0].out_dim, o1 = (u->obs_dim + 1) * H;
     SplitNets sp{};
-    if (keep_split) sp = ws.split;
+    if (more) sp = ws.split;
     if (H == 256) launch_adam_split<256>(ctx->stream, a, o1, sp);
     else if (H == 128) launch_adam_split<128>(ctx->stream, a, o1, sp);
     else launch_adam_split<64>(ctx->stream, a, o1, sp);
