@@ -244,73 +244,7 @@ __global__ __launch_bounds__(GAE_LOADERS + 64) void gae_fed_kernel(int T, int N,
     }
 }
 
-// ---------------------------------------------------------------- advantage normalisation
-// Three launches: per-block sums; per-block sums of squared deviations; (x - mean) /
-// (sqrt(var + 1e-8) + 1e-8).  Two-pass variance like the reference (ppo.mojo:2356-2371), with fp32
-// sums taken blockwise.  Every block of the second and third launch adds the (at most 1024) block
-// sums up itself, all in the same order: a few L2 reads against two more launches of one block.
-constexpr int NORM_BLOCKS = 1024, NORM_U = 4;
-
-// sum(in[0..nb)) / n in every thread
-MRL_DEV float mean_of_blocks(const float *__restrict__ in, int nb, int n, float *smem) {
-    float s = 0.0f;
-    for (int i = threadIdx.x; i < nb; i += blockDim.x) s += in[i];
-    s = block_sum(s, smem);
-    if (threadIdx.x == 0) smem[0] = s / (float)n;
-    __syncthreads();
-    const float m = smem[0];
-    __syncthreads();
-    return m;
-}
-
-// sums == nullptr: out[b] = sum x; else out[b] = sum (x - mean)^2, sums = the first form's block sums
-__global__ __launch_bounds__(TPB) void partial_sum_kernel(const float *__restrict__ x, int n,
-                                                          const float *__restrict__ sums,
-                                                          float *__restrict__ out) {
-    __shared__ float smem[4];
-    const long stride = (long)gridDim.x * blockDim.x;
-    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    float a[NORM_U];
-    const bool full = i + (NORM_U - 1) * stride < n;
-    if (full)   // the first elements are on their way while the mean is formed
-#pragma unroll
-        for (int k = 0; k < NORM_U; ++k) a[k] = x[i + k * stride];
-    const float mean = sums ? mean_of_blocks(sums, gridDim.x, n, smem) : 0.0f;
-    float s = 0.0f;
-    auto add = [&](float v) {
-        const float d = v - mean;
-        s += sums ? d * d : v;
-    };
-    if (full) {
-        for (;;) {
-#pragma unroll
-            for (int k = 0; k < NORM_U; ++k) add(a[k]);
-            i += NORM_U * stride;
-            if (i + (NORM_U - 1) * stride >= n) break;
-#pragma unroll
-            for (int k = 0; k < NORM_U; ++k) a[k] = x[i + k * stride];
-        }
-    }
-    for (; i < n; i += stride) add(x[i]);
-    s = block_sum(s, smem);
-    if (threadIdx.x == 0) out[blockIdx.x] = s;
-}
-
-__global__ __launch_bounds__(TPB) void normalize_apply_kernel(float *__restrict__ x, int n, int nb,
-                                                              const float *__restrict__ sums,
-                                                              const float *__restrict__ squares) {
-    __shared__ float smem[4];
-    const float mean = mean_of_blocks(sums, nb, n, smem);
-    const float variance = mean_of_blocks(squares, nb, n, smem);
-    const float std = sqrtf(variance + 1e-8f);
-    const long stride = (long)gridDim.x * blockDim.x;
-#pragma unroll NORM_U
-    for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) x[i] = (x[i] - mean) / (std + 1e-8f);
-}
-
-// ---------------------------------------------------------------- reward RunningMeanStd
-// core/utils/normalization.mojo:188-292 in Float64: batch mean and variance (two passes), merged
-// into (count, mean, var_sum) with Chan's formula; normalise with var = 1 while count < 2.
+// ---------------------------------------------------------------- Float64 sums of a block
 MRL_DEV double wave_sum_d(double v) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
@@ -328,6 +262,93 @@ MRL_DEV double block_sum_d(double v, double *smem) {
     return t;
 }
 
+// ---------------------------------------------------------------- advantage normalisation
+// (x - mean) / (sqrt(var + 1e-8) + 1e-8) in two launches: sums of d and d^2 per block, d = x - x[0] in Float64; then
+// every block forms mean and variance from the block sums and normalises its share.  The reference takes the variance
+// in a second pass over x (ppo.mojo:2356-2371), in fp32; here x[0] is one of the values, so that (mean d)^2 is at most
+// n var and what cancels in var = mean d^2 - (mean d)^2 stays below 2^-53 n var.  x is read twice instead of three times,
+// in 16-byte pieces where it lies on 16 bytes (W = 4).  What bounds it: memory, and the start of two
+// launches.  us at 1000 / 131072 / 1 M / 4 M / 8 M values: 6.5 / 7.5 / 8.9 / 12.6 / 16.5 (off 16 bytes 6.5 / 8.4 / 9.8 / 16.2 /
+// 25.6); three launches with fp32 sums of 4-byte loads took 9.3 / 9.9 / 13.2 / 18.2 / 24.0.
+constexpr int NORM_BLOCKS = 512, NORM_U = 4;   // (two blocks per CU: fewer block sums for every block to read)
+
+// x in pieces of W floats: f(piece index, W values by reference) over this thread's pieces, NORM_U requested at a time, the
+// first of them ahead of `before`; then tail(index) over the elements behind the last whole piece
+template <int W, class Before, class Piece, class Tail>
+MRL_DEV void norm_walk(const float *x, int n, Before &&before, Piece &&piece, Tail &&tail) {
+    typedef float V __attribute__((ext_vector_type(W)));
+    const V *xv = reinterpret_cast<const V *>(x);
+    const long units = n / W, stride = (long)gridDim.x * blockDim.x;
+    long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    V v[NORM_U];
+    auto request = [&]() {
+#pragma unroll
+        for (int k = 0; k < NORM_U; ++k)
+            if (i + k * stride < units) v[k] = xv[i + k * stride];
+    };
+    request();
+    before();
+    while (i < units) {
+#pragma unroll
+        for (int k = 0; k < NORM_U; ++k)
+            if (i + k * stride < units) piece(i + k * stride, v[k]);
+        i += NORM_U * stride;
+        request();
+    }
+    if (W > 1 && blockIdx.x == 0 && threadIdx.x < n - units * W) tail(units * W + threadIdx.x);
+}
+
+// sums[2 b], sums[2 b + 1]: block b's sums of d and d^2; sums[2 blocks] = x[0]
+template <int W>
+__global__ __launch_bounds__(TPB) void norm_sums_kernel(const float *__restrict__ x, int n, double *__restrict__ sums) {
+    __shared__ double smem[4];
+    const double pivot = (double)x[0];
+    double s = 0.0, q = 0.0;
+    auto add = [&](float v) {
+        const double d = (double)v - pivot;
+        s += d;
+        q += d * d;
+    };
+    norm_walk<W>(x, n, []() {}, [&](long, auto v) {
+#pragma unroll
+        for (int j = 0; j < W; ++j) add(v[j]);
+    }, [&](long i) { add(x[i]); });
+    s = block_sum_d(s, smem);
+    q = block_sum_d(q, smem);
+    if (threadIdx.x == 0) {
+        sums[2 * blockIdx.x] = s;
+        sums[2 * blockIdx.x + 1] = q;
+        if (blockIdx.x == 0) sums[2 * gridDim.x] = pivot;
+    }
+}
+
+template <int W>
+__global__ __launch_bounds__(TPB) void normalize_apply_kernel(float *x, int n, const double *__restrict__ sums) {
+    __shared__ double smem[4];
+    float mean, den;
+    auto stats = [&]() {
+        double s = 0.0, q = 0.0;
+        for (int i = threadIdx.x; i < (int)gridDim.x; i += TPB) {
+            s += sums[2 * i];
+            q += sums[2 * i + 1];
+        }
+        s = block_sum_d(s, smem) / n;
+        q = block_sum_d(q, smem) / n;
+        double var = q - s * s;
+        if (var < 0.0) var = 0.0;
+        mean = (float)(sums[2 * gridDim.x] + s);
+        den = sqrtf((float)var + 1e-8f) + 1e-8f;
+    };
+    norm_walk<W>(x, n, stats, [&](long i, auto v) {
+#pragma unroll
+        for (int j = 0; j < W; ++j) v[j] = (v[j] - mean) / den;
+        reinterpret_cast<decltype(v) *>(x)[i] = v;
+    }, [&](long i) { x[i] = (x[i] - mean) / den; });
+}
+
+// ---------------------------------------------------------------- reward RunningMeanStd
+// core/utils/normalization.mojo:188-292 in Float64: batch mean and variance (two passes), merged
+// into (count, mean, var_sum) with Chan's formula; normalise with var = 1 while count < 2.
 // mean_ptr == nullptr: out[b] = sum x; else out[b] = sum (x - *mean_ptr)^2
 __global__ __launch_bounds__(TPB) void rms_partial_kernel(const float *__restrict__ x, int n,
                                                           const double *__restrict__ mean_ptr,
@@ -690,11 +711,16 @@ int mrl_normalize_advantages(mrl_ctx *ctx, float *x, int n) {
     MRL_CHECK_ARG(n >= 0, "mrl_normalize_advantages: negative size");
     if (n == 0) return MRL_OK;
     MRL_CHECK_ARG(x, "mrl_normalize_advantages: NULL buffer");
-    const int nb = std::min(NORM_BLOCKS, grid_for(n, TPB));
-    float *sums = ctx->reduce_scratch, *squares = sums + NORM_BLOCKS;
-    hipLaunchKernelGGL(partial_sum_kernel, dim3(nb), dim3(TPB), 0, ctx->stream, x, n, (const float *)nullptr, sums);
-    hipLaunchKernelGGL(partial_sum_kernel, dim3(nb), dim3(TPB), 0, ctx->stream, x, n, (const float *)sums, squares);
-    hipLaunchKernelGGL(normalize_apply_kernel, dim3(nb), dim3(TPB), 0, ctx->stream, x, n, nb, sums, squares);
+    const bool wide = reinterpret_cast<uintptr_t>(x) % 16 == 0;
+    const dim3 grid(std::min(NORM_BLOCKS, std::max(1, grid_for(wide ? n / 4 : n, TPB)))), block(TPB);
+    double *sums = reinterpret_cast<double *>(ctx->reduce_scratch);   // 2 * NORM_BLOCKS + 1 of 2048
+    if (wide) {
+        hipLaunchKernelGGL(norm_sums_kernel<4>, grid, block, 0, ctx->stream, x, n, sums);
+        hipLaunchKernelGGL(normalize_apply_kernel<4>, grid, block, 0, ctx->stream, x, n, sums);
+    } else {
+        hipLaunchKernelGGL(norm_sums_kernel<1>, grid, block, 0, ctx->stream, x, n, sums);
+        hipLaunchKernelGGL(normalize_apply_kernel<1>, grid, block, 0, ctx->stream, x, n, sums);
+    }
     MRL_CHECK_LAUNCH();
     return MRL_OK;
 }
