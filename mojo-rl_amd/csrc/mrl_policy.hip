@@ -19,6 +19,7 @@
 #include "mrl_host.hpp"
 #include "mrl_device.hpp"
 #include "mlp_tile.hpp"
+#include "mlp_rows16.hpp"
 #include "policy_sample.hpp"
 
 namespace mrl {
@@ -106,6 +107,59 @@ __global__ __launch_bounds__(H == 256 && TPW == 1 ? 2 * H : 4 * H / TPW) void po
     }
 }
 
+// The same step in 16-row tiles with a net per workgroup, grid = (row tiles, nets): half the matrix chain of a 32-row tile,
+// the hidden layer's weights requested whole, into registers, before anything else needs them.  Same bits.  Taken while
+// they get a CU each at H = 256 (whose workgroup holds W1 in registers), two at H = 128, four at H = 64.  us, against 32
+// rows (its smaller batches with a net per workgroup too), 16 / 1000 / 4096 rows:  H = 64, 4 inputs 4.1 : 8.9, 5.3 : 10.0,
+// 5.6 : 10.2;  H = 128, 17 inputs 7.0 : 10.6, 8.2 : 11.8, 9.6 : 12.0;  H = 256, 17 inputs 13.7 : 18.8, 15.0 : 19.8, and 2048
+// rows 15.0 : 20.0 (in two rounds it would lose).
+template <int H, int ACT, bool GAUSS>
+__global__ __launch_bounds__(rows_threads(H)) void policy16_kernel(
+    const float *__restrict__ obs, int n, int IN, int A, const float *__restrict__ actor_p,
+    const float *__restrict__ critic_p, uint32_t seed, float *__restrict__ actions,
+    float *__restrict__ r_obs, float *__restrict__ r_actions, float *__restrict__ r_logp,
+    float *__restrict__ r_values) {
+    using F = Rows16Forward<H, ACT>;
+    constexpr int RUN = F::RUN, LD = PA_MAX + 1;
+    __shared__ typename F::Lds lds;
+    __shared__ float part[PR16 * PA_MAX];
+    const int t = threadIdx.x, row0 = blockIdx.x * PR16, nrow = min(PR16, n - row0);
+    const bool actor = blockIdx.y == 0;
+    auto none = [](int, int, const float (&)[RUN], const float (&)[RUN]) {};
+    F::run(lds, actor ? actor_p : critic_p, obs + (long)row0 * IN, nrow, IN, actor ? A : 1, GAUSS && actor,
+           [&](int r, int j, float v) {
+               if (actor) r_obs[(long)(row0 + r) * IN + j] = v;
+           }, none, none);
+    if (!actor) {
+        if (t < nrow) r_values[row0 + t] = lds.ys[t * LD];
+    } else if (!GAUSS) {
+        if (t < nrow) {
+            const int i = row0 + t;
+            int sel;
+            float logp;
+            sample_categorical_few(lds.ys + t * LD, A, seed, i, sel, logp);
+            actions[i] = (float)sel;
+            r_actions[i] = (float)sel;
+            r_logp[i] = logp;
+        }
+    } else {   // (as in policy_kernel: a lane per env and action component)
+        for (int e = t; e < nrow * A; e += F::T) {
+            const int r = e / A, j = e - r * A;
+            float act;
+            part[r * PA_MAX + j] = sample_gaussian_part(lds.ys + r * LD + j, lds.w2s + HEAD_LOG_STD(H) + j, 1, A, j, seed,
+                                                        row0 + r, &act);
+            actions[(long)row0 * A + e] = act;
+            r_actions[(long)row0 * A + e] = act;
+        }
+        __syncthreads();
+        if (t < nrow) {
+            float logp = 0.0f;
+            for (int j = 0; j < A; ++j) logp = logp + part[t * PA_MAX + j];
+            r_logp[row0 + t] = logp;
+        }
+    }
+}
+
 // true when the pair (actor, critic) has the shape this kernel is specialised for
 constexpr int PTPW = 2;   // accumulator tiles per wavefront in the policy kernel (1 measured no faster)
 constexpr int POLICY_SPLIT_BELOW = 256;   // CUs of the MI355X: up to this many workgroups run side by side
@@ -136,6 +190,26 @@ int launch_policy(mrl_ctx *ctx, const mrl_mlp_desc &a, const mrl_mlp_desc &c, bo
     int H = 0, act = 0;
     if (!policy_fusable(a, c, gauss, &H, &act)) return MRL_E_UNSUPPORTED;
     const int IN = a.layers[0].in_dim, A = a.layers[2].out_dim;
+    if (2 * ((n + PR16 - 1) / PR16) <= (H == 256 ? 1 : H == 128 ? 2 : 4) * ctx->n_cus) {
+        const dim3 grid(((unsigned)n + PR16 - 1) / PR16, 2), block(rows_threads(H));
+#define MRL_LAUNCH16(HH, AA, GG)                                                                       \
+    hipLaunchKernelGGL((policy16_kernel<HH, AA, GG>), grid, block, 0, ctx->stream, obs, n, IN, A, ap, cp, seed, actions, \
+                       r_obs, r_actions, r_logp, r_values)
+#define MRL_LAUNCH16_ACT(HH)                                                                           \
+    do {                                                                                               \
+        if (gauss && act == 1) MRL_LAUNCH16(HH, 1, true);                                              \
+        else if (gauss) MRL_LAUNCH16(HH, 2, true);                                                     \
+        else if (act == 1) MRL_LAUNCH16(HH, 1, false);                                                 \
+        else MRL_LAUNCH16(HH, 2, false);                                                               \
+    } while (0)
+        if (H == 256) MRL_LAUNCH16_ACT(256);
+        else if (H == 128) MRL_LAUNCH16_ACT(128);
+        else MRL_LAUNCH16_ACT(64);
+#undef MRL_LAUNCH16_ACT
+#undef MRL_LAUNCH16
+        MRL_CHECK_LAUNCH();
+        return MRL_OK;
+    }
     // few row tiles: actor and critic of a tile go to workgroups of their own (twice the CUs at work),
     // at hidden width 256 with one column tile per wavefront (eight wavefronts per net: two per SIMD,
     // where a workgroup of four would leave each SIMD a single wavefront with nothing to overlap)

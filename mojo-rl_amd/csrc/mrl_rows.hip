@@ -20,147 +20,43 @@
 
 namespace mrl {
 
-constexpr int rows_threads(int H) { return H == 64 ? 256 : 512; }
-
-// a row's run of 4 NT consecutive floats, 16 bytes at a time where the address allows it
-template <int N>
-MRL_DEV void store_run(float *p, const float (&y)[N], bool vec) {
-    if (vec) {
-#pragma unroll
-        for (int j = 0; j < N; j += 4) *reinterpret_cast<f32x4 *>(p + j) = f32x4{y[j], y[j + 1], y[j + 2], y[j + 3]};
-    } else {
-#pragma unroll
-        for (int j = 0; j < N; ++j) p[j] = y[j];
-    }
-}
-
-// Forward of 16 rows.  Both hidden layers are computed transposed (output columns on the accumulator's rows), so that a
-// lane ends up with 4 NT consecutive columns of one batch row, which it writes to LDS and to the cache in wide pieces.
-// k ascends through every product, so the bits are those of the 32-row tile (mlp_tile16.hpp).
+// Forward with the reference's per-layer cache (null: none), Rows16Forward per workgroup.
 template <int H, int ACT>
 __global__ __launch_bounds__(rows_threads(H)) void mlp3_fwd16_kernel(int B, int IN, Mlp3Net nn) {
-    constexpr int T = rows_threads(H), NW = T / 64, NT = H / 16 / NW, R = PR16, RUN = 4 * NT;
-    constexpr int FLD = H + 20, K0 = PIN_MAX / 4, KS = H / 4;
-    static_assert(NT == 1 || NT == 2, "one float or one float2 of a weight row per lane");
-    __shared__ float xs[R * XS_LD];
-    __shared__ __align__(16) float h1f[R * FLD];
-    __shared__ float h2[R * (H + 1)];
-    __shared__ float ys[R * (PA_MAX + 1)];
-    __shared__ __align__(16) float w2s[HEAD_LDS(H)];
-    const float *__restrict__ params = nn.params;
+    using F = Rows16Forward<H, ACT>;
+    constexpr int T = F::T, RUN = F::RUN, R = PR16;
+    __shared__ typename F::Lds lds;
     float *__restrict__ cache = nn.cache;
     const int A = nn.A;
     const bool GAUSS = nn.gauss != 0;
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6, g = lane >> 4, n = lane & 15;
+    const int t = threadIdx.x;
     const long row0 = (long)blockIdx.x * R;
     const int nrow = (int)min((long)R, B - row0);
     float *c0 = cache, *c1 = cache + (size_t)B * (IN + H), *c2 = c1 + (size_t)B * 2 * H;
-    const int col_w = 16 * NT * w + NT * n;        // this lane's weight columns; tile q holds column col_w + q
-    const int col_d = 16 * NT * w + RUN * g;       // its output columns, RUN of them, of batch row n
-    const float *W0 = params, *b0 = params + IN * H, *W1 = b0 + H, *b1 = W1 + H * H;
-
-    // ---- everything from global memory is requested first, the rows ahead of the weights that hide behind them
-    constexpr int XQ = (R * 16 + T - 1) / T;
-    float xa[XQ], xb[XQ];
-#pragma unroll
-    for (int q = 0; q < XQ; ++q) {
-        const int r = (t + q * T) >> 4, j = t & 15;
-        xa[q] = r < nrow && j < IN ? nn.x[(row0 + r) * IN + j] : 0.0f;
-        xb[q] = r < nrow && j + 16 < IN ? nn.x[(row0 + r) * IN + j + 16] : 0.0f;
-    }
-    float w0[K0][NT], bias0[RUN], bias1[RUN];
-#pragma unroll
-    for (int s = 0; s < K0; ++s)
-#pragma unroll
-        for (int q = 0; q < NT; ++q) w0[s][q] = 4 * s + g < IN ? W0[(4 * s + g) * H + col_w + q] : 0.0f;
-#pragma unroll
-    for (int j = 0; j < RUN; ++j) { bias0[j] = b0[col_d + j]; bias1[j] = b1[col_d + j]; }
-    stage_head(params + IN * H + H + H * H + H, H, A, GAUSS, w2s, t, T);
-    __builtin_amdgcn_sched_barrier(0);
-    float w1[KS][NT];
-#pragma unroll
-    for (int s = 0; s < KS; ++s)
-#pragma unroll
-        for (int q = 0; q < NT; ++q) w1[s][q] = W1[(4 * s + g) * H + col_w + q];
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int q = 0; q < XQ; ++q) {
-        const int r = (t + q * T) >> 4, j = t & 15;
-        if (r < R) {
-            if (j < IN) xs[r * XS_LD + j] = xa[q];
-            if (j + 16 < IN) xs[r * XS_LD + j + 16] = xb[q];
-            if (cache != nullptr && r < nrow) {
-                if (j < IN) c0[(row0 + r) * (IN + H) + j] = xa[q];
-                if (j + 16 < IN) c0[(row0 + r) * (IN + H) + j + 16] = xb[q];
-            }
-        }
-    }
-    __syncthreads();
-
-    // ---- layer 0: D[column 4 g + v of tile q][batch row n]
-    const bool put = cache != nullptr && n < nrow;
     const bool vec0 = IN % 4 == 0 && (reinterpret_cast<uintptr_t>(c0) & 15) == 0;
     const bool vec1 = (reinterpret_cast<uintptr_t>(c1) & 15) == 0;   // (c2 lies a multiple of 2 H floats behind it)
-    {
-        f32x4 d[NT];
-#pragma unroll
-        for (int q = 0; q < NT; ++q) d[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int s = 0; s < K0; ++s) {
-            if (4 * s < IN) {
-                const float x = 4 * s + g < IN ? xs[n * XS_LD + 4 * s + g] : 0.0f;
-#pragma unroll
-                for (int q = 0; q < NT; ++q) d[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(w0[s][q], x, d[q], 0, 0, 0);
-            }
-        }
-        float pre[RUN], y[RUN];
-#pragma unroll
-        for (int j = 0; j < RUN; ++j) {
-            pre[j] = d[j % NT][j / NT] + bias0[j];
-            y[j] = activate<ACT>(pre[j]);
-        }
-        store_run<RUN>(h1f + n * FLD + col_d, y, true);
-        if (put) {
-            store_run<RUN>(c0 + (row0 + n) * (IN + H) + IN + col_d, ACT == 1 ? pre : y, vec0);
-            store_run<RUN>(c1 + (row0 + n) * (2 * H) + col_d, y, vec1);
-        }
-    }
-    __syncthreads();
-
-    // ---- layer 1
-    {
-        f32x4 d[NT];
-#pragma unroll
-        for (int q = 0; q < NT; ++q) d[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            const float x = h1f[n * FLD + 4 * s + g];
-#pragma unroll
-            for (int q = 0; q < NT; ++q) d[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(w1[s][q], x, d[q], 0, 0, 0);
-        }
-        float pre[RUN], y[RUN];
-#pragma unroll
-        for (int j = 0; j < RUN; ++j) {
-            pre[j] = d[j % NT][j / NT] + bias1[j];
-            y[j] = activate<ACT>(pre[j]);
-            h2[n * (H + 1) + col_d + j] = y[j];
-        }
-        if (put) {
-            store_run<RUN>(c1 + (row0 + n) * (2 * H) + H + col_d, ACT == 1 ? pre : y, vec1);
-            store_run<RUN>(c2 + (row0 + n) * H + col_d, y, vec1);
-        }
-    }
-    __syncthreads();
-    head16<H>(w2s, A, h2, ys, PA_MAX + 1, t, T);
-    __syncthreads();
+    F::run(lds, nn.params, nn.x + row0 * IN, nrow, IN, A, GAUSS,
+           [&](int r, int j, float v) {
+               if (cache != nullptr) c0[(row0 + r) * (IN + H) + j] = v;
+           },
+           [&](int n, int col, const float (&pre)[RUN], const float (&y)[RUN]) {
+               if (cache == nullptr) return;
+               store_run<RUN>(c0 + (row0 + n) * (IN + H) + IN + col, ACT == 1 ? pre : y, vec0);
+               store_run<RUN>(c1 + (row0 + n) * (2 * H) + col, y, vec1);
+           },
+           [&](int n, int col, const float (&pre)[RUN], const float (&y)[RUN]) {
+               if (cache == nullptr) return;
+               store_run<RUN>(c1 + (row0 + n) * (2 * H) + H + col, ACT == 1 ? pre : y, vec1);
+               store_run<RUN>(c2 + (row0 + n) * H + col, y, vec1);
+           });
     const int ld = GAUSS ? 2 * A : A;
     for (int i = t; i < nrow * ld; i += T) {
         const int r = i / ld, a = i - r * ld;
         float v;
         if (a < A) {
-            v = ys[r * (PA_MAX + 1) + a];
+            v = lds.ys[r * (PA_MAX + 1) + a];
         } else {   // state-independent log_std, clamped (deep_rl/model/stochastic_actor.mojo:260-275)
-            v = w2s[HEAD_LOG_STD(H) + (a - A)];
+            v = lds.w2s[HEAD_LOG_STD(H) + (a - A)];
             v = v < -5.0f ? -5.0f : (v > 2.0f ? 2.0f : v);
         }
         nn.out[(row0 + r) * ld + a] = v;
