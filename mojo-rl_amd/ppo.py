@@ -207,15 +207,23 @@ class RolloutBuffers:
         return r
 
 
+def _row_ptr(t, at):
+    """_ptr(t[at:]) without the slice, for a float32 vector and a place inside it."""
+    if type(at) is int and 0 <= at < t.numel() and t.dtype is torch.float32 and t.dim() == 1:
+        return _ptr(t) + 4 * at
+    return _ptr(t[at:])
+
+
 def policy_step(ctx, rb, t, sample_seed, actions):
     """Policy half of collection step t on rb.obs (actor + critic forward, sampling, pre-step store into
     rollout row t); `actions` [N * act_width] receives what the envs are to be stepped with.  Enqueue only."""
     N, od, aw = rb.n_envs, rb.env.OBS_DIM, rb.act_width
     name = "mrl_policy_step_gaussian" if rb.continuous else "mrl_policy_step_discrete"
+    # the pointers to rollout row t by arithmetic: a slice object costs more than the launch
     _lib.call(name, ctx.handle, C.byref(rb.actor.desc), C.byref(rb.critic.desc), N, _ptr(rb.obs),
               _ptr(rb.actor_params), _ptr(rb.critic_params), int(sample_seed) & 0xFFFFFFFF, _ptr(actions),
-              _ptr(rb.r_obs[t * N * od:]), _ptr(rb.r_actions[t * N * aw:]), _ptr(rb.r_log_probs[t * N:]),
-              _ptr(rb.r_values[t * N:]))
+              _row_ptr(rb.r_obs, t * N * od), _row_ptr(rb.r_actions, t * N * aw), _row_ptr(rb.r_log_probs, t * N),
+              _row_ptr(rb.r_values, t * N))
 
 
 def rollout_step(ctx, desc, t, sample_seed, step_seed=0, reset_seed=0):
