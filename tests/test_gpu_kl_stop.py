@@ -56,3 +56,46 @@ def test_epoch_equals_single_minibatches_across_the_stop(mrl, cont, H, n_mb):
     for name in ("kl_flag", "actor_state", "critic_state", "actor_grads", "critic_grads", "kl", "g_actor_out", "g_values",
                  "actor_out", "values"):
         assert torch.equal(getattr(one, name), getattr(whole, name)), name
+
+
+@pytest.mark.parametrize("H", [64, 128, 256])
+@pytest.mark.parametrize("cont", [False, True], ids=["discrete", "continuous"])
+def test_the_stop_of_a_minibatch_holds_for_every_workgroup_of_its_own_update(mrl, cont, H):
+    """The launch that would apply a minibatch is the one that raises the flag.  None of its workgroups may take part of the
+    update, whichever of them runs late: other work shares the chip, and parameters and moments must not move by a bit."""
+    ctx = mrl.DeviceContext("cuda:0")
+    E = mrl.HalfCheetahPlanarV2 if cont else mrl.LunarLanderV2
+    A = E.ACTION_DIM if cont else E.NUM_ACTIONS
+    lay = mrl.LinearTanh if cont else mrl.LinearReLU
+    actor = mrl.seq(lay(E.OBS_DIM, H), lay(H, H), mrl.StochasticActor(H, A) if cont else mrl.Linear(H, A))
+    critic = mrl.seq(lay(E.OBS_DIM, H), lay(H, H), mrl.Linear(H, 1))
+    N, T = 97, 5
+    g = torch.Generator(device="cuda").manual_seed(H)
+    rb = mrl.ppo.RolloutBuffers(ctx, E, actor, critic, N, T)
+    rb.actor_params = (torch.rand(actor.PARAM_SIZE, device="cuda", generator=g) - 0.5) * 0.2
+    rb.critic_params = (torch.rand(critic.PARAM_SIZE, device="cuda", generator=g) - 0.5) * 0.2
+    rb.r_obs.normal_(generator=g)
+    if not cont:
+        rb.r_actions.copy_(torch.randint(0, A, (N * T,), device="cuda", generator=g).float())
+    rb.r_log_probs.fill_(9.0)                                  # a mean KL far above any target
+    cls = mrl.ppo.ContinuousUpdate if cont else mrl.ppo.DiscreteUpdate
+    upd = cls(ctx, rb, N * T, mrl.Adam(lr=1e-2), mrl.Adam(lr=1e-2), target_kl=0.01)
+    upd.advantages.normal_(generator=g)
+    upd.returns.normal_(generator=g)
+    upd.actor_state.uniform_(generator=g)
+    upd.critic_state.uniform_(generator=g)
+    kept = [t.clone() for t in (rb.actor_params, rb.critic_params, upd.actor_state, upd.critic_state)]
+    perm = torch.randperm(N * T, device="cuda", generator=g).to(torch.int32)
+    side, filler = torch.cuda.Stream(), torch.zeros(1 << 24, device="cuda")
+    side.wait_stream(torch.cuda.current_stream())
+    for k in range(20):
+        with torch.cuda.stream(side):
+            for _ in range(4):
+                filler.add_(1.0)
+        upd.reset_kl()
+        upd.minibatch_step(perm)
+        ctx.synchronize()
+        assert upd.kl_flag.tolist()[0] == 1 and upd.kl_flag.tolist()[2] == 0
+        for was, now in zip(kept, (rb.actor_params, rb.critic_params, upd.actor_state, upd.critic_state)):
+            assert torch.equal(was, now), k
+    side.synchronize()
