@@ -329,6 +329,9 @@ __global__ __launch_bounds__(UTPB) void clip_adam2_kernel(AdamArgs a) {
 // The fused nets (hidden width H, W1 at offset o1): the first H * H / 2048 workgroups take eight consecutive columns of
 // W1 per thread and keep the split operand copies of mlp_split.hpp in step (null: not kept); the others take the
 // remaining parameters one per thread.  Everything that does not depend on the verdict is requested ahead of it.
+// Parameters lie on 16 bytes (the row tiles need that); gradients and moments may lie on any float, for instance as slices
+// of one vector: the same 16-byte accesses reach them there.
+typedef float f32x4a4 __attribute__((ext_vector_type(4), aligned(4)));
 template <int H>
 __global__ __launch_bounds__(UTPB) void clip_adam_split_kernel(AdamArgs a, int o1, SplitNets sp) {
     constexpr int WB = H * H / (8 * UTPB), ROWS = 8 * UTPB / H, TLD = H + 4;
@@ -349,14 +352,15 @@ __global__ __launch_bounds__(UTPB) void clip_adam_split_kernel(AdamArgs a, int o
     }
     const int rl = t / (H / 8), c8 = t % (H / 8), row = blockIdx.x * ROWS + rl;
     const size_t off = (size_t)o1 + (size_t)row * H + 8 * c8;
-    f32x4 p[2], g[2], st[4];
+    f32x4 p[2];
+    f32x4a4 g[2], st[4];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
         p[k] = *reinterpret_cast<const f32x4 *>(net.p + off + 4 * k);
-        g[k] = *reinterpret_cast<const f32x4 *>(net.g + off + 4 * k);
+        g[k] = *reinterpret_cast<const f32x4a4 *>(net.g + off + 4 * k);
     }
 #pragma unroll
-    for (int k = 0; k < 4; ++k) st[k] = *reinterpret_cast<const f32x4 *>(net.state + off + 2 * k);
+    for (int k = 0; k < 4; ++k) st[k] = *reinterpret_cast<const f32x4a4 *>(net.state + off + 2 * k);
     if (!clip_verdict(a, smem, scale)) return;
     f32x8 pn;
 #pragma unroll
@@ -370,13 +374,13 @@ __global__ __launch_bounds__(UTPB) void clip_adam_split_kernel(AdamArgs a, int o
     }
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
-        *reinterpret_cast<f32x4 *>(net.g + off + 4 * k) = g[k];
+        *reinterpret_cast<f32x4a4 *>(net.g + off + 4 * k) = g[k];
         const f32x4 q = {pn[4 * k], pn[4 * k + 1], pn[4 * k + 2], pn[4 * k + 3]};
         *reinterpret_cast<f32x4 *>(net.p + off + 4 * k) = q;
         *reinterpret_cast<f32x4 *>(tile + rl * TLD + 8 * c8 + 4 * k) = q;
     }
 #pragma unroll
-    for (int k = 0; k < 4; ++k) *reinterpret_cast<f32x4 *>(net.state + off + 2 * k) = st[k];
+    for (int k = 0; k < 4; ++k) *reinterpret_cast<f32x4a4 *>(net.state + off + 2 * k) = st[k];
     if (sp.wf[0] == nullptr) return;
     bf16x8 pc[SPLIT];
     split8(pn, pc);
@@ -435,12 +439,10 @@ static int update_check(const mrl_update *u, const char *who) {
 // advantage statistics of up to STATS_MAX minibatches
 constexpr int SCR_KL = 0, SCR_ARRIVED = 1024, SCR_SQ = 2048, SCR_STATS = 4096, STATS_MAX = 2048;
 
-// both nets of the fused shapes, buffers that 16-byte accesses can reach, a KL sum per row tile
+// both nets of the fused shapes, parameters that 16-byte loads can reach, a KL sum per row tile
 static bool update_paired(const mrl_update *u) {
-    uintptr_t all = 0;
-    for (const float *p : {u->actor_params, u->critic_params, u->actor_grads, u->critic_grads, u->actor_state, u->critic_state})
-        all |= reinterpret_cast<uintptr_t>(p);
-    return mlp3_pair_fusable(u->actor, u->critic) && all % 16 == 0 && (u->minibatch + 31) / 32 <= 1024;
+    return mlp3_pair_fusable(u->actor, u->critic) && reinterpret_cast<uintptr_t>(u->actor_params) % 16 == 0 &&
+           reinterpret_cast<uintptr_t>(u->critic_params) % 16 == 0 && (u->minibatch + 31) / 32 <= 1024;
 }
 
 static void adam_args(const mrl_update *u, int actor_t, int critic_t, AdamArgs &a) {
