@@ -218,7 +218,7 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
 #pragma unroll
             for (int rt = 0; rt < RT; ++rt) {
 #pragma unroll
-                for (int v = 0; v < 4; ++v) h2v[rt][q][v] = activate<ACT>(hi[rt][q][v] + lo[rt][q][v] + bias1[q][v]);
+                for (int v = 0; v < 4; ++v) h2v[rt][q][v] = activate<ACT>(split_sum(hi[rt][q][v], lo[rt][q][v]) + bias1[q][v]);
                 *reinterpret_cast<f32x4 *>(h2f + (16 * rt + n) * FLD + c) = h2v[rt][q];
             }
         }
@@ -412,7 +412,7 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
             for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
                 for (int v = 0; v < 4; ++v)
-                    g0[q][rt][v] = (hi[rt][q][v] + lo[rt][q][v]) *
+                    g0[q][rt][v] = split_sum(hi[rt][q][v], lo[rt][q][v]) *
                                    act_deriv_out<ACT>(h1f[(16 * rt + 4 * g + v) * FLD + 16 * (NT * w + q) + n]);
         // dW0[i][c] of the tile = sum over rows of x[row][i] g0[row][c]; row IN of x^T holds ones
         for (int it = 0; 16 * it <= IN; ++it) {
@@ -543,7 +543,7 @@ __global__ __launch_bounds__(512) void dw_frag_kernel(DwFrag d, int steps, int s
             for (int b = 0; b < NB; ++b)
 #pragma unroll
                 for (int v = 0; v < 4; ++v)
-                    sum[(32 * wr + 16 * a + 4 * g + v) * RLD + 64 * wc + 16 * b + n] = hi[a][b][v] + lo[a][b][v];
+                    sum[(32 * wr + 16 * a + 4 * g + v) * RLD + 64 * wc + 16 * b + n] = split_sum(hi[a][b][v], lo[a][b][v]);
     }
     __syncthreads();
     if (half == 1) return;
@@ -555,7 +555,7 @@ __global__ __launch_bounds__(512) void dw_frag_kernel(DwFrag d, int steps, int s
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 const int r = 32 * wr + 16 * a + 4 * g + v, c = 64 * wc + 16 * b + n;
-                out[(size_t)r * H + c] = sum[r * RLD + c] + (hi[a][b][v] + lo[a][b][v]);
+                out[(size_t)r * H + c] = sum[r * RLD + c] + split_sum(hi[a][b][v], lo[a][b][v]);
             }
 }
 
