@@ -36,3 +36,27 @@ def test_integer_gradients_are_exact(mrl, tiles, H):
     want = torch.cat([t.reshape(-1) for t in (X.T @ g0, g0.sum(0), h1.T @ g1, g1.sum(0), h2.T @ G, G.sum(0))])
     assert float(want.abs().max()) < 2 ** 24
     assert torch.equal(grads.double(), want)
+
+
+@pytest.mark.parametrize("tiles,rows", [(64, 16), (127, 16), (4096, 32), (16384, 32)])
+def test_rounding_of_many_tiles(mrl, tiles, rows):
+    """The head's bias gradient is the sum of the output gradients: rows of a tile one after the other, tiles 64 at a time as
+    a tree.  With all terms in [1, 2) every partial sum is below the result, and an addition rounds by 2^-24 of it at most."""
+    B, H = rows * tiles, 64
+    model = mrl.seq(mrl.LinearReLU(3, H), mrl.LinearReLU(H, H), mrl.Linear(H, 1))
+    ctx = mrl.DeviceContext("cuda:0")
+    g = torch.Generator(device="cuda").manual_seed(tiles)
+    p = (torch.rand(model.PARAM_SIZE, device="cuda", generator=g) - 0.5) * 0.2
+    go = torch.rand(B, device="cuda", generator=g) + 1.0
+    out, cache, grads = (torch.zeros(n, device="cuda") for n in (B, B * model.CACHE_SIZE, model.PARAM_SIZE))
+    model.forward_gpu_ws(ctx, out, torch.randn(B * 3, device="cuda", generator=g), p, cache)
+    model.backward_gpu_ws(ctx, None, go, p, cache, grads)
+    ctx.synchronize()
+    want = float(go.double().sum())
+    # In units of 2^-24 of the result: the tiles' own sums, whose roundings are independent of one another, and the last
+    # bias below 4 together, the groups of 64 tiles 1 each at worst, of which independent roundings to nearest leave a
+    # sixteenth (their mean is a quarter of the worst, half of it on the way up, and they add up like a root: from 64 groups
+    # on an eighth of that), and 1 for the result itself.  One tile after the other would be 64 times the groups.
+    groups = max(1, tiles // 64)
+    bound = (4 + groups / 16 + 1) * 2.0 ** -24
+    assert abs(float(grads[-1]) - want) <= bound * want, (float(grads[-1]) / want - 1) * 2 ** 24
