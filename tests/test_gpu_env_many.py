@@ -21,6 +21,9 @@ def odd_rows(name, s, rng):
         s[0::9, 17 + 91 + 21 + 102] = 5.0                                    # a joint missing: stepped by the second launch
         s[3::9, 17 + 1] -= 0.6                                               # torso deep in the ground
         s[6::9, 17 + 3] = torch.from_numpy(rng.normal(0, 20, len(range(6, n, 9))).astype(np.float32))
+        s[1::9, 245] = 999.0                                                 # the step limit, also of rows with a missing
+        s[0::18, 245] = 999.0                                                # joint and of the last, started group of eight
+        s[-1, 245] = 999.0
         return
     bodies, joints, edges = 24, 104, 173
     ec = edges + 128 * 6
@@ -63,8 +66,50 @@ def test_many_equals_workgroup_form(mrl, ctx, name, batch):  # noqa: F811
         for got, want, what in ((plain, ref, "states"), (r1, r0, "rewards"), (d1, d0, "dones"), (o1, o0, "obs"), (r2, r0, "rewards"), (d2, d0, "dones")):
             same = (bits(got) == bits(want)).view(batch, -1).all(1)
             assert bool(same.all()), (what, t, torch.nonzero(~same).flatten()[:8].tolist())
-        if t >= 57:
-            assert float(d0.sum()) > (1 if name == "BipedalWalkerV2" else -1)
+        if t == 57 or (t > 57 and name == "BipedalWalkerV2"):               # (HalfCheetah ends at the step limit only)
+            assert float(d0.sum()) > 1
         E.selective_reset_kernel_gpu(ctx, ref, d0, 77 + t)
         assert torch.equal(bits(states), bits(ref))
         assert torch.equal(bits(o2.view(batch, -1)), bits(ref.view(batch, -1)[:, :E.OBS_DIM].contiguous()))
+
+
+@pytest.mark.parametrize("name,batch", [("BipedalWalkerV2", 4097), ("HalfCheetahPlanarV2", 8193)])
+def test_episode_accounting(mrl, ctx, name, batch):  # noqa: F811
+    """rollout_step above the switch: rewards, dones and rows as the workgroup form's on the same actions, running returns and
+    lengths and the list of finished episodes as those rewards add up to, for rows of either wiring."""
+    E = getattr(mrl, name)
+    steps, H, part = 6, 64, 1024
+    rng = np.random.default_rng(batch)
+    actor = mrl.seq(mrl.LinearTanh(E.OBS_DIM, H), mrl.LinearTanh(H, H), mrl.StochasticActor(H, E.ACTION_DIM))
+    critic = mrl.seq(mrl.LinearTanh(E.OBS_DIM, H), mrl.LinearTanh(H, H), mrl.Linear(H, 1))
+    g = torch.Generator(device="cuda").manual_seed(3)
+    rb = mrl.ppo.RolloutBuffers(ctx, E, actor, critic, batch, steps)
+    rb.actor_params = (torch.rand(actor.PARAM_SIZE, device="cuda", generator=g) - 0.5) * 0.2
+    rb.critic_params = (torch.rand(critic.PARAM_SIZE, device="cuda", generator=g) - 0.5) * 0.2
+    E.reset_kernel_gpu(ctx, rb.states, 5)
+    desc = rb.descriptor()
+    ret, length = torch.zeros(batch, device="cuda"), torch.zeros(batch, device="cuda")
+    finished = []
+    for t in range(steps):
+        if t in (1, 4):
+            odd_rows(name, rb.states.view(batch, -1), rng)
+        rb.obs.copy_(rb.states.view(batch, -1)[:, :E.OBS_DIM].reshape(-1).nan_to_num())
+        ref, r, d = rb.states.clone(), torch.zeros(batch, device="cuda"), torch.zeros(batch, device="cuda")
+        o = torch.zeros(batch * E.OBS_DIM, device="cuda")
+        mrl.ppo.rollout_step(ctx, desc, t, 100 + t, 0, 77 + t)
+        rows = slice(t * batch, (t + 1) * batch)
+        actions = rb.r_actions[t * batch * E.ACTION_DIM:(t + 1) * batch * E.ACTION_DIM]
+        for i in range(0, batch, part):
+            m = min(part, batch - i)
+            cut = lambda x, w: x[i * w:(i + m) * w]  # noqa: E731, B023
+            E.step_kernel_gpu(ctx, cut(ref, E.STATE_SIZE), cut(actions, E.ACTION_DIM), cut(r, 1), cut(d, 1), cut(o, E.OBS_DIM), 0)
+        assert torch.equal(bits(rb.r_rewards[rows]), bits(r)) and torch.equal(rb.r_dones[rows], d)
+        ret, length, over = ret + r, length + 1, d > 0.5
+        finished += list(zip(ret[over].nan_to_num(7.0).tolist(), length[over].tolist()))
+        ret[over], length[over] = 0.0, 0.0
+        E.selective_reset_kernel_gpu(ctx, ref, d, 77 + t)
+        assert torch.equal(bits(rb.states), bits(ref))
+        assert torch.equal(bits(rb.ep_return), bits(ret)) and torch.equal(rb.ep_length, length)
+    n = int(rb.done_count)
+    assert n == len(finished) and batch // 9 < n <= rb.done_cap
+    assert sorted(zip(rb.done_returns[:n].nan_to_num(7.0).tolist(), rb.done_lengths[:n].tolist())) == sorted(finished)

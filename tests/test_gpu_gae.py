@@ -1,4 +1,5 @@
-"""compute_gae at the edges of its groups of envs and chunks of steps; normalize_advantages around its unrolled sums."""
+"""compute_gae at the edges of its groups of envs and chunks of steps; normalize_advantages at sizes of a
+hundred thousand values and more."""
 import numpy as np
 import pytest
 import torch
@@ -43,5 +44,8 @@ def test_normalize_blocks(mrl, ctx, n):
     x = d(a)
     mrl.ppo.normalize_advantages(ctx, x)
     ctx.synchronize()
-    # sums of at most 20 terms a thread, then trees: relative error of mean and variance below 32 * 2^-24
-    np.testing.assert_allclose(x.cpu().numpy(), want, rtol=4e-6, atol=4e-6)
+    # sums in Float64; the fp32 mean is off by 2^-25 |mean|, and x - mean, the variance's root, its two sums and the quotient
+    # by 2^-24 each of the result (test_gpu_normalize.py takes the pieces, blocks and grid apart)
+    den = np.sqrt(a64.var() + 1e-8) + 1e-8
+    bound = 2.0 ** -24 * abs(a64.mean()) / den + 8 * 2.0 ** -24 * np.abs(want) + 1e-12
+    assert (np.abs(x.cpu().numpy() - want) <= bound).all()

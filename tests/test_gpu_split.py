@@ -1,6 +1,6 @@
 """The minibatch update's products on the bf16 matrix cores with split operands (three bf16 pieces per float, the six
-largest of the nine products): against Float64 they must not be further off than the fp32 matrix instructions that the
-stand-alone forward and backward use.  Both are measured in the same test, on inputs and weights of the agents' size, and
+largest of the nine products): against Float64 they must not be further off than the fp32 matrix instructions of the
+layer-by-layer kernels.  Both are measured in the same test, on inputs and weights of the agents' size, and
 at tile edges (one row, a started 16- and 32-row tile, the sizes where the tile height changes)."""
 import pytest
 import torch
@@ -45,10 +45,23 @@ def test_split_products_are_as_close_to_float64_as_fp32(mrl, ctx, H, IN, MB, rel
     upd.returns.normal_(generator=g)
     v64, g64 = _ref(p0, IN, H, x.view(MB, IN), upd.returns, relu)
     upd.minibatch_step(torch.arange(MB, dtype=torch.int32, device="cuda"))
-    # the same with the fp32 matrix instructions
-    v32, cache, g32 = (torch.zeros(n, device="cuda") for n in (MB, MB * critic.CACHE_SIZE, critic.PARAM_SIZE))
-    critic.forward_gpu_ws(ctx, v32, x, p0, cache)
-    critic.backward_gpu_ws(ctx, None, (v32 - upd.returns) / MB, p0, cache, g32)
+    # the same with the fp32 matrix instructions: a layer per model (the three together would take the fused kernels)
+    models = [lay(IN, H), lay(H, H), mrl.Linear(H, 1)]
+    acts, caches, parts, off = [x], [], [], 0
+    for m in models:
+        parts.append(p0[off:off + m.PARAM_SIZE].clone())
+        off += m.PARAM_SIZE
+        y, cache = torch.zeros(MB * m.OUT_DIM, device="cuda"), torch.zeros(MB * m.CACHE_SIZE, device="cuda")
+        m.forward_gpu_ws(ctx, y, acts[-1], parts[-1], cache)
+        acts.append(y)
+        caches.append(cache)
+    v32, grad, g32 = acts[-1], (acts[-1] - upd.returns) / MB, []
+    for m, p, cache, below in zip(models[::-1], parts[::-1], caches[::-1], acts[-2::-1]):
+        gp, gx = torch.zeros(m.PARAM_SIZE, device="cuda"), torch.zeros(below.numel(), device="cuda")
+        m.backward_gpu_ws(ctx, gx, grad, p, cache, gp)
+        g32.insert(0, gp)
+        grad = gx
+    g32 = torch.cat(g32)
     ctx.synchronize()
     err = lambda a, b: float((a.double() - b).norm() / b.norm())
     ev, ev32, eg, eg32 = err(upd.values, v64), err(v32, v64), err(upd.critic_grads, g64), err(g32, g64)
