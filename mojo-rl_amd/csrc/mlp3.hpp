@@ -45,7 +45,7 @@ struct FwdLoss {
     // it behind their first requests.  0.6 us of a minibatch's 51 at H = 256 and 4096 rows, for the 45 of one behind the stop.)
     int dw_in_tiles;                                      // forward + backward: the row tiles leave their dW1 as well
     int mb, A, continuous, clip_value;                    // A = actions (discrete) or action width (continuous)
-    float clip_eps, ent_coef, value_coef, target_kl;
+    float clip_eps, ent_coef, value_coef;
 };
 
 bool mlp3_fusable(const mrl_mlp_desc &d, int *H, int *act, bool *gauss);

@@ -17,17 +17,15 @@
 
 namespace mrl {
 
-// grid = (row tiles, nets): blockIdx.y picks the net, so that an actor and a critic that read the
-// same inputs go through the chip side by side
+// grid = row tiles
 template <int H, int ACT>
-__global__ __launch_bounds__(2 * H) void mlp3_fwd_kernel(int B, int IN, Mlp3Nets nets) {
+__global__ __launch_bounds__(2 * H) void mlp3_fwd_kernel(int B, int IN, Mlp3Net nn) {
     constexpr int T = 2 * H;   // one 32-column accumulator tile per wavefront
     __shared__ float xs[PR * XS_LD];
     __shared__ float hT[H * HT_LD];
     __shared__ float h2[PR * (H + 1)];
     __shared__ float ys[PR * (PA_MAX + 1)];
     __shared__ __align__(16) float w2s[HEAD_LDS(H)];
-    const Mlp3Net &nn = nets.n[blockIdx.y];
     const float *__restrict__ x = nn.x;
     const float *__restrict__ params = nn.params;
     float *__restrict__ out = nn.out;
@@ -87,11 +85,11 @@ __global__ __launch_bounds__(2 * H) void mlp3_fwd_kernel(int B, int IN, Mlp3Nets
 
 // Flat gradient vector of each net from the pieces: weight blocks = sum over the batch splits of
 // `partial`, bias rows and the log_std tail (Gaussian head) = sum over the row tiles of the column
-// sums the backward-dx kernel left.  The nets' vectors lie back to back in `partial`.
+// sums the tiles left.  The nets' vectors lie back to back in `partial`.
 struct SumNets {
     float *grads[2];
     const float *ls_part[2], *db_part[2], *thin_part[2];
-    int P[2], A[2], gauss[2];
+    int P[2], A[2];
     int n, IN, H;
     int thin_stride[2];   // floats per row tile in thin_part, per net
     const int32_t *skip;   // as FwdLoss::skip
@@ -165,7 +163,7 @@ __global__ __launch_bounds__(256) void sum3_kernel(const float *__restrict__ par
             n = tiles;
         }
         else if (bias_layer < 0 && i >= o1 && i < o1 + H * H) { p = partial + gi; stride = (size_t)Ptot; n = splits; }
-        else if (bias_layer < 0) {   // a weight of layer 0 or of the head: per-tile pieces of the dx kernel
+        else if (bias_layer < 0) {   // a weight of layer 0 or of the head: per-tile pieces
             p = sn.thin_part[net] + (i < o1 ? i : (size_t)IN * H + (i - o2));
             stride = (size_t)sn.thin_stride[net];
             n = tiles;
@@ -250,26 +248,26 @@ static bool fwd_rows_16(int n_cus, int H, int batch) {
 }
 
 template <int H, int ACT>
-static void launch_fwd_t(mrl_ctx *ctx, int batch, int IN, const Mlp3Nets &nets) {
-    hipLaunchKernelGGL((mlp3_fwd_kernel<H, ACT>), dim3((batch + PR - 1) / PR), dim3(2 * H), 0, ctx->stream, batch, IN, nets);
+static void launch_fwd_t(mrl_ctx *ctx, int batch, int IN, const Mlp3Net &nn) {
+    hipLaunchKernelGGL((mlp3_fwd_kernel<H, ACT>), dim3((batch + PR - 1) / PR), dim3(2 * H), 0, ctx->stream, batch, IN, nn);
 }
 int mlp3_forward(mrl_ctx *ctx, const mrl_mlp_desc &d, int batch, const float *in, const float *params,
                  float *out, float *cache) {
     int H = 0, act = 0;
     bool gauss = false;
     if (!mlp3_fusable(d, &H, &act, &gauss)) return MRL_E_UNSUPPORTED;
-    Mlp3Nets io{};
-    io.n[0].x = in; io.n[0].params = params; io.n[0].out = out; io.n[0].cache = cache;
-    io.n[0].A = d.layers[2].out_dim;
-    io.n[0].gauss = gauss ? 1 : 0;
+    Mlp3Net nn{};
+    nn.x = in; nn.params = params; nn.out = out; nn.cache = cache;
+    nn.A = d.layers[2].out_dim;
+    nn.gauss = gauss ? 1 : 0;
     const int IN = d.layers[0].in_dim;
-    if (fwd_rows_16(ctx->n_cus, H, batch)) return launch_fwd16(ctx, H, act, batch, IN, io.n[0]);
-    if (H == 256 && act == 1) launch_fwd_t<256, 1>(ctx, batch, IN, io);
-    else if (H == 256) launch_fwd_t<256, 2>(ctx, batch, IN, io);
-    else if (H == 128 && act == 1) launch_fwd_t<128, 1>(ctx, batch, IN, io);
-    else if (H == 128) launch_fwd_t<128, 2>(ctx, batch, IN, io);
-    else if (act == 1) launch_fwd_t<64, 1>(ctx, batch, IN, io);
-    else launch_fwd_t<64, 2>(ctx, batch, IN, io);
+    if (fwd_rows_16(ctx->n_cus, H, batch)) return launch_fwd16(ctx, H, act, batch, IN, nn);
+    if (H == 256 && act == 1) launch_fwd_t<256, 1>(ctx, batch, IN, nn);
+    else if (H == 256) launch_fwd_t<256, 2>(ctx, batch, IN, nn);
+    else if (H == 128 && act == 1) launch_fwd_t<128, 1>(ctx, batch, IN, nn);
+    else if (H == 128) launch_fwd_t<128, 2>(ctx, batch, IN, nn);
+    else if (act == 1) launch_fwd_t<64, 1>(ctx, batch, IN, nn);
+    else launch_fwd_t<64, 2>(ctx, batch, IN, nn);
     MRL_CHECK_LAUNCH();
     return MRL_OK;
 }
@@ -302,7 +300,6 @@ static int sum_tiles(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets,
         sn.thin_stride[i] = nn.thin_stride;
         sn.P[i] = net_P(*descs[i]);
         sn.A[i] = nn.A;
-        sn.gauss[i] = nn.gauss;
         Ptot += sn.P[i];
     }
     const int sum_blocks = grid_for(Ptot, 256);

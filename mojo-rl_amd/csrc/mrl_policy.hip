@@ -210,18 +210,18 @@ int launch_policy(mrl_ctx *ctx, const mrl_mlp_desc &a, const mrl_mlp_desc &c, bo
         MRL_CHECK_LAUNCH();
         return MRL_OK;
     }
-    // few row tiles: actor and critic of a tile go to workgroups of their own (twice the CUs at work),
-    // at hidden width 256 with one column tile per wavefront (eight wavefronts per net: two per SIMD,
-    // where a workgroup of four would leave each SIMD a single wavefront with nothing to overlap)
+    // few row tiles at hidden width 256 (at the others the 16-row tiles take them): actor and critic of a tile go
+    // to workgroups of their own (twice the CUs at work), with one column tile per wavefront (eight wavefronts per net:
+    // two per SIMD, where a workgroup of four would leave each SIMD a single wavefront with nothing to overlap)
     const int tiles = (n + PR - 1) / PR;
-    const bool split = 2 * tiles <= POLICY_SPLIT_BELOW;
+    const bool split = H == 256 && 2 * tiles <= POLICY_SPLIT_BELOW;
     dim3 grid(tiles, split ? 2 : 1);
 #define MRL_LAUNCH(HH, AA, GG)                                                                         \
-    if ((split && HH == 256) || HH == 128)                                                              \
+    if (split || HH == 128)                                                                            \
         hipLaunchKernelGGL((policy_kernel<HH, AA, GG, 1>), grid, dim3((split ? 2 : 4) * HH), 0, ctx->stream, obs, \
                            n, IN, A, ap, cp, seed, actions, r_obs, r_actions, r_logp, r_values);        \
     else                                                                                                \
-        hipLaunchKernelGGL((policy_kernel<HH, AA, GG, PTPW>), grid, dim3((split ? 2 : 4) * HH / PTPW), 0, ctx->stream, obs, \
+        hipLaunchKernelGGL((policy_kernel<HH, AA, GG, PTPW>), grid, dim3(4 * HH / PTPW), 0, ctx->stream, obs, \
                            n, IN, A, ap, cp, seed, actions, r_obs, r_actions, r_logp, r_values)
     if (gauss) {
         if (H == 256 && act == 1) MRL_LAUNCH(256, 1, true);

@@ -489,7 +489,6 @@ static int update_minibatch_paired(mrl_ctx *ctx, const mrl_update *u, const int3
     fl.mb = mb; fl.A = cont ? u->act_width : head; fl.continuous = cont ? 1 : 0;
     fl.clip_value = u->clip_value ? 1 : 0;
     fl.clip_eps = u->clip_epsilon; fl.ent_coef = u->entropy_coef; fl.value_coef = u->value_loss_coef;
-    fl.target_kl = u->target_kl;
     float *grads[2] = {u->actor_grads, u->critic_grads};
     int sq_blocks = 0;   // > 0: the sums over the tiles already left the sum-of-squares partials
     int rc = mlp3_update_n(ctx, descs, mb, io, ws, grads, u->max_grad_norm > 0.0f ? ctx->upd_scratch + SCR_SQ : nullptr,
