@@ -40,9 +40,9 @@ struct FwdLoss {
     float *g_actor_out, *g_values, *kl;                   // [mb, head], [mb], [mb]
     float *kl_part;                                       // [row tiles] sums of the tiles' KL estimates, for the test
     int32_t *kl_flag;                                     // null: no test (nothing is left in kl_part)
-    const int32_t *skip;                                  // not null and *skip != 0: nothing of this minibatch is needed
-    // (The kernels request the word first, always -- without a flag some other word is read, and not looked at -- and test
-    // it behind their first requests.  0.6 us of a minibatch's 51 at H = 256 and 4096 rows, for the 45 of one behind the stop.)
+    const int32_t *skip;                                  // *skip != 0: nothing of this minibatch is needed (null: a word that is 0)
+    // (The kernels request the word first, always, and test it behind their first requests.  0.6 us of a minibatch's 51 at
+    // H = 256 and 4096 rows, for the 45 of one behind the stop.)
     int dw_in_tiles;                                      // forward + backward: the row tiles leave their dW1 as well
     int mb, A, continuous, clip_value;                    // A = actions (discrete) or action width (continuous)
     float clip_eps, ent_coef, value_coef;

@@ -34,7 +34,7 @@ struct DwFrag {
     int n;        // nets
     const unsigned short *x[2], *g[2];
     int off[2];   // of the net's W1 gradient in a split's partial vector
-    const int32_t *skip;   // as FwdLoss::skip
+    const int32_t *skip;   // as FwdLoss::skip, never null
 };
 
 template <int H, int ACT, int RT>
@@ -69,7 +69,7 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
     const bool actor = blockIdx.y == 0;
 
     // ---- everything that does not depend on an earlier phase is requested first.  Rows: sixteen lanes each.
-    const int skip = *(fl.skip != nullptr ? fl.skip : fl.idx);   // (tested once these requests are out)
+    const int skip = *fl.skip;   // (tested once these requests are out)
     __builtin_amdgcn_sched_barrier(0);
     constexpr int XQ = (R * 16 + T - 1) / T;
     long xsrc[XQ];
@@ -118,7 +118,7 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
         }
     }
     if (actor && fl.adv_stats != nullptr) { l_mean = fl.adv_stats[0]; l_std = fl.adv_stats[1]; }
-    if (fl.skip != nullptr && skip != 0) return;
+    if (skip != 0) return;
     // (the weights last: a wavefront's loads come back in order, and the rows are waited for first)
     __builtin_amdgcn_sched_barrier(0);
     bf16x8 wq[PF][NT][SPLIT];
@@ -483,7 +483,7 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
 template <int H>
 __global__ __launch_bounds__(512) void dw_frag_kernel(DwFrag d, int steps, int steps_per, int splits, int Ptot,
                                                       float *__restrict__ partial) {
-    const int skip = *(d.skip != nullptr ? d.skip : reinterpret_cast<const int32_t *>(d.x[0]));
+    const int skip = *d.skip;
     __builtin_amdgcn_sched_barrier(0);
     constexpr int XCDS = 8, TN = 128, tiles_n = H / TN, tiles = tiles_n * (H / 64), NB = 4, RLD = TN + 4;
     static_assert(H % TN == 0, "whole tiles");
@@ -525,7 +525,7 @@ __global__ __launch_bounds__(512) void dw_frag_kernel(DwFrag d, int steps, int s
             for (int a = 0; a < 2; ++a) mfma_split(fa[u][a], fb[u][b], hi[a][b], lo[a][b]);
     };
     if (k0 < k1) fetch(k0, 0);
-    if (d.skip != nullptr && skip != 0) return;
+    if (skip != 0) return;
     for (int k = k0; k < k1; k += 4) {   // two k-steps per round, so that the buffers keep their names
         if (k + 2 < k1) fetch(k + 2, 1);
         __builtin_amdgcn_sched_barrier(0);

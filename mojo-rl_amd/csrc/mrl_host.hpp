@@ -32,7 +32,7 @@ struct mrl_ctx {
     size_t rollout_ws_floats;
     // scratch of the minibatch update: per-block KL partials [0, 1024), their arrival counter
     // (int, at float index 1024; zero between launches), the word of env_step_many (int, FOREIGN_WORD),
-    // sum-of-squares partials [2048, 4096),
+    // a word that stays 0 (NEVER_WORD), sum-of-squares partials [2048, 4096),
     // advantage {mean, std} of up to 2048 minibatches [4096, 8192)
     float *upd_scratch;
     int foreign_call;   // env_step_many calls so far
@@ -92,6 +92,10 @@ constexpr int FOREIGN_WORD = 1028;
 bool env_step_many_pays(const mrl_ctx *ctx, int env_id, int batch);
 void env_step_many(mrl_ctx *ctx, int env_id, int batch, float *states, const float *actions, float *rewards, float *dones,
                    float *obs, bool autoreset, uint64_t reset_seed, const Accounting &acc);
+
+// where the kernels of a minibatch that no KL stop can skip look for one
+constexpr int NEVER_WORD = 1032;
+inline const int32_t *never_skip(const mrl_ctx *ctx) { return reinterpret_cast<const int32_t *>(ctx->upd_scratch + NEVER_WORD); }
 
 // CartPole's per-env step counters for the rows at `states` (created zeroed on first use)
 int cartpole_side(mrl_ctx *ctx, const float *states, int batch, int32_t **out);

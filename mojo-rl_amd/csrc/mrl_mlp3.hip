@@ -92,7 +92,7 @@ struct SumNets {
     int P[2], A[2];
     int n, IN, H;
     int thin_stride[2];   // floats per row tile in thin_part, per net
-    const int32_t *skip;   // as FwdLoss::skip
+    const int32_t *skip;   // as FwdLoss::skip, never null
     int hh_in_tiles;   // the H x H block is summed from the row tiles' pieces (behind dW0 and dW2) instead of `partial`
 };
 
@@ -137,7 +137,7 @@ MRL_DEV float sum_strided(const float *__restrict__ p, size_t stride, int n) {
 
 __global__ __launch_bounds__(256) void sum3_kernel(const float *__restrict__ partial, int splits, int Ptot,
                                                    int tiles, SumNets sn, float *__restrict__ sq_part) {
-    const int skip = *(sn.skip != nullptr ? sn.skip : reinterpret_cast<const int32_t *>(partial));
+    const int skip = *sn.skip;
     __builtin_amdgcn_sched_barrier(0);
     __shared__ float red[2][4];
     const int gi = blockIdx.x * blockDim.x + threadIdx.x;
@@ -174,7 +174,7 @@ __global__ __launch_bounds__(256) void sum3_kernel(const float *__restrict__ par
             stride = (size_t)(2 * H + PA_MAX);
             n = tiles;
         }
-        if (sn.skip == nullptr || skip == 0) {
+        if (skip == 0) {
             s = sum_strided(p, stride, n);
             sn.grads[net][i] = s;
         }
@@ -377,6 +377,7 @@ int mlp3_update_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int batch, Mlp
     }
     FwdLoss fl = loss;
     fl.dw_in_tiles = ws.dw_in_tiles ? 1 : 0;
+    if (fl.skip == nullptr) fl.skip = never_skip(ctx);
     int rc = launch_fb(ctx, H, act, batch, descs[0]->layers[0].in_dim, ws.rows, io, fl);
     if (rc) return rc;
     if (!ws.dw_in_tiles) {
@@ -420,10 +421,10 @@ int mlp3_backward(mrl_ctx *ctx, const mrl_mlp_desc &d, int batch, const float *g
     rc = launch_bwd(ctx, H, act, batch, IN, ws.rows, nn, ws.dw_in_tiles);
     if (rc) return rc;
     if (!ws.dw_in_tiles) {
-        rc = launch_dw_frag(ctx, H, 1, batch, ws, P, P, (IN + 1) * H, nullptr);
+        rc = launch_dw_frag(ctx, H, 1, batch, ws, P, P, (IN + 1) * H, never_skip(ctx));
         if (rc) return rc;
     }
-    return sum_tiles(ctx, ds, 1, io, ws.tiles, ws.dw_in_tiles, ws.partial, ws.splits, gs, nullptr, nullptr, nullptr);
+    return sum_tiles(ctx, ds, 1, io, ws.tiles, ws.dw_in_tiles, ws.partial, ws.splits, gs, nullptr, nullptr, never_skip(ctx));
 }
 
 }  // namespace mrl
