@@ -352,7 +352,8 @@ int mrl_rollout_step(mrl_ctx *ctx, const mrl_rollout *r, int t, uint32_t sample_
 int mrl_rollout_steps(mrl_ctx *ctx, const mrl_rollout *r, int t0, int n_steps, uint32_t sample_seed,
                       uint32_t sample_stride, uint64_t step_seed, uint64_t step_stride,
                       uint64_t reset_seed, uint64_t reset_stride);
-/* 1 when mrl_rollout_steps runs this descriptor as one launch per call, 0 when it issues the
+/* 1 when mrl_rollout_steps runs this descriptor as one launch per call on a context of the current
+ * device (how many envs pay depends on its number of CUs), 0 when it issues the
  * steps one by one (no counterpart in the reference: a caller that times launches asks this). */
 int mrl_rollout_fused(const mrl_rollout *r);
 

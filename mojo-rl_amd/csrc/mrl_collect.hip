@@ -377,11 +377,9 @@ static bool agent_nets(const mrl_rollout *r, int obs, int head, bool gauss, int 
     return true;
 }
 
-// n_cus = 0: the form for a device of unknown size is asked for (mrl_rollout_fused has no context)
 static CollectPlan collect_plan(const mrl_rollout *r, int n_cus) {
     const bool gauss = r->num_actions == 0;
     CollectPlan p{FORM_STEPS, 0, 0};
-    if (n_cus == 0) n_cus = 256;
     const int id = r->env_id;
     int obs = 0, head = 0;
     // Up to this many envs per CU the walkers' fused kernels are the faster way; with more, their 16-env workgroups
@@ -432,7 +430,15 @@ using namespace mrl;
 extern "C" {
 
 int mrl_rollout_fused(const mrl_rollout *r) {
-    return r != nullptr && collect_plan(r, 0).form != FORM_STEPS ? 1 : 0;
+    if (r == nullptr) return 0;
+    // (the current device, which is the context's where the call is made beside mrl_rollout_steps; without one, an MI355X)
+    int device = 0, n_cus = 0;
+    if (hipGetDevice(&device) != hipSuccess ||
+        hipDeviceGetAttribute(&n_cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) {
+        (void)hipGetLastError();
+        n_cus = 256;
+    }
+    return collect_plan(r, n_cus).form != FORM_STEPS ? 1 : 0;
 }
 
 int mrl_rollout_steps(mrl_ctx *ctx, const mrl_rollout *r, int t0, int n_steps, uint32_t sample_seed,
