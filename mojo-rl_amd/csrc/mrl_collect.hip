@@ -382,25 +382,32 @@ static CollectPlan collect_plan(const mrl_rollout *r, int n_cus) {
     CollectPlan p{FORM_STEPS, 0, 0};
     const int id = r->env_id;
     int obs = 0, head = 0;
-    // Up to this many envs per CU the walkers' fused kernels are the faster way; with more, their 16-env workgroups
-    // come round after round while the stand-alone kernels fill the chip.  us per step, fused against two launches,
-    // hidden width 64 / 256: HalfCheetah (one workgroup per CU) 4096 envs 69 / 73 : 84 / 88, 8192 envs 136 / 146 :
-    // 82 / 99; Walker2d 8192 envs 23.6 / 43.6 : 26.2 / 44.7, 16384 envs 46.6 / 86.6 : 31.2 / 76.5; CarRacing 8192 envs
-    // 38 / 61 : 46 / 65, 16384 envs 76 / 121 : 72 / 116; Hopper 16384 envs 19 / 69 : 25 / 69, 32768 envs 38 / 136 :
-    // 35 / 130; BipedalWalker 32768 envs 265 / 305 : 318 / 409.
-    int envs_per_cu = 0;   // 0: no limit
     if (id == MRL_ENV_BIPEDAL) { obs = BipedalWalker::OBS; head = BipedalWalker::ACT_W; }
-    else if (id == MRL_ENV_HALFCHEETAH) { obs = HalfCheetah::OBS; head = HalfCheetah::ACT_W; envs_per_cu = 16; }
-    else if (id == MRL_ENV_CARRACING) { obs = cr::OBS; head = cr::ACT; envs_per_cu = 32; }
-    else if (id == MRL_ENV_HOPPER_PLANAR) { obs = planar::Hopper::OBS; head = planar::Hopper::ACT; envs_per_cu = 64; }
-    else if (id == MRL_ENV_WALKER2D_PLANAR) { obs = planar::Walker2d::OBS; head = planar::Walker2d::ACT; envs_per_cu = 32; }
+    else if (id == MRL_ENV_HALFCHEETAH) { obs = HalfCheetah::OBS; head = HalfCheetah::ACT_W; }
+    else if (id == MRL_ENV_CARRACING) { obs = cr::OBS; head = cr::ACT; }
+    else if (id == MRL_ENV_HOPPER_PLANAR) { obs = planar::Hopper::OBS; head = planar::Hopper::ACT; }
+    else if (id == MRL_ENV_WALKER2D_PLANAR) { obs = planar::Walker2d::OBS; head = planar::Walker2d::ACT; }
     if (head > 0) {
-        if (envs_per_cu > 0 && r->n_envs > envs_per_cu * n_cus) return p;
         // (the planar rows hold doubles; the weight rows are read with 16-byte loads)
         if (id >= MRL_ENV_HOPPER_PLANAR && reinterpret_cast<uintptr_t>(r->states) % 8 != 0) return p;
         if (reinterpret_cast<uintptr_t>(r->actor_params) % 16 != 0 || reinterpret_cast<uintptr_t>(r->critic_params) % 16 != 0)
             return p;
-        if (gauss && agent_nets(r, obs, head, true, &p.H, &p.act)) p.form = FORM_WALKER;
+        if (!gauss || !agent_nets(r, obs, head, true, &p.H, &p.act)) return p;
+        // Up to this many envs per CU the walkers' fused kernels are the faster way; with more, their 16-env workgroups
+        // come round after round while the stand-alone kernels fill the chip.  us per step, fused against two launches,
+        // hidden width 64 / 256:
+        //   HalfCheetah (one workgroup per CU)  4096 envs 68 / 73 : 74 / 88,  8192 envs 136 / 147 : 74 / 99;
+        //   Walker2d  4096 envs 12.4 / 22.3 : 17.7 / 31.7,  4200 envs 24.0 / 43.8 : 22.6 / 47.5,  8192 envs 24.4 / 44.0 : 19.9 / 44.5
+        //     (width 128 27.7 : 27.4),  16384 envs 47 / 87 : 31 / 76;
+        //   CarRacing  4096 envs 20 / 31 : 28 / 41,  8192 envs 39 / 61 : 41 / 65,  16384 envs 76 / 121 : 72 / 116;
+        //   Hopper  8192 envs 9.6 / 36 : 15.3 / 39,  16384 envs 22 / 70 : 26 / 69,  32768 envs 38 / 138 : 36 / 129;
+        //   BipedalWalker  4096 envs 36 / 41 : 47 / 60,  8192 envs 70 / 81 : 71 / 97,  12288 envs 105 / 121 : 90 / 134,
+        //     16384 envs 139 / 160 : 97 / 140,  32768 envs 274 / 315 : 162 / 251.
+        int envs_per_cu = 32;
+        if (id == MRL_ENV_HALFCHEETAH || (id == MRL_ENV_WALKER2D_PLANAR && p.H == 64)) envs_per_cu = 16;
+        else if (id == MRL_ENV_BIPEDAL && p.H == 256) envs_per_cu = 48;
+        else if (id == MRL_ENV_HOPPER_PLANAR) envs_per_cu = 64;
+        if (r->n_envs <= envs_per_cu * n_cus) p.form = FORM_WALKER;
         return p;
     }
     if ((id == MRL_ENV_LUNARLANDER && !gauss) || (id == MRL_ENV_LUNARLANDER_CONTINUOUS && gauss)) {

@@ -66,27 +66,27 @@ def _pair(mrl, ctx, N, T, hidden, kind, env="lunar"):
 
 @pytest.mark.parametrize("env,N,T,hidden,kind", [
     ("lunar", 8192, 12, 256, "relu"), ("lunar", 1000, 9, 256, "tanh"), ("lunar", 77, 5, 256, "relu"),
-    ("lunar", 300, 6, 64, "relu"),            # not fusable: the loop of single steps behind the same call
+    ("lunar", 300, 6, 64, "relu"),            # (width 64: the 16-row kernel)
     # above 8192 envs the single steps run the one-lane-per-env step kernel (rows in global memory,
     # detection inline, accounting and reset by the env's lane) against the fused kernel's 32-row workgroups
     ("lunar", 9001, 8, 256, "relu"), ("lunarc", 9001, 6, 256, "tanh"),
     ("cartpole", 8192, 12, 64, "relu"), ("cartpole", 77, 7, 64, "tanh"),
     ("pendulum", 8192, 12, 64, "tanh"), ("pendulum", 1000, 9, 64, "relu"),
-    ("cartpole", 300, 6, 256, "relu"),        # not fusable
+    ("cartpole", 300, 6, 256, "relu"),        # (another hidden width)
     ("lunarc", 8192, 12, 256, "tanh"), ("lunarc", 77, 6, 256, "relu"), ("lunarc", 300, 6, 64, "tanh"),
     # the walkers: legs on the ground from the first step (contacts, joint limits, lidar), falls and
     # step-limit endings with in-place resets inside the launch
     ("bipedal", 4096, 12, 256, "tanh"), ("bipedal", 77, 7, 256, "relu"), ("bipedal", 500, 64, 256, "tanh"),
     ("cheetah", 4096, 12, 256, "tanh"), ("cheetah", 77, 7, 256, "relu"), ("cheetah", 500, 64, 256, "tanh"),
-    ("cheetah", 300, 5, 64, "tanh"),          # not fusable
+    ("cheetah", 300, 5, 64, "tanh"),          # (another hidden width)
     # CarRacing: tiles are visited from the first step on (the flags an env wrote are read back by later
     # steps of the same launch), truncations rebuild the track inside the launch
     ("car", 4096, 12, 256, "tanh"), ("car", 77, 7, 256, "relu"), ("car", 300, 48, 256, "tanh"),
-    ("car", 100, 5, 64, "tanh"),              # not fusable
+    ("car", 100, 5, 64, "tanh"),              # (another hidden width)
     # the Float64 planar envs: unhealthy torsos end episodes from the first step on, resets inside the launch
     ("hopper", 4096, 12, 256, "tanh"), ("hopper", 77, 7, 256, "relu"), ("hopper", 500, 64, 256, "tanh"),
     ("walker2d", 4096, 12, 256, "tanh"), ("walker2d", 77, 7, 256, "relu"), ("walker2d", 500, 64, 256, "tanh"),
-    ("hopper", 100, 5, 64, "tanh"),           # not fusable
+    ("hopper", 100, 5, 64, "tanh"),           # (another hidden width)
 ])
 def test_rollout_steps_equals_single_steps(mrl, ctx, env, N, T, hidden, kind):
     print("case", env, N, T, hidden, kind, flush=True)
