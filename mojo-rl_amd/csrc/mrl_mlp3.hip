@@ -99,10 +99,11 @@ struct SumNets {
 // n terms of `p`, `stride` floats apart.  The chain of memory round trips is what this takes, so up to 64 terms are
 // requested at a time, and the last few of a number that is no multiple of 8 go out together as well: with a
 // request at a time behind the last 16, the sum over 63 tiles took 8.7 us of a minibatch's 31 (H = 128, 1000 rows), now 5.3.
-// What is requested together is added up as a tree of neighbours, in the order it comes back: one term after the other,
-// twice the tiles (16 rows each where there were 32) had made the gradients of 2048-row minibatches (H = 256, 24 inputs)
-// less exact, 1.43e-7 -> 1.55e-7 off Float64; as a tree 0.75e-7, in the same time (a tree of the two halves, which waits
-// for the last request before it adds, cost 1.5 us of an update's 50 per minibatch).
+// They are added one after the other, or (TREE) what is requested together as a tree of neighbours, in the order it comes
+// back.  The pieces of 16-row tiles take the tree: they are twice as many as those of 32-row tiles, and one after the other
+// their roundings had made the gradients of 2048-row minibatches (H = 256, 24 inputs) less exact, 1.43e-7 -> 1.55e-7 off
+// Float64; as a tree 0.75e-7, in the same time.
+template <bool TREE>
 MRL_DEV float sum_strided(const float *__restrict__ p, size_t stride, int n) {
     float s = 0.0f;
     auto whole = [&](auto width) {
@@ -110,11 +111,16 @@ MRL_DEV float sum_strided(const float *__restrict__ p, size_t stride, int n) {
         float v[W];
 #pragma unroll
         for (int k = 0; k < W; ++k) v[k] = p[(size_t)k * stride];
+        if constexpr (TREE) {
 #pragma unroll
-        for (int d = 1; d < W; d *= 2)
+            for (int d = 1; d < W; d *= 2)
 #pragma unroll
-            for (int k = 0; k < W; k += 2 * d) v[k] += v[k + d];
-        s += v[0];
+                for (int k = 0; k < W; k += 2 * d) v[k] += v[k + d];
+            s += v[0];
+        } else {
+#pragma unroll
+            for (int k = 0; k < W; ++k) s += v[k];
+        }
         p += W * stride;
         n -= W;
     };
@@ -135,6 +141,7 @@ MRL_DEV float sum_strided(const float *__restrict__ p, size_t stride, int n) {
     return s;
 }
 
+template <bool TREE>
 __global__ __launch_bounds__(256) void sum3_kernel(const float *__restrict__ partial, int splits, int Ptot,
                                                    int tiles, SumNets sn, float *__restrict__ sq_part) {
     const int skip = *sn.skip;
@@ -175,7 +182,7 @@ __global__ __launch_bounds__(256) void sum3_kernel(const float *__restrict__ par
             n = tiles;
         }
         if (skip == 0) {
-            s = sum_strided(p, stride, n);
+            s = sum_strided<TREE>(p, stride, n);
             sn.grads[net][i] = s;
         }
     }
@@ -279,17 +286,16 @@ static void dw_splits(int n_nets, int batch, int *splits, int *rows_per) {
     *splits = (batch + *rows_per - 1) / *rows_per;
 }
 
-// The sums over row tiles and batch splits into the flat gradients (hh_in_tiles: the tiles left the H x H weight
-// gradients too).
-static int sum_tiles(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, const Mlp3Nets &io, int tiles, bool hh_in_tiles,
-                     const float *partial, int splits, float *const *grads, float *sq_part, int *sq_blocks, const int32_t *skip) {
+// The sums over row tiles and batch splits into the flat gradients.
+static int sum_tiles(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, const Mlp3Nets &io, const UpdateWs &ws,
+                     float *const *grads, float *sq_part, int *sq_blocks, const int32_t *skip) {
     const int IN = descs[0]->layers[0].in_dim, H = descs[0]->layers[0].out_dim;
     SumNets sn{};
     sn.n = n_nets;
     sn.IN = IN;
     sn.skip = skip;
     sn.H = H;
-    sn.hh_in_tiles = hh_in_tiles ? 1 : 0;
+    sn.hh_in_tiles = ws.dw_in_tiles ? 1 : 0;
     int Ptot = 0;
     for (int i = 0; i < n_nets; ++i) {
         const Mlp3Net &nn = io.n[i];
@@ -305,8 +311,11 @@ static int sum_tiles(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets,
     const int sum_blocks = grid_for(Ptot, 256);
     if (sum_blocks > 1024) sq_part = nullptr;   // more partials than the caller's buffer holds
     if (sq_blocks) *sq_blocks = sq_part ? sum_blocks : 0;
-    hipLaunchKernelGGL(sum3_kernel, dim3(sum_blocks), dim3(256), 0, ctx->stream, partial, splits, Ptot, tiles,
-                       sn, sq_part);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(sum_blocks), dim3(256), 0, ctx->stream, ws.partial, ws.splits, Ptot, ws.tiles, sn, sq_part);
+    };
+    if (ws.rows == 16) launch(sum3_kernel<true>);
+    else launch(sum3_kernel<false>);
     MRL_CHECK_LAUNCH();
     return MRL_OK;
 }
@@ -385,7 +394,7 @@ int mlp3_update_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int batch, Mlp
         rc = launch_dw_frag(ctx, H, 2, batch, ws, P0, P0 + net_P(*descs[1]), (descs[0]->layers[0].in_dim + 1) * H, fl.skip);
         if (rc) return rc;
     }
-    return sum_tiles(ctx, descs, 2, io, ws.tiles, ws.dw_in_tiles, ws.partial, ws.splits, grads, sq_part, sq_blocks, fl.skip);
+    return sum_tiles(ctx, descs, 2, io, ws, grads, sq_part, sq_blocks, fl.skip);
 }
 
 // true when [a, a + na) and [b, b + nb) (floats) share memory
@@ -424,7 +433,7 @@ int mlp3_backward(mrl_ctx *ctx, const mrl_mlp_desc &d, int batch, const float *g
         rc = launch_dw_frag(ctx, H, 1, batch, ws, P, P, (IN + 1) * H, never_skip(ctx));
         if (rc) return rc;
     }
-    return sum_tiles(ctx, ds, 1, io, ws.tiles, ws.dw_in_tiles, ws.partial, ws.splits, gs, nullptr, nullptr, never_skip(ctx));
+    return sum_tiles(ctx, ds, 1, io, ws, gs, nullptr, nullptr, never_skip(ctx));
 }
 
 }  // namespace mrl

@@ -64,10 +64,18 @@ def test_split_products_are_as_close_to_float64_as_fp32(mrl, ctx, H, IN, MB, rel
     g32 = torch.cat(g32)
     ctx.synchronize()
     err = lambda a, b: float((a.double() - b).norm() / b.norm())
+    hh = slice((IN + 1) * H, (IN + 1) * H + H * H)                       # dW1, a split product at H = 256
     ev, ev32, eg, eg32 = err(upd.values, v64), err(v32, v64), err(upd.critic_grads, g64), err(g32, g64)
-    print("  values %.2e (fp32 %.2e)  gradients %.2e (fp32 %.2e)" % (ev, ev32, eg, eg32), flush=True)
+    ew, ew32 = err(upd.critic_grads[hh], g64[hh]), err(g32[hh], g64[hh])
+    print("  values %.2e (fp32 %.2e)  gradients %.2e (fp32 %.2e)  dW1 %.2e (fp32 %.2e)" % (ev, ev32, eg, eg32, ew, ew32), flush=True)
     # Over a thousand rows and more the errors average: the split products may not add to what fp32 shows (a quarter for
     # the spread of two independent sets of roundings).  A handful of rows shows single roundings, half an ulp = 6e-8
     # each: the value is the last of the chain h1, h2, head, bias (four).
     floor = 1e-7 if MB > 1000 else 3e-7
-    assert ev <= max(1.25 * ev32, floor) and eg <= max(1.25 * eg32, floor)
+    assert ev <= max(1.25 * ev32, floor)
+    if H == 256:
+        assert ew <= max(1.25 * ew32, floor)
+    # the other gradients are sums over the row tiles, n = MB / 32 pieces one after the other: partial sums of k pieces of
+    # either sign are sqrt(k / n) of the result, each rounded with a variance of (2^-24 of it)^2 / 3 at most, which is
+    # 2^-24 sqrt(n / 6) together (the layer-by-layer kernels have sums of their own in eg32)
+    assert eg <= max(1.25 * eg32 + 2.0**-24 * (MB / 32 / 6)**0.5, floor)

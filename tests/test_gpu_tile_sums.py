@@ -38,25 +38,25 @@ def test_integer_gradients_are_exact(mrl, tiles, H):
     assert torch.equal(grads.double(), want)
 
 
-@pytest.mark.parametrize("tiles,rows", [(64, 16), (127, 16), (4096, 32), (16384, 32)])
-def test_rounding_of_many_tiles(mrl, tiles, rows):
-    """The head's bias gradient is the sum of the output gradients: rows of a tile one after the other, tiles 64 at a time as
-    a tree.  With all terms in [1, 2) every partial sum is below the result, and an addition rounds by 2^-24 of it at most."""
-    B, H = rows * tiles, 64
-    model = mrl.seq(mrl.LinearReLU(3, H), mrl.LinearReLU(H, H), mrl.Linear(H, 1))
+def test_rounding_of_16_row_tiles(mrl):
+    """The head's bias gradient is the sum of the output gradients: rows of a tile one after the other, 256 tiles of 16 rows
+    in four trees of 64.  With all terms in [1, 2), V the result, a rounded sum v is off by at most 2^-24 v, with a variance of
+    a third of that square at most: V / 4 .. V along the four trees 1.9 V^2, within the trees 0.5 V^2, within the tiles 0.02 V^2,
+    so a root mean square below 0.9 * 2^-24 V; one tile after the other it would be 5.3.  64 sums estimate it to 9 %: 1.2."""
+    B, H, o = 4096, 64, 8
+    model = mrl.seq(mrl.LinearReLU(3, H), mrl.LinearReLU(H, H), mrl.Linear(H, o))
     ctx = mrl.DeviceContext("cuda:0")
-    g = torch.Generator(device="cuda").manual_seed(tiles)
+    g = torch.Generator(device="cuda").manual_seed(5)
     p = (torch.rand(model.PARAM_SIZE, device="cuda", generator=g) - 0.5) * 0.2
-    go = torch.rand(B, device="cuda", generator=g) + 1.0
-    out, cache, grads = (torch.zeros(n, device="cuda") for n in (B, B * model.CACHE_SIZE, model.PARAM_SIZE))
+    out, cache, grads = (torch.zeros(n, device="cuda") for n in (B * o, B * model.CACHE_SIZE, model.PARAM_SIZE))
     model.forward_gpu_ws(ctx, out, torch.randn(B * 3, device="cuda", generator=g), p, cache)
-    model.backward_gpu_ws(ctx, None, go, p, cache, grads)
-    ctx.synchronize()
-    want = float(go.double().sum())
-    # In units of 2^-24 of the result: the tiles' own sums, whose roundings are independent of one another, and the last
-    # bias below 4 together, the groups of 64 tiles 1 each at worst, of which independent roundings to nearest leave a
-    # sixteenth (their mean is a quarter of the worst, half of it on the way up, and they add up like a root: from 64 groups
-    # on an eighth of that), and 1 for the result itself.  One tile after the other would be 64 times the groups.
-    groups = max(1, tiles // 64)
-    bound = (4 + groups / 16 + 1) * 2.0 ** -24
-    assert abs(float(grads[-1]) - want) <= bound * want, (float(grads[-1]) / want - 1) * 2 ** 24
+    off = []
+    for _ in range(8):
+        go = torch.rand(B * o, device="cuda", generator=g) + 1.0
+        model.backward_gpu_ws(ctx, None, go, p, cache, grads)
+        ctx.synchronize()
+        want = go.double().view(B, o).sum(0)
+        off.append((grads[-o:].double() - want) / want * 2 ** 24)
+    rms = float(torch.cat(off).pow(2).mean().sqrt())
+    print("rms", rms)
+    assert rms < 1.2
