@@ -65,8 +65,9 @@ MRL_DEV void mfma_split(const bf16x8 (&a)[SPLIT], const bf16x8 (&b)[SPLIT], f32x
     lo = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[0], b[1], lo, 0, 0, 0);
 }
 
-// what hi and lo add up to
-MRL_DEV float split_sum(float hi, float lo) { return fabsf(hi) == INFINITY ? hi : hi + lo; }
+// what hi and lo add up to; a lo that is NaN, beside an infinite (or NaN) hi, becomes a finite number (v_med3_f32 takes the
+// lowest of the others), which leaves hi what it is
+MRL_DEV float split_sum(float hi, float lo) { return hi + __builtin_amdgcn_fmed3f(lo, -__FLT_MAX__, __FLT_MAX__); }
 
 // A hidden layer's weights W [H, H] as operands, split, in the order the lanes read them: piece p of the 8 elements
 // that lane `lane` holds in k-step ks (32 of the contracted index) of column tile ct (16 of the other index) starts at
