@@ -8,7 +8,12 @@
 //   * terrain stays in global memory; a phase stages the few edges near the env in LDS;
 //   * contacts go straight to their place in the env's list: the eight lanes take eight (body, vertex) pairs at a time,
 //     count first, then write behind the counts of the lanes before them;
-//   * rows of foreign wiring are left alone and stepped by a second launch, which ends at once where there are none.
+//   * rows of foreign wiring are left alone and stepped by a second launch, which ends at once where there are none
+//     (4.5 us of launch and of one word read, counted below).  No reset of this library makes such rows: a caller's own
+//     joint table does.  One lane steps such a row, from global memory, behind the other rows instead of beside them: us per
+//     step, workgroup form -> this one, one such row / every ninth / all:  BipedalWalker  8200 envs 85 -> 184 / 230 -> 233 /
+//     200 -> 242,  65536 envs 469 -> 340 / 1306 -> 922 / 1158 -> 1020;  HalfCheetah  8200 envs 212 -> 270 / 300 -> 321 / 374 -> 229,
+//     65536 envs 544 -> 468 / 1746 -> 1171 / 2121 -> 907.
 // Same operations on the same values as the workgroup forms: identical results bit for bit.
 //
 // What bounds it: the vector units' instruction stream, two to four wavefronts of dependent chains per SIMD
