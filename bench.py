@@ -329,13 +329,13 @@ def main():
         tflops = FWD_FLOPS * N_ENVS * steps_per_launch / (launch_us * 1e-6) / 1e12
         act_id = 1 if ACT == "relu" else 2
         name = {"lunarlander": "mrl::collect_kernel<mrl::LunarLander, %d, %d, false>" % (HIDDEN, act_id),
-                "cartpole": "mrl::collect_classic_kernel<mrl::CartPoleSlot, %d, false>" % act_id,
+                "cartpole": "mrl::collect_classic16_kernel<mrl::CartPoleSlot, 64, %d, false>" % act_id,
                 "pendulum": "mrl::collect_classic_kernel<mrl::PendulumSlot, %d, true>" % act_id,
-                "bipedal": "mrl::collect_walker_kernel<mrl::BipedalWalker, %d, false>" % act_id,
-                "halfcheetah": "mrl::collect_walker_kernel<mrl::HalfCheetah16, %d, true>" % act_id,
-                "carracing": "mrl::collect_car_kernel<%d>" % act_id,
-                "hopper": "mrl::collect_planar_kernel<mrl::planar::Hopper, %d>" % act_id,
-                "walker2d": "mrl::collect_planar_kernel<mrl::planar::Walker2d, %d>" % act_id}[args.workload]
+                "bipedal": "mrl::collect_walker_kernel<mrl::BipedalWalker, 256, %d, false>" % act_id,
+                "halfcheetah": "mrl::collect_walker_kernel<mrl::HalfCheetah16, 256, %d, true>" % act_id,
+                "carracing": "mrl::collect_car_kernel<256, %d>" % act_id,
+                "hopper": "mrl::collect_planar_kernel<mrl::planar::Hopper, 256, %d>" % act_id,
+                "walker2d": "mrl::collect_planar_kernel<mrl::planar::Walker2d, 256, %d>" % act_id}[args.workload]
         roofline = {"kernel": name + " (policy forward + sampling + env step + auto-reset + rollout stores, %d steps per launch)" % steps_per_launch,
                     "bound": "mfma", "achieved": tflops, "peak": MFMA_FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
                     "frac": tflops / MFMA_FP32_PEAK_TFLOPS,
