@@ -23,7 +23,10 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=o
 # coefficients of exp / log / sincos, two registers each) out of the loop into registers of their own,
 # the register allocator then spills them, and every use becomes a dependent load from private memory in
 # the middle of the solver wavefront's chain.  Without that pass these kernels need no private memory.
-EXTRA_FLAGS = {f: ["-mllvm", "-disable-machine-licm"] for f in ["mrl_collect.hip"] + COLLECT16}
+# In the stand-alone env kernels the lifted constants push scalar registers out instead.  Where a saved scalar register is
+# the first thing in a block, the register allocator of this compiler has been seen to put vector copies next, ahead of the
+# instruction that widens the lane mask again, so that lanes outside the mask lose the value.
+EXTRA_FLAGS = {f: ["-mllvm", "-disable-machine-licm"] for f in ["mrl_collect.hip", "mrl_env.hip", "mrl_env_many.hip"] + COLLECT16}
 
 
 def _run(cmd, verbose):

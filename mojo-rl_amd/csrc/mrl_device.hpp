@@ -4,8 +4,8 @@
 // of the same arithmetic):
 //   * every translation unit is built with -ffp-contract=off: a*b+c is two roundings
 //     unless fmaf() is written out;
-//   * fp32 sin/cos of an fp32 angle are the correctly rounded values, computed through
-//     the fp64 routine and rounded once;
+//   * fp32 sin/cos of an fp32 angle are the correctly rounded values, computed in fp64 and
+//     rounded once;
 //   * fp32 exp/log where an index or a branch depends on the last bit (action sampling, the PPO
 //     ratio and its clip test) are the correctly rounded values as well;
 //   * fp32 divide and sqrt are IEEE (hipcc default for gfx9).
@@ -17,15 +17,133 @@
 
 namespace mrl {
 
-MRL_DEV float sin32(float x) { return (float)::sin((double)x); }
-MRL_DEV float cos32(float x) { return (float)::cos((double)x); }
+// The remainder of ax, finite and above 2^20, against multiples of pi / 2, and the multiple, on the lanes with `large`
+// (Payne and Hanek's method, in integers): ax = M 2^E; the bits of 1 / (2 pi) from bit E on, times M, are the fraction of a
+// turn, to 104 bits and more.  No branch on a lane's own value: where such a branch ends, the compiler has been seen to save
+// a register that lives across it before it widens the lane mask again.
+MRL_DEV void reduce_large(float ax, bool large, double &r, int &q) {
+    const uint32_t bits = __float_as_uint(ax), M = (bits & 0x7FFFFFu) | 0x800000u;
+    const uint32_t at = (bits >> 23) - 150u + 32u, word = at >> 5, shift = at & 31u;   // (the first 32 bits: zeros for E < 0)
+    constexpr uint32_t T[9] = {0x00000000u, 0x28BE60DBu, 0x9391054Au, 0x7F09D5F4u, 0x7D4D3770u, 0x36D8A566u, 0x4F10E410u, 0x7F9458EAu, 0xF7AEF158u};
+    uint32_t t[5];
+#pragma unroll
+    for (int j = 0; j < 5; ++j) {
+        t[j] = T[j];
+#pragma unroll
+        for (int i = 1; i < 5; ++i) t[j] = word == (uint32_t)i ? T[i + j] : t[j];
+    }
+    uint32_t w[4], p[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) w[j] = (uint32_t)(((((uint64_t)t[j] << 32) | t[j + 1]) << shift) >> 32);
+    uint64_t carry = 0;
+#pragma unroll
+    for (int j = 3; j >= 0; --j) {
+        carry = (uint64_t)M * w[j] + carry;
+        p[j] = (uint32_t)carry;
+        carry >>= 32;
+    }
+    const uint32_t quarter = (p[0] + 0x20000000u) >> 30;
+    const double turn = (double)(int)(p[0] - (quarter << 30)) * 0x1p-32 + ((double)p[1] * 0x1p-64 + (double)p[2] * 0x1p-96);
+    const double rem = fma(turn, 6.283185307179586, turn * 2.4492935982947064e-16);
+    r = large ? rem : r;
+    q = large ? (int)quarter : q;
+}
+
+// Sine and cosine of an fp32 angle, rounded once from Float64.  An env step takes a dozen of them in a row on the one
+// wavefront that everything waits for, and a wavefront alone issues an instruction every six cycles whether it depends on
+// the last one or not, so what counts is the number of instructions: the argument less k pi/2 (pi/2 in two pieces; the fma's
+// product is exact), both polynomials of the remainder r, |r| <= pi/4 (interpolated at the Chebyshev points, off by less than
+// 2^-55), and the quadrant's choice among the two rounded values.  237 cycles a call where the library's pair takes 441.
+// The bits are the library's, rounded: compared on every fp32 value (one pair differs, +-2.8616508e15, whose sine is 1.3e-9 of
+// an ulp off the middle between two floats).
+struct SinCosK {
+    double two_over_pi = 0.6366197723675814, half_pi = 1.5707963267948966, half_pi_lo = 6.123233995736766e-17;
+    double s1 = -0.16666666666666666, s2 = 0.008333333333330936, s3 = -0.00019841269836740532, s4 = 2.7557316093198404e-06,
+           s5 = -2.5051129896450185e-08, s6 = 1.5917988979397435e-10;
+    double c1 = 0.041666666666666664, c2 = -0.0013888888888887389, c3 = 2.48015872987544e-05, c4 = -2.755731726587808e-07,
+           c5 = 2.087614504941318e-09, c6 = -1.138254464534925e-11;
+    // The constants in scalar registers for as long as the caller keeps the struct: without, every use moves their
+    // halves there again, 30 instructions a call.
+    static MRL_DEV SinCosK held() {
+        SinCosK k;
+        asm volatile("" : "+s"(k.two_over_pi), "+s"(k.half_pi), "+s"(k.half_pi_lo), "+s"(k.s1), "+s"(k.s2), "+s"(k.s3),
+                     "+s"(k.s4), "+s"(k.s5), "+s"(k.s6));
+        asm volatile("" : "+s"(k.c1), "+s"(k.c2), "+s"(k.c3), "+s"(k.c4), "+s"(k.c5), "+s"(k.c6));
+        return k;
+    }
+};
+// of the angle q pi / 2 + r, with x's sign
+MRL_DEV void sincos_reduced(float x, double r, int q, const SinCosK &k, float &s, float &c) {
+    const double u = r * r;
+    double ps = fma(k.s6, u, k.s5), pc = fma(k.c6, u, k.c5);
+    ps = fma(ps, u, k.s4); pc = fma(pc, u, k.c4);
+    ps = fma(ps, u, k.s3); pc = fma(pc, u, k.c3);
+    ps = fma(ps, u, k.s2); pc = fma(pc, u, k.c2);
+    ps = fma(ps, u, k.s1); pc = fma(pc, u, k.c1);
+    const float fs = (float)fma(r * u, ps, r), fc = (float)fma(fma(u, pc, -0.5), u, 1.0);
+    const uint32_t a = __float_as_uint((q & 1) ? fc : fs), b = __float_as_uint((q & 1) ? fs : fc);
+    s = __uint_as_float(a ^ ((uint32_t)(q & 2) << 30) ^ (__float_as_uint(x) & 0x80000000u));
+    c = __uint_as_float(b ^ ((uint32_t)((q + 1) & 2) << 30));
+}
+MRL_DEV void sincos32(float x, float &s, float &c, const SinCosK &k = SinCosK{}) {
+    const float ax = fabsf(x);
+    const bool far = __any(ax > 0x1p20f);   // (beyond, pi / 2 in two pieces is too short)
+    const double xd = (double)ax;
+    const double n = __builtin_rint(xd * k.two_over_pi);
+    double r = fma(-n, k.half_pi_lo, fma(-n, k.half_pi, xd));
+    int q = (int)n;
+    sincos_reduced(x, r, q, k, s, c);
+    if (__builtin_expect(far, 0)) {
+        reduce_large(ax, ax > 0x1p20f && ax < __builtin_inff(), r, q);
+        sincos_reduced(x, r, q, k, s, c);
+    }
+}
+// the same without the test, which is a third of its time, for a caller that knows |x| <= 2^20 or finds out later
+MRL_DEV void sincos32_near(float x, float &s, float &c, const SinCosK &k) {
+    const double xd = (double)fabsf(x);
+    const double n = __builtin_rint(xd * k.two_over_pi);
+    sincos_reduced(x, fma(-n, k.half_pi_lo, fma(-n, k.half_pi, xd)), (int)n, k, s, c);
+}
+MRL_DEV float sin32(float x) {
+    float s, c;
+    sincos32(x, s, c);
+    return s;
+}
+MRL_DEV float cos32(float x) {
+    float s, c;
+    sincos32(x, s, c);
+    return c;
+}
 MRL_DEV float exp32(float x) { return (float)::exp((double)x); }
-MRL_DEV float log32(float x) { return (float)::log((double)x); }
-MRL_DEV void sincos32(float x, float &s, float &c) {
-    double ds, dc;
-    ::sincos((double)x, &ds, &dc);
-    s = (float)ds;
-    c = (float)dc;
+// log of an fp32 value, rounded once from Float64: x = 2^e m, m in [sqrt(1/2), sqrt(2)), log m = 2 f + f^3 Q(f^2) with
+// f = (m - 1) / (m + 1) (Q interpolated at the Chebyshev points, off by less than 2^-57).  237 cycles a call where the
+// library's takes 424; the same bits, rounded, on every fp32 value.
+MRL_DEV float log32(float x) {
+    const double xd = (double)x;
+    double m = __builtin_amdgcn_frexp_mant(xd);
+    int e = __builtin_amdgcn_frexp_exp(xd);
+    const bool low = m < 0.7071067811865476;
+    m = low ? m + m : m;
+    e = low ? e - 1 : e;
+    const double n = m - 1.0, d = m + 1.0;
+    double y = __builtin_amdgcn_rcp(d);
+    y = fma(fma(-d, y, 1.0), y, y);
+    y = fma(fma(-d, y, 1.0), y, y);
+    double f = n * y;
+    f = fma(fma(-d, f, n), y, f);
+    const double u = f * f;
+    double q = 0.14617808833650164;
+    q = fma(q, u, 0.15331611566227585);
+    q = fma(q, u, 0.18182892438088938);
+    q = fma(q, u, 0.2222221108928466);
+    q = fma(q, u, 0.28571428626254625);
+    q = fma(q, u, 0.3999999999989889);
+    q = fma(q, u, 0.666666666666667);
+    const double ed = (double)e;
+    const double t = fma(f * u, q, ed * 2.3190468138462996e-17);   // (ln 2 in two pieces)
+    float r = (float)fma(ed, 0.6931471805599453, fma(2.0, f, t));
+    if (!(x > 0.0f && x < __builtin_inff())) r = x == 0.0f ? -__builtin_inff() : (x < 0.0f ? __builtin_nanf("") : x);
+    return r;
 }
 
 // x / d for a divisor that is divided by again and again (a joint's summed inverse inertia, a contact's
