@@ -28,9 +28,6 @@ namespace bw {
 
 constexpr int LANES_PER_ENV = 8;
 
-// a single body behind the register-form contact functions of physics2d_reg.hpp
-struct OneBody { static constexpr int NUM_BODIES = 1; };
-
 // The exchanges of a joint slot as DPP row shifts (rows are 16 lanes: two groups shift side by side; a
 // lane at a group's edge picks up a value that it never uses).
 //   from_parent: the parent of body b is the body before it, except upper leg 2 (3), whose parent is
@@ -77,7 +74,7 @@ MRL_DEV void physics_lanes(float *row, float *contacts, int n, int lane) {
     const int kidmask = b == 0 ? 3 : b == 1 ? 2 : b == 3 ? 4 : 0;
 
     const float gx = (float)0.0, gy = (float)-10.0, dt = (float)(1.0 / FPS), friction = (float)2.5, restitution = (float)0.0;
-    const float baumgarte = (float)0.2, slop = (float)0.005;
+    const float baumgarte = (float)0.2;
 
     const float *J = row + L::JOINTS_OFF + j * JOINT_SIZE;
     const float lax = J[J_AX], lay = J[J_AY], lbx = J[J_BX], lby = J[J_BY];
@@ -125,22 +122,23 @@ MRL_DEV void physics_lanes(float *row, float *contacts, int n, int lane) {
     const float p_sin = from_parent(sin_a, b), p_cos = from_parent(cos_a, b), p_ang = from_parent(ang, b);
     const float rax = lax * p_cos - lay * p_sin, ray = lax * p_sin + lay * p_cos;
     const float rbx = lbx * cos_a - lby * sin_a, rby = lbx * sin_a + lby * cos_a;
-    float inv_k11, inv_k12, inv_k22;
-    {
-        const float inv_ma = p_im, inv_ia = p_ii, inv_mb = im, inv_ib = ii;
-        const float k11 = inv_ma + inv_mb + inv_ia * ray * ray + inv_ib * rby * rby;
-        const float k12 = -inv_ia * rax * ray - inv_ib * rbx * rby;
-        const float k22 = inv_ma + inv_mb + inv_ia * rax * rax + inv_ib * rbx * rbx;
-        float det = k11 * k22 - k12 * k12;
-        if (det < 1e-10f) det = 1e-10f;
-        const float inv_det = 1.0f / det;
-        inv_k11 = k22 * inv_det; inv_k12 = -k12 * inv_det; inv_k22 = k11 * inv_det;
-    }
-    const float eff = p_ii + ii;
-    const float reff = 1.0f / eff;   // the limit and motor terms of every sweep divide by eff (div_by)
+    JointSweep q;
+    q.rax = rax; q.ray = ray; q.rbx = rbx; q.rby = rby;
+    q.ima = p_im; q.iia = p_ii; q.imb = im; q.iib = ii;
+    joint_inverse(p_im, p_ii, im, ii, rax, ray, rbx, rby, q.inv_k11, q.inv_k12, q.inv_k22);
+    q.eff = p_ii + ii;
+    q.reff = 1.0f / q.eff;
     const float angle_error = (ang - p_ang) - jref;
-    const float spring_term = -jstiff * angle_error;
-    const float rel_angle = ang - p_ang - jref;
+    q.spring_term = -jstiff * angle_error;
+    q.damp = jdamp;
+    const bool turns = q.eff > 1e-10f, limited = turns && (jflags & JF_LIMIT) != 0;
+    q.spring = turns && (jflags & JF_SPRING) != 0;
+    joint_limits(q, limited, ang - p_ang - jref, jlo, jhi);
+    q.motor = turns && (jflags & JF_MOTOR) != 0;
+    q.motor_speed = motor_speed;
+    q.max_impulse = max_torque * dt;
+    JointTerms any{false, false, false};
+    any.add(q, child);
 
     // ---- velocity iterations: my contacts in list order, then the joints slot by slot
     for (int it = 0; it < 6; ++it) {
@@ -160,61 +158,14 @@ MRL_DEV void physics_lanes(float *row, float *contacts, int n, int lane) {
         }
 #pragma unroll
         for (int s = 0; s < 3; ++s) {
-            // joints/revolute.mojo:100-320 for the joint whose child I am, when its slot is s
-            const float vxa = from_parent(vx, b), vya = from_parent(vy, b), wa = from_parent(w, b);
-            const float inv_ma = p_im, inv_ia = p_ii, inv_mb = im, inv_ib = ii;
-            const float vxb = vx, vyb = vy, wb = w;
-            const float va_anchor_x = vxa - wa * ray, va_anchor_y = vya + wa * rax;
-            const float vb_anchor_x = vxb - wb * rby, vb_anchor_y = vyb + wb * rbx;
-            const float cdot_x = vb_anchor_x - va_anchor_x, cdot_y = vb_anchor_y - va_anchor_y;
-            const float impulse_x = -(inv_k11 * cdot_x + inv_k12 * cdot_y);
-            const float impulse_y = -(inv_k12 * cdot_x + inv_k22 * cdot_y);
-            const float n_vxa = vxa - inv_ma * impulse_x, n_vya = vya - inv_ma * impulse_y;
-            const float n_vxb = vxb + inv_mb * impulse_x, n_vyb = vyb + inv_mb * impulse_y;
-            float cur_wa = wa - inv_ia * (rax * impulse_y - ray * impulse_x);
-            float cur_wb = wb + inv_ib * (rbx * impulse_y - rby * impulse_x);
-            const float e = eff;
-            if (jflags & JF_SPRING) {
-                const float rel_omega = wb - wa;
-                const float spring_torque = spring_term - jdamp * rel_omega;
-                const float angular_impulse = spring_torque * dt;
-                if (e > 1e-10f) {
-                    cur_wa = cur_wa - div_by(inv_ia * angular_impulse, e, reff);
-                    cur_wb = cur_wb + div_by(inv_ib * angular_impulse, e, reff);
-                }
-            }
-            if (jflags & JF_LIMIT) {
-                const float rel_omega = cur_wb - cur_wa;
-                if (e > 1e-10f) {
-                    float limit_impulse = 0.0f;
-                    const float stop = div_by(-rel_omega, e, reff);   // the same quotient on both sides of the test
-                    if (rel_angle <= jlo) {
-                        if (rel_omega < 0.0f) limit_impulse = stop;
-                    } else if (rel_angle >= jhi) {
-                        if (rel_omega > 0.0f) limit_impulse = stop;
-                    }
-                    if (limit_impulse != 0.0f) {
-                        cur_wa = cur_wa - inv_ia * limit_impulse;
-                        cur_wb = cur_wb + inv_ib * limit_impulse;
-                    }
-                }
-            }
-            if (jflags & JF_MOTOR) {
-                const float rel_omega = cur_wb - cur_wa;
-                const float speed_error = motor_speed - rel_omega;
-                if (e > 1e-10f) {
-                    float motor_impulse = div_by(speed_error, e, reff);
-                    const float max_impulse = max_torque * dt;
-                    if (motor_impulse > max_impulse) motor_impulse = max_impulse;
-                    if (motor_impulse < -max_impulse) motor_impulse = -max_impulse;
-                    cur_wa = cur_wa - inv_ia * motor_impulse;
-                    cur_wb = cur_wb + inv_ib * motor_impulse;
-                }
-            }
+            // the joint whose child I am, when its slot is s (in any other slot its result is not used)
+            float vxa = from_parent(vx, b), vya = from_parent(vy, b), wa = from_parent(w, b);
+            float vxb = vx, vyb = vy, wb = w;
+            joint_velocity(q, any, dt, vxa, vya, wa, vxb, vyb, wb);
             // the parent takes its new velocity from the child of this slot, the child keeps its own
-            const float g_vx = from_kid(s, n_vxa, b), g_vy = from_kid(s, n_vya, b), g_w = from_kid(s, cur_wa, b);
+            const float g_vx = from_kid(s, vxa, b), g_vy = from_kid(s, vya, b), g_w = from_kid(s, wa, b);
             if ((kidmask >> s) & 1) { vx = g_vx; vy = g_vy; w = g_w; }
-            if (myslot == s) { vx = n_vxb; vy = n_vyb; w = cur_wb; }
+            if (myslot == s) { vx = vxb; vy = vyb; w = wb; }
         }
     }
     // ---- integrate positions (integrators/euler.mojo:132-183)
@@ -238,66 +189,40 @@ MRL_DEV void physics_lanes(float *row, float *contacts, int n, int lane) {
     sincos32(ang, sin_a, cos_a);
     // ---- position iterations: my contacts (solvers/impulse.mojo:333-402), then the joints
     // (joints/revolute.mojo:323-495) slot by slot
+    bool stale = false;   // my body has turned since its sine and cosine were taken
     for (int it = 0; it < 2; ++it) {
         for (unsigned m = mine; m; m &= m - 1) {
             const int c = __ffs((int)m) - 1;
             const float *C = contacts + c * CONTACT_SIZE;
             B1.x[0] = x; B1.y[0] = y;
-            contact_position<OneBody>(B1, 0, C[C_NX], C[C_NY], C[C_DEPTH], baumgarte, slop);
+            contact_position<OneBody>(B1, 0, C[C_NX], C[C_NY], C[C_DEPTH], baumgarte);
             x = B1.x[0]; y = B1.y[0];
         }
 #pragma unroll
         for (int s = 0; s < 3; ++s) {
-            const float xa = from_parent(x, b), ya = from_parent(y, b), angle_a = from_parent(ang, b);
-            const float inv_ma = p_im, inv_ia = p_ii, inv_mb = im, inv_ib = ii;
-            const float xb = x, yb = y, angle_b = ang;
+            float xa = from_parent(x, b), ya = from_parent(y, b), angle_a = from_parent(ang, b);
             const float s_a = from_parent(sin_a, b), c_a = from_parent(cos_a, b);
-            const float s_b = sin_a, c_b = cos_a;
+            float xb = x, yb = y, angle_b = ang;
             const float r_ax = lax * c_a - lay * s_a, r_ay = lax * s_a + lay * c_a;
-            const float r_bx = lbx * c_b - lby * s_b, r_by = lbx * s_b + lby * c_b;
-            const float anchor_ax = xa + r_ax, anchor_ay = ya + r_ay;
-            const float anchor_bx = xb + r_bx, anchor_by = yb + r_by;
-            const float cx = anchor_bx - anchor_ax, cy = anchor_by - anchor_ay;
-            const float error = sqrtf(cx * cx + cy * cy);
-            float n_xa = xa, n_ya = ya, n_aa = angle_a, n_xb = xb, n_yb = yb, n_ab = angle_b;
-            if (!(error < slop)) {
-                const float k11 = inv_ma + inv_mb + inv_ia * r_ay * r_ay + inv_ib * r_by * r_by;
-                const float k12 = -inv_ia * r_ax * r_ay - inv_ib * r_bx * r_by;
-                const float k22 = inv_ma + inv_mb + inv_ia * r_ax * r_ax + inv_ib * r_bx * r_bx;
-                float det = k11 * k22 - k12 * k12;
-                if (det < 1e-10f) det = 1e-10f;
-                const float inv_det = 1.0f / det;
-                const float ik11 = k22 * inv_det, ik12 = -k12 * inv_det, ik22 = k11 * inv_det;
-                const float correction_x = -baumgarte * (ik11 * cx + ik12 * cy);
-                const float correction_y = -baumgarte * (ik12 * cx + ik22 * cy);
-                n_xa = xa - inv_ma * correction_x;
-                n_ya = ya - inv_ma * correction_y;
-                n_xb = xb + inv_mb * correction_x;
-                n_yb = yb + inv_mb * correction_y;
-                float cur_a = angle_a - inv_ia * (r_ax * correction_y - r_ay * correction_x);
-                float cur_b = angle_b + inv_ib * (r_bx * correction_y - r_by * correction_x);
-                if (jflags & JF_LIMIT) {
-                    const float relative_angle = cur_b - cur_a - jref;
-                    const float e = inv_ia + inv_ib;
-                    if (e > 1e-10f) {
-                        float angle_correction = 0.0f;
-                        if (relative_angle < jlo) angle_correction = baumgarte * (jlo - relative_angle);
-                        else if (relative_angle > jhi) angle_correction = baumgarte * (jhi - relative_angle);
-                        if (angle_correction != 0.0f) {
-                            cur_a = cur_a - div_by(inv_ia * angle_correction, e, reff);
-                            cur_b = cur_b + div_by(inv_ib * angle_correction, e, reff);
-                        }
-                    }
-                }
-                n_aa = cur_a;
-                n_ab = cur_b;
+            const float r_bx = lbx * cos_a - lby * sin_a, r_by = lbx * sin_a + lby * cos_a;
+            bool moved = false;
+            if (myslot == s)
+                moved = joint_position(p_im, p_ii, im, ii, q.eff, q.reff, r_ax, r_ay, r_bx, r_by, limited, jlo, jhi, jref, baumgarte,
+                                       xa, ya, angle_a, xb, yb, angle_b);
+            const bool any_moved = __any(moved);   // (a joint within the slop hands back what it was given)
+            if (any_moved) {
+                const float g_x = from_kid(s, xa, b), g_y = from_kid(s, ya, b), g_a = from_kid(s, angle_a, b);
+                if ((kidmask >> s) & 1) { x = g_x; y = g_y; ang = g_a; }
+                if (myslot == s) { x = xb; y = yb; ang = angle_b; }
             }
-            const float g_x = from_kid(s, n_xa, b), g_y = from_kid(s, n_ya, b), g_a = from_kid(s, n_aa, b);
-            if ((kidmask >> s) & 1) { x = g_x; y = g_y; ang = g_a; }
-            if (myslot == s) { x = n_xb; y = n_yb; ang = n_ab; }
             // (the last slot moves leg 2's segments only: the second iteration reads them in its last two slots,
             // behind another of these, and nothing reads them after the second iteration)
-            if (s != 2) sincos32(ang, sin_a, cos_a);
+            if (s == 2) {
+                stale = any_moved;
+            } else if (any_moved || stale) {
+                sincos32(ang, sin_a, cos_a);
+                stale = false;
+            }
         }
     }
     // ---- bodies and cleared forces back into the row

@@ -129,7 +129,7 @@ MRL_DEV void step_lanes(float *row, const float *shapes, const float *action, in
     const int kidmask = b == 0 ? 3 : b == 1 ? 2 : (b == 2 || b == 4) ? 4 : b == 5 ? 8 : 0;
 
     const float gx = (float)0.0, gy = (float)-9.81, dt = (float)0.01, friction = (float)0.9, restitution = (float)0.0;
-    const float baumgarte = (float)0.2, slop = (float)0.005;
+    const float baumgarte = (float)0.2;
 
     // ---- the action into the joint motors (child lane of joint j), as hc::step_row does
     float *J = row + L::JOINTS_OFF + j * JOINT_SIZE;
@@ -160,8 +160,16 @@ MRL_DEV void step_lanes(float *row, const float *shapes, const float *action, in
 #pragma unroll
     for (int v = 0; v < 4; ++v) { lvx[v] = S[2 + v * 2]; lvy[v] = S[3 + v * 2]; }
     const float p_im = from_parent(im, b), p_ii = from_parent(ii, b);
-    const float eff = p_ii + ii;
-    const float reff = 1.0f / eff;   // the limit and motor terms of every sweep divide by eff (div_by)
+    JointSweep q;   // the joint whose child I am
+    q.ima = p_im; q.iia = p_ii; q.imb = im; q.iib = ii;
+    q.eff = p_ii + ii;
+    q.reff = 1.0f / q.eff;
+    const bool turns = q.eff > 1e-10f, limited = turns && (jflags & JF_LIMIT) != 0;
+    q.spring = turns && (jflags & JF_SPRING) != 0;
+    q.motor = turns && (jflags & JF_MOTOR) != 0;
+    q.damp = jdamp;
+    q.motor_speed = motor_speed;
+    q.max_impulse = max_torque * dt;
     const double x_before = (double)x;   // meaningful on lane 0 (the torso)
 
     // sine and cosine of my body's angle, kept in step with it (recomputed whenever the angle may have
@@ -189,8 +197,8 @@ MRL_DEV void step_lanes(float *row, const float *shapes, const float *action, in
             const bool hit = body && v < n_verts && penetration > 0.0f;
             // compacted in vertex order
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                if (hit && found == q) { cpx[q] = world_x; cpy[q] = world_y; cdepth[q] = penetration; }
+            for (int c = 0; c < 4; ++c) {
+                if (hit && found == c) { cpx[c] = world_x; cpy[c] = world_y; cdepth[c] = penetration; }
             }
             found += hit ? 1 : 0;
         }
@@ -206,153 +214,52 @@ MRL_DEV void step_lanes(float *row, const float *shapes, const float *action, in
         // (solvers/impulse.mojo:115-190) ...
         const float nx = 0.0f, ny = 1.0f;
         ContactFixed cf[4];
-        float jn[4], jt[4];
+        float jn[4], jt[4], push_out[4];
+        RegBodies<OneBody> B1;
+        B1.x[0] = x; B1.y[0] = y; B1.im[0] = im; B1.ii[0] = ii;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            jn[q] = jt[q] = 0.0f;
-            ContactFixed f;
-            f.nx = nx; f.ny = ny;
-            f.inv_mass_a = im; f.inv_inertia_a = ii;
-            const float inv_mass_b = 0.0f, inv_inertia_b = 0.0f;
-            f.ra_x = cpx[q] - x; f.ra_y = cpy[q] - y;
-            const float rb_x = cpx[q] - cpx[q], rb_y = cpy[q] - cpy[q];
-            const float ra_cross_n = f.ra_x * ny - f.ra_y * nx;
-            const float rb_cross_n = rb_x * ny - rb_y * nx;
-            float k = f.inv_mass_a + inv_mass_b;
-            k = k + f.inv_inertia_a * ra_cross_n * ra_cross_n;
-            k = k + inv_inertia_b * rb_cross_n * rb_cross_n;
-            f.k = k;
-            const float tangent_x = -ny, tangent_y = nx;
-            const float ra_cross_t = f.ra_x * tangent_y - f.ra_y * tangent_x;
-            const float rb_cross_t = rb_x * tangent_y - rb_y * tangent_x;
-            float k_t = f.inv_mass_a + inv_mass_b;
-            k_t = k_t + f.inv_inertia_a * ra_cross_t * ra_cross_t;
-            k_t = k_t + inv_inertia_b * rb_cross_t * rb_cross_t;
-            f.k_t = k_t;
-            f.rk = 1.0f / k;
-            f.rk_t = 1.0f / k_t;
-            cf[q] = f;
+        for (int c = 0; c < 4; ++c) {
+            jn[c] = jt[c] = push_out[c] = 0.0f;
+            cf[c] = ContactFixed{0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 1.0f, 1.0f, 1.0f, 1.0f};
+            if (!__any(c < kept)) continue;
+            cf[c] = contact_prepare<OneBody>(B1, 0, cpx[c], cpy[c], nx, ny);
+            // what each position sweep moves the body up by (solvers/impulse.mojo:333-402): the depth stays as detected
+            const float total = im + 0.0f;
+            const float correction = cdepth[c] - SOLVER_SLOP;
+            if (c < kept && correction > 0.0f && total != 0.0f) push_out[c] = baumgarte * correction * im / total;
         }
         // ... and the joint's lever arms, K^-1 and limit angle (joints/revolute.mojo:90-200), by the child
         const float p_sin = from_parent(sin_a, b), p_cos = from_parent(cos_a, b);
         const float p_ang = from_parent(ang, b);
         const float rax = lax * p_cos - lay * p_sin, ray = lax * p_sin + lay * p_cos;
         const float rbx = lbx * cos_a - lby * sin_a, rby = lbx * sin_a + lby * cos_a;
-        float inv_k11, inv_k12, inv_k22;
-        {
-            const float inv_ma = p_im, inv_ia = p_ii, inv_mb = im, inv_ib = ii;
-            const float k11 = inv_ma + inv_mb + inv_ia * ray * ray + inv_ib * rby * rby;
-            const float k12 = -inv_ia * rax * ray - inv_ib * rbx * rby;
-            const float k22 = inv_ma + inv_mb + inv_ia * rax * rax + inv_ib * rbx * rbx;
-            float det = k11 * k22 - k12 * k12;
-            if (det < 1e-10f) det = 1e-10f;
-            const float inv_det = 1.0f / det;
-            inv_k11 = k22 * inv_det; inv_k12 = -k12 * inv_det; inv_k22 = k11 * inv_det;
-        }
+        q.rax = rax; q.ray = ray; q.rbx = rbx; q.rby = rby;
+        joint_inverse(p_im, p_ii, im, ii, rax, ray, rbx, rby, q.inv_k11, q.inv_k12, q.inv_k22);
         const float angle_error = (ang - p_ang) - jref;
-        const float spring_term = -jstiff * angle_error;
-        const float rel_angle = ang - p_ang - jref;
+        q.spring_term = -jstiff * angle_error;
+        joint_limits(q, limited, ang - p_ang - jref, jlo, jhi);
+        JointTerms any{false, false, false};
+        any.add(q, child);
 
         // ---- velocity iterations: my contacts, then the joints slot by slot
         for (int it = 0; it < 4; ++it) {
+            B1.vx[0] = vx; B1.vy[0] = vy; B1.w[0] = w;
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                if (q >= kept) break;
-                // one contact of solvers/impulse.mojo:192-331 on my body
-                const ContactFixed &f = cf[q];
-                float vel_a_x = vx, vel_a_y = vy, omega_a = w;
-                const float vel_b_x = 0.0f, vel_b_y = 0.0f, omega_b = 0.0f, rb_x = 0.0f, rb_y = 0.0f;
-                float vel_at_a_x = vel_a_x - omega_a * f.ra_y, vel_at_a_y = vel_a_y + omega_a * f.ra_x;
-                float vel_at_b_x = vel_b_x - omega_b * rb_y, vel_at_b_y = vel_b_y + omega_b * rb_x;
-                float rel_vel_x = vel_at_a_x - vel_at_b_x, rel_vel_y = vel_at_a_y - vel_at_b_y;
-                const float vel_normal = rel_vel_x * f.nx + rel_vel_y * f.ny;
-                if (!(vel_normal < 0.0f)) continue;
-                float j_normal = div_by(-(1.0f + restitution) * vel_normal, f.k, f.rk);
-                const float old_impulse = jn[q];
-                float new_impulse = old_impulse + j_normal;
-                if (new_impulse < 0.0f) new_impulse = 0.0f;
-                jn[q] = new_impulse;
-                j_normal = new_impulse - old_impulse;
-                const float impulse_x = j_normal * f.nx, impulse_y = j_normal * f.ny;
-                vel_a_x = vel_a_x + impulse_x * f.inv_mass_a;
-                vel_a_y = vel_a_y + impulse_y * f.inv_mass_a;
-                omega_a = omega_a + (f.ra_x * impulse_y - f.ra_y * impulse_x) * f.inv_inertia_a;
-                vel_at_a_x = vel_a_x - omega_a * f.ra_y; vel_at_a_y = vel_a_y + omega_a * f.ra_x;
-                vel_at_b_x = vel_b_x - omega_b * rb_y; vel_at_b_y = vel_b_y + omega_b * rb_x;
-                rel_vel_x = vel_at_a_x - vel_at_b_x; rel_vel_y = vel_at_a_y - vel_at_b_y;
-                const float tangent_x = -f.ny, tangent_y = f.nx;
-                const float vel_tangent = rel_vel_x * tangent_x + rel_vel_y * tangent_y;
-                float j_tangent = div_by(-vel_tangent, f.k_t, f.rk_t);
-                const float max_friction = friction * new_impulse;
-                const float old_tangent = jt[q];
-                float new_tangent = old_tangent + j_tangent;
-                if (new_tangent > max_friction) new_tangent = max_friction;
-                else if (new_tangent < -max_friction) new_tangent = -max_friction;
-                jt[q] = new_tangent;
-                j_tangent = new_tangent - old_tangent;
-                const float friction_x = j_tangent * tangent_x, friction_y = j_tangent * tangent_y;
-                vx = vel_a_x + friction_x * f.inv_mass_a;
-                vy = vel_a_y + friction_y * f.inv_mass_a;
-                w = omega_a + (f.ra_x * friction_y - f.ra_y * friction_x) * f.inv_inertia_a;
+            for (int c = 0; c < 4; ++c) {   // solvers/impulse.mojo:192-331
+                if (!__any(c < kept)) break;
+                contact_velocity<OneBody>(B1, 0, cf[c], jn[c], jt[c], friction, restitution, c < kept);
             }
+            vx = B1.vx[0]; vy = B1.vy[0]; w = B1.w[0];
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
-                // joints/revolute.mojo:100-320 for the joint whose child I am, when its slot is s
-                const float vxa = from_parent(vx, b), vya = from_parent(vy, b), wa = from_parent(w, b);
-                const float inv_ma = p_im, inv_ia = p_ii, inv_mb = im, inv_ib = ii;
-                const float vxb = vx, vyb = vy, wb = w;
-                const float va_anchor_x = vxa - wa * ray, va_anchor_y = vya + wa * rax;
-                const float vb_anchor_x = vxb - wb * rby, vb_anchor_y = vyb + wb * rbx;
-                const float cdot_x = vb_anchor_x - va_anchor_x, cdot_y = vb_anchor_y - va_anchor_y;
-                const float impulse_x = -(inv_k11 * cdot_x + inv_k12 * cdot_y);
-                const float impulse_y = -(inv_k12 * cdot_x + inv_k22 * cdot_y);
-                const float n_vxa = vxa - inv_ma * impulse_x, n_vya = vya - inv_ma * impulse_y;
-                const float n_vxb = vxb + inv_mb * impulse_x, n_vyb = vyb + inv_mb * impulse_y;
-                float cur_wa = wa - inv_ia * (rax * impulse_y - ray * impulse_x);
-                float cur_wb = wb + inv_ib * (rbx * impulse_y - rby * impulse_x);
-                const float e = eff;
-                if (jflags & JF_SPRING) {
-                    const float rel_omega = wb - wa;
-                    const float spring_torque = spring_term - jdamp * rel_omega;
-                    const float angular_impulse = spring_torque * dt;
-                    if (e > 1e-10f) {
-                        cur_wa = cur_wa - div_by(inv_ia * angular_impulse, e, reff);
-                        cur_wb = cur_wb + div_by(inv_ib * angular_impulse, e, reff);
-                    }
-                }
-                if (jflags & JF_LIMIT) {
-                    const float rel_omega = cur_wb - cur_wa;
-                    if (e > 1e-10f) {
-                        float limit_impulse = 0.0f;
-                        const float stop = div_by(-rel_omega, e, reff);   // the same quotient on both sides of the test
-                        if (rel_angle <= jlo) {
-                            if (rel_omega < 0.0f) limit_impulse = stop;
-                        } else if (rel_angle >= jhi) {
-                            if (rel_omega > 0.0f) limit_impulse = stop;
-                        }
-                        if (limit_impulse != 0.0f) {
-                            cur_wa = cur_wa - inv_ia * limit_impulse;
-                            cur_wb = cur_wb + inv_ib * limit_impulse;
-                        }
-                    }
-                }
-                if (jflags & JF_MOTOR) {
-                    const float rel_omega = cur_wb - cur_wa;
-                    const float speed_error = motor_speed - rel_omega;
-                    if (e > 1e-10f) {
-                        float motor_impulse = div_by(speed_error, e, reff);
-                        const float max_impulse = max_torque * dt;
-                        if (motor_impulse > max_impulse) motor_impulse = max_impulse;
-                        if (motor_impulse < -max_impulse) motor_impulse = -max_impulse;
-                        cur_wa = cur_wa - inv_ia * motor_impulse;
-                        cur_wb = cur_wb + inv_ib * motor_impulse;
-                    }
-                }
+                // the joint whose child I am, when its slot is s (in any other slot its result is not used)
+                float vxa = from_parent(vx, b), vya = from_parent(vy, b), wa = from_parent(w, b);
+                float vxb = vx, vyb = vy, wb = w;
+                joint_velocity(q, any, dt, vxa, vya, wa, vxb, vyb, wb);
                 // the parent takes its new velocity from the child of this slot, the child keeps its own
-                const float g_vx = from_kid_slot(s, n_vxa, b), g_vy = from_kid_slot(s, n_vya, b);
-                const float g_w = from_kid_slot(s, cur_wa, b);
+                const float g_vx = from_kid_slot(s, vxa, b), g_vy = from_kid_slot(s, vya, b), g_w = from_kid_slot(s, wa, b);
                 if ((kidmask >> s) & 1) { vx = g_vx; vy = g_vy; w = g_w; }
-                if (myslot == s) { vx = n_vxb; vy = n_vyb; w = cur_wb; }
+                if (myslot == s) { vx = vxb; vy = vyb; w = wb; }
             }
         }
         // ---- integrate positions (integrators/euler.mojo:132-183)
@@ -376,73 +283,42 @@ MRL_DEV void step_lanes(float *row, const float *shapes, const float *action, in
         sincos32(ang, sin_a, cos_a);
         // ---- position iterations: my contacts (solvers/impulse.mojo:333-402), then the joints
         // (joints/revolute.mojo:323-495) slot by slot
+        bool stale = false;   // my body has turned since its sine and cosine were taken
         for (int it = 0; it < 2; ++it) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                if (q >= kept) break;
-                float correction = cdepth[q] - slop;
-                if (correction <= 0.0f) continue;
-                correction = baumgarte * correction;
-                const float inv_mass_a = im, inv_mass_b = 0.0f;
-                const float total = inv_mass_a + inv_mass_b;
-                if (total == 0.0f) continue;
-                const float correction_a = correction * inv_mass_a / total;
-                x = x + nx * correction_a;
-                y = y + ny * correction_a;
+            for (int c = 0; c < 4; ++c) {
+                if (!__any(c < kept)) break;
+                if (push_out[c] > 0.0f) {
+                    x = x + nx * push_out[c];
+                    y = y + ny * push_out[c];
+                }
             }
 #pragma unroll
             for (int s = 0; s < 4; ++s) {
-                const float xa = from_parent(x, b), ya = from_parent(y, b), angle_a = from_parent(ang, b);
-                const float inv_ma = p_im, inv_ia = p_ii, inv_mb = im, inv_ib = ii;
-                const float xb = x, yb = y, angle_b = ang;
+                float xa = from_parent(x, b), ya = from_parent(y, b), angle_a = from_parent(ang, b);
                 const float s_a = from_parent(sin_a, b), c_a = from_parent(cos_a, b);
-                const float s_b = sin_a, c_b = cos_a;
+                float xb = x, yb = y, angle_b = ang;
                 const float r_ax = lax * c_a - lay * s_a, r_ay = lax * s_a + lay * c_a;
-                const float r_bx = lbx * c_b - lby * s_b, r_by = lbx * s_b + lby * c_b;
-                const float anchor_ax = xa + r_ax, anchor_ay = ya + r_ay;
-                const float anchor_bx = xb + r_bx, anchor_by = yb + r_by;
-                const float cx = anchor_bx - anchor_ax, cy = anchor_by - anchor_ay;
-                const float error = sqrtf(cx * cx + cy * cy);
-                float n_xa = xa, n_ya = ya, n_aa = angle_a, n_xb = xb, n_yb = yb, n_ab = angle_b;
-                if (!(error < slop)) {
-                    const float k11 = inv_ma + inv_mb + inv_ia * r_ay * r_ay + inv_ib * r_by * r_by;
-                    const float k12 = -inv_ia * r_ax * r_ay - inv_ib * r_bx * r_by;
-                    const float k22 = inv_ma + inv_mb + inv_ia * r_ax * r_ax + inv_ib * r_bx * r_bx;
-                    float det = k11 * k22 - k12 * k12;
-                    if (det < 1e-10f) det = 1e-10f;
-                    const float inv_det = 1.0f / det;
-                    const float ik11 = k22 * inv_det, ik12 = -k12 * inv_det, ik22 = k11 * inv_det;
-                    const float correction_x = -baumgarte * (ik11 * cx + ik12 * cy);
-                    const float correction_y = -baumgarte * (ik12 * cx + ik22 * cy);
-                    n_xa = xa - inv_ma * correction_x;
-                    n_ya = ya - inv_ma * correction_y;
-                    n_xb = xb + inv_mb * correction_x;
-                    n_yb = yb + inv_mb * correction_y;
-                    float cur_a = angle_a - inv_ia * (r_ax * correction_y - r_ay * correction_x);
-                    float cur_b = angle_b + inv_ib * (r_bx * correction_y - r_by * correction_x);
-                    if (jflags & JF_LIMIT) {
-                        const float relative_angle = cur_b - cur_a - jref;
-                        const float e = inv_ia + inv_ib;
-                        if (e > 1e-10f) {
-                            float angle_correction = 0.0f;
-                            if (relative_angle < jlo) angle_correction = baumgarte * (jlo - relative_angle);
-                            else if (relative_angle > jhi) angle_correction = baumgarte * (jhi - relative_angle);
-                            if (angle_correction != 0.0f) {
-                                cur_a = cur_a - div_by(inv_ia * angle_correction, e, reff);
-                                cur_b = cur_b + div_by(inv_ib * angle_correction, e, reff);
-                            }
-                        }
-                    }
-                    n_aa = cur_a;
-                    n_ab = cur_b;
+                const float r_bx = lbx * cos_a - lby * sin_a, r_by = lbx * sin_a + lby * cos_a;
+                bool moved = false;
+                if (myslot == s)
+                    moved = joint_position(p_im, p_ii, im, ii, q.eff, q.reff, r_ax, r_ay, r_bx, r_by, limited, jlo, jhi, jref, baumgarte,
+                                           xa, ya, angle_a, xb, yb, angle_b);
+                const bool any_moved = __any(moved);   // (a joint within the slop hands back what it was given)
+                if (any_moved) {
+                    const float g_x = from_kid_slot(s, xa, b), g_y = from_kid_slot(s, ya, b);
+                    const float g_a = from_kid_slot(s, angle_a, b);
+                    if ((kidmask >> s) & 1) { x = g_x; y = g_y; ang = g_a; }
+                    if (myslot == s) { x = xb; y = yb; ang = angle_b; }
                 }
-                const float g_x = from_kid_slot(s, n_xa, b), g_y = from_kid_slot(s, n_ya, b);
-                const float g_a = from_kid_slot(s, n_aa, b);
-                if ((kidmask >> s) & 1) { x = g_x; y = g_y; ang = g_a; }
-                if (myslot == s) { x = n_xb; y = n_yb; ang = n_ab; }
                 // (the last slot moves the front shin and foot only, which the second iteration reads in its
                 // last two slots, behind two more of these; after the second iteration the next sub-step reads all)
-                if (!(it == 0 && s == 3)) sincos32(ang, sin_a, cos_a);
+                if (it == 0 && s == 3) {
+                    stale = any_moved;
+                } else if (any_moved || stale) {
+                    sincos32(ang, sin_a, cos_a);
+                    stale = false;
+                }
             }
         }
     }

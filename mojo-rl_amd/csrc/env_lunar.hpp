@@ -370,9 +370,9 @@ MRL_DEV void step_finish(float *row, float *contacts, int n_given, const float *
     int step_count = c.step_count;
     const float gx = (float)0.0, gy = (float)-10.0, dt = (float)DT;
     const float friction = (float)0.1, restitution = (float)0.0;
-    const float baumgarte = (float)0.2, slop = (float)0.005;
+    const float baumgarte = (float)0.2;
     const int n = reg_physics_substep<L, Topology, false, true>(row, shapes, contacts, gx, gy, dt, friction,
-                                                                restitution, baumgarte, slop, 6, 2, n_given);
+                                                                restitution, baumgarte, 6, 2, n_given);
 
     step_count += 1;
     float obs[8];

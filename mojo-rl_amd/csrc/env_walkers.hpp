@@ -408,7 +408,7 @@ template <bool LIDAR = true>
 MRL_DEV void step_finish(float *row, float *contacts, int n_given, const float *shapes, const float *act,
                          float &reward, float &done) {
     int n = reg_physics_substep<L, Topology, false, false>(row, shapes, contacts, (float)0.0, (float)-10.0, (float)(1.0 / FPS),
-                                      (float)2.5, (float)0.0, (float)0.2, (float)0.005, 6, 2, n_given);
+                                      (float)2.5, (float)0.0, (float)0.2, 6, 2, n_given);
     step_tail<LIDAR>(row, contacts, n, act, reward, done, row + L::META_OFF);
 }
 
@@ -566,7 +566,7 @@ MRL_DEV void step_row(float *row, float *contacts, const float *shapes, int env,
     int n = 0;
     for (int s = 0; s < 5; ++s)
         n = reg_physics_substep<L, Topology, true, false>(row, shapes, contacts, (float)0.0, (float)-9.81, (float)0.01, (float)0.9,
-                                     (float)0.0, (float)0.2, (float)0.005, 4, 2);
+                                     (float)0.0, (float)0.2, 4, 2);
     const double x_after = B[IDX_X], torso_z = B[IDX_Y];
     const double forward_velocity = (x_after - x_before) / (0.01 * (double)5);
     const double forward_reward = 1.0 * forward_velocity;
