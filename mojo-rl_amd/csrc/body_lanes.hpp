@@ -104,21 +104,21 @@ struct LaneContact {
     ContactFixed f;
     float jn, jt;
     float push_x, push_y;   // what a position sweep moves the body by (solvers/impulse.mojo:333-402; the depth stays as detected)
-    bool push;
+    float push;             // 1: it does (a flag in a vector register: lane masks are short)
 
     MRL_DEV void prepare(const LaneBody &B, bool live, float px, float py, float nx, float ny, float depth, float baumgarte) {
         f = contact_prepare<OneBody>(B, 0, px, py, nx, ny);
         jn = jt = 0.0f;
         const float correction = depth - SOLVER_SLOP, total = B.im[0] + 0.0f;
-        push = live && !(correction <= 0.0f) && total != 0.0f;
+        push = live && !(correction <= 0.0f) && total != 0.0f ? 1.0f : 0.0f;
         const float by = baumgarte * correction * B.im[0] / total;
         push_x = nx * by;
         push_y = ny * by;
     }
     MRL_DEV void position(LaneBody &B) const {
         const float x = B.x[0] + push_x, y = B.y[0] + push_y;
-        B.x[0] = push ? x : B.x[0];
-        B.y[0] = push ? y : B.y[0];
+        B.x[0] = push != 0.0f ? x : B.x[0];
+        B.y[0] = push != 0.0f ? y : B.y[0];
     }
 };
 
@@ -150,13 +150,13 @@ struct LaneListContacts {
         rest = mine;
 #pragma unroll
         for (int r = 0; r < REG; ++r) {
-            if (!__any(r < count)) break;
+            if (!any_lane(r < count)) break;
             const int i = r < count ? __ffs((int)rest) - 1 : 0;
             rest &= rest - 1u;
             const float *C = cts + i * CONTACT_SIZE;
             c[r].prepare(B, r < count, C[C_PX], C[C_PY], C[C_NX], C[C_NY], C[C_DEPTH], baumgarte);
         }
-        if (!__any(rest != 0)) return;
+        if (!any_lane(rest != 0)) return;
         for (unsigned m = rest; m; m &= m - 1) {
             const int i = __ffs((int)m) - 1;
             float *C = cts + i * CONTACT_SIZE, *K = masses(i);
@@ -168,10 +168,10 @@ struct LaneListContacts {
     MRL_DEV void velocity(LaneBody &B, float friction, float restitution) {
 #pragma unroll
         for (int r = 0; r < REG; ++r) {
-            if (!__any(r < count)) return;
+            if (!any_lane(r < count)) return;
             contact_velocity<OneBody>(B, 0, c[r].f, c[r].jn, c[r].jt, friction, restitution, r < count);
         }
-        if (!__any(rest != 0)) return;
+        if (!any_lane(rest != 0)) return;
         for (unsigned m = rest; m; m &= m - 1) {
             const int i = __ffs((int)m) - 1;
             float *C = cts + i * CONTACT_SIZE;
@@ -188,13 +188,10 @@ struct LaneListContacts {
     MRL_DEV void position(LaneBody &B, float baumgarte) const {
 #pragma unroll
         for (int r = 0; r < REG; ++r) {
-            if (!__any(r < count)) return;
-            const bool push = r < count && c[r].push;
-            const float x = B.x[0] + c[r].push_x, y = B.y[0] + c[r].push_y;
-            B.x[0] = push ? x : B.x[0];
-            B.y[0] = push ? y : B.y[0];
+            if (!any_lane(r < count)) return;
+            c[r].position(B);
         }
-        if (!__any(rest != 0)) return;
+        if (!any_lane(rest != 0)) return;
         for (unsigned m = rest; m; m &= m - 1) {
             const int i = __ffs((int)m) - 1;
             const float *C = cts + i * CONTACT_SIZE;
@@ -335,17 +332,18 @@ struct LaneJoints {
         if constexpr (S > 3) velocity_slot<3>(B, dt);
     }
 
-    // slot SL of a position sweep (joints/revolute.mojo:323-495); false when no joint of the wavefront's is off by more
-    // than the slop, that is when nothing moved
+    // slot SL of a position sweep (joints/revolute.mojo:323-495); the lanes that moved: zero when no joint of the
+    // wavefront's is off by more than the slop
     template <int SL>
-    MRL_DEV bool position_slot(LaneBody &B, float sn, float cs, float baumgarte) const {
+    MRL_DEV uint64_t position_slot(LaneBody &B, float sn, float cs, float baumgarte) const {
         constexpr int e = SL & 1, ctrl = R::CTRL[SL];
         const float im = B.im[0], ii = B.ii[0];
         const float qx = ax[e] * cs - ay[e] * sn, qy = ax[e] * sn + ay[e] * cs;
         const float px = B.x[0] + qx, py = B.y[0] + qy;
         const float dx = px - dpp_xchg<ctrl>(px), dy = py - dpp_xchg<ctrl>(py);
         const bool off = in[SL] && !(dx * dx + dy * dy < SOLVER_SLOP_SQ);
-        if (!__any(off)) return false;
+        const uint64_t moved = __builtin_amdgcn_ballot_w64(off);
+        if (moved == 0) return 0;
         // K^-1 and the correction by the child
         float i11, i12, i22;
         joint_inverse(p_im, p_ii, im, ii, dpp_xchg<ctrl>(qx), dpp_xchg<ctrl>(qy), qx, qy, i11, i12, i22);
@@ -364,7 +362,7 @@ struct LaneJoints {
         B.x[0] = off ? x : B.x[0];
         B.y[0] = off ? y : B.y[0];
         B.ang[0] = off ? a : B.ang[0];
-        return true;
+        return moved;
     }
 
     // The position sweeps from (B, sn, cs), which keep in step but for the last slot's turn where nothing reads it.
@@ -373,7 +371,7 @@ struct LaneJoints {
     MRL_DEV bool position_sweeps(LaneBody &B, float &sn, float &cs, const Contacts &contacts, float baumgarte,
                                  const SinCosK &K) const {
         float widest = 0.0f;
-        bool stale = false;   // a body has turned since its sine and cosine were taken
+        uint64_t stale = 0;   // not zero: a body has turned since its sine and cosine were taken
         auto turn = [&]() {
             if (NEAR) sincos32_near(B.ang[0], sn, cs, K);
             else sincos32(B.ang[0], sn, cs, K);
@@ -384,22 +382,22 @@ struct LaneJoints {
             contacts.position(B, baumgarte);
             auto slot = [&](auto sl) {
                 constexpr int SL = decltype(sl)::value;
-                const bool moved = position_slot<SL>(B, sn, cs, baumgarte);
+                const uint64_t moved = position_slot<SL>(B, sn, cs, baumgarte);
                 if (SL == S - 1 && !R::LAST_TURNS_FIRST) {
                     // (the bodies of the last slot are next read behind another turn, if at all)
                     if (it + 1 < ITERS || !R::ANGLES_AFTER) { stale = stale | moved; return; }
                 } else if (SL == S - 1 && it + 1 == ITERS && !R::ANGLES_AFTER) {
                     return;
                 }
-                if (moved | stale) turn();
-                stale = false;
+                if ((moved | stale) != 0) turn();
+                stale = 0;
             };
             slot(std::integral_constant<int, 0>{});
             slot(std::integral_constant<int, 1>{});
             if constexpr (S > 2) slot(std::integral_constant<int, 2>{});
             if constexpr (S > 3) slot(std::integral_constant<int, 3>{});
         }
-        return !NEAR || !__any(widest > 0x1p20f);
+        return !NEAR || !any_lane(widest > 0x1p20f);
     }
 };
 
@@ -407,7 +405,7 @@ struct LaneJoints {
 // (sn, cs) of the angles, contacts loaded; out: (sn, cs) of the new angles where R::ANGLES_AFTER.
 template <class R, int VEL, int POS, class Contacts>
 MRL_DEV void body_lanes_solve(LaneBody &B, LaneJoints<R> &J, Contacts &contacts, float &sn, float &cs, float dt, float friction,
-                              float restitution, float baumgarte, const SinCosK &K) {
+                              float restitution, float baumgarte) {
     J.prepare(B, sn, cs);
 #pragma unroll 1
     for (int it = 0; it < VEL; ++it) {
@@ -415,6 +413,7 @@ MRL_DEV void body_lanes_solve(LaneBody &B, LaneJoints<R> &J, Contacts &contacts,
         J.velocity_sweep(B, dt);
     }
     lane_integrate_position(B, dt);
+    const SinCosK K = SinCosK::held();
     sincos32(B.ang[0], sn, cs, K);
     const float x = B.x[0], y = B.y[0], ang = B.ang[0], s0 = sn, c0 = cs;
     if (__builtin_expect(J.template position_sweeps<true, POS>(B, sn, cs, contacts, baumgarte, K), 1)) return;

@@ -38,7 +38,6 @@ MRL_DEV void physics_lanes(float *row, float *contacts, int n, int lane) {
     const int b = has ? body : 0;
     const float gx = (float)0.0, gy = (float)-10.0, dt = (float)(1.0 / FPS), friction = (float)2.5, restitution = (float)0.0;
     const float baumgarte = (float)0.2;
-    const SinCosK K = SinCosK::held();
 
     LaneBody B;
     lane_body_load<L>(B, row, b);
@@ -49,8 +48,8 @@ MRL_DEV void physics_lanes(float *row, float *contacts, int n, int lane) {
     LaneListContacts<L, 2> list;
     list.load(B, contacts, n, body, baumgarte);
     float sn, cs;
-    sincos32(B.ang[0], sn, cs, K);
-    body_lanes_solve<Wiring, 6, 2>(B, J, list, sn, cs, dt, friction, restitution, baumgarte, K);
+    sincos32(B.ang[0], sn, cs);
+    body_lanes_solve<Wiring, 6, 2>(B, J, list, sn, cs, dt, friction, restitution, baumgarte);
     if (has) lane_body_store<L>(B, row, b);
     // ---- observation entries 0 .. 7 and 9 .. 12 (observe_state: the same expressions on the same values), every
     // body's lane its own: the hull 0 .. 3, a leg segment its angle and angular velocity against its parent's.

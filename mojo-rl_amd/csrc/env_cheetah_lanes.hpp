@@ -87,14 +87,14 @@ struct GroundContacts {
     MRL_DEV void velocity(LaneBody &B, float friction, float restitution) {
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            if (!__any(k < kept)) return;
+            if (!any_lane(k < kept)) return;
             contact_velocity<OneBody>(B, 0, c[k].f, c[k].jn, c[k].jt, friction, restitution, k < kept);
         }
     }
     MRL_DEV void position(LaneBody &B, float) const {
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            if (!__any(k < kept)) return;
+            if (!any_lane(k < kept)) return;
             c[k].position(B);
         }
     }
@@ -107,7 +107,6 @@ MRL_DEV void step_lanes(float *row, const float *shapes, const float *action, in
     const int l = lane & 7, base = lane & ~7, body = lane_body<Wiring>(l);
     const bool has = body < 7;
     const int b = has ? body : 0;
-    const SinCosK K = SinCosK::held();
 
     const float gx = (float)0.0, gy = (float)-9.81, dt = (float)0.01, friction = (float)0.9, restitution = (float)0.0;
     const float baumgarte = (float)0.2;
@@ -138,7 +137,7 @@ MRL_DEV void step_lanes(float *row, const float *shapes, const float *action, in
     const double x_before = (double)B.x[0];   // meaningful on lane 0 (the torso)
 
     float sn, cs;
-    sincos32(B.ang[0], sn, cs, K);
+    sincos32(B.ang[0], sn, cs);
     GroundContacts contacts;
     contacts.kept = 0;
 #pragma unroll 1
@@ -163,7 +162,7 @@ MRL_DEV void step_lanes(float *row, const float *shapes, const float *action, in
         // the list of an env is cut at MAX_CONTACTS in (body, vertex) order: contacts before mine are counted, where the
         // list can be that long
         contacts.kept = found;
-        if (__any(found > L::MAX_CONTACTS / 7)) {
+        if (any_lane(found > L::MAX_CONTACTS / 7)) {
             int before = 0;
 #pragma unroll
             for (int o = 0; o < 7; ++o) {
@@ -175,10 +174,10 @@ MRL_DEV void step_lanes(float *row, const float *shapes, const float *action, in
         }
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            if (!__any(c < contacts.kept)) break;
+            if (!any_lane(c < contacts.kept)) break;
             contacts.c[c].prepare(B, c < contacts.kept, px[c], py[c], 0.0f, 1.0f, 0.0f - py[c], baumgarte);
         }
-        body_lanes_solve<Wiring, 4, 2>(B, J, contacts, sn, cs, dt, friction, restitution, baumgarte, K);
+        body_lanes_solve<Wiring, 4, 2>(B, J, contacts, sn, cs, dt, friction, restitution, baumgarte);
     }
     // ---- bodies and forces back into the row, then the rest of the step on the torso's lane
     if (has) lane_body_store<L>(B, row, b);

@@ -62,13 +62,14 @@ struct SinCosK {
            s5 = -2.5051129896450185e-08, s6 = 1.5917988979397435e-10;
     double c1 = 0.041666666666666664, c2 = -0.0013888888888887389, c3 = 2.48015872987544e-05, c4 = -2.755731726587808e-07,
            c5 = 2.087614504941318e-09, c6 = -1.138254464534925e-11;
-    // The constants in scalar registers for as long as the caller keeps the struct: without, every use moves their
-    // halves there again, 30 instructions a call.
+    // The constants in registers for as long as the caller keeps the struct: without, every use moves their halves into
+    // scalar registers again, 30 instructions a call.  (Vector registers: the kernels that ask for it are short of
+    // scalar ones, which would come and go through lanes of a vector register.)
     static MRL_DEV SinCosK held() {
         SinCosK k;
-        asm volatile("" : "+s"(k.two_over_pi), "+s"(k.half_pi), "+s"(k.half_pi_lo), "+s"(k.s1), "+s"(k.s2), "+s"(k.s3),
-                     "+s"(k.s4), "+s"(k.s5), "+s"(k.s6));
-        asm volatile("" : "+s"(k.c1), "+s"(k.c2), "+s"(k.c3), "+s"(k.c4), "+s"(k.c5), "+s"(k.c6));
+        asm volatile("" : "+v"(k.two_over_pi), "+v"(k.half_pi), "+v"(k.half_pi_lo), "+v"(k.s1), "+v"(k.s2), "+v"(k.s3),
+                     "+v"(k.s4), "+v"(k.s5), "+v"(k.s6));
+        asm volatile("" : "+v"(k.c1), "+v"(k.c2), "+v"(k.c3), "+v"(k.c4), "+v"(k.c5), "+v"(k.c6));
         return k;
     }
 };
@@ -145,6 +146,9 @@ MRL_DEV float log32(float x) {
     if (!(x > 0.0f && x < __builtin_inff())) r = x == 0.0f ? -__builtin_inff() : (x < 0.0f ? __builtin_nanf("") : x);
     return r;
 }
+
+// whether any active lane says so, straight from the compare
+MRL_DEV bool any_lane(bool p) { return __builtin_amdgcn_ballot_w64(p) != 0; }
 
 // x / d for a divisor that is divided by again and again (a joint's summed inverse inertia, a contact's
 // effective mass over the sweeps of a step), given r = 1.0f / d, the IEEE reciprocal taken once: two

@@ -183,7 +183,7 @@ MRL_DEV void contact_velocity(RegBodies<L> &B, int ia, const ContactFixed &f, fl
     float rel_vel_x = vel_at_a_x - vel_at_b_x, rel_vel_y = vel_at_a_y - vel_at_b_y;
     const float vel_normal = rel_vel_x * normal_x + rel_vel_y * normal_y;
     const bool push = live && vel_normal < 0.0f;
-    if (!__any(push)) return;
+    if (!any_lane(push)) return;
 
     float j_normal = div_by(-(1.0f + restitution) * vel_normal, f.k, f.rk);
     const float old_impulse = jn;
@@ -264,14 +264,14 @@ struct RegContacts {
     MRL_DEV void velocity_sweep(RegBodies<L> &B, float friction, float restitution) {
 #pragma unroll
         for (int c = 0; c < MC; ++c) {
-            if (!__any(c < n)) break;
+            if (!any_lane(c < n)) break;
             contact_velocity<L>(B, body[c], f[c], jn[c], jt[c], friction, restitution, c < n);
         }
     }
     MRL_DEV void position_sweep(RegBodies<L> &B, float baumgarte) const {
 #pragma unroll
         for (int c = 0; c < MC; ++c) {
-            if (!__any(c < n)) break;
+            if (!any_lane(c < n)) break;
             if (c < n) contact_position<L>(B, body[c], f[c].nx, f[c].ny, depth[c], baumgarte);
         }
     }
@@ -348,8 +348,8 @@ MRL_DEV void joint_limits(JointSweep &q, bool limited, float rel_angle, float lo
 struct JointTerms {
     bool spring, limit, motor;
     MRL_DEV void add(const JointSweep &q, bool active = true) {
-        const bool s = __any(active && q.spring), l = __any(active && (q.below == 0.0f || q.above == 0.0f));
-        const bool m = __any(active && q.motor);
+        const bool s = any_lane(active && q.spring), l = any_lane(active && (q.below == 0.0f || q.above == 0.0f));
+        const bool m = any_lane(active && q.motor);
         spring = spring | s;
         limit = limit | l;
         motor = motor | m;
