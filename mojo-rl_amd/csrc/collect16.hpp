@@ -31,7 +31,7 @@ struct Critic16Split {
 // while the actor of 16 rows takes half the matrix time of 32 (v_mfma_f32_16x16x4_f32, same bits as
 // the 32-row tiles): few envs are stepped faster spread 16 to a CU than packed 32 to half the CUs.
 //   all four wavefronts     actor  OBS -> H -> H -> A, 64 columns each;
-//   the solver wavefront    sampling, env step (one env per lane 0 .. 15), accounting, resets;
+//   the solver wavefront    sampling, env step (four lanes per env, one per body: env_lunar.hpp), accounting, resets;
 //   the other three         contact detection, then the critic (H = 256: 80 / 96 / 80 columns) at a
 //                           barrier of their own.
 // Two such workgroups fit a CU (LDS, registers), but running them side by side does not pay: on this
@@ -40,6 +40,8 @@ struct Critic16Split {
 // of both times), so one workgroup's env step does not hide behind the other's forward passes, and
 // two solver wavefronts of 16 envs cost twice the vector time of one with 32.  With more than 16 envs
 // per CU the 32-row kernel above is the faster one (8192 envs: 38.6 against 39.8 us per step).
+// us per step with one lane per env : four: 777 envs, H = 64 19.4 : 12.9 (its solver wavefront: 22 of 37 thousand cycles in
+// the physics before); 4096 envs, H = 64 18.8 : 12.6, H = 256, where the critic is the longer path, 23.9 : 21.6.
 // The solver wavefront is 0 in the lower half of the grid and 2 in the upper half: workgroups i and
 // i + grid / 2 share a CU when the grid is twice the CU count, and their solvers then sit on
 // different SIMDs.
@@ -89,10 +91,13 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
         sync_failed = 0;
     }
     __syncthreads();
-    // solver wavefront, lane = env slot: the env's running episode return and length stay in registers
-    const bool owner = (t >> 6) == sw && (t & 63) < nenv;
-    float ep_return = owner ? a.acc.ep_return[env0 + (t & 63)] : 0.0f;
-    float ep_length = owner ? a.acc.ep_length[env0 + (t & 63)] : 0.0f;
+    // solver wavefront, four lanes per env: the env's running episode return and length stay in registers of the first,
+    // and whether its wiring is the kind's own (no step changes it, a reset makes it so) in all four
+    const int my_env = (t & 63) >> 2;
+    const bool owner = (t >> 6) == sw && my_env < nenv && (t & 3) == 0;
+    float ep_return = owner ? a.acc.ep_return[env0 + my_env] : 0.0f;
+    float ep_length = owner ? a.acc.ep_length[env0 + my_env] : 0.0f;
+    int wired = my_env < nenv && E::lanes_ok(rows + my_env * S::STRIDE) ? 1 : 0;
 
     for (int k = 0; k < a.n_steps; ++k) {
         // Nothing but the rows is carried from one step to the next: the thread index, the block's
@@ -132,35 +137,35 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
         if (vw == 0) {
             // ---- sample, then the env step of env_block.hpp with the contacts the helpers detect
             typename E::Carry carry{};
-            if (lane < ne) {
-                const int i = env0 + lane;
+            const int e = lane >> 2;
+            const bool first = (lane & 3) == 0 && e < ne;
+            if (first) {
+                const int i = env0 + e;
                 float logp;
                 if (GAUSS) {
                     float av[PA_MAX];
-                    logp = sample_gaussian(logits + lane * (PA_MAX + 1), w2a + HEAD_LOG_STD(H), A, sseed, i, av);
+                    logp = sample_gaussian(logits + e * (PA_MAX + 1), w2a + HEAD_LOG_STD(H), A, sseed, i, av);
                     for (int j = 0; j < A; ++j) {
-                        act[lane * AW + j] = av[j];
-                        a.r_actions[(row + lane) * AW + j] = av[j];
+                        act[e * AW + j] = av[j];
+                        a.r_actions[(row + e) * AW + j] = av[j];
                     }
                 } else {
                     int sel;
-                    sample_categorical_few(logits + lane * (PA_MAX + 1), A, sseed, i, sel, logp);
-                    act[lane] = (float)sel;
-                    a.r_actions[row + lane] = (float)sel;
+                    sample_categorical_few(logits + e * (PA_MAX + 1), A, sseed, i, sel, logp);
+                    act[e] = (float)sel;
+                    a.r_actions[row + e] = (float)sel;
                 }
-                a.r_logp[row + lane] = logp;
-                carry = E::step_begin(rows + lane * S::STRIDE, i, act + lane * AW, shapes);
+                a.r_logp[row + e] = logp;
+                carry = E::step_begin(rows + e * S::STRIDE, i, act + e * AW, shapes);
             }
             detect_sync.target += detect_sync.nwaves;
             detect_sync.wait_for(detect_sync.target);
+            float r = 0.0f, d = 0.0f;
+            step_finish_quads<E, CAP>(rows, cts, shapes, dlist, dcount, carry, wired != 0, lane, ne, r, d);
             bool finished = false;
-            if (lane < ne) {
-                float *mine = cts + lane * S::CSTRIDE;
-                const int n = merge_vertex_lists<E, CAP>(dlist, dcount, lane, mine);
-                float r, d;
-                E::step_finish(rows + lane * S::STRIDE, mine, n, shapes, carry, r, d);
-                a.r_rewards[row + lane] = r;
-                a.r_dones[row + lane] = d;
+            if (first) {
+                a.r_rewards[row + e] = r;
+                a.r_dones[row + e] = d;
                 ep_return = ep_return + r;
                 ep_length = ep_length + 1.0f;
                 finished = d > 0.5f;
@@ -174,7 +179,9 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
                     ep_length = 0.0f;
                 }
             }
-            reset_rows<E>(rows, &was_reset, __ballot(finished), a.reset_seed + (uint64_t)k * a.reset_stride, env0, lane);
+            const unsigned long long fin = quad_envs(__ballot(finished));
+            wired |= (int)((fin >> e) & 1ull);
+            reset_rows<E>(rows, &was_reset, fin, a.reset_seed + (uint64_t)k * a.reset_stride, env0, lane);
         } else {
             // ---- contact detection: (body, vertex) task m * 4 + lane / 16 of env slot lane % 16, a
             // second pass on helper 0 for the tasks beyond twelve
@@ -208,8 +215,8 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
     }
 
     if (owner) {
-        a.acc.ep_return[env0 + (t & 63)] = ep_return;
-        a.acc.ep_length[env0 + (t & 63)] = ep_length;
+        a.acc.ep_return[env0 + my_env] = ep_return;
+        a.acc.ep_length[env0 + my_env] = ep_length;
     }
     for (int i = t; i < nenv * E::OBS; i += T) {
         const int r = i / E::OBS, c = i - r * E::OBS;

@@ -81,6 +81,14 @@ struct LunarLander {
                                     float &d) {
         ll::step_finish(row, cts, n, shapes, c, r, d);
     }
+    // the same in parts, the physics by the four lanes of an env (step_finish_quads)
+    static MRL_DEV bool row_done(const float *row) { return row[L::META_OFF + ll::META_DONE] > 0.5f; }
+    static MRL_DEV bool lanes_ok(const float *row) { return ll::lanes_row_ok(row); }
+    static MRL_DEV void physics_lanes(float *row, float *cts, int n, int lane) { ll::physics_lanes(row, cts, n, lane); }
+    static MRL_DEV int physics_one(float *row, float *cts, int n, const float *shapes) { return ll::step_physics(row, cts, n, shapes); }
+    static MRL_DEV void step_tail(float *row, const float *cts, int n, const Carry &c, float &r, float &d) {
+        ll::step_tail(row, cts, n, c, r, d);
+    }
 };
 
 // LunarLanderV2 behind the continuous-action trait (the reference overloads step_kernel_gpu on
@@ -399,6 +407,78 @@ MRL_DEV int merge_vertex_list_of_task(const float *dlist, const int *dcount, int
     return redo ? -1 : (total < E::L::MAX_CONTACTS ? total : E::L::MAX_CONTACTS);
 }
 
+// merge_vertex_lists by the four lanes of an env (lanes 4 e .. of the wavefront): each moves the lists of a quarter of the
+// tasks, in order, behind those of the lanes before it.  Every lane returns the count.
+template <class E, int CAP>
+MRL_DEV int merge_vertex_lists_quads(const float *dlist, const int *dcount, int e, int l, float *mine) {
+    constexpr int PER = (E::DETECT_TASKS + 3) / 4;
+    int m[PER], own = 0;
+    bool redo = false;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        const int k = l * PER + i;
+        m[i] = k < E::DETECT_TASKS ? dcount[k * E::EPB + e] : 0;
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        redo = redo || m[i] < 0;
+        m[i] = m[i] < 0 ? 0 : (m[i] < CAP ? m[i] : CAP);
+        own += m[i];
+    }
+    // sums over the lanes of the quad: a redo counts in the high half
+    const int v = own + (redo ? 1 << 16 : 0);
+    const int q0 = __builtin_amdgcn_mov_dpp(v, 0x00, 0xF, 0xF, true), q1 = __builtin_amdgcn_mov_dpp(v, 0x55, 0xF, 0xF, true);
+    const int q2 = __builtin_amdgcn_mov_dpp(v, 0xAA, 0xF, 0xF, true), q3 = __builtin_amdgcn_mov_dpp(v, 0xFF, 0xF, 0xF, true);
+    const int total = q0 + q1 + q2 + q3;
+    if (any_lane(own > 0)) {
+        int at = (l > 0 ? q0 & 0xFFFF : 0) + (l > 1 ? q1 & 0xFFFF : 0) + (l > 2 ? q2 & 0xFFFF : 0);
+        for (int i = 0; i < PER; ++i) {
+            const float *src = dlist + ((l * PER + i) * E::EPB + e) * detect_stride(CAP);
+            for (int c = 0; c < m[i] && at < E::L::MAX_CONTACTS; ++c, ++at) {
+                float rec[CONTACT_SIZE];
+#pragma unroll
+                for (int f = 0; f < CONTACT_SIZE; ++f) rec[f] = src[c * CONTACT_SIZE + f];
+#pragma unroll
+                for (int f = 0; f < CONTACT_SIZE; ++f) mine[at * CONTACT_SIZE + f] = rec[f];
+            }
+        }
+    }
+    const int n = (total & 0xFFFF) < E::L::MAX_CONTACTS ? total & 0xFFFF : E::L::MAX_CONTACTS;
+    return total >= 1 << 16 ? -1 : n;
+}
+
+MRL_DEV void wave_sync_rows() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// E::step_finish for the 16 envs of one wavefront, four lanes per env, given the contact lists of the detection tasks: the
+// physics with one lane per body, the rest by the first lane of each env, which returns reward and done.  An env whose
+// wiring is not its kind's own (`ok` false), or with a list that overflowed, is stepped by its first lane alone.
+template <class E, int CAP>
+MRL_DEV void step_finish_quads(float *rows, float *cts, const float *shapes, const float *dlist, const int *dcount,
+                               const typename E::Carry &carry, bool ok, int lane, int ne, float &r, float &d) {
+    using S = Stage<E>;
+    const int e = lane >> 2, l = lane & 3;
+    if (e >= ne) return;
+    float *row = rows + e * S::STRIDE, *mine = cts + e * S::CSTRIDE;
+    wave_sync_rows();   // (the engines' velocities, written by the first lanes)
+    int n = merge_vertex_lists_quads<E, CAP>(dlist, dcount, e, l, mine);
+    wave_sync_rows();
+    const bool moves = !E::row_done(row), quad = moves && n >= 0 && ok;
+    if (quad) E::physics_lanes(row, mine, n, lane);
+    else if (moves && l == 0) n = E::physics_one(row, mine, n, shapes);
+    wave_sync_rows();
+    if (l == 0) E::step_tail(row, mine, n, carry, r, d);
+}
+// bits 4 e of a mask of first lanes as bits e
+MRL_DEV unsigned long long quad_envs(unsigned long long m) {
+    unsigned long long out = 0;
+    for (; m; m &= m - 1) out |= 1ull << ((__ffsll((long long)m) - 1) >> 2);
+    return out;
+}
+
 // One step of the block's LDS-resident rows (all threads of the block call it, between two
 // __syncthreads of the caller): wavefront 0 steps one env per lane, the other wavefronts detect
 // contacts where the env splits that off.  `actions` = the actions of the block's envs
@@ -429,12 +509,19 @@ MRL_DEV void phys_step_block(float *rows, float *cts, const float *shapes, float
         constexpr int AT_ONCE = (E::THREADS / WAVE - 1) * PER_WAVE;
         static_assert((GROUP == 16 || GROUP == 32) && AT_ONCE > 0, "16 or 32 rows per workgroup, wavefront 0 and at least one more");
         const int wave = tid / WAVE, lane = tid % WAVE;
+        constexpr bool QUADS = GROUP * 4 == WAVE;   // four lanes per env in wavefront 0, else one
+        const int slot = QUADS ? lane >> 2 : lane;
+        const bool first = slot < nenv && (!QUADS || (lane & 3) == 0);
         typename E::Carry carry{};
         EpisodeSums sums{0.0f, 0.0f};
+        bool ok = false;
         if (wave == 0) {
-            if (lane < nenv) sums = account_before(acc, lane);
-            if (lane < nenv)
-                carry = E::step_begin(rows + lane * S::STRIDE, env0 + lane, actions + (size_t)lane * E::ACT_W, shapes);
+            if (first) sums = account_before(acc, slot);
+            if constexpr (QUADS) {
+                if (slot < nenv) ok = E::lanes_ok(rows + slot * S::STRIDE);
+            }
+            if (first)
+                carry = E::step_begin(rows + slot * S::STRIDE, env0 + slot, actions + (size_t)slot * E::ACT_W, shapes);
         } else {
             const int e = lane % GROUP;
 #pragma unroll 1
@@ -444,20 +531,26 @@ MRL_DEV void phys_step_block(float *rows, float *cts, const float *shapes, float
         __syncthreads();
         if (wave == 0) {
             bool finished = false;
-            if (lane < nenv) {
-                float *mine = cts + lane * S::CSTRIDE;
-                const int n = merge_vertex_lists<E>(dlist, dcount, lane, mine);
-                const int env = env0 + lane;
-                float r, d;
-                E::step_finish(rows + lane * S::STRIDE, mine, n, shapes, carry, r, d);
+            float r = 0.0f, d = 0.0f;
+            if constexpr (QUADS) {
+                step_finish_quads<E, DETECT_CAP>(rows, cts, shapes, dlist, dcount, carry, ok, lane, nenv, r, d);
+            } else if (first) {
+                float *mine = cts + slot * S::CSTRIDE;
+                const int n = merge_vertex_lists<E>(dlist, dcount, slot, mine);
+                E::step_finish(rows + slot * S::STRIDE, mine, n, shapes, carry, r, d);
+            }
+            if (first) {
                 if (rewards != nullptr) {
-                    rewards[env - env0] = r;
-                    dones[env - env0] = d;
+                    rewards[slot] = r;
+                    dones[slot] = d;
                 }
-                account(acc, env - env0, r, d, sums);
+                account(acc, slot, r, d, sums);
                 finished = d > 0.5f;
             }
-            if (AUTORESET) reset_rows<E>(rows, was_reset, __ballot(finished), reset_seed, env0, lane);
+            if (AUTORESET) {
+                const unsigned long long fin = __ballot(finished);
+                reset_rows<E>(rows, was_reset, QUADS ? quad_envs(fin) : fin, reset_seed, env0, lane);
+            }
         }
     } else {
         typename E::Carry carry{};

@@ -11,7 +11,7 @@
 // Philox(seed = env + 12345, offset = step_count), reset seed
 // Int(f32(seed)) * 2654435761 + (env + 1) * 12345.
 #pragma once
-#include "physics2d_reg.hpp"
+#include "body_lanes.hpp"
 
 namespace mrl {
 namespace ll {
@@ -319,6 +319,41 @@ MRL_DEV void apply_wind(float *row, int step_count, const float *shapes) {
     B[IDX_OMEGA] = (float)(omega + domega);
 }
 
+// The physics with one lane per body (body_lanes.hpp): lanes 4 e .. 4 e + 3 of a wavefront are the lander, leg 1, leg 2 and
+// an idle one of env e.  Both joints hold the lander, so they stay one after the other; what the lanes share is everything
+// about a body of its own -- integration, sines and cosines, contacts -- and each joint's two halves.
+constexpr int LANES_PER_ENV = 4;
+struct Wiring {
+    static constexpr int LANES = 4, SLOTS = 2;
+    static constexpr uint32_t BODY = 0xF210u;
+    static constexpr int CTRL[2] = {0xB1, 0x4E};           // l ^ 1, l ^ 2
+    static constexpr uint32_t IN[2] = {0x3u, 0x5u}, CHILD[2] = {0x2u, 0x4u};
+    static constexpr uint32_t JOINT[2] = {0x0000u, 0x0101u};
+    static constexpr bool SPRING = true, MOTOR = false, ANGLES_AFTER = false, LAST_TURNS_FIRST = true;
+};
+MRL_DEV bool lanes_row_ok(const float *row) { return body_lanes_row_ok<L, Topology, Wiring>(row); }
+
+// step_physics by the four lanes of an env, given its n >= 0 contacts
+MRL_DEV void physics_lanes(float *row, float *contacts, int n, int lane) {
+    const int l = lane & 3, body = lane_body<Wiring>(l);
+    const bool has = body < L::NUM_BODIES;
+    const int b = has ? body : 0;
+    const float gx = (float)0.0, gy = (float)-10.0, dt = (float)DT;
+    const float friction = (float)0.1, restitution = (float)0.0, baumgarte = (float)0.2;
+    LaneBody B;
+    lane_body_load<L>(B, row, b);
+    const float *F = row + L::FORCES_OFF + b * 3;
+    lane_integrate_velocity(B, F[0], F[1], F[2], gx, gy, dt);
+    LaneJoints<Wiring> J;
+    J.load<L>(row, l, B, dt);
+    LaneListContacts<L, 2> list;
+    list.load(B, contacts, n, body, baumgarte);
+    float sn, cs;
+    sincos32(B.ang[0], sn, cs);
+    body_lanes_solve<Wiring, 6, 2>(B, J, list, sn, cs, dt, friction, restitution, baumgarte);
+    if (has) lane_body_store<L>(B, row, b);
+}
+
 MRL_DEV StepCarry step_begin(float *row, int env, int action, const float *shapes) {
     StepCarry c;
     c.skip = row[L::META_OFF + META_DONE] > 0.5f;
@@ -359,8 +394,17 @@ MRL_DEV StepCarry step_begin_continuous(float *row, int env, const float *a, con
     return c;
 }
 
-MRL_DEV void step_finish(float *row, float *contacts, int n_given, const float *shapes, const StepCarry &c,
-                         float &reward, float &done) {
+// the physics of a step in the one-lane form, with the `n_given` contacts given (< 0: detects them); returns their number
+MRL_DEV int step_physics(float *row, float *contacts, int n_given, const float *shapes) {
+    const float gx = (float)0.0, gy = (float)-10.0, dt = (float)DT;
+    const float friction = (float)0.1, restitution = (float)0.0;
+    const float baumgarte = (float)0.2;
+    return reg_physics_substep<L, Topology, false, true>(row, shapes, contacts, gx, gy, dt, friction, restitution, baumgarte,
+                                                         6, 2, n_given);
+}
+
+// everything after the physics: observation, reward, termination
+MRL_DEV void step_tail(float *row, const float *contacts, int n, const StepCarry &c, float &reward, float &done) {
     if (c.skip) {
         reward = 0.0f;
         done = 1.0f;
@@ -368,12 +412,6 @@ MRL_DEV void step_finish(float *row, float *contacts, int n_given, const float *
     }
     const double m_power = c.m_power, s_power = c.s_power;
     int step_count = c.step_count;
-    const float gx = (float)0.0, gy = (float)-10.0, dt = (float)DT;
-    const float friction = (float)0.1, restitution = (float)0.0;
-    const float baumgarte = (float)0.2;
-    const int n = reg_physics_substep<L, Topology, false, true>(row, shapes, contacts, gx, gy, dt, friction,
-                                                                restitution, baumgarte, 6, 2, n_given);
-
     step_count += 1;
     float obs[8];
     observe(row, obs);
@@ -405,6 +443,13 @@ MRL_DEV void step_finish(float *row, float *contacts, int n_given, const float *
     row[L::META_OFF + META_DONE] = terminated ? 1.0f : 0.0f;
     reward = r;
     done = terminated ? 1.0f : 0.0f;
+}
+
+MRL_DEV void step_finish(float *row, float *contacts, int n_given, const float *shapes, const StepCarry &c,
+                         float &reward, float &done) {
+    int n = 0;
+    if (!c.skip) n = step_physics(row, contacts, n_given, shapes);
+    step_tail(row, contacts, n, c, reward, done);
 }
 
 // one env step on an LDS-resident row by one lane; `contacts` = this lane's contact scratch

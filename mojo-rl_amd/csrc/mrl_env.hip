@@ -2,7 +2,8 @@
 //
 // Physics envs: a workgroup handles EPB consecutive env rows.  The rows are contiguous in the
 // reference's [B, STATE_SIZE] buffer, so all wavefronts of the block copy them HBM -> LDS with
-// coalesced 16-byte loads, one lane of wavefront 0 per env then steps it entirely out of LDS
+// coalesced 16-byte loads, wavefront 0 (LunarLander: four lanes per env, 16 envs; BipedalWalker: eight lanes per env, two
+// wavefronts) then steps them entirely out of LDS
 // (row stride odd => the lanes touch distinct banks for any field) while the other wavefronts
 // detect its contacts where the env splits that off, and the fields that a step can change are
 // copied back with coalesced stores.  HBM sees each row once in and the changed part once out;
@@ -146,8 +147,9 @@ __global__ __launch_bounds__(E::THREADS) void phys_step_kernel(float *states, co
 // The same step with one lane per ENV and the rows left in global memory (64 envs per single-wavefront
 // workgroup, only the contact scratch in LDS): nothing is shared between lanes, so a batch that fills the
 // chip runs at the rate of the vector units instead of at the latency of one workgroup's phase chain.
-// Used from E::LANE_FROM envs on (LunarLander: one wavefront's step lasts 44 us whatever the batch, the
-// 32-row workgroup's 33 us, but a CU holds five of these wavefronts and one such workgroup).
+// Used from E::LANE_FROM envs on (LunarLander: one wavefront's step lasts 40 us whatever the batch, the
+// 16-row workgroup's 19 .. 22 us, but a CU holds five of these wavefronts and two such workgroups; with 32 rows and one
+// lane per env the workgroup took 30 .. 33 us).
 template <class E, bool AUTORESET>
 __global__ __launch_bounds__(64) void phys_step_lane_kernel(float *states, const float *actions, float *rewards,
                                                             float *dones, float *obs, const float *shapes_g, int batch,
@@ -579,11 +581,11 @@ static int env_step_impl(mrl_ctx *ctx, int env_id, int batch, float *states, con
                                autoreset ? 1 : 0, reset_seed, acc);
             break;
         case MRL_ENV_LUNARLANDER:
-            launch_phys_step<LunarLander>(ctx, batch, states, actions, rewards, dones, obs, ctx->ll_shapes,
+            launch_phys_step<Rows16<LunarLander>>(ctx, batch, states, actions, rewards, dones, obs, ctx->ll_shapes,
                                           autoreset, reset_seed, acc);
             break;
         case MRL_ENV_LUNARLANDER_CONTINUOUS:
-            launch_phys_step<LunarLanderContinuous>(ctx, batch, states, actions, rewards, dones, obs, ctx->ll_shapes,
+            launch_phys_step<Rows16<LunarLanderContinuous>>(ctx, batch, states, actions, rewards, dones, obs, ctx->ll_shapes,
                                                     autoreset, reset_seed, acc);
             break;
         case MRL_ENV_BIPEDAL:
