@@ -72,6 +72,9 @@ int mrl_ctx_create(void *hip_stream, mrl_ctx **out) {
     CTX_TRY(hipMemset(c->upd_scratch, 0, sizeof(float) * 8192));
     CTX_TRY(hipHostMalloc((void **)&c->sync_error, 64, hipHostMallocDefault));
     *c->sync_error = 0;
+    c->stop_seen = c->sync_error + 8;
+    *c->stop_seen = 0;
+    c->stop_call = 0;
     {
         int rc = mrl::clip_static_setup(c->device);
         if (rc != MRL_OK) { mrl_ctx_destroy(c); return rc; }

@@ -41,6 +41,10 @@ struct mrl_ctx {
     // writes directly) and the kernel ends normally.  mrl_ctx_synchronize reports and clears it.
     unsigned spin_limit;
     int *sync_error;
+    // A multi-minibatch update's call number, and the number of the last call whose KL stop the device has seen (pinned, like
+    // sync_error): the host leaves launches away that would find the stop raised and do nothing.
+    int stop_call;
+    int *stop_seen;
     // CarRacingV2: 0 = the CPU env's reward / termination arithmetic (default), 1 = the GPU trait's
     int car_trait_form;
     // phase timing: events recorded on `stream` at phase boundaries while armed
