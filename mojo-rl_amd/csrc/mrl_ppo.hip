@@ -141,12 +141,19 @@ __global__ __launch_bounds__(64) void gae_kernel(int T, int N, const float *__re
 // step.  What a plain scan waits for is memory, so the chain gets a wavefront of its own and eight
 // others feed it: a workgroup has G envs; its loaders fetch K = 512 / G * R steps at a time (index
 // t * N + env: rows of G consecutive floats), form delta, which needs no neighbour but the value one
-// step later, and leave (delta, done) in LDS; one wavefront scans the chunk in place; the loaders
-// store advantages and returns.  Three chunks are in LDS at once, one per stage, and the next one's
-// loads are in flight meanwhile.  What bounds it now is the chain (about 50 cycles a step) up to 16 envs
+// step later, and leave (delta, decay or 0 where the episode ends) in LDS, two steps to 16 bytes; one wavefront scans
+// the chunk in place; the loaders store advantages and returns.  A step of the scan is one product, by the multiplication
+// whose zero times anything is zero, and one sum, and half a load and a store.  Three chunks are in LDS at once, one per stage, and the next one's
+// loads are in flight meanwhile.  What bounds it now is the chain (about 35 cycles a step; as product, sum, test and two LDS accesses 50) up to 16 envs
 // per CU, then the memory (T = 1000, N = 8192: 5.6 TB/s).  Same operations in the same order as the scan.  A chunk's rows, and
 // the value row above it, are read two barriers before the first of them is stored, so outputs may
 // share memory with the inputs.  deep_agents/ppo/ppo.mojo:2317-2353
+// a * b, and 0 where a or b is zero, whatever the other one is
+MRL_DEV float mul_zero_wins(float a, float b) {
+    float r;
+    asm("v_mul_legacy_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
 constexpr int GAE_LOADERS = 512;   // threads; one more wavefront scans
 
 template <int G, int R>
@@ -154,8 +161,8 @@ __global__ __launch_bounds__(GAE_LOADERS + 64) void gae_fed_kernel(int T, int N,
                                                                const float *dones, const float *bootstrap, float gamma,
                                                                float decay, float *adv, float *ret) {
     constexpr int K = GAE_LOADERS / G * R, U = 16;
-    static_assert(K % U == 0, "");
-    __shared__ float2 buf[3][K * G];
+    static_assert(K % U == 0 && R % 2 == 0, "whole pairs per loader, whole groups per chunk");
+    __shared__ __align__(16) float4 buf[3][K / 2 * G];   // [step pair][env]: (delta, factor) of the later step and of the one before it
     // two groups of 16 share a 128-byte line: they go to one XCD (workgroup b runs on XCD b % 8), eight
     // workgroups apart, so that one L2 sees both halves
     const int b = blockIdx.x;
@@ -191,12 +198,14 @@ __global__ __launch_bounds__(GAE_LOADERS + 64) void gae_fed_kernel(int T, int N,
     for (int it = 0; it < C + 2; ++it) {
         if (!scanner) {
             if (it < C) {
-                float2 *B = buf[it % 3] + top * G + lane;
+                float4 *B = buf[it % 3] + top / 2 * G + lane;
                 float nv = next;
 #pragma unroll
-                for (int j = 0; j < R; ++j) {
-                    B[j * G] = make_float2(r[j] + gamma * (d[j] > 0.5f ? 0.0f : nv) - v[j], d[j]);
-                    nv = v[j];
+                for (int j = 0; j < R; j += 2) {
+                    const bool e0 = d[j] > 0.5f, e1 = d[j + 1] > 0.5f;
+                    B[j / 2 * G] = make_float4(r[j] + gamma * (e0 ? 0.0f : nv) - v[j], e0 ? 0.0f : decay,
+                                               r[j + 1] + gamma * (e1 ? 0.0f : v[j]) - v[j + 1], e1 ? 0.0f : decay);
+                    nv = v[j + 1];
                 }
             }
             float vs[R];
@@ -204,12 +213,16 @@ __global__ __launch_bounds__(GAE_LOADERS + 64) void gae_fed_kernel(int T, int N,
             for (int j = 0; j < R; ++j) { vs[j] = v2[j]; v2[j] = v1[j]; v1[j] = v[j]; }
             if (it + 1 < C) request(it + 1);
             if (it >= 2) {
-                const float2 *B = buf[(it - 2) % 3] + top * G + lane;
+                const float4 *B = buf[(it - 2) % 3] + top / 2 * G + lane;
                 const int t0 = T - (it - 1) * K;
                 const long row0 = (long)t0 * N;
                 float a[R];
 #pragma unroll
-                for (int j = 0; j < R; ++j) a[j] = B[j * G].x;
+                for (int j = 0; j < R; j += 2) {
+                    const float4 q = B[j / 2 * G];
+                    a[j] = q.x;
+                    a[j + 1] = q.z;
+                }
                 if (t0 >= 0 && group * G + G <= N) {
 #pragma unroll
                     for (int j = 0; j < R; ++j) { out(adv, row0, off[j], a[j]); out(ret, row0, off[j], a[j] + vs[j]); }
@@ -220,24 +233,25 @@ __global__ __launch_bounds__(GAE_LOADERS + 64) void gae_fed_kernel(int T, int N,
                 }
             }
         } else if (it >= 1 && it <= C && threadIdx.x < GAE_LOADERS + G) {
-            float2 *B = buf[(it - 1) % 3] + lane;
+            float4 *B = buf[(it - 1) % 3] + lane;
             const int rows = min(K, T - (it - 1) * K);   // (up to U - 1 rows below t = 0 are scanned and never stored)
-            float2 x[U], n[U];
+            float4 x[U / 2], n[U / 2];
 #pragma unroll
-            for (int j = 0; j < U; ++j) x[j] = B[j * G];
+            for (int j = 0; j < U / 2; ++j) x[j] = B[j * G];
 #pragma unroll 2
             for (int k = 0; k < rows; k += U) {
-                const int kn = min(k + U, K - U);
+                const int kn = min(k + U, K - U) / 2;
 #pragma unroll
-                for (int j = 0; j < U; ++j) n[j] = B[(kn + j) * G];
+                for (int j = 0; j < U / 2; ++j) n[j] = B[(kn + j) * G];
 #pragma unroll
-                for (int j = 0; j < U; ++j) {
-                    if (x[j].y > 0.5f) gae = 0.0f;
-                    gae = x[j].x + decay * gae;
-                    B[(k + j) * G].x = gae;
+                for (int j = 0; j < U / 2; ++j) {
+                    const float g0 = x[j].x + mul_zero_wins(x[j].y, gae);
+                    gae = x[j].z + mul_zero_wins(x[j].w, g0);
+                    B[(k / 2 + j) * G].x = g0;
+                    B[(k / 2 + j) * G].z = gae;
                 }
 #pragma unroll
-                for (int j = 0; j < U; ++j) x[j] = n[j];
+                for (int j = 0; j < U / 2; ++j) x[j] = n[j];
             }
         }
         __syncthreads();
@@ -689,7 +703,8 @@ int mrl_gae(mrl_ctx *ctx, int T, int N, const float *rewards, const float *value
     if (T == 0 || N == 0) return MRL_OK;
     MRL_CHECK_ARG(rewards && values && dones && bootstrap && adv && ret, "mrl_gae: NULL buffer");
     // The narrowest groups that still give every group a CU of its own; with a wavefront of envs per CU the plain scan
-    // is the faster one.  us, plain / groups of 16 / 32 / 64: T = 1000, N = 1000: 57.5 / 22.2 / 26.3 / 30.5; N = 4096:
+    // is the faster one.  us, plain / groups of 16 / 32 / 64 (with a test in the chain; now 18.4 at N = 1000, 19.2 at
+    // N = 4096, 28.3 at N = 8192): T = 1000, N = 1000: 57.5 / 22.2 / 26.3 / 30.5; N = 4096:
     // 57.7 / 23.2 / 26.2 / 32.0; N = 8192: 58.0 / 43.0 / 29.1 / 35.2; T = 64, N = 16384: 6.4 / 10.6 / 7.4 / 5.8;
     // N = 65536: 13.4 / - / - / 21.2.
     const float g = (float)gamma, decay = (float)(gamma * lam);
