@@ -25,29 +25,24 @@ struct Critic16Split {
 };
 
 // ---------------------------------------------------------------- 16 rows per workgroup
-// The same step for a workgroup of four wavefronts and 16 envs, for launches with at most 16 envs
-// per CU.  A step is a chain -- actor on the matrix cores, then sampling and the env step on ONE
-// wavefront's vector unit -- and the env step costs the same whether 16 or 32 lanes carry an env,
-// while the actor of 16 rows takes half the matrix time of 32 (v_mfma_f32_16x16x4_f32, same bits as
-// the 32-row tiles): few envs are stepped faster spread 16 to a CU than packed 32 to half the CUs.
+// A workgroup of four wavefronts and 16 envs.  A step is a chain -- actor on the matrix cores, then sampling and the env
+// step on ONE wavefront's vector unit --, and beside it the critic, whose value is only stored.
 //   all four wavefronts     actor  OBS -> H -> H -> A, 64 columns each;
 //   the solver wavefront    sampling, env step (four lanes per env, one per body: env_lunar.hpp), accounting, resets;
 //   the other three         contact detection, then the critic (H = 256: 80 / 96 / 80 columns) at a
 //                           barrier of their own.
-// Two such workgroups fit a CU (LDS, registers), but running them side by side does not pay: on this
-// hardware a SIMD issues either a matrix or a vector instruction, never both at once (a wavefront of
-// dependent v_fma_f32 that shares its SIMD with a wavefront issuing v_mfma back to back takes the sum
-// of both times), so one workgroup's env step does not hide behind the other's forward passes, and
-// two solver wavefronts of 16 envs cost twice the vector time of one with 32.  With more than 16 envs
-// per CU the 32-row kernel above is the faster one (8192 envs: 38.6 against 39.8 us per step).
+// Two such workgroups fit a CU (LDS, registers).  On this hardware a SIMD issues either a matrix or a vector instruction,
+// never both at once (a wavefront of dependent v_fma_f32 that shares its SIMD with a wavefront issuing v_mfma back to back
+// takes the sum of both times), so at H = 256 the second one costs what its forward passes cost (4096 : 8192 envs 21.2 :
+// 31.5 us per step); still, since the solver carries four lanes per env, two of 16 rows are ahead of one of 32 rows with one
+// lane per env and the critic on six wavefronts (33.0).
 // us per step with one lane per env : four: 777 envs, H = 64 19.4 : 12.9 (its solver wavefront: 22 of 37 thousand cycles in
 // the physics before); 4096 envs, H = 64 18.8 : 12.6, H = 256, where the critic is the longer path, 23.9 : 21.6.
 // The solver wavefront is 0 in the lower half of the grid and 2 in the upper half: workgroups i and
 // i + grid / 2 share a CU when the grid is twice the CU count, and their solvers then sit on
 // different SIMDs.
-template <class EB, int H, int ACT, bool GAUSS>
+template <class E, int H, int ACT, bool GAUSS>
 __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
-    using E = Rows16<EB>;
     using S = Stage<E>;
     constexpr int IN = E::OBS, AW = E::ACT_W, R = PR16, T = E::THREADS;
     constexpr int NTA = H / 64;   // actor: column tiles per wavefront
@@ -209,7 +204,7 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
         // thread reads the same word after the barrier) and end normally
         if (sync_failed != 0u) break;
     }
-    if (sync_failed != 0u) {   // as in collect_kernel: nothing of a block whose wait gave up is stored
+    if (sync_failed != 0u) {   // nothing of a block whose wait gave up is stored
         if (t == 0) *a.sync_error = 1;
         return;
     }
@@ -377,7 +372,7 @@ __global__ __launch_bounds__(512, 4) void collect_classic16_kernel(CollectArgs a
 // the workgroups of `grid` = 16 envs each; side: CartPole's step counters
 template <int H, int ACT>
 int launch_collect16_t(mrl_ctx *ctx, const mrl_rollout *r, const CollectArgs &a, int32_t *side) {
-    const dim3 grid(grid_for(r->n_envs, PR16)), block(Rows16<LunarLander>::THREADS);
+    const dim3 grid(grid_for(r->n_envs, PR16)), block(LunarLander::THREADS);
     if (r->env_id == MRL_ENV_LUNARLANDER)
         hipLaunchKernelGGL((collect16_kernel<LunarLander, H, ACT, false>), grid, block, 0, ctx->stream, a);
     else if (r->env_id == MRL_ENV_LUNARLANDER_CONTINUOUS)

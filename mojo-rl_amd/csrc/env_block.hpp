@@ -45,7 +45,7 @@ MRL_DEV void account(const Accounting &acc, int i, float r, float d) { account(a
 
 struct LunarLander {
     using L = ll::L;
-    static constexpr int STATE = ll::STATE, OBS = ll::OBS, ACT_W = 1, EPB = 32, THREADS = 512;
+    static constexpr int STATE = ll::STATE, OBS = ll::OBS, ACT_W = 1, EPB = 16, THREADS = 256;
     static constexpr int LANE_FROM = 8193;   // batch from which the stand-alone step runs one lane per env
     static constexpr int DYN_END = L::JOINTS_OFF, NSHAPE = ll::NSHAPE_FLOATS;
     static MRL_DEV void step(float *row, float *cts, const float *shapes, int env, const float *a,
@@ -63,8 +63,8 @@ struct LunarLander {
     static MRL_DEV void reset_wave(float *row, uint64_t seed, int env, int lane) {
         ll::reset_row_wave(row, ll::combined_seed(seed, env), lane);
     }
-    // contact detection runs beside the engines of wavefront 0: every half of wavefronts 1 .. 7
-    // takes one (body, vertex) pair of the block's 32 envs -- hull 6 vertices, legs 4 each
+    // contact detection runs beside the engines of wavefront 0: every quarter of wavefronts 1 .. 3
+    // takes one (body, vertex) pair of the block's 16 envs at a time -- hull 6 vertices, legs 4 each
     static constexpr int DETECT_TASKS = 14, DETECT_WORDS = 0;
     static MRL_DEV void detect_share(const float *, const float *, int, unsigned *) {}
     static MRL_DEV void detect_task(int k, int &body, int &vertex, int &max_verts) {
@@ -344,43 +344,10 @@ MRL_DEV void detect_vertex_task(const float *rows, const float *shapes, float *d
         CAP, near);
 }
 
-// concatenates env slot e's lists in (body, vertex) order into `mine`, cut at MAX_CONTACTS;
-// returns the contact count, or -1 when some list asks for detection to be redone
-template <class E, int CAP = DETECT_CAP>
-MRL_DEV int merge_vertex_lists(const float *dlist, const int *dcount, int e, float *mine) {
-    // all counts first (independent loads, one round trip), then only the lists that hold something:
-    // most steps of most envs have no contact at all
-    int m[E::DETECT_TASKS];
-#pragma unroll
-    for (int k = 0; k < E::DETECT_TASKS; ++k) m[k] = dcount[k * E::EPB + e];
-    bool redo = false, any = false;
-#pragma unroll
-    for (int k = 0; k < E::DETECT_TASKS; ++k) {
-        redo |= m[k] < 0;
-        any |= m[k] > 0;
-    }
-    int n = 0;
-    if (any) {
-#pragma unroll
-        for (int k = 0; k < E::DETECT_TASKS; ++k) {
-            const float *src = dlist + (k * E::EPB + e) * detect_stride(CAP);
-            for (int c = 0; c < m[k] && c < CAP && n < E::L::MAX_CONTACTS; ++c, ++n) {
-                // a record is read whole before it is written (the two LDS ranges never overlap, which the
-                // compiler cannot see: it would wait for every float on its own)
-                float rec[CONTACT_SIZE];
-#pragma unroll
-                for (int f = 0; f < CONTACT_SIZE; ++f) rec[f] = src[c * CONTACT_SIZE + f];
-#pragma unroll
-                for (int f = 0; f < CONTACT_SIZE; ++f) mine[n * CONTACT_SIZE + f] = rec[f];
-            }
-        }
-    }
-    return redo ? -1 : n;
-}
-
-// merge_vertex_lists by the lanes that made the lists: the lane of (env slot e, task) moves its own list to
-// its place in the env's merged list -- behind the contacts of the tasks before it -- so that all lists move
-// at once.  Returns what merge_vertex_lists returns (every lane of the env gets the same value).
+// Concatenates env slot e's lists in (body, vertex) order into `mine`, cut at MAX_CONTACTS, by the lanes that made the
+// lists: the lane of (env slot e, task) moves its own list to its place -- behind the contacts of the tasks before it -- so
+// that all lists move at once.  Every lane of the env returns the contact count, or -1 when some list asks for detection to
+// be redone.
 template <class E, int CAP = DETECT_CAP>
 MRL_DEV int merge_vertex_list_of_task(const float *dlist, const int *dcount, int e, int task, float *mine) {
     int m[E::DETECT_TASKS];
@@ -407,7 +374,7 @@ MRL_DEV int merge_vertex_list_of_task(const float *dlist, const int *dcount, int
     return redo ? -1 : (total < E::L::MAX_CONTACTS ? total : E::L::MAX_CONTACTS);
 }
 
-// merge_vertex_lists by the four lanes of an env (lanes 4 e .. of the wavefront): each moves the lists of a quarter of the
+// The same by the four lanes of an env (lanes 4 e .. of the wavefront): each moves the lists of a quarter of the
 // tasks, in order, behind those of the lanes before it.  Every lane returns the count.
 template <class E, int CAP>
 MRL_DEV int merge_vertex_lists_quads(const float *dlist, const int *dcount, int e, int l, float *mine) {
@@ -507,19 +474,16 @@ MRL_DEV void phys_step_block(float *rows, float *cts, const float *shapes, float
         // (a wavefront holds WAVE / EPB tasks at a time; a block with fewer such groups than tasks takes turns)
         constexpr int NT = E::DETECT_TASKS, GROUP = E::EPB, PER_WAVE = WAVE / GROUP;
         constexpr int AT_ONCE = (E::THREADS / WAVE - 1) * PER_WAVE;
-        static_assert((GROUP == 16 || GROUP == 32) && AT_ONCE > 0, "16 or 32 rows per workgroup, wavefront 0 and at least one more");
+        static_assert(GROUP * 4 == WAVE && AT_ONCE > 0, "16 rows per workgroup, wavefront 0 and at least one more");
         const int wave = tid / WAVE, lane = tid % WAVE;
-        constexpr bool QUADS = GROUP * 4 == WAVE;   // four lanes per env in wavefront 0, else one
-        const int slot = QUADS ? lane >> 2 : lane;
-        const bool first = slot < nenv && (!QUADS || (lane & 3) == 0);
+        const int slot = lane >> 2;   // (wavefront 0: four lanes per env)
+        const bool first = slot < nenv && (lane & 3) == 0;
         typename E::Carry carry{};
         EpisodeSums sums{0.0f, 0.0f};
         bool ok = false;
         if (wave == 0) {
             if (first) sums = account_before(acc, slot);
-            if constexpr (QUADS) {
-                if (slot < nenv) ok = E::lanes_ok(rows + slot * S::STRIDE);
-            }
+            if (slot < nenv) ok = E::lanes_ok(rows + slot * S::STRIDE);
             if (first)
                 carry = E::step_begin(rows + slot * S::STRIDE, env0 + slot, actions + (size_t)slot * E::ACT_W, shapes);
         } else {
@@ -532,13 +496,7 @@ MRL_DEV void phys_step_block(float *rows, float *cts, const float *shapes, float
         if (wave == 0) {
             bool finished = false;
             float r = 0.0f, d = 0.0f;
-            if constexpr (QUADS) {
-                step_finish_quads<E, DETECT_CAP>(rows, cts, shapes, dlist, dcount, carry, ok, lane, nenv, r, d);
-            } else if (first) {
-                float *mine = cts + slot * S::CSTRIDE;
-                const int n = merge_vertex_lists<E>(dlist, dcount, slot, mine);
-                E::step_finish(rows + slot * S::STRIDE, mine, n, shapes, carry, r, d);
-            }
+            step_finish_quads<E, DETECT_CAP>(rows, cts, shapes, dlist, dcount, carry, ok, lane, nenv, r, d);
             if (first) {
                 if (rewards != nullptr) {
                     rewards[slot] = r;
@@ -549,7 +507,7 @@ MRL_DEV void phys_step_block(float *rows, float *cts, const float *shapes, float
             }
             if (AUTORESET) {
                 const unsigned long long fin = __ballot(finished);
-                reset_rows<E>(rows, was_reset, QUADS ? quad_envs(fin) : fin, reset_seed, env0, lane);
+                reset_rows<E>(rows, was_reset, quad_envs(fin), reset_seed, env0, lane);
             }
         }
     } else {
@@ -612,10 +570,6 @@ MRL_DEV void phys_step_block(float *rows, float *cts, const float *shapes, float
                     float *mine = cts + tid * S::CSTRIDE;
                     if (lanes_n >= 0) E::step_tail(rows + tid * S::STRIDE, mine, lanes_n, carry, r, d);
                     else E::step_finish(rows + tid * S::STRIDE, mine, -1, shapes, carry, r, d);
-                } else if constexpr (E::DETECT_TASKS > 0) {
-                    float *mine = cts + tid * S::CSTRIDE;
-                    const int n = merge_vertex_lists<E>(dlist, dcount, tid, mine);
-                    E::step_finish(rows + tid * S::STRIDE, mine, n, shapes, carry, r, d);
                 } else {
                     E::step(rows + tid * S::STRIDE, cts + tid * S::CSTRIDE, shapes, env,
                             actions + (size_t)tid * E::ACT_W, r, d);
@@ -669,12 +623,5 @@ constexpr int detect_count_ints() { return E::DETECT_TASKS * E::EPB + 1 + E::DET
 // LDS floats of the per-task contact lists that phys_step_block needs (0: the env detects inline)
 template <class E, int CAP = DETECT_CAP>
 constexpr int detect_list_floats() { return E::DETECT_TASKS * E::EPB * detect_stride(CAP); }
-
-// An env's traits with 16 rows per workgroup of four wavefronts (the fused collection kernel runs
-// two such workgroups per CU, so that one's env step overlaps the other's policy forward)
-template <class Base>
-struct Rows16 : Base {
-    static constexpr int EPB = 16, THREADS = 256;
-};
 
 }  // namespace mrl

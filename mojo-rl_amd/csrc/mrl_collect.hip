@@ -1,23 +1,14 @@
-// Fused collection kernel: many rollout steps of a block's envs in ONE launch.
+// Fused collection: many rollout steps of a block's envs in ONE launch.
 //
 // Envs do not interact and the policy does not change during a rollout, so a workgroup can take
-// its 32 envs through any number of steps on its own: the env rows stay in LDS from the first step
+// its envs through any number of steps on its own: the env rows stay in LDS (registers) from the first step
 // to the last (HBM sees them once in and once out per launch, however many steps), the
 // observation tile feeds the policy straight from those rows, and the sampled actions reach the
-// env step through LDS.  Per step and block:
-//   actor    OBS -> H -> H -> A on the fp32 matrix cores by all eight wavefronts (the 32 x H tiles
-//            of mlp_tile.hpp, weights streamed from L2);
-//   then, side by side,
-//     wavefront 0        categorical / Gaussian sampling, then the env step of env_block.hpp (one
-//                        env per lane), reward / done of rollout row t, episode accounting,
-//                        in-place reset;
-//     wavefronts 1 .. 7  contact detection for that env step;
-//     all of these but   then the critic  OBS -> H -> H -> 1  (its value is only stored, so it does
-//     wavefront 4        not hold up the env step; the six wavefronts meet at a barrier of their own,
-//                        and wavefront 4, which shares wavefront 0's SIMD, stays out of its way);
-//   rollout row t of obs, action, log-prob and value written on the way.
+// env step through LDS; rollout row t is written on the way.
 // No workgroup waits for another, so there is nothing between two steps but the block's own
 // barriers; the launch ends when every block has done its n_steps.
+// The kernels: collect16.hpp (LunarLander, CartPole, Pendulum), collect_walkers.hpp (the others), and for many CartPole /
+// Pendulum envs the one below; the entry that picks one, or single steps, is at the end of the file.
 //
 // It gives what n_steps calls of mrl_rollout_step give (same per-env streams: seeds are affine
 // in the step number), except that the finished-episode list is appended in the order in which
@@ -40,202 +31,8 @@ extern template int launch_collect16_t<128, 2>(mrl_ctx *, const mrl_rollout *, c
 extern template int launch_collect16_t<256, 1>(mrl_ctx *, const mrl_rollout *, const CollectArgs &, int32_t *);
 extern template int launch_collect16_t<256, 2>(mrl_ctx *, const mrl_rollout *, const CollectArgs &, int32_t *);
 
-template <class E, int H, int ACT, bool GAUSS>
-__global__ __launch_bounds__(E::THREADS) void collect_kernel(CollectArgs a) {
-    using S = Stage<E>;
-    constexpr int IN = E::OBS, AW = E::ACT_W, NW = E::THREADS / WAVE;
-    // the critic runs on the six wavefronts that do not share a SIMD with wavefront 0 (1, 2, 3, 5, 6,
-    // 7: two per SIMD, so that one's MFMAs cover the other's loads and epilogues; wavefront 0's solver
-    // keeps its SIMD's issue slots to itself); its eight column tiles are dealt out 3 / 3 / 2 per SIMD
-    constexpr int CRITIC_TPW = 2, CRITIC_WAVES = 6, CRITIC_T = CRITIC_WAVES * WAVE;
-    static_assert(E::EPB == PR && E::THREADS == 2 * H && NW == 8 && H == 256, "one 32-row policy tile per block");
-    static_assert(IN <= PIN_MAX && AW <= PA_MAX && E::DETECT_TASKS > 0, "policy tile limits; split-off detection");
-    __shared__ float rows[PR * S::STRIDE];
-    __shared__ float xs[PR * XS_LD];
-    __shared__ __align__(16) float w2s[2][HEAD_LDS(H)];
-    __shared__ float logits[PR * (PA_MAX + 1)];
-    __shared__ float vals[PR];
-    __shared__ float act[PR * PA_MAX];
-    __shared__ float shapes[E::NSHAPE];
-    __shared__ unsigned long long was_reset;
-    __shared__ unsigned sync_critic, sync_detect, sync_failed;
-    __shared__ int ncontacts[PR];   // an env's contact count after the merge of its lists (-1: detect again)
-    __shared__ float hTc[H * HT_LD];   // the critic's activation tile (live during the env step)
-    // the actor's activation tile and the env step's contact scratch are never live together
-    constexpr int LIST_F = detect_list_floats<E>() + 1;
-    constexpr int ENV_F = PR * S::CSTRIDE + LIST_F + detect_count_ints<E>();
-    __shared__ float overlay[cmax<H * HT_LD, ENV_F>()];
-    float *cts = overlay, *dlist = cts + PR * S::CSTRIDE;
-    int *dcount = reinterpret_cast<int *>(dlist + LIST_F);
-
-    const int t = threadIdx.x;
-    const int env0 = blockIdx.x * PR;
-    const int nenv = min(PR, a.n_envs - env0);
-    const int N = a.n_envs;
-    float *gbase = a.states + (size_t)env0 * E::STATE;
-
-    S::in(rows, gbase, nenv, t);
-    for (int i = t; i < E::NSHAPE; i += E::THREADS) shapes[i] = a.shapes[i];
-    {
-        const int net = t / H;
-        const float *p = net ? a.critic_p : a.actor_p;
-        stage_head(p + IN * H + H + H * H + H, H, net ? 1 : a.A, GAUSS && net == 0, w2s[net], t % H, H);
-    }
-    if (t == 0) {
-        was_reset = 0;
-        sync_critic = 0;
-        sync_detect = 0;
-        sync_failed = 0;
-    }
-    if (t < PR) ncontacts[t] = 0;   // read by the solver also when the detection's wait gave up
-    __syncthreads();
-    // wavefront 0, lane = env slot: the env's running episode return and length stay in registers
-    const bool owner = t < nenv;
-    float ep_return = owner ? a.acc.ep_return[env0 + t] : 0.0f;
-    float ep_length = owner ? a.acc.ep_length[env0 + t] : 0.0f;
-    static_assert((E::DETECT_TASKS + 1) / 2 <= NW - 1, "two detection tasks per wavefront besides wavefront 0");
-
-    // Per step: every wavefront runs the actor (the action is what the env step waits for); then
-    // wavefront 0 samples and steps the envs, wavefronts 1 .. 7 detect their contacts, and all of
-    // these but wavefront 4 go on to run the critic, whose value is only stored -- off the critical path.
-    for (int k = 0; k < a.n_steps; ++k) {
-        // Nothing but the rows is carried from one step to the next: the thread index, the block's
-        // env count and the parameter pointers pass through empty asm statements at the top of each
-        // step, so the optimiser cannot keep what it derives from them (addresses, predicates, the
-        // step-invariant operand values) live through the env step, whose solver needs the registers.
-        int tid = t, ne = __builtin_amdgcn_readfirstlane(nenv), A = __builtin_amdgcn_readfirstlane(a.A), zero = 0;
-        asm volatile("" : "+v"(tid), "+s"(zero), "+s"(ne), "+s"(A) : : "memory");
-        const float *pa = a.actor_p + zero, *pc = a.critic_p + zero;
-        const size_t row = (size_t)(a.t0 + k) * N + env0;   // this block's slice of rollout row t
-        const uint32_t sseed = a.sample_seed + (uint32_t)k * a.sample_stride;
-        const int wave = tid / WAVE, lane = tid % WAVE;
-        // the barriers of the wavefront groups, rebuilt every step from the step number (the critic's
-        // hidden stack meets three times per step, the detection once), so that nothing of them is
-        // carried through the env step in registers
-        WaveGroupSync critic_sync{&sync_critic, (unsigned)k * 3u * CRITIC_WAVES, (unsigned)CRITIC_WAVES, &sync_failed, a.spin_limit};
-        WaveGroupSync detect_sync{&sync_detect, (unsigned)k * 2u * (NW - 1), (unsigned)(NW - 1), &sync_failed, a.spin_limit};
-        // ---- actor, all wavefronts
-        {
-            HiddenOperands<H, 1, 32> ops;
-            ops.load(pa, IN, tid);
-            for (int i = tid; i < PR * IN; i += E::THREADS) {
-                const int r = i / IN, c = i - r * IN;
-                float v = 0.0f;
-                if (r < ne) {
-                    v = rows[r * S::STRIDE + c];
-                    a.r_obs[row * IN + i] = v;
-                }
-                xs[r * XS_LD + c] = v;
-            }
-            __syncthreads();
-            hidden_stack<H, ACT, 1, 32, true>(pa, IN, xs, overlay, overlay, TileCache{}, ops, tid);
-            head<H>(w2s[0], A, overlay, logits, PA_MAX + 1, tid, E::THREADS);
-            __syncthreads();   // logits complete; the actor's tile is dead from here on
-        }
-        if (wave == 0) {
-            // ---- sample, then the env step of env_block.hpp with the contacts of wavefronts 1 .. 3
-            typename E::Carry carry{};
-            if (lane < ne) {
-                const int i = env0 + lane;
-                float logp;
-                if (GAUSS) {
-                    float av[PA_MAX];
-                    logp = sample_gaussian(logits + lane * (PA_MAX + 1), w2s[0] + HEAD_LOG_STD(H), A, sseed, i, av);
-                    for (int j = 0; j < A; ++j) {
-                        act[lane * AW + j] = av[j];
-                        a.r_actions[(row + lane) * AW + j] = av[j];
-                    }
-                } else {
-                    int sel;
-                    sample_categorical_few(logits + lane * (PA_MAX + 1), A, sseed, i, sel, logp);
-                    act[lane] = (float)sel;
-                    a.r_actions[row + lane] = (float)sel;
-                }
-                a.r_logp[row + lane] = logp;
-                carry = E::step_begin(rows + lane * S::STRIDE, i, act + lane * AW, shapes);
-            }
-            // (the detecting wavefronts meet twice: lists complete, then every list moved to its place in its env's list)
-            detect_sync.target += 2 * detect_sync.nwaves;
-            detect_sync.wait_for(detect_sync.target);
-            bool finished = false;
-            int slot = 0;
-            float fin_return = 0.0f, fin_length = 0.0f;
-            if (lane < ne) {
-                float *mine = cts + lane * S::CSTRIDE;
-                const int n = ncontacts[lane];
-                float r, d;
-                E::step_finish(rows + lane * S::STRIDE, mine, n, shapes, carry, r, d);
-                // rollout row t and the episode accounting of account(), on the running sums that
-                // this lane carries for its env
-                a.r_rewards[row + lane] = r;
-                a.r_dones[row + lane] = d;
-                ep_return = ep_return + r;
-                ep_length = ep_length + 1.0f;
-                finished = d > 0.5f;
-                if (finished) {
-                    // the slot in the finished-episode list comes back from L2 while the row is rebuilt
-                    slot = atomicAdd(a.acc.done_count, 1);
-                    fin_return = ep_return;
-                    fin_length = ep_length;
-                    ep_return = 0.0f;
-                    ep_length = 0.0f;
-                }
-            }
-            reset_rows<E>(rows, &was_reset, __ballot(finished), a.reset_seed + (uint64_t)k * a.reset_stride, env0, lane);
-            if (finished && slot < a.acc.done_cap) {
-                a.acc.done_returns[slot] = fin_return;
-                a.acc.done_lengths[slot] = fin_length;
-            }
-        } else {
-            // ---- contact detection: one (body, vertex) task per half of wavefronts 1 .. 7
-            const int task = (wave - 1) * 2 + lane / (WAVE / 2), e = lane % (WAVE / 2);
-            if (task < E::DETECT_TASKS && e < ne) detect_vertex_task<E>(rows, shapes, dlist, dcount, task, e);
-            // the lists are merged by the lanes that made them, all at once, instead of one after the other by
-            // the solver's wavefront: once every list of the block is in, each lane moves its own
-            detect_sync();
-            if (task < E::DETECT_TASKS && e < ne) {
-                const int n = merge_vertex_list_of_task<E>(dlist, dcount, e, task, cts + e * S::CSTRIDE);
-                if (task == 0) ncontacts[e] = n;
-            }
-            detect_sync.arrive();
-            if (wave != 4) {
-                // ---- critic, on its own barrier: member g = 0 .. 5 of the group is wavefront g + 1
-                // (g < 3) or g + 2; members g and g + 3 share a SIMD and take tiles {2, 1}, {2, 1}, {1, 1}
-                const int g = wave < 4 ? wave - 1 : wave - 2;
-                const int tl = g * WAVE + lane;   // index among the critic's threads
-                const int tile0 = g < 2 ? 2 * g : g + 2, tiles = g < 2 ? 2 : 1;
-                HiddenOperands<H, CRITIC_TPW, 16> ops;
-                ops.load(pc, IN, tl, tile0, tiles);
-                hidden_stack<H, ACT, CRITIC_TPW, 16, true>(pc, IN, xs, hTc, hTc, TileCache{}, ops, tl, critic_sync);
-                head<H>(w2s[1], 1, hTc, vals, 1, tl, CRITIC_T);
-            }
-        }
-        __syncthreads();   // env step done, values complete
-        if (tid < ne) a.r_values[row + tid] = vals[tid];
-        // a wait that gave up: the block's results are void from here on; leave the loop (every
-        // thread reads the same word after the barrier) and end normally
-        if (sync_failed != 0u) break;
-    }
-    if (sync_failed != 0u) {
-        // a wait gave up: the step in progress ran on data that was never produced.  Nothing of it is
-        // stored: rows, observations and episode sums of this block keep the values from before the launch
-        if (t == 0) *a.sync_error = 1;
-        return;
-    }
-
-    if (owner) {
-        a.acc.ep_return[env0 + t] = ep_return;
-        a.acc.ep_length[env0 + t] = ep_length;
-    }
-    for (int i = t; i < nenv * E::OBS; i += E::THREADS) {
-        const int r = i / E::OBS, c = i - r * E::OBS;
-        a.obs[(size_t)env0 * E::OBS + i] = rows[r * S::STRIDE + c];
-    }
-    S::out(rows, gbase, nenv, t, 0, E::STATE);
-}
-
 // ---------------------------------------------------------------- CartPole / Pendulum
-// The same idea for the envs whose state is a handful of floats: a workgroup of four wavefronts
+// For the envs whose state is a handful of floats, in numbers: a workgroup of four wavefronts
 // (two on the actor, two on the critic, hidden width 64, one 32-column tile each) takes its 32
 // envs through all the steps of the launch.  Each wavefront's share of the hidden layers' weights
 // is loaded into registers once, before the first step; lanes 0 .. 31 of wavefront 0 carry one
@@ -351,7 +148,6 @@ enum CollectForm {
     FORM_STEPS,      // no fused kernel: the steps are issued one by one
     FORM_WALKER,     // collect_walkers.hpp
     FORM_ROWS16,     // collect16.hpp
-    FORM_LANDER32,   // collect_kernel
     FORM_CLASSIC32   // collect_classic_kernel
 };
 struct CollectPlan {
@@ -412,12 +208,11 @@ static CollectPlan collect_plan(const mrl_rollout *r, int n_cus) {
     }
     if ((id == MRL_ENV_LUNARLANDER && !gauss) || (id == MRL_ENV_LUNARLANDER_CONTINUOUS && gauss)) {
         if (!agent_nets(r, LunarLander::OBS, 0, gauss, &p.H, &p.act)) return p;
-        // With at most 16 envs per CU the 16-row kernel (a shorter chain per step); beyond that, at hidden width
-        // 256, the 32-row kernel, whose single solver wavefront per CU steps twice the envs in the same time; the
-        // narrower nets stay with two 16-row workgroups per CU, and above those with the stand-alone kernels
-        // (from there on their env step runs one lane per env).
-        if (r->n_envs <= n_cus * PR16 || (p.H != 256 && r->n_envs <= 2 * n_cus * PR16)) p.form = FORM_ROWS16;
-        else if (p.H == 256) p.form = FORM_LANDER32;
+        // Hidden width 256: always in one launch.  The narrower nets up to 128 envs per CU, beyond which the stand-alone
+        // kernels fill the chip (their env step runs one lane per env).  us per step, one launch : two per step, at
+        // 16384 / 32768 / 65536 envs: H = 64 27 : 53, 52 : 68, 106 : 93; H = 128 35 : 59, 68 : 81, 137 : 126;
+        // H = 256 at 8192 / 32768 / 131072 (one launch with 32 rows and one lane per env : this) 33.0 : 31.5, 132 : 125, 529 : 490.
+        if (p.H == 256 || r->n_envs <= 8 * n_cus * PR16) p.form = FORM_ROWS16;
         return p;
     }
     if (id == MRL_ENV_CARTPOLE && !gauss) obs = cartpole::OBS;
@@ -507,14 +302,6 @@ int mrl_rollout_steps(mrl_ctx *ctx, const mrl_rollout *r, int t0, int n_steps, u
         else MRL_COLLECT(256);
 #undef MRL_COLLECT
         if (rc) return rc;
-    } else if (r->env_id == MRL_ENV_LUNARLANDER) {
-        const dim3 block(LunarLander::THREADS);
-        if (plan.act == 1) hipLaunchKernelGGL((collect_kernel<LunarLander, 256, 1, false>), grid, block, 0, ctx->stream, a);
-        else hipLaunchKernelGGL((collect_kernel<LunarLander, 256, 2, false>), grid, block, 0, ctx->stream, a);
-    } else if (r->env_id == MRL_ENV_LUNARLANDER_CONTINUOUS) {
-        const dim3 block(LunarLander::THREADS);
-        if (plan.act == 1) hipLaunchKernelGGL((collect_kernel<LunarLanderContinuous, 256, 1, true>), grid, block, 0, ctx->stream, a);
-        else hipLaunchKernelGGL((collect_kernel<LunarLanderContinuous, 256, 2, true>), grid, block, 0, ctx->stream, a);
     } else if (r->env_id == MRL_ENV_CARTPOLE) {
         if (plan.act == 1) hipLaunchKernelGGL((collect_classic_kernel<CartPoleSlot, 1, false>), grid, dim3(CLASSIC_THREADS), 0, ctx->stream, a, side);
         else hipLaunchKernelGGL((collect_classic_kernel<CartPoleSlot, 2, false>), grid, dim3(CLASSIC_THREADS), 0, ctx->stream, a, side);

@@ -581,11 +581,11 @@ static int env_step_impl(mrl_ctx *ctx, int env_id, int batch, float *states, con
                                autoreset ? 1 : 0, reset_seed, acc);
             break;
         case MRL_ENV_LUNARLANDER:
-            launch_phys_step<Rows16<LunarLander>>(ctx, batch, states, actions, rewards, dones, obs, ctx->ll_shapes,
+            launch_phys_step<LunarLander>(ctx, batch, states, actions, rewards, dones, obs, ctx->ll_shapes,
                                           autoreset, reset_seed, acc);
             break;
         case MRL_ENV_LUNARLANDER_CONTINUOUS:
-            launch_phys_step<Rows16<LunarLanderContinuous>>(ctx, batch, states, actions, rewards, dones, obs, ctx->ll_shapes,
+            launch_phys_step<LunarLanderContinuous>(ctx, batch, states, actions, rewards, dones, obs, ctx->ll_shapes,
                                                     autoreset, reset_seed, acc);
             break;
         case MRL_ENV_BIPEDAL:
