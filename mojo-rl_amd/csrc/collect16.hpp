@@ -33,8 +33,8 @@ struct Critic16Split {
 //                           barrier of their own.
 // Two such workgroups fit a CU (LDS, registers).  On this hardware a SIMD issues either a matrix or a vector instruction,
 // never both at once (a wavefront of dependent v_fma_f32 that shares its SIMD with a wavefront issuing v_mfma back to back
-// takes the sum of both times), so at H = 256 the second one costs what its forward passes cost (4096 : 8192 envs 21.2 :
-// 31.5 us per step); still, since the solver carries four lanes per env, two of 16 rows are ahead of one of 32 rows with one
+// takes the sum of both times), so at H = 256 the second one costs what its forward passes cost (4096 : 8192 envs 19.2 :
+// 29.2 us per step); still, since the solver carries four lanes per env, two of 16 rows are ahead of one of 32 rows with one
 // lane per env and the critic on six wavefronts (33.0).
 // us per step with one lane per env : four: 777 envs, H = 64 19.4 : 12.9 (its solver wavefront: 22 of 37 thousand cycles in
 // the physics before); 4096 envs, H = 64 18.8 : 12.6, H = 256, where the critic is the longer path, 23.9 : 21.6.

@@ -17,6 +17,7 @@
 
 namespace mrl {
 
+typedef float floatx2 __attribute__((ext_vector_type(2)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 constexpr int PR16 = 16;            // rows per tile
@@ -107,48 +108,101 @@ MRL_DEV void hidden16_layer0(const float *xs, float *hT, const Hidden16Operands<
     }
 }
 
+// a pointer that is the same in all lanes of a wavefront, in scalar registers
+MRL_DEV const float *wave_uniform(const float *p) {
+    const uint64_t u = reinterpret_cast<uint64_t>(p);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)u), hi = __builtin_amdgcn_readfirstlane((int)(u >> 32));
+    return reinterpret_cast<const float *>((uint64_t)hi << 32 | lo);
+}
+
+// Where a lane's operands of a weight row lie: byte offsets from the row's start, which stays a scalar.
+template <int NT>
+struct Tile16Lane {
+    uint32_t o, ox;
+    MRL_DEV Tile16Lane(int H, int c0, int lane) {
+        const int g = lane >> 4, n = lane & 15, col = g * H + c0;
+        o = 4u * (uint32_t)(col + (NT >= 4 ? 4 : NT) * n);
+        ox = 4u * (uint32_t)(col + 64 + (NT == 5 ? 1 : 2) * n);
+    }
+    // ahead of a block's loads: the widening of the offsets stays beside them, where it folds into the address mode
+    MRL_DEV void here() { asm("" : "+v"(o), "+v"(ox)); }
+    MRL_DEV void load(const float *row, float (&b)[NT]) const {
+        typedef const char __attribute__((address_space(1))) *Row;
+        Row r = (Row)(reinterpret_cast<const char *>(row));
+        asm("" : "+s"(r));   // (not folded into the lanes' offsets, which would make every address a 64-bit vector sum)
+        if constexpr (NT >= 4) {
+            const floatx4 v = *(const floatx4 __attribute__((address_space(1))) *)(r + o);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) b[q] = v[q];
+            if constexpr (NT == 5) b[4] = *(const float __attribute__((address_space(1))) *)(r + ox);
+            if constexpr (NT == 6) {
+                const floatx2 x = *(const floatx2 __attribute__((address_space(1))) *)(r + ox);
+                b[4] = x[0]; b[5] = x[1];
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < NT; ++q) b[q] = *(const float __attribute__((address_space(1))) *)(r + o + 4 * q);
+        }
+    }
+};
+
 // Layer 1: weights streamed from L2 one block of KB k-steps ahead of the MFMAs (KB = H / 4: all of them are in
 // `ops`, which is then left as it is); h2 [16][H + 1] receives act(layer 1) row-major.  before_h2() is called between
-// the last read of hT and the first write of h2.
+// the last read of hT and the first write of h2.  The blocks alternate between two register sets, and a load's
+// address is a scalar pair and a 32-bit lane offset: with one set copied to the other, the copies at a block's start
+// waited for its last load, and with 64-bit vector addresses they were 129 instructions beside the 40 MFMAs of a
+// five-tile block (now 56), on a SIMD that issues one or the other.  us per rollout step before : now, hidden width 256:
+// LunarLander 4096 envs 21.2 : 19.2, 8192 envs 31.5 : 29.2, CartPole 1024 envs 13.0 : 10.8; width 128, LunarLander 4096
+// envs 14.5 : 13.7.
 template <int H, int IN, int ACT, int NT, int KB, class Before>
 MRL_DEV void hidden16_layer1(const float *__restrict__ p, const float *hT, float *h2, Hidden16Operands<H, IN, NT, KB> &ops,
                              int c0, int lane, Before &&before_h2) {
-    static_assert((H / 4) % KB == 0, "whole blocks of k-steps");
+    constexpr int NBLK = H / (4 * KB);
+    static_assert((H / 4) % KB == 0 && (NBLK == 1 || NBLK % 2 == 0), "whole pairs of blocks of k-steps");
     const int g = lane >> 4, n = lane & 15;
     const float *W1 = p + IN * H + H;
     floatx4 c[NT];
 #pragma unroll
     for (int q = 0; q < NT; ++q) c[q] = floatx4{0};
-    float a[KB], na[KB], nb[KB][NT];
+    auto fetch = [&](const float *ht, const float *w, Tile16Lane<NT> &at, float (&a)[KB], float (&b)[KB][NT]) {
+        at.here();
 #pragma unroll
-    for (int j = 0; j < KB; ++j) a[j] = hT[(4 * j + g) * HT16_LD + n];
-    constexpr int NBLK = H / (4 * KB);
-    for (int blk = 0; blk < NBLK; ++blk) {
-        const bool more = blk + 1 < NBLK;
-        if (more) {
-#pragma unroll
-            for (int j = 0; j < KB; ++j) {
-                const int k = 4 * ((blk + 1) * KB + j) + g;
-                na[j] = hT[k * HT16_LD + n];
-                tile16_load_b<NT>(W1 + k * H + c0, n, nb[j]);
-            }
+        for (int j = 0; j < KB; ++j) {
+            a[j] = ht[4 * j * HT16_LD];
+            at.load(w + 4 * j * H, b[j]);
         }
-        // keep the next block's loads ahead of this block's MFMAs
-        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto product = [&](const float (&a)[KB], const float (&b)[KB][NT]) {
+        __builtin_amdgcn_sched_barrier(0);   // the loads above stay ahead of these MFMAs
 #pragma unroll
         for (int j = 0; j < KB; ++j) {
 #pragma unroll
-            for (int q = 0; q < NT; ++q)
-                c[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], ops.bv[j][q], c[q], 0, 0, 0);
+            for (int q = 0; q < NT; ++q) c[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j], b[j][q], c[q], 0, 0, 0);
         }
-        if (more) {
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    const float *ht = hT + g * HT16_LD + n;
+    float a[KB];
 #pragma unroll
-            for (int j = 0; j < KB; ++j) {
-                a[j] = na[j];
-#pragma unroll
-                for (int q = 0; q < NT; ++q) ops.bv[j][q] = nb[j][q];
-            }
+    for (int j = 0; j < KB; ++j) a[j] = ht[4 * j * HT16_LD];
+    if constexpr (NBLK == 1) {
+        product(a, ops.bv);
+    } else {
+        Tile16Lane<NT> at(H, c0, lane);
+        W1 = wave_uniform(W1);
+        float na[KB], nb[KB][NT];
+        constexpr int HT_BLK = 4 * KB * HT16_LD, W_BLK = 4 * KB * H;
+        for (int blk = 2; blk < NBLK; blk += 2) {
+            fetch(ht + HT_BLK, W1 + W_BLK, at, na, nb);
+            product(a, ops.bv);
+            fetch(ht + 2 * HT_BLK, W1 + 2 * W_BLK, at, a, ops.bv);
+            product(na, nb);
+            ht += 2 * HT_BLK;
+            W1 += 2 * W_BLK;
         }
+        fetch(ht + HT_BLK, W1 + W_BLK, at, na, nb);
+        product(a, ops.bv);
+        product(na, nb);
     }
     before_h2();
 #pragma unroll
