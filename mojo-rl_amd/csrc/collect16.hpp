@@ -49,7 +49,7 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
     constexpr Critic16Split<H> CS{};
     constexpr int CAP = 3;      // records per (body, vertex) list: two contacts, the third signals overflow
     constexpr int KBA = 8;      // k-steps of layer-1 weights fetched ahead
-    static_assert(IN <= PIN_MAX && AW <= PA_MAX && E::DETECT_TASKS > 0 && E::DETECT_TASKS <= 24, "tile limits; split-off detection");
+    static_assert(IN <= PIN_MAX && AW <= PA_MAX && E::DETECT_TASKS >= 12 && E::DETECT_TASKS <= 16, "tile limits; split-off detection");
     __shared__ float rows[R * S::STRIDE];
     __shared__ float xs[R * XS_LD];
     __shared__ __align__(16) float w2a[HEAD_LDS(H)];
@@ -58,6 +58,7 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
     __shared__ float vals[R];
     __shared__ float act[R * PA_MAX];
     __shared__ float shapes[E::NSHAPE];
+    __shared__ ll::EngineDraw draws[R];
     __shared__ unsigned long long was_reset;
     __shared__ unsigned sync_critic, sync_detect, sync_failed;
     __shared__ float hTc[H * HT16_LD];              // the critic's activation tile (live during the env step)
@@ -129,32 +130,43 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
             head16<H>(w2a, A, overlay, logits, PA_MAX + 1, tid, T);
             __syncthreads();   // logits complete; the actor's tile is dead from here on
         }
+        if (vw == 0) {   // ---- sample
+            const int e = lane >> 2;
+            const bool first = (lane & 3) == 0;
+            if (e < ne) {
+                const int i = env0 + e;
+                const float *lg = logits + e * (PA_MAX + 1);
+                if (GAUSS) {
+                    for (int j = lane & 3; j < A; j += 4) {   // (one component a lane)
+                        float av;
+                        sample_gaussian_part(lg + j, w2a + HEAD_LOG_STD(H) + j, 1, A, j, sseed, i, &av);
+                        act[e * AW + j] = av;
+                    }
+                } else if (A <= 4) {
+                    const int sel = sample_categorical_quad(lg, A, sseed, i, lane & 3);
+                    if (first) act[e] = (float)sel;
+                } else if (first) {
+                    int sel;
+                    float logp;
+                    sample_categorical_few(lg, A, sseed, i, sel, logp);
+                    act[e] = (float)sel;
+                }
+            }
+        } else if (vw == 3 && lane < ne) {   // ---- what the engines need whatever the action is
+            draws[lane] = ll::engine_draw(rows + lane * S::STRIDE, env0 + lane);
+        }
+        {   // ---- contact detection: a (body, vertex) task of env slot lane % 16 each, four a helper, the solver the rest
+            const int task = (vw == 0 ? 12 : 4 * (vw - 1)) + lane / R, e = lane % R;
+            if (task < E::DETECT_TASKS && e < ne) detect_vertex_task<E, CAP>(rows, shapes, dlist, dcount, task, e);
+        }
         if (vw == 0) {
-            // ---- sample, then the env step of env_block.hpp with the contacts the helpers detect
+            // ---- the env step of env_block.hpp with the contacts detected
             typename E::Carry carry{};
             const int e = lane >> 2;
             const bool first = (lane & 3) == 0 && e < ne;
-            if (first) {
-                const int i = env0 + e;
-                float logp;
-                if (GAUSS) {
-                    float av[PA_MAX];
-                    logp = sample_gaussian(logits + e * (PA_MAX + 1), w2a + HEAD_LOG_STD(H), A, sseed, i, av);
-                    for (int j = 0; j < A; ++j) {
-                        act[e * AW + j] = av[j];
-                        a.r_actions[(row + e) * AW + j] = av[j];
-                    }
-                } else {
-                    int sel;
-                    sample_categorical_few(logits + e * (PA_MAX + 1), A, sseed, i, sel, logp);
-                    act[e] = (float)sel;
-                    a.r_actions[row + e] = (float)sel;
-                }
-                a.r_logp[row + e] = logp;
-                carry = E::step_begin(rows + e * S::STRIDE, i, act + e * AW, shapes);
-            }
             detect_sync.target += detect_sync.nwaves;
             detect_sync.wait_for(detect_sync.target);
+            if (first) carry = E::step_begin(rows + e * S::STRIDE, env0 + e, act + e * AW, shapes, draws + e);
             float r = 0.0f, d = 0.0f;
             step_finish_quads<E, CAP>(rows, cts, shapes, dlist, dcount, carry, wired != 0, lane, ne, r, d);
             bool finished = false;
@@ -178,13 +190,24 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
             wired |= (int)((fin >> e) & 1ull);
             reset_rows<E>(rows, &was_reset, fin, a.reset_seed + (uint64_t)k * a.reset_stride, env0, lane);
         } else {
-            // ---- contact detection: (body, vertex) task m * 4 + lane / 16 of env slot lane % 16, a
-            // second pass on helper 0 for the tasks beyond twelve
-            const int m = vw - 1, e = lane % R;
-            if (e < ne)
-                for (int task = m * 4 + lane / R; task < E::DETECT_TASKS; task += 12)
-                    detect_vertex_task<E, CAP>(rows, shapes, dlist, dcount, task, e);
+            // ---- the draw once more, for the rollout's action and log-probability, which nothing of the step waits for
+            const int m = vw - 1;
             detect_sync.arrive();
+            if (m == 0 && lane < ne) {
+                const int i = env0 + lane;
+                const float *lg = logits + lane * (PA_MAX + 1);
+                float logp;
+                if (GAUSS) {
+                    float av[PA_MAX];
+                    logp = sample_gaussian(lg, w2a + HEAD_LOG_STD(H), A, sseed, i, av);
+                    for (int j = 0; j < A; ++j) a.r_actions[(row + lane) * AW + j] = av[j];
+                } else {
+                    int sel;
+                    sample_categorical_few(lg, A, sseed, i, sel, logp);
+                    a.r_actions[row + lane] = (float)sel;
+                }
+                a.r_logp[row + lane] = logp;
+            }
             // ---- critic on the three helpers, at their own barrier
             const int tl = m * WAVE + lane;
             auto critic = [&](auto tiles, int c0) {

@@ -74,8 +74,8 @@ struct LunarLander {
     }
     static constexpr bool LANES_PHYSICS = false;   // (BipedalWalker: the physics by one lane per body)
     using Carry = ll::StepCarry;
-    static MRL_DEV Carry step_begin(float *row, int env, const float *a, const float *shapes) {
-        return ll::step_begin(row, env, (int)a[0], shapes);
+    static MRL_DEV Carry step_begin(float *row, int env, const float *a, const float *shapes, const ll::EngineDraw *draw = nullptr) {
+        return ll::step_begin(row, env, (int)a[0], shapes, draw);
     }
     static MRL_DEV void step_finish(float *row, float *cts, int n, const float *shapes, const Carry &c, float &r,
                                     float &d) {
@@ -101,8 +101,8 @@ struct LunarLanderContinuous : LunarLander {
         const Carry c = ll::step_begin_continuous(row, env, a, shapes);
         ll::step_finish(row, cts, -1, shapes, c, r, d);
     }
-    static MRL_DEV Carry step_begin(float *row, int env, const float *a, const float *shapes) {
-        return ll::step_begin_continuous(row, env, a, shapes);
+    static MRL_DEV Carry step_begin(float *row, int env, const float *a, const float *shapes, const ll::EngineDraw *draw = nullptr) {
+        return ll::step_begin_continuous(row, env, a, shapes, draw);
     }
 };
 

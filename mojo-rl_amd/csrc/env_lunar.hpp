@@ -247,17 +247,31 @@ MRL_DEV void reset_row_wave(float *row, uint64_t cseed, int lane) {
     __builtin_amdgcn_wave_barrier();
 }
 
+// What the engines need that does not hang on the action: a kernel may work it out on another wavefront.
+struct EngineDraw {
+    double tip_x, tip_y, dispersion_x, dispersion_y;
+};
+MRL_DEV EngineDraw engine_draw(const float *row, int env, int step_count) {
+    EngineDraw d;
+    ::sincos((double)row[L::BODIES_OFF + IDX_ANGLE], &d.tip_x, &d.tip_y);
+    Uniform4 rv = philox_uniform4((uint64_t)((int64_t)env + 12345), (uint64_t)step_count, 0);
+    d.dispersion_x = ((double)rv.v[0] * 2.0 - 1.0) / SCALE;
+    d.dispersion_y = ((double)rv.v[1] * 2.0 - 1.0) / SCALE;
+    return d;
+}
+MRL_DEV EngineDraw engine_draw(const float *row, int env) {
+    return engine_draw(row, env, (int)row[L::META_OFF + META_STEP]);
+}
+
+// given: the step's EngineDraw (null: taken here, if an engine fires)
 MRL_DEV void apply_engines(float *row, int env, int step_count, double m_power, double s_power,
-                           double direction) {
+                           double direction, const EngineDraw *given) {
     if (m_power == 0.0 && s_power == 0.0) return;
     float *B = row + L::BODIES_OFF;
-    double angle = B[IDX_ANGLE], vx = B[IDX_VX], vy = B[IDX_VY], omega = B[IDX_OMEGA];
-    double tip_x, tip_y;
-    ::sincos(angle, &tip_x, &tip_y);
+    double vx = B[IDX_VX], vy = B[IDX_VY], omega = B[IDX_OMEGA];
+    const EngineDraw draw = given != nullptr ? *given : engine_draw(row, env, step_count);
+    const double tip_x = draw.tip_x, tip_y = draw.tip_y, dispersion_x = draw.dispersion_x, dispersion_y = draw.dispersion_y;
     double side_x = -tip_y, side_y = tip_x;
-    Uniform4 rv = philox_uniform4((uint64_t)((int64_t)env + 12345), (uint64_t)step_count, 0);
-    double dispersion_x = ((double)rv.v[0] * 2.0 - 1.0) / SCALE;
-    double dispersion_y = ((double)rv.v[1] * 2.0 - 1.0) / SCALE;
     double dvx = 0.0, dvy = 0.0, domega = 0.0;
     if (m_power > 0.0) {
         double main_y_offset = 4.0 / SCALE;
@@ -354,7 +368,7 @@ MRL_DEV void physics_lanes(float *row, float *contacts, int n, int lane) {
     if (has) lane_body_store<L>(B, row, b);
 }
 
-MRL_DEV StepCarry step_begin(float *row, int env, int action, const float *shapes) {
+MRL_DEV StepCarry step_begin(float *row, int env, int action, const float *shapes, const EngineDraw *draw = nullptr) {
     StepCarry c;
     c.skip = row[L::META_OFF + META_DONE] > 0.5f;
     c.step_count = (int)row[L::META_OFF + META_STEP];
@@ -365,7 +379,7 @@ MRL_DEV StepCarry step_begin(float *row, int env, int action, const float *shape
     else if (action == 3) { c.s_power = 1.0; direction = 1.0; }
     if (!c.skip) {
         apply_wind(row, c.step_count, shapes);
-        apply_engines(row, env, c.step_count, c.m_power, c.s_power, direction);
+        apply_engines(row, env, c.step_count, c.m_power, c.s_power, direction, draw);
     }
     return c;
 }
@@ -374,7 +388,8 @@ MRL_DEV StepCarry step_begin(float *row, int env, int action, const float *shape
 // fp64 like the rest of the engine arithmetic): a[0] in [-1, 1] is the main throttle, remapped to
 // (a0 + 1) / 2 and clipped to [0, 1]; a[1] clipped to [-1, 1] fires the left (< -0.5) or right
 // (> 0.5) engine with power (|a1| - 0.5) * 2.  Both engines can fire in one step.
-MRL_DEV StepCarry step_begin_continuous(float *row, int env, const float *a, const float *shapes) {
+MRL_DEV StepCarry step_begin_continuous(float *row, int env, const float *a, const float *shapes,
+                                        const EngineDraw *draw = nullptr) {
     StepCarry c;
     c.skip = row[L::META_OFF + META_DONE] > 0.5f;
     c.step_count = (int)row[L::META_OFF + META_STEP];
@@ -389,7 +404,7 @@ MRL_DEV StepCarry step_begin_continuous(float *row, int env, const float *a, con
     c.m_power = m_power; c.s_power = s_power;
     if (!c.skip) {
         apply_wind(row, c.step_count, shapes);
-        apply_engines(row, env, c.step_count, m_power, s_power, direction);
+        apply_engines(row, env, c.step_count, m_power, s_power, direction, draw);
     }
     return c;
 }

@@ -148,6 +148,11 @@ MRL_DEV float log32(float x) {
 }
 
 // whether any active lane says so, straight from the compare
+// the value of lane L of every four
+template <int L>
+MRL_DEV float quad_bcast(float x) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), L * 0x55, 0xF, 0xF, true));
+}
 MRL_DEV bool any_lane(bool p) { return __builtin_amdgcn_ballot_w64(p) != 0; }
 
 // x / d for a divisor that is divided by again and again (a joint's summed inverse inertia, a contact's

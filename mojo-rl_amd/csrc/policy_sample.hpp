@@ -65,6 +65,27 @@ MRL_DEV void sample_categorical_few(const float *l, int A, uint32_t seed, int i,
     logp = log32(pr + 1e-8f);
 }
 
+// The action alone, for at most four actions, by the four lanes of an env (l: lane & 3, all four active): each takes the
+// exponential and the quotient of one action, the sums run over the actions in the same order, and every lane returns the
+// drawn action.  Bit for bit the draw of the two above: an action beyond A is minus infinity to the maximum and adds 0.
+MRL_DEV int sample_categorical_quad(const float *logits, int A, uint32_t seed, int i, int l) {
+    uint32_t rng = seed ^ ((uint32_t)i * 2654435761u);
+    rng = xorshift32(rng);
+    const float u = random_uniform(rng);
+    const float mine = l < A ? logits[l] : -__builtin_inff();
+    float max_logit = quad_bcast<0>(mine);
+    auto larger = [&](float x) { if (x > max_logit) max_logit = x; };
+    larger(quad_bcast<1>(mine));
+    larger(quad_bcast<2>(mine));
+    larger(quad_bcast<3>(mine));
+    const float e = l < A ? exp32(mine - max_logit) : 0.0f;
+    const float sum_exp = quad_bcast<0>(e) + quad_bcast<1>(e) + quad_bcast<2>(e) + quad_bcast<3>(e);
+    const float prob = e / sum_exp;
+    const float c0 = quad_bcast<0>(prob), c1 = c0 + quad_bcast<1>(prob);
+    const float c2 = c1 + quad_bcast<2>(prob), c3 = c2 + quad_bcast<3>(prob);
+    return u < c0 ? 0 : A > 1 && u < c1 ? 1 : A > 2 && u < c2 ? 2 : A > 3 && u < c3 ? 3 : 0;
+}
+
 // Gaussian sampling (deep_agents/ppo/kernels.mojo:12-98) of components j0 .. j0 + m of an action
 // with A components: one Philox stream per (env, component), Box-Muller, clamped log_std;
 // returns the summed log-probability of those components and leaves them in act[0 .. m).
