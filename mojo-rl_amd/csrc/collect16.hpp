@@ -16,8 +16,8 @@ namespace mrl {
 template <int A, int B>
 constexpr int cmax() { return A > B ? A : B; }
 
-// column tiles of 16 of the critic on the three helpers: helper 0, which has a second detection pass, never more
-// than the others
+// column tiles of 16 of the critic on the three helpers: helper 0, which draws the action once more, never more than the
+// others
 template <int H>
 struct Critic16Split {
     static constexpr int TILES = H / 16;
@@ -28,16 +28,20 @@ struct Critic16Split {
 // A workgroup of four wavefronts and 16 envs.  A step is a chain -- actor on the matrix cores, then sampling and the env
 // step on ONE wavefront's vector unit --, and beside it the critic, whose value is only stored.
 //   all four wavefronts     actor  OBS -> H -> H -> A, 64 columns each;
-//   the solver wavefront    sampling, env step (four lanes per env, one per body: env_lunar.hpp), accounting, resets;
-//   the other three         contact detection, then the critic (H = 256: 80 / 96 / 80 columns) at a
-//                           barrier of their own.
+//   the solver wavefront    sampling (four lanes per env), two of the fourteen detection tasks, env step (four lanes per
+//                           env, one per body: env_lunar.hpp), accounting, resets;
+//   the other three         contact detection, what the engines need whatever the action is, the action's log-probability,
+//                           then the critic (H = 256: 80 / 96 / 80 columns) at a barrier of their own.
 // Two such workgroups fit a CU (LDS, registers).  On this hardware a SIMD issues either a matrix or a vector instruction,
 // never both at once (a wavefront of dependent v_fma_f32 that shares its SIMD with a wavefront issuing v_mfma back to back
-// takes the sum of both times), so at H = 256 the second one costs what its forward passes cost (4096 : 8192 envs 19.2 :
-// 29.2 us per step); still, since the solver carries four lanes per env, two of 16 rows are ahead of one of 32 rows with one
+// takes the sum of both times), so at H = 256 the second one costs what its forward passes cost (4096 : 8192 envs 18.7 :
+// 29.0 us per step); still, since the solver carries four lanes per env, two of 16 rows are ahead of one of 32 rows with one
 // lane per env and the critic on six wavefronts (33.0).
 // us per step with one lane per env : four: 777 envs, H = 64 19.4 : 12.9 (its solver wavefront: 22 of 37 thousand cycles in
-// the physics before); 4096 envs, H = 64 18.8 : 12.6, H = 256, where the critic is the longer path, 23.9 : 21.6.
+// the physics before); 4096 envs, H = 64 18.8 : 12.6, H = 256, where the critic is the longer path, 23.9 : 21.6.  The engines'
+// sines and the log-probability off the solver, its detection in one pass of all four wavefronts: H = 64, 777 envs
+// 11.46 : 11.26, 4096 envs 11.86 : 11.55 (thousand cycles of a step there: actor 5.0, sample 1.1, detection 3.5, wait 0.8,
+// engines 1.6, physics and tail 12, reset 1).
 // The solver wavefront is 0 in the lower half of the grid and 2 in the upper half: workgroups i and
 // i + grid / 2 share a CU when the grid is twice the CU count, and their solvers then sit on
 // different SIMDs.
@@ -286,7 +290,8 @@ struct PendulumSlot {
 // log-probability, which nothing of the step waits for, is taken by another wavefront beside the env step.  Lanes
 // 0 .. 15 of wavefront 0 carry one env each in registers.  Up to hidden width 128 the hidden layers' weights stay in
 // registers for the whole launch (the bound of four wavefronts per SIMD lets two workgroups share a CU).
-// CartPole, hidden width 64, us per step at 1024 / 4096 envs: 32 rows 4.88 / 4.66, this form 3.04 / 3.11; hidden width
+// CartPole, hidden width 64, us per step at 1024 / 4096 envs: 32 rows 4.88 / 4.66, this form 3.04 / 3.11 (2.50 at 1024 envs
+// with the head's sums in DPP instructions); hidden width
 // 128 and 256 as a policy and an env-step launch per step 16.9 and 19.4, in this form 5.95 and 13.4.  (The critic a
 // phase behind the actor, its second layer beside the env step: 3.30 at width 64, 7.2 at 128 -- on one SIMD matrix and
 // vector instructions of different wavefronts take turns --, 12.5 at 256.)

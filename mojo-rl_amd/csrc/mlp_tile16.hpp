@@ -228,12 +228,32 @@ MRL_DEV void hidden_stack16(const float *__restrict__ p, const float *xs, float 
     sync();
 }
 
+// Sum over TPR neighbouring lanes (all of a wavefront's rows of 16 active or none of a group), added in the order of the
+// exchanges with lane ^ TPR / 2, ..., lane ^ 1, without the LDS crossbar: once lanes i and i ^ 8 hold the same sum, what
+// stands four lanes back in the row of 16 is what stands at i ^ 4.
+template <int CTRL>
+MRL_DEV float dpp_add(float x) {
+    return x + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, true));
+}
+template <int TPR>
+MRL_DEV float butterfly_sum(float x) {
+    static_assert(TPR == 4 || TPR == 8 || TPR == 16, "a quad, half a row or a row of lanes");
+    if constexpr (TPR == 16) x = dpp_add<0x128>(x);                       // row_ror:8
+    if constexpr (TPR == 16) x = dpp_add<0x124>(x);                       // row_ror:4
+    if constexpr (TPR == 8) x += __shfl_xor(x, 4, 64);
+    x = dpp_add<0x4E>(x);                                                 // quad_perm [2, 3, 0, 1]
+    return dpp_add<0xB1>(x);                                              // quad_perm [1, 0, 3, 2]
+}
+
 // head_rows of mlp_tile.hpp for 16 rows; PITCH = floats per padded weight row in w2s (PA_MAX for a
 // head staged with stage_head, 1 for a single-output head stored as a plain column followed by its
-// bias).  Same lane split per row and same butterfly, hence the same bits as head_rows.
+// bias).  Same lane split per row and same butterfly, hence the same bits as head_rows.  Serial latency bounds it (2.8 to 3.7
+// thousand cycles of a rollout step, of 24 to 46): all of a lane's operands are requested ahead of its products, and the
+// sums go over the lanes in DPP instructions instead of the LDS crossbar; CartPole, hidden width 64, 1024 envs 2.70 : 2.50
+// us per step, LunarLander, hidden width 256, 4096 envs 19.3 : 18.7.
 template <int H, int NA, int PITCH>
 MRL_DEV void head_rows16(const float *w2s, int A, const float *h2, float *out, int out_ld, int t, int nthreads) {
-    constexpr int CP = 16, TPR = H / CP;
+    constexpr int CP = 16, TPR = H / CP, BLK = NA == 8 ? 8 : 16;
     static_assert(64 % TPR == 0, "the lanes of a row sit in one wavefront");
     static_assert(NA == 1 || (PITCH == PA_MAX && (NA == 4 || NA == 8)), "one float, one float4 or two per padded row");
     const float *b2 = w2s + H * PITCH;
@@ -242,28 +262,35 @@ MRL_DEV void head_rows16(const float *w2s, int A, const float *h2, float *out, i
         float acc[NA];
 #pragma unroll
         for (int a = 0; a < NA; ++a) acc[a] = 0.0f;
-#pragma unroll 8
-        for (int i = 0; i < CP; ++i) {
-            const int nn = part * CP + ((i + part) & (CP - 1));
-            const float hv = h2[r * (H + 1) + nn];
-            if (NA == 1) {
-                acc[0] = fmaf(hv, w2s[nn * PITCH], acc[0]);
-            } else {
-                const float4 wa = *reinterpret_cast<const float4 *>(w2s + nn * PITCH);
-                acc[0] = fmaf(hv, wa.x, acc[0]); acc[1] = fmaf(hv, wa.y, acc[1]);
-                acc[2] = fmaf(hv, wa.z, acc[2]); acc[3] = fmaf(hv, wa.w, acc[3]);
-                if (NA == 8) {
-                    const float4 wb = *reinterpret_cast<const float4 *>(w2s + nn * PITCH + 4);
-                    acc[4] = fmaf(hv, wb.x, acc[4]); acc[5] = fmaf(hv, wb.y, acc[5]);
-                    acc[6] = fmaf(hv, wb.z, acc[6]); acc[7] = fmaf(hv, wb.w, acc[7]);
+        // (element i is column (i + part) & 15 of the part: up to 15 - part it lies i behind the first, then 16 less)
+        const float *hp = h2 + r * (H + 1) + part * CP + part, *wp = w2s + (part * CP + part) * PITCH;
+#pragma unroll
+        for (int b = 0; b < CP; b += BLK) {
+            float hv[BLK], wv[BLK][NA];
+#pragma unroll
+            for (int j = 0; j < BLK; ++j) {
+                const int i = b + j, back = i + part < CP ? 0 : CP;
+                hv[j] = hp[i - back];
+                const float *w = wp + (i - back) * PITCH;
+                if (NA == 1) {
+                    wv[j][0] = w[0];
+                } else {
+#pragma unroll
+                    for (int a = 0; a < NA; a += 4) {
+                        const float4 x = *reinterpret_cast<const float4 *>(w + a);
+                        wv[j][a] = x.x; wv[j][a + 1] = x.y; wv[j][a + 2] = x.z; wv[j][a + 3] = x.w;
+                    }
                 }
+            }
+#pragma unroll
+            for (int j = 0; j < BLK; ++j) {
+#pragma unroll
+                for (int a = 0; a < NA; ++a) acc[a] = fmaf(hv[j], wv[j][a], acc[a]);
             }
         }
 #pragma unroll
         for (int a = 0; a < NA; ++a) {
-            float v = acc[a];
-#pragma unroll
-            for (int off = TPR / 2; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+            const float v = butterfly_sum<TPR>(acc[a]);
             if (part == 0 && a < A) out[r * out_ld + a] = v + b2[a];
         }
     }
