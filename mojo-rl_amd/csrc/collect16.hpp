@@ -34,13 +34,13 @@ struct Critic16Split {
 //                           then the critic (H = 256: 80 / 96 / 80 columns) at a barrier of their own.
 // Two such workgroups fit a CU (LDS, registers).  On this hardware a SIMD issues either a matrix or a vector instruction,
 // never both at once (a wavefront of dependent v_fma_f32 that shares its SIMD with a wavefront issuing v_mfma back to back
-// takes the sum of both times), so at H = 256 the second one costs what its forward passes cost (4096 : 8192 envs 18.7 :
-// 29.0 us per step); still, since the solver carries four lanes per env, two of 16 rows are ahead of one of 32 rows with one
+// takes the sum of both times), so at H = 256 the second one costs what its forward passes cost (4096 : 8192 envs 18.5 :
+// 27.3 us per step); still, since the solver carries four lanes per env, two of 16 rows are ahead of one of 32 rows with one
 // lane per env and the critic on six wavefronts (33.0).
 // us per step with one lane per env : four: 777 envs, H = 64 19.4 : 12.9 (its solver wavefront: 22 of 37 thousand cycles in
 // the physics before); 4096 envs, H = 64 18.8 : 12.6, H = 256, where the critic is the longer path, 23.9 : 21.6.  The engines'
 // sines and the log-probability off the solver, its detection in one pass of all four wavefronts: H = 64, 777 envs
-// 11.46 : 11.26, 4096 envs 11.86 : 11.55 (thousand cycles of a step there: actor 5.0, sample 1.1, detection 3.5, wait 0.8,
+// 11.46 : 11.26, 4096 envs 11.86 : 11.55 (11.2 since the step's first loads are no longer waited for; thousand cycles of a step there: actor 5.0, sample 1.1, detection 3.5, wait 0.8,
 // engines 1.6, physics and tail 12, reset 1).
 // The solver wavefront is 0 in the lower half of the grid and 2 in the upper half: workgroups i and
 // i + grid / 2 share a CU when the grid is twice the CU count, and their solvers then sit on
@@ -119,15 +119,7 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
         {
             Hidden16Operands<H, IN, NTA, KBA> ops;
             ops.load(pa, 16 * NTA * wave, lane);
-            for (int i = tid; i < R * IN; i += T) {
-                const int r = i / IN, c = i - r * IN;
-                float v = 0.0f;
-                if (r < ne) {
-                    v = rows[r * S::STRIDE + c];
-                    a.r_obs[row * IN + i] = v;
-                }
-                xs[r * XS_LD + c] = v;
-            }
+            stage_observations<IN, T>(xs, a.r_obs + row * IN, ne, tid, [&](int r, int c) { return rows[r * S::STRIDE + c]; });
             __syncthreads();
             BlockSync bs;
             hidden_stack16<H, IN, ACT, NTA, KBA, true>(pa, xs, overlay, overlay, ops, 16 * NTA * wave, lane, bs);

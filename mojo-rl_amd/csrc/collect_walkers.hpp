@@ -64,15 +64,7 @@ MRL_DEV void policy16_gauss(const CollectArgs &a, ObsAt obs_at, int tid, int ne,
         float *tile = tiles + net * (H * HT16_LD);
         Hidden16Operands<H, IN, NT, KBA> ops;
         ops.load(p, 16 * NT * (wave & 3), lane);
-        for (int i = tid; i < R * IN; i += T) {
-            const int r = i / IN, c = i - r * IN;
-            float v = 0.0f;
-            if (r < ne) {
-                v = obs_at(r, c);
-                a.r_obs[row * IN + i] = v;
-            }
-            xs[r * XS_LD + c] = v;
-        }
+        stage_observations<IN, T>(xs, a.r_obs + row * IN, ne, tid, obs_at);
         __syncthreads();
         BlockSync bs;
         hidden_stack16<H, IN, ACT, NT, KBA, true>(p, xs, tile, tile, ops, 16 * NT * (wave & 3), lane, bs);
@@ -203,15 +195,7 @@ __global__ __launch_bounds__(512) void collect_walker_kernel(CollectArgs a) {
         // SIMD); the critic, whose value is only stored, runs beside the solver on wavefronts 2, 3, 6 and 7 --
         // the two SIMDs that do not host wavefronts 0 and 1.  Both groups meet at bounded barriers of their
         // own, rebuilt every step from the step number.
-        for (int i = tid; i < R * IN; i += T) {
-            const int r = i / IN, c = i - r * IN;
-            float v = 0.0f;
-            if (r < ne) {
-                v = rows[r * S::STRIDE + c];
-                a.r_obs[row * IN + i] = v;
-            }
-            xs[r * XS_LD + c] = v;
-        }
+        stage_observations<IN, T>(xs, a.r_obs + row * IN, ne, tid, [&](int r, int c) { return rows[r * S::STRIDE + c]; });
         __syncthreads();
         if (wave < 4) {
             WaveGroupSync actor_sync{&sync_actor, (unsigned)k * ACTOR16_ROUNDS * 4u, 4u, &sync_failed, a.spin_limit};
@@ -399,15 +383,7 @@ __global__ __launch_bounds__(512) void collect_planar_kernel(CollectArgs a) {
         const uint32_t sseed = a.sample_seed + (uint32_t)k * a.sample_stride;
         const uint64_t rseed = a.reset_seed + (uint64_t)k * a.reset_stride;
         const int wave = tid / WAVE, lane = tid % WAVE;
-        for (int i = tid; i < R * IN; i += T) {
-            const int r = i / IN, c = i - r * IN;
-            float v = 0.0f;
-            if (r < ne) {
-                v = rows[r * M::STATE + c];
-                a.r_obs[row * IN + i] = v;
-            }
-            xs[r * XS_LD + c] = v;
-        }
+        stage_observations<IN, T>(xs, a.r_obs + row * IN, ne, tid, [&](int r, int c) { return rows[r * M::STATE + c]; });
         __syncthreads();
         if (wave < 4) {
             WaveGroupSync actor_sync{&sync_actor, (unsigned)k * ACTOR16_ROUNDS * 4u, 4u, &sync_failed, a.spin_limit};
