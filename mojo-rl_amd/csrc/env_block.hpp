@@ -46,7 +46,7 @@ MRL_DEV void account(const Accounting &acc, int i, float r, float d) { account(a
 struct LunarLander {
     using L = ll::L;
     static constexpr int STATE = ll::STATE, OBS = ll::OBS, ACT_W = 1, EPB = 16, THREADS = 256;
-    static constexpr int LANE_FROM = 8193;   // batch from which the stand-alone step runs one lane per env
+    static constexpr int LANE_FROM = 16385;   // batch from which the stand-alone step runs one lane per env
     static constexpr int DYN_END = L::JOINTS_OFF, NSHAPE = ll::NSHAPE_FLOATS;
     static MRL_DEV void step(float *row, float *cts, const float *shapes, int env, const float *a,
                              float &r, float &d) {

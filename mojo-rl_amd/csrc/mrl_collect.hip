@@ -192,13 +192,13 @@ static CollectPlan collect_plan(const mrl_rollout *r, int n_cus) {
         // Up to this many envs per CU the walkers' fused kernels are the faster way; with more, their 16-env workgroups
         // come round after round while the stand-alone kernels fill the chip.  us per step, fused against two launches,
         // hidden width 64 / 256:
-        //   HalfCheetah (one workgroup per CU)  4096 envs 68 / 73 : 74 / 88,  8192 envs 136 / 147 : 74 / 99;
+        //   HalfCheetah (one workgroup per CU)  4096 envs 46 / 51 : 55 / 68,  8192 envs 93 / 103 : 56 / 80;
         //   Walker2d  4096 envs 12.4 / 22.3 : 17.7 / 31.7,  4200 envs 24.0 / 43.8 : 22.6 / 47.5,  8192 envs 24.4 / 44.0 : 19.9 / 44.5
         //     (width 128 27.7 : 27.4),  16384 envs 47 / 87 : 31 / 76;
         //   CarRacing  4096 envs 20 / 31 : 28 / 41,  8192 envs 39 / 61 : 41 / 65,  16384 envs 76 / 121 : 72 / 116;
         //   Hopper  8192 envs 9.6 / 36 : 15.3 / 39,  16384 envs 22 / 70 : 26 / 69,  32768 envs 38 / 138 : 36 / 129;
-        //   BipedalWalker  4096 envs 36 / 41 : 47 / 60,  8192 envs 70 / 81 : 71 / 97,  12288 envs 105 / 121 : 90 / 134,
-        //     16384 envs 139 / 160 : 97 / 140,  32768 envs 274 / 315 : 162 / 251.
+        //   BipedalWalker  4096 envs 30 / 36 : 40 / 53,  8192 envs 58 / 70 : 68 / 93,  12288 envs 86 / 104 : 85 / 129,
+        //     16384 envs 114 / 138 : 91 / 135.
         int envs_per_cu = 32;
         if (id == MRL_ENV_HALFCHEETAH || (id == MRL_ENV_WALKER2D_PLANAR && p.H == 64)) envs_per_cu = 16;
         else if (id == MRL_ENV_BIPEDAL && p.H == 256) envs_per_cu = 48;
@@ -210,8 +210,8 @@ static CollectPlan collect_plan(const mrl_rollout *r, int n_cus) {
         if (!agent_nets(r, LunarLander::OBS, 0, gauss, &p.H, &p.act)) return p;
         // Hidden width 256: always in one launch.  The narrower nets up to 128 envs per CU, beyond which the stand-alone
         // kernels fill the chip (their env step runs one lane per env).  us per step, one launch : two per step, at
-        // 16384 / 32768 / 65536 envs: H = 64 27 : 53, 52 : 68, 106 : 93; H = 128 35 : 59, 68 : 81, 137 : 126;
-        // H = 256 at 8192 / 32768 / 131072 (one launch with 32 rows and one lane per env : this) 33.0 : 31.5, 132 : 125, 529 : 490.
+        // 16384 / 32768 / 65536 envs: H = 64 28 : 53, 53 : 68, 103 : 94; H = 128 35 : 59, 68 : 81, 137 : 126; H = 256
+        // 59 : 94, 116 : 152, 229 : 268.
         if (p.H == 256 || r->n_envs <= 8 * n_cus * PR16) p.form = FORM_ROWS16;
         return p;
     }

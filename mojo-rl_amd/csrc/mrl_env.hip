@@ -7,7 +7,7 @@
 // (row stride odd => the lanes touch distinct banks for any field) while the other wavefronts
 // detect its contacts where the env splits that off, and the fields that a step can change are
 // copied back with coalesced stores.  HBM sees each row once in and the changed part once out;
-// nothing is re-read.  (LunarLander above 8192 envs: one lane per env on rows left in global memory,
+// nothing is re-read.  (LunarLander above 16384 envs: one lane per env on rows left in global memory,
 // phys_step_lane_kernel; BipedalWalker above 4096 and HalfCheetah above 8192 envs: mrl_env_many.hip.)
 #include <cmath>
 #include "mrl_host.hpp"
@@ -147,9 +147,9 @@ __global__ __launch_bounds__(E::THREADS) void phys_step_kernel(float *states, co
 // The same step with one lane per ENV and the rows left in global memory (64 envs per single-wavefront
 // workgroup, only the contact scratch in LDS): nothing is shared between lanes, so a batch that fills the
 // chip runs at the rate of the vector units instead of at the latency of one workgroup's phase chain.
-// Used from E::LANE_FROM envs on (LunarLander: one wavefront's step lasts 40 us whatever the batch, the
-// 16-row workgroup's 19 .. 22 us, but a CU holds five of these wavefronts and two such workgroups; with 32 rows and one
-// lane per env the workgroup took 30 .. 33 us).
+// Used from E::LANE_FROM envs on (LunarLander: one wavefront's step lasts 40 us up to five of
+// them on every CU, the 16-row workgroups' a round of 19 .. 22 us and longer rounds as several share a CU: us per step of the
+// workgroups : of this form at 8200 / 12288 / 16384 / 32768 envs 22.2 : 40.2, 31.2 : 40.7, 37.2 : 40.9, 61.2 : 45.2).
 template <class E, bool AUTORESET>
 __global__ __launch_bounds__(64) void phys_step_lane_kernel(float *states, const float *actions, float *rewards,
                                                             float *dones, float *obs, const float *shapes_g, int batch,

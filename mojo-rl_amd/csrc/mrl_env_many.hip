@@ -17,11 +17,11 @@
 // Same operations on the same values as the workgroup forms: identical results bit for bit.
 //
 // What bounds it: the vector units' instruction stream, two to four wavefronts of dependent chains per SIMD
-// (BipedalWalker: 168 registers and 14.6 KB of LDS, eleven wavefronts per CU, 72 us a round against 54 us for one alone;
-// HalfCheetah: 128 registers, four wavefronts per SIMD, 128 us a round against 66 us for one alone).
+// (BipedalWalker: 168 registers and 14.6 KB of LDS, eleven wavefronts per CU; HalfCheetah: 128 registers, four wavefronts
+// per SIMD).
 // us per step, workgroup form -> this one:
-//   BipedalWalker  4096: 40 -> 61   5000: 68 -> 62   8192: 77 -> 64   16384: 150 -> 76   65536: 549 -> 208   131072: 1093 -> 371
-//   HalfCheetah    8192: 66 -> 68  10000: 129 -> 87                   16384: 130 -> 88   65536: 508 -> 257   131072: 1010 -> 479
+//   BipedalWalker  4096: 34 -> 56   5000: 56 -> 57   8192: 65 -> 59   16384: 126 -> 70   65536: 450 -> 184
+//   HalfCheetah    8192: 47 -> 49  10000: 91 -> 60                   16384: 92 -> 64   65536: 357 -> 181
 #include <cmath>
 #include "mrl_host.hpp"
 #include "env_block.hpp"

@@ -65,3 +65,26 @@ def test_mixed_rows_match_the_oracle(mrl, orc, name, n):
         np.testing.assert_array_equal(got, rows, err_msg="step %d" % t)
         np.testing.assert_array_equal(r.cpu().numpy(), r_h)
         np.testing.assert_array_equal(d.cpu().numpy(), d_h)
+
+
+@pytest.mark.parametrize("n", [8193, 16384, 16385])
+def test_lunar_step_where_the_forms_change_over(mrl, orc, n):
+    """Up to 16384 envs four lanes an env, beyond one lane an env: the oracle's bits on both sides."""
+    print("lunar switch", n, flush=True)
+    E = mrl.LunarLanderV2
+    ctx = mrl.DeviceContext("cuda:0")
+    rng = np.random.default_rng(n)
+    rows = np.zeros((n, 192), np.float32)
+    orc.orc_ll_reset_batch(rows, n, 3)
+    rows[:, 8:47].reshape(n, 3, 13)[:, :, 1] -= rng.uniform(7.5, 9.4, n).astype(np.float32)[:, None]
+    s = torch.from_numpy(rows.reshape(-1)).cuda()
+    r, d, o = (torch.zeros(k, device="cuda") for k in (n, n, n * 8))
+    r_h, d_h, o_h = np.zeros(n, np.float32), np.zeros(n, np.float32), np.zeros((n, 8), np.float32)
+    for t in range(4):
+        act = rng.integers(0, 4, n).astype(np.float32)
+        E.step_kernel_gpu(ctx, s, torch.from_numpy(act).cuda(), r, d, o, t)
+        orc.orc_ll_step_batch(rows, act, r_h, d_h, o_h, n, 8)
+        ctx.synchronize()
+        np.testing.assert_array_equal(s.cpu().numpy().view(np.uint32).reshape(n, 192), rows.view(np.uint32))
+        np.testing.assert_array_equal(r.cpu().numpy(), r_h)
+        np.testing.assert_array_equal(d.cpu().numpy(), d_h)
