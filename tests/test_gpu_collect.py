@@ -138,7 +138,7 @@ def _low_start(E, N, seed, orc):
     return s_h
 
 
-# up to 4096 envs (16 per CU) run the 16-row kernel, more the 32-row kernel
+# one workgroup of 16 envs per CU and two
 @pytest.mark.parametrize("env,kind,N", [("lunar", "relu", 2048), ("lunarc", "tanh", 2048), ("lunar", "tanh", 77),
                                         ("lunar", "relu", 4128), ("lunarc", "relu", 4128)])
 def test_fused_collection_through_contacts(mrl, ctx, orc, env, kind, N):
@@ -220,8 +220,8 @@ def test_fused_collection_through_contacts(mrl, ctx, orc, env, kind, N):
 
 @pytest.mark.parametrize("env,N", [("lunar", 600), ("lunarc", 600), ("lunar", 4128), ("lunarc", 4128)])
 def test_fused_collection_with_wind(mrl, orc, env, N):
-    """Wind and turbulence switched on for the context: the fused kernels (16-row form up to 4096 envs,
-    32-row form above) against the oracle with the same setting, step by step on the kernel's own
+    """Wind and turbulence switched on for the context: the fused kernels (one workgroup per CU up
+    to 4096 envs, two above) against the oracle with the same setting, step by step on the kernel's own
     actions, and the same range as one launch against the single steps, bit for bit.  The rows start
     at different step counts, which is the time the gusts are a function of."""
     import numpy as np
