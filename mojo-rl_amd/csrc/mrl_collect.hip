@@ -219,9 +219,11 @@ static CollectPlan collect_plan(const mrl_rollout *r, int n_cus) {
     else if (id == MRL_ENV_PENDULUM && gauss) obs = pendulum::OBS;
     else return p;
     if (!agent_nets(r, obs, 0, gauss, &p.H, &p.act)) return p;
-    // (hidden width 64, us per step of CartPole at 1024 / 4096 / 8192 / 16384 envs: 16 rows 3.75 / 3.71 / 5.20 / 9.86,
-    // 32 rows 4.88 / 4.66 / 4.75 / 6.20: with more than 16 envs per CU a second workgroup shares the matrix units)
-    p.form = (p.H == 64 && r->n_envs > n_cus * PR16) ? FORM_CLASSIC32 : FORM_ROWS16;
+    // Hidden width 64, us per step, 16 rows : 32 rows.  CartPole at 4096 / 5000 / 6144 / 7168 / 8192 / 16384 envs 2.7 : 4.2,
+    // 3.5 : 4.4, 3.9 : 4.3, 4.4 : 4.3, 5.0 : 4.3, 9.8 : 5.9; Pendulum at 6144 / 8192 / 12288 / 16384 / 32768 envs 4.0 : 4.4,
+    // 4.0 : 4.3, 5.0 : 6.2, 6.8 : 6.3, 12.5 : 12.2: with more than 16 envs per CU workgroups share the matrix units.
+    const int rows16_per_cu = id == MRL_ENV_CARTPOLE ? 24 : 48;
+    p.form = (p.H == 64 && r->n_envs > rows16_per_cu * n_cus) ? FORM_CLASSIC32 : FORM_ROWS16;
     return p;
 }
 

@@ -13,6 +13,7 @@ pytestmark = pytest.mark.gpu
     ("cartpole", 1, 30, 64, "relu"), ("cartpole", 17, 40, 128, "tanh"), ("cartpole", 4097, 8, 128, "relu"),
     ("cartpole", 4096, 8, 64, "tanh"), ("cartpole", 4097, 8, 64, "tanh"), ("cartpole", 4111, 6, 256, "relu"),
     ("pendulum", 1, 9, 128, "tanh"), ("pendulum", 33, 9, 256, "relu"), ("pendulum", 4097, 6, 64, "tanh"), ("pendulum", 4100, 6, 128, "tanh"),
+    ("cartpole", 6144, 6, 64, "tanh"), ("cartpole", 6145, 6, 64, "relu"), ("pendulum", 12288, 6, 64, "relu"), ("pendulum", 12289, 6, 64, "tanh"),
     ("lunar", 1, 9, 64, "relu"), ("lunar", 33, 9, 128, "tanh"), ("lunar", 8192, 6, 64, "relu"), ("lunar", 8193, 6, 128, "relu"),
     ("lunarc", 17, 9, 128, "tanh"), ("lunarc", 4099, 6, 64, "tanh"),
     ("bipedal", 17, 9, 64, "tanh"), ("bipedal", 333, 40, 128, "relu"), ("bipedal", 8193, 9, 128, "tanh"), ("bipedal", 12288, 9, 256, "relu"),
