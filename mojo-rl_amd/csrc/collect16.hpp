@@ -37,11 +37,11 @@ struct Critic16Split {
 // takes the sum of both times), so at H = 256 the second one costs what its forward passes cost (4096 : 8192 envs 18.5 :
 // 27.3 us per step); still, since the solver carries four lanes per env, two of 16 rows are ahead of one of 32 rows with one
 // lane per env and the critic on six wavefronts (33.0).
-// us per step with one lane per env : four: 777 envs, H = 64 19.4 : 12.9 (its solver wavefront: 22 of 37 thousand cycles in
-// the physics before); 4096 envs, H = 64 18.8 : 12.6, H = 256, where the critic is the longer path, 23.9 : 21.6.  The engines'
+// One lane per env : four, us per step: 777 envs, H = 64 19.4 : 12.9 (its solver wavefront: 22 of 37 thousand cycles in the
+// physics before); 4096 envs, H = 64 18.8 : 12.6, H = 256, where the critic is the longer path, 23.9 : 21.6.  The engines'
 // sines and the log-probability off the solver, its detection in one pass of all four wavefronts: H = 64, 777 envs
-// 11.46 : 11.26, 4096 envs 11.86 : 11.55 (11.2 since the step's first loads are no longer waited for; thousand cycles of a step there: actor 5.0, sample 1.1, detection 3.5, wait 0.8,
-// engines 1.6, physics and tail 12, reset 1).
+// 11.46 : 11.26, 4096 envs 11.86 : 11.55 (11.2 since a step's first loads are no longer waited for; thousand cycles of a
+// step there: actor 5.0, sample 1.1, detection 3.5, wait 0.8, engines 1.6, physics and tail 12, reset 1).
 // The solver wavefront is 0 in the lower half of the grid and 2 in the upper half: workgroups i and
 // i + grid / 2 share a CU when the grid is twice the CU count, and their solvers then sit on
 // different SIMDs.
