@@ -1,6 +1,7 @@
 // PPO elementwise and reduction kernels: samplers, GAE, advantage normalisation, minibatch
 // gather, loss gradients, global-norm clipping, Adam.  All are HBM-bound: one pass over the
 // data, coalesced, reductions by wavefront shuffles and one small second stage.
+#include <cmath>
 #include "mrl_host.hpp"
 #include "mrl_device.hpp"
 #include "ppo_grads.hpp"
@@ -136,27 +137,31 @@ __global__ __launch_bounds__(64) void gae_kernel(int T, int N, const float *__re
     }
 }
 
-// Below about one wavefront of envs per CU the plain scan waits for memory most of the time (T = 1000,
-// N = 4096: 63 waits on 64 CUs).  A = delta + decay * A is a serial chain per env, but a short one: three dependent instructions a
-// step.  What a plain scan waits for is memory, so the chain gets a wavefront of its own and eight
-// others feed it: a workgroup has G envs; its loaders fetch K = 512 / G * R steps at a time (index
-// t * N + env: rows of G consecutive floats), form delta, which needs no neighbour but the value one
-// step later, and leave (delta, decay or 0 where the episode ends) in LDS, two steps to 16 bytes; one wavefront scans
-// the chunk in place; the loaders store advantages and returns.  A step of the scan is one product, by the multiplication
-// whose zero times anything is zero, and one sum, and half a load and a store.  Three chunks are in LDS at once, one per stage, and the next one's
-// loads are in flight meanwhile.  What bounds it now is the chain (about 35 cycles a step; as product, sum, test and two LDS accesses 50) up to 16 envs
-// per CU, then the memory (T = 1000, N = 8192: 5.6 TB/s).  Same operations in the same order as the scan.  A chunk's rows, and
-// the value row above it, are read two barriers before the first of them is stored, so outputs may
-// share memory with the inputs.  deep_agents/ppo/ppo.mojo:2317-2353
 // a * b, and 0 where a or b is zero, whatever the other one is
 MRL_DEV float mul_zero_wins(float a, float b) {
     float r;
     asm("v_mul_legacy_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
     return r;
 }
+
+// Below about one wavefront of envs per CU the plain scan waits for memory most of the time (T = 1000,
+// N = 4096: 63 waits on 64 CUs).  A = delta + decay * A is a serial chain per env, but a short one: three dependent instructions a
+// step.  What a plain scan waits for is memory, so the chain gets a wavefront of its own and eight
+// others feed it: a workgroup has G envs; its loaders fetch K = 512 / G * R steps at a time (index
+// t * N + env: rows of G consecutive floats), form delta, which needs no neighbour but the value one
+// step later, and leave (delta, factor) in LDS, two steps to 16 bytes; one wavefront scans the chunk in place; the
+// loaders store advantages and returns.  Three chunks are in LDS at once, one per stage, and the next one's loads are in
+// flight meanwhile.  The factor is the decay, or 0 where the episode ends, and a step of the scan is one product, by the
+// multiplication whose zero times anything is zero, one sum, and half a load and a store.  EXACT, for a decay that is zero or
+// not finite: an episode's end could not be told from the decay there, and a zero times it is not zero; the factor is 1 or
+// 0, the scan selects by it and multiplies by the decay (the one more test is 50 cycles a step instead of 35).
+// What bounds it now is the chain up to 16 envs
+// per CU, then the memory (T = 1000, N = 8192: 5.6 TB/s).  Same operations in the same order as the scan (the sign of a zero
+// aside).  A chunk's rows, and the value row above it, are read two barriers before the first of them is stored, so outputs may
+// share memory with the inputs.  deep_agents/ppo/ppo.mojo:2317-2353
 constexpr int GAE_LOADERS = 512;   // threads; one more wavefront scans
 
-template <int G, int R>
+template <int G, int R, bool EXACT>
 __global__ __launch_bounds__(GAE_LOADERS + 64) void gae_fed_kernel(int T, int N, const float *rewards, const float *values,
                                                                const float *dones, const float *bootstrap, float gamma,
                                                                float decay, float *adv, float *ret) {
@@ -172,6 +177,7 @@ __global__ __launch_bounds__(GAE_LOADERS + 64) void gae_fed_kernel(int T, int N,
     const bool scanner = threadIdx.x >= GAE_LOADERS;
     const int C = (T + K - 1) / K;
     if (group * G >= N) return;
+    const float factor = EXACT ? 1.0f : decay;
 
     float r[R], v[R], d[R], v1[R], v2[R], next = 0.0f, gae = 0.0f;
     // A chunk's rows end at its uniform base row T - (c + 1) K (below 0 in a ragged last chunk; only rows t >= 0 are
@@ -193,6 +199,7 @@ __global__ __launch_bounds__(GAE_LOADERS + 64) void gae_fed_kernel(int T, int N,
         if (c == 0 && top == 0) next = bootstrap[ec];
         else next = in(values, row0, max(off[0] + 4u * N, low));
     };
+    auto decayed = [&](float f, float a) { return EXACT ? decay * (f == 0.0f ? 0.0f : a) : mul_zero_wins(f, a); };
     if (!scanner) request(0);
     else __builtin_amdgcn_s_setprio(3);   // the chain goes before the loaders of its SIMD
     for (int it = 0; it < C + 2; ++it) {
@@ -203,8 +210,8 @@ __global__ __launch_bounds__(GAE_LOADERS + 64) void gae_fed_kernel(int T, int N,
 #pragma unroll
                 for (int j = 0; j < R; j += 2) {
                     const bool e0 = d[j] > 0.5f, e1 = d[j + 1] > 0.5f;
-                    B[j / 2 * G] = make_float4(r[j] + gamma * (e0 ? 0.0f : nv) - v[j], e0 ? 0.0f : decay,
-                                               r[j + 1] + gamma * (e1 ? 0.0f : v[j]) - v[j + 1], e1 ? 0.0f : decay);
+                    B[j / 2 * G] = make_float4(r[j] + gamma * (e0 ? 0.0f : nv) - v[j], e0 ? 0.0f : factor,
+                                               r[j + 1] + gamma * (e1 ? 0.0f : v[j]) - v[j + 1], e1 ? 0.0f : factor);
                     nv = v[j + 1];
                 }
             }
@@ -245,8 +252,8 @@ __global__ __launch_bounds__(GAE_LOADERS + 64) void gae_fed_kernel(int T, int N,
                 for (int j = 0; j < U / 2; ++j) n[j] = B[(kn + j) * G];
 #pragma unroll
                 for (int j = 0; j < U / 2; ++j) {
-                    const float g0 = x[j].x + mul_zero_wins(x[j].y, gae);
-                    gae = x[j].z + mul_zero_wins(x[j].w, g0);
+                    const float g0 = x[j].x + decayed(x[j].y, gae);
+                    gae = x[j].z + decayed(x[j].w, g0);
                     B[(k / 2 + j) * G].x = g0;
                     B[(k / 2 + j) * G].z = gae;
                 }
@@ -712,11 +719,14 @@ int mrl_gae(mrl_ctx *ctx, int T, int N, const float *rewards, const float *value
         hipLaunchKernelGGL(kernel, dim3(groups), dim3(threads), 0, ctx->stream, T, N, rewards, values, dones,
                            bootstrap, g, decay, adv, ret);
     };
+    const bool exact = decay == 0.0f || !std::isfinite(decay);
+#define MRL_GAE_FED(G, R, groups) (exact ? launch(gae_fed_kernel<G, R, true>, groups) : launch(gae_fed_kernel<G, R, false>, groups))
     if (T > 1 << 30) launch(gae_kernel, grid_for(N, 64), 64);   // (the chunked form counts rows past T in 32 bits)
-    else if (N <= 16 * ctx->n_cus) launch(gae_fed_kernel<16, 2>, (grid_for(N, 16) + 15) / 16 * 16);
-    else if (N <= 32 * ctx->n_cus) launch(gae_fed_kernel<32, 4>, grid_for(N, 32));
-    else if (N <= 64 * ctx->n_cus) launch(gae_fed_kernel<64, 4>, grid_for(N, 64));
+    else if (N <= 16 * ctx->n_cus) MRL_GAE_FED(16, 2, (grid_for(N, 16) + 15) / 16 * 16);
+    else if (N <= 32 * ctx->n_cus) MRL_GAE_FED(32, 4, grid_for(N, 32));
+    else if (N <= 64 * ctx->n_cus) MRL_GAE_FED(64, 4, grid_for(N, 64));
     else launch(gae_kernel, grid_for(N, 64), 64);
+#undef MRL_GAE_FED
     MRL_CHECK_LAUNCH();
     return MRL_OK;
 }
