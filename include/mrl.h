@@ -250,6 +250,10 @@ int mrl_permutation_from_uniforms(mrl_ctx *ctx, int32_t *indices, int n, const d
  * int32; [2] and [3] belong to mrl_ppo_update_minibatch).  Replaces
  * the per-minibatch D2H copy + host mean of ppo.mojo:2557-2573 / ppo_continuous.mojo:3062-3086. */
 int mrl_kl_check(mrl_ctx *ctx, const float *kl, int mb, float target_kl, int32_t *flag);
+/* The library's own fp32 sine, cosine and logarithm of x[0..n), each output may be NULL: the correctly rounded values for
+ * every x.  Env steps, samplers and losses take the same functions in their kernels, and index and branch decisions hang on
+ * their last bits; this is how a test (or a host restatement of an env) gets at them. */
+int mrl_math32(mrl_ctx *ctx, const float *x, int n, float *sine, float *cosine, float *logarithm);
 /* params[i] = lo + u_i (hi - lo): the uniform fills behind Xavier / Kaiming
  * (deep_rl/initializer/initializers.mojo:69-104) and StochasticActor.init_params_small
  * (deep_rl/model/stochastic_actor.mojo:95-128); u from Philox(seed). */

@@ -109,6 +109,7 @@ SIGNATURES = {
     "mrl_permutation": [P, P, I, U64],
     "mrl_permutation_from_uniforms": [P, P, I, P, P],
     "mrl_kl_check": [P, P, I, F, P],
+    "mrl_math32": [P, P, I, P, P, P],
     "mrl_init_uniform": [P, P, I, F, F, U64],
     "mrl_policy_step_discrete": [P, DP, DP, I, P, P, P, U32, P, P, P, P, P],
     "mrl_policy_step_gaussian": [P, DP, DP, I, P, P, P, U32, P, P, P, P, P],

@@ -17,11 +17,10 @@
 
 namespace mrl {
 
-// The remainder of ax, finite and above 2^20, against multiples of pi / 2, and the multiple, on the lanes with `large`
-// (Payne and Hanek's method, in integers): ax = M 2^E; the bits of 1 / (2 pi) from bit E on, times M, are the fraction of a
-// turn, to 104 bits and more.  No branch on a lane's own value: where such a branch ends, the compiler has been seen to save
-// a register that lives across it before it widens the lane mask again.
-MRL_DEV void reduce_large(float ax, bool large, double &r, int &q) {
+// The remainder r + tail of ax, finite and above 2^20, against multiples of pi / 2, and the multiple (Payne and Hanek's method,
+// in integers): ax = M 2^E; the bits of 1 / (2 pi) from bit E on, times M, are the fraction of a turn, to 104 bits and
+// more.
+MRL_DEV void reduce_large(float ax, double &r, double &tail, int &q) {
     const uint32_t bits = __float_as_uint(ax), M = (bits & 0x7FFFFFu) | 0x800000u;
     const uint32_t at = (bits >> 23) - 150u + 32u, word = at >> 5, shift = at & 31u;   // (the first 32 bits: zeros for E < 0)
     constexpr uint32_t T[9] = {0x00000000u, 0x28BE60DBu, 0x9391054Au, 0x7F09D5F4u, 0x7D4D3770u, 0x36D8A566u, 0x4F10E410u, 0x7F9458EAu, 0xF7AEF158u};
@@ -43,10 +42,13 @@ MRL_DEV void reduce_large(float ax, bool large, double &r, int &q) {
         carry >>= 32;
     }
     const uint32_t quarter = (p[0] + 0x20000000u) >> 30;
-    const double turn = (double)(int)(p[0] - (quarter << 30)) * 0x1p-32 + ((double)p[1] * 0x1p-64 + (double)p[2] * 0x1p-96);
-    const double rem = fma(turn, 6.283185307179586, turn * 2.4492935982947064e-16);
-    r = large ? rem : r;
-    q = large ? (int)quarter : q;
+    const double high = (double)(int)(p[0] - (quarter << 30)) * 0x1p-32, low = (double)p[1] * 0x1p-64 + (double)p[2] * 0x1p-96;
+    const double turn = high + low, off = low - (turn - high);
+    const double two_pi = 6.283185307179586, rem = turn * two_pi;
+    const double more = fma(turn, two_pi, -rem) + fma(turn, 2.4492935982947064e-16, off * two_pi);   // (2 pi in two pieces)
+    r = rem + more;
+    tail = more - (r - rem);
+    q = (int)quarter;
 }
 
 // Sine and cosine of an fp32 angle, rounded once from Float64.  An env step takes a dozen of them in a row on the one
@@ -54,8 +56,8 @@ MRL_DEV void reduce_large(float ax, bool large, double &r, int &q) {
 // the last one or not, so what counts is the number of instructions: the argument less k pi/2 (pi/2 in two pieces; the fma's
 // product is exact), both polynomials of the remainder r, |r| <= pi/4 (interpolated at the Chebyshev points, off by less than
 // 2^-55), and the quadrant's choice among the two rounded values.  237 cycles a call where the library's pair takes 441.
-// The bits are the library's, rounded: compared on every fp32 value (one pair differs, +-2.8616508e15, whose sine is 1.3e-9 of
-// an ulp off the middle between two floats).
+// Beyond 2^20 the remainder is carried in two pieces: the cosine of +-2.8616508e15 is 1.3e-9 of an ulp off the middle between
+// two floats.  Compared with the rounded Float64 functions of a C library on every finite fp32 value: no difference.
 struct SinCosK {
     double two_over_pi = 0.6366197723675814, half_pi = 1.5707963267948966, half_pi_lo = 6.123233995736766e-17;
     double s1 = -0.16666666666666666, s2 = 0.008333333333330936, s3 = -0.00019841269836740532, s4 = 2.7557316093198404e-06,
@@ -73,15 +75,17 @@ struct SinCosK {
         return k;
     }
 };
-// of the angle q pi / 2 + r, with x's sign
-MRL_DEV void sincos_reduced(float x, double r, int q, const SinCosK &k, float &s, float &c) {
+// of the angle q pi / 2 + r (+ tail), with x's sign
+template <bool TAIL = false>
+MRL_DEV void sincos_reduced(float x, double r, int q, const SinCosK &k, float &s, float &c, double tail = 0.0) {
     const double u = r * r;
     double ps = fma(k.s6, u, k.s5), pc = fma(k.c6, u, k.c5);
     ps = fma(ps, u, k.s4); pc = fma(pc, u, k.c4);
     ps = fma(ps, u, k.s3); pc = fma(pc, u, k.c3);
     ps = fma(ps, u, k.s2); pc = fma(pc, u, k.c2);
     ps = fma(ps, u, k.s1); pc = fma(pc, u, k.c1);
-    const float fs = (float)fma(r * u, ps, r), fc = (float)fma(fma(u, pc, -0.5), u, 1.0);
+    const float fs = (float)(TAIL ? r + fma(r * u, ps, tail) : fma(r * u, ps, r));
+    const float fc = (float)(TAIL ? 1.0 + fma(fma(u, pc, -0.5), u, -r * tail) : fma(fma(u, pc, -0.5), u, 1.0));
     const uint32_t a = __float_as_uint((q & 1) ? fc : fs), b = __float_as_uint((q & 1) ? fs : fc);
     s = __uint_as_float(a ^ ((uint32_t)(q & 2) << 30) ^ (__float_as_uint(x) & 0x80000000u));
     c = __uint_as_float(b ^ ((uint32_t)((q + 1) & 2) << 30));
@@ -91,12 +95,18 @@ MRL_DEV void sincos32(float x, float &s, float &c, const SinCosK &k = SinCosK{})
     const bool far = __any(ax > 0x1p20f);   // (beyond, pi / 2 in two pieces is too short)
     const double xd = (double)ax;
     const double n = __builtin_rint(xd * k.two_over_pi);
-    double r = fma(-n, k.half_pi_lo, fma(-n, k.half_pi, xd));
-    int q = (int)n;
-    sincos_reduced(x, r, q, k, s, c);
+    sincos_reduced(x, fma(-n, k.half_pi_lo, fma(-n, k.half_pi, xd)), (int)n, k, s, c);
     if (__builtin_expect(far, 0)) {
-        reduce_large(ax, ax > 0x1p20f && ax < __builtin_inff(), r, q);
-        sincos_reduced(x, r, q, k, s, c);
+        // (No branch on a lane's own value: at the end of one the compiler has been seen to save registers that live across
+        // it before it widens the lane mask again; build.py looks for that.)
+        const bool large = ax > 0x1p20f && ax < __builtin_inff();
+        double r, tail;
+        float ls, lc;
+        int q;
+        reduce_large(ax, r, tail, q);
+        sincos_reduced<true>(x, r, q, k, ls, lc, tail);
+        s = large ? ls : s;
+        c = large ? lc : c;
     }
 }
 // the same without the test, which is a third of its time, for a caller that knows |x| <= 2^20 or finds out later
@@ -147,12 +157,12 @@ MRL_DEV float log32(float x) {
     return r;
 }
 
-// whether any active lane says so, straight from the compare
 // the value of lane L of every four
 template <int L>
 MRL_DEV float quad_bcast(float x) {
     return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), L * 0x55, 0xF, 0xF, true));
 }
+// whether any active lane says so, straight from the compare
 MRL_DEV bool any_lane(bool p) { return __builtin_amdgcn_ballot_w64(p) != 0; }
 
 // x / d for a divisor that is divided by again and again (a joint's summed inverse inertia, a contact's

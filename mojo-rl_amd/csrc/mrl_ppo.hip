@@ -73,6 +73,17 @@ __global__ __launch_bounds__(TPB) void obs_noise_kernel(float *__restrict__ obs,
     obs[e] = obs[e] + noise * noise_std;
 }
 
+__global__ __launch_bounds__(TPB) void math32_kernel(const float *__restrict__ x, int n, float *__restrict__ sine,
+                                                     float *__restrict__ cosine, float *__restrict__ logarithm) {
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    float s, c;
+    sincos32(x[i], s, c);
+    if (sine != nullptr) sine[i] = s;
+    if (cosine != nullptr) cosine[i] = c;
+    if (logarithm != nullptr) logarithm[i] = log32(x[i]);
+}
+
 // ---------------------------------------------------------------- GAE
 // One lane per env scans t = T-1 .. 0; index t*N + env makes every step of the scan a
 // coalesced row access.  The scan itself is serial, its loads are not: the rows of the next
@@ -802,6 +813,16 @@ int mrl_kl_check(mrl_ctx *ctx, const float *kl, int mb, float target_kl, int32_t
     MRL_CHECK_ARG(mb > 0, "mrl_kl_check: minibatch must be positive");
     MRL_CHECK_ARG(kl && flag, "mrl_kl_check: NULL buffer");
     hipLaunchKernelGGL(kl_check_kernel, dim3(1), dim3(TPB), 0, ctx->stream, kl, mb, target_kl, flag);
+    MRL_CHECK_LAUNCH();
+    return MRL_OK;
+}
+
+int mrl_math32(mrl_ctx *ctx, const float *x, int n, float *sine, float *cosine, float *logarithm) {
+    MRL_CHECK_ARG(ctx, "mrl_math32: ctx is NULL");
+    MRL_CHECK_ARG(n >= 0, "mrl_math32: negative size");
+    if (n == 0) return MRL_OK;
+    MRL_CHECK_ARG(x, "mrl_math32: NULL buffer");
+    hipLaunchKernelGGL(math32_kernel, dim3(grid_for(n, TPB)), dim3(TPB), 0, ctx->stream, x, n, sine, cosine, logarithm);
     MRL_CHECK_LAUNCH();
     return MRL_OK;
 }
