@@ -23,6 +23,9 @@
 //   CHILD[e]  bit l: lane l is the child in its slot of parity e
 //   JOINT[e]  nibble l: the joint of lane l's slot of parity e (0 where it has none)
 //   SPRING, MOTOR: whether every joint has that term (all have a limit)
+// These are the terms that the env's reset gives its joints.  A caller may have changed a row's: where a joint of the
+// wavefront's has others (or a limit the wrong way round, or nothing to turn), the step runs on a second instance that decides
+// every term lane by lane (ANY).
 #pragma once
 #include "physics2d_reg.hpp"
 
@@ -38,21 +41,34 @@ MRL_DEV int lane_body(int l) { return (int)((R::BODY >> (4 * l)) & 15u); }
 template <class R>
 MRL_DEV int lane_joint(int e, int l) { return (int)(((e ? R::JOINT[1] : R::JOINT[0]) >> (4 * l)) & 15u); }
 
-// true when the row's joints are what the lanes assume: the wiring T, the terms R names, each with something to turn
+// true when the row's joints are wired as the lanes assume.  (A motor that no step sets keeps the caller's torque, and a
+// negative one turns both bodies the same way, which the halves do not.)
 template <class L, class T, class R>
 MRL_DEV bool body_lanes_row_ok(const float *row) {
     if ((int)row[L::JOINT_COUNT_OFF] != L::MAX_JOINTS) return false;
     bool ok = true;
+#pragma unroll
+    for (int j = 0; j < L::MAX_JOINTS; ++j) {
+        const float *J = row + L::JOINTS_OFF + j * JOINT_SIZE;
+        ok = ok && (int)J[J_TYPE] == 0 && (int)J[J_BODY_A] == T::a(j) && (int)J[J_BODY_B] == T::b(j);
+        if (!R::MOTOR) ok = ok && (((int)J[J_FLAGS] & JF_MOTOR) == 0 || J[J_MAX_TORQUE] >= 0.0f);
+    }
+    return ok;
+}
+
+// true when the joints of such a row have the terms that R names, limits in order and something to turn
+template <class L, class T, class R>
+MRL_DEV bool body_lanes_row_usual(const float *row) {
     constexpr int FLAGS = JF_LIMIT | (R::SPRING ? JF_SPRING : 0) | (R::MOTOR ? JF_MOTOR : 0);
+    bool usual = true;
 #pragma unroll
     for (int j = 0; j < L::MAX_JOINTS; ++j) {
         const float *J = row + L::JOINTS_OFF + j * JOINT_SIZE;
         const float ia = row[L::BODIES_OFF + T::a(j) * BODY_SIZE + IDX_INV_INERTIA];
         const float ib = row[L::BODIES_OFF + T::b(j) * BODY_SIZE + IDX_INV_INERTIA];
-        ok = ok && (int)J[J_TYPE] == 0 && (int)J[J_BODY_A] == T::a(j) && (int)J[J_BODY_B] == T::b(j) &&
-             ((int)J[J_FLAGS] & (JF_LIMIT | JF_SPRING | JF_MOTOR)) == FLAGS && J[J_LO] <= J[J_HI] && ia + ib > 1e-10f;
+        usual = usual && ((int)J[J_FLAGS] & (JF_LIMIT | JF_SPRING | JF_MOTOR)) == FLAGS && J[J_LO] <= J[J_HI] && ia + ib > 1e-10f;
     }
-    return ok;
+    return usual;
 }
 
 // the velocities of the lane's body are B.vx[0] .., its place B.x[0] ..
@@ -202,20 +218,20 @@ struct LaneListContacts {
 
 // ---------------------------------------------------------------- joints
 
+// a lane's place in the wiring, l: lane in the env's group
 template <class R>
-struct LaneJoints {
+struct LaneSlots {
     static constexpr int S = R::SLOTS;
     bool in[S], child[2];
-    // by parity of the slot, from the lane's own side (the parent's are the child's negated, its bounds swapped)
-    float ax[2], ay[2];                  // my anchor
-    float eff[2], reff[2];
-    float lo[2], hi[2], ref[2], speed[2], max_impulse[2], damp[2];
-    // of the joint whose child I am
-    float p_im, p_ii, c_ref, c_lo, c_hi, c_stiff;
-    // fixed during a velocity phase
-    float rx[2], ry[2], k11[2], k12[2], k22[2], below[2], above[2], spring[2];
 
-    // the value that my partner holds, in my slot of parity e
+    MRL_DEV explicit LaneSlots(int l) {
+#pragma unroll
+        for (int s = 0; s < S; ++s) in[s] = ((R::IN[s] >> l) & 1u) != 0;
+        child[0] = ((R::CHILD[0] >> l) & 1u) != 0;
+        child[1] = ((R::CHILD[1] >> l) & 1u) != 0;
+    }
+
+    // the value that my partner holds, in my slot of parity E
     template <int E>
     MRL_DEV float partner(float v) const {
         const float a = dpp_xchg<R::CTRL[E]>(v);
@@ -232,32 +248,74 @@ struct LaneJoints {
         const float a = partner<0>(v0), b = partner<1>(v1);
         return child[0] ? a : b;
     }
+};
 
-    // the constants of a step; l: lane in the env's group
+template <class R, bool ANY>
+struct LaneJoints : LaneSlots<R> {
+    using Slots = LaneSlots<R>;
+    using Slots::S;
+    using Slots::in;
+    using Slots::child;
+    using Slots::parent;
+    static constexpr bool SPRING = R::SPRING || ANY, MOTOR = R::MOTOR || ANY, ALL = ANY;
+    // by parity of the slot, from the lane's own side (the parent's are the child's negated, its bounds swapped)
+    float ax[2], ay[2];                  // my anchor
+    float eff[2], reff[2];
+    float lo[2], hi[2], ref[2], speed[2], max_impulse[2], damp[2];
+    bool springs[2], motors[2];          // (ANY)
+    // of the joint whose child I am
+    float p_im, p_ii, c_ref, c_lo, c_hi, c_stiff;
+    // fixed during a velocity phase
+    float rx[2], ry[2], k11[2], k12[2], k22[2], below[2], above[2], spring[2];
+
+    MRL_DEV explicit LaneJoints(int l) : Slots(l) {}
+
+    // whether the joint whose child I am, if there is one, has the terms R names
+    template <class L>
+    MRL_DEV bool usual(const float *row, int l, const LaneBody &B) const {
+        constexpr int FLAGS = JF_LIMIT | (R::SPRING ? JF_SPRING : 0) | (R::MOTOR ? JF_MOTOR : 0);
+        const int flags = (int)row[L::JOINTS_OFF + lane_joint<R>(child[0] ? 0 : 1, l) * JOINT_SIZE + J_FLAGS];
+        return !(child[0] || child[1]) || ((flags & (JF_LIMIT | JF_SPRING | JF_MOTOR)) == FLAGS && c_lo <= c_hi && p_ii + B.ii[0] > 1e-10f);
+    }
+
+    // the constants of a step
     template <class L>
     MRL_DEV void load(const float *row, int l, const LaneBody &B, float dt) {
-#pragma unroll
-        for (int s = 0; s < S; ++s) in[s] = ((R::IN[s] >> l) & 1u) != 0;
+        p_im = parent(B.im[0], B.im[0]); p_ii = parent(B.ii[0], B.ii[0]);
+        eff[0] = this->template partner<0>(B.ii[0]) + B.ii[0];
+        eff[1] = this->template partner<1>(B.ii[0]) + B.ii[0];
+        // (a limit that is not there: bounds that no angle is beyond)
+        const float none = __builtin_nanf("");
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
-            child[e] = ((R::CHILD[e] >> l) & 1u) != 0;
             const float *J = row + L::JOINTS_OFF + lane_joint<R>(e, l) * JOINT_SIZE;
             ax[e] = J[child[e] ? J_BX : J_AX]; ay[e] = J[child[e] ? J_BY : J_AY];
             const float l0 = J[J_LO], h0 = J[J_HI], r0 = J[J_REF];
             lo[e] = child[e] ? l0 : -h0; hi[e] = child[e] ? h0 : -l0; ref[e] = child[e] ? r0 : -r0;
-            if (R::MOTOR) {
+            if (MOTOR) {
                 const float v0 = J[J_MOTOR_SPEED];
                 speed[e] = child[e] ? v0 : -v0;
                 max_impulse[e] = J[J_MAX_TORQUE] * dt;
             }
-            if (R::SPRING) damp[e] = J[J_DAMP];
+            if (SPRING) damp[e] = J[J_DAMP];
+            if (ANY) {
+                const int flags = (int)J[J_FLAGS];
+                const bool turns = eff[e] > 1e-10f, limited = turns && (flags & JF_LIMIT) != 0;
+                springs[e] = turns && (flags & JF_SPRING) != 0;
+                motors[e] = turns && (flags & JF_MOTOR) != 0;
+                lo[e] = limited ? lo[e] : none;
+                hi[e] = limited ? hi[e] : none;
+                eff[e] = turns ? eff[e] : 1.0f;
+            }
         }
         const float *J = row + L::JOINTS_OFF + lane_joint<R>(child[0] ? 0 : 1, l) * JOINT_SIZE;
         c_ref = J[J_REF]; c_lo = J[J_LO]; c_hi = J[J_HI];
-        if (R::SPRING) c_stiff = J[J_STIFF];
-        p_im = parent(B.im[0], B.im[0]); p_ii = parent(B.ii[0], B.ii[0]);
-        eff[0] = partner<0>(B.ii[0]) + B.ii[0];
-        eff[1] = partner<1>(B.ii[0]) + B.ii[0];
+        if (SPRING) c_stiff = J[J_STIFF];
+        if (ANY) {
+            const bool limited = ((int)J[J_FLAGS] & JF_LIMIT) != 0 && p_ii + B.ii[0] > 1e-10f;
+            c_lo = limited ? c_lo : none;
+            c_hi = limited ? c_hi : none;
+        }
         reff[0] = 1.0f / eff[0];
         reff[1] = 1.0f / eff[1];
     }
@@ -276,19 +334,20 @@ struct LaneJoints {
         const float rel_angle = B.ang[0] - p_ang - c_ref, inf = __builtin_inff();
         const float c_below = rel_angle <= c_lo ? 0.0f : -inf;
         const float c_above = !(rel_angle <= c_lo) && rel_angle >= c_hi ? 0.0f : inf;
-        const float c_spring = R::SPRING ? -c_stiff * rel_angle : 0.0f;
+        const float c_spring = SPRING ? -c_stiff * rel_angle : 0.0f;
         hand<0>(c11, c12, c22, c_below, c_above, c_spring);
         hand<1>(c11, c12, c22, c_below, c_above, c_spring);
     }
     template <int E>
     MRL_DEV void hand(float c11, float c12, float c22, float c_below, float c_above, float c_spring) {
-        const float h11 = partner<E>(c11), h12 = partner<E>(c12), h22 = partner<E>(c22);
-        const float hb = partner<E>(c_below), ha = partner<E>(c_above);
+        auto partner = [&](float v) { return Slots::template partner<E>(v); };
+        const float h11 = partner(c11), h12 = partner(c12), h22 = partner(c22);
+        const float hb = partner(c_below), ha = partner(c_above);
         k11[E] = child[E] ? c11 : h11; k12[E] = child[E] ? c12 : h12; k22[E] = child[E] ? c22 : h22;
         below[E] = child[E] ? c_below : -ha;
         above[E] = child[E] ? c_above : -hb;
-        if (R::SPRING) {
-            const float hs = partner<E>(c_spring);
+        if (SPRING) {
+            const float hs = partner(c_spring);
             spring[E] = child[E] ? c_spring : -hs;
         }
     }
@@ -303,9 +362,10 @@ struct LaneJoints {
         const float jx = k11[e] * dx + k12[e] * dy, jy = k12[e] * dx + k22[e] * dy;
         const float vx = B.vx[0] - im * jx, vy = B.vy[0] - im * jy;
         float cw = w - ii * (rx[e] * jy - ry[e] * jx);
-        if (R::SPRING) {
+        if (SPRING) {
             const float torque = spring[e] - damp[e] * (w - dpp_xchg<ctrl>(w));   // (velocities from before the point impulse)
-            cw = cw + div_by(ii * (torque * dt), eff[e], reff[e]);
+            const float to = cw + div_by(ii * (torque * dt), eff[e], reff[e]);
+            cw = !ANY || springs[e] ? to : cw;
         }
         {
             const float d = cw - dpp_xchg<ctrl>(cw);
@@ -314,12 +374,13 @@ struct LaneJoints {
             const float to = cw - ii * q;
             cw = acts ? to : cw;
         }
-        if (R::MOTOR) {
+        if (MOTOR) {
             const float d = cw - dpp_xchg<ctrl>(cw);
             float q = div_by(speed[e] - d, eff[e], reff[e]);
             q = q > max_impulse[e] ? max_impulse[e] : q;
             q = q < -max_impulse[e] ? -max_impulse[e] : q;
-            cw = cw + ii * q;
+            const float to = cw + ii * q;
+            cw = !ANY || motors[e] ? to : cw;
         }
         B.vx[0] = in[SL] ? vx : B.vx[0];
         B.vy[0] = in[SL] ? vy : B.vy[0];
@@ -355,7 +416,9 @@ struct LaneJoints {
         {
             const float rel = a - dpp_xchg<ctrl>(a) - ref[e];
             const bool low = rel < lo[e], high = rel > hi[e];
-            const float c = baumgarte * ((low ? lo[e] : hi[e]) - rel);
+            // (beyond both: of limits the wrong way round, where the child's lower one counts)
+            const bool to_lo = ANY && !child[e] ? !high : low;
+            const float c = baumgarte * ((to_lo ? lo[e] : hi[e]) - rel);
             const float to = a + div_by(ii * c, eff[e], reff[e]);
             a = (low || high) && c != 0.0f ? to : a;
         }
@@ -403,8 +466,8 @@ struct LaneJoints {
 
 // One physics step (sub-step): velocity sweeps, integration, position sweeps.  In: velocities with the forces applied,
 // (sn, cs) of the angles, contacts loaded; out: (sn, cs) of the new angles where R::ANGLES_AFTER.
-template <class R, int VEL, int POS, class Contacts>
-MRL_DEV void body_lanes_solve(LaneBody &B, LaneJoints<R> &J, Contacts &contacts, float &sn, float &cs, float dt, float friction,
+template <class R, bool ANY, int VEL, int POS, class Contacts>
+MRL_DEV void body_lanes_solve(LaneBody &B, LaneJoints<R, ANY> &J, Contacts &contacts, float &sn, float &cs, float dt, float friction,
                               float restitution, float baumgarte) {
     J.prepare(B, sn, cs);
 #pragma unroll 1
@@ -420,6 +483,20 @@ MRL_DEV void body_lanes_solve(LaneBody &B, LaneJoints<R> &J, Contacts &contacts,
     B.x[0] = x; B.y[0] = y; B.ang[0] = ang;
     sn = s0; cs = c0;
     J.template position_sweeps<false, POS>(B, sn, cs, contacts, baumgarte, K);
+}
+
+// f(the lane's joints): J as loaded, or with every term decided lane by lane where one of the wavefront's lanes is `odd`.
+// us where every row is, such rows in the one-lane form : now: HalfCheetah step of 1000 / 65536 envs 190 : 42, 788 : 206,
+// rollout of 4096 envs (H = 64, 32 steps) 7659 : 1350; BipedalWalker 82 : 25, 798 : 178, 2048 envs 2661 : 845.
+template <class L, class R, class F>
+MRL_DEV void with_joints(LaneJoints<R, false> &J, const float *row, int l, const LaneBody &B, float dt, bool odd, F &&f) {
+    if (__builtin_expect(any_lane(odd), 0)) {
+        LaneJoints<R, true> A(l);
+        A.template load<L>(row, l, B, dt);
+        f(A);
+    } else {
+        f(J);
+    }
 }
 
 }  // namespace mrl

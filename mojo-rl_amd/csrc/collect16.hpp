@@ -92,12 +92,12 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
     }
     __syncthreads();
     // solver wavefront, four lanes per env: the env's running episode return and length stay in registers of the first,
-    // and whether its wiring is the kind's own (no step changes it, a reset makes it so) in all four
+    // and what its wiring is (E::lanes_wired) in all four
     const int my_env = (t & 63) >> 2;
     const bool owner = (t >> 6) == sw && my_env < nenv && (t & 3) == 0;
     float ep_return = owner ? a.acc.ep_return[env0 + my_env] : 0.0f;
     float ep_length = owner ? a.acc.ep_length[env0 + my_env] : 0.0f;
-    int wired = my_env < nenv && E::lanes_ok(rows + my_env * S::STRIDE) ? 1 : 0;
+    int wired = my_env < nenv ? E::lanes_wired(rows + my_env * S::STRIDE) : 0;
 
     for (int k = 0; k < a.n_steps; ++k) {
         // Nothing but the rows is carried from one step to the next: the thread index, the block's
@@ -164,7 +164,7 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
             detect_sync.wait_for(detect_sync.target);
             if (first) carry = E::step_begin(rows + e * S::STRIDE, env0 + e, act + e * AW, shapes, draws + e);
             float r = 0.0f, d = 0.0f;
-            step_finish_quads<E, CAP>(rows, cts, shapes, dlist, dcount, carry, wired != 0, lane, ne, r, d);
+            step_finish_quads<E, CAP>(rows, cts, shapes, dlist, dcount, carry, wired, lane, ne, r, d);
             bool finished = false;
             if (first) {
                 a.r_rewards[row + e] = r;
@@ -183,7 +183,7 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
                 }
             }
             const unsigned long long fin = quad_envs(__ballot(finished));
-            wired |= (int)((fin >> e) & 1ull);
+            wired = ((fin >> e) & 1ull) != 0 ? 1 : wired;
             reset_rows<E>(rows, &was_reset, fin, a.reset_seed + (uint64_t)k * a.reset_stride, env0, lane);
         } else {
             // ---- the draw once more, for the rollout's action and log-probability, which nothing of the step waits for

@@ -43,19 +43,22 @@ MRL_DEV void physics_lanes(float *row, float *contacts, int n, int lane) {
     lane_body_load<L>(B, row, b);
     const float *F = row + L::FORCES_OFF + b * 3;
     lane_integrate_velocity(B, F[0], F[1], F[2], gx, gy, dt);
-    LaneJoints<Wiring> J;
-    J.load<L>(row, l, B, dt);
+    LaneJoints<Wiring, false> usual(l);
+    usual.load<L>(row, l, B, dt);
     LaneListContacts<L, 2> list;
     list.load(B, contacts, n, body, baumgarte);
     float sn, cs;
     sincos32(B.ang[0], sn, cs);
-    body_lanes_solve<Wiring, 6, 2>(B, J, list, sn, cs, dt, friction, restitution, baumgarte);
+    with_joints<L>(usual, row, l, B, dt, !usual.usual<L>(row, l, B), [&](auto &J) {
+        body_lanes_solve<Wiring, std::decay_t<decltype(J)>::ALL, 6, 2>(B, J, list, sn, cs, dt, friction, restitution, baumgarte);
+    });
     if (has) lane_body_store<L>(B, row, b);
     // ---- observation entries 0 .. 7 and 9 .. 12 (observe_state: the same expressions on the same values), every
     // body's lane its own: the hull 0 .. 3, a leg segment its angle and angular velocity against its parent's.
     // The contact flags (8, 13) and the lidar are left to what follows (step_tail<false, false>).
     {
-        const double p_ang = (double)J.parent(B.ang[0], B.ang[0]), p_w = (double)J.parent(B.w[0], B.w[0]);
+        const LaneSlots<Wiring> slots(l);
+        const double p_ang = (double)slots.parent(B.ang[0], B.ang[0]), p_w = (double)slots.parent(B.w[0], B.w[0]);
         if (body == 0) {
             const double hull_angle = B.ang[0], hull_omega = B.w[0], hull_vx = B.vx[0], hull_vy = B.vy[0];
             row[0] = (float)hull_angle;

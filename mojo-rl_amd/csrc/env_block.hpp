@@ -83,8 +83,9 @@ struct LunarLander {
     }
     // the same in parts, the physics by the four lanes of an env (step_finish_quads)
     static MRL_DEV bool row_done(const float *row) { return row[L::META_OFF + ll::META_DONE] > 0.5f; }
-    static MRL_DEV bool lanes_ok(const float *row) { return ll::lanes_row_ok(row); }
-    static MRL_DEV void physics_lanes(float *row, float *cts, int n, int lane) { ll::physics_lanes(row, cts, n, lane); }
+    static MRL_DEV int lanes_wired(const float *row) { return ll::lanes_wired(row); }
+    template <bool ANY>
+    static MRL_DEV void physics_lanes(float *row, float *cts, int n, int lane) { ll::physics_lanes<ANY>(row, cts, n, lane); }
     static MRL_DEV int physics_one(float *row, float *cts, int n, const float *shapes) { return ll::step_physics(row, cts, n, shapes); }
     static MRL_DEV void step_tail(float *row, const float *cts, int n, const Carry &c, float &r, float &d) {
         ll::step_tail(row, cts, n, c, r, d);
@@ -422,10 +423,10 @@ MRL_DEV void wave_sync_rows() {
 
 // E::step_finish for the 16 envs of one wavefront, four lanes per env, given the contact lists of the detection tasks: the
 // physics with one lane per body, the rest by the first lane of each env, which returns reward and done.  An env whose
-// wiring is not its kind's own (`ok` false), or with a list that overflowed, is stepped by its first lane alone.
+// wiring is not its kind's own (`wired` 0: E::lanes_wired), or with a list that overflowed, is stepped by its first lane alone.
 template <class E, int CAP>
 MRL_DEV void step_finish_quads(float *rows, float *cts, const float *shapes, const float *dlist, const int *dcount,
-                               const typename E::Carry &carry, bool ok, int lane, int ne, float &r, float &d) {
+                               const typename E::Carry &carry, int wired, int lane, int ne, float &r, float &d) {
     using S = Stage<E>;
     const int e = lane >> 2, l = lane & 3;
     if (e >= ne) return;
@@ -433,9 +434,14 @@ MRL_DEV void step_finish_quads(float *rows, float *cts, const float *shapes, con
     wave_sync_rows();   // (the engines' velocities, written by the first lanes)
     int n = merge_vertex_lists_quads<E, CAP>(dlist, dcount, e, l, mine);
     wave_sync_rows();
-    const bool moves = !E::row_done(row), quad = moves && n >= 0 && ok;
-    if (quad) E::physics_lanes(row, mine, n, lane);
-    else if (moves && l == 0) n = E::physics_one(row, mine, n, shapes);
+    const bool moves = !E::row_done(row);
+    // (rows that are not the reset's behind one branch: with a second one in their way, usual rows took 0.7 % longer)
+    if (moves && n >= 0 && wired == 1) {
+        E::template physics_lanes<false>(row, mine, n, lane);
+    } else if (moves) {
+        if (n >= 0 && wired == 2) E::template physics_lanes<true>(row, mine, n, lane);
+        else if (l == 0) n = E::physics_one(row, mine, n, shapes);
+    }
     wave_sync_rows();
     if (l == 0) E::step_tail(row, mine, n, carry, r, d);
 }
@@ -480,10 +486,10 @@ MRL_DEV void phys_step_block(float *rows, float *cts, const float *shapes, float
         const bool first = slot < nenv && (lane & 3) == 0;
         typename E::Carry carry{};
         EpisodeSums sums{0.0f, 0.0f};
-        bool ok = false;
+        int wired = 0;
         if (wave == 0) {
             if (first) sums = account_before(acc, slot);
-            if (slot < nenv) ok = E::lanes_ok(rows + slot * S::STRIDE);
+            if (slot < nenv) wired = E::lanes_wired(rows + slot * S::STRIDE);
             if (first)
                 carry = E::step_begin(rows + slot * S::STRIDE, env0 + slot, actions + (size_t)slot * E::ACT_W, shapes);
         } else {
@@ -496,7 +502,7 @@ MRL_DEV void phys_step_block(float *rows, float *cts, const float *shapes, float
         if (wave == 0) {
             bool finished = false;
             float r = 0.0f, d = 0.0f;
-            step_finish_quads<E, DETECT_CAP>(rows, cts, shapes, dlist, dcount, carry, ok, lane, nenv, r, d);
+            step_finish_quads<E, DETECT_CAP>(rows, cts, shapes, dlist, dcount, carry, wired, lane, nenv, r, d);
             if (first) {
                 if (rewards != nullptr) {
                     rewards[slot] = r;

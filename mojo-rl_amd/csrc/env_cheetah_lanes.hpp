@@ -39,8 +39,7 @@ MRL_DEV void wave_sync_lds() {
 template <class V>
 MRL_DEV V group_get(V v, int base, int src) { return __shfl(v, base + src, 64); }
 
-// true when the row has the wiring and shapes this form assumes (the motors' speeds and torques are the step's own; any
-// flags but limit and motor, or a joint with nothing to turn, are the one-lane form's)
+// true when the row has the wiring and shapes this form assumes
 MRL_DEV bool lanes_row_ok(const float *row, const float *shapes) {
     bool ok = body_lanes_row_ok<L, Topology, Wiring>(row);
     for (int b = 0; b < 7; ++b) {
@@ -127,8 +126,8 @@ MRL_DEV void step_lanes(float *row, const float *shapes, const float *action, in
     lane_body_load<L>(B, row, b);
     const float *F = row + L::FORCES_OFF + b * 3;
     float fx = F[0], fy = F[1], tau = F[2];
-    LaneJoints<Wiring> J;
-    J.load<L>(row, l, B, dt);
+    LaneJoints<Wiring, false> usual(l);
+    usual.load<L>(row, l, B, dt);
     const float *S = shapes + (int)row[L::BODIES_OFF + b * BODY_SIZE + IDX_SHAPE] * SHAPE_SIZE;
     const int n_verts = has ? (int)S[1] : 0;
     float lvx[4], lvy[4];
@@ -140,45 +139,47 @@ MRL_DEV void step_lanes(float *row, const float *shapes, const float *action, in
     sincos32(B.ang[0], sn, cs);
     GroundContacts contacts;
     contacts.kept = 0;
+    with_joints<L>(usual, row, l, B, dt, !usual.usual<L>(row, l, B), [&](auto &J) {
 #pragma unroll 1
-    for (int sub = 0; sub < 5; ++sub) {
-        lane_integrate_velocity(B, fx, fy, tau, gx, gy, dt);
-        fx = fy = tau = 0.0f;   // the forces are cleared at the end of every sub-step
-        // ---- contacts, compacted in vertex order
-        float px[4] = {0.0f, 0.0f, 0.0f, 0.0f}, py[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        int found = 0;
+        for (int sub = 0; sub < 5; ++sub) {
+            lane_integrate_velocity(B, fx, fy, tau, gx, gy, dt);
+            fx = fy = tau = 0.0f;   // the forces are cleared at the end of every sub-step
+            // ---- contacts, compacted in vertex order
+            float px[4] = {0.0f, 0.0f, 0.0f, 0.0f}, py[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            int found = 0;
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const float world_x = B.x[0] + lvx[v] * cs - lvy[v] * sn;
-            const float world_y = B.y[0] + lvx[v] * sn + lvy[v] * cs;
-            const bool hit = v < n_verts && 0.0f - world_y > 0.0f;
+            for (int v = 0; v < 4; ++v) {
+                const float world_x = B.x[0] + lvx[v] * cs - lvy[v] * sn;
+                const float world_y = B.y[0] + lvx[v] * sn + lvy[v] * cs;
+                const bool hit = v < n_verts && 0.0f - world_y > 0.0f;
 #pragma unroll
-            for (int c = 0; c <= v; ++c) {
-                px[c] = hit && found == c ? world_x : px[c];
-                py[c] = hit && found == c ? world_y : py[c];
+                for (int c = 0; c <= v; ++c) {
+                    px[c] = hit && found == c ? world_x : px[c];
+                    py[c] = hit && found == c ? world_y : py[c];
+                }
+                found += hit ? 1 : 0;
             }
-            found += hit ? 1 : 0;
-        }
-        // the list of an env is cut at MAX_CONTACTS in (body, vertex) order: contacts before mine are counted, where the
-        // list can be that long
-        contacts.kept = found;
-        if (any_lane(found > L::MAX_CONTACTS / 7)) {
-            int before = 0;
+            // the list of an env is cut at MAX_CONTACTS in (body, vertex) order: contacts before mine are counted, where the
+            // list can be that long
+            contacts.kept = found;
+            if (any_lane(found > L::MAX_CONTACTS / 7)) {
+                int before = 0;
 #pragma unroll
-            for (int o = 0; o < 7; ++o) {
-                const int c = group_get(found, base, Wiring::LANE_OF[o]);
-                before += o < body ? c : 0;
+                for (int o = 0; o < 7; ++o) {
+                    const int c = group_get(found, base, Wiring::LANE_OF[o]);
+                    before += o < body ? c : 0;
+                }
+                const int left = L::MAX_CONTACTS - before;
+                contacts.kept = left < 0 ? 0 : (left > found ? found : left);
             }
-            const int left = L::MAX_CONTACTS - before;
-            contacts.kept = left < 0 ? 0 : (left > found ? found : left);
-        }
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            if (!any_lane(c < contacts.kept)) break;
-            contacts.c[c].prepare(B, c < contacts.kept, px[c], py[c], 0.0f, 1.0f, 0.0f - py[c], baumgarte);
+            for (int c = 0; c < 4; ++c) {
+                if (!any_lane(c < contacts.kept)) break;
+                contacts.c[c].prepare(B, c < contacts.kept, px[c], py[c], 0.0f, 1.0f, 0.0f - py[c], baumgarte);
+            }
+            body_lanes_solve<Wiring, std::decay_t<decltype(J)>::ALL, 4, 2>(B, J, contacts, sn, cs, dt, friction, restitution, baumgarte);
         }
-        body_lanes_solve<Wiring, 4, 2>(B, J, contacts, sn, cs, dt, friction, restitution, baumgarte);
-    }
+    });
     // ---- bodies and forces back into the row, then the rest of the step on the torso's lane
     if (has) lane_body_store<L>(B, row, b);
     int penalised = 0;   // contacts of the last sub-step on anything but the feet (bodies 3 and 6)
@@ -191,7 +192,8 @@ MRL_DEV void step_lanes(float *row, const float *shapes, const float *action, in
     // entries: the torso its height, angle and velocity, a leg segment its angle and angular velocity
     // against its parent's
     {
-        const double p_ang = (double)J.parent(B.ang[0], B.ang[0]), p_w = (double)J.parent(B.w[0], B.w[0]);
+        const LaneSlots<Wiring> slots(l);
+        const double p_ang = (double)slots.parent(B.ang[0], B.ang[0]), p_w = (double)slots.parent(B.w[0], B.w[0]);
         if (body == 0) {
             row[0] = B.y[0]; row[1] = B.ang[0]; row[8] = B.vx[0]; row[9] = B.vy[0]; row[10] = B.w[0];
         } else if (has) {

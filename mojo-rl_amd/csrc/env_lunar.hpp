@@ -345,9 +345,14 @@ struct Wiring {
     static constexpr uint32_t JOINT[2] = {0x0000u, 0x0101u};
     static constexpr bool SPRING = true, MOTOR = false, ANGLES_AFTER = false, LAST_TURNS_FIRST = true;
 };
-MRL_DEV bool lanes_row_ok(const float *row) { return body_lanes_row_ok<L, Topology, Wiring>(row); }
+// 0: a row that the lanes cannot step, 1: one with the joint terms of the reset, 2: with others.  No step changes it, and a reset
+// makes it 1.
+MRL_DEV int lanes_wired(const float *row) {
+    return !body_lanes_row_ok<L, Topology, Wiring>(row) ? 0 : body_lanes_row_usual<L, Topology, Wiring>(row) ? 1 : 2;
+}
 
-// step_physics by the four lanes of an env, given its n >= 0 contacts
+// step_physics by the four lanes of an env, given its n >= 0 contacts; ANY: a row of other joint terms
+template <bool ANY>
 MRL_DEV void physics_lanes(float *row, float *contacts, int n, int lane) {
     const int l = lane & 3, body = lane_body<Wiring>(l);
     const bool has = body < L::NUM_BODIES;
@@ -358,13 +363,13 @@ MRL_DEV void physics_lanes(float *row, float *contacts, int n, int lane) {
     lane_body_load<L>(B, row, b);
     const float *F = row + L::FORCES_OFF + b * 3;
     lane_integrate_velocity(B, F[0], F[1], F[2], gx, gy, dt);
-    LaneJoints<Wiring> J;
-    J.load<L>(row, l, B, dt);
+    LaneJoints<Wiring, ANY> J(l);
+    J.template load<L>(row, l, B, dt);
     LaneListContacts<L, 2> list;
     list.load(B, contacts, n, body, baumgarte);
     float sn, cs;
     sincos32(B.ang[0], sn, cs);
-    body_lanes_solve<Wiring, 6, 2>(B, J, list, sn, cs, dt, friction, restitution, baumgarte);
+    body_lanes_solve<Wiring, ANY, 6, 2>(B, J, list, sn, cs, dt, friction, restitution, baumgarte);
     if (has) lane_body_store<L>(B, row, b);
 }
 
