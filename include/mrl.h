@@ -115,6 +115,10 @@ int mrl_ctx_reserve(mrl_ctx *ctx, uint64_t mlp_floats, uint64_t rollout_floats);
 #define MRL_DEFAULT_SPIN_LIMIT (1u << 22)
 int mrl_ctx_set_spin_limit(mrl_ctx *ctx, unsigned polls);
 
+/* How many of its minibatches the context's last mrl_ppo_update_minibatch / _epoch call enqueued: all of them,
+ * or fewer where the host saw the KL stop while it was enqueueing (those left away would have done nothing). */
+int mrl_ctx_update_enqueued(mrl_ctx *ctx, int *minibatches);
+
 /* Device-time accounting per phase, the counterpart of the perf_counter_ns phase timers that
  * train_gpu prints (deep_agents/ppo/ppo.mojo:2062-2067, :2777-2838) measured with HIP events on
  * the context's stream instead of host enqueue times.  mrl_profile_begin arms it (at most

@@ -57,6 +57,12 @@ class DeviceContext:
         wait that gives up makes the next synchronize() raise; a tiny value exercises that path."""
         _lib.call("mrl_ctx_set_spin_limit", self.handle, int(polls))
 
+    def update_enqueued(self):
+        """How many minibatches the last update call enqueued (fewer than it was given: the KL stop was seen meanwhile)."""
+        n = C.c_int(0)
+        _lib.call("mrl_ctx_update_enqueued", self.handle, C.byref(n))
+        return n.value
+
     PHASES = ("policy_fwd", "sample_store", "env_step", "post_store", "collect")
 
     def profile_begin(self, max_marks=8192, sample_every=1):

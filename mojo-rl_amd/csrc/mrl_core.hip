@@ -75,6 +75,7 @@ int mrl_ctx_create(void *hip_stream, mrl_ctx **out) {
     c->stop_seen = c->sync_error + 8;
     *c->stop_seen = 0;
     c->stop_call = 0;
+    c->upd_enqueued = 0;
     {
         int rc = mrl::clip_static_setup(c->device);
         if (rc != MRL_OK) { mrl_ctx_destroy(c); return rc; }
@@ -131,6 +132,12 @@ int mrl_ctx_reserve(mrl_ctx *ctx, uint64_t mlp_floats, uint64_t rollout_floats) 
 int mrl_ctx_set_spin_limit(mrl_ctx *ctx, unsigned polls) {
     MRL_CHECK_ARG(ctx != nullptr, "mrl_ctx_set_spin_limit: ctx is NULL");
     ctx->spin_limit = polls == 0 ? MRL_DEFAULT_SPIN_LIMIT : polls;
+    return MRL_OK;
+}
+
+int mrl_ctx_update_enqueued(mrl_ctx *ctx, int *minibatches) {
+    MRL_CHECK_ARG(ctx != nullptr && minibatches != nullptr, "mrl_ctx_update_enqueued: NULL argument");
+    *minibatches = ctx->upd_enqueued;
     return MRL_OK;
 }
 

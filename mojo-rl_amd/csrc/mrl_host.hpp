@@ -45,6 +45,7 @@ struct mrl_ctx {
     // sync_error): the host leaves launches away that would find the stop raised and do nothing.
     int stop_call;
     int *stop_seen;
+    int upd_enqueued;   // minibatches that the last update call enqueued
     // CarRacingV2: 0 = the CPU env's reward / termination arithmetic (default), 1 = the GPU trait's
     int car_trait_form;
     // phase timing: events recorded on `stream` at phase boundaries while armed

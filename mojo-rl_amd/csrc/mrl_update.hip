@@ -571,10 +571,12 @@ static int update_minibatch_layers(mrl_ctx *ctx, const mrl_update *u, const int3
 // Minibatches 0 .. n - 1 of `indices`, with step counts t0 + 1 ..
 static int update_minibatches(mrl_ctx *ctx, const mrl_update *u, const int32_t *indices, int n, int actor_t0, int critic_t0) {
     int rc;
+    ctx->upd_enqueued = 0;
     if (!update_paired(u)) {
         for (int k = 0; k < n; ++k) {
             rc = update_minibatch_layers(ctx, u, indices + (size_t)k * u->minibatch, actor_t0 + k + 1, critic_t0 + k + 1);
             if (rc) return rc;
+            ctx->upd_enqueued += 1;
         }
         return MRL_OK;
     }
@@ -608,6 +610,7 @@ static int update_minibatches(mrl_ctx *ctx, const mrl_update *u, const int32_t *
         rc = update_minibatch_paired(ctx, u, indices + (size_t)k * u->minibatch, actor_t0 + k + 1, critic_t0 + k + 1,
                                      stats + 2 * (k - s0), ws, k + 1 < n);
         if (rc) return rc;
+        ctx->upd_enqueued += 1;
     }
     return MRL_OK;
 }
@@ -638,6 +641,7 @@ int mrl_minibatch_adv_stats(mrl_ctx *ctx, const int32_t *indices, const float *a
 int mrl_ppo_update_epoch(mrl_ctx *ctx, const mrl_update *u, const int32_t *indices, int n_minibatches,
                          int actor_t0, int critic_t0) {
     MRL_CHECK_ARG(ctx != nullptr, "mrl_ppo_update_epoch: ctx is NULL");
+    ctx->upd_enqueued = 0;
     int rc = update_check(u, "mrl_ppo_update_epoch");
     if (rc) return rc;
     MRL_CHECK_ARG(n_minibatches >= 0 && actor_t0 >= 0 && critic_t0 >= 0, "mrl_ppo_update_epoch: negative count");
