@@ -138,14 +138,9 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
                         sample_gaussian_part(lg + j, w2a + HEAD_LOG_STD(H) + j, 1, A, j, sseed, i, &av);
                         act[e * AW + j] = av;
                     }
-                } else if (A <= 4) {
+                } else {   // (four actions: the entry refuses any other head)
                     const int sel = sample_categorical_quad(lg, A, sseed, i, lane & 3);
                     if (first) act[e] = (float)sel;
-                } else if (first) {
-                    int sel;
-                    float logp;
-                    sample_categorical_few(lg, A, sseed, i, sel, logp);
-                    act[e] = (float)sel;
                 }
             }
         } else if (vw == 3 && lane < ne) {   // ---- what the engines need whatever the action is

@@ -77,11 +77,7 @@ struct LunarLander {
     static MRL_DEV Carry step_begin(float *row, int env, const float *a, const float *shapes, const ll::EngineDraw *draw = nullptr) {
         return ll::step_begin(row, env, (int)a[0], shapes, draw);
     }
-    static MRL_DEV void step_finish(float *row, float *cts, int n, const float *shapes, const Carry &c, float &r,
-                                    float &d) {
-        ll::step_finish(row, cts, n, shapes, c, r, d);
-    }
-    // the same in parts, the physics by the four lanes of an env (step_finish_quads)
+    // the rest of a step in parts, the physics by the four lanes of an env (step_finish_quads)
     static MRL_DEV bool row_done(const float *row) { return row[L::META_OFF + ll::META_DONE] > 0.5f; }
     static MRL_DEV int lanes_wired(const float *row) { return ll::lanes_wired(row); }
     template <bool ANY>
@@ -329,7 +325,7 @@ MRL_DEV void reset_rows_block(float *rows, unsigned long long mask, uint64_t see
 }
 
 // Per-(body, vertex) contact lists of phys_step_block: CAP records per list (a vertex that fills
-// its list sends the env back to detection inside step_finish), list stride in floats.
+// its list sends the env back to detection by one lane), list stride in floats.
 constexpr int DETECT_CAP = 4;
 constexpr int detect_stride(int cap) { return (cap * CONTACT_SIZE) | 1; }
 constexpr int DETECT_STRIDE = detect_stride(DETECT_CAP);
@@ -452,17 +448,17 @@ MRL_DEV unsigned long long quad_envs(unsigned long long m) {
     return out;
 }
 
-// One step of the block's LDS-resident rows (all threads of the block call it, between two
-// __syncthreads of the caller): wavefront 0 steps one env per lane, the other wavefronts detect
-// contacts where the env splits that off.  `actions` = the actions of the block's envs
-// ([nenv][ACT_W], global or LDS), rewards / dones = the block's slice of the per-step outputs
-// (may be null), acc = rollout accounting with its pointers already offset to the block's first
-// env.  AUTORESET: rows that finished are re-initialised in place and recorded in *was_reset.
-// (what phys_step_block runs beside the one-lane-per-body solver when the caller has nothing for it)
+// what phys_step_block runs beside the one-lane-per-body solver when the caller has nothing for it
 struct NoSideJob {
     MRL_DEV void operator()(int) const {}
 };
 
+// One step of the block's LDS-resident rows (all threads of the block call it, between two
+// __syncthreads of the caller): wavefront 0 (LANES_PHYSICS envs: 0 and 1) steps the envs, four or
+// eight lanes each, the other wavefronts detect contacts.  `actions` = the actions of the block's envs
+// ([nenv][ACT_W], global or LDS), rewards / dones = the block's slice of the per-step outputs
+// (may be null), acc = rollout accounting with its pointers already offset to the block's first
+// env.  AUTORESET: rows that finished are re-initialised in place and recorded in *was_reset.
 // `side`: work of the caller's that the wavefronts without a part in the one-lane-per-body solver (LANES_PHYSICS
 // envs: wavefronts 2 and up) do while wavefronts 0 and 1 run it, called as side(tid) between the two block
 // barriers around the solver; it must not touch the rows or the contact scratch `cts`.
@@ -476,7 +472,7 @@ MRL_DEV void phys_step_block(float *rows, float *cts, const float *shapes, float
         // wavefront 0: first half of the step (reads and writes velocities only); the halves of the
         // other wavefronts: contacts of one (body, vertex) pair each (read positions only), into
         // lists of their own.  A vertex that fills its list, or a body whose shape the task table
-        // does not cover, sends that env back to detection inside step_finish.
+        // does not cover, sends that env back to detection by its first lane (step_finish_quads).
         // (a wavefront holds WAVE / EPB tasks at a time; a block with fewer such groups than tasks takes turns)
         constexpr int NT = E::DETECT_TASKS, GROUP = E::EPB, PER_WAVE = WAVE / GROUP;
         constexpr int AT_ONCE = (E::THREADS / WAVE - 1) * PER_WAVE;

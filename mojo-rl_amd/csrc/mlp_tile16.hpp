@@ -237,10 +237,9 @@ MRL_DEV float dpp_add(float x) {
 }
 template <int TPR>
 MRL_DEV float butterfly_sum(float x) {
-    static_assert(TPR == 4 || TPR == 8 || TPR == 16, "a quad, half a row or a row of lanes");
+    static_assert(TPR == 4 || TPR == 16, "a quad or a row of lanes");
     if constexpr (TPR == 16) x = dpp_add<0x128>(x);                       // row_ror:8
     if constexpr (TPR == 16) x = dpp_add<0x124>(x);                       // row_ror:4
-    if constexpr (TPR == 8) x += __shfl_xor(x, 4, 64);
     x = dpp_add<0x4E>(x);                                                 // quad_perm [2, 3, 0, 1]
     return dpp_add<0xB1>(x);                                              // quad_perm [1, 0, 3, 2]
 }
@@ -298,8 +297,8 @@ MRL_DEV void head_rows16(const float *w2s, int A, const float *h2, float *out, i
 
 template <int H>
 MRL_DEV void head16(const float *w2s, int A, const float *h2, float *out, int out_ld, int t, int nthreads) {
-    if constexpr (H == 128) return head_chain<H, PR16, PA_MAX>(w2s, A, h2, out, out_ld, t);
-    if (A == 1) head_rows16<H, 1, PA_MAX>(w2s, A, h2, out, out_ld, t, nthreads);
+    if constexpr (H == 128) head_chain<H, PR16, PA_MAX>(w2s, A, h2, out, out_ld, t);
+    else if (A == 1) head_rows16<H, 1, PA_MAX>(w2s, A, h2, out, out_ld, t, nthreads);
     else if (A <= 4) head_rows16<H, 4, PA_MAX>(w2s, A, h2, out, out_ld, t, nthreads);
     else head_rows16<H, 8, PA_MAX>(w2s, A, h2, out, out_ld, t, nthreads);
 }
