@@ -148,13 +148,6 @@ __global__ __launch_bounds__(64) void gae_kernel(int T, int N, const float *__re
     }
 }
 
-// a * b, and 0 where a or b is zero, whatever the other one is
-MRL_DEV float mul_zero_wins(float a, float b) {
-    float r;
-    asm("v_mul_legacy_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
-    return r;
-}
-
 // Below about one wavefront of envs per CU the plain scan waits for memory most of the time (T = 1000,
 // N = 4096: 63 waits on 64 CUs).  A = delta + decay * A is a serial chain per env, but a short one: three dependent instructions a
 // step.  What a plain scan waits for is memory, so the chain gets a wavefront of its own and eight
@@ -166,11 +159,19 @@ MRL_DEV float mul_zero_wins(float a, float b) {
 // multiplication whose zero times anything is zero, one sum, and half a load and a store.  EXACT, for a decay that is zero or
 // not finite: an episode's end could not be told from the decay there, and a zero times it is not zero; the factor is 1 or
 // 0, the scan selects by it and multiplies by the decay (the one more test is 50 cycles a step instead of 35).
-// What bounds it now is the chain up to 16 envs
-// per CU, then the memory (T = 1000, N = 8192: 5.6 TB/s).  Same operations in the same order as the scan (the sign of a zero
+// What bounds it: on inputs that are in the caches (a rollout just written) the chain up to 16 envs per CU, T = 1000,
+// N = 4096 19.5 us, then the memory (N = 8192: 5.7 TB/s); on inputs that are not, the trip to HBM, which a chunk's scan of a
+// microsecond no longer covers one chunk ahead: 29.8 us, 40.2 at N = 8192.  Same operations in the same order as the scan (the sign of a zero
 // aside).  A chunk's rows, and the value row above it, are read two barriers before the first of them is stored, so outputs may
 // share memory with the inputs.  deep_agents/ppo/ppo.mojo:2317-2353
 constexpr int GAE_LOADERS = 512;   // threads; one more wavefront scans
+
+// a * b, and 0 where a or b is zero, whatever the other one is
+MRL_DEV float mul_zero_wins(float a, float b) {
+    float r;
+    asm("v_mul_legacy_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
 
 template <int G, int R, bool EXACT>
 __global__ __launch_bounds__(GAE_LOADERS + 64) void gae_fed_kernel(int T, int N, const float *rewards, const float *values,
@@ -721,10 +722,14 @@ int mrl_gae(mrl_ctx *ctx, int T, int N, const float *rewards, const float *value
     if (T == 0 || N == 0) return MRL_OK;
     MRL_CHECK_ARG(rewards && values && dones && bootstrap && adv && ret, "mrl_gae: NULL buffer");
     // The narrowest groups that still give every group a CU of its own; with a wavefront of envs per CU the plain scan
-    // is the faster one.  us, plain / groups of 16 / 32 / 64 (with a test in the chain; now 18.4 at N = 1000, 19.2 at
-    // N = 4096, 28.3 at N = 8192): T = 1000, N = 1000: 57.5 / 22.2 / 26.3 / 30.5; N = 4096:
-    // 57.7 / 23.2 / 26.2 / 32.0; N = 8192: 58.0 / 43.0 / 29.1 / 35.2; T = 64, N = 16384: 6.4 / 10.6 / 7.4 / 5.8;
-    // N = 65536: 13.4 / - / - / 21.2.
+    // is the faster one.  us, plain / groups of 16 / 32 / 64, inputs in the caches : 700 MB of others read in between, T = 1000:
+    //   N = 1000   57.1 / 18.7 / 19.8 / 29.2 : 61.2 / 22.4 / 28.7 / 45.7
+    //   N = 4096   57.9 / 19.5 / 20.8 / 30.6 : 65.1 / 29.8 / 35.6 / 49.7
+    //   N = 4200   57.8 / 27.6 / 25.1 / 34.5 : 67.3 / 38.9 / 38.1 / 54.7
+    //   N = 8192   58.1 / 31.3 / 28.5 / 34.1 : 69.2 / 47.8 / 40.2 / 55.2
+    //   N = 8300   58.1 / 55.5 / 50.0 / 39.9 : 72.4 / 70.5 / 68.8 / 61.7
+    //   N = 16384  78.5 / 107 / 81.5 / 70.4 : 76.9 / 106 / 80.4 / 70.1
+    // T = 64: up to N = 8192 all 5.5 to 6.2, the call; N = 16384 6.5 / 8.2 / 5.7 / 5.6, N = 65536 13.5 / 26.8 / 19.3 / 16.8.
     const float g = (float)gamma, decay = (float)(gamma * lam);
     auto launch = [&](auto kernel, int groups, int threads = GAE_LOADERS + 64) {
         hipLaunchKernelGGL(kernel, dim3(groups), dim3(threads), 0, ctx->stream, T, N, rewards, values, dones,
