@@ -192,13 +192,13 @@ static CollectPlan collect_plan(const mrl_rollout *r, int n_cus) {
         // Up to this many envs per CU the walkers' fused kernels are the faster way; with more, their 16-env workgroups
         // come round after round while the stand-alone kernels fill the chip.  us per step, fused against two launches,
         // hidden width 64 / 256:
-        //   HalfCheetah (one workgroup per CU)  4096 envs 46 / 51 : 55 / 68,  8192 envs 93 / 103 : 56 / 80;
+        //   HalfCheetah (one workgroup per CU)  4096 envs 40 / 45 : 49 / 63,  8192 envs 80 / 90 : 50 / 75;
         //   Walker2d  4096 envs 12.4 / 22.3 : 17.7 / 31.7,  4200 envs 24.0 / 43.8 : 22.6 / 47.5,  8192 envs 24.4 / 44.0 : 19.9 / 44.5
         //     (width 128 27.7 : 27.4),  16384 envs 47 / 87 : 31 / 76;
         //   CarRacing  4096 envs 20 / 31 : 28 / 41,  8192 envs 39 / 61 : 41 / 65,  16384 envs 76 / 121 : 72 / 116;
         //   Hopper  8192 envs 9.6 / 36 : 15.3 / 39,  16384 envs 22 / 70 : 26 / 69,  32768 envs 38 / 138 : 36 / 129;
-        //   BipedalWalker  4096 envs 30 / 36 : 40 / 53,  8192 envs 58 / 70 : 68 / 93,  12288 envs 86 / 104 : 85 / 129,
-        //     16384 envs 114 / 138 : 91 / 135.
+        //   BipedalWalker  4096 envs 28 / 34 : 39 / 53,  8192 envs 56 / 66 : 67 / 91,  12288 envs 83 / 99 : 83 / 127,
+        //     16384 envs 110 / 132 : 90 / 133.
         int envs_per_cu = 32;
         if (id == MRL_ENV_HALFCHEETAH || (id == MRL_ENV_WALKER2D_PLANAR && p.H == 64)) envs_per_cu = 16;
         else if (id == MRL_ENV_BIPEDAL && p.H == 256) envs_per_cu = 48;

@@ -20,8 +20,8 @@
 // (BipedalWalker: 168 registers and 14.6 KB of LDS, eleven wavefronts per CU; HalfCheetah: 128 registers, four wavefronts
 // per SIMD).
 // us per step, workgroup form -> this one:
-//   BipedalWalker  4096: 34 -> 56   5000: 56 -> 57   8192: 65 -> 59   16384: 126 -> 70   65536: 450 -> 184
-//   HalfCheetah    8192: 47 -> 49  10000: 91 -> 60                   16384: 92 -> 64   65536: 357 -> 181
+//   BipedalWalker  4096: 33 -> 56   5000: 56 -> 56   8192: 64 -> 58   16384: 125 -> 70   65536: 446 -> 182
+//   HalfCheetah    8192: 42 -> 49  10000: 80 -> 60                   16384: 82 -> 64   65536: 317 -> 177
 #include <cmath>
 #include "mrl_host.hpp"
 #include "env_block.hpp"
