@@ -110,7 +110,9 @@ int mrl_ctx_reserve(mrl_ctx *ctx, uint64_t mlp_floats, uint64_t rollout_floats);
  * the last synchronize wrote is void then: a workgroup that gave up stores neither its env rows nor its
  * observations nor its episode sums (they keep the values from before the launch), the other workgroups'
  * envs have advanced, and rollout rows and the finished-episode list hold a mixture -- reset the envs
- * and clear done_count before collecting again.  No counterpart
+ * and clear done_count before collecting again.  The fused minibatch update has one such wait, of its last
+ * kernel's workgroups for each other's sums of squares: a workgroup that gives up leaves its share of the
+ * parameters, gradients and moments as they were, so parameters and optimiser state hold a mixture.  No counterpart
  * in the reference; a tiny limit is how a test exercises the error path without hanging anything. */
 #define MRL_DEFAULT_SPIN_LIMIT (1u << 22)
 int mrl_ctx_set_spin_limit(mrl_ctx *ctx, unsigned polls);

@@ -40,9 +40,10 @@ struct FwdLoss {
     float *g_actor_out, *g_values, *kl;                   // [mb, head], [mb], [mb]
     float *kl_part;                                       // [row tiles] sums of the tiles' KL estimates, for the test
     int32_t *kl_flag;                                     // null: no test (nothing is left in kl_part)
-    const int32_t *skip;                                  // *skip != 0: nothing of this minibatch is needed (null: a word that is 0)
+    const int32_t *skip;                                  // *skip != 0: nothing of this minibatch is needed
     // (The kernels request the word first, always, and test it behind their first requests.  0.6 us of a minibatch's 51 at
     // H = 256 and 4096 rows, for the 45 of one behind the stop.)
+    uint64_t *posts; int n_posts;                         // words to clear for the kernel that applies the update
     int dw_in_tiles;                                      // forward + backward: the row tiles leave their dW1 as well
     int mb, A, continuous, clip_value;                    // A = actions (discrete) or action width (continuous)
     float clip_eps, ent_coef, value_coef;
@@ -68,10 +69,13 @@ struct UpdateWs {
 };
 int mlp3_update_ws(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, int batch, const float *const *params, UpdateWs *out);
 int launch_split_weights(mrl_ctx *ctx, int H, const SplitNets &s, int n_nets);
+// the tiles and, where they do not leave it themselves, the hidden layers' weight gradient: pieces, not yet added up
+int mlp3_update_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int batch, Mlp3Nets io, const UpdateWs &ws, const FwdLoss &loss);
+struct SumNets;   // tile_sums.hpp
+SumNets mlp3_sum_nets(const mrl_mlp_desc *const *descs, int n_nets, const UpdateWs &ws, float *const *grads, const int32_t *skip);
 // sq_part (nullable): receives per-block sums of squares of the gradients, [net * 1024 + block];
 // *sq_blocks = number of blocks written (0 when none were)
-int mlp3_update_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int batch, Mlp3Nets io, const UpdateWs &ws,
-                  float *const *grads, float *sq_part, int *sq_blocks, const FwdLoss &loss);
+int mlp3_sum_tiles(mrl_ctx *ctx, const SumNets &sn, int tile_rows, float *sq_part, int *sq_blocks);
 int launch_fwd16(mrl_ctx *ctx, int H, int act, int batch, int IN, const Mlp3Net &nn);
 int launch_bwd(mrl_ctx *ctx, int H, int act, int batch, int IN, int rows, const Mlp3Net &nn, bool dw_in_tiles);
 int launch_dw_frag(mrl_ctx *ctx, int H, int n_nets, int batch, const UpdateWs &ws, int P0, int Ptot, int w1_off, const int32_t *skip);

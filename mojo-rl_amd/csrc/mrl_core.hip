@@ -58,6 +58,17 @@ int mrl_ctx_create(void *hip_stream, mrl_ctx **out) {
     c->spin_limit = MRL_DEFAULT_SPIN_LIMIT;
     CTX_TRY(hipGetDevice(&c->device));
     CTX_TRY(hipDeviceGetAttribute(&c->n_cus, hipDeviceAttributeMultiprocessorCount, c->device));
+    c->stream_cus = c->n_cus;
+    {
+        uint32_t mask[32] = {};   // (1024 CUs)
+        int set = 0;
+        if (hipExtStreamGetCUMask(c->stream, 32, mask) == hipSuccess) {
+            for (uint32_t m : mask) set += __builtin_popcount(m);
+            if (set > 0) c->stream_cus = std::min(c->n_cus, set);
+        } else {
+            (void)hipGetLastError();
+        }
+    }
     mrl::ll::Shapes sh = mrl::ll::make_shapes();
     CTX_TRY(hipMalloc(&c->ll_shapes, sizeof(sh)));
     CTX_TRY(hipMemcpy(c->ll_shapes, &sh, sizeof(sh), hipMemcpyHostToDevice));

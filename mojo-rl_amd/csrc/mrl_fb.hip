@@ -119,6 +119,8 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
     }
     if (actor && fl.adv_stats != nullptr) { l_mean = fl.adv_stats[0]; l_std = fl.adv_stats[1]; }
     if (skip != 0) return;
+    if (blockIdx.x == 0 && actor)
+        for (int i = t; i < fl.n_posts; i += T) fl.posts[i] = 0;
     // (the weights last: a wavefront's loads come back in order, and the rows are waited for first)
     __builtin_amdgcn_sched_barrier(0);
     bf16x8 wq[PF][NT][SPLIT];

@@ -13,7 +13,7 @@
 #include "mlp_tile.hpp"
 #include "mlp_split.hpp"
 #include "mlp3.hpp"
-#include <type_traits>
+#include "tile_sums.hpp"
 
 namespace mrl {
 
@@ -83,107 +83,21 @@ __global__ __launch_bounds__(2 * H) void mlp3_fwd_kernel(int B, int IN, Mlp3Net 
     }
 }
 
-// Flat gradient vector of each net from the pieces: weight blocks = sum over the batch splits of
-// `partial`, bias rows and the log_std tail (Gaussian head) = sum over the row tiles of the column
-// sums the tiles left.  The nets' vectors lie back to back in `partial`.
-struct SumNets {
-    float *grads[2];
-    const float *ls_part[2], *db_part[2], *thin_part[2];
-    int P[2], A[2];
-    int n, IN, H;
-    int thin_stride[2];   // floats per row tile in thin_part, per net
-    const int32_t *skip;   // as FwdLoss::skip, never null
-    int hh_in_tiles;   // the H x H block is summed from the row tiles' pieces (behind dW0 and dW2) instead of `partial`
-};
-
-// n terms of `p`, `stride` floats apart.  The chain of memory round trips is what this takes, so up to 64 terms are
-// requested at a time, and the last few of a number that is no multiple of 8 go out together as well: with a
-// request at a time behind the last 16, the sum over 63 tiles took 8.7 us of a minibatch's 31 (H = 128, 1000 rows), now 5.3.
-// They are added one after the other, or (TREE) what is requested together as a tree of neighbours, in the order it comes
-// back.  The pieces of 16-row tiles take the tree: they are twice as many as those of 32-row tiles, and one after the other
-// their roundings had made the gradients of 2048-row minibatches (H = 256, 24 inputs) less exact, 1.43e-7 -> 1.55e-7 off
-// Float64; as a tree 0.75e-7, in the same time.
 template <bool TREE>
-MRL_DEV float sum_strided(const float *__restrict__ p, size_t stride, int n) {
-    float s = 0.0f;
-    auto whole = [&](auto width) {
-        constexpr int W = decltype(width)::value;
-        float v[W];
-#pragma unroll
-        for (int k = 0; k < W; ++k) v[k] = p[(size_t)k * stride];
-        if constexpr (TREE) {
-#pragma unroll
-            for (int d = 1; d < W; d *= 2)
-#pragma unroll
-                for (int k = 0; k < W; k += 2 * d) v[k] += v[k + d];
-            s += v[0];
-        } else {
-#pragma unroll
-            for (int k = 0; k < W; ++k) s += v[k];
-        }
-        p += W * stride;
-        n -= W;
-    };
-    while (n >= 64) whole(std::integral_constant<int, 64>{});
-    if (n >= 32) whole(std::integral_constant<int, 32>{});
-    if (n >= 16) whole(std::integral_constant<int, 16>{});
-    if (n >= 8) whole(std::integral_constant<int, 8>{});
-    if (n > 0) {
-        float v[7];
-#pragma unroll
-        for (int k = 0; k < 7; ++k) {
-            v[k] = *p;
-            p += k + 1 < n ? stride : 0;   // (past the end: the last term again, not added)
-        }
-#pragma unroll
-        for (int k = 0; k < 7; ++k) s += k < n ? v[k] : 0.0f;
-    }
-    return s;
-}
-
-template <bool TREE>
-__global__ __launch_bounds__(256) void sum3_kernel(const float *__restrict__ partial, int splits, int Ptot,
-                                                   int tiles, SumNets sn, float *__restrict__ sq_part) {
+__global__ __launch_bounds__(256) void sum3_kernel(SumNets sn, float *__restrict__ sq_part) {
     const int skip = *sn.skip;
     __builtin_amdgcn_sched_barrier(0);
     __shared__ float red[2][4];
     const int gi = blockIdx.x * blockDim.x + threadIdx.x;
-    int net = 0;
+    const int P0 = sn.net[0].P, net = sn.n > 1 && gi >= P0 ? 1 : 0, i = gi - (net ? P0 : 0);
     float s = 0.0f;
-    if (gi < Ptot) {
-        int i = gi;
-        if (sn.n > 1 && i >= sn.P[0]) { net = 1; i -= sn.P[0]; }
-        const int IN = sn.IN, H = sn.H, A = sn.A[net];
-        const int o1 = (IN + 1) * H, o2 = o1 + (H + 1) * H, o3 = o2 + (H + 1) * A;
-        // which bias row (or the log_std tail) does i fall in?  -1: a weight
-        int bias_layer = -1, j = 0;
-        if (i >= IN * H && i < o1) { bias_layer = 0; j = i - IN * H; }
-        else if (i >= o1 + H * H && i < o2) { bias_layer = 1; j = i - (o1 + H * H); }
-        else if (i >= o2 + H * A && i < o3) { bias_layer = 2; j = i - (o2 + H * A); }
-        else if (i >= o3) { bias_layer = 3; j = i - o3; }
-        const float *p;
-        size_t stride;
-        int n;
-        if (bias_layer < 0 && i >= o1 && i < o1 + H * H && sn.hh_in_tiles) {
-            p = sn.thin_part[net] + (size_t)IN * H + (size_t)H * A + (i - o1);
-            stride = (size_t)sn.thin_stride[net];
-            n = tiles;
-        }
-        else if (bias_layer < 0 && i >= o1 && i < o1 + H * H) { p = partial + gi; stride = (size_t)Ptot; n = splits; }
-        else if (bias_layer < 0) {   // a weight of layer 0 or of the head: per-tile pieces
-            p = sn.thin_part[net] + (i < o1 ? i : (size_t)IN * H + (i - o2));
-            stride = (size_t)sn.thin_stride[net];
-            n = tiles;
-        }
-        else if (bias_layer == 3) { p = sn.ls_part[net] + j; stride = (size_t)A; n = tiles; }
-        else {
-            p = sn.db_part[net] + (bias_layer == 0 ? 0 : (bias_layer == 1 ? H : 2 * H)) + j;
-            stride = (size_t)(2 * H + PA_MAX);
-            n = tiles;
-        }
+    if (i < sn.net[net].P) {
+        const int o1 = (sn.IN + 1) * sn.H, HH = sn.H * sn.H;
+        const SumTerms inner = hidden_terms(sn.net[net], i - o1), outer = thin_terms(sn.net[net], sn.IN, sn.H, sn.tiles, i);
+        const bool in = i >= o1 && i < o1 + HH;
         if (skip == 0) {
-            s = sum_strided<TREE>(p, stride, n);
-            sn.grads[net][i] = s;
+            s = sum_terms<TREE, float>({in ? inner.p : outer.p, in ? inner.stride : outer.stride, in ? inner.n : outer.n});
+            sn.net[net].grads[i] = s;
         }
     }
     if (sq_part == nullptr) return;
@@ -286,36 +200,48 @@ static void dw_splits(int n_nets, int batch, int *splits, int *rows_per) {
     *splits = (batch + *rows_per - 1) / *rows_per;
 }
 
-// The sums over row tiles and batch splits into the flat gradients.
-static int sum_tiles(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, const Mlp3Nets &io, const UpdateWs &ws,
-                     float *const *grads, float *sq_part, int *sq_blocks, const int32_t *skip) {
+// where the pieces of a call's gradients lie
+SumNets mlp3_sum_nets(const mrl_mlp_desc *const *descs, int n_nets, const UpdateWs &ws, float *const *grads, const int32_t *skip) {
     const int IN = descs[0]->layers[0].in_dim, H = descs[0]->layers[0].out_dim;
     SumNets sn{};
     sn.n = n_nets;
     sn.IN = IN;
     sn.skip = skip;
     sn.H = H;
-    sn.hh_in_tiles = ws.dw_in_tiles ? 1 : 0;
-    int Ptot = 0;
+    sn.tiles = ws.tiles;
+    int Ptot = 0, at = 0;
+    for (int i = 0; i < n_nets; ++i) Ptot += net_P(*descs[i]);
     for (int i = 0; i < n_nets; ++i) {
-        const Mlp3Net &nn = io.n[i];
-        sn.grads[i] = grads[i];
-        sn.ls_part[i] = nn.ls_part;
-        sn.db_part[i] = nn.db_part;
-        sn.thin_part[i] = nn.thin_part;
-        sn.thin_stride[i] = nn.thin_stride;
-        sn.P[i] = net_P(*descs[i]);
-        sn.A[i] = nn.A;
-        Ptot += sn.P[i];
+        const Mlp3Net &from = ws.net[i];
+        SumNet &net = sn.net[i];
+        net.grads = grads[i];
+        net.ls = from.ls_part;
+        net.db = from.db_part;
+        net.thin = from.thin_part;
+        net.thin_stride = from.thin_stride;
+        net.P = net_P(*descs[i]);
+        net.A = descs[i]->layers[2].out_dim;
+        if (ws.dw_in_tiles) {   // behind dW0 and dW2 of every tile
+            net.hidden = from.thin_part + (size_t)IN * H + (size_t)H * net.A;
+            net.hidden_stride = from.thin_stride;
+            net.hidden_n = ws.tiles;
+        } else {                // the nets' vectors lie back to back in a split's
+            net.hidden = ws.partial + at + (IN + 1) * H;
+            net.hidden_stride = Ptot;
+            net.hidden_n = ws.splits;
+        }
+        at += net.P;
     }
-    const int sum_blocks = grid_for(Ptot, 256);
+    return sn;
+}
+
+// The sums over row tiles and batch splits into the flat gradients.
+int mlp3_sum_tiles(mrl_ctx *ctx, const SumNets &sn, int tile_rows, float *sq_part, int *sq_blocks) {
+    const int sum_blocks = grid_for(sn.net[0].P + (sn.n > 1 ? sn.net[1].P : 0), 256);
     if (sum_blocks > 1024) sq_part = nullptr;   // more partials than the caller's buffer holds
     if (sq_blocks) *sq_blocks = sq_part ? sum_blocks : 0;
-    auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(sum_blocks), dim3(256), 0, ctx->stream, ws.partial, ws.splits, Ptot, ws.tiles, sn, sq_part);
-    };
-    if (ws.rows == 16) launch(sum3_kernel<true>);
-    else launch(sum3_kernel<false>);
+    if (tile_rows == 16) hipLaunchKernelGGL(sum3_kernel<true>, dim3(sum_blocks), dim3(256), 0, ctx->stream, sn, sq_part);
+    else hipLaunchKernelGGL(sum3_kernel<false>, dim3(sum_blocks), dim3(256), 0, ctx->stream, sn, sq_part);
     MRL_CHECK_LAUNCH();
     return MRL_OK;
 }
@@ -370,8 +296,7 @@ int mlp3_update_ws(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int n_nets, i
     return MRL_OK;
 }
 
-int mlp3_update_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int batch, Mlp3Nets io, const UpdateWs &ws,
-                  float *const *grads, float *sq_part, int *sq_blocks, const FwdLoss &loss) {
+int mlp3_update_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int batch, Mlp3Nets io, const UpdateWs &ws, const FwdLoss &loss) {
     int H = 0, act = 0;
     bool gauss = false;
     for (int i = 0; i < 2; ++i) {
@@ -386,7 +311,6 @@ int mlp3_update_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int batch, Mlp
     }
     FwdLoss fl = loss;
     fl.dw_in_tiles = ws.dw_in_tiles ? 1 : 0;
-    if (fl.skip == nullptr) fl.skip = never_skip(ctx);
     int rc = launch_fb(ctx, H, act, batch, descs[0]->layers[0].in_dim, ws.rows, io, fl);
     if (rc) return rc;
     if (!ws.dw_in_tiles) {
@@ -394,7 +318,7 @@ int mlp3_update_n(mrl_ctx *ctx, const mrl_mlp_desc *const *descs, int batch, Mlp
         rc = launch_dw_frag(ctx, H, 2, batch, ws, P0, P0 + net_P(*descs[1]), (descs[0]->layers[0].in_dim + 1) * H, fl.skip);
         if (rc) return rc;
     }
-    return sum_tiles(ctx, descs, 2, io, ws, grads, sq_part, sq_blocks, fl.skip);
+    return MRL_OK;
 }
 
 // true when [a, a + na) and [b, b + nb) (floats) share memory
@@ -433,7 +357,7 @@ int mlp3_backward(mrl_ctx *ctx, const mrl_mlp_desc &d, int batch, const float *g
         rc = launch_dw_frag(ctx, H, 1, batch, ws, P, P, (IN + 1) * H, never_skip(ctx));
         if (rc) return rc;
     }
-    return sum_tiles(ctx, ds, 1, io, ws, gs, nullptr, nullptr, never_skip(ctx));
+    return mlp3_sum_tiles(ctx, mlp3_sum_nets(ds, 1, ws, gs, never_skip(ctx)), ws.rows, nullptr, nullptr);
 }
 
 }  // namespace mrl

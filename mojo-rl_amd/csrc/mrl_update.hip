@@ -4,8 +4,8 @@
 // forward, loss gradients, KL test, backward, global-norm clip, Adam (and the log_std clamp).
 // The actor and the critic do not depend on each other inside a minibatch, so when both have one
 // of the fused shapes they run side by side in every launch, and a row tile never leaves its
-// workgroup between the forward pass and the way back (mrl_fb.hip): 3 or 4 launches per minibatch (forward + loss
-// gradients + KL test + backward; dW of the hidden layer, where the tiles do not leave it; sum; clip + Adam) instead
+// workgroup between the forward pass and the way back (mrl_fb.hip): 2 or 3 launches per minibatch (forward + loss
+// gradients + KL test + backward; dW of the hidden layer, where the tiles do not leave it; sum + clip + Adam) instead
 // of about 40.  The minibatch is not gathered: the forward reads its rows from the rollout through the indices and the loss
 // normalises the advantage with statistics computed ahead (once per epoch for all minibatches).
 // Other net shapes go layer by layer: gather + normalise, forward, loss gradients + KL test,
@@ -22,6 +22,7 @@
 #include "mrl_device.hpp"
 #include "mlp_split.hpp"
 #include "mlp3.hpp"
+#include "tile_sums.hpp"
 #include "ppo_grads.hpp"
 
 namespace mrl {
@@ -301,12 +302,15 @@ MRL_DEV bool clip_verdict(const AdamArgs &a, float *smem, float &scale) {
 }
 
 // Adam (adam.mojo:52-105) on one parameter: gi = its clipped gradient
-MRL_DEV float adam_one(const AdamArgs &a, const AdamNet &net, float p, float gi, float &m, float &v) {
+template <class Args>
+MRL_DEV float adam_one(const Args &a, const AdamNet &net, float p, float gi, float &m, float &v) {
     m = a.beta1 * m + a.omb1 * gi;
     v = a.beta2 * v + a.omb2 * gi * gi;
     const float m_hat = m / net.bc1, v_hat = v / net.bc2;
     return p - net.lr * m_hat / (sqrtf(v_hat) + a.eps);
 }
+
+MRL_DEV float clamp_log_std(float p) { return p < -5.0f ? -5.0f : (p > 2.0f ? 2.0f : p); }
 
 // clip + Adam + log_std clamp (kernels.mojo:842-873) of element i
 MRL_DEV void adam_element(const AdamArgs &a, const AdamNet &net, int i, float p0, float g0, float2 mv, float scale) {
@@ -314,7 +318,7 @@ MRL_DEV void adam_element(const AdamArgs &a, const AdamNet &net, int i, float p0
     net.g[i] = gi;
     float p = adam_one(a, net, p0, gi, mv.x, mv.y);
     net.state[i] = mv;
-    if (i >= net.clamp_off && i < net.clamp_off + net.clamp_n) p = p < -5.0f ? -5.0f : (p > 2.0f ? 2.0f : p);
+    if (i >= net.clamp_off && i < net.clamp_off + net.clamp_n) p = clamp_log_std(p);
     net.p[i] = p;
 }
 
@@ -336,7 +340,6 @@ __global__ __launch_bounds__(UTPB) void clip_adam2_kernel(AdamArgs a) {
 // remaining parameters one per thread.  Everything that does not depend on the verdict is requested ahead of it.
 // Parameters lie on 16 bytes (the row tiles need that); gradients and moments may lie on any float, for instance as slices
 // of one vector: the same 16-byte accesses reach them there.
-typedef float f32x4a4 __attribute__((ext_vector_type(4), aligned(4)));
 template <int H>
 __global__ __launch_bounds__(UTPB) void clip_adam_split_kernel(AdamArgs a, int o1, SplitNets sp) {
     constexpr int WB = H * H / (8 * UTPB), ROWS = 8 * UTPB / H, TLD = H + 4;
@@ -411,6 +414,220 @@ static void launch_adam_split(hipStream_t st, const AdamArgs &a, int o1, const S
                        st, a, o1, sp);
 }
 
+// The sums over the tiles and splits, clip and Adam in one launch (the fused nets again).  A workgroup adds up the pieces of
+// its parameters, leaves the sum of their squares in `posts` for the others of its net, waits until all of these
+// are there and goes on to Adam with its gradients in registers: what crosses the chip between the two is 8 bytes per workgroup,
+// not the gradients, and a launch less is 2.5 us.  What bounds it: four trips to memory one after the other -- arguments,
+// pieces, the squares out, the squares in (H = 64, 256 rows: 8.5 thousand cycles, of which the pieces 2.8, the exchange 3.9),
+// and from H = 128 on the pieces' bytes (10 and 15 MB at 1000 and 4096 rows).  us per minibatch with sum3_kernel and
+// clip_adam_split_kernel : in one launch: H = 64, 256 rows 18.0 : 14.5; H = 128, 1000 rows 27.7 : 24.9; H = 256,
+// 4096 rows 55.5 : 52.7.
+//
+// The wait needs every workgroup of the grid on the chip, so the host takes this kernel only where the grid is no larger
+// than the CUs that the stream may use (sum_adam_fits); a CU holds four of these workgroups (256 threads, at most 128
+// registers), so that four such grids, from as many streams, hold no place that another one waits for, whatever
+// else comes and goes beside them.  And it is bounded: a workgroup that gives up after spin_limit polls reports it and
+// updates nothing.
+// W1: VW neighbouring columns per thread, so that a workgroup holds ROWS whole rows; the rest one parameter per thread.
+struct SumAdam {
+    struct Net {
+        AdamNet adam;
+        SumNet sum;
+        unsigned short *wf, *wb;   // split copies of W1; null: not kept
+    } net[2];
+    float max_norm, beta1, beta2, omb1, omb2, eps;
+    int IN, tiles;
+    const int32_t *skip;      // never null
+    uint64_t *posts;          // [net][gridDim.x]: 2^32 + the bits of a workgroup's sum of squares; zero before the launch
+    unsigned spin_limit;
+    int *sync_error;
+    int32_t *stop;            // the KL early stop's flag words; without a test a place with a zero and kl_n = 0
+    const float *kl_part;     // the row tiles' sums, never null
+    int kl_n, kl_mb;
+    float target_kl;
+    int *stop_seen;           // as AdamArgs::stop_seen, null: nobody looks
+    int stop_call;
+};
+
+template <int H, bool TREE>
+__global__ __launch_bounds__(UTPB, 4) void sum_adam_kernel(SumAdam k) {
+    constexpr int VW = H == 256 ? 4 : 1, E = UTPB * VW, ROWS = E / H, WB = H * H / E, TLD = H + 4, NW = UTPB / 64;
+    constexpr int KL_MOST = 1024;     // row tiles (update_paired)
+    typedef float MV __attribute__((ext_vector_type(2 * VW), aligned(4)));
+    typedef float V1 __attribute__((ext_vector_type(VW), aligned(4)));
+    typedef std::conditional_t<VW == 1, float, f32x4> Sum;
+    __shared__ __align__(16) float tile[ROWS * TLD];
+    __shared__ float sq_s[NW], kl_s[NW], total_s;
+    __shared__ int state_s;    // 0: update, 1: the KL stop, 2: the wait gave up
+    const int ynet = blockIdx.y, t = threadIdx.x;
+    const SumAdam::Net net = k.net[ynet];
+    const bool test = k.kl_n > 0;
+    // ---- requests
+    const int32_t skip = *k.skip, raised = k.stop[0];
+    float klq[KL_MOST / UTPB];
+#pragma unroll
+    for (int j = 0; j < KL_MOST / UTPB; ++j) klq[j] = k.kl_part[max(min(t + j * UTPB, k.kl_n - 1), 0)];
+    const int o1 = (k.IN + 1) * H;
+    const int TB = gridDim.x - WB;                    // the thin layers' workgroups go first: theirs are the long sums
+    const bool hidden = (int)blockIdx.x >= TB;
+    const int e0 = ((int)blockIdx.x - TB) * E + VW * t;                // element of W1
+    int i = blockIdx.x * UTPB + t;                    // a thin layer's parameter
+    if (i >= o1) i += H * H;
+    const bool mine = hidden || i < net.adam.n;
+    if (hidden) i = o1 + e0;
+    else i = min(i, net.adam.n - 1);
+    V1 p = V1{};
+    MV mv = MV{};
+    Sum s = Sum{};
+    if (hidden) {
+        p = *reinterpret_cast<const V1 *>(net.adam.p + i);
+        mv = *reinterpret_cast<const MV *>(net.adam.state + i);
+        __builtin_amdgcn_sched_barrier(0);
+        s = sum_terms<TREE, Sum>(hidden_terms(net.sum, e0));
+    } else {
+        const float2 one = net.adam.state[i];
+        p[0] = net.adam.p[i];
+        __builtin_amdgcn_sched_barrier(0);
+        const float x = sum_terms<TREE, float>(thin_terms(net.sum, k.IN, H, k.tiles, i));
+        mv[0] = one.x;
+        mv[1] = one.y;
+        if constexpr (VW == 1) s = mine ? x : 0.0f;
+        else s[0] = mine ? x : 0.0f;
+    }
+    // ---- the KL verdict, the same in every workgroup, and the norm
+    float q = 0.0f, kl = 0.0f;
+    if constexpr (VW == 1) q = s * s;
+    else q = (s[0] * s[0] + s[1] * s[1]) + (s[2] * s[2] + s[3] * s[3]);
+#pragma unroll
+    for (int j = 0; j < KL_MOST / UTPB; ++j) kl += t + j * UTPB < k.kl_n ? klq[j] : 0.0f;
+    q = dpp_wave_sum(q);
+    kl = dpp_wave_sum(kl);
+    if ((t & 63) == 0) { sq_s[t >> 6] = q; kl_s[t >> 6] = kl; }
+    __syncthreads();
+    if (t < 64) {
+        const float mean = ((kl_s[0] + kl_s[1]) + (kl_s[2] + kl_s[3])) / (float)k.kl_mb;
+        const bool over = test && mean > k.target_kl;
+        const bool first = __builtin_amdgcn_readfirstlane(raised) == 0;
+        const bool stop = test && (!first || over);
+        int state = stop ? 1 : 0;
+        float total = 0.0f;
+        if (!stop && k.max_norm > 0.0f) {
+            uint64_t *post = k.posts + (size_t)ynet * gridDim.x;
+            if (t == 0) {
+                const float own = (sq_s[0] + sq_s[1]) + (sq_s[2] + sq_s[3]);
+                __hip_atomic_store(post + blockIdx.x, (1ull << 32) | __float_as_uint(own), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+            // lane t takes the words t, t + 64, ..., one wait after the other: all but the first find theirs there
+            unsigned polls = 0;
+            for (int b0 = 0; b0 < (int)gridDim.x; b0 += 64) {
+                const bool in = b0 + t < (int)gridDim.x;
+                uint64_t word = 0;
+                for (;;) {
+                    if (in && word == 0) word = __hip_atomic_load(post + b0 + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if (!any_lane(in && word == 0)) break;
+                    if (++polls > k.spin_limit) { state = 2; break; }
+                }
+                total += __uint_as_float((uint32_t)word);
+            }
+            total = dpp_wave_sum(total);
+        }
+        if (t == 0) {
+            total_s = total;
+            state_s = state;
+            if (state == 2) __hip_atomic_store(k.sync_error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            if (stop && k.stop_seen != nullptr && blockIdx.x == 0 && ynet == 0)
+                __hip_atomic_store(k.stop_seen, k.stop_call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            if (test && first && blockIdx.x == 0 && ynet == 0) {
+                k.stop[1] = __float_as_int(mean);
+                if (over) k.stop[0] = 1;
+            }
+        }
+    }
+    __syncthreads();
+    const int state = state_s;
+    if (state != 0) {
+        // The gradients as they are.  (Nothing else hangs on `skip`: a workgroup of this launch may raise it while a wavefront
+        // reads it.)
+        if (state == 1 && skip == 0) {
+            if (hidden) *reinterpret_cast<V1 *>(net.adam.g + i) = s;
+            else if (mine) {
+                if constexpr (VW == 1) net.adam.g[i] = s;
+                else net.adam.g[i] = s[0];
+            }
+        }
+        return;
+    }
+    float scale = 1.0f;
+    if (k.max_norm > 0.0f) {
+        const float norm = sqrtf(total_s);
+        scale = norm > k.max_norm ? k.max_norm / (norm + 1e-8f) : 1.0f;
+    }
+    if (test && blockIdx.x == 0 && ynet == 0 && t == 0) k.stop[2] = k.stop[2] + 1;
+    V1 g = V1{};
+#pragma unroll
+    for (int j = 0; j < VW; ++j) {
+        if constexpr (VW == 1) g[j] = s * scale;
+        else g[j] = s[j] * scale;
+        if (j > 0 && !hidden) continue;
+        float m = mv[2 * j], v = mv[2 * j + 1];
+        p[j] = adam_one(k, net.adam, p[j], g[j], m, v);
+        mv[2 * j] = m;
+        mv[2 * j + 1] = v;
+    }
+    if (!hidden) {
+        if (!mine) return;
+        const bool clamped = i >= net.adam.clamp_off && i < net.adam.clamp_off + net.adam.clamp_n;
+        net.adam.g[i] = g[0];
+        net.adam.state[i] = make_float2(mv[0], mv[1]);
+        net.adam.p[i] = clamped ? clamp_log_std(p[0]) : p[0];
+        return;
+    }
+    *reinterpret_cast<V1 *>(net.adam.g + i) = g;
+    *reinterpret_cast<V1 *>(net.adam.p + i) = p;
+    *reinterpret_cast<MV *>(net.adam.state + i) = mv;
+    if (net.wf == nullptr) return;
+    // ---- the split copies: eight columns of a row, ROWS rows of a column
+    const int row0 = ((int)blockIdx.x - TB) * ROWS;
+#pragma unroll
+    for (int j = 0; j < VW; ++j) tile[(VW * t) / H * TLD + (VW * t) % H + j] = p[j];
+    __syncthreads();
+    if (t < E / 8) {
+        const int c8 = t % (H / 8), rl = t / (H / 8), row = row0 + rl;
+        f32x8 x;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] = tile[rl * TLD + 8 * c8 + j];
+        bf16x8 pc[SPLIT];
+        split8(x, pc);
+#pragma unroll
+        for (int j = 0; j < SPLIT; ++j)
+            *reinterpret_cast<bf16x8 *>(net.wb + split_frag<H>(c8 >> 2, row >> 4, j, (c8 & 3) * 16 + (row & 15))) = pc[j];
+    }
+    const int col = t - (UTPB - H);     // (at small widths the last wavefronts)
+    if (col >= 0) {
+        typedef float FR __attribute__((ext_vector_type(ROWS)));
+        typedef __bf16 BR __attribute__((ext_vector_type(ROWS)));
+        FR x;
+#pragma unroll
+        for (int j = 0; j < ROWS; ++j) x[j] = tile[j * TLD + col];
+        BR pc[SPLIT];
+        split_n<ROWS>(x, pc);
+        const int k8 = row0 >> 3;
+#pragma unroll
+        for (int j = 0; j < SPLIT; ++j)
+            *reinterpret_cast<BR *>(net.wf + split_frag<H>(k8 >> 2, col >> 4, j, (k8 & 3) * 16 + (col & 15)) + (row0 & 7)) = pc[j];
+    }
+}
+
+static int sum_adam_blocks(int H, const AdamArgs &a) {   // per net
+    return H * H / (UTPB * (H == 256 ? 4 : 1)) + grid_for(std::max(a.nets.n[0].n, a.nets.n[1].n) - H * H, UTPB);
+}
+template <int H>
+static void launch_sum_adam(hipStream_t st, const SumAdam &k, int blocks, bool tree) {
+    const dim3 grid(blocks, 2);
+    if (tree) hipLaunchKernelGGL((sum_adam_kernel<H, true>), grid, dim3(UTPB), 0, st, k);
+    else hipLaunchKernelGGL((sum_adam_kernel<H, false>), grid, dim3(UTPB), 0, st, k);
+}
+
 }  // namespace mrl
 
 using namespace mrl;
@@ -443,6 +660,7 @@ static int update_check(const mrl_update *u, const char *who) {
 // floats of ctx->upd_scratch: KL partials, their arrival counter, sum-of-squares partials, and the
 // advantage statistics of up to STATS_MAX minibatches
 constexpr int SCR_KL = 0, SCR_ARRIVED = 1024, SCR_SQ = 2048, SCR_STATS = 4096, STATS_MAX = 2048;
+constexpr int POSTS_MAX = 1024;   // 8-byte words of sum_adam_kernel where the sum-of-squares partials lie otherwise
 
 // both nets of the fused shapes, parameters that 16-byte loads can reach, a KL sum per row tile
 static bool update_paired(const mrl_update *u) {
@@ -490,27 +708,59 @@ static int update_minibatch_paired(mrl_ctx *ctx, const mrl_update *u, const int3
     fl.g_actor_out = u->g_actor_out; fl.g_values = u->g_values; fl.kl = u->kl;
     fl.kl_part = ctx->upd_scratch + SCR_KL;
     fl.kl_flag = u->target_kl > 0.0f ? u->kl_flag : nullptr;
-    fl.skip = more ? fl.kl_flag : nullptr;
+    fl.skip = more && fl.kl_flag != nullptr ? fl.kl_flag : never_skip(ctx);
     fl.mb = mb; fl.A = cont ? u->act_width : head; fl.continuous = cont ? 1 : 0;
     fl.clip_value = u->clip_value ? 1 : 0;
     fl.clip_eps = u->clip_epsilon; fl.ent_coef = u->entropy_coef; fl.value_coef = u->value_loss_coef;
-    float *grads[2] = {u->actor_grads, u->critic_grads};
-    int sq_blocks = 0;   // > 0: the sums over the tiles already left the sum-of-squares partials
-    int rc = mlp3_update_n(ctx, descs, mb, io, ws, grads, u->max_grad_norm > 0.0f ? ctx->upd_scratch + SCR_SQ : nullptr,
-                           &sq_blocks, fl);
-    if (rc) return rc;
     AdamArgs a{};
     adam_args(u, actor_t, critic_t, a);
-    a.partial = ctx->upd_scratch + SCR_SQ;
-    a.nb = sq_blocks;
-    a.part_stride = 1024;
     a.kl_part = u->target_kl > 0.0f ? ctx->upd_scratch + SCR_KL : nullptr;
     a.kl_n = ws.tiles;
     a.stop_seen = more && a.stop != nullptr ? ctx->stop_seen : nullptr;
     a.stop_call = ctx->stop_call;
     const int H = u->actor.layers[0].out_dim, o1 = (u->obs_dim + 1) * H;
+    const int blocks = sum_adam_blocks(H, a);
+    const bool one_launch = 2 * blocks <= std::min(ctx->stream_cus, POSTS_MAX);
+    if (one_launch) {
+        fl.posts = reinterpret_cast<uint64_t *>(ctx->upd_scratch + SCR_SQ);
+        fl.n_posts = 2 * blocks;
+    }
+    int rc = mlp3_update_n(ctx, descs, mb, io, ws, fl);
+    if (rc) return rc;
+    float *grads[2] = {u->actor_grads, u->critic_grads};
+    const SumNets sn = mlp3_sum_nets(descs, 2, ws, grads, fl.skip);
+    if (one_launch) {
+        SumAdam k{};
+        for (int i = 0; i < 2; ++i)
+            k.net[i] = {a.nets.n[i], sn.net[i], more ? ws.split.wf[i] : nullptr, more ? ws.split.wb[i] : nullptr};
+        k.max_norm = a.max_norm;
+        k.beta1 = a.beta1; k.beta2 = a.beta2; k.omb1 = a.omb1; k.omb2 = a.omb2; k.eps = a.eps;
+        k.IN = sn.IN; k.tiles = sn.tiles; k.skip = sn.skip;
+        k.posts = fl.posts;
+        k.spin_limit = ctx->spin_limit;
+        k.sync_error = ctx->sync_error;
+        const bool test = a.stop != nullptr;
+        k.stop = test ? a.stop : const_cast<int32_t *>(never_skip(ctx));
+        k.kl_part = ctx->upd_scratch + SCR_KL;
+        k.kl_n = test ? ws.tiles : 0;
+        k.kl_mb = mb;
+        k.target_kl = a.target_kl;
+        k.stop_seen = a.stop_seen;
+        k.stop_call = a.stop_call;
+        if (H == 256) launch_sum_adam<256>(ctx->stream, k, blocks, ws.rows == 16);
+        else if (H == 128) launch_sum_adam<128>(ctx->stream, k, blocks, ws.rows == 16);
+        else launch_sum_adam<64>(ctx->stream, k, blocks, ws.rows == 16);
+        MRL_CHECK_LAUNCH();
+        return MRL_OK;
+    }
     SplitNets sp{};
     if (more) sp = ws.split;
+    int sq_blocks = 0;   // > 0: the sums over the tiles already left the sum-of-squares partials
+    rc = mlp3_sum_tiles(ctx, sn, ws.rows, u->max_grad_norm > 0.0f ? ctx->upd_scratch + SCR_SQ : nullptr, &sq_blocks);
+    if (rc) return rc;
+    a.partial = ctx->upd_scratch + SCR_SQ;
+    a.nb = sq_blocks;
+    a.part_stride = 1024;
     if (H == 256) launch_adam_split<256>(ctx->stream, a, o1, sp);
     else if (H == 128) launch_adam_split<128>(ctx->stream, a, o1, sp);
     else launch_adam_split<64>(ctx->stream, a, o1, sp);
