@@ -280,6 +280,31 @@ MRL_DEV void stage_head(const float *__restrict__ W2, int H, int A, bool with_lo
     }
 }
 
+// The same in two halves, for T threads: the requests, and, once other requests are out too, the copy into LDS.  (In one
+// piece the copy waits for everything requested before it: 600 cycles and more of a kernel that has more to request.)
+// No branches on a lane's own place: such a load would be waited for at the branch's end.
+template <int H, int T>
+struct HeadLoads {
+    static constexpr int TOTAL = HEAD_LDS(H), N = (TOTAL + T - 1) / T;
+    float v[N];
+    MRL_DEV void load(const float *__restrict__ W2, int A, bool with_log_std, int t) {
+        const int rows = H + 1 + (with_log_std ? 1 : 0);
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const int i = t + k * T;
+            v[k] = W2[min(i / PA_MAX, rows - 1) * A + min(i % PA_MAX, A - 1)];
+        }
+    }
+    MRL_DEV void store(float *w2s, int A, bool with_log_std, int t) const {
+        const int rows = H + 1 + (with_log_std ? 1 : 0);
+#pragma unroll
+        for (int k = 0; k < N; ++k) {
+            const int i = t + k * T;
+            if (TOTAL % T == 0 || i < TOTAL) w2s[i] = i / PA_MAX < rows && i % PA_MAX < A ? v[k] : 0.0f;
+        }
+    }
+};
+
 // out[r][a] = h2[r] . W2[:, a] + b2[a] for the block's rows; TPR = H/16 lanes cooperate per row,
 // each over 16 consecutive columns that it walks from a different starting point (the lanes of a
 // wavefront then spread over the LDS banks, for the activations and for the padded weight rows

@@ -56,7 +56,7 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
     __shared__ __align__(16) float w2s[HEAD_LDS(H)];
     __shared__ float red[NW * R * (PA_MAX + 1)];
     __shared__ float g2s[R * GLD];
-    const Mlp3Net &nn = nets.n[blockIdx.y];
+    const Mlp3Net nn = nets.n[blockIdx.y];
     const float *__restrict__ params = nn.params;
     const int A = nn.A;
     const bool GAUSS = nn.gauss != 0;
@@ -68,20 +68,21 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
     float *__restrict__ thin_part = nn.thin_part + (size_t)blockIdx.x * (size_t)nn.thin_stride;
     const bool actor = blockIdx.y == 0;
 
-    // ---- everything that does not depend on an earlier phase is requested first.  Rows: sixteen lanes each.
+    // ---- Everything that does not depend on an earlier phase is requested first, the rows' indices (sixteen lanes a row;
+    // the loss: eight) ahead of everything.  A lane past the last row, input or output asks for the last one's
+    // value and drops it when it is used: behind a branch of its own every request would be waited for.
     const int skip = *fl.skip;   // (tested once these requests are out)
-    __builtin_amdgcn_sched_barrier(0);
     constexpr int XQ = (R * 16 + T - 1) / T;
-    long xsrc[XQ];
-    float xa[XQ], xb[XQ];
+    const int32_t *__restrict__ idx = fl.idx + row0;
+    int xsrc[XQ];
 #pragma unroll
-    for (int q = 0; q < XQ; ++q) {
-        const int r = (t + q * T) >> 4;
-        xsrc[q] = (r < nrow) ? fl.idx[row0 + r] : -1;
-    }
+    for (int q = 0; q < XQ; ++q) xsrc[q] = idx[min((t + q * T) >> 4, nrow - 1)];
     const int lr = t >> 3, lj = t & 7;           // loss lanes: eight per row
     const bool loss_row = lr < nrow && t < 8 * R;
-    const long lsrc = loss_row ? fl.idx[row0 + lr] : 0;
+    const int lsrc = idx[min(lr, nrow - 1)];
+    const float *lp_a = actor ? fl.r_adv : fl.r_ret, *lp_b = actor ? fl.r_logp : fl.r_val;
+    const float *stats = fl.adv_stats != nullptr ? fl.adv_stats : fl.r_adv;    // (of the advantages; or any place with a value)
+    const int act_w = fl.continuous ? fl.A : 1;
     float w0[NT][K0];
     f32x4 bias0[NT], bias1[NT];
     {
@@ -90,38 +91,29 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
         for (int q = 0; q < NT; ++q) {
             const int c = 16 * (NT * w + q);
 #pragma unroll
-            for (int s = 0; s < K0; ++s) w0[q][s] = 4 * s + g < IN ? W0[(4 * s + g) * H + c + n] : 0.0f;
+            for (int s = 0; s < K0; ++s)
+                if (s == 0 || 4 * s < IN) w0[q][s] = W0[min(4 * s + g, IN - 1) * H + c + n];
             bias0[q] = *reinterpret_cast<const f32x4 *>(b0 + c + 4 * g);
             bias1[q] = *reinterpret_cast<const f32x4 *>(b1 + c + 4 * g);
         }
     }
-    stage_head(params + IN * H + H + H * H + H, H, A, GAUSS, w2s, t, T);
+    HeadLoads<H, T> head;
+    const float *W2 = params + IN * H + H + H * H + H;
+    head.load(W2, A, GAUSS, t);
+    const float l_mean = stats[0], l_std = stats[fl.adv_stats != nullptr ? 1 : 0];
+    float ls = W2[(H + (GAUSS ? 1 : 0)) * A + min(lj, A - 1)];    // log_std (no Gaussian head: a bias, not used)
+    __builtin_amdgcn_sched_barrier(0);
+    float xa[XQ], xb[XQ];
 #pragma unroll
     for (int q = 0; q < XQ; ++q) {
+        const float *x = fl.r_obs + (size_t)xsrc[q] * IN;
         const int j = t & 15;
-        xa[q] = 0.0f; xb[q] = 0.0f;
-        if (xsrc[q] >= 0) {
-            if (j < IN) xa[q] = fl.r_obs[(size_t)xsrc[q] * IN + j];
-            if (j + 16 < IN) xb[q] = fl.r_obs[(size_t)xsrc[q] * IN + j + 16];
-        }
+        xa[q] = x[min(j, IN - 1)];
+        xb[q] = x[min(j + 16, IN - 1)];
     }
-    float l_a = 0.0f, l_b = 0.0f, l_act = 0.0f, l_mean = 0.0f, l_std = 1.0f;   // critic: return, old value; actor: advantage, log-prob
-    if (loss_row) {
-        if (!actor) {
-            l_a = fl.r_ret[lsrc];
-            if (fl.clip_value) l_b = fl.r_val[lsrc];
-        } else {
-            l_a = fl.r_adv[lsrc];
-            l_b = fl.r_logp[lsrc];
-            if (!fl.continuous) l_act = fl.r_act[lsrc];
-            else if (lj < A) l_act = fl.r_act[lsrc * A + lj];
-        }
-    }
-    if (actor && fl.adv_stats != nullptr) { l_mean = fl.adv_stats[0]; l_std = fl.adv_stats[1]; }
+    // critic: return, old value; actor: advantage, log-prob, action (component)
+    const float l_a = lp_a[lsrc], l_b = lp_b[lsrc], l_act = fl.r_act[(size_t)lsrc * act_w + min(lj, act_w - 1)];
     if (skip != 0) return;
-    if (blockIdx.x == 0 && actor)
-        for (int i = t; i < fl.n_posts; i += T) fl.posts[i] = 0;
-    // (the weights last: a wavefront's loads come back in order, and the rows are waited for first)
     __builtin_amdgcn_sched_barrier(0);
     bf16x8 wq[PF][NT][SPLIT];
     auto fetch = [&](const unsigned short *__restrict__ src, int ks, bf16x8 (&dst)[NT][SPLIT]) {
@@ -131,19 +123,26 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
             for (int p = 0; p < SPLIT; ++p)
                 dst[q][p] = *reinterpret_cast<const bf16x8 *>(src + split_frag<H>(ks, NT * w + q, p, lane));
     };
-#pragma unroll
-    for (int i = 0; i < PF; ++i) fetch(nn.wf, i, wq[i]);
-    __builtin_amdgcn_sched_barrier(0);
+    // under the wait for the rows: the head into LDS, and what of the loss needs no output
+    if (blockIdx.x == 0 && actor)
+        for (int i = t; i < fl.n_posts; i += T) fl.posts[i] = 0;
     for (int i = t; i < R * GLD; i += T) g2s[i] = 0.0f;
+    head.store(w2s, A, GAUSS, t);
+    const float std = actor && fl.continuous && t < 8 * R ? gaussian_std(ls, lj < A) : 1.0f;
 #pragma unroll
     for (int q = 0; q < XQ; ++q) {
         const int r = (t + q * T) >> 4, j = t & 15;
         if (r < R) {
-            if (j < IN) xs[r * XLD + j] = xa[q];
-            if (j + 16 < IN) xs[r * XLD + j + 16] = xb[q];
+            if (j < IN) xs[r * XLD + j] = r < nrow ? xa[q] : 0.0f;
+            if (j + 16 < IN) xs[r * XLD + j + 16] = r < nrow ? xb[q] : 0.0f;
             if (j == 0) xs[r * XLD + IN] = 1.0f;     // the bias gradient of layer 0 as row IN of x^T g0
         }
     }
+    // (the weights last: another wavefront's rows would wait behind them)
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < PF; ++i) fetch(nn.wf, i, wq[i]);
+    __builtin_amdgcn_sched_barrier(0);
     __syncthreads();
 
     // ---- layer 0, transposed: D[column 4 g + v][batch row n]
@@ -166,7 +165,7 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
                 for (int q = 0; q < NT; ++q)
 #pragma unroll
                     for (int rt = 0; rt < RT; ++rt)
-                        d[q][rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(w0[q][s], x[rt][s], d[q][rt], 0, 0, 0);
+                        d[q][rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(4 * s + g < IN ? w0[q][s] : 0.0f, x[rt][s], d[q][rt], 0, 0, 0);
             }
         }
 #pragma unroll
@@ -271,11 +270,10 @@ __global__ __launch_bounds__(fb_threads(H)) void mlp3_fb_kernel(int B, int IN, M
             float adv = l_a, kl;
             if (fl.adv_stats != nullptr) adv = (adv - l_mean) / (l_std + 1e-8f);
             if (fl.continuous) {
-                const float ls = w2s[HEAD_LOG_STD(H) + lj];
                 if (loss_row && lj < A)   // state-independent log_std, clamped (stochastic_actor.mojo:260-275)
                     nn.out[b * ld + A + lj] = ls < -5.0f ? -5.0f : (ls > 2.0f ? 2.0f : ls);
                 float gm, gs;
-                kl = actor_grad_gaussian_lanes(mine, ls, l_act, lj, lane & ~7, adv, l_b, fl.mb, A, fl.clip_eps,
+                kl = actor_grad_gaussian_lanes(mine, ls, std, l_act, lj, lane & ~7, adv, l_b, fl.mb, A, fl.clip_eps,
                                                fl.ent_coef, gm, gs);
                 if (loss_row && lj < A) {
                     g2row[lj] = gm;

@@ -173,15 +173,20 @@ MRL_DEV float actor_grad_gaussian_one(int b, const float *__restrict__ actor_out
                                    clip_eps, ent_coef, grad_out + (long)b * 2 * A);
 }
 
+// a lane's standard deviation for the function below, whenever its log_std is there (1 for j >= A)
+MRL_DEV float gaussian_std(float log_std_j, bool in) {
+    const float log_std = log_std_j < -5.0f ? -5.0f : (log_std_j > 2.0f ? 2.0f : log_std_j);
+    return in ? exp32(log_std) : 1.0f;
+}
+
 // actor_grad_gaussian_row by eight lanes of a wavefront (lanes base .. base + 7, A <= 8), lane j on action
-// component j (its mean, raw log_std and action; anything for j >= A): one exp(log_std) per lane, the
+// component j (its mean, raw log_std, standard deviation and action; anything for j >= A): one exp(log_std) per lane, the
 // log-probability summed over the lanes' terms in component order.  gm / gs = gradient slots j and A + j.
-MRL_DEV float actor_grad_gaussian_lanes(float mean_j, float log_std_j, float act_j, int j, int base, float advantage,
+MRL_DEV float actor_grad_gaussian_lanes(float mean_j, float log_std_j, float std, float act_j, int j, int base, float advantage,
                                         float old_log_prob, int mb, int A, float clip_eps, float ent_coef, float &gm,
                                         float &gs) {
     const float eps = 1e-6f, log_2pi = (float)1.8378770664093453;
     const float log_std = log_std_j < -5.0f ? -5.0f : (log_std_j > 2.0f ? 2.0f : log_std_j);
-    const float std = j < A ? exp32(log_std) : 1.0f;
     float lg;
     {
         float an = (act_j - mean_j) / (std + eps);
