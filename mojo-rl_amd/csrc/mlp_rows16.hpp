@@ -87,23 +87,29 @@ struct Rows16Forward {
         const int col_d = 16 * NT * w + RUN * g;       // its output columns, RUN of them, of batch row n
         const float *W0 = params, *b0 = params + IN * H, *W1 = b0 + H, *b1 = W1 + H * H;
 
-        // ---- everything from global memory is requested first, the rows ahead of the weights that hide behind them
+        // ---- Everything from global memory is requested first, the rows ahead of the weights that hide behind them.  A lane
+        // past the last row or input asks for the last one's value and drops it when it is used: behind a branch of its own,
+        // or with the head's copy into LDS in between, a request would wait for the ones before it.
         constexpr int XQ = (R * 16 + T - 1) / T;
         float xa[XQ], xb[XQ];
 #pragma unroll
         for (int q = 0; q < XQ; ++q) {
-            const int r = (t + q * T) >> 4, j = t & 15;
-            xa[q] = r < nrow && j < IN ? x[r * IN + j] : 0.0f;
-            xb[q] = r < nrow && j + 16 < IN ? x[r * IN + j + 16] : 0.0f;
+            const float *xr = x + min((t + q * T) >> 4, nrow - 1) * IN;
+            const int j = t & 15;
+            xa[q] = xr[min(j, IN - 1)];
+            xb[q] = xr[min(j + 16, IN - 1)];
         }
         float w0[K0][NT], bias0[RUN], bias1[RUN];
 #pragma unroll
         for (int s = 0; s < K0; ++s)
+            if (s == 0 || 4 * s < IN) {
 #pragma unroll
-            for (int q = 0; q < NT; ++q) w0[s][q] = 4 * s + g < IN ? W0[(4 * s + g) * H + col_w + q] : 0.0f;
+                for (int q = 0; q < NT; ++q) w0[s][q] = W0[min(4 * s + g, IN - 1) * H + col_w + q];
+            }
 #pragma unroll
         for (int j = 0; j < RUN; ++j) { bias0[j] = b0[col_d + j]; bias1[j] = b1[col_d + j]; }
-        stage_head(params + IN * H + H + H * H + H, H, A, GAUSS, l.w2s, t, T);
+        HeadLoads<H, T> head;
+        head.load(params + IN * H + H + H * H + H, A, GAUSS, t);
         __builtin_amdgcn_sched_barrier(0);
         float w1[KS][NT];
 #pragma unroll
@@ -115,14 +121,15 @@ struct Rows16Forward {
         for (int q = 0; q < XQ; ++q) {
             const int r = (t + q * T) >> 4, j = t & 15;
             if (r < R) {
-                if (j < IN) l.xs[r * XS_LD + j] = xa[q];
-                if (j + 16 < IN) l.xs[r * XS_LD + j + 16] = xb[q];
+                if (j < IN) l.xs[r * XS_LD + j] = r < nrow ? xa[q] : 0.0f;
+                if (j + 16 < IN) l.xs[r * XS_LD + j + 16] = r < nrow ? xb[q] : 0.0f;
                 if (r < nrow) {
                     if (j < IN) on_x(r, j, xa[q]);
                     if (j + 16 < IN) on_x(r, j + 16, xb[q]);
                 }
             }
         }
+        head.store(l.w2s, A, GAUSS, t);
         __syncthreads();
 
         // ---- layer 0: D[column 4 g + v of tile q][batch row n]
@@ -135,7 +142,7 @@ struct Rows16Forward {
                 if (4 * s < IN) {
                     const float xk = 4 * s + g < IN ? l.xs[n * XS_LD + 4 * s + g] : 0.0f;
 #pragma unroll
-                    for (int q = 0; q < NT; ++q) d[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(w0[s][q], xk, d[q], 0, 0, 0);
+                    for (int q = 0; q < NT; ++q) d[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(4 * s + g < IN ? w0[s][q] : 0.0f, xk, d[q], 0, 0, 0);
                 }
             }
             float pre[RUN], y[RUN];

@@ -97,38 +97,38 @@ __global__ __launch_bounds__(rows_threads(H)) void mlp3_bwd_kernel(int B, int IN
     float *__restrict__ db_part = nn.db_part + (size_t)blockIdx.x * (2 * H + PA_MAX);
     float *__restrict__ thin_part = nn.thin_part + (size_t)blockIdx.x * (size_t)nn.thin_stride;
 
-    // ---- everything from global memory is requested first, the rows ahead of the weights that hide behind them
+    // ---- everything from global memory is requested first, the rows ahead of the weights that hide behind them (as in
+    // Rows16Forward: a lane past the end asks for the last value and drops it when it is used)
     f32x4 v1[HQ], v2[HQ];
     const bool vec = (reinterpret_cast<uintptr_t>(c1) & 15) == 0;    // (c2 lies a multiple of 2 H floats behind it)
 #pragma unroll
     for (int q = 0; q < HQ; ++q) {
-        const int e = 4 * (t + q * T), r = e / H, c = e % H;
-        v1[q] = v2[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        if (r < nrow) {
-            const float *s1 = c1 + (row0 + r) * (2 * H) + c, *s2 = c2 + (row0 + r) * H + c;
-            if (vec) {
-                v1[q] = *reinterpret_cast<const f32x4 *>(s1);
-                v2[q] = *reinterpret_cast<const f32x4 *>(s2);
-            } else {
-                v1[q] = f32x4{s1[0], s1[1], s1[2], s1[3]};
-                v2[q] = f32x4{s2[0], s2[1], s2[2], s2[3]};
-            }
+        const int e = 4 * (t + q * T), r = min(e / H, nrow - 1), c = e % H;
+        const float *s1 = c1 + (row0 + r) * (2 * H) + c, *s2 = c2 + (row0 + r) * H + c;
+        if (vec) {
+            v1[q] = *reinterpret_cast<const f32x4 *>(s1);
+            v2[q] = *reinterpret_cast<const f32x4 *>(s2);
+        } else {
+            v1[q] = f32x4{s1[0], s1[1], s1[2], s1[3]};
+            v2[q] = f32x4{s2[0], s2[1], s2[2], s2[3]};
         }
     }
     constexpr int XQ = (R * 16 + T - 1) / T, GQ = (R * GLD + T - 1) / T;
     float xa[XQ], xb[XQ], gq[GQ];
 #pragma unroll
     for (int q = 0; q < XQ; ++q) {
-        const int r = (t + q * T) >> 4, j = t & 15;
-        xa[q] = r < nrow && j < IN ? c0[(row0 + r) * (IN + H) + j] : 0.0f;
-        xb[q] = r < nrow && j + 16 < IN ? c0[(row0 + r) * (IN + H) + j + 16] : 0.0f;
+        const float *x = c0 + (row0 + min((t + q * T) >> 4, nrow - 1)) * (IN + H);
+        const int j = t & 15;
+        xa[q] = x[min(j, IN - 1)];
+        xb[q] = x[min(j + 16, IN - 1)];
     }
 #pragma unroll
     for (int q = 0; q < GQ; ++q) {
         const int i = t + q * T, r = i / GLD, a = i - r * GLD;
-        gq[q] = r < nrow && a < ld ? grad_out[(row0 + r) * ld + a] : 0.0f;
+        gq[q] = grad_out[(row0 + min(r, nrow - 1)) * ld + min(a, ld - 1)];
     }
-    stage_head(W1 + H * H + H, H, A, false, w2s, t, T);
+    HeadLoads<H, T> head;
+    head.load(W1 + H * H + H, A, false, t);
     __builtin_amdgcn_sched_barrier(0);
     // W1^T as operand: k-slot g of step v in group s is column 16 s + 4 g + v of W1, for both operands
     f32x4 w1[NT][NS];
@@ -142,31 +142,34 @@ __global__ __launch_bounds__(rows_threads(H)) void mlp3_bwd_kernel(int B, int IN
     for (int it = 0; it < 2; ++it)
 #pragma unroll
         for (int q = 0; q < NT; ++q) {
-            w0[it][q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            if (nn.grad_in != nullptr && 16 * it + n < IN)
-                w0[it][q] = *reinterpret_cast<const f32x4 *>(W0 + (16 * it + n) * H + 16 * (NT * w + q) + 4 * g);
+            if (nn.grad_in != nullptr)
+                w0[it][q] = *reinterpret_cast<const f32x4 *>(W0 + min(16 * it + n, IN - 1) * H + 16 * (NT * w + q) + 4 * g);
         }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int q = 0; q < HQ; ++q) {
         const int e = 4 * (t + q * T), r = e / H, c = e % H;
         if (r < R) {
-            *reinterpret_cast<f32x4 *>(h1f + r * FLD + c) = v1[q];
-            *reinterpret_cast<f32x4 *>(h2f + r * FLD + c) = v2[q];
+            const f32x4 none = {0.0f, 0.0f, 0.0f, 0.0f};
+            *reinterpret_cast<f32x4 *>(h1f + r * FLD + c) = r < nrow ? v1[q] : none;
+            *reinterpret_cast<f32x4 *>(h2f + r * FLD + c) = r < nrow ? v2[q] : none;
         }
     }
 #pragma unroll
     for (int q = 0; q < XQ; ++q) {
         const int r = (t + q * T) >> 4, j = t & 15;
         if (r < R) {
-            if (j < IN) xs[r * XLD + j] = xa[q];
-            if (j + 16 < IN) xs[r * XLD + j + 16] = xb[q];
+            if (j < IN) xs[r * XLD + j] = r < nrow ? xa[q] : 0.0f;
+            if (j + 16 < IN) xs[r * XLD + j + 16] = r < nrow ? xb[q] : 0.0f;
             if (j == 0) xs[r * XLD + IN] = 1.0f;     // the bias gradient of layer 0 as row IN of x^T g0
         }
     }
 #pragma unroll
-    for (int q = 0; q < GQ; ++q)
-        if (t + q * T < R * GLD) g2s[t + q * T] = gq[q];
+    for (int q = 0; q < GQ; ++q) {
+        const int i = t + q * T, r = i / GLD, a = i - r * GLD;
+        if (i < R * GLD) g2s[i] = r < nrow && a < ld ? gq[q] : 0.0f;
+    }
+    head.store(w2s, A, false, t);
     __syncthreads();
 
     // ---- back through the head and layer 1's activation: g1^T[column 4 g + v][batch row n]
