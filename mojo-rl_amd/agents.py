@@ -53,7 +53,6 @@ class _PPOAgentBase:
         N, T = self.n_envs, self.rollout_len
         env.reset_kernel_gpu(ctx, rb.states, seed)
         rb.obs.copy_(rb.states.view(N, env.STATE_SIZE)[:, :env.OBS_DIM].reshape(-1))
-        rb.ep_return.zero_(); rb.ep_length.zero_()
         noise_std = float(getattr(self, "obs_noise_std", 0.0)) if self.continuous else 0.0
         if noise_std > 0.0:
             ppo.add_obs_noise(ctx, rb.obs, N, noise_std, 42)      # ppo_continuous.mojo:2557-2564
