@@ -406,6 +406,11 @@ int mrl_ppo_update_minibatch(mrl_ctx *ctx, const mrl_update *u, const int32_t *i
  * runs with step counts actor_t0 + k + 1 / critic_t0 + k + 1 */
 int mrl_ppo_update_epoch(mrl_ctx *ctx, const mrl_update *u, const int32_t *indices, int n_minibatches,
                          int actor_t0, int critic_t0);
+/* The same for a caller that waits for the epoch's end right behind it (to read kl_flag): with a KL test the call itself waits
+ * so that it is never more than `ahead` (>= 1) minibatches ahead of the device, and so few launches are left to run once the
+ * stop is up.  Where the device does not come on for 50 ms the call goes on without waiting, and a capture never waits. */
+int mrl_ppo_update_epoch_ahead(mrl_ctx *ctx, const mrl_update *u, const int32_t *indices, int n_minibatches,
+                               int actor_t0, int critic_t0, int ahead);
 
 /* The statistics that the fused update normalises a minibatch's advantages with
  * (deep_agents/ppo/ppo.mojo:2478-2511 with the kernel at :637-653 -- mean and variance over the

@@ -119,6 +119,7 @@ SIGNATURES = {
     "mrl_rollout_fused": [RP],
     "mrl_ppo_update_minibatch": [P, UP, P, I, I],
     "mrl_ppo_update_epoch": [P, UP, P, I, I, I],
+    "mrl_ppo_update_epoch_ahead": [P, UP, P, I, I, I, I],
     "mrl_minibatch_adv_stats": [P, P, P, I, I, P],
 }
 _SPECIAL = {"mrl_version": (C.c_int, []), "mrl_last_error": (C.c_char_p, [])}

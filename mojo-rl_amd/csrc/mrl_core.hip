@@ -86,6 +86,9 @@ int mrl_ctx_create(void *hip_stream, mrl_ctx **out) {
     c->stop_seen = c->sync_error + 8;
     *c->stop_seen = 0;
     c->stop_call = 0;
+    c->upd_reached = reinterpret_cast<unsigned *>(c->sync_error + 12);
+    *c->upd_reached = 0;
+    c->upd_count = 0;
     c->upd_enqueued = 0;
     {
         int rc = mrl::clip_static_setup(c->device);

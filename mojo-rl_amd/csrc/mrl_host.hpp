@@ -46,6 +46,9 @@ struct mrl_ctx {
     // sync_error): the host leaves launches away that would find the stop raised and do nothing.
     int stop_call;
     int *stop_seen;
+    // Minibatches of updates with a KL test enqueued so far, and how many of them the device has come to (pinned, written by
+    // the kernel that applies them).
+    unsigned upd_count, *upd_reached;
     int upd_enqueued;   // minibatches that the last update call enqueued
     // CarRacingV2: 0 = the CPU env's reward / termination arithmetic (default), 1 = the GPU trait's
     int car_trait_form;

@@ -24,6 +24,7 @@
 #include "mlp3.hpp"
 #include "tile_sums.hpp"
 #include "ppo_grads.hpp"
+#include <chrono>
 
 namespace mrl {
 
@@ -255,6 +256,8 @@ struct AdamArgs {
     // not null: where the host looks for the stop while it enqueues a call's minibatches; gets the call's number
     int *stop_seen;
     int stop_call;
+    // not null: gets the number of this minibatch, for the host to see how far the device is
+    unsigned *reached, count;
 };
 
 // Whether the update is applied (it is not once stop[0] != 0), and the factor of the global-norm clip (ppo.mojo:382-534;
@@ -283,6 +286,8 @@ MRL_DEV bool clip_verdict(const AdamArgs &a, float *smem, float &scale) {
             const float mean = sum / (float)a.kl_mb;
             const bool over = a.kl_part != nullptr && mean > a.target_kl;
             stop_s = raised != 0 || over;
+            if (a.reached != nullptr && blockIdx.x == 0 && blockIdx.y == 0)
+                __hip_atomic_store(a.reached, a.count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             if (stop_s && a.stop_seen != nullptr && blockIdx.x == 0 && blockIdx.y == 0)
                 __hip_atomic_store(a.stop_seen, a.stop_call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             if (a.kl_part != nullptr && raised == 0 && blockIdx.x == 0 && blockIdx.y == 0) {
@@ -445,8 +450,8 @@ struct SumAdam {
     const float *kl_part;     // the row tiles' sums, never null
     int kl_n, kl_mb;
     float target_kl;
-    int *stop_seen;           // as AdamArgs::stop_seen, null: nobody looks
-    int stop_call;
+    int *stop_seen, stop_call;        // as in AdamArgs
+    unsigned *reached, count;
 };
 
 template <int H, bool TREE>
@@ -535,6 +540,8 @@ __global__ __launch_bounds__(UTPB, 4) void sum_adam_kernel(SumAdam k) {
             total_s = total;
             state_s = state;
             if (state == 2) __hip_atomic_store(k.sync_error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            if (k.reached != nullptr && blockIdx.x == 0 && ynet == 0)
+                __hip_atomic_store(k.reached, k.count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             if (stop && k.stop_seen != nullptr && blockIdx.x == 0 && ynet == 0)
                 __hip_atomic_store(k.stop_seen, k.stop_call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             if (test && first && blockIdx.x == 0 && ynet == 0) {
@@ -692,8 +699,9 @@ static void adam_args(const mrl_update *u, int actor_t, int critic_t, AdamArgs &
 // ws.split holds the hidden layers' current weights; more: another minibatch of the same call follows.  Then the copies
 // are kept in step with the updated weights, and once the KL stop is up nothing is computed: no parameter moves any more,
 // and what else the call leaves (gradients, outputs, KL estimates) is its last minibatch's, which is always computed.
+// watched: the host looks how far the device is.
 static int update_minibatch_paired(mrl_ctx *ctx, const mrl_update *u, const int32_t *indices, int actor_t, int critic_t,
-                                   const float *stats, const UpdateWs &ws, bool more) {
+                                   const float *stats, const UpdateWs &ws, bool more, bool watched) {
     const bool cont = u->continuous != 0;
     const int mb = u->minibatch, head = mrl_mlp_out_dim(&u->actor);
     const mrl_mlp_desc *descs[2] = {&u->actor, &u->critic};
@@ -718,6 +726,10 @@ static int update_minibatch_paired(mrl_ctx *ctx, const mrl_update *u, const int3
     a.kl_n = ws.tiles;
     a.stop_seen = more && a.stop != nullptr ? ctx->stop_seen : nullptr;
     a.stop_call = ctx->stop_call;
+    if (watched) {
+        a.reached = ctx->upd_reached;
+        a.count = ++ctx->upd_count;
+    }
     const int H = u->actor.layers[0].out_dim, o1 = (u->obs_dim + 1) * H;
     const int blocks = sum_adam_blocks(H, a);
     const bool one_launch = 2 * blocks <= std::min(ctx->stream_cus, POSTS_MAX);
@@ -747,6 +759,8 @@ static int update_minibatch_paired(mrl_ctx *ctx, const mrl_update *u, const int3
         k.target_kl = a.target_kl;
         k.stop_seen = a.stop_seen;
         k.stop_call = a.stop_call;
+        k.reached = a.reached;
+        k.count = a.count;
         if (H == 256) launch_sum_adam<256>(ctx->stream, k, blocks, ws.rows == 16);
         else if (H == 128) launch_sum_adam<128>(ctx->stream, k, blocks, ws.rows == 16);
         else launch_sum_adam<64>(ctx->stream, k, blocks, ws.rows == 16);
@@ -818,8 +832,11 @@ static int update_minibatch_layers(mrl_ctx *ctx, const mrl_update *u, const int3
     return MRL_OK;
 }
 
-// Minibatches 0 .. n - 1 of `indices`, with step counts t0 + 1 ..
-static int update_minibatches(mrl_ctx *ctx, const mrl_update *u, const int32_t *indices, int n, int actor_t0, int critic_t0) {
+constexpr auto AHEAD_PATIENCE = std::chrono::milliseconds(50);
+
+// Minibatches 0 .. n - 1 of `indices`, with step counts t0 + 1 ..; ahead > 0: the caller waits for the end anyway, and with a
+// KL test the host stays within that many minibatches of the device
+static int update_minibatches(mrl_ctx *ctx, const mrl_update *u, const int32_t *indices, int n, int actor_t0, int critic_t0, int ahead) {
     int rc;
     ctx->upd_enqueued = 0;
     if (!update_paired(u)) {
@@ -840,15 +857,31 @@ static int update_minibatches(mrl_ctx *ctx, const mrl_update *u, const int32_t *
     rc = launch_split_weights(ctx, u->actor.layers[0].out_dim, ws.split, 2);
     if (rc) return rc;
     // Behind the KL stop every launch ends at once, but a launch is 2.5 us of the device and up to 4 of the host.  So the host
-    // looks, without waiting, whether the device has reported the stop for this call's number, and then goes on with
-    // the last minibatch (which is always computed).  A capture records all of them: nothing runs meanwhile, and a number is
+    // looks whether the device has reported the stop for this call's number, and then goes on with
+    // the last minibatch (which is always computed); and it may stay within `ahead` minibatches of the device, because what it has
+    // enqueued beyond the stop runs.  Where the device does not come on for AHEAD_PATIENCE, for whatever reason, the host
+    // stops waiting for the rest of the call.  A capture records all of them: nothing runs meanwhile, and a number is
     // never used again.  CartPole, 1024 envs x 128 steps, H = 64, 512 minibatches of 256 rows an epoch of which
-    // the stop leaves a few dozen: train_gpu 4.9 -> 1.46 ms.
+    // the stop leaves a few dozen, us per train_gpu: 4900 when all were launched, 1105 without the limit, 878 with it.
     ctx->stop_call += 1;
     const volatile int *seen = ctx->stop_seen;
+    const volatile unsigned *reached = ctx->upd_reached;
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    bool watched = u->target_kl > 0.0f && ahead > 0 && n > ahead;
+    if (watched && hipStreamIsCapturing(ctx->stream, &capturing) != hipSuccess) {
+        (void)hipGetLastError();
+        watched = false;
+    }
+    watched = watched && capturing == hipStreamCaptureStatusNone;
+    bool patient = watched;
     float *stats = ctx->upd_scratch + SCR_STATS;
     int have_stats = -1;   // the first of the STATS_MAX minibatches whose advantage statistics are there
     for (int k = 0; k < n; ++k) {
+        if (patient && k >= ahead) {
+            const auto since = std::chrono::steady_clock::now();
+            while (ctx->upd_count - *reached >= (unsigned)ahead && *seen != ctx->stop_call && patient)
+                patient = std::chrono::steady_clock::now() - since < AHEAD_PATIENCE;
+        }
         if (u->target_kl > 0.0f && *seen == ctx->stop_call) k = n - 1;
         const int s0 = k / STATS_MAX * STATS_MAX;
         if (u->norm_adv_per_minibatch && s0 != have_stats) {   // of many minibatches in one launch
@@ -858,7 +891,7 @@ static int update_minibatches(mrl_ctx *ctx, const mrl_update *u, const int32_t *
             have_stats = s0;
         }
         rc = update_minibatch_paired(ctx, u, indices + (size_t)k * u->minibatch, actor_t0 + k + 1, critic_t0 + k + 1,
-                                     stats + 2 * (k - s0), ws, k + 1 < n);
+                                     stats + 2 * (k - s0), ws, k + 1 < n, watched);
         if (rc) return rc;
         ctx->upd_enqueued += 1;
     }
@@ -872,7 +905,7 @@ int mrl_ppo_update_minibatch(mrl_ctx *ctx, const mrl_update *u, const int32_t *i
     if (rc) return rc;
     MRL_CHECK_ARG(indices != nullptr && actor_t >= 1 && critic_t >= 1,
                   "mrl_ppo_update_minibatch: need indices and step counts >= 1");
-    return update_minibatches(ctx, u, indices, 1, actor_t - 1, critic_t - 1);
+    return update_minibatches(ctx, u, indices, 1, actor_t - 1, critic_t - 1, 0);
 }
 
 int mrl_minibatch_adv_stats(mrl_ctx *ctx, const int32_t *indices, const float *advantages, int minibatch,
@@ -888,15 +921,26 @@ int mrl_minibatch_adv_stats(mrl_ctx *ctx, const int32_t *indices, const float *a
     return MRL_OK;
 }
 
+static int update_epoch(mrl_ctx *ctx, const mrl_update *u, const int32_t *indices, int n_minibatches, int actor_t0, int critic_t0,
+                        int ahead, const char *who) {
+    MRL_CHECK_ARG(ctx != nullptr, "%s: ctx is NULL", who);
+    ctx->upd_enqueued = 0;
+    int rc = update_check(u, who);
+    if (rc) return rc;
+    MRL_CHECK_ARG(n_minibatches >= 0 && actor_t0 >= 0 && critic_t0 >= 0, "%s: negative count", who);
+    MRL_CHECK_ARG(n_minibatches == 0 || indices != nullptr, "%s: indices is NULL", who);
+    return n_minibatches == 0 ? MRL_OK : update_minibatches(ctx, u, indices, n_minibatches, actor_t0, critic_t0, ahead);
+}
+
 int mrl_ppo_update_epoch(mrl_ctx *ctx, const mrl_update *u, const int32_t *indices, int n_minibatches,
                          int actor_t0, int critic_t0) {
-    MRL_CHECK_ARG(ctx != nullptr, "mrl_ppo_update_epoch: ctx is NULL");
-    ctx->upd_enqueued = 0;
-    int rc = update_check(u, "mrl_ppo_update_epoch");
-    if (rc) return rc;
-    MRL_CHECK_ARG(n_minibatches >= 0 && actor_t0 >= 0 && critic_t0 >= 0, "mrl_ppo_update_epoch: negative count");
-    MRL_CHECK_ARG(n_minibatches == 0 || indices != nullptr, "mrl_ppo_update_epoch: indices is NULL");
-    return n_minibatches == 0 ? MRL_OK : update_minibatches(ctx, u, indices, n_minibatches, actor_t0, critic_t0);
+    return update_epoch(ctx, u, indices, n_minibatches, actor_t0, critic_t0, 0, "mrl_ppo_update_epoch");
+}
+
+int mrl_ppo_update_epoch_ahead(mrl_ctx *ctx, const mrl_update *u, const int32_t *indices, int n_minibatches,
+                               int actor_t0, int critic_t0, int ahead) {
+    MRL_CHECK_ARG(ahead >= 1, "mrl_ppo_update_epoch_ahead: ahead must be positive");
+    return update_epoch(ctx, u, indices, n_minibatches, actor_t0, critic_t0, ahead, "mrl_ppo_update_epoch_ahead");
 }
 
 }  // extern "C"

@@ -116,3 +116,26 @@ def test_captured_update_records_every_minibatch(mrl):
     del graph
     gctx.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("busy", [False, True])
+def test_the_host_stays_a_few_minibatches_ahead(mrl, busy):
+    """What is enqueued behind the stop is a few minibatches; and where the device does not come to the update for longer than
+    the host waits, all of them are, with the same results."""
+    print("ahead", busy, flush=True)
+    n_mb, ctx = 400, mrl.DeviceContext("cuda:0")
+    build, same, perm = case(mrl, n_mb, ctx)
+    (rb1, one), (rb2, whole) = build(0.05), build(0.05)
+    for k in range(n_mb):
+        one.minibatch_step(perm[k * MB:(k + 1) * MB])
+    ctx.synchronize()
+    if busy:
+        filler = torch.zeros(1 << 28, device="cuda")
+        for _ in range(400):        # 2 GiB of traffic each, a third of a millisecond and more
+            filler.add_(1.0)
+    assert whole.run_epoch(perm)[0]
+    applied = int(whole.kl_flag[2])
+    assert 0 < applied < n_mb // 2
+    # the minibatch that raised the stop, the six that the host may be ahead, the one that it was about to enqueue, the last
+    assert ctx.update_enqueued() <= (n_mb if busy else applied + 9)
+    same(one, whole, rb1, rb2)
