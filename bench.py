@@ -329,8 +329,8 @@ def main():
         tflops = FWD_FLOPS * N_ENVS * steps_per_launch / (launch_us * 1e-6) / 1e12
         act_id = 1 if ACT == "relu" else 2
         name = {"lunarlander": "mrl::collect16_kernel<mrl::LunarLander, %d, %d, false>" % (HIDDEN, act_id),
-                "cartpole": "mrl::collect_classic16_kernel<mrl::CartPoleSlot, 64, %d, false>" % act_id,
-                "pendulum": "mrl::collect_classic_kernel<mrl::PendulumSlot, %d, true>" % act_id,
+                "cartpole": "mrl::collect_cartpole16_h64_kernel<%d>" % act_id,
+                "pendulum": "mrl::collect_pendulum16_h64_kernel<%d>" % act_id,
                 "bipedal": "mrl::collect_walker_kernel<mrl::BipedalWalker, 256, %d, false>" % act_id,
                 "halfcheetah": "mrl::collect_walker_kernel<mrl::HalfCheetah16, 256, %d, true>" % act_id,
                 "carracing": "mrl::collect_car_kernel<256, %d>" % act_id,

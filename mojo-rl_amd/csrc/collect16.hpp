@@ -234,32 +234,15 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
     S::out(rows, gbase, nenv, t, 0, E::STATE);
 }
 
-struct CartPoleSlot {
-    static constexpr int OBS = cartpole::OBS, ACT_W = 1, HEAD = 2;   // HEAD: outputs of the actor's head
-    float s[4];
-    int32_t steps;
-    MRL_DEV void load(const float *states, const int32_t *side, int i) {
-        const float4 v = reinterpret_cast<const float4 *>(states)[i];
-        s[0] = v.x; s[1] = v.y; s[2] = v.z; s[3] = v.w;
-        steps = side[i];
-    }
-    MRL_DEV void store(float *states, int32_t *side, int i) const {
-        reinterpret_cast<float4 *>(states)[i] = make_float4(s[0], s[1], s[2], s[3]);
-        side[i] = steps;
-    }
-    MRL_DEV float obs(int k) const { return s[k]; }
-    MRL_DEV void step(const float *act, float &r, float &d) { cartpole::step(s, steps, (int)act[0], r, d); }
-    MRL_DEV void reset(int i, uint64_t seed) { cartpole::reset(s, steps, i, (uint32_t)seed); }
-};
 struct PendulumSlot {
-    static constexpr int OBS = pendulum::OBS, ACT_W = 1, HEAD = 1;
+    static constexpr int OBS = pendulum::OBS;
     float s[8];
-    MRL_DEV void load(const float *states, const int32_t *, int i) {
+    MRL_DEV void load(const float *states, int i) {
         const float4 *row = reinterpret_cast<const float4 *>(states) + 2 * (size_t)i;
         const float4 a = row[0], b = row[1];
         s[0] = a.x; s[1] = a.y; s[2] = a.z; s[3] = a.w; s[4] = b.x; s[5] = b.y; s[6] = b.z; s[7] = b.w;
     }
-    MRL_DEV void store(float *states, int32_t *, int i) const {
+    MRL_DEV void store(float *states, int i) const {
         float4 *row = reinterpret_cast<float4 *>(states) + 2 * (size_t)i;
         row[0] = make_float4(s[0], s[1], s[2], s[3]);
         row[1] = make_float4(s[4], s[5], s[6], s[7]);
@@ -273,18 +256,391 @@ struct PendulumSlot {
 // A step of these envs is one dependent chain (observation -> two layers on the matrix cores -> head -> sample -> env
 // step) of a few thousand cycles, whatever the number of envs.  Sixteen rows per workgroup of eight wavefronts (four
 // per net, H / 4 columns each, 16x16x4 tiles: the bits of the 32-row tiles) make its matrix part a quarter of that of
-// a 32-row workgroup with two wavefronts per net, the number of head outputs is a compile-time constant, and the
-// log-probability, which nothing of the step waits for, is taken by another wavefront beside the env step.  Lanes
-// 0 .. 15 of wavefront 0 carry one env each in registers.  Up to hidden width 128 the hidden layers' weights stay in
-// registers for the whole launch (the bound of four wavefronts per SIMD lets two workgroups share a CU).
-// CartPole, hidden width 64, us per step at 1024 / 4096 envs: 32 rows 4.88 / 4.66, this form 3.04 / 3.11 (2.50 at 1024 envs
-// with the head's sums in DPP instructions); hidden width
-// 128 and 256 as a policy and an env-step launch per step 16.9 and 19.4, in this form 5.95 and 13.4.  (The critic a
-// phase behind the actor, its second layer beside the env step: 3.30 at width 64, 7.2 at 128 -- on one SIMD matrix and
-// vector instructions of different wavefronts take turns --, 12.5 at 256.)
-template <class C, int H, int ACT, bool GAUSS>
-__global__ __launch_bounds__(512, 4) void collect_classic16_kernel(CollectArgs a, int32_t *side) {
-    constexpr int IN = C::OBS, AW = C::ACT_W, A = C::HEAD, R = PR16, T = 512, NT = H / 64;
+// a 32-row workgroup with two wavefronts per net, and the number of head outputs is a compile-time constant.  Up to
+// hidden width 128 the hidden layers' weights stay in registers for the whole launch (the bound of four wavefronts per
+// SIMD lets two workgroups share a CU).  What a step does not need in turn is not in the chain:
+//   * CartPole has two actions: while wavefront 0 takes the actor's head and draws, wavefront 5 takes the env step with
+//     both, and the draw picks one of two rows;
+//   * the states of envs that start again (wavefront 6), the uniform numbers of the draw (2) and Pendulum's normal
+//     numbers (2) depend on seeds alone: each is there a step ahead;
+//   * log-probability, rollout row and episode sums are taken a step later (CartPole), or beside the env step (Pendulum).
+// (The critic a phase behind the actor where it has the actor's SIMDs: slower at widths 64 and 128 -- on one SIMD matrix and
+// vector instructions of different wavefronts take turns; width 64 gives it two SIMDs that the draw does not use.)
+// A step's chain waits for its longest wavefront at three barriers; thousand cycles of CartPole's at width 64 and 1024 envs,
+// with all of it in turn 5.9 in four barriers, now 3.1: layer 0 0.6, layer 1 1.2, head and draw (beside the critic's
+// second layer) 1.3.  us per step before : now, CartPole at 1024 / 4096 / 8192 / 16384 / 32768 envs 2.55 : 1.36, 2.65 : 1.42,
+// 4.25 : 2.12, 5.91 : 4.10, 14.3 : 8.0; width 128, 1024 envs 5.66 : 4.59; width 256 10.5 : 10.4.  Pendulum at 1024 / 8192 /
+// 16384 / 32768 envs 2.77 : 1.86, 3.92 : 3.08, 6.22 : 5.87, 12.0 : 11.4; width 128, 1024 envs 6.36 : 6.07; width 256 11.8 :
+// 11.3.  (From 8192 CartPole and 16384 Pendulum envs on, before, in 32-row workgroups with one env a lane in turn.)
+// Action, reward and done flag of a step into the rollout, and the episode sums, a lane per env of one wavefront.  Finished episodes wait
+// in LDS until some dozens are there: their places in the list come from one counter of the whole chip, at which a request
+// per step and workgroup were what a step of 4096 envs waited for.  (All lanes of the wavefront make the calls.)
+struct EpisodeBooks {
+    static constexpr int R = PR16;
+    struct Waiting { float ret[WAVE], len[WAVE]; };
+    float ep_return = 0.0f, ep_length = 0.0f;
+    int waiting = 0;
+    MRL_DEV void begin(const CollectArgs &a, int env, bool mine) {
+        if (mine) {
+            ep_return = a.acc.ep_return[env];
+            ep_length = a.acc.ep_length[env];
+        }
+    }
+    MRL_DEV void list(const CollectArgs &a, const Waiting &w, int lane) {
+        int first = 0;
+        if (lane == 0) first = atomicAdd(a.acc.done_count, waiting);
+        first = __builtin_amdgcn_readfirstlane(first);
+        if (lane < waiting && first + lane < a.acc.done_cap) {
+            a.acc.done_returns[first + lane] = w.ret[lane];
+            a.acc.done_lengths[first + lane] = w.len[lane];
+        }
+        waiting = 0;
+    }
+    MRL_DEV void rewards(const CollectArgs &a, Waiting &w, size_t at, float action, float r, float d, int lane, bool mine) {
+        if (mine) {
+            a.r_actions[at] = action;
+            a.r_rewards[at] = r;
+            a.r_dones[at] = d;
+        }
+        ep_return = ep_return + r;
+        ep_length = ep_length + 1.0f;
+        const bool finished = mine && d > 0.5f;
+        const unsigned long long all = __ballot(finished);
+        if (all == 0) return;
+        if (finished) {
+            const int i = waiting + __popcll(all & ((1ull << lane) - 1));
+            w.ret[i] = ep_return;
+            w.len[i] = ep_length;
+        }
+        ep_return = finished ? 0.0f : ep_return;
+        ep_length = finished ? 0.0f : ep_length;
+        waiting += __popcll(all);
+        if (waiting > WAVE - R) list(a, w, lane);
+    }
+    MRL_DEV void end(const CollectArgs &a, const Waiting &w, int env, int lane, bool mine) {
+        if (waiting > 0) list(a, w, lane);
+        if (mine) {
+            a.acc.ep_return[env] = ep_return;
+            a.acc.ep_length[env] = ep_length;
+        }
+    }
+};
+
+// What a CartPole workgroup has in LDS beside its nets.  The envs' rows behind the last step, one per action and env: a new
+// episode's where that action ended one.  Of step k, at [k & 1]: the action drawn, its probability, both actions' rewards and
+// done flags; and, there a step ahead, new episodes' rows and the numbers of the draw.
+struct CartPoleRows {
+    static constexpr int R = PR16, A = 2, SLD = 5;
+    float rows[A][R][SLD];
+    int32_t steps[A][R];
+    float rew[2][A][R], don[2][A][R], prob[2][R];
+    int32_t drawn[2][R];
+    float fresh[2][R][SLD], uniform[2][R];
+
+    // as if a step with action 0 had led here; lanes 0 .. R - 1
+    MRL_DEV void load(const CollectArgs &a, const int32_t *side, int env0, int nenv, int e) {
+        float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        int32_t n = 0;
+        if (e < nenv) {
+            v = reinterpret_cast<const float4 *>(a.states)[env0 + e];
+            n = side[env0 + e];
+        }
+#pragma unroll
+        for (int j = 0; j < A; ++j) {
+            rows[j][e][0] = v.x; rows[j][e][1] = v.y; rows[j][e][2] = v.z; rows[j][e][3] = v.w;
+            steps[j][e] = n;
+        }
+        drawn[1][e] = 0;
+    }
+    MRL_DEV void store(const CollectArgs &a, int32_t *side, int env0, int e) const {
+        const int sel = drawn[(a.n_steps + 1) & 1][e];
+        const float *s = rows[sel][e];
+        reinterpret_cast<float4 *>(a.states)[env0 + e] = make_float4(s[0], s[1], s[2], s[3]);
+        side[env0 + e] = steps[sel][e];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) a.obs[(size_t)(env0 + e) * 4 + c] = s[c];
+    }
+    // the operand of layer 0: input `lane >> 4` of row `lane & 15`
+    MRL_DEV float input(int before, int lane) const {
+        const int n = lane & 15, g = lane >> 4, sel = drawn[before][n];
+        const float x0 = rows[0][n][g], x1 = rows[1][n][g];
+        return sel != 0 ? x1 : x0;
+    }
+    MRL_DEV void make_fresh(const CollectArgs &a, int k, int env0, int e) {
+        float s[4];
+        int32_t none;
+        cartpole::reset(s, none, env0 + e, (uint32_t)(a.reset_seed + (uint64_t)k * a.reset_stride));
+#pragma unroll
+        for (int c = 0; c < 4; ++c) fresh[k & 1][e][c] = s[c];
+    }
+    MRL_DEV void make_uniform(const CollectArgs &a, int k, int env0, int e) {
+        uniform[k & 1][e] = categorical_uniform(a.sample_seed + (uint32_t)k * a.sample_stride, env0 + e);
+    }
+    MRL_DEV void book(EpisodeBooks &b, const CollectArgs &a, EpisodeBooks::Waiting &w, size_t at, int q, int lane, bool mine) const {
+        const int e = lane & (R - 1), sel = drawn[q][e];
+        b.rewards(a, w, at, (float)sel, rew[q][sel][e], don[q][sel][e], lane, mine);
+    }
+    MRL_DEV void draw(int now, int e, int l, float logit) {
+        float pr;
+        const int sel = sample_categorical_quad(logit, A, uniform[now][e], l, pr);
+        if (l == 0) {
+            drawn[now][e] = sel;
+            prob[now][e] = pr;
+        }
+    }
+};
+
+// The env step of one wavefront, lanes 0 .. 15 with action 0, 16 .. 31 with action 1 (the others repeat them), in three
+// pieces that a caller may place at either side of a barrier.
+struct CartPoleStep {
+    float s[4], again[4];
+    cartpole::Push push;
+    int32_t n;
+    MRL_DEV void begin(const CartPoleRows &c, const CollectArgs &a, size_t row, int ne, int now, int lane) {
+        const int e = lane & 15, from = c.drawn[now ^ 1][e];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            s[j] = c.rows[from][e][j];
+            again[j] = c.fresh[now][e][j];
+        }
+        n = c.steps[from][e];
+        if (lane < ne) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) a.r_obs[(row + lane) * 4 + j] = s[j];
+        }
+    }
+    MRL_DEV void middle(int lane) {
+        push = cartpole::push(s, (lane >> 4) & 1);
+        asm volatile("" : "+v"(push.sintheta), "+v"(push.costheta), "+v"(push.temp));   // (here, not where they are used)
+    }
+    MRL_DEV void end(CartPoleRows &c, int now, int lane) {
+        const int e = lane & 15, act = (lane >> 4) & 1;
+        float r, d;
+        cartpole::step(s, n, push, r, d);
+        if (lane < 32) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) c.rows[act][e][j] = d > 0.5f ? again[j] : s[j];
+            c.steps[act][e] = d > 0.5f ? 0 : n;
+            c.rew[now][act][e] = r;
+            c.don[now][act][e] = d;
+        }
+    }
+};
+
+// Hidden widths 128 and 256: four wavefronts per net.
+template <int H, int ACT>
+__global__ __launch_bounds__(512, 4) void collect_cartpole16_kernel(CollectArgs a, int32_t *side) {
+    constexpr int IN = cartpole::OBS, A = 2, R = PR16, T = 512, NT = H / 64;
+    constexpr bool RESIDENT = H <= 128;
+    constexpr int KB = RESIDENT ? H / 4 : 8;   // k-steps of layer-1 weights held (all of them, or the next block)
+    __shared__ CartPoleRows c;
+    __shared__ float vals[2][R];
+    __shared__ float hT[2][H * HT16_LD];
+    __shared__ float h2[2][R * (H + 1)];
+    __shared__ float logits[R * (PA_MAX + 1)];
+    __shared__ __align__(16) float w2a[HEAD_LDS(H)];
+    __shared__ float w2c[H + 1];
+    const int t = threadIdx.x;
+    const int env0 = blockIdx.x * R;
+    const int nenv = min(R, a.n_envs - env0);
+    const int N = a.n_envs;
+    __shared__ EpisodeBooks::Waiting finished;
+    const bool keeper = t / WAVE == 1;   // wavefront 1, a lane per env
+    EpisodeBooks books;
+    books.begin(a, env0 + t - WAVE, keeper && t - WAVE < nenv);
+    if (t < R) {
+        c.load(a, side, env0, nenv, t);
+        c.make_fresh(a, 0, env0, t);
+        c.make_uniform(a, 0, env0, t);
+    }
+    stage_head(a.actor_p + IN * H + H + H * H + H, H, A, false, w2a, t, T);
+    for (int i = t; i < H + 1; i += T) w2c[i] = a.critic_p[IN * H + H + H * H + H + i];
+    Hidden16Operands<H, IN, NT, KB> ops;
+    if (RESIDENT) ops.load(t >= T / 2 ? a.critic_p : a.actor_p, 16 * NT * ((t / WAVE) & 3), t % WAVE);
+    __syncthreads();
+
+    auto book = [&](int k, int e, int ne) {   // what step k leaves beside the envs' rows
+        const size_t at = (size_t)(a.t0 + k) * N + env0 + e;
+        c.book(books, a, finished, at, k & 1, e, e < ne);
+        if (e >= ne) return;
+        a.r_logp[at] = log32(c.prob[k & 1][e] + 1e-8f);
+        a.r_values[at] = vals[k & 1][e];
+    };
+    for (int k = 0; k < a.n_steps; ++k) {
+        // (the empty asm keeps what the optimiser derives from these values inside the step)
+        int tid = t, ne = __builtin_amdgcn_readfirstlane(nenv), zero = 0;
+        asm volatile("" : "+v"(tid), "+s"(zero), "+s"(ne) : : "memory");
+        const int wave = tid / WAVE, lane = tid % WAVE, net = wave >> 2, c0 = 16 * NT * (wave & 3);
+        const int now = k & 1, before = now ^ 1;
+        const float *p = (net ? a.critic_p : a.actor_p) + zero;
+        if (!RESIDENT) ops.load(p, c0, lane);
+        const float a0[1] = {c.input(before, lane)};
+        hidden16_layer0_of<H, IN, ACT, NT, KB>(a0, hT[net], ops, c0, lane);
+        __syncthreads();
+        hidden16_layer1<H, IN, ACT, NT, KB>(p, hT[net], h2[net], ops, c0, lane, [] {});
+        __syncthreads();
+        // ---- heads (hidden width 256: on all wavefronts of the net; 128: the actor's on 0, the critic's on 7) and draw
+        if (H == 256) {
+            if (net == 0) head16<H>(w2a, A, h2[0], logits, PA_MAX + 1, tid, T / 2);
+            else head16_value<H>(w2c, h2[1], vals[now], tid - T / 2, T / 2);
+            __syncthreads();
+        } else if (wave == 7) {
+            head16_value<H>(w2c, h2[1], vals[now], lane, WAVE);
+        }
+        if (wave == 0) {
+            const int e = lane >> 2, l = lane & 3;
+            if (H != 256) {
+                head16<H>(w2a, A, h2[0], logits, PA_MAX + 1, lane, WAVE);
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");   // (this wavefront's own writes)
+            }
+            c.draw(now, e, l, logits[e * (PA_MAX + 1) + (l & 1)]);
+        } else if (wave == 5) {
+            CartPoleStep step;
+            step.begin(c, a, (size_t)(a.t0 + k) * N + env0, ne, now, lane);
+            step.middle(lane);
+            step.end(c, now, lane);
+        } else if (wave == 1) {
+            if (k > 0) book(k - 1, lane, ne);
+        } else if (wave == 2) {
+            if (lane < R) c.make_uniform(a, k + 1, env0, lane);
+        } else if (wave == 3) {
+            if (lane < R) c.make_fresh(a, k + 1, env0, lane);
+        }
+        __syncthreads();
+    }
+    if (keeper) {
+        if (a.n_steps > 0) book(a.n_steps - 1, t - WAVE, nenv);
+        books.end(a, finished, env0 + t - WAVE, t - WAVE, t - WAVE < nenv);
+    }
+    if (t < nenv) c.store(a, side, env0, t);
+}
+
+// Hidden width 64.  The critic's products are as long as the actor's and nothing of a step waits for the value, so the
+// critic has two wavefronts of its own, on SIMDs 2 and 3, which take its second layer while wavefront 0 draws; its head follows a
+// step later.  The chain of a step is the actor's: layer 0 | layer 1 | head and draw.
+//   wavefronts 0 .. 3   layer 0           layer 1              0: head, draw; 1: what step k + 1 needs of its seeds
+//              4        rewards of k - 1  critic's head k - 1  log-probability of k - 1
+//              5        rows              the env step ...     ... with both actions
+//              6, 7     critic's layer 0  critic's layer 1 ... ...
+template <int ACT>
+__global__ __launch_bounds__(512, 4) void collect_cartpole16_h64_kernel(CollectArgs a, int32_t *side) {
+    constexpr int H = 64, IN = cartpole::OBS, A = 2, R = PR16, T = 512, KB = H / 4;
+    constexpr int EARLY = 8;   // k-steps of the critic's layer 1 beside the actor's (2, 4, 7: 1.35, 1.33, 1.31 us per step)
+    __shared__ CartPoleRows c;
+    __shared__ float hT[2][H * HT16_LD];
+    __shared__ float h2[2][R * (H + 1)];
+    __shared__ __align__(16) float w2a[HEAD_LDS(H)];
+    __shared__ float w2c[H + 1];
+    __shared__ EpisodeBooks::Waiting finished;
+    const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t / WAVE), lane = t % WAVE;
+    const int env0 = blockIdx.x * R;
+    const int nenv = min(R, a.n_envs - env0);
+    const int N = a.n_envs;
+    if (t < R) {
+        c.load(a, side, env0, nenv, t);
+        c.make_fresh(a, 0, env0, t);
+        c.make_uniform(a, 0, env0, t);
+    }
+    stage_head(a.actor_p + IN * H + H + H * H + H, H, A, false, w2a, t, T);
+    for (int i = t; i < H + 1; i += T) w2c[i] = a.critic_p[IN * H + H + H * H + H + i];
+    const bool last = a.n_steps > 0;
+    const size_t row0 = (size_t)a.t0 * N + env0;   // the first step's rollout row
+    if (wave < 4) {
+        Hidden16Operands<H, IN, 1, KB> ops;
+        const int c0 = 16 * wave;
+        ops.load(a.actor_p, c0, lane);
+        __syncthreads();
+        const int e = lane >> 2, l = lane & 3;
+        HeadRow16<H, A, PA_MAX> head;
+        head.load(w2a, l);
+        for (int k = 0; k < a.n_steps; ++k) {
+            const int now = k & 1;
+            const float a0[1] = {c.input(now ^ 1, lane)};
+            hidden16_layer0_of<H, IN, ACT, 1, KB>(a0, hT[0], ops, c0, lane);
+            __syncthreads();
+            floatx4 p[1] = {floatx4{0}};
+            hidden16_layer1_steps<H, 0, KB>(hT[0], ops, p, lane);
+            hidden16_layer1_end<H, IN, ACT, 1, KB>(p, h2[0], ops, c0, lane);
+            __syncthreads();
+            if (wave == 0) {
+                float out[A];
+                head.sums(h2[0], e, l, out);   // (in all four lanes of a row)
+                c.draw(now, e, l, l == 0 ? out[0] : out[1]);
+            } else if (wave == 1 && lane < R) {
+                c.make_uniform(a, k + 1, env0, lane);
+                c.make_fresh(a, k + 1, env0, lane);
+            }
+            __syncthreads();
+        }
+    } else if (wave == 4) {
+        const bool mine = lane < nenv;
+        EpisodeBooks books;
+        books.begin(a, env0 + lane, mine);
+        __syncthreads();
+        HeadRow16<H, 1, 1> head;
+        head.load(w2c, lane & 3);
+        float prob = 0.0f;
+        auto rewards = [&](int k) {
+            c.book(books, a, finished, row0 + (size_t)k * N + lane, k & 1, lane, mine);
+            prob = c.prob[k & 1][lane & (R - 1)];
+        };
+        auto value = [&](int k) {
+            float out[1];
+            head.sums(h2[1], lane >> 2, lane & 3, out);
+            if ((lane & 3) == 0 && lane >> 2 < nenv) a.r_values[row0 + (size_t)k * N + (lane >> 2)] = out[0];
+        };
+        auto logp = [&](int k) {
+            if (mine) a.r_logp[row0 + (size_t)k * N + lane] = log32(prob + 1e-8f);
+        };
+        for (int k = 0; k < a.n_steps; ++k) {
+            if (k > 0) rewards(k - 1);
+            __syncthreads();
+            if (k > 0) value(k - 1);
+            __syncthreads();
+            if (k > 0) logp(k - 1);
+            __syncthreads();
+        }
+        if (last) {
+            rewards(a.n_steps - 1);
+            value(a.n_steps - 1);
+            logp(a.n_steps - 1);
+        }
+        books.end(a, finished, env0 + lane, lane, mine);
+    } else if (wave == 5) {
+        __syncthreads();
+        for (int k = 0; k < a.n_steps; ++k) {
+            CartPoleStep step;
+            step.begin(c, a, row0 + (size_t)k * N, nenv, k & 1, lane);
+            __syncthreads();
+            step.middle(lane);
+            __syncthreads();
+            step.end(c, k & 1, lane);
+            __syncthreads();
+        }
+        if (lane < nenv) c.store(a, side, env0, lane);
+    } else {
+        Hidden16Operands<H, IN, 2, KB> ops;
+        const int c0 = 32 * (wave - 6);
+        ops.load(a.critic_p, c0, lane);
+        __syncthreads();
+        for (int k = 0; k < a.n_steps; ++k) {
+            const float a0[1] = {c.input((k & 1) ^ 1, lane)};
+            hidden16_layer0_of<H, IN, ACT, 2, KB>(a0, hT[1], ops, c0, lane);
+            __syncthreads();
+            floatx4 p[2] = {floatx4{0}, floatx4{0}};
+            hidden16_layer1_steps<H, 0, EARLY>(hT[1], ops, p, lane);
+            __syncthreads();
+            hidden16_layer1_steps<H, EARLY, KB>(hT[1], ops, p, lane);
+            hidden16_layer1_end<H, IN, ACT, 2, KB>(p, h2[1], ops, c0, lane);
+            __syncthreads();
+        }
+    }
+}
+
+// Lanes 0 .. 15 of wavefront 0 carry one env each in registers.
+template <int H, int ACT>
+__global__ __launch_bounds__(512, 4) void collect_pendulum16_kernel(CollectArgs a) {
+    constexpr int IN = PendulumSlot::OBS, A = 1, R = PR16, T = 512, NT = H / 64;
     constexpr bool RESIDENT = H <= 128;
     constexpr int KB = RESIDENT ? H / 4 : 8;   // k-steps of layer-1 weights held (all of them, or the next block)
     __shared__ float xs[R * XS_LD];
@@ -292,6 +648,7 @@ __global__ __launch_bounds__(512, 4) void collect_classic16_kernel(CollectArgs a
     __shared__ float h2[2][R * (H + 1)];
     __shared__ float logits[R * (PA_MAX + 1)];
     __shared__ float vals[R];
+    __shared__ float noise[2][R];     // step k's normal numbers at [k & 1]
     __shared__ __align__(16) float w2a[HEAD_LDS(H)];
     __shared__ float w2c[H + 1];
     const int t = threadIdx.x;
@@ -299,24 +656,22 @@ __global__ __launch_bounds__(512, 4) void collect_classic16_kernel(CollectArgs a
     const int nenv = min(R, a.n_envs - env0);
     const int N = a.n_envs;
     const bool owner = t < nenv;   // lanes 0 .. nenv - 1 of wavefront 0: one env each
-    C slot{};
+    PendulumSlot slot{};
     float ep_return = 0.0f, ep_length = 0.0f;
     if (owner) {
-        slot.load(a.states, side, env0 + t);
+        slot.load(a.states, env0 + t);
         ep_return = a.acc.ep_return[env0 + t];
         ep_length = a.acc.ep_length[env0 + t];
     }
-    stage_head(a.actor_p + IN * H + H + H * H + H, H, A, GAUSS, w2a, t, T);
+    stage_head(a.actor_p + IN * H + H + H * H + H, H, A, true, w2a, t, T);
     for (int i = t; i < H + 1; i += T) w2c[i] = a.critic_p[IN * H + H + H * H + H + i];
     for (int i = t; i < R * XS_LD; i += T) xs[i] = 0.0f;
     Hidden16Operands<H, IN, NT, KB> ops;
     if (RESIDENT) ops.load(t >= T / 2 ? a.critic_p : a.actor_p, 16 * NT * ((t / WAVE) & 3), t % WAVE);
+    if (t / WAVE == 2 && t % WAVE < R) noise[0][t % WAVE] = gaussian_noise(a.sample_seed, env0 + t % WAVE, A, 0);
     __syncthreads();
     // the policy does not change during the launch: exp(log_std) of the Gaussian head once for all the steps
-    float stdv[A];
-#pragma unroll
-    for (int j = 0; j < A; ++j)
-        stdv[j] = GAUSS ? exp32(gaussian_log_std(w2a[HEAD_LOG_STD(H) + j])) : 1.0f;
+    const float stdv = exp32(gaussian_log_std(w2a[HEAD_LOG_STD(H)]));
 
     for (int k = 0; k < a.n_steps; ++k) {
         // (the empty asm keeps what the optimiser derives from these values inside the step)
@@ -341,19 +696,14 @@ __global__ __launch_bounds__(512, 4) void collect_classic16_kernel(CollectArgs a
         if (net == 0) head16<H>(w2a, A, h2[0], logits, PA_MAX + 1, tid, T / 2);
         else head16_value<H>(w2c, h2[1], vals, tid - T / 2, T / 2);
         __syncthreads();
+        const int i = env0 + lane;
+        if (wave == 2 && lane < R) noise[(k + 1) & 1][lane] = gaussian_noise(sseed + a.sample_stride, i, A, 0);
         if (wave > 1 || lane >= ne) continue;
         // wavefronts 0 and 1 draw the action; 1 goes on to its log-probability and the rollout row, 0 to the env step
-        const int i = env0 + lane;
-        float av[A], logp;
-        if (GAUSS) {
-            logp = sample_gaussian(logits + lane * (PA_MAX + 1), w2a + HEAD_LOG_STD(H), A, sseed, i, av, stdv);
-        } else {
-            int sel;
-            sample_categorical_few(logits + lane * (PA_MAX + 1), A, sseed, i, sel, logp);
-            av[0] = (float)sel;
-        }
+        float av[A];
+        const float logp = sample_gaussian(logits + lane * (PA_MAX + 1), w2a + HEAD_LOG_STD(H), A, sseed, i, av, &stdv, noise[k & 1] + lane);
         if (wave == 1) {
-            for (int j = 0; j < AW; ++j) a.r_actions[(row + lane) * AW + j] = av[j];
+            a.r_actions[row + lane] = av[0];
             a.r_logp[row + lane] = logp;
             a.r_values[row + lane] = vals[lane];
             continue;
@@ -376,12 +726,178 @@ __global__ __launch_bounds__(512, 4) void collect_classic16_kernel(CollectArgs a
         }
     }
     if (owner) {
-        slot.store(a.states, side, env0 + t);
+        slot.store(a.states, env0 + t);
 #pragma unroll
         for (int c = 0; c < IN; ++c) a.obs[(size_t)(env0 + t) * IN + c] = slot.obs(c);
         a.acc.ep_return[env0 + t] = ep_return;
         a.acc.ep_length[env0 + t] = ep_length;
     }
+}
+
+// Hidden width 64, as CartPole's: the critic on two wavefronts of its own.  Wavefront 0 carries the envs, in all four lanes of
+// one's row of the head, and goes on from the head's sum to the action and the env step.
+//   wavefronts 0 .. 3   layer 0           layer 1              0: head, env step; 1: the normal numbers of step k + 1
+//              4        rewards of k - 1  critic's head k - 1  log-probability of k - 1
+//              5        observations out  sine of the angle
+//              6, 7     critic's layer 0  critic's layer 1 ... ...
+template <int ACT>
+__global__ __launch_bounds__(512, 4) void collect_pendulum16_h64_kernel(CollectArgs a) {
+    constexpr int H = 64, IN = pendulum::OBS, R = PR16, T = 512, KB = H / 4, EARLY = 8;
+    struct Row { float obs[IN], theta, sine; };
+    __shared__ Row rows[R];
+    __shared__ float noise[2][R], mean[R], action[R], rew[R], don[R];
+    __shared__ float hT[2][H * HT16_LD];
+    __shared__ float h2[2][R * (H + 1)];
+    __shared__ __align__(16) float w2a[HEAD_LDS(H)];
+    __shared__ float w2c[H + 1];
+    __shared__ EpisodeBooks::Waiting finished;
+    const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t / WAVE), lane = t % WAVE;
+    const int env0 = blockIdx.x * R;
+    const int nenv = min(R, a.n_envs - env0);
+    const int N = a.n_envs;
+    const size_t row0 = (size_t)a.t0 * N + env0;   // the first step's rollout row
+    const int e = lane >> 2, l = lane & 3;
+    stage_head(a.actor_p + IN * H + H + H * H + H, H, 1, true, w2a, t, T);
+    for (int i = t; i < H + 1; i += T) w2c[i] = a.critic_p[IN * H + H + H * H + H + i];
+    auto input = [&](float (&a0)[1]) {
+        const int g = lane >> 4;
+        a0[0] = g < IN ? rows[lane & 15].obs[g < IN ? g : 0] : 0.0f;
+    };
+    if (wave < 4) {
+        PendulumSlot slot{};
+        if (wave == 0) {
+            if (e < nenv) slot.load(a.states, env0 + e);
+            if (l == 0) {
+#pragma unroll
+                for (int c = 0; c < IN; ++c) rows[e].obs[c] = slot.obs(c);
+                rows[e].theta = slot.s[3];
+            }
+        } else if (wave == 1 && lane < R) {
+            noise[0][lane] = gaussian_noise(a.sample_seed, env0 + lane, 1, 0);
+        }
+        Hidden16Operands<H, IN, 1, KB> ops;
+        const int c0 = 16 * wave;
+        ops.load(a.actor_p, c0, lane);
+        __syncthreads();
+        HeadRow16<H, 1, PA_MAX> head;
+        head.load(w2a, l);
+        const float std = exp32(gaussian_log_std(w2a[HEAD_LOG_STD(H)]));
+        for (int k = 0; k < a.n_steps; ++k) {
+            float a0[1];
+            input(a0);
+            hidden16_layer0_of<H, IN, ACT, 1, KB>(a0, hT[0], ops, c0, lane);
+            __syncthreads();
+            floatx4 p[1] = {floatx4{0}};
+            hidden16_layer1_steps<H, 0, KB>(hT[0], ops, p, lane);
+            hidden16_layer1_end<H, IN, ACT, 1, KB>(p, h2[0], ops, c0, lane);
+            __syncthreads();
+            if (wave == 0) {
+                const float sine = rows[e].sine, z = noise[k & 1][e];
+                float mu[1], r, d;
+                head.sums(h2[0], e, l, mu);
+                const float u = mu[0] + std * z;
+                pendulum::step(slot.s, u, sine, r, d);
+                if (d > 0.5f) slot.reset(env0 + e, a.reset_seed + (uint64_t)k * a.reset_stride);
+                if (l == 0) {
+#pragma unroll
+                    for (int c = 0; c < IN; ++c) rows[e].obs[c] = slot.obs(c);
+                    rows[e].theta = slot.s[3];
+                    mean[e] = mu[0];
+                    action[e] = u;
+                    rew[e] = r;
+                    don[e] = d;
+                }
+            } else if (wave == 1 && lane < R) {
+                noise[(k + 1) & 1][lane] = gaussian_noise(a.sample_seed + (uint32_t)(k + 1) * a.sample_stride, env0 + lane, 1, 0);
+            }
+            __syncthreads();
+        }
+        if (wave == 0 && l == 0 && e < nenv) {
+            slot.store(a.states, env0 + e);
+#pragma unroll
+            for (int c = 0; c < IN; ++c) a.obs[(size_t)(env0 + e) * IN + c] = slot.obs(c);
+        }
+    } else if (wave == 4) {
+        const bool mine = lane < nenv;
+        const int q = lane & (R - 1);
+        EpisodeBooks books;
+        books.begin(a, env0 + lane, mine);
+        __syncthreads();
+        HeadRow16<H, 1, 1> head;
+        head.load(w2c, l);
+        const float log_std = gaussian_log_std(w2a[HEAD_LOG_STD(H)]), std = exp32(log_std);
+        float u = 0.0f, mu = 0.0f;
+        auto rewards = [&](int k) {
+            u = action[q];
+            mu = mean[q];
+            books.rewards(a, finished, row0 + (size_t)k * N + lane, u, rew[q], don[q], lane, mine);
+        };
+        auto value = [&](int k) {
+            float out[1];
+            head.sums(h2[1], e, l, out);
+            if (l == 0 && e < nenv) a.r_values[row0 + (size_t)k * N + e] = out[0];
+        };
+        auto logp = [&](int k) {
+            if (mine) a.r_logp[row0 + (size_t)k * N + lane] = 0.0f + gaussian_logp(u, mu, log_std, std);
+        };
+        for (int k = 0; k < a.n_steps; ++k) {
+            if (k > 0) rewards(k - 1);
+            __syncthreads();
+            if (k > 0) value(k - 1);
+            __syncthreads();
+            if (k > 0) logp(k - 1);
+            __syncthreads();
+        }
+        if (a.n_steps > 0) {
+            rewards(a.n_steps - 1);
+            value(a.n_steps - 1);
+            logp(a.n_steps - 1);
+        }
+        books.end(a, finished, env0 + lane, lane, mine);
+    } else if (wave == 5) {
+        __syncthreads();
+        for (int k = 0; k < a.n_steps; ++k) {
+            const int q = lane & (R - 1);
+            const float theta = rows[q].theta;
+            if (lane < nenv) {
+#pragma unroll
+                for (int c = 0; c < IN; ++c) a.r_obs[(row0 + (size_t)k * N + lane) * IN + c] = rows[q].obs[c];
+            }
+            __syncthreads();
+            if (lane < R) rows[lane].sine = sin32(theta);
+            __syncthreads();
+            __syncthreads();
+        }
+    } else {
+        Hidden16Operands<H, IN, 2, KB> ops;
+        const int c0 = 32 * (wave - 6);
+        ops.load(a.critic_p, c0, lane);
+        __syncthreads();
+        for (int k = 0; k < a.n_steps; ++k) {
+            float a0[1];
+            input(a0);
+            hidden16_layer0_of<H, IN, ACT, 2, KB>(a0, hT[1], ops, c0, lane);
+            __syncthreads();
+            floatx4 p[2] = {floatx4{0}, floatx4{0}};
+            hidden16_layer1_steps<H, 0, EARLY>(hT[1], ops, p, lane);
+            __syncthreads();
+            hidden16_layer1_steps<H, EARLY, KB>(hT[1], ops, p, lane);
+            hidden16_layer1_end<H, IN, ACT, 2, KB>(p, h2[1], ops, c0, lane);
+            __syncthreads();
+        }
+    }
+}
+
+template <int H, int ACT>
+void launch_cartpole16(mrl_ctx *ctx, dim3 grid, const CollectArgs &a, int32_t *side) {
+    if constexpr (H == 64) hipLaunchKernelGGL((collect_cartpole16_h64_kernel<ACT>), grid, dim3(512), 0, ctx->stream, a, side);
+    else hipLaunchKernelGGL((collect_cartpole16_kernel<H, ACT>), grid, dim3(512), 0, ctx->stream, a, side);
+}
+
+template <int H, int ACT>
+void launch_pendulum16(mrl_ctx *ctx, dim3 grid, const CollectArgs &a) {
+    if constexpr (H == 64) hipLaunchKernelGGL((collect_pendulum16_h64_kernel<ACT>), grid, dim3(512), 0, ctx->stream, a);
+    else hipLaunchKernelGGL((collect_pendulum16_kernel<H, ACT>), grid, dim3(512), 0, ctx->stream, a);
 }
 
 // the workgroups of `grid` = 16 envs each; side: CartPole's step counters
@@ -393,9 +909,9 @@ int launch_collect16_t(mrl_ctx *ctx, const mrl_rollout *r, const CollectArgs &a,
     else if (r->env_id == MRL_ENV_LUNARLANDER_CONTINUOUS)
         hipLaunchKernelGGL((collect16_kernel<LunarLanderContinuous, H, ACT, true>), grid, block, 0, ctx->stream, a);
     else if (r->env_id == MRL_ENV_CARTPOLE)
-        hipLaunchKernelGGL((collect_classic16_kernel<CartPoleSlot, H, ACT, false>), grid, dim3(512), 0, ctx->stream, a, side);
+        launch_cartpole16<H, ACT>(ctx, grid, a, side);
     else
-        hipLaunchKernelGGL((collect_classic16_kernel<PendulumSlot, H, ACT, true>), grid, dim3(512), 0, ctx->stream, a, side);
+        launch_pendulum16<H, ACT>(ctx, grid, a);
     MRL_CHECK_LAUNCH();
     return MRL_OK;
 }

@@ -17,16 +17,25 @@ namespace cartpole {
 
 constexpr int STATE = 4, OBS = 4;
 
-MRL_DEV void step(float s[4], int32_t &steps, int action, float &reward, float &done) {
-    const float GRAVITY = (float)9.8, TOTAL_MASS = (float)(1.0 + 0.1), POLE_MASS = (float)0.1;
-    const float POLE_HALF_LENGTH = (float)0.5, POLE_MASS_LENGTH = (float)(0.1 * 0.5);
-    const float FORCE_MAG = (float)10.0, TAU = (float)0.02;
-    const float X_THRESHOLD = (float)2.4, THETA_THRESHOLD = (float)0.2095;
-    float x = s[0], x_dot = s[1], theta = s[2], theta_dot = s[3];
+// the step's first half: the angle's sine and cosine, and what the force does
+struct Push { float sintheta, costheta, temp; };
+MRL_DEV Push push(const float s[4], int action) {
+    const float TOTAL_MASS = (float)(1.0 + 0.1), POLE_MASS_LENGTH = (float)(0.1 * 0.5), FORCE_MAG = (float)10.0;
+    float theta = s[2], theta_dot = s[3];
     float force = (action == 1) ? FORCE_MAG : -FORCE_MAG;
     float sintheta, costheta;
     sincos32(theta, sintheta, costheta);
     float temp = (force + POLE_MASS_LENGTH * theta_dot * theta_dot * sintheta) / TOTAL_MASS;
+    return {sintheta, costheta, temp};
+}
+
+MRL_DEV void step(float s[4], int32_t &steps, const Push &push, float &reward, float &done) {
+    const float GRAVITY = (float)9.8, TOTAL_MASS = (float)(1.0 + 0.1), POLE_MASS = (float)0.1;
+    const float POLE_HALF_LENGTH = (float)0.5, POLE_MASS_LENGTH = (float)(0.1 * 0.5);
+    const float TAU = (float)0.02;
+    const float X_THRESHOLD = (float)2.4, THETA_THRESHOLD = (float)0.2095;
+    float x = s[0], x_dot = s[1], theta = s[2], theta_dot = s[3];
+    float sintheta = push.sintheta, costheta = push.costheta, temp = push.temp;
     float thetaacc = (GRAVITY * sintheta - costheta * temp) /
                      (POLE_HALF_LENGTH *
                       ((float)(4.0 / 3.0) - POLE_MASS * costheta * costheta / TOTAL_MASS));
@@ -43,6 +52,9 @@ MRL_DEV void step(float s[4], int32_t &steps, int action, float &reward, float &
     done = (terminated || truncated) ? 1.0f : 0.0f;
     reward = terminated ? 0.0f : 1.0f;
 }
+MRL_DEV void step(float s[4], int32_t &steps, int action, float &reward, float &done) {
+    step(s, steps, push(s, action), reward, done);
+}
 
 MRL_DEV void reset(float s[4], int32_t &steps, int env, uint32_t seed) {
     uint32_t rng = xorshift32((uint32_t)((uint64_t)env * 2654435761ull + (uint64_t)seed));
@@ -57,14 +69,14 @@ namespace pendulum {
 
 constexpr int STATE = 8, OBS = 3;
 
-MRL_DEV void step(float s[8], float action, float &reward, float &done) {
+// sin_theta: of s[3]
+MRL_DEV void step(float s[8], float action, float sin_theta, float &reward, float &done) {
     const float max_speed = (float)8.0, max_torque = (float)2.0, dt = (float)0.05;
     const float g = (float)10.0, m = (float)1.0, l = (float)1.0;
     float theta = s[3], theta_dot = s[2];
     float u = action * max_torque;
     if (u > max_torque) u = max_torque;
     else if (u < -max_torque) u = -max_torque;
-    float sin_theta = sin32(theta);
     float theta_acc = (3.0f * g) / (2.0f * l) * sin_theta + (3.0f / (m * l * l)) * u;
     theta_dot = theta_dot + theta_acc * dt;
     theta = theta + theta_dot * dt;
@@ -84,6 +96,7 @@ MRL_DEV void step(float s[8], float action, float &reward, float &done) {
     reward = r;
     done = d;
 }
+MRL_DEV void step(float s[8], float action, float &reward, float &done) { step(s, action, sin32(s[3]), reward, done); }
 
 MRL_DEV void reset(float s[8], int env, uint64_t seed) {
     int64_t seed_i = (int64_t)(float)seed;

@@ -118,17 +118,11 @@ struct Hidden16Operands {
     }
 };
 
-// Layer 0 of a tile: xs[16][XS_LD] holds the inputs, hT [H][HT16_LD] receives act(layer 0) k-major.
+// Layer 0 of a tile: a0[kk] = input 4 kk + g of row n, hT [H][HT16_LD] receives act(layer 0) k-major.
 template <int H, int IN, int ACT, int NT, int KB>
-MRL_DEV void hidden16_layer0(const float *xs, float *hT, const Hidden16Operands<H, IN, NT, KB> &ops, int c0, int lane) {
+MRL_DEV void hidden16_layer0_of(const float (&a0)[(IN + 3) / 4], float *hT, const Hidden16Operands<H, IN, NT, KB> &ops, int c0, int lane) {
     constexpr int K0 = (IN + 3) / 4;
     const int g = lane >> 4, n = lane & 15;
-    float a0[K0];
-#pragma unroll
-    for (int kk = 0; kk < K0; ++kk) {
-        const int k = 4 * kk + g;
-        a0[kk] = k < IN ? xs[n * XS_LD + k] : 0.0f;
-    }
     floatx4 c[NT];
 #pragma unroll
     for (int q = 0; q < NT; ++q) c[q] = floatx4{0};
@@ -143,6 +137,45 @@ MRL_DEV void hidden16_layer0(const float *xs, float *hT, const Hidden16Operands<
         const int col = tile16_col<NT>(c0, q, n);
 #pragma unroll
         for (int v = 0; v < 4; ++v) hT[col * HT16_LD + 4 * g + v] = activate<ACT>(c[q][v] + ops.bias0[q]);
+    }
+}
+// the same from xs[16][XS_LD]
+template <int H, int IN, int ACT, int NT, int KB>
+MRL_DEV void hidden16_layer0(const float *xs, float *hT, const Hidden16Operands<H, IN, NT, KB> &ops, int c0, int lane) {
+    constexpr int K0 = (IN + 3) / 4;
+    const int g = lane >> 4, n = lane & 15;
+    float a0[K0];
+#pragma unroll
+    for (int kk = 0; kk < K0; ++kk) {
+        const int k = 4 * kk + g;
+        a0[kk] = k < IN ? xs[n * XS_LD + k] : 0.0f;
+    }
+    hidden16_layer0_of<H, IN, ACT, NT, KB>(a0, hT, ops, c0, lane);
+}
+
+// Biases and activation of layer 1: h2 [16][H + 1] receives act(c + bias) row-major.
+template <int H, int IN, int ACT, int NT, int KB>
+MRL_DEV void hidden16_layer1_end(const floatx4 (&c)[NT], float *h2, const Hidden16Operands<H, IN, NT, KB> &ops, int c0, int lane) {
+    const int g = lane >> 4, n = lane & 15;
+#pragma unroll
+    for (int q = 0; q < NT; ++q) {
+        const int col = tile16_col<NT>(c0, q, n);
+#pragma unroll
+        for (int v = 0; v < 4; ++v) h2[(4 * g + v) * (H + 1) + col] = activate<ACT>(c[q][v] + ops.bias1[q]);
+    }
+}
+// k-steps J0 .. J1 - 1 of layer 1 with all its weights held
+template <int H, int J0, int J1, int IN, int NT>
+MRL_DEV void hidden16_layer1_steps(const float *hT, const Hidden16Operands<H, IN, NT, H / 4> &ops, floatx4 (&c)[NT], int lane) {
+    const float *ht = hT + (lane >> 4) * HT16_LD + (lane & 15);
+    float a[J1 - J0];
+#pragma unroll
+    for (int j = J0; j < J1; ++j) a[j - J0] = ht[4 * j * HT16_LD];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = J0; j < J1; ++j) {
+#pragma unroll
+        for (int q = 0; q < NT; ++q) c[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[j - J0], ops.bv[j][q], c[q], 0, 0, 0);
     }
 }
 
@@ -205,12 +238,7 @@ MRL_DEV void hidden16_layer1(const float *__restrict__ p, const float *hT, float
         product(na, nb);
     }
     before_h2();
-#pragma unroll
-    for (int q = 0; q < NT; ++q) {
-        const int col = tile16_col<NT>(c0, q, n);
-#pragma unroll
-        for (int v = 0; v < 4; ++v) h2[(4 * g + v) * (H + 1) + col] = activate<ACT>(c[q][v] + ops.bias1[q]);
-    }
+    hidden16_layer1_end<H, IN, ACT, NT, KB>(c, h2, ops, c0, lane);
 }
 
 // Hidden stack of one net for the block's 16 rows on the wavefronts that share it (each with its
@@ -251,47 +279,81 @@ MRL_DEV float butterfly_sum(float x) {
 // sums go over the lanes in DPP instructions instead of the LDS crossbar; CartPole, hidden width 64, 1024 envs 2.70 : 2.50
 // us per step, LunarLander, hidden width 256, 4096 envs 19.3 : 18.7.
 template <int H, int NA, int PITCH>
-MRL_DEV void head_rows16(const float *w2s, int A, const float *h2, float *out, int out_ld, int t, int nthreads) {
+MRL_DEV void head_row16(const float *w2s, const float *h2, int r, int part, float (&out)[NA]) {
     constexpr int CP = 16, TPR = H / CP, BLK = NA == 8 ? 8 : 16;
     static_assert(64 % TPR == 0, "the lanes of a row sit in one wavefront");
     static_assert(NA == 1 || (PITCH == PA_MAX && (NA == 4 || NA == 8)), "one float, one float4 or two per padded row");
     const float *b2 = w2s + H * PITCH;
-    for (int pair = t; pair < PR16 * TPR; pair += nthreads) {
-        const int r = pair / TPR, part = pair % TPR;
-        float acc[NA];
+    float acc[NA];
 #pragma unroll
-        for (int a = 0; a < NA; ++a) acc[a] = 0.0f;
-        // (element i is column (i + part) & 15 of the part: up to 15 - part it lies i behind the first, then 16 less)
-        const float *hp = h2 + r * (H + 1) + part * CP + part, *wp = w2s + (part * CP + part) * PITCH;
+    for (int a = 0; a < NA; ++a) acc[a] = 0.0f;
+    // (element i is column (i + part) & 15 of the part: up to 15 - part it lies i behind the first, then 16 less)
+    const float *hp = h2 + r * (H + 1) + part * CP + part, *wp = w2s + (part * CP + part) * PITCH;
 #pragma unroll
-        for (int b = 0; b < CP; b += BLK) {
-            float hv[BLK], wv[BLK][NA];
+    for (int b = 0; b < CP; b += BLK) {
+        float hv[BLK], wv[BLK][NA];
 #pragma unroll
-            for (int j = 0; j < BLK; ++j) {
-                const int i = b + j, back = i + part < CP ? 0 : CP;
-                hv[j] = hp[i - back];
-                const float *w = wp + (i - back) * PITCH;
-                if (NA == 1) {
-                    wv[j][0] = w[0];
-                } else {
+        for (int j = 0; j < BLK; ++j) {
+            const int i = b + j, back = i + part < CP ? 0 : CP;
+            hv[j] = hp[i - back];
+            const float *w = wp + (i - back) * PITCH;
+            if (NA == 1) {
+                wv[j][0] = w[0];
+            } else {
 #pragma unroll
-                    for (int a = 0; a < NA; a += 4) {
-                        const float4 x = *reinterpret_cast<const float4 *>(w + a);
-                        wv[j][a] = x.x; wv[j][a + 1] = x.y; wv[j][a + 2] = x.z; wv[j][a + 3] = x.w;
-                    }
+                for (int a = 0; a < NA; a += 4) {
+                    const float4 x = *reinterpret_cast<const float4 *>(w + a);
+                    wv[j][a] = x.x; wv[j][a + 1] = x.y; wv[j][a + 2] = x.z; wv[j][a + 3] = x.w;
                 }
             }
-#pragma unroll
-            for (int j = 0; j < BLK; ++j) {
-#pragma unroll
-                for (int a = 0; a < NA; ++a) acc[a] = fmaf(hv[j], wv[j][a], acc[a]);
-            }
         }
+#pragma unroll
+        for (int j = 0; j < BLK; ++j) {
+#pragma unroll
+            for (int a = 0; a < NA; ++a) acc[a] = fmaf(hv[j], wv[j][a], acc[a]);
+        }
+    }
+#pragma unroll
+    for (int a = 0; a < NA; ++a) out[a] = butterfly_sum<TPR>(acc[a]) + b2[a];   // (in all lanes of the row)
+}
+// The same, of one or two outputs, with a lane's weights in registers from call to call.
+template <int H, int NA, int PITCH>
+struct HeadRow16 {
+    static constexpr int CP = 16, TPR = H / CP;
+    float w[CP][NA], b[NA];
+    MRL_DEV void load(const float *w2s, int part) {
 #pragma unroll
         for (int a = 0; a < NA; ++a) {
-            const float v = butterfly_sum<TPR>(acc[a]);
-            if (part == 0 && a < A) out[r * out_ld + a] = v + b2[a];
+            b[a] = w2s[H * PITCH + a];
+#pragma unroll
+            for (int i = 0; i < CP; ++i) w[i][a] = w2s[(part * CP + ((i + part) & (CP - 1))) * PITCH + a];
         }
+    }
+    MRL_DEV void sums(const float *h2, int r, int part, float (&out)[NA]) const {
+        const float *hp = h2 + r * (H + 1) + part * CP + part;
+        float hv[CP], acc[NA];
+#pragma unroll
+        for (int i = 0; i < CP; ++i) hv[i] = hp[i - (i + part < CP ? 0 : CP)];
+#pragma unroll
+        for (int a = 0; a < NA; ++a) acc[a] = 0.0f;
+#pragma unroll
+        for (int i = 0; i < CP; ++i)
+#pragma unroll
+            for (int a = 0; a < NA; ++a) acc[a] = fmaf(hv[i], w[i][a], acc[a]);
+#pragma unroll
+        for (int a = 0; a < NA; ++a) out[a] = butterfly_sum<TPR>(acc[a]) + b[a];
+    }
+};
+template <int H, int NA, int PITCH>
+MRL_DEV void head_rows16(const float *w2s, int A, const float *h2, float *out, int out_ld, int t, int nthreads) {
+    constexpr int TPR = H / 16;
+    for (int pair = t; pair < PR16 * TPR; pair += nthreads) {
+        const int r = pair / TPR, part = pair % TPR;
+        float v[NA];
+        head_row16<H, NA, PITCH>(w2s, h2, r, part, v);
+#pragma unroll
+        for (int a = 0; a < NA; ++a)
+            if (part == 0 && a < A) out[r * out_ld + a] = v[a];
     }
 }
 

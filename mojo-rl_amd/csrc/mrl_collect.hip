@@ -7,8 +7,8 @@
 // env step through LDS; rollout row t is written on the way.
 // No workgroup waits for another, so there is nothing between two steps but the block's own
 // barriers; the launch ends when every block has done its n_steps.
-// The kernels: collect16.hpp (LunarLander, CartPole, Pendulum), collect_walkers.hpp (the others), and for many CartPole /
-// Pendulum envs the one below; the entry that picks one, or single steps, is at the end of the file.
+// The kernels: collect16.hpp (LunarLander, CartPole, Pendulum), collect_walkers.hpp (the others); here the entry that picks
+// one, or single steps.
 //
 // It gives what n_steps calls of mrl_rollout_step give (same per-env streams: seeds are affine
 // in the step number), except that the finished-episode list is appended in the order in which
@@ -31,124 +31,11 @@ extern template int launch_collect16_t<128, 2>(mrl_ctx *, const mrl_rollout *, c
 extern template int launch_collect16_t<256, 1>(mrl_ctx *, const mrl_rollout *, const CollectArgs &, int32_t *);
 extern template int launch_collect16_t<256, 2>(mrl_ctx *, const mrl_rollout *, const CollectArgs &, int32_t *);
 
-// ---------------------------------------------------------------- CartPole / Pendulum
-// For the envs whose state is a handful of floats, in numbers: a workgroup of four wavefronts
-// (two on the actor, two on the critic, hidden width 64, one 32-column tile each) takes its 32
-// envs through all the steps of the launch.  Each wavefront's share of the hidden layers' weights
-// is loaded into registers once, before the first step; lanes 0 .. 31 of wavefront 0 carry one
-// env each in registers -- state, step counter, episode sums -- and do sampling, step,
-// accounting and reset in place.  A step is one dependent chain (observation -> two layers on
-// the matrix cores -> head -> sample -> env step), so the time of a step does not depend on the
-// number of envs until there are more workgroups than the chip holds at once.
-constexpr int CLASSIC_TPW = 1;   // accumulator tiles per wavefront: 1 = two wavefronts per net
-constexpr int CLASSIC_THREADS = 2 * hidden_threads(64, CLASSIC_TPW);
-
-template <class C, int ACT, bool GAUSS>
-__global__ __launch_bounds__(CLASSIC_THREADS) void collect_classic_kernel(CollectArgs a, int32_t *side) {
-    constexpr int H = 64, TPW = CLASSIC_TPW, TN = hidden_threads(H, TPW), IN = C::OBS, AW = C::ACT_W;
-    constexpr int KB = H / 2;   // all of layer 1 in one block of k-steps: its weights stay in registers
-    static_assert(IN <= PIN_MAX, "observation fits the input tile");
-    __shared__ float xs[PR * XS_LD];
-    __shared__ float hT[2][H * HT_LD];
-    __shared__ float h2[2][PR * (H + 1)];
-    __shared__ float logits[PR * (PA_MAX + 1)];
-    __shared__ float vals[PR];
-    __shared__ __align__(16) float w2s[2][HEAD_LDS(H)];
-    const int t = threadIdx.x;
-    const int env0 = blockIdx.x * PR;
-    const int nenv = min(PR, a.n_envs - env0);
-    const int N = a.n_envs;
-    const bool owner = t < nenv;   // lanes 0 .. nenv - 1 of wavefront 0: one env each
-    C slot{};
-    float ep_return = 0.0f, ep_length = 0.0f;
-    if (owner) {
-        slot.load(a.states, side, env0 + t);
-        ep_return = a.acc.ep_return[env0 + t];
-        ep_length = a.acc.ep_length[env0 + t];
-    }
-    {
-        const int net = t / TN;
-        const float *p = net ? a.critic_p : a.actor_p;
-        stage_head(p + IN * H + H + H * H + H, H, net ? 1 : a.A, GAUSS && net == 0, w2s[net], t % TN, TN);
-    }
-    for (int i = t; i < PR * XS_LD; i += CLASSIC_THREADS) xs[i] = 0.0f;
-    // the hidden layers' weights of this wavefront's column tiles, loaded once for all the steps
-    HiddenOperands<H, TPW, KB> ops;
-    ops.load(t / TN ? a.critic_p : a.actor_p, IN, t);
-    __syncthreads();
-    // the policy does not change during the launch: exp(log_std) of the Gaussian head once for all the steps
-    float stdv[PA_MAX];
-#pragma unroll
-    for (int j = 0; j < PA_MAX; ++j) stdv[j] = (GAUSS && owner && j < a.A) ? exp32(gaussian_log_std(w2s[0][HEAD_LOG_STD(H) + j])) : 1.0f;
-
-    for (int k = 0; k < a.n_steps; ++k) {
-        // (the empty asm keeps what the optimiser derives from these values inside the step)
-        int tid = t, ne = __builtin_amdgcn_readfirstlane(nenv), A = __builtin_amdgcn_readfirstlane(a.A), zero = 0;
-        asm volatile("" : "+v"(tid), "+s"(zero), "+s"(ne), "+s"(A) : : "memory");
-        const int net = tid / TN;
-        const float *p = (net ? a.critic_p : a.actor_p) + zero;
-        const size_t row = (size_t)(a.t0 + k) * N + env0;   // this block's slice of rollout row t
-        const uint32_t sseed = a.sample_seed + (uint32_t)k * a.sample_stride;
-        if (tid < ne) {
-#pragma unroll
-            for (int c = 0; c < IN; ++c) {
-                const float v = slot.obs(c);
-                xs[tid * XS_LD + c] = v;
-                a.r_obs[(row + tid) * IN + c] = v;
-            }
-        }
-        __syncthreads();
-        hidden_stack<H, ACT, TPW, KB>(p, IN, xs, hT[net], h2[net], TileCache{}, ops, tid);
-        if (net == 0) head<H>(w2s[0], A, h2[0], logits, PA_MAX + 1, tid % TN, TN);
-        else head<H>(w2s[1], 1, h2[1], vals, 1, tid % TN, TN);
-        __syncthreads();
-        if (tid < ne) {
-            const int i = env0 + tid;
-            float av[PA_MAX], logp;
-            if (GAUSS) {
-                logp = sample_gaussian(logits + tid * (PA_MAX + 1), w2s[0] + HEAD_LOG_STD(H), A, sseed, i, av, stdv);
-                for (int j = 0; j < A; ++j) a.r_actions[(row + tid) * AW + j] = av[j];
-            } else {
-                int sel;
-                sample_categorical_few(logits + tid * (PA_MAX + 1), A, sseed, i, sel, logp);
-                av[0] = (float)sel;
-                a.r_actions[row + tid] = av[0];
-            }
-            a.r_logp[row + tid] = logp;
-            a.r_values[row + tid] = vals[tid];
-            float r, d;
-            slot.step(av, r, d);
-            a.r_rewards[row + tid] = r;
-            a.r_dones[row + tid] = d;
-            ep_return = ep_return + r;
-            ep_length = ep_length + 1.0f;
-            if (d > 0.5f) {
-                const int s = atomicAdd(a.acc.done_count, 1);
-                if (s < a.acc.done_cap) {
-                    a.acc.done_returns[s] = ep_return;
-                    a.acc.done_lengths[s] = ep_length;
-                }
-                ep_return = 0.0f;
-                ep_length = 0.0f;
-                slot.reset(i, a.reset_seed + (uint64_t)k * a.reset_stride);
-            }
-        }
-    }
-    if (owner) {
-        slot.store(a.states, side, env0 + t);
-#pragma unroll
-        for (int c = 0; c < IN; ++c) a.obs[(size_t)(env0 + t) * IN + c] = slot.obs(c);
-        a.acc.ep_return[env0 + t] = ep_return;
-        a.acc.ep_length[env0 + t] = ep_length;
-    }
-}
-
 // What mrl_rollout_steps runs a descriptor with.
 enum CollectForm {
     FORM_STEPS,      // no fused kernel: the steps are issued one by one
     FORM_WALKER,     // collect_walkers.hpp
-    FORM_ROWS16,     // collect16.hpp
-    FORM_CLASSIC32   // collect_classic_kernel
+    FORM_ROWS16      // collect16.hpp
 };
 struct CollectPlan {
     CollectForm form;
@@ -219,11 +106,7 @@ static CollectPlan collect_plan(const mrl_rollout *r, int n_cus) {
     else if (id == MRL_ENV_PENDULUM && gauss) obs = pendulum::OBS;
     else return p;
     if (!agent_nets(r, obs, 0, gauss, &p.H, &p.act)) return p;
-    // Hidden width 64, us per step, 16 rows : 32 rows.  CartPole at 4096 / 5000 / 6144 / 7168 / 8192 / 16384 envs 2.7 : 4.2,
-    // 3.5 : 4.4, 3.9 : 4.3, 4.4 : 4.3, 5.0 : 4.3, 9.8 : 5.9; Pendulum at 6144 / 8192 / 12288 / 16384 / 32768 envs 4.0 : 4.4,
-    // 4.0 : 4.3, 5.0 : 6.2, 6.8 : 6.3, 12.5 : 12.2: with more than 16 envs per CU workgroups share the matrix units.
-    const int rows16_per_cu = id == MRL_ENV_CARTPOLE ? 24 : 48;
-    p.form = (p.H == 64 && r->n_envs > rows16_per_cu * n_cus) ? FORM_CLASSIC32 : FORM_ROWS16;
+    p.form = FORM_ROWS16;
     return p;
 }
 
@@ -286,7 +169,6 @@ int mrl_rollout_steps(mrl_ctx *ctx, const mrl_rollout *r, int t0, int n_steps, u
     a.spin_limit = ctx->spin_limit;
     a.sync_error = ctx->sync_error;
     a.car_trait_form = ctx->car_trait_form;
-    const dim3 grid(grid_for(r->n_envs, PR));
     int32_t *side = nullptr;
     if (r->env_id == MRL_ENV_CARTPOLE) {
         rc = cartpole_side(ctx, r->states, r->n_envs, &side);
@@ -294,23 +176,15 @@ int mrl_rollout_steps(mrl_ctx *ctx, const mrl_rollout *r, int t0, int n_steps, u
     }
     profile_step_begin(ctx);
     profile_mark(ctx, -1);
-    if (plan.form == FORM_WALKER || plan.form == FORM_ROWS16) {
-        const bool w = plan.form == FORM_WALKER, relu = plan.act == 1;
-#define MRL_COLLECT(HH)                                                                                          \
-    rc = w ? (relu ? launch_collect_walker_t<HH, 1>(ctx, r, a) : launch_collect_walker_t<HH, 2>(ctx, r, a))       \
+    const bool w = plan.form == FORM_WALKER, relu = plan.act == 1;
+#define MRL_COLLECT(HH)                                                                                     \
+    rc = w ? (relu ? launch_collect_walker_t<HH, 1>(ctx, r, a) : launch_collect_walker_t<HH, 2>(ctx, r, a)) \
            : (relu ? launch_collect16_t<HH, 1>(ctx, r, a, side) : launch_collect16_t<HH, 2>(ctx, r, a, side))
-        if (plan.H == 64) MRL_COLLECT(64);
-        else if (plan.H == 128) MRL_COLLECT(128);
-        else MRL_COLLECT(256);
+    if (plan.H == 64) MRL_COLLECT(64);
+    else if (plan.H == 128) MRL_COLLECT(128);
+    else MRL_COLLECT(256);
 #undef MRL_COLLECT
-        if (rc) return rc;
-    } else if (r->env_id == MRL_ENV_CARTPOLE) {
-        if (plan.act == 1) hipLaunchKernelGGL((collect_classic_kernel<CartPoleSlot, 1, false>), grid, dim3(CLASSIC_THREADS), 0, ctx->stream, a, side);
-        else hipLaunchKernelGGL((collect_classic_kernel<CartPoleSlot, 2, false>), grid, dim3(CLASSIC_THREADS), 0, ctx->stream, a, side);
-    } else {
-        if (plan.act == 1) hipLaunchKernelGGL((collect_classic_kernel<PendulumSlot, 1, true>), grid, dim3(CLASSIC_THREADS), 0, ctx->stream, a, side);
-        else hipLaunchKernelGGL((collect_classic_kernel<PendulumSlot, 2, true>), grid, dim3(CLASSIC_THREADS), 0, ctx->stream, a, side);
-    }
+    if (rc) return rc;
     MRL_CHECK_LAUNCH();
     profile_mark(ctx, MRL_PHASE_COLLECT);
     profile_step_end(ctx);
