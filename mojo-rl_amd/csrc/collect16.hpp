@@ -234,6 +234,331 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
     S::out(rows, gbase, nenv, t, 0, E::STATE);
 }
 
+// Reward and done flag of a step into the rollout, and the episode sums, a lane per env of one wavefront.  Finished episodes wait
+// in LDS until some dozens are there: their places in the list come from one counter of the whole chip, at which a request
+// per step and workgroup were what a step of 4096 envs waited for.  (All lanes of the wavefront make the calls.)
+struct EpisodeBooks {
+    static constexpr int R = PR16;
+    struct Waiting { float ret[WAVE], len[WAVE]; };
+    float ep_return = 0.0f, ep_length = 0.0f;
+    int waiting = 0;
+    MRL_DEV void begin(const CollectArgs &a, int env, bool mine) {
+        if (mine) {
+            ep_return = a.acc.ep_return[env];
+            ep_length = a.acc.ep_length[env];
+        }
+    }
+    MRL_DEV void list(const CollectArgs &a, const Waiting &w, int lane) {
+        int first = 0;
+        if (lane == 0) first = atomicAdd(a.acc.done_count, waiting);
+        first = __builtin_amdgcn_readfirstlane(first);
+        if (lane < waiting && first + lane < a.acc.done_cap) {
+            a.acc.done_returns[first + lane] = w.ret[lane];
+            a.acc.done_lengths[first + lane] = w.len[lane];
+        }
+        waiting = 0;
+    }
+    MRL_DEV void rewards(const CollectArgs &a, Waiting &w, size_t at, float r, float d, int lane, bool mine) {
+        if (mine) {
+            a.r_rewards[at] = r;
+            a.r_dones[at] = d;
+        }
+        ep_return = ep_return + r;
+        ep_length = ep_length + 1.0f;
+        const bool finished = mine && d > 0.5f;
+        const unsigned long long all = __ballot(finished);
+        if (all == 0) return;
+        if (finished) {
+            const int i = waiting + __popcll(all & ((1ull << lane) - 1));
+            w.ret[i] = ep_return;
+            w.len[i] = ep_length;
+        }
+        ep_return = finished ? 0.0f : ep_return;
+        ep_length = finished ? 0.0f : ep_length;
+        waiting += __popcll(all);
+        if (waiting > WAVE - R) list(a, w, lane);
+    }
+    MRL_DEV void end(const CollectArgs &a, const Waiting &w, int env, int lane, bool mine) {
+        if (waiting > 0) list(a, w, lane);
+        if (mine) {
+            a.acc.ep_return[env] = ep_return;
+            a.acc.ep_length[env] = ep_length;
+        }
+    }
+};
+
+// The same with eight wavefronts, for as many envs as leave every CU one workgroup: nothing shares a SIMD with a second
+// solver then, and what the solver wavefront's chain does not need in turn has wavefronts of its own.  A step is
+//   wavefront 0       actor columns | draw, the lander's push picked | merge, physics, reward | resets
+//             1, 2, 3 actor columns | 1: the rollout row of step k - 1; 2: the numbers of the draw of k + 1; 3: engines | ...
+//             4 .. 7  observations out, contact detection (14 tasks of 16 envs) beside the actor | critic ...
+// The engines (double precision) push the lander in one of four ways: wavefront 3 takes all four, a lane per (env, action),
+// beside the draw.  (Two continuous actions: its lanes take what the engines need whatever the action is.)  The critic runs
+// on wavefronts 5 to 7, at hidden width 256 on 1 to 3 as well: the SIMDs that the solver does not use.  Weights up to width
+// 128 stay in registers (wavefront 0, whose solver wants them: width 64).
+// us per step, four wavefronts : eight: 777 envs, H = 64 11.04 : 9.09, H = 128 13.2 : 10.8, H = 256 18.2 : 15.8; 4096 envs
+// 11.04 : 9.09, 13.3 : 10.9, 18.5 : 16.0; two continuous actions, 777 envs, 13.0 : 11.3, 15.5 : 13.3, 19.9 : 17.0.  Thousand
+// cycles of a step at H = 64 (of 20.9; 25 with four): actor and draw 3.7, wait for detection and engines 1.8, merge, physics
+// and reward 13.1, resets 1.6; at H = 256 (35): actor 13.7, draw and wait 3, physics 13, resets 1.6, wait for the critic 3.5.
+template <class E, int H, int ACT, bool GAUSS>
+__global__ __launch_bounds__(512, 2) void collect16_wide_kernel(CollectArgs a) {
+    using S = Stage<E>;
+    constexpr int IN = E::OBS, AW = E::ACT_W, A = GAUSS ? 2 : 4, R = PR16, T = 512, CAP = 3;
+    constexpr int NTA = H / 64, KB = H <= 128 ? H / 4 : 8, KB0 = H == 64 ? KB : 8;   // (wavefront 0's)
+    constexpr int K0 = IN / 4, TILES = H / 16;
+    constexpr int CW = H == 256 ? 6 : 3;                                             // the critic's wavefronts
+    static_assert(IN % 4 == 0 && E::DETECT_TASKS <= 16, "whole k-steps; detection in one pass of four wavefronts");
+    __shared__ float rows[R * S::STRIDE];
+    __shared__ float xs[R * XS_LD];
+    __shared__ __align__(16) float w2a[HEAD_LDS(H)];
+    __shared__ float w2c[H + 1];
+    __shared__ float logits[R * (PA_MAX + 1)];
+    __shared__ float shapes[E::NSHAPE];
+    __shared__ ll::EngineDraw draws[R];
+    __shared__ ll::Velocity pushes[R][4];
+    __shared__ unsigned long long was_reset;
+    __shared__ unsigned sync_actor, sync_critic, sync_detect, sync_failed, give_up[2];
+    __shared__ float hT[2][H * HT16_LD], h2[2][R * (H + 1)];
+    __shared__ float cts[R * S::CSTRIDE], dlist[detect_list_floats<E, CAP>() + 1];
+    __shared__ int dcount[detect_count_ints<E>()];
+    // of step k at [k & 1]: numbers of the draw (there a step ahead), actions, probabilities / means, rewards, done flags, values
+    __shared__ float numbers[2][R * AW], acts[2][R * AW], chance[2][R * AW], rew[2][R], don[2][R], vals[2][R];
+    __shared__ EpisodeBooks::Waiting finished;
+
+    const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t / WAVE);
+    const int env0 = blockIdx.x * R;
+    const int nenv = min(R, a.n_envs - env0);
+    const int N = a.n_envs;
+    float *gbase = a.states + (size_t)env0 * E::STATE;
+    const size_t row0 = (size_t)a.t0 * N + env0;   // the first step's rollout row
+
+    if (t < E::THREADS) S::in(rows, gbase, nenv, t);
+    for (int i = t; i < E::NSHAPE; i += T) shapes[i] = a.shapes[i];
+    stage_head(a.actor_p + IN * H + H + H * H + H, H, A, GAUSS, w2a, t, T);
+    for (int i = t; i < H + 1; i += T) w2c[i] = a.critic_p[IN * H + H + H * H + H + i];
+    auto make_numbers = [&](int k, int lane) {
+        if (lane >= R * AW) return;
+        const uint32_t seed = a.sample_seed + (uint32_t)k * a.sample_stride;
+        const int i = env0 + lane / AW;
+        numbers[k & 1][lane] = GAUSS ? gaussian_noise(seed, i, A, lane % AW) : categorical_uniform(seed, i);
+    };
+    if (wave == 2) make_numbers(0, t % WAVE);
+    if (t == 0) {
+        was_reset = 0;
+        sync_actor = sync_critic = sync_detect = sync_failed = 0;
+        give_up[0] = give_up[1] = 0;
+    }
+    __syncthreads();
+
+    // Every role counts the same steps, and all meet at the barrier that ends one.  The wavefront-group barriers' counts follow
+    // from the step's number.
+    constexpr unsigned ACTOR_MEETS = H == 256 ? 3 : 2;
+    auto actor_sync = [&](int k) { return WaveGroupSync{&sync_actor, (unsigned)k * 4u * ACTOR_MEETS, 4u, &sync_failed, a.spin_limit}; };
+    auto critic_sync = [&](int k) { return WaveGroupSync{&sync_critic, (unsigned)k * 2u * CW, (unsigned)CW, &sync_failed, a.spin_limit}; };
+    auto detect_sync = [&](int k) { return WaveGroupSync{&sync_detect, (unsigned)k * 5u, 5u, &sync_failed, a.spin_limit}; };
+    // actor: layers on wavefronts 0 .. 3; at width 256 the head as well, into `logits`
+    auto actor = [&](auto &ops, const float *pa, int k, int tid) {
+        const int lane = tid % WAVE, n = lane & 15, g = lane >> 4, c0 = 16 * NTA * (tid / WAVE);
+        float a0[K0];
+#pragma unroll
+        for (int kk = 0; kk < K0; ++kk) a0[kk] = rows[n * S::STRIDE + 4 * kk + g];
+        WaveGroupSync sync = actor_sync(k);
+        hidden16_layer0_of<H, IN, ACT>(a0, hT[0], ops, c0, lane);
+        sync();
+        hidden16_layer1<H, IN, ACT>(pa, hT[0], h2[0], ops, c0, lane, [] {});
+        sync();
+        if constexpr (H == 256) {
+            head16<H>(w2a, A, h2[0], logits, PA_MAX + 1, tid, 4 * WAVE);
+            sync();
+        }
+    };
+    // critic, on the wavefronts m = 0 .. CW - 1 of its own: once the observations are out, which detection's barrier tells
+    auto critic = [&](auto &ops, const float *pc, int k, int m, int c0, int lane) {
+        WaveGroupSync detect = detect_sync(k), sync = critic_sync(k);
+        detect.wait_for(detect.target + detect.nwaves);
+        hidden16_layer0<H, IN, ACT>(xs, hT[1], ops, c0, lane);
+        sync();
+        hidden16_layer1<H, IN, ACT>(pc, hT[1], h2[1], ops, c0, lane, [] {});
+        sync();
+        head16_value<H>(w2c, h2[1], vals[k & 1], m * WAVE + lane, CW * WAVE);
+    };
+    // A wait that gave up voids the workgroup's results: all leave behind the same barrier, which wavefront 0 decides ahead of it.
+    auto step_end = [&](int k) {
+        __syncthreads();
+        return give_up[k & 1] != 0u;
+    };
+
+    if (wave == 0) {
+        const int lane0 = t;
+        int wired = lane0 >> 2 < nenv ? E::lanes_wired(rows + (lane0 >> 2) * S::STRIDE) : 0;
+        Hidden16Operands<H, IN, NTA, KB0> ops;
+        if (H == 64) ops.load(a.actor_p, 0, lane0);
+        const float std = GAUSS && (lane0 & 3) < A ? exp32(gaussian_log_std(w2a[HEAD_LOG_STD(H) + (lane0 & 3)])) : 1.0f;
+        for (int k = 0; k < a.n_steps; ++k) {
+            // (Nothing but the rows is carried from one step to the next: the empty asm keeps what the optimiser derives from
+            // these values out of the registers that the solver needs.)
+            int lane = lane0, ne = __builtin_amdgcn_readfirstlane(nenv), zero = 0;
+            asm volatile("" : "+v"(lane), "+s"(zero), "+s"(ne) : : "memory");
+            const float *pa = a.actor_p + zero;
+            const int e = lane >> 2, l = lane & 3, now = k & 1;
+            float *row = rows + e * S::STRIDE;
+            if (H != 64) ops.load(pa, 0, lane);
+            actor(ops, pa, k, lane);
+            float mine;
+            if constexpr (H == 64) {
+                float out[4];
+                head_row16<H, 4, PA_MAX>(w2a, h2[0], e, l, out);
+                mine = l == 0 ? out[0] : l == 1 ? out[1] : l == 2 ? out[2] : out[3];
+            } else {
+                if (H == 128) {
+                    head16<H>(w2a, A, h2[0], logits, PA_MAX + 1, lane, WAVE);
+                    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");   // (this wavefront's own writes)
+                }
+                mine = logits[e * (PA_MAX + 1) + (l < A ? l : 0)];
+            }
+            WaveGroupSync detect = detect_sync(k);
+            typename E::Carry carry{};
+            const bool first = l == 0 && e < ne;
+            if constexpr (GAUSS) {
+                const float u = mine + std * numbers[now][e * AW + (l < A ? l : 0)];
+                if (l < A) {
+                    acts[now][e * AW + l] = u;
+                    chance[now][e * AW + l] = mine;
+                }
+                const float both[2] = {quad_bcast<0>(u), quad_bcast<1>(u)};
+                detect.wait_for(detect.target + detect.nwaves);
+                if (first) carry = E::step_begin(row, env0 + e, both, shapes, draws + e);
+            } else {
+                float pr;
+                const int sel = sample_categorical_quad(mine, A, numbers[now][e], l, pr);
+                if (l == 0) {
+                    acts[now][e] = (float)sel;
+                    chance[now][e] = pr;
+                }
+                detect.wait_for(detect.target + detect.nwaves);
+                if (first) carry = ll::step_begin_pushed(row, sel, pushes[e][sel]);
+            }
+            float r = 0.0f, d = 0.0f;
+            step_finish_quads<E, CAP>(rows, cts, shapes, dlist, dcount, carry, wired, lane, ne, r, d);
+            const bool over = first && d > 0.5f;
+            if (first) {
+                rew[now][e] = r;
+                don[now][e] = d;
+            }
+            const unsigned long long fin = quad_envs(__ballot(over));
+            wired = ((fin >> e) & 1ull) != 0 ? 1 : wired;
+            reset_rows<E>(rows, &was_reset, fin, a.reset_seed + (uint64_t)k * a.reset_stride, env0, lane);
+            if (lane == 0) give_up[now] = __hip_atomic_load(&sync_failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            if (step_end(k)) break;
+        }
+    } else if (wave < 4) {
+        const int lane0 = t % WAVE;
+        Hidden16Operands<H, IN, NTA, KB> ops;
+        if (H <= 128) ops.load(a.actor_p, 16 * NTA * wave, lane0);
+        EpisodeBooks books;
+        const bool mine = wave == 1 && lane0 < nenv;
+        books.begin(a, env0 + lane0, mine);
+        float log_std[AW], std[AW];
+#pragma unroll
+        for (int j = 0; j < AW; ++j) {
+            log_std[j] = GAUSS ? gaussian_log_std(w2a[HEAD_LOG_STD(H) + j]) : 0.0f;
+            std[j] = GAUSS ? exp32(log_std[j]) : 1.0f;
+        }
+        auto book = [&](int k, int lane) {   // what step k leaves beside the rows
+            const size_t at = row0 + (size_t)k * N + lane;
+            const int q = k & 1, e = lane & (R - 1);
+            if (mine) {
+                float logp = 0.0f;
+#pragma unroll
+                for (int j = 0; j < AW; ++j) {
+                    const float u = acts[q][e * AW + j], c = chance[q][e * AW + j];
+                    a.r_actions[at * AW + j] = u;
+                    if (GAUSS) logp = logp + gaussian_logp(u, c, log_std[j], std[j]);
+                    else logp = log32(c + 1e-8f);
+                }
+                a.r_logp[at] = logp;
+                a.r_values[at] = vals[q][e];
+            }
+            books.rewards(a, finished, at, rew[q][e], don[q][e], lane, mine);
+        };
+        int done = 0;   // steps taken
+        for (int k = 0; k < a.n_steps; ++k) {
+            int lane = lane0, zero = 0;
+            asm volatile("" : "+v"(lane), "+s"(zero) : : "memory");
+            const float *pa = a.actor_p + zero, *pc = a.critic_p + zero;
+            if (H == 256) ops.load(pa, 16 * NTA * wave, lane);
+            actor(ops, pa, k, wave * WAVE + lane);
+            if (wave == 1) {
+                if (k > 0) book(k - 1, lane);
+            } else if (wave == 2) {
+                make_numbers(k + 1, lane);
+            } else {
+                const int e = GAUSS ? lane : lane >> 2;
+                if (e < nenv) {
+                    const float *row = rows + e * S::STRIDE;
+                    if constexpr (GAUSS) draws[e] = ll::engine_draw(row, env0 + e);
+                    else pushes[e][lane & 3] = ll::pushed(row, env0 + e, lane & 3, shapes);
+                }
+                detect_sync(k).arrive();
+            }
+            if constexpr (H == 256) {   // (columns: 1, 2, 1 of the sixteen tiles here, four on each of the others)
+                auto share = [&](auto tiles, int m, int c0) {
+                    Hidden16Operands<H, IN, decltype(tiles)::value, 8> cops;
+                    cops.load(pc, c0, lane);
+                    critic(cops, pc, k, m, c0, lane);
+                };
+                if (wave == 2) share(std::integral_constant<int, 2>{}, 1, 16);
+                else share(std::integral_constant<int, 1>{}, wave - 1, wave == 1 ? 0 : 48);
+            }
+            done = k + 1;
+            if (step_end(k)) break;
+        }
+        if (wave == 1 && sync_failed == 0u) {
+            if (done > 0) book(done - 1, lane0);
+            books.end(a, finished, env0 + lane0, lane0, mine);
+        }
+    } else {
+        const int lane0 = t % WAVE, v = wave - 4;
+        auto helper = [&](auto tiles, int m, int c0) {
+            constexpr int NT = decltype(tiles)::value;
+            Hidden16Operands<H, IN, NT == 0 ? 1 : NT, KB> ops;
+            if (NT > 0 && H <= 128) ops.load(a.critic_p, c0, lane0);
+            for (int k = 0; k < a.n_steps; ++k) {
+                int lane = lane0, ne = __builtin_amdgcn_readfirstlane(nenv), zero = 0;
+                asm volatile("" : "+v"(lane), "+s"(zero), "+s"(ne) : : "memory");
+                const float *pc = a.critic_p + zero;
+                stage_observations<IN, 4 * WAVE>(xs, a.r_obs + (row0 + (size_t)k * N) * IN, ne, v * WAVE + lane,
+                                                 [&](int r, int c) { return rows[r * S::STRIDE + c]; });
+                const int task = 4 * v + lane / R, e = lane % R;
+                if (task < E::DETECT_TASKS && e < ne) detect_vertex_task<E, CAP>(rows, shapes, dlist, dcount, task, e);
+                detect_sync(k).arrive();
+                if constexpr (NT > 0) {
+                    if (H == 256) ops.load(pc, c0, lane);
+                    critic(ops, pc, k, m, c0, lane);
+                }
+                if (step_end(k)) break;
+            }
+        };
+        // (wavefront 4 has the solver's SIMD)
+        constexpr int C0 = H == 256 ? 4 : 0, N0 = (TILES - C0) / 3, N1 = (TILES - C0 - N0) / 2, N2 = TILES - C0 - N0 - N1;
+        static_assert(C0 + N0 + N1 + N2 == TILES, "all of the critic's columns");
+        if (v == 0) helper(std::integral_constant<int, 0>{}, 0, 0);
+        else if (v == 1) helper(std::integral_constant<int, N0>{}, CW - 3, 16 * C0);
+        else if (v == 2) helper(std::integral_constant<int, N1>{}, CW - 2, 16 * (C0 + N0));
+        else helper(std::integral_constant<int, N2>{}, CW - 1, 16 * (C0 + N0 + N1));
+    }
+    __syncthreads();
+    if (sync_failed != 0u) {   // nothing of a workgroup whose wait gave up is stored
+        if (t == 0) *a.sync_error = 1;
+        return;
+    }
+    for (int i = t; i < nenv * E::OBS; i += T) {
+        const int r = i / E::OBS, c = i - r * E::OBS;
+        a.obs[(size_t)env0 * E::OBS + i] = rows[r * S::STRIDE + c];
+    }
+    if (t < E::THREADS) S::out(rows, gbase, nenv, t, 0, E::STATE);
+}
+
 struct PendulumSlot {
     static constexpr int OBS = pendulum::OBS;
     float s[8];
@@ -272,60 +597,6 @@ struct PendulumSlot {
 // 4.25 : 2.12, 5.91 : 4.10, 14.3 : 8.0; width 128, 1024 envs 5.66 : 4.59; width 256 10.5 : 10.4.  Pendulum at 1024 / 8192 /
 // 16384 / 32768 envs 2.77 : 1.86, 3.92 : 3.08, 6.22 : 5.87, 12.0 : 11.4; width 128, 1024 envs 6.36 : 6.07; width 256 11.8 :
 // 11.3.  (From 8192 CartPole and 16384 Pendulum envs on, before, in 32-row workgroups with one env a lane in turn.)
-// Action, reward and done flag of a step into the rollout, and the episode sums, a lane per env of one wavefront.  Finished episodes wait
-// in LDS until some dozens are there: their places in the list come from one counter of the whole chip, at which a request
-// per step and workgroup were what a step of 4096 envs waited for.  (All lanes of the wavefront make the calls.)
-struct EpisodeBooks {
-    static constexpr int R = PR16;
-    struct Waiting { float ret[WAVE], len[WAVE]; };
-    float ep_return = 0.0f, ep_length = 0.0f;
-    int waiting = 0;
-    MRL_DEV void begin(const CollectArgs &a, int env, bool mine) {
-        if (mine) {
-            ep_return = a.acc.ep_return[env];
-            ep_length = a.acc.ep_length[env];
-        }
-    }
-    MRL_DEV void list(const CollectArgs &a, const Waiting &w, int lane) {
-        int first = 0;
-        if (lane == 0) first = atomicAdd(a.acc.done_count, waiting);
-        first = __builtin_amdgcn_readfirstlane(first);
-        if (lane < waiting && first + lane < a.acc.done_cap) {
-            a.acc.done_returns[first + lane] = w.ret[lane];
-            a.acc.done_lengths[first + lane] = w.len[lane];
-        }
-        waiting = 0;
-    }
-    MRL_DEV void rewards(const CollectArgs &a, Waiting &w, size_t at, float action, float r, float d, int lane, bool mine) {
-        if (mine) {
-            a.r_actions[at] = action;
-            a.r_rewards[at] = r;
-            a.r_dones[at] = d;
-        }
-        ep_return = ep_return + r;
-        ep_length = ep_length + 1.0f;
-        const bool finished = mine && d > 0.5f;
-        const unsigned long long all = __ballot(finished);
-        if (all == 0) return;
-        if (finished) {
-            const int i = waiting + __popcll(all & ((1ull << lane) - 1));
-            w.ret[i] = ep_return;
-            w.len[i] = ep_length;
-        }
-        ep_return = finished ? 0.0f : ep_return;
-        ep_length = finished ? 0.0f : ep_length;
-        waiting += __popcll(all);
-        if (waiting > WAVE - R) list(a, w, lane);
-    }
-    MRL_DEV void end(const CollectArgs &a, const Waiting &w, int env, int lane, bool mine) {
-        if (waiting > 0) list(a, w, lane);
-        if (mine) {
-            a.acc.ep_return[env] = ep_return;
-            a.acc.ep_length[env] = ep_length;
-        }
-    }
-};
-
 // What a CartPole workgroup has in LDS beside its nets.  The envs' rows behind the last step, one per action and env: a new
 // episode's where that action ended one.  Of step k, at [k & 1]: the action drawn, its probability, both actions' rewards and
 // done flags; and, there a step ahead, new episodes' rows and the numbers of the draw.
@@ -378,7 +649,8 @@ struct CartPoleRows {
     }
     MRL_DEV void book(EpisodeBooks &b, const CollectArgs &a, EpisodeBooks::Waiting &w, size_t at, int q, int lane, bool mine) const {
         const int e = lane & (R - 1), sel = drawn[q][e];
-        b.rewards(a, w, at, (float)sel, rew[q][sel][e], don[q][sel][e], lane, mine);
+        if (mine) a.r_actions[at] = (float)sel;
+        b.rewards(a, w, at, rew[q][sel][e], don[q][sel][e], lane, mine);
     }
     MRL_DEV void draw(int now, int e, int l, float logit) {
         float pr;
@@ -830,7 +1102,9 @@ __global__ __launch_bounds__(512, 4) void collect_pendulum16_h64_kernel(CollectA
         auto rewards = [&](int k) {
             u = action[q];
             mu = mean[q];
-            books.rewards(a, finished, row0 + (size_t)k * N + lane, u, rew[q], don[q], lane, mine);
+            const size_t at = row0 + (size_t)k * N + lane;
+            if (mine) a.r_actions[at] = u;
+            books.rewards(a, finished, at, rew[q], don[q], lane, mine);
         };
         auto value = [&](int k) {
             float out[1];
@@ -904,8 +1178,13 @@ void launch_pendulum16(mrl_ctx *ctx, dim3 grid, const CollectArgs &a) {
 template <int H, int ACT>
 int launch_collect16_t(mrl_ctx *ctx, const mrl_rollout *r, const CollectArgs &a, int32_t *side) {
     const dim3 grid(grid_for(r->n_envs, PR16)), block(LunarLander::THREADS);
-    if (r->env_id == MRL_ENV_LUNARLANDER)
+    const bool wide = (int)grid.x <= ctx->n_cus;
+    if (r->env_id == MRL_ENV_LUNARLANDER && wide)
+        hipLaunchKernelGGL((collect16_wide_kernel<LunarLander, H, ACT, false>), grid, dim3(512), 0, ctx->stream, a);
+    else if (r->env_id == MRL_ENV_LUNARLANDER)
         hipLaunchKernelGGL((collect16_kernel<LunarLander, H, ACT, false>), grid, block, 0, ctx->stream, a);
+    else if (r->env_id == MRL_ENV_LUNARLANDER_CONTINUOUS && wide)
+        hipLaunchKernelGGL((collect16_wide_kernel<LunarLanderContinuous, H, ACT, true>), grid, dim3(512), 0, ctx->stream, a);
     else if (r->env_id == MRL_ENV_LUNARLANDER_CONTINUOUS)
         hipLaunchKernelGGL((collect16_kernel<LunarLanderContinuous, H, ACT, true>), grid, block, 0, ctx->stream, a);
     else if (r->env_id == MRL_ENV_CARTPOLE)

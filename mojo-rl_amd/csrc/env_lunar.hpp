@@ -263,12 +263,23 @@ MRL_DEV EngineDraw engine_draw(const float *row, int env) {
     return engine_draw(row, env, (int)row[L::META_OFF + META_STEP]);
 }
 
-// given: the step's EngineDraw (null: taken here, if an engine fires)
-MRL_DEV void apply_engines(float *row, int env, int step_count, double m_power, double s_power,
-                           double direction, const EngineDraw *given) {
-    if (m_power == 0.0 && s_power == 0.0) return;
-    float *B = row + L::BODIES_OFF;
-    double vx = B[IDX_VX], vy = B[IDX_VY], omega = B[IDX_OMEGA];
+// the lander's, which is all that wind and engines change
+struct Velocity {
+    float vx, vy, omega;
+    static MRL_DEV Velocity of(const float *row) {
+        const float *B = row + L::BODIES_OFF;
+        return {B[IDX_VX], B[IDX_VY], B[IDX_OMEGA]};
+    }
+    MRL_DEV void to(float *row) const {
+        float *B = row + L::BODIES_OFF;
+        B[IDX_VX] = vx; B[IDX_VY] = vy; B[IDX_OMEGA] = omega;
+    }
+};
+
+// given: the step's EngineDraw (null: taken here)
+MRL_DEV void add_engines(Velocity &v, const float *row, int env, int step_count, double m_power, double s_power,
+                         double direction, const EngineDraw *given) {
+    double vx = v.vx, vy = v.vy, omega = v.omega;
     const EngineDraw draw = given != nullptr ? *given : engine_draw(row, env, step_count);
     const double tip_x = draw.tip_x, tip_y = draw.tip_y, dispersion_x = draw.dispersion_x, dispersion_y = draw.dispersion_y;
     double side_x = -tip_y, side_y = tip_x;
@@ -298,9 +309,15 @@ MRL_DEV void apply_engines(float *row, int env, int step_count, double m_power, 
         double torque = r_x * impulse_y - r_y * impulse_x;
         domega += torque / LANDER_INERTIA;
     }
-    B[IDX_VX] = (float)(vx + dvx);
-    B[IDX_VY] = (float)(vy + dvy);
-    B[IDX_OMEGA] = (float)(omega + domega);
+    v.vx = (float)(vx + dvx);
+    v.vy = (float)(vy + dvy);
+    v.omega = (float)(omega + domega);
+}
+MRL_DEV void apply_engines(float *row, int env, int step_count, double m_power, double s_power, double direction, const EngineDraw *given) {
+    if (m_power == 0.0 && s_power == 0.0) return;
+    Velocity v = Velocity::of(row);
+    add_engines(v, row, env, step_count, m_power, s_power, direction, given);
+    v.to(row);
 }
 
 // An env step in two halves, so that contact detection -- which reads positions only -- can run
@@ -319,18 +336,22 @@ struct StepCarry {
 // otherwise tanh(sin(0.02 t) + sin(pi 0.01 t)) times the power as an impulse on the lander's vx and
 // omega, in Float64, before the engines.  t is the row's step count, as in the GPU trait (:2041-2105):
 // the row has no slot for the CPU env's two running indices.
-MRL_DEV void apply_wind(float *row, int step_count, const float *shapes) {
-    if (!(shapes[WIND_OFF] > 0.5f)) return;
-    if (row[6] > 0.5f || row[7] > 0.5f) return;
+MRL_DEV bool windy(const float *row, const float *shapes) { return shapes[WIND_OFF] > 0.5f && !(row[6] > 0.5f || row[7] > 0.5f); }
+MRL_DEV void add_wind(Velocity &v, int step_count, const float *shapes) {
     const double k = 0.01, t = (double)step_count, pi = 3.14159265358979323846;
     const double wind_mag = ::tanh(::sin(0.02 * t) + ::sin(pi * k * t)) * (double)shapes[WIND_OFF + 1];
     const double torque_mag = ::tanh(::sin(0.02 * t) + ::sin(pi * k * t)) * (double)shapes[WIND_OFF + 2];
-    float *B = row + L::BODIES_OFF;
-    const double vx = (double)B[IDX_VX], omega = (double)B[IDX_OMEGA];
+    const double vx = (double)v.vx, omega = (double)v.omega;
     const double dvx = wind_mag * DT / LANDER_MASS;
     const double domega = torque_mag * DT / LANDER_INERTIA;
-    B[IDX_VX] = (float)(vx + dvx);
-    B[IDX_OMEGA] = (float)(omega + domega);
+    v.vx = (float)(vx + dvx);
+    v.omega = (float)(omega + domega);
+}
+MRL_DEV void apply_wind(float *row, int step_count, const float *shapes) {
+    if (!windy(row, shapes)) return;
+    Velocity v = Velocity::of(row);
+    add_wind(v, step_count, shapes);
+    v.to(row);
 }
 
 // The physics with one lane per body (body_lanes.hpp): lanes 4 e .. 4 e + 3 of a wavefront are the lander, leg 1, leg 2 and
@@ -373,15 +394,38 @@ MRL_DEV void physics_lanes(float *row, float *contacts, int n, int lane) {
     if (has) lane_body_store<L>(B, row, b);
 }
 
-MRL_DEV StepCarry step_begin(float *row, int env, int action, const float *shapes, const EngineDraw *draw = nullptr) {
+// `direction`: of the side engines
+MRL_DEV StepCarry carry_of(const float *row, int action, double &direction) {
     StepCarry c;
     c.skip = row[L::META_OFF + META_DONE] > 0.5f;
     c.step_count = (int)row[L::META_OFF + META_STEP];
     c.m_power = 0.0; c.s_power = 0.0;
-    double direction = 0.0;
+    direction = 0.0;
     if (action == 2) c.m_power = 1.0;
     else if (action == 1) { c.s_power = 1.0; direction = -1.0; }
     else if (action == 3) { c.s_power = 1.0; direction = 1.0; }
+    return c;
+}
+// the lander's velocity with wind and engines
+MRL_DEV Velocity pushed(const float *row, int env, int action, const float *shapes) {
+    double direction;
+    const StepCarry c = carry_of(row, action, direction);
+    Velocity v = Velocity::of(row);
+    if (!c.skip) {
+        if (windy(row, shapes)) add_wind(v, c.step_count, shapes);
+        if (action != 0) add_engines(v, row, env, c.step_count, c.m_power, c.s_power, direction, nullptr);
+    }
+    return v;
+}
+// the rest of step_begin, the push given
+MRL_DEV StepCarry step_begin_pushed(float *row, int action, const Velocity &push) {
+    double direction;
+    push.to(row);
+    return carry_of(row, action, direction);
+}
+MRL_DEV StepCarry step_begin(float *row, int env, int action, const float *shapes, const EngineDraw *draw = nullptr) {
+    double direction;
+    const StepCarry c = carry_of(row, action, direction);
     if (!c.skip) {
         apply_wind(row, c.step_count, shapes);
         apply_engines(row, env, c.step_count, c.m_power, c.s_power, direction, draw);
