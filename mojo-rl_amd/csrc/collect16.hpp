@@ -9,7 +9,7 @@
 #include "policy_sample.hpp"
 #include "env_block.hpp"
 #include "env_classic.hpp"
-#include "collect_args.hpp"
+#include "collect_books.hpp"
 
 namespace mrl {
 
@@ -233,59 +233,6 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
     }
     S::out(rows, gbase, nenv, t, 0, E::STATE);
 }
-
-// Reward and done flag of a step into the rollout, and the episode sums, a lane per env of one wavefront.  Finished episodes wait
-// in LDS until some dozens are there: their places in the list come from one counter of the whole chip, at which a request
-// per step and workgroup were what a step of 4096 envs waited for.  (All lanes of the wavefront make the calls.)
-struct EpisodeBooks {
-    static constexpr int R = PR16;
-    struct Waiting { float ret[WAVE], len[WAVE]; };
-    float ep_return = 0.0f, ep_length = 0.0f;
-    int waiting = 0;
-    MRL_DEV void begin(const CollectArgs &a, int env, bool mine) {
-        if (mine) {
-            ep_return = a.acc.ep_return[env];
-            ep_length = a.acc.ep_length[env];
-        }
-    }
-    MRL_DEV void list(const CollectArgs &a, const Waiting &w, int lane) {
-        int first = 0;
-        if (lane == 0) first = atomicAdd(a.acc.done_count, waiting);
-        first = __builtin_amdgcn_readfirstlane(first);
-        if (lane < waiting && first + lane < a.acc.done_cap) {
-            a.acc.done_returns[first + lane] = w.ret[lane];
-            a.acc.done_lengths[first + lane] = w.len[lane];
-        }
-        waiting = 0;
-    }
-    MRL_DEV void rewards(const CollectArgs &a, Waiting &w, size_t at, float r, float d, int lane, bool mine) {
-        if (mine) {
-            a.r_rewards[at] = r;
-            a.r_dones[at] = d;
-        }
-        ep_return = ep_return + r;
-        ep_length = ep_length + 1.0f;
-        const bool finished = mine && d > 0.5f;
-        const unsigned long long all = __ballot(finished);
-        if (all == 0) return;
-        if (finished) {
-            const int i = waiting + __popcll(all & ((1ull << lane) - 1));
-            w.ret[i] = ep_return;
-            w.len[i] = ep_length;
-        }
-        ep_return = finished ? 0.0f : ep_return;
-        ep_length = finished ? 0.0f : ep_length;
-        waiting += __popcll(all);
-        if (waiting > WAVE - R) list(a, w, lane);
-    }
-    MRL_DEV void end(const CollectArgs &a, const Waiting &w, int env, int lane, bool mine) {
-        if (waiting > 0) list(a, w, lane);
-        if (mine) {
-            a.acc.ep_return[env] = ep_return;
-            a.acc.ep_length[env] = ep_length;
-        }
-    }
-};
 
 // The same with eight wavefronts, for as many envs as leave every CU one workgroup: nothing shares a SIMD with a second
 // solver then, and what the solver wavefront's chain does not need in turn has wavefronts of its own.  A step is

@@ -35,7 +35,7 @@
 #include "env_cheetah_lanes.hpp"
 #include "env_car.hpp"
 #include "env_planar.hpp"
-#include "collect_args.hpp"
+#include "collect_books.hpp"
 
 namespace mrl {
 
@@ -90,33 +90,35 @@ MRL_DEV void policy16_gauss(const CollectArgs &a, ObsAt obs_at, int tid, int ne,
 }
 
 // The actor's half of policy16_gauss by wavefronts 0 .. 3 alone (the observation tile xs is complete, every
-// thread of the four passes its tid): hidden stack on `tile`, Gaussian sampling, rollout row t of action and
-// log-prob; leaves the actions in act[env][AW].  The four wavefronts meet at `sync`, five rounds per call.
+// thread of the four passes its tid): hidden stack on `tile`, the draw from the normal numbers in `b`, which takes the
+// actions.  The four wavefronts meet at `sync`, five rounds per call.
 template <int H, int IN, int AW, int ACT>
-MRL_DEV void actor16_gauss(const CollectArgs &a, int tid, int ne, int A, int zero, size_t row, uint32_t sseed, int env0,
-                           const float *xs, float *tile, const float *w2a, float *logits, float *act, float *part,
-                           WaveGroupSync &sync) {
+MRL_DEV void actor16_gauss(const CollectArgs &a, int tid, int zero, int k, const float *xs, float *tile, const float *w2a,
+                           float *logits, GaussBooks<AW> &b, WaveGroupSync &sync) {
     constexpr int KBA = 8, TA = 4 * WAVE, NT = H / 64;
     const int wave = tid / WAVE, lane = tid % WAVE;
     const float *p = a.actor_p + zero;
     Hidden16Operands<H, IN, NT, KBA> ops;
     ops.load(p, 16 * NT * wave, lane);
     hidden_stack16<H, IN, ACT, NT, KBA, true>(p, xs, tile, tile, ops, 16 * NT * wave, lane, sync);
-    head16<H>(w2a, A, tile, logits, PA_MAX + 1, tid, TA);
+    head16<H>(w2a, AW, tile, logits, PA_MAX + 1, tid, TA);
     sync();   // means complete
-    for (int e = tid; e < ne * A; e += TA) {
-        const int r = e / A, j = e - r * A;
-        float av;
-        part[r * PA_MAX + j] = sample_gaussian_part(logits + r * (PA_MAX + 1) + j, w2a + HEAD_LOG_STD(H) + j, 1, A, j,
-                                                    sseed, env0 + r, &av);
-        act[r * AW + j] = av;
-        a.r_actions[row * AW + e] = av;
-    }
-    sync();   // actions and the log-probability terms complete
-    if (tid < ne) {
-        float logp = 0.0f;
-        for (int j = 0; j < A; ++j) logp = logp + part[tid * PA_MAX + j];
-        a.r_logp[row + tid] = logp;
+    if (tid < PR16 * AW) b.draw(k, tid, logits[tid / AW * (PA_MAX + 1) + tid % AW]);
+    sync();   // actions complete
+}
+// What wavefronts 4 .. 7 do beside it: the normal numbers of step k + 1 (4, 6) and the rollout row of step k - 1 (5).  (The
+// draws took 2.5 thousand cycles of a step between the head and the env step, the episode sums in global memory 1 to 2
+// thousand behind it.  us per step, 4096 envs, H = 64 / 256, in line : here:
+// Hopper 7.65 / 19.4 : 6.41 / 19.0, Walker2d 11.3 / 20.4 : 9.85 / 19.3, BipedalWalker 27.7 / 33.4 : 26.1 / 31.7, HalfCheetah
+// 40.7 / 45.8 : 39.2 / 44.2.)
+template <int AW>
+MRL_DEV void beside_actor16(const CollectArgs &a, int wave, int lane, int k, int env0, int ne, GaussBooks<AW> &b, EpisodeBooks &books) {
+    static_assert(PR16 * AW <= 2 * WAVE, "a lane per env and component");
+    if (wave == 5) {
+        if (k > 0) b.book(books, a, k - 1, env0, lane, lane < ne);
+    } else if (wave != 7) {
+        const int i = (wave == 4 ? 0 : WAVE) + lane;
+        if (i < PR16 * AW) b.make_noise(a, k + 1, env0, i);
     }
 }
 constexpr unsigned ACTOR16_ROUNDS = 5, CRITIC16_ROUNDS = 3;
@@ -148,9 +150,7 @@ __global__ __launch_bounds__(512) void collect_walker_kernel(CollectArgs a) {
     __shared__ __align__(16) float w2a[HEAD_LDS(H)];
     __shared__ float w2c[H + 1];                    // the critic's head: column of H weights, then the bias
     __shared__ float logits[R * (PA_MAX + 1)];
-    __shared__ float vals[R];
-    __shared__ float act[R * PA_MAX];               // [env][AW]
-    __shared__ float part[R * PA_MAX];              // log-probability per (env, component)
+    __shared__ GaussBooks<AW> b;
     __shared__ float shapes[E::NSHAPE];
     __shared__ unsigned long long was_reset;
     __shared__ unsigned sync_actor, sync_critic, sync_failed;   // barriers of the actor's and the critic's wavefronts
@@ -174,6 +174,9 @@ __global__ __launch_bounds__(512) void collect_walker_kernel(CollectArgs a) {
     for (int i = t; i < E::NSHAPE; i += T) shapes[i] = a.shapes[i];
     stage_head(a.actor_p + IN * H + H + H * H + H, H, a.A, true, w2a, t, T);
     for (int i = t; i < H + 1; i += T) w2c[i] = a.critic_p[IN * H + H + H * H + H + i];
+    b.begin(a, a.actor_p + IN * H + H + H * H + H + (H + 1) * AW, env0, t);
+    EpisodeBooks books;   // wavefront 5's
+    books.begin(a, env0 + t - 5 * WAVE, t >= 5 * WAVE && t - 5 * WAVE < nenv);
     if (t == 0) {
         was_reset = 0;
         sync_actor = 0;
@@ -184,10 +187,10 @@ __global__ __launch_bounds__(512) void collect_walker_kernel(CollectArgs a) {
 
     for (int k = 0; k < a.n_steps; ++k) {
         // nothing but the rows is carried from one step to the next (see collect16_kernel)
-        int tid = t, ne = __builtin_amdgcn_readfirstlane(nenv), A = __builtin_amdgcn_readfirstlane(a.A), zero = 0;
-        asm volatile("" : "+v"(tid), "+s"(zero), "+s"(ne), "+s"(A) : : "memory");
+        int tid = t, ne = __builtin_amdgcn_readfirstlane(nenv), zero = 0;
+        asm volatile("" : "+v"(tid), "+s"(zero), "+s"(ne) : : "memory");
+        const int now = k & 1;
         const size_t row = (size_t)(a.t0 + k) * N + env0;   // this block's slice of rollout row t
-        const uint32_t sseed = a.sample_seed + (uint32_t)k * a.sample_stride;
         const uint64_t rseed = a.reset_seed + (uint64_t)k * a.reset_stride;
         const int wave = tid / WAVE, lane = tid % WAVE;
         // The env step keeps wavefronts 0 and 1 busy for most of the step (the solver with one lane per body)
@@ -199,44 +202,42 @@ __global__ __launch_bounds__(512) void collect_walker_kernel(CollectArgs a) {
         __syncthreads();
         if (wave < 4) {
             WaveGroupSync actor_sync{&sync_actor, (unsigned)k * ACTOR16_ROUNDS * 4u, 4u, &sync_failed, a.spin_limit};
-            actor16_gauss<H, IN, AW, ACT>(a, tid, ne, A, zero, row, sseed, env0, xs, overlay, w2a, logits, act, part, actor_sync);
+            actor16_gauss<H, IN, AW, ACT>(a, tid, zero, k, xs, overlay, w2a, logits, b, actor_sync);
+        } else {
+            beside_actor16<AW>(a, wave, lane, k, env0, ne, b, books);
         }
         float *critic_tile = overlay + CRITIC_OFF;   // (above the env step's contact scratch cts)
-        // ---- env step with auto-reset, reward / done into rollout row t, episode accounting
-        Accounting acc = a.acc;
-        acc.r_rewards = a.r_rewards + (size_t)(a.t0 + k) * N;
-        acc.r_dones = a.r_dones + (size_t)(a.t0 + k) * N;
-        acc = acc.at(env0);
+        // ---- env step with auto-reset
         if constexpr (!LANES) {
             // (the critic's tile lies over contact lists that are spent by the time the solver runs)
             auto side = [&](int th) {
-                critic16_side<H, IN, ACT>(a, zero, k, th, xs, critic_tile, w2c, vals, &sync_critic, &sync_failed);
+                critic16_side<H, IN, ACT>(a, zero, k, th, xs, critic_tile, w2c, b.vals[now], &sync_critic, &sync_failed);
             };
-            phys_step_block<E, true>(rows, cts, shapes, dlist, dcount, &was_reset, act, nullptr, nullptr, env0, ne,
-                                     rseed, acc, tid, side);
+            phys_step_block<E, true>(rows, cts, shapes, dlist, dcount, &was_reset, b.act[now], b.rew[now], b.don[now], env0, ne,
+                                     rseed, Accounting{}, tid, side);
         } else {
             // HalfCheetah: eight lanes per env, eight envs per wavefront, on wavefronts 0 and 1; a row
             // whose wiring is not HalfCheetah's own is stepped by lane 0 of its group in the one-lane form
             if (wave < 2) {
-                const int slot = wave * 8 + (lane >> 3), b = lane & 7;
+                const int slot = wave * 8 + (lane >> 3), l = lane & 7;
                 const bool live = slot < ne;
                 float *rowp = rows + slot * S::STRIDE;
                 const int env = env0 + (live ? slot : 0);
-                const float *ap = act + (live ? slot : 0) * AW;
+                const float *ap = b.act[now] + (live ? slot : 0) * AW;
                 const bool ok = live && hc::lanes_row_ok(rowp, shapes);
                 float r = 0.0f, d = 0.0f;
                 if (ok) hc::step_lanes(rowp, shapes, ap, lane, r, d);
-                else if (live && b == 0) hc::step_row(rowp, cts + slot * S::CSTRIDE, shapes, env, ap, r, d);
-                if (live && b == 0) {
-                    account(acc, slot, r, d);
+                else if (live && l == 0) hc::step_row(rowp, cts + slot * S::CSTRIDE, shapes, env, ap, r, d);
+                if (live && l == 0) {
+                    b.rew[now][slot] = r;
+                    b.don[now][slot] = d;
                     if (d > 0.5f) E::reset(rowp, rseed, env);
                 }
             } else {
-                critic16_side<H, IN, ACT>(a, zero, k, tid, xs, critic_tile, w2c, vals, &sync_critic, &sync_failed);
+                critic16_side<H, IN, ACT>(a, zero, k, tid, xs, critic_tile, w2c, b.vals[now], &sync_critic, &sync_failed);
             }
         }
         __syncthreads();   // env step done: the rows hold the next observation
-        if (tid < ne) a.r_values[row + tid] = vals[tid];
         // a wait that gave up: the block's results are void from here on; leave the loop and end normally
         if (sync_failed != 0u) break;
     }
@@ -245,6 +246,11 @@ __global__ __launch_bounds__(512) void collect_walker_kernel(CollectArgs a) {
         // observations are not stored and keep the values from before the launch
         if (t == 0) *a.sync_error = 1;
         return;
+    }
+    if (t / WAVE == 5) {
+        const int lane = t % WAVE;
+        if (a.n_steps > 0) b.book(books, a, a.n_steps - 1, env0, lane, lane < nenv);
+        books.end(a, b.finished, env0 + lane, lane, lane < nenv);
     }
 
     for (int i = t; i < nenv * E::OBS; i += T) {
@@ -353,9 +359,7 @@ __global__ __launch_bounds__(512) void collect_planar_kernel(CollectArgs a) {
     __shared__ __align__(16) float w2a[HEAD_LDS(H)];
     __shared__ float w2c[H + 1];
     __shared__ float logits[R * (PA_MAX + 1)];
-    __shared__ float vals[R];
-    __shared__ float act[R * PA_MAX];
-    __shared__ float part[R * PA_MAX];
+    __shared__ GaussBooks<AW> b;
     __shared__ unsigned sync_actor, sync_critic, sync_failed;
     __shared__ __align__(16) float tiles[2 * H * HT16_LD];
 
@@ -368,6 +372,9 @@ __global__ __launch_bounds__(512) void collect_planar_kernel(CollectArgs a) {
     for (int i = t; i < nenv * (M::STATE / 2); i += T) l2[i] = g2[i];
     stage_head(a.actor_p + IN * H + H + H * H + H, H, a.A, true, w2a, t, T);
     for (int i = t; i < H + 1; i += T) w2c[i] = a.critic_p[IN * H + H + H * H + H + i];
+    b.begin(a, a.actor_p + IN * H + H + H * H + H + (H + 1) * AW, env0, t);
+    EpisodeBooks books;   // wavefront 5's
+    books.begin(a, env0 + t - 5 * WAVE, t >= 5 * WAVE && t - 5 * WAVE < nenv);
     if (t == 0) {
         sync_actor = 0;
         sync_critic = 0;
@@ -377,44 +384,47 @@ __global__ __launch_bounds__(512) void collect_planar_kernel(CollectArgs a) {
 
     for (int k = 0; k < a.n_steps; ++k) {
         // nothing but the rows is carried from one step to the next (see collect16_kernel)
-        int tid = t, ne = __builtin_amdgcn_readfirstlane(nenv), A = __builtin_amdgcn_readfirstlane(a.A), zero = 0;
-        asm volatile("" : "+v"(tid), "+s"(zero), "+s"(ne), "+s"(A) : : "memory");
+        int tid = t, ne = __builtin_amdgcn_readfirstlane(nenv), zero = 0;
+        asm volatile("" : "+v"(tid), "+s"(zero), "+s"(ne) : : "memory");
+        const int now = k & 1;
         const size_t row = (size_t)(a.t0 + k) * N + env0;
-        const uint32_t sseed = a.sample_seed + (uint32_t)k * a.sample_stride;
         const uint64_t rseed = a.reset_seed + (uint64_t)k * a.reset_stride;
         const int wave = tid / WAVE, lane = tid % WAVE;
         stage_observations<IN, T>(xs, a.r_obs + row * IN, ne, tid, [&](int r, int c) { return rows[r * M::STATE + c]; });
         __syncthreads();
         if (wave < 4) {
             WaveGroupSync actor_sync{&sync_actor, (unsigned)k * ACTOR16_ROUNDS * 4u, 4u, &sync_failed, a.spin_limit};
-            actor16_gauss<H, IN, AW, ACT>(a, tid, ne, A, zero, row, sseed, env0, xs, tiles, w2a, logits, act, part, actor_sync);
+            actor16_gauss<H, IN, AW, ACT>(a, tid, zero, k, xs, tiles, w2a, logits, b, actor_sync);
+        } else {
+            beside_actor16<AW>(a, wave, lane, k, env0, ne, b, books);
         }
         if (wave == 0) {
             if (lane < ne) {
-                Accounting acc = a.acc;
-                acc.r_rewards = a.r_rewards + (size_t)(a.t0 + k) * N;
-                acc.r_dones = a.r_dones + (size_t)(a.t0 + k) * N;
-                acc = acc.at(env0);
                 float *rowp = rows + lane * M::STATE;
                 planar::State<M> s;
                 s.load(rowp);
                 float r, d;
-                planar::step<M>(s, act + lane * AW, r, d);
-                account(acc, lane, r, d);
+                planar::step<M>(s, b.act[now] + lane * AW, r, d);
+                b.rew[now][lane] = r;
+                b.don[now][lane] = d;
                 if (d > 0.5f) planar::reset<M>(s, planar::combined_seed(rseed, env0 + lane));
                 s.store(rowp);
             }
         } else {
-            critic16_side<H, IN, ACT>(a, zero, k, tid, xs, tiles + H * HT16_LD, w2c, vals, &sync_critic, &sync_failed);
+            critic16_side<H, IN, ACT>(a, zero, k, tid, xs, tiles + H * HT16_LD, w2c, b.vals[now], &sync_critic, &sync_failed);
         }
         __syncthreads();   // env step done: the rows hold the next observation
-        if (tid < ne) a.r_values[row + tid] = vals[tid];
         if (sync_failed != 0u) break;
     }
     if (sync_failed != 0u) {
         // a wait gave up: the block's rows and observations keep the values from before the launch
         if (t == 0) *a.sync_error = 1;
         return;
+    }
+    if (t / WAVE == 5) {
+        const int lane = t % WAVE;
+        if (a.n_steps > 0) b.book(books, a, a.n_steps - 1, env0, lane, lane < nenv);
+        books.end(a, b.finished, env0 + lane, lane, lane < nenv);
     }
     for (int i = t; i < nenv * IN; i += T) {
         const int r = i / IN, c = i - r * IN;
