@@ -26,6 +26,7 @@
 // the step number), except that the finished-episode list is appended in the order in which blocks
 // get there rather than step by step.
 #pragma once
+#include <type_traits>
 #include "mrl_host.hpp"
 #include "mrl_device.hpp"
 #include "mlp_tile.hpp"
@@ -138,6 +139,29 @@ MRL_DEV void critic16_side(const CollectArgs &a, int zero, int k, int tid, const
     ops.load(p, 16 * NT * g, lane);
     hidden_stack16<H, IN, ACT, NT, KBA, true>(p, xs, tile, tile, ops, 16 * NT * g, lane, sync);
     head16_value<H>(w2c, tile, vals, g * WAVE + lane, 4 * WAVE);
+}
+
+// The same at hidden width 256 where only wavefront 0 has the env step: on six wavefronts, 1 to 3 and 5 to 7, of the other
+// three SIMDs (1, 2, 1 and 4, 4, 4 column tiles).  On two SIMDs the critic is 24 thousand cycles beside a step of 16.  us per
+// step, two SIMDs : three: Hopper 18.2 : 16.0 (256 envs), 19.0 : 17.1 (4096), Walker2d 18.6 : 16.2, 19.3 : 17.4; at width 128,
+// where the step is the longer one or nearly, 10.4 : 10.0 and 12.4 : 12.7, at width 64 6.4 : 6.6 and 9.8 : 9.8.
+template <int H, int IN, int ACT>
+MRL_DEV void critic16_wide(const CollectArgs &a, int zero, int k, int wave, int lane, const float *xs, float *tile, const float *w2c,
+                           float *vals, unsigned *sync_word, unsigned *failed) {
+    static_assert(H == 256, "sixteen column tiles");
+    constexpr unsigned CW = 6;
+    const float *p = a.critic_p + zero;
+    auto share = [&](auto tiles, int m, int c0) {
+        constexpr int NT = decltype(tiles)::value;
+        WaveGroupSync sync{sync_word, (unsigned)k * CRITIC16_ROUNDS * CW, CW, failed, a.spin_limit};
+        Hidden16Operands<H, IN, NT, 8> ops;
+        ops.load(p, c0, lane);
+        hidden_stack16<H, IN, ACT, NT, 8, true>(p, xs, tile, tile, ops, c0, lane, sync);
+        head16_value<H>(w2c, tile, vals, m * WAVE + lane, CW * WAVE);
+    };
+    if (wave > 4) share(std::integral_constant<int, 4>{}, wave - 5, 64 * (wave - 5));
+    else if (wave == 2) share(std::integral_constant<int, 2>{}, 4, 208);
+    else if (wave < 4) share(std::integral_constant<int, 1>{}, wave == 1 ? 3 : 5, wave == 1 ? 192 : 240);
 }
 
 template <class E, int H, int ACT, bool LANES>
@@ -411,7 +435,9 @@ __global__ __launch_bounds__(512) void collect_planar_kernel(CollectArgs a) {
                 s.store(rowp);
             }
         } else {
-            critic16_side<H, IN, ACT>(a, zero, k, tid, xs, tiles + H * HT16_LD, w2c, b.vals[now], &sync_critic, &sync_failed);
+            float *tile = tiles + H * HT16_LD;
+            if constexpr (H == 256) critic16_wide<H, IN, ACT>(a, zero, k, wave, lane, xs, tile, w2c, b.vals[now], &sync_critic, &sync_failed);
+            else critic16_side<H, IN, ACT>(a, zero, k, tid, xs, tile, w2c, b.vals[now], &sync_critic, &sync_failed);
         }
         __syncthreads();   // env step done: the rows hold the next observation
         if (sync_failed != 0u) break;
