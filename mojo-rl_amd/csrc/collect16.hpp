@@ -238,15 +238,19 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
 // solver then, and what the solver wavefront's chain does not need in turn has wavefronts of its own.  A step is
 //   wavefront 0       actor columns | draw, the lander's push picked | merge, physics, reward | resets
 //             1, 2, 3 actor columns | 1: the rollout row of step k - 1; 2: the numbers of the draw of k + 1; 3: engines | ...
-//             4 .. 7  observations out, contact detection (14 tasks of 16 envs) beside the actor | critic ...
+//             4 .. 7  contact detection (14 tasks of 16 envs) beside the actor | critic ...
+// Up to width 128 wavefront 2, which has none of the critic there, also puts the observations out and makes the rows of all envs
+// as if each started again, so that the solver copies one where it used to build it (1.6 thousand cycles a step); at 256 the
+// critic is the longer path already (16.0 : 16.2 us per step with the observations on it).
 // The engines (double precision) push the lander in one of four ways: wavefront 3 takes all four, a lane per (env, action),
 // beside the draw.  (Two continuous actions: its lanes take what the engines need whatever the action is.)  The critic runs
 // on wavefronts 5 to 7, at hidden width 256 on 1 to 3 as well: the SIMDs that the solver does not use.  Weights up to width
 // 128 stay in registers (wavefront 0, whose solver wants them: width 64).
-// us per step, four wavefronts : eight: 777 envs, H = 64 11.04 : 9.09, H = 128 13.2 : 10.8, H = 256 18.2 : 15.8; 4096 envs
-// 11.04 : 9.09, 13.3 : 10.9, 18.5 : 16.0; two continuous actions, 777 envs, 13.0 : 11.3, 15.5 : 13.3, 19.9 : 17.0.  Thousand
-// cycles of a step at H = 64 (of 20.9; 25 with four): actor and draw 3.7, wait for detection and engines 1.8, merge, physics
-// and reward 13.1, resets 1.6; at H = 256 (35): actor 13.7, draw and wait 3, physics 13, resets 1.6, wait for the critic 3.5.
+// us per step, four wavefronts : eight (without those rows): 777 envs, H = 64 11.04 : 8.63 (9.09), H = 128 13.2 : 10.4 (10.8),
+// H = 256 18.2 : 15.8; 4096 envs 11.04 : 8.82 (9.09), 13.3 : 10.5 (10.9), 18.5 : 16.0; two continuous actions, 777 envs, 13.0 :
+// 10.9, 15.5 : 13.0, 19.9 : 17.0.  Thousand cycles of a step at H = 64 (of 20; 25 with four): actor and draw 3.7, wait for
+// detection and engines 1.5, merge, physics and reward 13.1; at H = 256 (35): actor 13.7, draw and wait 3, physics 13, resets
+// 1.6, wait for the critic 3.5.
 template <class E, int H, int ACT, bool GAUSS>
 __global__ __launch_bounds__(512, 2) void collect16_wide_kernel(CollectArgs a) {
     using S = Stage<E>;
@@ -254,6 +258,8 @@ __global__ __launch_bounds__(512, 2) void collect16_wide_kernel(CollectArgs a) {
     constexpr int NTA = H / 64, KB = H <= 128 ? H / 4 : 8, KB0 = H == 64 ? KB : 8;   // (wavefront 0's)
     constexpr int K0 = IN / 4, TILES = H / 16;
     constexpr int CW = H == 256 ? 6 : 3;                                             // the critic's wavefronts
+    constexpr bool FRESH = H <= 128;   // wavefront 2 has time for new episodes' rows (at 256 it has columns of the critic)
+    constexpr unsigned DETECTING = FRESH ? 6 : 5;   // wavefronts 2 (which puts the observations out) .. 7; 3 .. 7
     static_assert(IN % 4 == 0 && E::DETECT_TASKS <= 16, "whole k-steps; detection in one pass of four wavefronts");
     __shared__ float rows[R * S::STRIDE];
     __shared__ float xs[R * XS_LD];
@@ -264,13 +270,14 @@ __global__ __launch_bounds__(512, 2) void collect16_wide_kernel(CollectArgs a) {
     __shared__ ll::EngineDraw draws[R];
     __shared__ ll::Velocity pushes[R][4];
     __shared__ unsigned long long was_reset;
-    __shared__ unsigned sync_actor, sync_critic, sync_detect, sync_failed, give_up[2];
+    __shared__ unsigned sync_actor, sync_critic, sync_detect, sync_fresh, sync_failed, give_up[2];
     __shared__ float hT[2][H * HT16_LD], h2[2][R * (H + 1)];
     __shared__ float cts[R * S::CSTRIDE], dlist[detect_list_floats<E, CAP>() + 1];
     __shared__ int dcount[detect_count_ints<E>()];
     // of step k at [k & 1]: numbers of the draw (there a step ahead), actions, probabilities / means, rewards, done flags, values
     __shared__ float numbers[2][R * AW], acts[2][R * AW], chance[2][R * AW], rew[2][R], don[2][R], vals[2][R];
     __shared__ EpisodeBooks::Waiting finished;
+    __shared__ float fresh[FRESH ? R * S::STRIDE : 1];   // the rows of envs that start again behind this step
 
     const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t / WAVE);
     const int env0 = blockIdx.x * R;
@@ -292,7 +299,7 @@ __global__ __launch_bounds__(512, 2) void collect16_wide_kernel(CollectArgs a) {
     if (wave == 2) make_numbers(0, t % WAVE);
     if (t == 0) {
         was_reset = 0;
-        sync_actor = sync_critic = sync_detect = sync_failed = 0;
+        sync_actor = sync_critic = sync_detect = sync_fresh = sync_failed = 0;
         give_up[0] = give_up[1] = 0;
     }
     __syncthreads();
@@ -302,7 +309,8 @@ __global__ __launch_bounds__(512, 2) void collect16_wide_kernel(CollectArgs a) {
     constexpr unsigned ACTOR_MEETS = H == 256 ? 3 : 2;
     auto actor_sync = [&](int k) { return WaveGroupSync{&sync_actor, (unsigned)k * 4u * ACTOR_MEETS, 4u, &sync_failed, a.spin_limit}; };
     auto critic_sync = [&](int k) { return WaveGroupSync{&sync_critic, (unsigned)k * 2u * CW, (unsigned)CW, &sync_failed, a.spin_limit}; };
-    auto detect_sync = [&](int k) { return WaveGroupSync{&sync_detect, (unsigned)k * 5u, 5u, &sync_failed, a.spin_limit}; };
+    auto detect_sync = [&](int k) { return WaveGroupSync{&sync_detect, (unsigned)k * DETECTING, DETECTING, &sync_failed, a.spin_limit}; };
+    auto fresh_sync = [&](int k) { return WaveGroupSync{&sync_fresh, (unsigned)k, 1u, &sync_failed, a.spin_limit}; };
     // actor: layers on wavefronts 0 .. 3; at width 256 the head as well, into `logits`
     auto actor = [&](auto &ops, const float *pa, int k, int tid) {
         const int lane = tid % WAVE, n = lane & 15, g = lane >> 4, c0 = 16 * NTA * (tid / WAVE);
@@ -394,7 +402,19 @@ __global__ __launch_bounds__(512, 2) void collect16_wide_kernel(CollectArgs a) {
             }
             const unsigned long long fin = quad_envs(__ballot(over));
             wired = ((fin >> e) & 1ull) != 0 ? 1 : wired;
-            reset_rows<E>(rows, &was_reset, fin, a.reset_seed + (uint64_t)k * a.reset_stride, env0, lane);
+            if constexpr (FRESH) {
+                if (fin != 0) {
+                    WaveGroupSync made = fresh_sync(k);
+                    made.wait_for(made.target + made.nwaves);
+                }
+                for (unsigned long long m = fin; m; m &= m - 1) {
+                    const int at = (__ffsll((long long)m) - 1) * S::STRIDE;
+#pragma unroll
+                    for (int c = lane; c < E::STATE; c += WAVE) rows[at + c] = fresh[at + c];
+                }
+            } else {
+                reset_rows<E>(rows, &was_reset, fin, a.reset_seed + (uint64_t)k * a.reset_stride, env0, lane);
+            }
             if (lane == 0) give_up[now] = __hip_atomic_load(&sync_failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             if (step_end(k)) break;
         }
@@ -430,15 +450,26 @@ __global__ __launch_bounds__(512, 2) void collect16_wide_kernel(CollectArgs a) {
         };
         int done = 0;   // steps taken
         for (int k = 0; k < a.n_steps; ++k) {
-            int lane = lane0, zero = 0;
-            asm volatile("" : "+v"(lane), "+s"(zero) : : "memory");
+            int lane = lane0, ne = __builtin_amdgcn_readfirstlane(nenv), zero = 0;
+            asm volatile("" : "+v"(lane), "+s"(zero), "+s"(ne) : : "memory");
             const float *pa = a.actor_p + zero, *pc = a.critic_p + zero;
             if (H == 256) ops.load(pa, 16 * NTA * wave, lane);
             actor(ops, pa, k, wave * WAVE + lane);
             if (wave == 1) {
                 if (k > 0) book(k - 1, lane);
             } else if (wave == 2) {
+                if constexpr (FRESH) {
+                    stage_observations<IN, WAVE>(xs, a.r_obs + (row0 + (size_t)k * N) * IN, ne, lane,
+                                                 [&](int r, int c) { return rows[r * S::STRIDE + c]; });
+                    detect_sync(k).arrive();
+                }
                 make_numbers(k + 1, lane);
+                if constexpr (FRESH) {
+                    const int e = lane >> 2;
+                    const uint64_t seed = a.reset_seed + (uint64_t)k * a.reset_stride;
+                    ll::reset_row_quad(fresh + e * S::STRIDE, ll::combined_seed(seed, env0 + e), lane & 3);
+                    fresh_sync(k).arrive();
+                }
             } else {
                 const int e = GAUSS ? lane : lane >> 2;
                 if (e < nenv) {
@@ -474,8 +505,9 @@ __global__ __launch_bounds__(512, 2) void collect16_wide_kernel(CollectArgs a) {
                 int lane = lane0, ne = __builtin_amdgcn_readfirstlane(nenv), zero = 0;
                 asm volatile("" : "+v"(lane), "+s"(zero), "+s"(ne) : : "memory");
                 const float *pc = a.critic_p + zero;
-                stage_observations<IN, 4 * WAVE>(xs, a.r_obs + (row0 + (size_t)k * N) * IN, ne, v * WAVE + lane,
-                                                 [&](int r, int c) { return rows[r * S::STRIDE + c]; });
+                if constexpr (!FRESH)
+                    stage_observations<IN, 4 * WAVE>(xs, a.r_obs + (row0 + (size_t)k * N) * IN, ne, v * WAVE + lane,
+                                                     [&](int r, int c) { return rows[r * S::STRIDE + c]; });
                 const int task = 4 * v + lane / R, e = lane % R;
                 if (task < E::DETECT_TASKS && e < ne) detect_vertex_task<E, CAP>(rows, shapes, dlist, dcount, task, e);
                 detect_sync(k).arrive();

@@ -184,6 +184,13 @@ MRL_DEV void reset_row(float *row, uint64_t cseed) {
     row[L::META_OFF + META_PREV_SHAPING] = shaping(obs);
 }
 
+// what the lanes of a wavefront have written is there for its others
+MRL_DEV void wave_sync_lanes() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Same row as reset_row, written by the 64 lanes of one wavefront together: the 13 Philox draws,
 // the 11 smoothed heights and the 10 edges each go to their own lane, the row is zero-filled in
 // stripes, and bodies / joints / counters are set by separate lanes.  Every value is computed by
@@ -245,6 +252,74 @@ MRL_DEV void reset_row_wave(float *row, uint64_t cseed, int lane) {
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
+}
+
+// The same row once more, by four neighbouring lanes (l: lane & 3): sixteen rows a wavefront, for a caller that wants them
+// ahead of need.  Every value by the same expressions as in reset_row.
+MRL_DEV void reset_row_quad(float *row, uint64_t cseed, int l) {
+    for (int k = l; k < STATE; k += 4) row[k] = 0.0f;
+    const Uniform4 rv = philox_uniform4(cseed, 0, 0);
+    float mine[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) mine[j] = philox_uniform4(cseed + 1000ull, 0, (uint64_t)(4 * j + l)).v[0];
+    double raw[TERRAIN_CHUNKS + 1];
+    static_assert(TERRAIN_CHUNKS == 11, "twelve draws, three a lane");
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        raw[4 * j] = (double)quad_bcast<0>(mine[j]) * (H_UNITS / 2.0);
+        raw[4 * j + 1] = (double)quad_bcast<1>(mine[j]) * (H_UNITS / 2.0);
+        raw[4 * j + 2] = (double)quad_bcast<2>(mine[j]) * (H_UNITS / 2.0);
+        raw[4 * j + 3] = (double)quad_bcast<3>(mine[j]) * (H_UNITS / 2.0);
+    }
+    auto height = [&](int c) {
+        double a = raw[0], b = raw[0], d = raw[1];
+#pragma unroll
+        for (int k = 1; k < TERRAIN_CHUNKS; ++k) {
+            a = c == k ? raw[k - 1] : a;
+            b = c == k ? raw[k] : b;
+            d = c == k ? raw[k == TERRAIN_CHUNKS - 1 ? k : k + 1] : d;
+        }
+        const float h = (float)((a + b + d) / 3.0);
+        return c >= TERRAIN_CHUNKS / 2 - 2 && c < TERRAIN_CHUNKS / 2 + 3 ? (float)HELIPAD_Y : h;
+    };
+    wave_sync_lanes();
+    const double x_spacing = W_UNITS / (double)(TERRAIN_CHUNKS - 1);
+#pragma unroll 1
+    for (int i = l; i < TERRAIN_CHUNKS - 1; i += 4) {
+        double x0 = 0.0 + (double)i * x_spacing, y0 = (double)height(i);
+        double x1 = 0.0 + (double)(i + 1) * x_spacing, y1 = (double)height(i + 1);
+        double dx = x1 - x0, dy = y1 - y0;
+        double length = ::sqrt(dx * dx + dy * dy);
+        double nx = -dy / length, ny = dx / length;
+        if (ny < 0) { nx = -nx; ny = -ny; }
+        float *E = row + L::EDGES_OFF + i * 6;
+        E[0] = (float)x0; E[1] = (float)y0; E[2] = (float)x1; E[3] = (float)y1;
+        E[4] = (float)nx; E[5] = (float)ny;
+    }
+    const double init_x = HELIPAD_X, init_y = H_UNITS;
+    const double init_vx = (((double)rv.v[0] * 2.0 - 1.0) * 1000.0) * DT / LANDER_MASS;
+    const double init_vy = (((double)rv.v[1] * 2.0 - 1.0) * 1000.0) * DT / LANDER_MASS;
+    const double leg_y = init_y - (10.0 / SCALE) - LEG_DOWN;
+    float *B = row + L::BODIES_OFF, *J = row + L::JOINTS_OFF;
+    if (l < 3)
+        set_body(B + l * BODY_SIZE, l == 0 ? init_x : l == 1 ? init_x - LEG_AWAY : init_x + LEG_AWAY, l == 0 ? init_y : leg_y,
+                 init_vx, init_vy, l == 0 ? LANDER_MASS : LEG_MASS, l == 0 ? LANDER_INERTIA : LEG_INERTIA, l);
+    if (l == 1 || l == 2)
+        set_joint(J + (l - 1) * JOINT_SIZE, l, l == 1 ? -LEG_AWAY : LEG_AWAY, -10.0 / SCALE, 0.0, LEG_H, l == 1 ? 0.4 : -0.9,
+                  l == 1 ? 0.9 : -0.4);
+    if (l == 3) {
+        row[L::EDGE_COUNT_OFF] = (float)(TERRAIN_CHUNKS - 1);
+        row[L::JOINT_COUNT_OFF] = 2.0f;
+    }
+    wave_sync_lanes();
+    if (l == 0) {
+        float obs[8];
+        observe(row, obs);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) row[k] = obs[k];
+        row[L::META_OFF + META_PREV_SHAPING] = shaping(obs);
+    }
+    wave_sync_lanes();
 }
 
 // What the engines need that does not hang on the action: a kernel may work it out on another wavefront.
