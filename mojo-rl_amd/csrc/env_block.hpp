@@ -63,6 +63,7 @@ struct LunarLander {
     static MRL_DEV void reset_wave(float *row, uint64_t seed, int env, int lane) {
         ll::reset_row_wave(row, ll::combined_seed(seed, env), lane);
     }
+    static constexpr bool FRESH_ROWS = false;
     // contact detection runs beside the engines of wavefront 0: every quarter of wavefronts 1 .. 3
     // takes one (body, vertex) pair of the block's 16 envs at a time -- hull 6 vertices, legs 4 each
     static constexpr int DETECT_TASKS = 14, DETECT_WORDS = 0;
@@ -101,6 +102,17 @@ struct LunarLanderContinuous : LunarLander {
     static MRL_DEV Carry step_begin(float *row, int env, const float *a, const float *shapes, const ll::EngineDraw *draw = nullptr) {
         return ll::step_begin_continuous(row, env, a, shapes, draw);
     }
+};
+
+// The stand-alone step of as few envs as leave every CU one workgroup at most, with eight wavefronts: detection takes one pass
+// instead of two, and while wavefront 0 has the physics another makes the rows of all envs as if each started again, so
+// that one that does is copied instead of built behind the step (6 to 8 thousand cycles, which the launch waits for where
+// any of its envs finishes).  us per step with auto-reset, four : eight wavefronts, at 64 / 1000 / 4096 envs: 14.8 : 12.6,
+// 19.1 : 15.6, 20.3 : 16.6; two continuous actions 14.0 : 12.0, 17.5 : 14.6, 18.8 : 15.7.
+template <class E>
+struct WideLunar : E {
+    static constexpr int THREADS = 512;
+    static constexpr bool FRESH_ROWS = true;
 };
 
 struct BipedalWalker {
@@ -459,6 +471,7 @@ struct NoSideJob {
 // ([nenv][ACT_W], global or LDS), rewards / dones = the block's slice of the per-step outputs
 // (may be null), acc = rollout accounting with its pointers already offset to the block's first
 // env.  AUTORESET: rows that finished are re-initialised in place and recorded in *was_reset.
+// fresh (E::FRESH_ROWS): room for as many rows as `rows` has.
 // `side`: work of the caller's that the wavefronts without a part in the one-lane-per-body solver (LANES_PHYSICS
 // envs: wavefronts 2 and up) do while wavefronts 0 and 1 run it, called as side(tid) between the two block
 // barriers around the solver; it must not touch the rows or the contact scratch `cts`.
@@ -466,7 +479,7 @@ template <class E, bool AUTORESET, class Side = NoSideJob>
 MRL_DEV void phys_step_block(float *rows, float *cts, const float *shapes, float *dlist, int *dcount,
                              unsigned long long *was_reset, const float *actions, float *rewards,
                              float *dones, int env0, int nenv, uint64_t reset_seed, const Accounting &acc,
-                             int tid = threadIdx.x, Side side = Side{}) {
+                             int tid = threadIdx.x, Side side = Side{}, float *fresh = nullptr) {
     using S = Stage<E>;
     if constexpr (E::DETECT_TASKS > 0 && E::POST_TASKS == 0) {
         // wavefront 0: first half of the step (reads and writes velocities only); the halves of the
@@ -508,8 +521,18 @@ MRL_DEV void phys_step_block(float *rows, float *cts, const float *shapes, float
                 finished = d > 0.5f;
             }
             if (AUTORESET) {
-                const unsigned long long fin = __ballot(finished);
-                reset_rows<E>(rows, was_reset, quad_envs(fin), reset_seed, env0, lane);
+                const unsigned long long fin = quad_envs(__ballot(finished));
+                if constexpr (!E::FRESH_ROWS) reset_rows<E>(rows, was_reset, fin, reset_seed, env0, lane);
+                else if (lane == 0) *was_reset = fin;
+            }
+        }
+        if constexpr (AUTORESET && E::FRESH_ROWS) {
+            if (wave == 4) ll::reset_row_quad(fresh + slot * S::STRIDE, ll::combined_seed(reset_seed, env0 + slot), lane & 3);
+            __syncthreads();
+            const unsigned long long fin = *was_reset;
+            for (unsigned long long m = fin; m; m &= m - 1) {
+                const int at = (__ffsll((long long)m) - 1) * S::STRIDE;
+                if (tid < E::STATE) rows[at + tid] = fresh[at + tid];
             }
         }
     } else {

@@ -99,6 +99,12 @@ __global__ __launch_bounds__(256) void pendulum_reset_kernel(float *states, floa
     if (selective) dones[i] = 0.0f;
 }
 
+template <class E>
+constexpr bool has_fresh_rows() {
+    if constexpr (E::DETECT_TASKS > 0 && E::POST_TASKS == 0) return E::FRESH_ROWS;
+    else return false;
+}
+
 // AUTORESET = false: step_kernel_gpu of the trait.  AUTORESET = true: step, then rows that
 // finished are re-initialised in place (selective reset) before the observation is copied out.
 template <class E, bool AUTORESET>
@@ -112,6 +118,7 @@ __device__ __forceinline__ void phys_step_body(float *states, const float *actio
     __shared__ unsigned long long was_reset;   // rows re-initialised by this launch, one bit each
     __shared__ float dlist[detect_list_floats<E>() + 1];
     __shared__ int dcount[detect_count_ints<E>()];
+    __shared__ float fresh[AUTORESET && has_fresh_rows<E>() ? E::EPB * S::STRIDE : 1];
     const int tid = threadIdx.x;
     const int env0 = blockIdx.x * E::EPB;
     const int nenv = min(E::EPB, batch - env0);
@@ -124,7 +131,7 @@ __device__ __forceinline__ void phys_step_body(float *states, const float *actio
 
     phys_step_block<E, AUTORESET>(rows, cts, shapes, dlist, dcount, &was_reset,
                                   actions + (size_t)env0 * E::ACT_W, rewards + env0, dones + env0, env0, nenv,
-                                  reset_seed, acc.at(env0));
+                                  reset_seed, acc.at(env0), tid, NoSideJob{}, fresh);
     __syncthreads();
 
     for (int i = tid; i < nenv * E::OBS; i += E::THREADS) {   // observation out: [nenv, OBS] contiguous
@@ -381,6 +388,10 @@ static int launch_phys_step(mrl_ctx *ctx, int batch, float *states, const float 
                             float *dones, float *obs, const float *shapes, bool autoreset,
                             uint64_t reset_seed, const Accounting &acc) {
     if constexpr (E::LANE_FROM > 0) {
+        if constexpr (!E::FRESH_ROWS) {
+            if (grid_for(batch, E::EPB) <= ctx->n_cus)
+                return launch_phys_step<WideLunar<E>>(ctx, batch, states, actions, rewards, dones, obs, shapes, autoreset, reset_seed, acc);
+        }
         if (batch >= E::LANE_FROM) {
             dim3 grid64(grid_for(batch, WAVE));
             if (autoreset)
