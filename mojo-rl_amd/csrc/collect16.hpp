@@ -16,8 +16,7 @@ namespace mrl {
 template <int A, int B>
 constexpr int cmax() { return A > B ? A : B; }
 
-// column tiles of 16 of the critic on the three helpers: helper 0, which draws the action once more, never more than the
-// others
+// column tiles of 16 of the critic on the three helpers: helper 0, which writes the rollout row, never more than the others
 template <int H>
 struct Critic16Split {
     static constexpr int TILES = H / 16;
@@ -29,9 +28,10 @@ struct Critic16Split {
 // step on ONE wavefront's vector unit --, and beside it the critic, whose value is only stored.
 //   all four wavefronts     actor  OBS -> H -> H -> A, 64 columns each;
 //   the solver wavefront    sampling (four lanes per env), two of the fourteen detection tasks, env step (four lanes per
-//                           env, one per body: env_lunar.hpp), accounting, resets;
-//   the other three         contact detection, what the engines need whatever the action is, the action's log-probability,
-//                           then the critic (H = 256: 80 / 96 / 80 columns) at a barrier of their own.
+//                           env, one per body: env_lunar.hpp), resets;
+//   the other three         contact detection, what the engines need whatever the action is, the rollout row of step k - 1 and
+//                           the draw's numbers of step k + 1, then the critic (H = 256: 80 / 96 / 80 columns) at a barrier
+//                           of their own.
 // Two such workgroups fit a CU (LDS, registers).  On this hardware a SIMD issues either a matrix or a vector instruction,
 // never both at once (a wavefront of dependent v_fma_f32 that shares its SIMD with a wavefront issuing v_mfma back to back
 // takes the sum of both times), so at H = 256 the second one costs what its forward passes cost (4096 : 8192 envs 18.5 :
@@ -41,7 +41,11 @@ struct Critic16Split {
 // physics before); 4096 envs, H = 64 18.8 : 12.6, H = 256, where the critic is the longer path, 23.9 : 21.6.  The engines'
 // sines and the log-probability off the solver, its detection in one pass of all four wavefronts: H = 64, 777 envs
 // 11.46 : 11.26, 4096 envs 11.86 : 11.55 (11.2 since a step's first loads are no longer waited for; thousand cycles of a
-// step there: actor 5.0, sample 1.1, detection 3.5, wait 0.8, engines 1.6, physics and tail 12, reset 1).
+// step there: actor 5.0, sample 1.1, detection 3.5, wait 0.8, engines 1.6, physics and tail 12, reset 1).  Numbers of the draw a
+// step ahead, rollout rows and episode sums a step later, at 8192 envs, H = 64 / 128 / 256: 12.2 / 16.2 / 27.6 : 12.1 / 15.9 /
+// 27.3, two continuous actions 14.8 / 19.2 / 30.4 : 14.7 / 18.7 / 29.8.  (32 envs a workgroup of eight wavefronts, a weight operand
+// for two row tiles, H = 256: 27.2 at 8192 envs, but 27.0 : 26.1 at 4097 and 53.6 : 44.7 at 9001: matrix and vector time of a
+// SIMD add up either way.)
 // The solver wavefront is 0 in the lower half of the grid and 2 in the upper half: workgroups i and
 // i + grid / 2 share a CU when the grid is twice the CU count, and their solvers then sit on
 // different SIMDs.
@@ -59,8 +63,9 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
     __shared__ __align__(16) float w2a[HEAD_LDS(H)];
     __shared__ float w2c[H + 1];                    // the critic's head: column of H weights, then the bias
     __shared__ float logits[R * (PA_MAX + 1)];
-    __shared__ float vals[R];
-    __shared__ float act[R * PA_MAX];
+    // of step k at [k & 1]: numbers of the draw (there a step ahead), actions, probabilities / means, rewards, done flags, values
+    __shared__ float numbers[2][R * AW], acts[2][R * AW], chance[2][R * AW], rew[2][R], don[2][R], vals[2][R];
+    __shared__ EpisodeBooks::Waiting listed;
     __shared__ float shapes[E::NSHAPE];
     __shared__ ll::EngineDraw draws[R];
     __shared__ unsigned long long was_reset;
@@ -90,13 +95,43 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
         sync_detect = 0;
         sync_failed = 0;
     }
+    auto make_numbers = [&](int k, int lane) {
+        if (lane >= R * AW) return;
+        const uint32_t seed = a.sample_seed + (uint32_t)k * a.sample_stride;
+        const int i = env0 + lane / AW;
+        numbers[k & 1][lane] = GAUSS ? gaussian_noise(seed, i, a.A, lane % AW) : categorical_uniform(seed, i);
+    };
+    if (t >= T - WAVE) make_numbers(0, t - (T - WAVE));
     __syncthreads();
-    // solver wavefront, four lanes per env: the env's running episode return and length stay in registers of the first,
-    // and what its wiring is (E::lanes_wired) in all four
+    // the first helper keeps the episode sums, a lane per env
+    const int t_books = t - WAVE * ((sw + 1) & 3);
+    EpisodeBooks books;
+    books.begin(a, env0 + t_books, t_books >= 0 && t_books < nenv);
+    auto book = [&](int k, int lane, int ne) {   // what step k leaves beside the rows
+        const size_t at = (size_t)(a.t0 + k) * N + env0 + lane;
+        const int q = k & 1, e = lane & (R - 1);
+        const bool mine = lane < ne;
+        if (mine) {
+            float logp = 0.0f;
+#pragma unroll
+            for (int j = 0; j < AW; ++j) {
+                const float u = acts[q][e * AW + j], c = chance[q][e * AW + j];
+                a.r_actions[at * AW + j] = u;
+                if (GAUSS) {
+                    const float log_std = gaussian_log_std(w2a[HEAD_LOG_STD(H) + j]);
+                    logp = logp + gaussian_logp(u, c, log_std, exp32(log_std));
+                } else {
+                    logp = log32(c + 1e-8f);
+                }
+            }
+            a.r_logp[at] = logp;
+            a.r_values[at] = vals[q][e];
+        }
+        books.rewards(a, listed, at, rew[q][e], don[q][e], lane, mine);
+    };
+    // solver wavefront, four lanes per env: what the env's wiring is (E::lanes_wired) in all four
     const int my_env = (t & 63) >> 2;
-    const bool owner = (t >> 6) == sw && my_env < nenv && (t & 3) == 0;
-    float ep_return = owner ? a.acc.ep_return[env0 + my_env] : 0.0f;
-    float ep_length = owner ? a.acc.ep_length[env0 + my_env] : 0.0f;
+    const float my_std = GAUSS && (t & 3) < AW ? exp32(gaussian_log_std(w2a[HEAD_LOG_STD(H) + (t & 3)])) : 1.0f;
     int wired = my_env < nenv ? E::lanes_wired(rows + my_env * S::STRIDE) : 0;
 
     for (int k = 0; k < a.n_steps; ++k) {
@@ -108,7 +143,6 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
         asm volatile("" : "+v"(tid), "+s"(zero), "+s"(ne), "+s"(A) : : "memory");
         const float *pa = a.actor_p + zero, *pc = a.critic_p + zero;
         const size_t row = (size_t)(a.t0 + k) * N + env0;   // this block's slice of rollout row t
-        const uint32_t sseed = a.sample_seed + (uint32_t)k * a.sample_stride;
         const int wave = tid / WAVE, lane = tid % WAVE;
         const int vw = (wave - sw) & 3;                     // 0: solver, 1 .. 3: helpers
         // the helpers' barriers, rebuilt every step from the step number (the critic's hidden stack meets
@@ -126,21 +160,25 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
             head16<H>(w2a, A, overlay, logits, PA_MAX + 1, tid, T);
             __syncthreads();   // logits complete; the actor's tile is dead from here on
         }
-        if (vw == 0) {   // ---- sample
-            const int e = lane >> 2;
-            const bool first = (lane & 3) == 0;
-            if (e < ne) {
-                const int i = env0 + e;
-                const float *lg = logits + e * (PA_MAX + 1);
-                if (GAUSS) {
-                    for (int j = lane & 3; j < A; j += 4) {   // (one component a lane)
-                        float av;
-                        sample_gaussian_part(lg + j, w2a + HEAD_LOG_STD(H) + j, 1, A, j, sseed, i, &av);
-                        act[e * AW + j] = av;
-                    }
-                } else {   // (four actions: the entry refuses any other head)
-                    const int sel = sample_categorical_quad(lg, A, sseed, i, lane & 3);
-                    if (first) act[e] = (float)sel;
+        const int now = k & 1;
+        float drawn[2] = {0.0f, 0.0f};
+        if (vw == 0) {   // ---- draw
+            const int e = lane >> 2, l = lane & 3;
+            const float logit = logits[e * (PA_MAX + 1) + (l < A ? l : 0)];
+            if (GAUSS) {   // (one component a lane)
+                const float u = logit + my_std * numbers[now][e * AW + (l < AW ? l : 0)];
+                if (l < AW) {
+                    acts[now][e * AW + l] = u;
+                    chance[now][e * AW + l] = logit;
+                }
+                drawn[0] = quad_bcast<0>(u);
+                drawn[1] = quad_bcast<1>(u);
+            } else {   // (four actions: the entry refuses any other head)
+                float pr;
+                drawn[0] = (float)sample_categorical_quad(logit, A, numbers[now][e], l, pr);
+                if (l == 0) {
+                    acts[now][e] = drawn[0];
+                    chance[now][e] = pr;
                 }
             }
         } else if (vw == 3 && lane < ne) {   // ---- what the engines need whatever the action is
@@ -157,48 +195,22 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
             const bool first = (lane & 3) == 0 && e < ne;
             detect_sync.target += detect_sync.nwaves;
             detect_sync.wait_for(detect_sync.target);
-            if (first) carry = E::step_begin(rows + e * S::STRIDE, env0 + e, act + e * AW, shapes, draws + e);
+            if (first) carry = E::step_begin(rows + e * S::STRIDE, env0 + e, drawn, shapes, draws + e);
             float r = 0.0f, d = 0.0f;
             step_finish_quads<E, CAP>(rows, cts, shapes, dlist, dcount, carry, wired, lane, ne, r, d);
-            bool finished = false;
             if (first) {
-                a.r_rewards[row + e] = r;
-                a.r_dones[row + e] = d;
-                ep_return = ep_return + r;
-                ep_length = ep_length + 1.0f;
-                finished = d > 0.5f;
-                if (finished) {
-                    const int slot = atomicAdd(a.acc.done_count, 1);
-                    if (slot < a.acc.done_cap) {
-                        a.acc.done_returns[slot] = ep_return;
-                        a.acc.done_lengths[slot] = ep_length;
-                    }
-                    ep_return = 0.0f;
-                    ep_length = 0.0f;
-                }
+                rew[now][e] = r;
+                don[now][e] = d;
             }
+            const bool finished = first && d > 0.5f;
             const unsigned long long fin = quad_envs(__ballot(finished));
             wired = ((fin >> e) & 1ull) != 0 ? 1 : wired;
             reset_rows<E>(rows, &was_reset, fin, a.reset_seed + (uint64_t)k * a.reset_stride, env0, lane);
         } else {
-            // ---- the draw once more, for the rollout's action and log-probability, which nothing of the step waits for
             const int m = vw - 1;
             detect_sync.arrive();
-            if (m == 0 && lane < ne) {
-                const int i = env0 + lane;
-                const float *lg = logits + lane * (PA_MAX + 1);
-                float logp;
-                if (GAUSS) {
-                    float av[PA_MAX];
-                    logp = sample_gaussian(lg, w2a + HEAD_LOG_STD(H), A, sseed, i, av);
-                    for (int j = 0; j < A; ++j) a.r_actions[(row + lane) * AW + j] = av[j];
-                } else {
-                    int sel;
-                    sample_categorical_few(lg, A, sseed, i, sel, logp);
-                    a.r_actions[row + lane] = (float)sel;
-                }
-                a.r_logp[row + lane] = logp;
-            }
+            if (m == 0 && k > 0) book(k - 1, lane, ne);
+            if (m == 1) make_numbers(k + 1, lane);
             // ---- critic on the three helpers, at their own barrier
             const int tl = m * WAVE + lane;
             auto critic = [&](auto tiles, int c0) {
@@ -210,10 +222,9 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
             if (m == 1) critic(std::integral_constant<int, CS.N1>{}, 16 * CS.N0);
             else if (m == 0) critic(std::integral_constant<int, CS.N0>{}, 0);
             else critic(std::integral_constant<int, CS.N2>{}, 16 * (CS.N0 + CS.N1));
-            head16_value<H>(w2c, hTc, vals, tl, 3 * WAVE);
+            head16_value<H>(w2c, hTc, vals[now], tl, 3 * WAVE);
         }
         __syncthreads();   // env step done, values complete
-        if (tid < ne) a.r_values[row + tid] = vals[tid];
         // a wait that gave up: the block's results are void from here on; leave the loop (every
         // thread reads the same word after the barrier) and end normally
         if (sync_failed != 0u) break;
@@ -223,9 +234,9 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
         return;
     }
 
-    if (owner) {
-        a.acc.ep_return[env0 + my_env] = ep_return;
-        a.acc.ep_length[env0 + my_env] = ep_length;
+    if (t_books >= 0 && t_books < WAVE) {
+        if (a.n_steps > 0) book(a.n_steps - 1, t_books, nenv);
+        books.end(a, listed, env0 + t_books, t_books, t_books < nenv);
     }
     for (int i = t; i < nenv * E::OBS; i += T) {
         const int r = i / E::OBS, c = i - r * E::OBS;
