@@ -93,15 +93,15 @@ MRL_DEV void policy16_gauss(const CollectArgs &a, ObsAt obs_at, int tid, int ne,
 // The actor's half of policy16_gauss by wavefronts 0 .. 3 alone (the observation tile xs is complete, every
 // thread of the four passes its tid): hidden stack on `tile`, the draw from the normal numbers in `b`, which takes the
 // actions.  The four wavefronts meet at `sync`, five rounds per call.
-template <int H, int IN, int AW, int ACT>
+// KB = H / 4: the weights are in `ops` already, for the whole launch.
+template <int H, int IN, int AW, int ACT, int KB>
 MRL_DEV void actor16_gauss(const CollectArgs &a, int tid, int zero, int k, const float *xs, float *tile, const float *w2a,
-                           float *logits, GaussBooks<AW> &b, WaveGroupSync &sync) {
-    constexpr int KBA = 8, TA = 4 * WAVE, NT = H / 64;
+                           float *logits, GaussBooks<AW> &b, Hidden16Operands<H, IN, H / 64, KB> &ops, WaveGroupSync &sync) {
+    constexpr int TA = 4 * WAVE, NT = H / 64;
     const int wave = tid / WAVE, lane = tid % WAVE;
     const float *p = a.actor_p + zero;
-    Hidden16Operands<H, IN, NT, KBA> ops;
-    ops.load(p, 16 * NT * wave, lane);
-    hidden_stack16<H, IN, ACT, NT, KBA, true>(p, xs, tile, tile, ops, 16 * NT * wave, lane, sync);
+    if (4 * KB < H) ops.load(p, 16 * NT * wave, lane);
+    hidden_stack16<H, IN, ACT, NT, KB, true>(p, xs, tile, tile, ops, 16 * NT * wave, lane, sync);
     head16<H>(w2a, AW, tile, logits, PA_MAX + 1, tid, TA);
     sync();   // means complete
     if (tid < PR16 * AW) b.draw(k, tid, logits[tid / AW * (PA_MAX + 1) + tid % AW]);
@@ -226,7 +226,8 @@ __global__ __launch_bounds__(512) void collect_walker_kernel(CollectArgs a) {
         __syncthreads();
         if (wave < 4) {
             WaveGroupSync actor_sync{&sync_actor, (unsigned)k * ACTOR16_ROUNDS * 4u, 4u, &sync_failed, a.spin_limit};
-            actor16_gauss<H, IN, AW, ACT>(a, tid, zero, k, xs, overlay, w2a, logits, b, actor_sync);
+            Hidden16Operands<H, IN, H / 64, 8> ops;
+            actor16_gauss<H, IN, AW, ACT>(a, tid, zero, k, xs, overlay, w2a, logits, b, ops, actor_sync);
         } else {
             beside_actor16<AW>(a, wave, lane, k, env0, ne, b, books);
         }
@@ -376,6 +377,9 @@ __global__ __launch_bounds__(512) void collect_car_kernel(CollectArgs a) {
 // finished rows in place, while the critic runs beside them on wavefronts 2, 3, 6 and 7.
 template <class M, int H, int ACT>
 __global__ __launch_bounds__(512) void collect_planar_kernel(CollectArgs a) {
+    // Widths up to which the actor's weights stay in registers.  Hopper's two workgroups a CU want no more than 128 of them.
+    // us per step, 4096 envs, loaded every step : held: Hopper, width 64, 6.41 : 6.32, Walker2d, 64 / 128, 9.85 / 12.4 : 9.61 / 11.8.
+    constexpr int HELD = M::STATE == planar::Hopper::STATE ? 64 : 128;
     constexpr int IN = M::OBS, AW = M::ACT, R = PR16, T = 512;
     static_assert(IN <= PIN_MAX && AW <= PA_MAX && M::STATE % 2 == 0, "tile limits; rows are whole doubles");
     __shared__ __align__(16) float rows[R * M::STATE];
@@ -397,6 +401,9 @@ __global__ __launch_bounds__(512) void collect_planar_kernel(CollectArgs a) {
     stage_head(a.actor_p + IN * H + H + H * H + H, H, a.A, true, w2a, t, T);
     for (int i = t; i < H + 1; i += T) w2c[i] = a.critic_p[IN * H + H + H * H + H + i];
     b.begin(a, a.actor_p + IN * H + H + H * H + H + (H + 1) * AW, env0, t);
+    constexpr int KB = H <= HELD ? H / 4 : 8;   // k-steps of the actor's layer 1 held (all of them, or the next block)
+    Hidden16Operands<H, IN, H / 64, KB> ops;
+    if (4 * KB == H && t < 4 * WAVE) ops.load(a.actor_p, 16 * (H / 64) * (t / WAVE), t % WAVE);
     EpisodeBooks books;   // wavefront 5's
     books.begin(a, env0 + t - 5 * WAVE, t >= 5 * WAVE && t - 5 * WAVE < nenv);
     if (t == 0) {
@@ -418,7 +425,7 @@ __global__ __launch_bounds__(512) void collect_planar_kernel(CollectArgs a) {
         __syncthreads();
         if (wave < 4) {
             WaveGroupSync actor_sync{&sync_actor, (unsigned)k * ACTOR16_ROUNDS * 4u, 4u, &sync_failed, a.spin_limit};
-            actor16_gauss<H, IN, AW, ACT>(a, tid, zero, k, xs, tiles, w2a, logits, b, actor_sync);
+            actor16_gauss<H, IN, AW, ACT>(a, tid, zero, k, xs, tiles, w2a, logits, b, ops, actor_sync);
         } else {
             beside_actor16<AW>(a, wave, lane, k, env0, ne, b, books);
         }

@@ -194,7 +194,7 @@ MRL_DEV float div_by(float x, float d, float r) {
 // tiny x, and 1 - y^2 in the backward pass inherits it.
 MRL_DEV float tanh_mlp(float x) {
     const float e = __builtin_amdgcn_exp2f(x * 2.8853900817779268f);   // 2 log2(e)
-    const float big = 1.0f - 2.0f * __builtin_amdgcn_rcpf(e + 1.0f);
+    const float big = fmaf(-2.0f, __builtin_amdgcn_rcpf(e + 1.0f), 1.0f);   // (twice a float is exact: one rounding either way)
     const float x2 = x * x;
     const float small = x * fmaf(x2, fmaf(x2, 0.13333333333333333f, -0.33333333333333333f), 1.0f);
     return fabsf(x) < 0.125f ? small : big;
