@@ -79,13 +79,15 @@ static CollectPlan collect_plan(const mrl_rollout *r, int n_cus) {
         // Up to this many envs per CU the walkers' fused kernels are the faster way; with more, their 16-env workgroups
         // come round after round while the stand-alone kernels fill the chip.  us per step, fused against two launches,
         // hidden width 64 / 256:
-        //   HalfCheetah (one workgroup per CU)  4096 envs 40 / 45 : 49 / 63,  8192 envs 80 / 90 : 50 / 75;
-        //   Walker2d  4096 envs 12.4 / 22.3 : 17.7 / 31.7,  4200 envs 24.0 / 43.8 : 22.6 / 47.5,  8192 envs 24.4 / 44.0 : 19.9 / 44.5
-        //     (width 128 27.7 : 27.4),  16384 envs 47 / 87 : 31 / 76;
+        //   HalfCheetah (one workgroup per CU)  4096 envs 39 / 44 : 49 / 63,  8192 envs 78 / 88 : 49 / 75;
+        //   Walker2d  4096 envs 9.2 / 16.2 : 17.3 / 31.7,  4200 envs 18.3 / 32.1 : 21.8 / 47.7,  8192 envs 18.4 / 32.3 : 19.2 / 44.7
+        //     (width 128 22.6 : 27.2),  16384 envs 37 / 64 : 31 / 76 (128 45 : 36);
         //   CarRacing  4096 envs 20 / 31 : 28 / 41,  8192 envs 39 / 61 : 41 / 65,  16384 envs 76 / 121 : 72 / 116;
-        //   Hopper  8192 envs 9.6 / 36 : 15.3 / 39,  16384 envs 22 / 70 : 26 / 69,  32768 envs 38 / 138 : 36 / 129;
-        //   BipedalWalker  4096 envs 28 / 34 : 39 / 53,  8192 envs 56 / 66 : 67 / 91,  12288 envs 83 / 99 : 83 / 127,
-        //     16384 envs 110 / 132 : 90 / 133.
+        //   Hopper  8192 envs 6.9 / 27 : 14.3 / 39,  16384 envs 19.5 / 54 : 25 / 68,  32768 envs 33 / 107 : 35 / 126;
+        //   BipedalWalker  4096 envs 26 / 31 : 39 / 53,  8192 envs 51 / 62 : 65 / 91,  12288 envs 77 / 93 : 84 / 127,
+        //     16384 envs 102 / 123 : 90 / 133.
+        // (The lines were drawn before the fused kernels had their present times: at width 256 Walker2d, Hopper and BipedalWalker,
+        // at 64 Walker2d and Hopper are ahead some way beyond theirs.)
         int envs_per_cu = 32;
         if (id == MRL_ENV_HALFCHEETAH || (id == MRL_ENV_WALKER2D_PLANAR && p.H == 64)) envs_per_cu = 16;
         else if (id == MRL_ENV_BIPEDAL && p.H == 256) envs_per_cu = 48;
