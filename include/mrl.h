@@ -110,12 +110,18 @@ int mrl_ctx_reserve(mrl_ctx *ctx, uint64_t mlp_floats, uint64_t rollout_floats);
  * the last synchronize wrote is void then: a workgroup that gave up stores neither its env rows nor its
  * observations nor its episode sums (they keep the values from before the launch), the other workgroups'
  * envs have advanced, and rollout rows and the finished-episode list hold a mixture -- reset the envs
- * and clear done_count before collecting again.  The fused minibatch update has one such wait, of its last
- * kernel's workgroups for each other's sums of squares: a workgroup that gives up leaves its share of the
- * parameters, gradients and moments as they were, so parameters and optimiser state hold a mixture.  No counterpart
- * in the reference; a tiny limit is how a test exercises the error path without hanging anything. */
+ * and clear done_count before collecting again.  No counterpart in the reference; a tiny limit is how a test
+ * exercises the error path without hanging anything. */
 #define MRL_DEFAULT_SPIN_LIMIT (1u << 22)
 int mrl_ctx_set_spin_limit(mrl_ctx *ctx, unsigned polls);
+
+/* The workgroups of the fused minibatch update's last kernel wait for each other's sums of squares.  After `polls` polls
+ * (MRL_DEFAULT_UPDATE_PATIENCE unless set here; 0 restores the default) a workgroup works out those that are missing by
+ * itself, with the same bits, so an update ends whatever other streams and processes hold of the device.  Where the spin limit
+ * above is smaller than this, as only a test has it, a workgroup gives up there: it leaves its share of the parameters, gradients
+ * and moments as they were, the next mrl_ctx_synchronize returns MRL_E_SYNC, and such an update cannot be issued again. */
+#define MRL_DEFAULT_UPDATE_PATIENCE 256u
+int mrl_ctx_set_update_patience(mrl_ctx *ctx, unsigned polls);
 
 /* How many of its minibatches the context's last mrl_ppo_update_minibatch / _epoch call enqueued: all of them,
  * or fewer where the host saw the KL stop while it was enqueueing (those left away would have done nothing). */

@@ -57,6 +57,11 @@ class DeviceContext:
         wait that gives up makes the next synchronize() raise; a tiny value exercises that path."""
         _lib.call("mrl_ctx_set_spin_limit", self.handle, int(polls))
 
+    def set_update_patience(self, polls):
+        """Polls after which a workgroup of the update's last kernel works out the sums of squares that it still waits for
+        by itself (0: the default); the results are the same bits."""
+        _lib.call("mrl_ctx_set_update_patience", self.handle, int(polls))
+
     def update_enqueued(self):
         """How many minibatches the last update call enqueued (fewer than it was given: the KL stop was seen meanwhile)."""
         n = C.c_int(0)

@@ -56,6 +56,7 @@ int mrl_ctx_create(void *hip_stream, mrl_ctx **out) {
     c->prof_every = 1;
     c->prof_active = true;
     c->spin_limit = MRL_DEFAULT_SPIN_LIMIT;
+    c->update_patience = MRL_DEFAULT_UPDATE_PATIENCE;
     CTX_TRY(hipGetDevice(&c->device));
     CTX_TRY(hipDeviceGetAttribute(&c->n_cus, hipDeviceAttributeMultiprocessorCount, c->device));
     c->stream_cus = c->n_cus;
@@ -146,6 +147,12 @@ int mrl_ctx_reserve(mrl_ctx *ctx, uint64_t mlp_floats, uint64_t rollout_floats) 
 int mrl_ctx_set_spin_limit(mrl_ctx *ctx, unsigned polls) {
     MRL_CHECK_ARG(ctx != nullptr, "mrl_ctx_set_spin_limit: ctx is NULL");
     ctx->spin_limit = polls == 0 ? MRL_DEFAULT_SPIN_LIMIT : polls;
+    return MRL_OK;
+}
+
+int mrl_ctx_set_update_patience(mrl_ctx *ctx, unsigned polls) {
+    MRL_CHECK_ARG(ctx != nullptr, "mrl_ctx_set_update_patience: ctx is NULL");
+    ctx->update_patience = polls == 0 ? MRL_DEFAULT_UPDATE_PATIENCE : polls;
     return MRL_OK;
 }
 

@@ -42,6 +42,7 @@ struct mrl_ctx {
     // writes directly) and the kernel ends normally.  mrl_ctx_synchronize reports and clears it.
     unsigned spin_limit;
     int *sync_error;
+    unsigned update_patience;   // polls of the update's last kernel for other workgroups' sums before it takes them itself
     // A multi-minibatch update's call number, and the number of the last call whose KL stop the device has seen (pinned, like
     // sync_error): the host leaves launches away that would find the stop raised and do nothing.
     int stop_call;

@@ -428,11 +428,12 @@ static void launch_adam_split(hipStream_t st, const AdamArgs &a, int o1, const S
 // clip_adam_split_kernel : in one launch: H = 64, 256 rows 18.0 : 14.5; H = 128, 1000 rows 27.7 : 24.9; H = 256,
 // 4096 rows 55.5 : 52.7.
 //
-// The wait needs every workgroup of the grid on the chip, so the host takes this kernel only where the grid is no larger
-// than the CUs that the stream may use (sum_adam_fits); a CU holds four of these workgroups (256 threads, at most 128
-// registers), so that four such grids, from as many streams, hold no place that another one waits for, whatever
-// else comes and goes beside them.  And it is bounded: a workgroup that gives up after spin_limit polls reports it and
-// updates nothing.
+// The wait is a short one where every workgroup of the grid is on the chip, so the host takes this kernel only where the grid
+// is no larger than the CUs that the stream may use.  It does not need that: other streams and processes may hold the places
+// of a part of the grid for as long as they like, also with waits of their own.  After `patience` polls a workgroup adds up the
+// squares that it still misses by itself, from the pieces, which nothing writes meanwhile: the same terms in the same order, so
+// the same bits.  (A limit of polls below that, which only a test sets, ends the wait before: the workgroup reports it and
+// updates nothing.)
 // W1: VW neighbouring columns per thread, so that a workgroup holds ROWS whole rows; the rest one parameter per thread.
 struct SumAdam {
     struct Net {
@@ -444,7 +445,7 @@ struct SumAdam {
     int IN, tiles;
     const int32_t *skip;      // never null
     uint64_t *posts;          // [net][gridDim.x]: 2^32 + the bits of a workgroup's sum of squares; zero before the launch
-    unsigned spin_limit;
+    unsigned patience, spin_limit;
     int *sync_error;
     int32_t *stop;            // the KL early stop's flag words; without a test a place with a zero and kl_n = 0
     const float *kl_part;     // the row tiles' sums, never null
@@ -463,7 +464,8 @@ __global__ __launch_bounds__(UTPB, 4) void sum_adam_kernel(SumAdam k) {
     typedef std::conditional_t<VW == 1, float, f32x4> Sum;
     __shared__ __align__(16) float tile[ROWS * TLD];
     __shared__ float sq_s[NW], kl_s[NW], total_s;
-    __shared__ int state_s;    // 0: update, 1: the KL stop, 2: the wait gave up
+    __shared__ uint64_t word_s[64];
+    __shared__ int state_s;    // 0: update, 1: the KL stop, 2: the wait gave up, 3: no longer waiting for the others' sums
     const int ynet = blockIdx.y, t = threadIdx.x;
     const SumAdam::Net net = k.net[ynet];
     const bool test = k.kl_n > 0;
@@ -474,13 +476,28 @@ __global__ __launch_bounds__(UTPB, 4) void sum_adam_kernel(SumAdam k) {
     for (int j = 0; j < KL_MOST / UTPB; ++j) klq[j] = k.kl_part[max(min(t + j * UTPB, k.kl_n - 1), 0)];
     const int o1 = (k.IN + 1) * H;
     const int TB = gridDim.x - WB;                    // the thin layers' workgroups go first: theirs are the long sums
-    const bool hidden = (int)blockIdx.x >= TB;
-    const int e0 = ((int)blockIdx.x - TB) * E + VW * t;                // element of W1
-    int i = blockIdx.x * UTPB + t;                    // a thin layer's parameter
-    if (i >= o1) i += H * H;
-    const bool mine = hidden || i < net.adam.n;
-    if (hidden) i = o1 + e0;
-    else i = min(i, net.adam.n - 1);
+    struct Place { bool hidden, mine; int e0, i; };   // element of W1, parameter
+    auto place = [&](int block) {
+        Place at;
+        at.hidden = block >= TB;
+        at.e0 = (block - TB) * E + VW * t;
+        int thin = block * UTPB + t;                  // a thin layer's parameter
+        if (thin >= o1) thin += H * H;
+        at.mine = at.hidden || thin < net.adam.n;
+        at.i = at.hidden ? o1 + at.e0 : min(thin, net.adam.n - 1);
+        return at;
+    };
+    auto thin_sum = [&](const Place &at) {
+        const float x = sum_terms<TREE, float>(thin_terms(net.sum, k.IN, H, k.tiles, at.i));
+        return at.mine ? x : 0.0f;
+    };
+    auto square = [](const Sum &s) {
+        if constexpr (VW == 1) return s * s;
+        else return (s[0] * s[0] + s[1] * s[1]) + (s[2] * s[2] + s[3] * s[3]);
+    };
+    const Place own_place = place(blockIdx.x);
+    const bool hidden = own_place.hidden, mine = own_place.mine;
+    const int i = own_place.i;
     V1 p = V1{};
     MV mv = MV{};
     Sum s = Sum{};
@@ -488,27 +505,30 @@ __global__ __launch_bounds__(UTPB, 4) void sum_adam_kernel(SumAdam k) {
         p = *reinterpret_cast<const V1 *>(net.adam.p + i);
         mv = *reinterpret_cast<const MV *>(net.adam.state + i);
         __builtin_amdgcn_sched_barrier(0);
-        s = sum_terms<TREE, Sum>(hidden_terms(net.sum, e0));
+        s = sum_terms<TREE, Sum>(hidden_terms(net.sum, own_place.e0));
     } else {
         const float2 one = net.adam.state[i];
         p[0] = net.adam.p[i];
         __builtin_amdgcn_sched_barrier(0);
-        const float x = sum_terms<TREE, float>(thin_terms(net.sum, k.IN, H, k.tiles, i));
+        const float x = thin_sum(own_place);
         mv[0] = one.x;
         mv[1] = one.y;
-        if constexpr (VW == 1) s = mine ? x : 0.0f;
-        else s[0] = mine ? x : 0.0f;
+        if constexpr (VW == 1) s = x;
+        else s[0] = x;
     }
     // ---- the KL verdict, the same in every workgroup, and the norm
-    float q = 0.0f, kl = 0.0f;
-    if constexpr (VW == 1) q = s * s;
-    else q = (s[0] * s[0] + s[1] * s[1]) + (s[2] * s[2] + s[3] * s[3]);
+    float q = square(s), kl = 0.0f;
 #pragma unroll
     for (int j = 0; j < KL_MOST / UTPB; ++j) kl += t + j * UTPB < k.kl_n ? klq[j] : 0.0f;
     q = dpp_wave_sum(q);
     kl = dpp_wave_sum(kl);
     if ((t & 63) == 0) { sq_s[t >> 6] = q; kl_s[t >> 6] = kl; }
     __syncthreads();
+    uint64_t *const post = k.posts + (size_t)ynet * gridDim.x;
+    auto post_word = [&](int block, float sum) {
+        __hip_atomic_store(post + block, (1ull << 32) | __float_as_uint(sum), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    auto posted = [&](int block) { return __hip_atomic_load(post + block, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
     if (t < 64) {
         const float mean = ((kl_s[0] + kl_s[1]) + (kl_s[2] + kl_s[3])) / (float)k.kl_mb;
         const bool over = test && mean > k.target_kl;
@@ -517,20 +537,17 @@ __global__ __launch_bounds__(UTPB, 4) void sum_adam_kernel(SumAdam k) {
         int state = stop ? 1 : 0;
         float total = 0.0f;
         if (!stop && k.max_norm > 0.0f) {
-            uint64_t *post = k.posts + (size_t)ynet * gridDim.x;
-            if (t == 0) {
-                const float own = (sq_s[0] + sq_s[1]) + (sq_s[2] + sq_s[3]);
-                __hip_atomic_store(post + blockIdx.x, (1ull << 32) | __float_as_uint(own), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
+            if (t == 0) post_word(blockIdx.x, (sq_s[0] + sq_s[1]) + (sq_s[2] + sq_s[3]));
             // lane t takes the words t, t + 64, ..., one wait after the other: all but the first find theirs there
             unsigned polls = 0;
-            for (int b0 = 0; b0 < (int)gridDim.x; b0 += 64) {
+            for (int b0 = 0; b0 < (int)gridDim.x && state == 0; b0 += 64) {
                 const bool in = b0 + t < (int)gridDim.x;
                 uint64_t word = 0;
                 for (;;) {
-                    if (in && word == 0) word = __hip_atomic_load(post + b0 + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    if (in && word == 0) word = posted(b0 + t);
                     if (!any_lane(in && word == 0)) break;
-                    if (++polls > k.spin_limit) { state = 2; break; }
+                    if (++polls >= k.patience) { state = 3; break; }
+                    if (polls > k.spin_limit) { state = 2; break; }
                 }
                 total += __uint_as_float((uint32_t)word);
             }
@@ -551,8 +568,46 @@ __global__ __launch_bounds__(UTPB, 4) void sum_adam_kernel(SumAdam k) {
         }
     }
     __syncthreads();
+    if (state_s == 3) {
+        // The words in the same order as above, lane t's t, t + 64, ...; one that is not there is worked out by all threads, as its
+        // own workgroup does it, and left for the others.
+        float total = 0.0f;
+        for (int b0 = 0; b0 < (int)gridDim.x; b0 += 64) {
+            const int n = min(64, (int)gridDim.x - b0);
+            if (t < n) word_s[t] = posted(b0 + t);
+            __syncthreads();
+            for (int j = 0; j < n; ++j) {
+                if (word_s[j] != 0) continue;
+                const Place at = place(b0 + j);
+                Sum x = Sum{};
+                if (at.hidden) {
+                    x = sum_terms<TREE, Sum>(hidden_terms(net.sum, at.e0));
+                } else {
+                    const float one = thin_sum(at);
+                    if constexpr (VW == 1) x = one;
+                    else x[0] = one;
+                }
+                const float sq = dpp_wave_sum(square(x));
+                if ((t & 63) == 0) sq_s[t >> 6] = sq;
+                __syncthreads();
+                if (t == j) {
+                    const float sum = (sq_s[0] + sq_s[1]) + (sq_s[2] + sq_s[3]);
+                    post_word(b0 + j, sum);
+                    word_s[j] = __float_as_uint(sum);
+                }
+                __syncthreads();
+            }
+            if (t < n) total += __uint_as_float((uint32_t)word_s[t]);
+            __syncthreads();
+        }
+        if (t < 64) {
+            total = dpp_wave_sum(total);
+            if (t == 0) total_s = total;
+        }
+        __syncthreads();
+    }
     const int state = state_s;
-    if (state != 0) {
+    if (state == 1 || state == 2) {
         // The gradients as they are.  (Nothing else hangs on `skip`: a workgroup of this launch may raise it while a wavefront
         // reads it.)
         if (state == 1 && skip == 0) {
@@ -749,6 +804,7 @@ static int update_minibatch_paired(mrl_ctx *ctx, const mrl_update *u, const int3
         k.beta1 = a.beta1; k.beta2 = a.beta2; k.omb1 = a.omb1; k.omb2 = a.omb2; k.eps = a.eps;
         k.IN = sn.IN; k.tiles = sn.tiles; k.skip = sn.skip;
         k.posts = fl.posts;
+        k.patience = ctx->update_patience;
         k.spin_limit = ctx->spin_limit;
         k.sync_error = ctx->sync_error;
         const bool test = a.stop != nullptr;

@@ -1,5 +1,5 @@
 """The update whose sums, clip and Adam are one launch against the two launches that a stream with few CUs takes, at sizes where
-the workgroups' shares end unevenly; and the one launch's bounded wait."""
+the workgroups' shares end unevenly; and the one launch's wait, which no other work on the device can keep from ending."""
 import ctypes
 import math
 
@@ -65,6 +65,79 @@ def test_one_launch_equals_two(mrl, env, H, MB, target, max_norm):
         assert torch.isfinite(a).all() and float(a.abs().max()) > 0
         # (three steps of 1e-3 from weights of 0.1, moments up to 1e-3: differences of 1e-6 of the largest value at most)
         assert float((a - b).abs().max()) <= 2e-6 * float(b.abs().max())
+
+
+def left(rb, upd):
+    return [t.clone() for t in (upd.actor_grads, upd.critic_grads, upd.actor_state, upd.critic_state, rb.actor_params, rb.critic_params,
+                                upd.kl_flag)]
+
+
+@pytest.mark.parametrize("env,H,MB", [("CartPoleEnv", 64, 2), ("PendulumV2", 64, 4200), ("LunarLanderV2", 128, 1000),
+                                      ("Walker2dPlanar", 128, 4100), ("HopperPlanar", 256, 17), ("BipedalWalkerV2", 256, 4100)])
+@pytest.mark.parametrize("target", [0.0, 1e30, 1e-30])
+def test_sums_that_are_not_there_are_worked_out(mrl, env, H, MB, target):
+    """A workgroup that does not wait for the others' sums takes them itself: the same bits, and nothing to report, also where the
+    limit of polls is one that a wait would not keep."""
+    print("no patience", env, H, MB, target, flush=True)
+    E, got = getattr(mrl, env), []
+    for patience in (0, 1):
+        ctx = mrl.DeviceContext("cuda:0")
+        rb, upd, perm = build(mrl, ctx, E, H, MB, target)
+        ctx.set_update_patience(patience)
+        if patience:
+            ctx.set_spin_limit(1)
+        upd.run_epoch(perm)
+        ctx.synchronize()
+        got.append(left(rb, upd))
+        ctx.close()
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+    assert torch.isfinite(got[0][4]).all()
+
+
+def test_places_for_a_part_of_the_grid(mrl):
+    """An update captured where every workgroup has a CU, replayed where the stream has eight of them; and six updates on streams of
+    their own."""
+    print("few places", flush=True)
+    E, streams = mrl.HalfCheetahPlanarV2, [torch.cuda.Stream() for _ in range(6)]
+    parts = []
+    for s in streams:
+        ctx = mrl.DeviceContext("cuda:0", stream=s)
+        parts.append((ctx,) + build(mrl, ctx, E, 256, 512, 0.0))
+    ctx, rb, upd, perm = parts[0]
+    first = left(rb, upd)
+
+    def restart(rb, upd):
+        for dst, src in zip((upd.actor_grads, upd.critic_grads, upd.actor_state, upd.critic_state, rb.actor_params, rb.critic_params), first):
+            dst.copy_(src)
+        torch.cuda.synchronize()
+
+    def epoch(upd, perm):   # (run_epoch with the step counts of a first one)
+        d = upd.descriptor()
+        mrl._lib.call("mrl_ppo_update_epoch", upd.ctx.handle, ctypes.byref(d), perm.data_ptr(), 3, 0, 0)
+
+    epoch(upd, perm)
+    ctx.synchronize()
+    want = left(rb, upd)
+    for c, r, u, p in parts:
+        restart(r, u)
+    for c, r, u, p in parts:
+        epoch(u, p)
+    for c, r, u, p in parts:
+        c.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(left(r, u), want))
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=streams[0]):
+        epoch(upd, perm)
+    few = masked_stream(8)
+    for replay in range(3):
+        restart(rb, upd)
+        with torch.cuda.stream(few):
+            graph.replay()
+        torch.cuda.synchronize()
+        ctx.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(left(rb, upd), want)), replay
+    del graph
 
 
 def test_a_wait_that_gives_up_is_reported(mrl):
