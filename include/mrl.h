@@ -94,6 +94,9 @@ int mrl_ctx_create(void *hip_stream, mrl_ctx **out);
 int mrl_ctx_destroy(mrl_ctx *ctx);
 /* blocks until the context's stream has drained; DeviceContext.synchronize() */
 int mrl_ctx_synchronize(mrl_ctx *ctx);
+/* What mrl_ctx_synchronize reports behind its wait (MRL_E_SYNC, see mrl_ctx_set_spin_limit), without one: for a caller that has
+ * just waited for the stream itself, by a copy to the host for instance (a synchronize of a drained stream is 30 to 40 us). */
+int mrl_ctx_check(mrl_ctx *ctx);
 
 /* Workspaces of the context, in floats: what they hold now (either pointer may be NULL), and a
  * request to hold at least that much (0 = leave as is; never shrinks).  mrl_ctx_reserve drains the
@@ -106,7 +109,7 @@ int mrl_ctx_reserve(mrl_ctx *ctx, uint64_t mlp_floats, uint64_t rollout_floats);
 /* The fused collection kernels let groups of wavefronts of a workgroup meet at barriers of their own
  * (counters in LDS).  Every such wait is bounded: after `polls` polls (MRL_DEFAULT_SPIN_LIMIT unless
  * set here; 0 restores the default) the waiting wavefront gives up, the workgroup stops stepping, the
- * kernel ends normally and the next mrl_ctx_synchronize returns MRL_E_SYNC (once).  What the calls since
+ * kernel ends normally and the next mrl_ctx_synchronize or mrl_ctx_check returns MRL_E_SYNC (once).  What the calls since
  * the last synchronize wrote is void then: a workgroup that gave up stores neither its env rows nor its
  * observations nor its episode sums (they keep the values from before the launch), the other workgroups'
  * envs have advanced, and rollout rows and the finished-episode list hold a mixture -- reset the envs

@@ -71,6 +71,7 @@ SIGNATURES = {
     "mrl_ctx_create": [P, C.POINTER(P)],
     "mrl_ctx_destroy": [P],
     "mrl_ctx_synchronize": [P],
+    "mrl_ctx_check": [P],
     "mrl_ctx_set_spin_limit": [P, C.c_uint],
     "mrl_ctx_set_update_patience": [P, C.c_uint],
     "mrl_ctx_update_enqueued": [P, C.POINTER(I)],

@@ -89,6 +89,7 @@ class _PPOAgentBase:
             upd.update(self.num_epochs, seed=seed * 7919 + metrics.rollouts)
             # the only read-back of the rollout: the finished episodes
             cnt = min(int(rb.done_count.item()), rb.done_cap)
+            ctx.check()   # (raises where a kernel gave up a wait, before anything of such a rollout is logged or saved)
             if cnt:
                 metrics.log_episodes(rb.done_returns[:cnt].tolist(), rb.done_lengths[:cnt].tolist())
             # auto-checkpoint whenever the episode count passes a multiple of checkpoint_every

@@ -41,6 +41,10 @@ class DeviceContext:
     def synchronize(self):
         _lib.call("mrl_ctx_synchronize", self.handle)
 
+    def check(self):
+        """What synchronize() raises where a kernel gave up a wait, for a caller that has waited for the stream already."""
+        _lib.call("mrl_ctx_check", self.handle)
+
     def workspace(self):
         """(mlp_floats, rollout_floats) that the context's two workspaces hold now."""
         import ctypes

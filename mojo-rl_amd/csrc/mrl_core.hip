@@ -118,16 +118,25 @@ int mrl_ctx_destroy(mrl_ctx *ctx) {
     return MRL_OK;
 }
 
+static int report_gave_up(mrl_ctx *ctx, const char *who) {
+    if (*(volatile int *)ctx->sync_error != 0) {
+        *ctx->sync_error = 0;
+        return mrl::set_error(MRL_E_SYNC, "%s: a kernel gave up waiting at one of its internal "
+                              "barriers (limit %u polls); the results of the calls since the last synchronize are void",
+                              who, ctx->spin_limit);
+    }
+    return MRL_OK;
+}
+
 int mrl_ctx_synchronize(mrl_ctx *ctx) {
     MRL_CHECK_ARG(ctx != nullptr, "mrl_ctx_synchronize: ctx is NULL");
     MRL_CHECK_HIP(hipStreamSynchronize(ctx->stream));
-    if (*(volatile int *)ctx->sync_error != 0) {
-        *ctx->sync_error = 0;
-        return mrl::set_error(MRL_E_SYNC, "mrl_ctx_synchronize: a kernel gave up waiting at one of its internal "
-                              "barriers (limit %u polls); the results of the calls since the last synchronize are void",
-                              ctx->spin_limit);
-    }
-    return MRL_OK;
+    return report_gave_up(ctx, "mrl_ctx_synchronize");
+}
+
+int mrl_ctx_check(mrl_ctx *ctx) {
+    MRL_CHECK_ARG(ctx != nullptr, "mrl_ctx_check: ctx is NULL");
+    return report_gave_up(ctx, "mrl_ctx_check");
 }
 
 int mrl_ctx_workspace(mrl_ctx *ctx, uint64_t *mlp_floats, uint64_t *rollout_floats) {

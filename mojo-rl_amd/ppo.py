@@ -352,8 +352,10 @@ class PPOUpdate:
 
     def kl_stopped(self):
         """Reads the device flag (one synchronising copy of 16 bytes): (stopped, last mean KL).
-        When the stop has fired the optimisers' step counters are set to the updates applied."""
+        When the stop has fired the optimisers' step counters are set to the updates applied.  Raises MrlError where a
+        kernel since the last synchronize gave up a wait: what it has left is not to be trained on."""
         f = self.kl_flag.cpu()
+        self.ctx.check()
         stopped = bool(f[0].item())
         if stopped:
             applied = int(f[2].item())

@@ -79,6 +79,22 @@ def test_continuous_agent_runs_on_the_walkers(mrl, env_name, obs_dim, action_dim
     assert agent.actor.optimizer.t > 0
 
 
+@pytest.mark.parametrize("target_kl", [0.0, 1e30])
+def test_a_wait_that_gives_up_ends_training(mrl, tmp_path, target_kl):
+    """A kernel that gave up a wait leaves void results: train_gpu raises, and neither logs nor saves what came of them."""
+    print("give up", target_kl, flush=True)
+    ctx, path = mrl.DeviceContext("cuda:0"), tmp_path / "agent.ckpt"
+    agent = mrl.DeepPPOAgent(obs_dim=8, num_actions=4, hidden_dim=64, rollout_len=128, n_envs=512, gpu_minibatch_size=4096,
+                             num_epochs=1, target_kl=target_kl, checkpoint_every=1, checkpoint_path=str(path))
+    ctx.set_spin_limit(1)
+    with pytest.raises(mrl.MrlError, match="internal barriers"):
+        agent.train_gpu(ctx, mrl.LunarLanderV2, num_episodes=10**9, max_rollouts=1)
+    assert not path.exists()
+    ctx.set_spin_limit(0)
+    m = agent.train_gpu(ctx, mrl.LunarLanderV2, num_episodes=10**9, max_rollouts=1)
+    assert m.rollouts == 1 and len(m.episode_rewards) > 0 and path.exists()
+
+
 def test_observation_noise_enters_the_rollout(mrl, orc):
     """obs_noise_std > 0 (ppo_continuous.mojo:2557-2564, :2705-2713): the policy sees noisy
     observations from the first step on, the env rows stay clean, and the stored observation of step
