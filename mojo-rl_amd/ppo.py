@@ -165,16 +165,12 @@ class RunningMeanStd:
 
 
 def _zeroed(device, **sizes):
-    """{name: a flat zeroed float32 tensor of that many elements, or an int32 one for (elements, torch.int32)}, slices of one
-    allocation, 256 bytes apart at least.  A training call makes three dozen of them: one fill instead of one each (1.7 us of
-    the device and 10 of the host apiece; CartPole, 1024 envs x 128 steps: 0.3 ms of a call's 1.2)."""
-    at, places = 0, []
-    for name, size in sizes.items():
-        n, dtype = size if isinstance(size, tuple) else (size, torch.float32)
-        places.append((name, at, n, dtype))
-        at += -(-n // 64) * 64
-    flat = torch.zeros(at, device=device)
-    return {name: flat[o:o + n] if dtype == torch.float32 else flat[o:o + n].view(dtype) for name, o, n, dtype in places}
+    """{name: a flat zeroed float32 tensor of that many elements, or an int32 one for (elements, torch.int32)}.  Each has memory
+    of its own, so that one can be replaced, saved or changed in place without the others; they are filled together.  A training
+    call makes three dozen of them (CartPole, 1024 envs x 128 steps): 68 us of the host, 200 with a fill each."""
+    made = {name: torch.empty(size[0] if isinstance(size, tuple) else size, device=device) for name, size in sizes.items()}
+    torch._foreach_zero_(list(made.values()))
+    return {name: made[name].view(size[1]) if isinstance(size, tuple) else made[name] for name, size in sizes.items()}
 
 
 class RolloutBuffers:

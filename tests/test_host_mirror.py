@@ -97,3 +97,24 @@ def test_bench_refuses_more_than_one_gpu():
     p = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py"), "--gpus", "2"],
                        capture_output=True, text=True, timeout=120)
     assert p.returncode != 0 and "one MI355X" in (p.stderr + p.stdout)
+
+
+def test_training_buffers_have_memory_of_their_own(mrl):
+    """Replacing, saving or changing one buffer leaves the others as they are: no shared allocation, no shared version counter."""
+    torch = pytest.importorskip("torch")
+    actor = mrl.seq(mrl.LinearReLU(4, 64), mrl.LinearReLU(64, 64), mrl.Linear(64, 2))
+    critic = mrl.seq(mrl.LinearReLU(4, 64), mrl.LinearReLU(64, 64), mrl.Linear(64, 1))
+    ctx = type("Ctx", (), dict(device=torch.device("cpu")))()
+    for pass_ in range(3):                                        # (later passes on memory that has been in use)
+        rb = mrl.ppo.RolloutBuffers(ctx, mrl.CartPoleEnv, actor, critic, 5, 3)
+        upd = mrl.ppo.PPOUpdate(ctx, rb, 4, mrl.Adam(), mrl.Adam())
+        buffers = [t for o in (rb, upd) for t in vars(o).values() if isinstance(t, torch.Tensor)]
+        assert len(buffers) == 35 and rb.done_count.dtype == upd.indices.dtype == upd.kl_flag.dtype == torch.int32
+        for t in buffers:
+            assert t.untyped_storage().nbytes() == 4 * t.numel() and t.is_contiguous() and t.dim() == 1
+            assert not t.any()
+        versions = [t._version for t in buffers]
+        rb.obs.add_(1.0)
+        assert [t._version for t in buffers if t is not rb.obs] == [v for v, t in zip(versions, buffers) if t is not rb.obs]
+        for t in buffers:
+            t.fill_(7)
