@@ -127,7 +127,7 @@ __global__ __launch_bounds__(256, 2) void collect16_kernel(CollectArgs a) {
             a.r_logp[at] = logp;
             a.r_values[at] = vals[q][e];
         }
-        books.rewards(a, listed, at, rew[q][e], don[q][e], lane, mine);
+        books.rewards(a, listed, k, at, rew[q][e], don[q][e], lane, mine);
     };
     // solver wavefront, four lanes per env: what the env's wiring is (E::lanes_wired) in all four
     const int my_env = (t & 63) >> 2;
@@ -457,7 +457,7 @@ __global__ __launch_bounds__(512, 2) void collect16_wide_kernel(CollectArgs a) {
                 a.r_logp[at] = logp;
                 a.r_values[at] = vals[q][e];
             }
-            books.rewards(a, finished, at, rew[q][e], don[q][e], lane, mine);
+            books.rewards(a, finished, k, at, rew[q][e], don[q][e], lane, mine);
         };
         int done = 0;   // steps taken
         for (int k = 0; k < a.n_steps; ++k) {
@@ -637,10 +637,10 @@ struct CartPoleRows {
     MRL_DEV void make_uniform(const CollectArgs &a, int k, int env0, int e) {
         uniform[k & 1][e] = categorical_uniform(a.sample_seed + (uint32_t)k * a.sample_stride, env0 + e);
     }
-    MRL_DEV void book(EpisodeBooks &b, const CollectArgs &a, EpisodeBooks::Waiting &w, size_t at, int q, int lane, bool mine) const {
-        const int e = lane & (R - 1), sel = drawn[q][e];
+    MRL_DEV void book(EpisodeBooks &b, const CollectArgs &a, EpisodeBooks::Waiting &w, int k, size_t at, int lane, bool mine) const {
+        const int q = k & 1, e = lane & (R - 1), sel = drawn[q][e];
         if (mine) a.r_actions[at] = (float)sel;
-        b.rewards(a, w, at, rew[q][sel][e], don[q][sel][e], lane, mine);
+        b.rewards(a, w, k, at, rew[q][sel][e], don[q][sel][e], lane, mine);
     }
     MRL_DEV void draw(int now, int e, int l, float logit) {
         float pr;
@@ -723,7 +723,7 @@ __global__ __launch_bounds__(512, 4) void collect_cartpole16_kernel(CollectArgs 
 
     auto book = [&](int k, int e, int ne) {   // what step k leaves beside the envs' rows
         const size_t at = (size_t)(a.t0 + k) * N + env0 + e;
-        c.book(books, a, finished, at, k & 1, e, e < ne);
+        c.book(books, a, finished, k, at, e, e < ne);
         if (e >= ne) return;
         a.r_logp[at] = log32(c.prob[k & 1][e] + 1e-8f);
         a.r_values[at] = vals[k & 1][e];
@@ -843,7 +843,7 @@ __global__ __launch_bounds__(512, 4) void collect_cartpole16_h64_kernel(CollectA
         head.load(w2c, lane & 3);
         float prob = 0.0f;
         auto rewards = [&](int k) {
-            c.book(books, a, finished, row0 + (size_t)k * N + lane, k & 1, lane, mine);
+            c.book(books, a, finished, k, row0 + (size_t)k * N + lane, lane, mine);
             prob = c.prob[k & 1][lane & (R - 1)];
         };
         auto value = [&](int k) {
@@ -1094,7 +1094,7 @@ __global__ __launch_bounds__(512, 4) void collect_pendulum16_h64_kernel(CollectA
             mu = mean[q];
             const size_t at = row0 + (size_t)k * N + lane;
             if (mine) a.r_actions[at] = u;
-            books.rewards(a, finished, at, rew[q], don[q], lane, mine);
+            books.rewards(a, finished, k, at, rew[q], don[q], lane, mine);
         };
         auto value = [&](int k) {
             float out[1];
