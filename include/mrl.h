@@ -130,6 +130,11 @@ int mrl_ctx_set_update_patience(mrl_ctx *ctx, unsigned polls);
  * or fewer where the host saw the KL stop while it was enqueueing (those left away would have done nothing). */
 int mrl_ctx_update_enqueued(mrl_ctx *ctx, int *minibatches);
 
+/* In how many launches the last minibatch of that call takes its gradients' sums, the clip and Adam: 1 where the grid of the one
+ * launch is no larger than the CUs that the context's stream may use, 2 elsewhere, 0 for a call of the layer-by-layer route or
+ * before the first. */
+int mrl_ctx_update_end_launches(mrl_ctx *ctx, int *launches);
+
 /* Device-time accounting per phase, the counterpart of the perf_counter_ns phase timers that
  * train_gpu prints (deep_agents/ppo/ppo.mojo:2062-2067, :2777-2838) measured with HIP events on
  * the context's stream instead of host enqueue times.  mrl_profile_begin arms it (at most

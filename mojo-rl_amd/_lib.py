@@ -75,6 +75,7 @@ SIGNATURES = {
     "mrl_ctx_set_spin_limit": [P, C.c_uint],
     "mrl_ctx_set_update_patience": [P, C.c_uint],
     "mrl_ctx_update_enqueued": [P, C.POINTER(I)],
+    "mrl_ctx_update_end_launches": [P, C.POINTER(I)],
     "mrl_ctx_workspace": [P, C.POINTER(C.c_uint64), C.POINTER(C.c_uint64)],
     "mrl_ctx_reserve": [P, C.c_uint64, C.c_uint64],
     "mrl_profile_begin": [P, I],

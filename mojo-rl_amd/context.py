@@ -72,6 +72,12 @@ class DeviceContext:
         _lib.call("mrl_ctx_update_enqueued", self.handle, C.byref(n))
         return n.value
 
+    def update_end_launches(self):
+        """In how many launches the last minibatch took its sums, clip and Adam (0: layer by layer)."""
+        n = C.c_int(0)
+        _lib.call("mrl_ctx_update_end_launches", self.handle, C.byref(n))
+        return n.value
+
     PHASES = ("policy_fwd", "sample_store", "env_step", "post_store", "collect")
 
     def profile_begin(self, max_marks=8192, sample_every=1):

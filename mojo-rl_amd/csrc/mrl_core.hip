@@ -91,6 +91,7 @@ int mrl_ctx_create(void *hip_stream, mrl_ctx **out) {
     *c->upd_reached = 0;
     c->upd_count = 0;
     c->upd_enqueued = 0;
+    c->upd_end_launches = 0;
     {
         int rc = mrl::clip_static_setup(c->device);
         if (rc != MRL_OK) { mrl_ctx_destroy(c); return rc; }
@@ -168,6 +169,12 @@ int mrl_ctx_set_update_patience(mrl_ctx *ctx, unsigned polls) {
 int mrl_ctx_update_enqueued(mrl_ctx *ctx, int *minibatches) {
     MRL_CHECK_ARG(ctx != nullptr && minibatches != nullptr, "mrl_ctx_update_enqueued: NULL argument");
     *minibatches = ctx->upd_enqueued;
+    return MRL_OK;
+}
+
+int mrl_ctx_update_end_launches(mrl_ctx *ctx, int *launches) {
+    MRL_CHECK_ARG(ctx != nullptr && launches != nullptr, "mrl_ctx_update_end_launches: NULL argument");
+    *launches = ctx->upd_end_launches;
     return MRL_OK;
 }
 

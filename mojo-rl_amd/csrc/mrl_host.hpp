@@ -51,6 +51,7 @@ struct mrl_ctx {
     // the kernel that applies them).
     unsigned upd_count, *upd_reached;
     int upd_enqueued;   // minibatches that the last update call enqueued
+    int upd_end_launches;   // of the last minibatch's sums, clip and Adam (0: layer by layer)
     // CarRacingV2: 0 = the CPU env's reward / termination arithmetic (default), 1 = the GPU trait's
     int car_trait_form;
     // phase timing: events recorded on `stream` at phase boundaries while armed

@@ -788,6 +788,7 @@ static int update_minibatch_paired(mrl_ctx *ctx, const mrl_update *u, const int3
     const int H = u->actor.layers[0].out_dim, o1 = (u->obs_dim + 1) * H;
     const int blocks = sum_adam_blocks(H, a);
     const bool one_launch = 2 * blocks <= std::min(ctx->stream_cus, POSTS_MAX);
+    ctx->upd_end_launches = one_launch ? 1 : 2;
     if (one_launch) {
         fl.posts = reinterpret_cast<uint64_t *>(ctx->upd_scratch + SCR_SQ);
         fl.n_posts = 2 * blocks;
@@ -894,7 +895,7 @@ constexpr auto AHEAD_PATIENCE = std::chrono::milliseconds(50);
 // KL test the host stays within that many minibatches of the device
 static int update_minibatches(mrl_ctx *ctx, const mrl_update *u, const int32_t *indices, int n, int actor_t0, int critic_t0, int ahead) {
     int rc;
-    ctx->upd_enqueued = 0;
+    ctx->upd_enqueued = ctx->upd_end_launches = 0;
     if (!update_paired(u)) {
         for (int k = 0; k < n; ++k) {
             rc = update_minibatch_layers(ctx, u, indices + (size_t)k * u->minibatch, actor_t0 + k + 1, critic_t0 + k + 1);
@@ -980,7 +981,7 @@ int mrl_minibatch_adv_stats(mrl_ctx *ctx, const int32_t *indices, const float *a
 static int update_epoch(mrl_ctx *ctx, const mrl_update *u, const int32_t *indices, int n_minibatches, int actor_t0, int critic_t0,
                         int ahead, const char *who) {
     MRL_CHECK_ARG(ctx != nullptr, "%s: ctx is NULL", who);
-    ctx->upd_enqueued = 0;
+    ctx->upd_enqueued = ctx->upd_end_launches = 0;
     int rc = update_check(u, who);
     if (rc) return rc;
     MRL_CHECK_ARG(n_minibatches >= 0 && actor_t0 >= 0 && critic_t0 >= 0, "%s: negative count", who);

@@ -52,12 +52,13 @@ def test_one_launch_equals_two(mrl, env, H, MB, target, max_norm):
     gradients, moments and steps, move by a few 2^-24."""
     print("one launch", env, H, MB, target, max_norm, flush=True)
     E, got = getattr(mrl, env), []
-    few = masked_stream(64)
-    for stream in (None, few):
+    few = masked_stream(32)     # (the smallest grid is 36 workgroups: width 64, 3 inputs)
+    for launches, stream in ((1, None), (2, few)):
         ctx = mrl.DeviceContext("cuda:0", stream=stream)
         rb, upd, perm = build(mrl, ctx, E, H, MB, target, max_norm)
         upd.run_epoch(perm)
         ctx.synchronize()
+        assert ctx.update_end_launches() == launches
         got.append([t.clone() for t in (upd.actor_grads, upd.critic_grads, upd.actor_state, upd.critic_state, rb.actor_params,
                                         rb.critic_params)])
         ctx.close()
