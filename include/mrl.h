@@ -367,10 +367,11 @@ int mrl_rollout_step(mrl_ctx *ctx, const mrl_rollout *r, int t, uint32_t sample_
  * and reset_seed + k * reset_stride (mod 2^64) -- the reference derives its per-step seeds from
  * the step counter in the same affine way.  Buffers end up as after n_steps calls of
  * mrl_rollout_step with those seeds, except that the order of the finished-episode list
- * (done_returns / done_lengths) inside the call is unspecified.  Where the env and the networks
+ * (done_returns / done_lengths) inside the call is unspecified (fused, about that in which the episodes end: the workgroups
+ * list theirs every sixteen steps).  Where the env and the networks
  * allow it (the agents' nets with hidden layers of 64, 128 or 256 and as many envs as make it the
- * faster way) the whole range is ONE launch: each workgroup keeps its 16 or 32 envs on the chip (rows
- * in LDS, or state in registers for CartPole and Pendulum) and alternates policy forward and env step
+ * faster way) the whole range is ONE launch: each workgroup keeps its 16 envs on the chip (rows
+ * in LDS, or state in registers for Pendulum) and alternates policy forward and env step
  * on them, so states and observations cross HBM once per call instead of twice per step; otherwise the
  * steps are issued one by one.  Enqueue only. */
 int mrl_rollout_steps(mrl_ctx *ctx, const mrl_rollout *r, int t0, int n_steps, uint32_t sample_seed,
@@ -420,9 +421,10 @@ int mrl_ppo_update_minibatch(mrl_ctx *ctx, const mrl_update *u, const int32_t *i
  * runs with step counts actor_t0 + k + 1 / critic_t0 + k + 1 */
 int mrl_ppo_update_epoch(mrl_ctx *ctx, const mrl_update *u, const int32_t *indices, int n_minibatches,
                          int actor_t0, int critic_t0);
-/* The same for a caller that waits for the epoch's end right behind it (to read kl_flag): with a KL test the call itself waits
- * so that it is never more than `ahead` (>= 1) minibatches ahead of the device, and so few launches are left to run once the
- * stop is up.  Where the device does not come on for 50 ms the call goes on without waiting, and a capture never waits. */
+/* The same for a caller that waits for the epoch's end right behind it (to read kl_flag): with a KL test and nets of the fused
+ * shapes the call itself waits so that it is never more than `ahead` (>= 1) minibatches ahead of the device, and so few launches
+ * are left to run once the stop is up.  Where the device does not come on for 50 ms the call goes on without waiting; a capture
+ * and the layer-by-layer route of other nets, whose minibatches behind the stop run in full, never wait. */
 int mrl_ppo_update_epoch_ahead(mrl_ctx *ctx, const mrl_update *u, const int32_t *indices, int n_minibatches,
                                int actor_t0, int critic_t0, int ahead);
 

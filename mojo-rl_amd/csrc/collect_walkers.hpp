@@ -9,22 +9,25 @@
 //            body solver on wavefronts 2, 3, 6 and 7 (the two SIMDs that the solver's wavefronts 0 and 1
 //            do not use).  CarRacing, whose env step takes every wavefront: both nets side by side
 //            (critic on wavefronts 4 .. 7) ahead of it;
-//   sample   one lane per (env, action component): every component has a Philox stream of its own;
+//   sample   one lane per (env, action component): every component has a Philox stream of its own (all but
+//            CarRacing: the normal numbers a step ahead, beside the actor);
 //   env step BipedalWalker: the workgroup-level step of env_block.hpp (contact detection on every
 //            wavefront, solver with one lane per body on wavefronts 0 and 1, lidar rays on every
 //            wavefront, wave-cooperative resets); HalfCheetah: one lane per body on wavefronts 0 and 1
 //            (env_cheetah_lanes.hpp); CarRacing: a wavefront per env, two rounds of eight (env_car.hpp);
 //            the tile tables stay in global memory and are staged through LDS every step (16 x 12 KB do
 //            not fit beside the rest); HopperPlanar / Walker2dPlanar: one lane per env on wavefront 0
-//            (Float64, env_planar.hpp), the critic beside it as for the walkers;
-//   rollout row t of obs, action, log-prob, value, reward, done written on the way.
+//            (Float64, env_planar.hpp), the critic beside it as for the walkers, at width 256 on the six
+//            wavefronts of the other three SIMDs;
+//   rollout row t of obs, action, log-prob, value, reward, done and the episode sums written on the way (all but
+//            CarRacing: a step later, by a wavefront that has the time beside the actor).
 // With these envs the step is 70 - 80 % env step, a chain of one or two wavefronts' instructions: what the
 // fusion buys is the launch gaps, the observation / action round trip through HBM, the staging of the rows
 // in and out of LDS every step, and a policy forward of a 16-row tile on one CU.
 //
 // It gives what n_steps calls of mrl_rollout_step give (same per-env streams: seeds are affine in
 // the step number), except that the finished-episode list is appended in the order in which blocks
-// get there rather than step by step.
+// get there, every sixteen steps (CarRacing: every step), rather than step by step.
 #pragma once
 #include <type_traits>
 #include "mrl_host.hpp"
@@ -372,9 +375,10 @@ __global__ __launch_bounds__(512) void collect_car_kernel(CollectArgs a) {
 }
 
 // HopperPlanar / Walker2dPlanar (env_planar.hpp): the rows (248 / 392 bytes, Float64 state behind the fp32
-// observation) stay in LDS over the whole launch; the actor runs on wavefronts 0 .. 3, then lanes 0 .. 15 of
-// wavefront 0 step one env each (Float64, state in registers for the four sub-steps), account and rebuild
-// finished rows in place, while the critic runs beside them on wavefronts 2, 3, 6 and 7.
+// observation) stay in LDS over the whole launch; the actor runs on wavefronts 0 .. 3, beside it the next step's normal
+// numbers (wavefronts 4 and 6) and the last step's rollout row and episode sums (5), then lanes 0 .. 15 of
+// wavefront 0 step one env each (Float64, state in registers for the four sub-steps) and rebuild
+// finished rows in place, while the critic runs beside them on wavefronts 2, 3, 6 and 7, at width 256 on 1 to 3 and 5 to 7.
 template <class M, int H, int ACT>
 __global__ __launch_bounds__(512) void collect_planar_kernel(CollectArgs a) {
     // Widths up to which the actor's weights stay in registers.  Hopper's two workgroups a CU want no more than 128 of them.

@@ -11,7 +11,7 @@
 // one, or single steps.
 //
 // It gives what n_steps calls of mrl_rollout_step give (same per-env streams: seeds are affine
-// in the step number), except that the finished-episode list is appended in the order in which
+// in the step number), except that the finished-episode list is appended, every sixteen steps, in the order in which
 // blocks get there rather than step by step.
 #include "mrl_host.hpp"
 #include "mrl_device.hpp"

@@ -93,10 +93,6 @@ MRL_DEV int sample_categorical_quad(float logit, int A, float u, int l, float &p
     prob_sel = sel == 0 ? p0 : sel == 1 ? p1 : sel == 2 ? p2 : p3;
     return sel;
 }
-MRL_DEV int sample_categorical_quad(const float *logits, int A, uint32_t seed, int i, int l) {
-    float unused;
-    return sample_categorical_quad(l < A ? logits[l] : 0.0f, A, categorical_uniform(seed, i), l, unused);
-}
 
 // Gaussian sampling (deep_agents/ppo/kernels.mojo:12-98) of components j0 .. j0 + m of an action
 // with A components: one Philox stream per (env, component), Box-Muller, clamped log_std;
