@@ -42,8 +42,9 @@ struct Critic16Split {
 // sines and the log-probability off the solver, its detection in one pass of all four wavefronts: H = 64, 777 envs
 // 11.46 : 11.26, 4096 envs 11.86 : 11.55 (11.2 since a step's first loads are no longer waited for; thousand cycles of a
 // step there: actor 5.0, sample 1.1, detection 3.5, wait 0.8, engines 1.6, physics and tail 12, reset 1).  Numbers of the draw a
-// step ahead, rollout rows and episode sums a step later, at 8192 envs, H = 64 / 128 / 256: 12.2 / 16.2 / 27.6 : 12.1 / 15.9 /
-// 27.3, two continuous actions 14.8 / 19.2 / 30.4 : 14.7 / 18.7 / 29.8.  (32 envs a workgroup of eight wavefronts, a weight operand
+// step ahead, rollout rows and episode sums a step later, at 8192 envs, H = 64 / 128 / 256: 14.3 / 16.1 / 27.5 : 14.2 / 15.8 /
+// 27.4, two continuous actions 14.8 / 19.2 / 30.5 : 14.4 / 18.7 / 29.8 (means over three to twelve freshly initialised policies; of
+// the twelve at 256 ten are faster, by 0.4 to 1.3 %, and two slower, by 1.2: how the two workgroups of a CU fall in with each other).  (32 envs a workgroup of eight wavefronts, a weight operand
 // for two row tiles, H = 256: 27.2 at 8192 envs, but 27.0 : 26.1 at 4097 and 53.6 : 44.7 at 9001: matrix and vector time of a
 // SIMD add up either way.)
 // The solver wavefront is 0 in the lower half of the grid and 2 in the upper half: workgroups i and
